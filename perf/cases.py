@@ -77,12 +77,12 @@ def draw(rng):
     if kind in ("dense", "packed"):
         dim = rng.choice([64, 128])
         kv = rng.choice([1, 2, 4, 8, 12])
-        heads = kv * rng.choice([1, 1, 2, 4]) if kv > 1 else rng.choice([4, 8])
+        heads = kv * rng.choice([1, 1, 2, 2 if kv > 8 else 4]) if kv > 1 else rng.choice([4, 8])
         if kind == "packed":
             return dict(kind=kind, tokens=_log_int(rng, 1024, 16384), longest=_log_int(rng, 128, 4096), heads=heads,
                         kv_heads=kv, dim=dim)
         seq = _log_int(rng, 128, 8192)
-        return dict(kind=kind, batch=max(1, _log_int(rng, 512, 16384) // seq), seq=seq, heads=min(heads, 32), kv_heads=kv,
+        return dict(kind=kind, batch=max(1, _log_int(rng, 512, 16384) // seq), seq=seq, heads=heads, kv_heads=kv,
                     dim=dim, causal=rng.random() < 0.6, padded=rng.random() < 0.4)
     if kind == "paged":
         kv = rng.choice([2, 4, 8])
