@@ -1,30 +1,35 @@
 // Flash attention forward + backward for gfx950 (CDNA4), bf16, causal, GQA.
 //
 // MI355X-native design (not a CUDA port):
-//  - mfma_f32_32x32x16_bf16 tiles; 64-wide waves; 8 waves per workgroup
-//    forward, 4-wave blocks backward.
-//  - ALL operand tiles live in LDS in ONE layout: "subtiled row-major"
-//    [D/16 col-groups][ROWS][16 elems] with 32 B row pitch (+16 B pad per
-//    group to stagger banks). Row-slice fragment reads (8 consecutive d at
-//    fixed row) are single 16 B vector loads; COLUMN fragment reads (the
-//    transposed consumption that previously needed separate [D][ROWS]
-//    tiles built with 64 scalar ds_write_b16 per thread per tile) use
-//    gfx950's ds_read_b64_tr_b16 hardware weave (guide T10).
-//    HW-verified semantics (tr16_probe, mfma_selftest.hip): each lane reads
-//    64 bits at its own address; within a 16-lane group, out[l][j] =
-//    pool[(l&15) + 16 j] where pool is the group's reads in lane order.
-//    With lane addressing row=(m>>2), byte=(m&3)*8 this delivers
-//    tile[row0+j][col m] per lane — a free 4x16 transpose with any row pitch.
-//  - forward: each wave owns 32 q rows; K/V tiles of 64 staged subtiled;
-//    QK^T operand-swapped (S^T = K.Q^T) so softmax is lane-local; defer-max
-//    rescale (T13); async-split staging (T14): next tile's global loads
-//    issue before this tile's MFMAs.
-//  - backward FA2-split: delta preprocess; dK/dV kernel (per kv-tile, GQA
-//    group in registers); dQ kernel (per q-tile). P/dS restage between the
-//    MFMA C-layout and A-fragment layout goes through a per-wave 2 KB
-//    subtiled tile: packed 8 B stores (4 consecutive rows of the C-layout
-//    share a lane) + tr-read A-fragments. Score tiles are processed in
-//    32-wide halves, halving live p/dp registers.
+//  - mfma_f32_32x32x16_bf16 tiles; 64-wide waves; a wave owns 32 query rows (forward,
+//    dQ) or 32 key/value rows (dK/dV); blocks of 4 waves, 2 for small forward grids.
+//  - ALL operand tiles live in LDS in ONE layout, column groups of 16 channels
+//    (tile_off below). Row-slice fragment reads (8 consecutive d at a fixed row) are
+//    single 16 B loads; COLUMN fragment reads use gfx950's ds_read_b64_tr_b16.
+//    HW-verified semantics (mfma_selftest.hip): each lane reads 64 bits at its own
+//    address; within a 16-lane group, out[l][j] = pool[(l&15) + 16 j] where pool is
+//    the group's reads in lane order. With lane addressing row=(m>>2), byte=(m&3)*8
+//    this delivers tile[row0+j][col m] per lane — a free 4x16 transpose.
+//  - No intermediate passes through LDS: every product whose operand is a result (P · V,
+//    P^T · dO, dS^T · Q, dS · K) is arranged so that the contracted index lies in a lane's
+//    registers, and takes them in the order of the C layout (frag_born).
+//  - All global loads of the next tile issue before the current tile's products; two LDS
+//    buffers, one barrier a tile.
+//  - backward: delta preprocess, then ONE launch whose blocks take key/value tiles (dK/dV)
+//    or query tiles (dQ); both form the scores again.
+//
+// What bounds it (B2 S2048 H16/8 D128, not causal): the matrix unit is busy 41 % of the forward
+// and 43 % of the backward, the vector unit 40 %, LDS 40 % of the time. The two waves of a SIMD overlap
+// little of their products and exponentials; running them one phase apart with barriers (726 TFLOP/s),
+// forming the next tile's scores under the softmax (830 at 245 registers, 196 at D64 for want of waves) and
+// eight-wave blocks were measured against the 835 of this form.
+//
+// TFLOP/s, forward 2 products / backward 5 products of the visible pairs, before -> after:
+//   B4 S4096 H32 D128 causal          forward 694 -> 800, backward 498 -> 612
+//   B1 S8192 H32/8 D128 causal        forward 730 -> 917, backward 490 -> 668
+//   B8 S1024 H12 D64 causal           forward 215 -> 350, backward 225 -> 326
+//   B16 S512 H12 D64                  forward 361 -> 525, backward 294 -> 443
+//   packed, 10 sequences of 256..4096 forward 216 -> 695, backward 197 -> 573
 //
 // Shapes: q [B,S,Hq,D], k/v [B,S,Hkv,D] ("bshd" — no transposes in the
 // model), D in {64,128}. lse/delta are [B,Hq,S] fp32.
@@ -45,14 +50,7 @@ namespace fa {
 
 constexpr int KVB = 64;     // kv rows per tile
 constexpr int QW = 32;      // q rows per wave (fwd / dq); kv rows per wave (dkdv)
-constexpr int NW = 8;       // waves per block (forward). NW=4 (two independent
-                            // blocks/CU for natural stagger) measured 319 vs 519
-                            // TF — the doubled K/V staging work loses more than
-                            // the barrier decoupling gains; struck.
-constexpr int NT = 512;     // threads per block (forward)
-// Backward kernels carry dK+dV (or dQ) accumulators plus K/V (or Q/dO)
-// fragments in registers (~380-450 VGPR+AGPR): 1 wave/SIMD — 4-wave blocks.
-constexpr int NWB = 4;
+constexpr int NWB = 4;     // waves of a backward block
 constexpr int NTB = 256;
 
 DEV_INLINE bf16x8_t ld_g16(const unsigned short* p) {
@@ -67,29 +65,56 @@ DEV_INLINE bf16x8_t ld_lds16(const char* lds, int byte) {
   return *reinterpret_cast<const bf16x8_t*>(lds + byte);
 }
 
-DEV_INLINE unsigned short bf_raw(__bf16 b) {
-  union { __bf16 b; unsigned short u; } c;
-  c.b = b;
-  return c.u;
-}
-
-DEV_INLINE __bf16 f2b(float f) {
-  union { unsigned short u; __bf16 b; } c;
-  c.u = f2bf(f);
-  return c.b;
-}
-
 // C-layout row for mfma_f32_32x32x16 register j (guide §3, HW-verified).
 DEV_INLINE constexpr int crow(int j, int half) { return (j & 3) + 8 * (j >> 2) + 4 * half; }
 
-// Subtiled row-major LDS tiles + ds_read_b64_tr_b16 column fragments live
-// in common.h (shared with grouped_gemm.hip); re-exported into this
-// namespace for the kernel bodies below.
-using cai::sub_pitch;
-using cai::sub_off;
-using cai::sub_bytes;
-using cai::ld_tr16;
-using cai::ld_frag_tr;
+// An operand tile in LDS: column groups of 16 channels, [D/16][ROWS][16], 32 bytes a row, 128 bytes
+// between the groups: a transposing read takes 128 contiguous bytes from each of two neighbouring
+// groups at a time, which then lie in different halves of the 64 banks. 16 bytes apart they collided: conflicts
+// were 49 % of the forward's active LDS cycles and are 37 % now, the rest in the row-slice reads. (Planes of 8
+// channels bring them to 16 % and no time: LDS is not what bounds these kernels.)
+template <int ROWS>
+__host__ __device__ constexpr int tile_pitch() { return ROWS * 32 + 128; }
+
+template <int ROWS>
+DEV_INLINE int tile_off(int row, int col) { return (col >> 4) * tile_pitch<ROWS>() + row * 32 + (col & 15) * 2; }
+
+template <int ROWS, int COLS>
+__host__ __device__ constexpr int tile_bytes() { return (COLS / 16) * tile_pitch<ROWS>(); }
+
+// Column fragment by transposing reads, in the order in which the C layout hands out its rows: lane l
+// receives tile[k_base + 8*(e>>2) + 4*(l>>5) + (e&3)][cg_base*16 + (l&31)], e = 0..7, so
+// that a packed run of eight C registers is the matching other operand.
+template <int ROWS>
+DEV_INLINE bf16x8_t frag_born(const char* tile, int lane, int k_base, int cg_base) {
+  const int m = lane & 15;
+  const int cg = cg_base + ((lane >> 4) & 1);
+  const int at = cg * tile_pitch<ROWS>() + (k_base + (lane >> 5) * 4 + (m >> 2)) * 32 + (m & 3) * 8;
+  const bf16x4_v lo = ld_tr16(tile, at);
+  const bf16x4_v hi = ld_tr16(tile, at + 8 * 32);
+  return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+}
+
+// Which (q tile, sequence, head) a block of the forward works on. Blocks of one (sequence, head) share an
+// XCD's L2. Packed batches run head by head, each head over all sequences: the other way round
+// the longest sequence is one XCD's work (10 sequences of 256..4096 tokens: 1488 against 463 us). Under a causal
+// mask the late tiles see the most keys: they start first. A grid that fits on the chip at once (two blocks a
+// CU) runs every second head the other way, so that a CU's two blocks are a long and a short one.
+template <bool VARLEN>
+DEV_INLINE void q_block(int B, int Hq, int causal, int& tile, int& b, int& h) {
+  int y;
+  xcd_swizzle_xy(tile, y);
+  const bool once = (int)(gridDim.x * gridDim.y) <= 512 && (y & 1);
+  if (causal && !once) tile = (int)gridDim.x - 1 - tile;
+  b = VARLEN ? y % B : y / Hq;
+  h = VARLEN ? y / B : y % Hq;
+}
+
+// Logical index of block f of nblocks so that every XCD (block f runs on XCD f % 8) gets a contiguous range.
+DEV_INLINE int xcd_chunk(int f, int nblocks) {
+  const int q = nblocks >> 3, r = nblocks & 7, xcd = f & 7;
+  return (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + (f >> 3);
+}
 
 // Synchronous staging: load + store back-to-back (transient registers).
 template <int D, int ROWS, int NT_>
@@ -106,21 +131,23 @@ struct RegStage {
   static_assert(ROWS * CPR % NT_ == 0, "RegStage: uneven chunking");
   bf16x8_t r[NCH];
 
+  // A wave's instruction covers 16 rows of 64 bytes: with whole rows per instruction the stores
+  // of a row's column groups met in the same LDS banks.
+  DEV_INLINE static int row_of(int i) { return ((int)(threadIdx.x + i * NT_) / (CPR * 16)) * 16 + ((threadIdx.x & 63) >> 2); }
+  DEV_INLINE static int col_of(int i) {
+    return ((((int)(threadIdx.x + i * NT_) >> 6) % (CPR / 4)) * 4 + (threadIdx.x & 3)) * 8;
+  }
+
   DEV_INLINE void load(const unsigned short* base, long tok_stride, int row0, int S) {
 #pragma unroll
     for (int i = 0; i < NCH; ++i) {
-      const int c = (int)threadIdx.x + i * NT_;
-      const int row = c / CPR, ch = c % CPR;
-      const int grow = max(min(row0 + row, S - 1), 0);
-      r[i] = ld_g16(base + (long)grow * tok_stride + ch * 8);
+      const int grow = max(min(row0 + row_of(i), S - 1), 0);
+      r[i] = ld_g16(base + (long)grow * tok_stride + col_of(i));
     }
   }
-  DEV_INLINE void store_subtiled(char* lds) const {
+  DEV_INLINE void store(char* lds) const {
 #pragma unroll
-    for (int i = 0; i < NCH; ++i) {
-      const int c = (int)threadIdx.x + i * NT_;
-      st_lds16(lds, sub_off<ROWS>(c / CPR, (c % CPR) * 8), r[i]);
-    }
+    for (int i = 0; i < NCH; ++i) st_lds16(lds, tile_off<ROWS>(row_of(i), col_of(i)), r[i]);
   }
 };
 
@@ -128,23 +155,14 @@ template <int D, int ROWS, int NT_>
 DEV_INLINE void stage_direct(char* lds, const unsigned short* base, long stride, int row0, int S) {
   RegStage<D, ROWS, NT_> st;
   st.load(base, stride, row0, S);
-  st.store_subtiled(lds);
-}
-
-// Swizzled byte offset inside a row-major LDS tile with ROWB bytes per row
-// (forward P tile only). XOR spreads a column access across the row's
-// 16-byte slots — guide §6 G4.
-template <int ROWB>
-DEV_INLINE int swz(int row, int byte_in_row) {
-  constexpr int CPR_MASK = (ROWB / 16) - 1;
-  return row * ROWB + (byte_in_row ^ ((row & CPR_MASK) << 4));
+  st.store(lds);
 }
 
 }  // namespace fa
 
 // ============================================================ forward kernel
 //
-// grid: (ceil(S/256), B*Hq). LDS: K_sub + V_sub + P[NW][32][KVB].
+// grid: (ceil(S / (32 NW)), B*Hq). LDS: two key and two value tiles.
 //
 // Mask generality (reference: colossalai/shardformer/layer/attn.py:139
 // prepare_attn_kwargs CAUSAL / PADDED / PADDED_CAUSAL + varlen):
@@ -158,8 +176,8 @@ DEV_INLINE int swz(int row, int byte_in_row) {
 //  - CUK (padded path only): SEPARATE kv-side valid counts — ring-attention
 //    pieces where the q chunk and the arriving kv chunk cover different
 //    parts of each padded sequence. null -> kv counts = CU.
-template <int D, bool VARLEN>
-__global__ __launch_bounds__(fa::NT) void fa_fwd_kernel(
+template <int D, int NW, bool VARLEN>
+__global__ __launch_bounds__(NW * 64, 2) void fa_fwd_kernel(
     const unsigned short* __restrict__ Q,
     const unsigned short* __restrict__ K,
     const unsigned short* __restrict__ V,
@@ -171,23 +189,17 @@ __global__ __launch_bounds__(fa::NT) void fa_fwd_kernel(
     int B, int S, int Sk, int Hq, int Hkv, float scale, int causal) {
   using namespace fa;
   extern __shared__ char smem[];
-  constexpr int KB_BYTES = sub_bytes<KVB, D>();
-  // double-buffered K/V: tile t+1 stages into the OTHER buffer while tile
-  // t is being consumed — one barrier per tile instead of two
-  // (no pointer array: LDS addrspace casts cannot form a static initializer)
-  char* Pw = smem + 4 * KB_BYTES;  // + wave*QW*KVB*2
-
+  constexpr int NT = NW * 64;
+  constexpr int KB_BYTES = tile_bytes<KVB, D>();
   const int lane = threadIdx.x & 63;
   const int w = threadIdx.x >> 6;
   const int half = lane >> 5;
   const int ln = lane & 31;
 
-  int swz_x, swz_y;
-  xcd_swizzle_xy(swz_x, swz_y);  // same-bh tiles share one XCD's L2 (K/V reuse)
-  const int bh = swz_y;
-  const int b = bh / Hq, h = bh % Hq;
+  int tile, b, h;
+  q_block<VARLEN>(B, Hq, causal, tile, b, h);
   const int hk = h / (Hq / Hkv);
-  const int q0 = swz_x * (NW * QW);
+  const int q0 = tile * (NW * QW);
   const int qw = q0 + w * QW;  // this wave's first q row
 
   long seq0 = 0;
@@ -211,20 +223,25 @@ __global__ __launch_bounds__(fa::NT) void fa_fwd_kernel(
   const long o_stride = (long)Hq * D;  // O/LSE are always packed
 
   constexpr int DSL = D / 16;  // MFMA K-slices over the head dim
-  char* P = Pw + w * (QW * KVB * 2);
 
   // ---- Q fragments (B-operand of S^T = K·Q^T): lane holds q-col (ln),
   //      d-rows half*8+[0..7] per 16-d slice — one 16 B load per slice.
-  const int q_my = min(qw + ln, Seff - 1);
+  // A negative scale moves into Q as an exact sign flip, so that the largest
+  // product of a row is its largest score.
+  const int q_my = max(min(qw + ln, Seff - 1), 0);
   bf16x8_t qf[DSL];
   {
     const unsigned short* qp = q_base + (long)q_my * qts + half * 8;
 #pragma unroll
     for (int sl = 0; sl < DSL; ++sl) qf[sl] = ld_g16(qp + sl * 16);
+    if (scale < 0.0f) {
+#pragma unroll
+      for (int sl = 0; sl < DSL; ++sl) qf[sl] = -qf[sl];
+    }
   }
 
-  const float scale2 = scale * 1.44269504f;  // scale * log2(e)
-  f32x16 oacc[D / 32];
+  const float scale2 = fabsf(scale) * 1.44269504f;  // |scale| * log2(e)
+  f32x16 oacc[D / 32];                              // O^T: column = q row (ln), rows = channels
 #pragma unroll
   for (int nb = 0; nb < D / 32; ++nb)
 #pragma unroll
@@ -232,177 +249,128 @@ __global__ __launch_bounds__(fa::NT) void fa_fwd_kernel(
   float m_run = -INFINITY, l_run = 0.0f;
 
   const int kv_tiles_all = (SeffK + KVB - 1) / KVB;
-  const int kv_tiles = causal ? min(kv_tiles_all, (q0 + NW * QW + KVB - 1) / KVB) : kv_tiles_all;
+  const int kv_tiles = causal ? min(kv_tiles_all, (min(q0 + NW * QW, Seff) + KVB - 1) / KVB) : kv_tiles_all;
 
-  // async-split staging (T14): tile 0 staged synchronously, tile t+1's global
-  // loads issue before tile t's compute and land in LDS after the barrier.
-  RegStage<D, KVB, NT> kstage, vstage;
-  // SeffK == 0 blocks skip the tile loop; the clamped loads stay in-bounds
-  kstage.load(k_base, kts, 0, SeffK);
-  vstage.load(v_base, kts, 0, SeffK);
-  kstage.store_subtiled(smem);
-  vstage.store_subtiled(smem + KB_BYTES);
-  __syncthreads();
+  // tiles this wave computes: those above its diagonal produce nothing (barriers stay uniform)
+  const int my_tiles = qw >= Seff ? 0 : (causal ? min(kv_tiles, (qw + QW - 1) / KVB + 1) : kv_tiles);
 
-  for (int t = 0; t < kv_tiles; ++t) {
-    const int k0 = t * KVB;
-    const bool has_next = (t + 1 < kv_tiles);
-    char* Klds = smem + (t & 1) * 2 * KB_BYTES;
-    char* Vlds = Klds + KB_BYTES;
-    if (has_next) {
-      kstage.load(k_base, kts, k0 + KVB, SeffK);
-      vstage.load(v_base, kts, k0 + KVB, SeffK);
+  constexpr int KB = KVB / 32;
+  const int q_abs = qw + ln;
+  char* Kbuf = smem;                 // [2] key tiles, then [2] value tiles
+  char* Vbuf = smem + 2 * KB_BYTES;
+
+  // ---- S^T = K · Q^T : KVB/32 32-k blocks. C: col = q (ln), row = k (crow).
+  auto scores = [&](const char* Klds, f32x16 (&s)[KB]) {
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+      for (int j = 0; j < 16; ++j) s[kb][j] = 0.0f;
+#pragma unroll
+    for (int sl = 0; sl < DSL; ++sl) {
+#pragma unroll
+      for (int kb = 0; kb < KB; ++kb)
+        s[kb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+            ld_lds16(Klds, tile_off<KVB>(kb * 32 + ln, sl * 16 + half * 8)), qf[sl], s[kb], 0, 0, 0);
     }
-    // waves entirely above the diagonal produce nothing (barriers stay uniform)
-    const bool active = !(causal && k0 > qw + QW - 1) && (qw < Seff);
-    if (active) {
-    // ---- S^T = K · Q^T : KVB/32 32-k blocks. C: col = q (ln), row = k (crow).
-    // The kb accumulator chains are independent: interleaving them keeps
-    // two MFMAs in flight instead of one serial 8-deep chain per block.
-    constexpr int KB = KVB / 32;
-    float p[KB][16];
-    {
-      f32x16 acc[KB];
-#pragma unroll
-      for (int kb = 0; kb < KB; ++kb)
-#pragma unroll
-        for (int j = 0; j < 16; ++j) acc[kb][j] = 0.0f;
-      // software-pipelined A-operand loads: slice sl+1's LDS reads issue
-      // UNDER slice sl's MFMAs (the ld->mfma dependency chain was the
-      // limiter — each b128 LDS read is ~64 cycles the MFMA waited out)
-      bf16x8_t kf_cur[KB], kf_nxt[KB];
-#pragma unroll
-      for (int kb = 0; kb < KB; ++kb)
-        kf_cur[kb] = ld_lds16(Klds, sub_off<KVB>(kb * 32 + ln, half * 8));
-#pragma unroll
-      for (int sl = 0; sl < DSL; ++sl) {
-        if (sl + 1 < DSL) {
-#pragma unroll
-          for (int kb = 0; kb < KB; ++kb)
-            kf_nxt[kb] = ld_lds16(Klds, sub_off<KVB>(kb * 32 + ln, (sl + 1) * 16 + half * 8));
-        }
-        __builtin_amdgcn_s_setprio(1);
-#pragma unroll
-        for (int kb = 0; kb < KB; ++kb)
-          acc[kb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf_cur[kb], qf[sl], acc[kb], 0, 0, 0);
-        __builtin_amdgcn_s_setprio(0);
-#pragma unroll
-        for (int kb = 0; kb < KB; ++kb) kf_cur[kb] = kf_nxt[kb];
-      }
-      // exp2-domain softmax: v_exp_f32 IS exp2, so fold scale*log2e into
-      // the copy-out and every __expf's hidden *log2e mul disappears.
-      // m_run / l_run / rowmax live in the log2 domain; LSE converts back
-      // at the epilogue.
-#pragma unroll
-      for (int kb = 0; kb < KB; ++kb)
-#pragma unroll
-        for (int j = 0; j < 16; ++j) p[kb][j] = acc[kb][j] * scale2;
-    }
-
-    // ---- online softmax over this tile's 64 scores of q-row (qw+ln)
-    const int q_abs = qw + ln;
-    float rowmax = -INFINITY;
-    // interior tiles (every row/col in range, strictly below the causal
-    // diagonal) skip the per-element mask math — at S=4096 that is ~94%
-    // of tiles, and the mask chain was ~4 VALU ops per score
-    const bool full = (k0 + KVB <= SeffK) && (qw + QW <= Seff) && (!causal || k0 + KVB - 1 <= qw);
-    if (full) {
-#pragma unroll
-      for (int kb = 0; kb < KB; ++kb)
-#pragma unroll
-        for (int j = 0; j < 16; ++j) rowmax = fmaxf(rowmax, p[kb][j]);
-    } else {
+  };
+  // interior tiles (every row/col in range, strictly below the causal diagonal) need no mask:
+  // at S=4096 that is ~94% of tiles, and the mask chain is ~4 VALU ops per score
+  auto masked = [&](int k0) { return !((k0 + KVB <= SeffK) && (qw + QW <= Seff) && (!causal || k0 + KVB - 1 <= qw)); };
+  auto mask = [&](int k0, f32x16 (&s)[KB]) {
 #pragma unroll
     for (int kb = 0; kb < KB; ++kb)
 #pragma unroll
       for (int j = 0; j < 16; ++j) {
         const int k_abs = k0 + kb * 32 + crow(j, half);
         const bool valid = (q_abs < Seff) && (k_abs < SeffK) && (!causal || k_abs <= q_abs);
-        if (!valid) p[kb][j] = -INFINITY;
-        rowmax = fmaxf(rowmax, p[kb][j]);
+        if (!valid) s[kb][j] = -INFINITY;
       }
-    }
+  };
+  auto largest = [&](const f32x16 (&s)[KB]) {
+    float r = s[0][0];
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+      for (int j = 0; j < 16; ++j) r = fmaxf(r, s[kb][j]);
+    return r;
+  };
+
+  // ---- online softmax of a tile's 64 scores of q-row (qw+ln). The running maximum is kept in the
+  // base-2 domain (v_exp_f32 is exp2); the scale enters with the fma that subtracts it.
+  // P in the order it was born in is the B operand of O^T += V^T · P^T: slot half*8+e of a 16-k step holds
+  // key 8*(e>>2) + 4*half + (e&3) of it, and the V column fragments are read in the same key
+  // order. P never passes through LDS.
+  bf16x8_t pb[KB][2];
+  auto softmax = [&](int k0, f32x16 (&s)[KB]) {
+    if (masked(k0)) mask(k0, s);
+    float rowmax = largest(s);
     rowmax = fmaxf(rowmax, __shfl_xor(rowmax, 32));
+    rowmax = rowmax == -INFINITY ? -INFINITY : rowmax * scale2;  // no 0 * inf
     // defer-max (guide T13): if this tile's max is within 8 of the running
     // max, keep the old max (P bounded by e^8, fine in fp32/bf16) and skip
     // the O-rescale pass entirely when every row defers.
     const bool defer = (m_run != -INFINITY) && (rowmax - m_run <= 11.5416f);  // 8 nats in log2
-    const float m_new = defer ? m_run : fmaxf(m_run, rowmax);
-    const float msafe = (m_new == -INFINITY) ? 0.0f : m_new;
-    const float corr =
-        defer ? 1.0f : ((m_run == -INFINITY) ? ((m_new == -INFINITY) ? 1.0f : 0.0f) : __builtin_amdgcn_exp2f(m_run - m_new));
+    if (!__all(defer)) {
+      const float m_new = defer ? m_run : fmaxf(m_run, rowmax);
+      const float corr = m_run == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m_run - m_new);  // nothing summed yet: 0
+#pragma unroll
+      for (int nb = 0; nb < D / 32; ++nb)
+#pragma unroll
+        for (int j = 0; j < 16; ++j) oacc[nb][j] *= corr;
+      l_run *= corr;
+      m_run = m_new;
+    }
+    const float msafe = (m_run == -INFINITY) ? 0.0f : m_run;
     float rowsum = 0.0f;
 #pragma unroll
     for (int kb = 0; kb < KB; ++kb)
 #pragma unroll
       for (int j = 0; j < 16; ++j) {
-        p[kb][j] = __builtin_amdgcn_exp2f(p[kb][j] - msafe);
-        rowsum += p[kb][j];
+        const float pv = __builtin_amdgcn_exp2f(fmaf(s[kb][j], scale2, -msafe));
+        rowsum += pv;
+        pb[kb][j >> 3][j & 7] = (__bf16)pv;
       }
-    rowsum += __shfl_xor(rowsum, 32);
-    m_run = m_new;
-    l_run = l_run * corr + rowsum;
-
-    // ---- stage P (bf16) into swizzled per-wave LDS: P[q=ln][k]
-    // C-regs j=0..3 within a group are 4 consecutive k values → 8 B packed.
+    l_run += rowsum;  // this lane's half of the row's keys; the halves meet at the end
+  };
+  auto values = [&](const char* Vlds) {
 #pragma unroll
     for (int kb = 0; kb < KB; ++kb)
 #pragma unroll
-      for (int jj = 0; jj < 4; ++jj) {
-        const int kcol = kb * 32 + 8 * jj + 4 * half;
-        short4v pk;
+      for (int s2 = 0; s2 < 2; ++s2)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) pk[e] = (short)f2bf(p[kb][jj * 4 + e]);
-        *reinterpret_cast<short4v*>(P + swz<KVB * 2>(ln, kcol * 2)) = pk;
-      }
+        for (int nb = 0; nb < D / 32; ++nb)
+          oacc[nb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+              frag_born<KVB>(Vlds, lane, kb * 32 + s2 * 16, nb * 2), pb[kb][s2], oacc[nb], 0, 0, 0);
+  };
 
-    // ---- rescale O accumulator by corr (per q-row, via shfl broadcast);
-    // skipped entirely when every row of the wave deferred (corr == 1)
-    if (!__all(corr == 1.0f)) {
-#pragma unroll
-      for (int j = 0; j < 16; ++j) {
-        const int r = crow(j, half);
-        const float c = __shfl(corr, r);  // corr for q-row r lives on lanes r, r+32
-#pragma unroll
-        for (int nb = 0; nb < D / 32; ++nb) oacc[nb][j] *= c;
-      }
+  RegStage<D, KVB, NT> kstage, vstage;
+  f32x16 sc[KB];
+  // async-split staging (T14): tile t+1's global loads issue before tile t's compute; their stores
+  // target the OTHER buffer, so that one barrier a tile does
+  // SeffK == 0 blocks skip the tile loop; the clamped loads stay in-bounds
+  kstage.load(k_base, kts, 0, SeffK);
+  vstage.load(v_base, kts, 0, SeffK);
+  kstage.store(Kbuf);
+  vstage.store(Vbuf);
+  __syncthreads();
+  for (int t = 0; t < kv_tiles; ++t) {
+    const bool more = t + 1 < kv_tiles;
+    if (more) {
+      kstage.load(k_base, kts, (t + 1) * KVB, SeffK);
+      vstage.load(v_base, kts, (t + 1) * KVB, SeffK);
     }
-
-    // ---- O += P · V  (A = P from LDS, B = V column-fragments via tr-read)
-    // software-pipelined: the NEXT (pa, vb) pair's LDS reads issue under
-    // the current MFMA so the ld->mfma chain never serializes
-    {
-      constexpr int KS = KVB / 16, NB = D / 32;
-      bf16x8_t pa_cur = ld_lds16(P, swz<KVB * 2>(ln, (half * 8) * 2));
-      bf16x8_t vb_cur = ld_frag_tr<KVB>(Vlds, lane, 0, 0);
-      bf16x8_t pa_nxt, vb_nxt;
-#pragma unroll
-      for (int ks = 0; ks < KS; ++ks) {
-#pragma unroll
-        for (int nb = 0; nb < NB; ++nb) {
-          if (nb + 1 < NB) {
-            vb_nxt = ld_frag_tr<KVB>(Vlds, lane, ks * 16, (nb + 1) * 2);
-          } else if (ks + 1 < KS) {
-            pa_nxt = ld_lds16(P, swz<KVB * 2>(ln, ((ks + 1) * 16 + half * 8) * 2));
-            vb_nxt = ld_frag_tr<KVB>(Vlds, lane, (ks + 1) * 16, 0);
-          }
-          __builtin_amdgcn_s_setprio(1);
-          oacc[nb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(pa_cur, vb_cur, oacc[nb], 0, 0, 0);
-          __builtin_amdgcn_s_setprio(0);
-          vb_cur = vb_nxt;
-          if (nb + 1 == NB) pa_cur = pa_nxt;
-        }
-      }
+    if (t < my_tiles) {
+      __builtin_amdgcn_s_setprio(1);
+      scores(Kbuf + (t & 1) * KB_BYTES, sc);
+      __builtin_amdgcn_s_setprio(0);
+      softmax(t * KVB, sc);
+      __builtin_amdgcn_s_setprio(1);
+      values(Vbuf + (t & 1) * KB_BYTES);
+      __builtin_amdgcn_s_setprio(0);
     }
-    }  // active
-
-    // stores target the OTHER buffer: no barrier needed before them, and
-    // the single barrier below covers both "stores visible" and "everyone
-    // done with this tile's buffer before it is reused two tiles on"
-    if (has_next) {
-      char* Kn = smem + ((t + 1) & 1) * 2 * KB_BYTES;
-      kstage.store_subtiled(Kn);
-      vstage.store_subtiled(Kn + KB_BYTES);
+    if (more) {
+      kstage.store(Kbuf + ((t + 1) & 1) * KB_BYTES);
+      vstage.store(Vbuf + ((t + 1) & 1) * KB_BYTES);
     }
     __syncthreads();
   }
@@ -411,26 +379,23 @@ __global__ __launch_bounds__(fa::NT) void fa_fwd_kernel(
   // batches) have l_run == 0 -> O = 0, LSE = -inf, which the backward uses
   // to mask them; the buffer extent S is still fully written.
   const int row_lim = VARLEN ? Seff : S;
-  if (qw >= row_lim) return;
+  l_run += __shfl_xor(l_run, 32);
+  if (q_abs >= row_lim) return;
   unsigned short* o_base = VARLEN ? O + (seq0 * Hq + h) * D : O + ((long)b * S * Hq + h) * D;
   float* lse_base = VARLEN ? LSE + (long)h * S + seq0 : LSE + ((long)b * Hq + h) * S;
+  const float inv_l = (l_run > 0.0f) ? 1.0f / l_run : 0.0f;
 #pragma unroll
-  for (int j = 0; j < 16; ++j) {
-    const int r = crow(j, half);
-    const float l_r = __shfl(l_run, r);
-    const float inv_l = (l_r > 0.0f) ? 1.0f / l_r : 0.0f;
-    const int q_abs = qw + r;
-    if (q_abs < row_lim) {
+  for (int nb = 0; nb < D / 32; ++nb)
 #pragma unroll
-      for (int nb = 0; nb < D / 32; ++nb) {
-        o_base[(long)q_abs * o_stride + nb * 32 + ln] = f2bf(oacc[nb][j] * inv_l);
-      }
+    for (int jj = 0; jj < 4; ++jj) {
+      short4v pk;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) pk[e] = (short)f2bf(oacc[nb][jj * 4 + e] * inv_l);
+      *reinterpret_cast<short4v*>(o_base + (long)q_abs * o_stride + nb * 32 + 8 * jj + 4 * half) = pk;
     }
-  }
-  if (lane < QW && qw + lane < row_lim) {
+  if (half == 0) {
     // back to nats: m_run is log2-domain
-    const float lse = (l_run > 0.0f) ? m_run * 0.6931472f + __logf(l_run) : -INFINITY;
-    lse_base[qw + lane] = lse;
+    lse_base[q_abs] = (l_run > 0.0f) ? m_run * 0.6931472f + __logf(l_run) : -INFINITY;
   }
 }
 
@@ -478,55 +443,57 @@ __global__ __launch_bounds__(256) void fa_delta_kernel(
   }
 }
 
-// ================================================= backward dK/dV kernel
+// ============================================================ backward kernel
 //
-// grid: (ceil(S/128) kv-tiles, B*Hkv). Each wave owns 32 kv rows; loops over
-// the GQA group's q-heads and that head's q-tiles (64 q rows staged subtiled
-// in LDS). dK/dV accumulate in registers across the whole loop. Score tiles
-// are processed in 32-q halves through a per-wave 2 KB P tile.
-// VAR experiment ladder (select at launch via CAI_FA_DKDV_VAR):
-//  0: async-split RegStage prefetch, K+V fragments resident, no occupancy
-//     bound (352 regs -> 1 wave/SIMD)
-//  1: same body, forced 2 waves/SIMD (256-reg cap -> ~75 spills)
-//  2: register diet for a TRUE 2 waves/SIMD: synchronous staging (no
-//     prefetch registers) + V fragments re-loaded from L1 each tile
-//  3: VAR 2 + K fragments also re-loaded (zero spill target)
-template <int D, int VAR, bool VARLEN = false>
-__global__ __launch_bounds__(fa::NTB, VAR >= 1 ? 2 : 1) void fa_bwd_dkdv_kernel(
-    const unsigned short* __restrict__ Q,
-    const unsigned short* __restrict__ K,
-    const unsigned short* __restrict__ V,
-    const unsigned short* __restrict__ dO,
-    const float* __restrict__ LSE,
-    const float* __restrict__ DELTA,
-    unsigned short* __restrict__ dK,
-    unsigned short* __restrict__ dV,
-    const int* __restrict__ CU,
-    const int* __restrict__ CUK,  // padded ring pieces: kv-side valid counts
+// One launch for dK/dV and dQ: the first n_kv blocks (a multiple of 8) take key/value tiles, the
+// others query tiles, so that both kinds share the CUs and no second stream is needed. Both form the
+// scores again; nothing is summed with atomics.
+//
+// In both parts the probabilities and their gradients are born with the row they are contracted
+// over in the registers of a lane (the C layout's rows), so a packed run of eight registers is an
+// operand of the next product as it stands and neither passes through LDS (frag_born reads the other
+// operand's columns in the same order).
+
+// A block of 4 waves owns 128 key/value rows, 32 a wave, and streams the query tiles of its group's heads
+// (32 rows, double-buffered). dK and dV stay in registers. What a query row adds (its -lse log2e and
+// -delta) enters as the accumulator the product starts from and as the exponent's addend; a row
+// that counts nothing (padding, or no visible key) has an addend of -inf.
+// GS blocks share a key/value tile's heads when there would be too few blocks otherwise; they leave
+// float32 partial sums in PART [GS][2][B * Sk * Hkv * D] for fa_bwd_sum_kernel.
+template <int D, bool VARLEN>
+DEV_INLINE void bwd_dkdv(
+    char* smem, int f, int nblocks,
+    const unsigned short* __restrict__ Q, const unsigned short* __restrict__ K,
+    const unsigned short* __restrict__ V, const unsigned short* __restrict__ dO,
+    const float* __restrict__ LSE, const float* __restrict__ DELTA,
+    unsigned short* __restrict__ dK, unsigned short* __restrict__ dV, float* __restrict__ PART, int GS,
+    const int* __restrict__ CU, const int* __restrict__ CUK,
     long qbs, long qts, long kbs, long kts, long dkbs, long dkts,
-    int B, int S, int Sk, int Hq, int Hkv, float scale, int causal) {
+    int tiles, int B, int S, int Sk, int Hq, int Hkv, float scale, int causal) {
   using namespace fa;
-  constexpr int QB = 64;  // q rows per staged tile
-  extern __shared__ char smem[];
-  constexpr int TB = sub_bytes<QB, D>();
-  constexpr int PB = sub_bytes<32, 32>();  // per-wave P tile: [q 32][kv 32]
-  char* Qlds = smem;
-  char* dOlds = smem + TB;
-  char* Pw = smem + 2 * TB;  // + wave*PB
-  float* lse_lds = reinterpret_cast<float*>(smem + 2 * TB + NWB * PB);
-  float* dta_lds = lse_lds + QB;
+  constexpr int QB = 32;
+  constexpr int TB = tile_bytes<QB, D>();
+  constexpr int DSL = D / 16, NB = D / 32;
+  char* Vlds = smem;                                     // [128 rows]
+  char* Qbuf = smem + tile_bytes<NWB * QW, D>();         // [2] query tiles, [2] dO tiles
+  char* dObuf = Qbuf + 2 * TB;
+  float* lse_lds = reinterpret_cast<float*>(dObuf + 2 * TB);  // [2][32] -lse log2e
+  float* dta_lds = lse_lds + 2 * QB;                          // [2][32] -delta
 
   const int lane = threadIdx.x & 63;
   const int w = threadIdx.x >> 6;
   const int half = lane >> 5;
   const int ln = lane & 31;
 
-  int swz_x, swz_y;
-  xcd_swizzle_xy(swz_x, swz_y);  // same-bh kv tiles share an XCD's L2 (Q/dO stream reuse)
-  const int bh = swz_y;
-  const int b = bh / Hkv, hk = bh % Hkv;
-  const int G = Hq / Hkv;
-  const int kv0 = swz_x * (NWB * QW);
+  f = xcd_chunk(f, nblocks);
+  // key/value tile fastest, then the part of the group's heads, then (sequence, kv head): their
+  // Q/dO streams meet in one XCD's L2. Under a causal mask the first tiles see the most queries.
+  const int kv0 = (f % tiles) * (NWB * QW);
+  const int part = (f / tiles) % GS;
+  const int y = f / (tiles * GS);
+  if (y >= B * Hkv) return;
+  const int b = VARLEN ? y % B : y / Hkv, hk = VARLEN ? y / B : y % Hkv;
+  const int G = Hq / Hkv / GS;                           // heads of this block
   const int kvw = kv0 + w * QW;  // this wave's first kv row
 
   long seq0 = 0;
@@ -538,312 +505,183 @@ __global__ __launch_bounds__(fa::NTB, VAR >= 1 ? 2 : 1) void fa_bwd_dkdv_kernel(
   } else if (CU != nullptr) {
     Seff = CU[b];
   }
-  // this kernel's OWN rows are kv (extent Sk); q streams over Seff
-  int SeffK = VARLEN ? Seff
+  // this part's OWN rows are kv (extent Sk); q streams over Seff
+  const int SeffK = VARLEN ? Seff
             : (CUK != nullptr ? CUK[b] : (CU != nullptr ? min(CU[b], Sk) : Sk));
 
   const unsigned short* k_base = VARLEN ? K + seq0 * kts + (long)hk * D : K + (long)b * kbs + (long)hk * D;
   const unsigned short* v_base = VARLEN ? V + seq0 * kts + (long)hk * D : V + (long)b * kbs + (long)hk * D;
+  const long do_stride = (long)Hq * D;
 
-  constexpr int DSL = D / 16;
-  char* P = Pw + w * PB;
-
-  // ---- K, V fragments (A-operands): lane row = kv (ln), d = sl*16+half*8+[0..7]
+  // ---- K fragments (B operand of S = Q · K^T): lane column = kv (ln), d = sl*16+half*8+[0..7]
   const int kv_my = max(min(kvw + ln, SeffK - 1), 0);
-  const unsigned short* vp = v_base + (long)kv_my * kts + half * 8;
-  const unsigned short* kp = k_base + (long)kv_my * kts + half * 8;
-  bf16x8_t kf[VAR == 3 ? 1 : DSL], vf[VAR >= 2 ? 1 : DSL];
+  bf16x8_t kf[DSL];
   {
+    const unsigned short* kp = k_base + (long)kv_my * kts + half * 8;
 #pragma unroll
-    for (int sl = 0; sl < DSL; ++sl) {
-      if (VAR != 3) kf[sl] = ld_g16(kp + sl * 16);
-      if (VAR < 2) vf[sl] = ld_g16(vp + sl * 16);
-    }
+    for (int sl = 0; sl < DSL; ++sl) kf[sl] = ld_g16(kp + sl * 16);
   }
+  // ---- V rows of the block (B operand of dP = dO · V^T): they do not fit into registers beside
+  // the two accumulators, each wave reads its own 32 rows from LDS
+  stage_direct<D, NWB * QW, NTB>(Vlds, v_base, kts, kv0, SeffK);
 
-  f32x16 dk_acc[D / 32], dv_acc[D / 32];
+  f32x16 dk_acc[NB], dv_acc[NB];
 #pragma unroll
-  for (int nb = 0; nb < D / 32; ++nb)
+  for (int nb = 0; nb < NB; ++nb)
 #pragma unroll
     for (int j = 0; j < 16; ++j) {
       dk_acc[nb][j] = 0.0f;
       dv_acc[nb][j] = 0.0f;
     }
 
-  const int qt_first = causal ? (kv0 / QB) : 0;
-  const int qt_last = (Seff + QB - 1) / QB;
+  const int qt_first = causal ? kv0 / QB : 0;
+  const int nq = max((Seff + QB - 1) / QB - qt_first, 0);   // query tiles of a head
+  const int steps = kv0 < SeffK ? nq * G : 0;
+  const float scale2 = scale * 1.44269504f;
 
   RegStage<D, QB, NTB> qstage, dostage;
-  for (int g = 0; g < G; ++g) {
-    const int h = hk * G + g;
+  float lse_r = 0.0f, dta_r = 0.0f;
+  auto fetch = [&](int step) {   // global loads of a step's query tile
+    const int h = hk * (Hq / Hkv) + part * G + step / nq;
+    const int qt0 = (qt_first + step % nq) * QB;
     const unsigned short* q_base = VARLEN ? Q + seq0 * qts + (long)h * D : Q + (long)b * qbs + (long)h * D;
     const unsigned short* do_base =
         VARLEN ? dO + (seq0 * Hq + h) * D : dO + ((long)b * S * Hq + h) * D;  // dO packed
-    const long do_stride = (long)Hq * D;
-    const float* lse_base = VARLEN ? LSE + (long)h * S + seq0 : LSE + ((long)b * Hq + h) * S;
-    const float* dta_base = VARLEN ? DELTA + (long)h * S + seq0 : DELTA + ((long)b * Hq + h) * S;
-
-    // prologue: stage the first q-tile of this head synchronously
-    if (VAR != 2) {
-      qstage.load(q_base, qts, qt_first * QB, Seff);
-      dostage.load(do_base, do_stride, qt_first * QB, Seff);
-    }
-    __syncthreads();  // previous head's compute done before overwriting LDS
-    if (VAR != 2) {
-      qstage.store_subtiled(Qlds);
-      dostage.store_subtiled(dOlds);
-    } else {
-      stage_direct<D, QB, NTB>(Qlds, q_base, qts, qt_first * QB, Seff);
-      stage_direct<D, QB, NTB>(dOlds, do_base, do_stride, qt_first * QB, Seff);
-    }
+    qstage.load(q_base, qts, qt0, Seff);
+    dostage.load(do_base, do_stride, qt0, Seff);
     if (threadIdx.x < QB) {
-      const int qr = max(min(qt_first * QB + (int)threadIdx.x, Seff - 1), 0);
-      lse_lds[threadIdx.x] = lse_base[qr];
-      dta_lds[threadIdx.x] = dta_base[qr];
+      const long at = (VARLEN ? (long)h * S + seq0 : ((long)b * Hq + h) * S) + min(qt0 + (int)threadIdx.x, Seff - 1);
+      lse_r = qt0 + (int)threadIdx.x < Seff ? LSE[at] : -INFINITY;
+      dta_r = DELTA[at];
     }
+  };
+  auto stash = [&](int buf) {
+    qstage.store(Qbuf + buf * TB);
+    dostage.store(dObuf + buf * TB);
+    if (threadIdx.x < QB) {
+      lse_lds[buf * QB + threadIdx.x] = lse_r == -INFINITY ? -INFINITY : -lse_r * 1.44269504f;
+      dta_lds[buf * QB + threadIdx.x] = -dta_r;
+    }
+  };
+  if (steps > 0) {
+    fetch(0);
+    stash(0);
+  }
+  __syncthreads();
+
+  for (int step = 0; step < steps; ++step) {
+    const int buf = step & 1;
+    const int qt0 = (qt_first + step % nq) * QB;
+    const bool more = step + 1 < steps;
+    if (more) fetch(step + 1);
+    const char* Qlds = Qbuf + buf * TB;
+    const char* dOlds = dObuf + buf * TB;
+    if (!(causal && qt0 + QB - 1 < kvw) && kvw < SeffK) {
+      // ---- S[q][kv] = Q · K^T and dP[q][kv] - delta[q] = dO · V^T - delta: column = kv (ln), row = q
+      f32x16 s, dp;
+      float addend[16];
+#pragma unroll
+      for (int a = 0; a < 4; ++a) {
+        const float4v l4 = *reinterpret_cast<const float4v*>(lse_lds + buf * QB + 8 * a + 4 * half);
+        const float4v d4 = *reinterpret_cast<const float4v*>(dta_lds + buf * QB + 8 * a + 4 * half);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          addend[4 * a + e] = l4[e];
+          dp[4 * a + e] = d4[e];
+          s[4 * a + e] = 0.0f;
+        }
+      }
+      __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+      for (int sl = 0; sl < DSL; ++sl) {
+        s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ld_lds16(Qlds, tile_off<QB>(ln, sl * 16 + half * 8)), kf[sl], s, 0, 0, 0);
+        dp = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ld_lds16(dOlds, tile_off<QB>(ln, sl * 16 + half * 8)),
+                                                     ld_lds16(Vlds, tile_off<NWB * QW>(w * QW + ln, sl * 16 + half * 8)),
+                                                     dp, 0, 0, 0);
+      }
+      __builtin_amdgcn_s_setprio(0);
+      // ---- P = exp(scale s - lse); dS = P (dP - delta), its scale waits for the epilogue
+      bf16x8_t pa[2], dsa[2];
+      const bool diagonal = causal && kvw + QW - 1 > qt0;
+#pragma unroll
+      for (int j = 0; j < 16; ++j) {
+        float pv = __builtin_amdgcn_exp2f(fmaf(s[j], scale2, addend[j]));
+        if (diagonal && kvw + ln > qt0 + crow(j, half)) pv = 0.0f;
+        pa[j >> 3][j & 7] = (__bf16)pv;
+        dsa[j >> 3][j & 7] = (__bf16)(pv * dp[j]);
+      }
+      // ---- dV += P^T · dO, dK += dS^T · Q (A: lane row = kv; B: columns of the tiles)
+      __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+      for (int s2 = 0; s2 < 2; ++s2)
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb) {
+          dv_acc[nb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(pa[s2], frag_born<QB>(dOlds, lane, s2 * 16, nb * 2), dv_acc[nb], 0, 0, 0);
+          dk_acc[nb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(dsa[s2], frag_born<QB>(Qlds, lane, s2 * 16, nb * 2), dk_acc[nb], 0, 0, 0);
+        }
+      __builtin_amdgcn_s_setprio(0);
+    }
+    // the stores target the other buffer: one barrier a step
+    if (more) stash(buf ^ 1);
     __syncthreads();
-
-    for (int qt = qt_first; qt < qt_last; ++qt) {
-      const int qt0 = qt * QB;
-      const bool has_next = (qt + 1 < qt_last);
-      if (VAR != 2 && has_next) {
-        qstage.load(q_base, qts, qt0 + QB, Seff);
-        dostage.load(do_base, do_stride, qt0 + QB, Seff);
-      }
-      const bool active = !(causal && qt0 + QB - 1 < kvw) && (kvw < SeffK);
-      if (active) {
-
-      // 32-q halves: live score state is p[16]+dp[16] instead of [2][16].
-#pragma unroll
-      for (int qb = 0; qb < 2; ++qb) {
-        // ---- S'^T[kv][q] = K · Q^T : C col = q (ln within half), row = kv.
-        f32x16 acc;
-#pragma unroll
-        for (int j = 0; j < 16; ++j) acc[j] = 0.0f;
-        // pipelined: slice sl+1's Q row-slice read issues under slice sl's MFMA
-        bf16x8_t qb_cur = ld_lds16(Qlds, sub_off<QB>(qb * 32 + ln, half * 8));
-        bf16x8_t qb_nxt;
-#pragma unroll
-        for (int sl = 0; sl < DSL; ++sl) {
-          if (sl + 1 < DSL)
-            qb_nxt = ld_lds16(Qlds, sub_off<QB>(qb * 32 + ln, (sl + 1) * 16 + half * 8));
-          bf16x8_t kfr = (VAR == 3) ? ld_g16(kp + sl * 16) : kf[VAR == 3 ? 0 : sl];
-          __builtin_amdgcn_s_setprio(1);
-          acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kfr, qb_cur, acc, 0, 0, 0);
-          __builtin_amdgcn_s_setprio(0);
-          qb_cur = qb_nxt;
-        }
-
-        // ---- P' = exp(scale*s - lse[q]), masked (interior blocks skip
-        // the per-element mask chain — most blocks at training seqlens)
-        float p[16];
-        {
-          const int q_abs = qt0 + qb * 32 + ln;
-          const float lse = lse_lds[qb * 32 + ln];
-          // exp2 domain: exp(a*s - l) = exp2(fma(a, s*log2e, -l*log2e))
-          const float scale2 = scale * 1.44269504f;
-          const float lse2 = lse * 1.44269504f;
-          const bool blk_full = (qt0 + qb * 32 + 32 <= Seff) && (kvw + QW <= SeffK) &&
-                                (!causal || kvw + QW - 1 <= qt0 + qb * 32);
-          if (blk_full) {
-#pragma unroll
-            for (int j = 0; j < 16; ++j)
-              p[j] = __builtin_amdgcn_exp2f(fmaf(acc[j], scale2, -lse2));
-          } else {
-#pragma unroll
-          for (int j = 0; j < 16; ++j) {
-            const int k_abs = kvw + crow(j, half);
-            const bool valid = (q_abs < Seff) && (k_abs < SeffK) && (!causal || k_abs <= q_abs) && (lse != -INFINITY);
-            p[j] = valid ? __builtin_amdgcn_exp2f(fmaf(acc[j], scale2, -lse2)) : 0.0f;
-          }
-          }
-        }
-
-        // ---- stage P' into the per-wave subtiled [q 32][kv 32] tile:
-        // C-regs j in a 4-group are 4 consecutive kv rows → packed 8 B store
-#pragma unroll
-        for (int jj = 0; jj < 4; ++jj) {
-          const int kv_loc = 8 * jj + 4 * half;
-          short4v pk;
-#pragma unroll
-          for (int e = 0; e < 4; ++e) pk[e] = (short)f2bf(p[jj * 4 + e]);
-          *reinterpret_cast<short4v*>(P + sub_off<32>(ln, kv_loc)) = pk;
-        }
-
-        // ---- dV += P' · dO  (A = P' via tr-read: lane row = kv, k = q-local;
-        //      B = dO column-fragments, k = q-global)
-        {
-          constexpr int NB = D / 32;
-          bf16x8_t pa_cur = ld_frag_tr<32>(P, lane, 0, 0);
-          bf16x8_t dob_cur = ld_frag_tr<QB>(dOlds, lane, qb * 32, 0);
-          bf16x8_t pa_nxt, dob_nxt;
-#pragma unroll
-          for (int ks2 = 0; ks2 < 2; ++ks2) {
-#pragma unroll
-            for (int nb = 0; nb < NB; ++nb) {
-              if (nb + 1 < NB) {
-                dob_nxt = ld_frag_tr<QB>(dOlds, lane, qb * 32 + ks2 * 16, (nb + 1) * 2);
-              } else if (ks2 == 0) {
-                pa_nxt = ld_frag_tr<32>(P, lane, 16, 0);
-                dob_nxt = ld_frag_tr<QB>(dOlds, lane, qb * 32 + 16, 0);
-              }
-              __builtin_amdgcn_s_setprio(1);
-              dv_acc[nb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(pa_cur, dob_cur, dv_acc[nb], 0, 0, 0);
-              __builtin_amdgcn_s_setprio(0);
-              dob_cur = dob_nxt;
-              if (nb + 1 == NB) pa_cur = pa_nxt;
-            }
-          }
-        }
-
-        // ---- dP'[kv][q] = V · dO^T  (A = V regs — VAR 2 re-loads each V
-        //      fragment from L1; the row is hot — B = dO row-slice reads)
-        f32x16 acc2;
-#pragma unroll
-        for (int j = 0; j < 16; ++j) acc2[j] = 0.0f;
-        bf16x8_t do_cur = ld_lds16(dOlds, sub_off<QB>(qb * 32 + ln, half * 8));
-        bf16x8_t do_nxt;
-        // VAR>=2 reloads V fragments from L1 — pipeline those too, the
-        // global-load latency was the serial chain here (PMC: both pipes idle)
-        bf16x8_t vf_cur = (VAR >= 2) ? ld_g16(vp) : vf[0];
-        bf16x8_t vf_nxt;
-#pragma unroll
-        for (int sl = 0; sl < DSL; ++sl) {
-          if (sl + 1 < DSL) {
-            do_nxt = ld_lds16(dOlds, sub_off<QB>(qb * 32 + ln, (sl + 1) * 16 + half * 8));
-            if (VAR >= 2) vf_nxt = ld_g16(vp + (sl + 1) * 16);
-          }
-          bf16x8_t vfr = (VAR >= 2) ? vf_cur : vf[VAR >= 2 ? 0 : sl];
-          acc2 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vfr, do_cur, acc2, 0, 0, 0);
-          do_cur = do_nxt;
-          vf_cur = vf_nxt;
-        }
-
-        // ---- dS' = scale * P' ⊙ (dP' - delta[q]) → overwrite P tile
-        {
-          const float dta = dta_lds[qb * 32 + ln];
-#pragma unroll
-          for (int jj = 0; jj < 4; ++jj) {
-            const int kv_loc = 8 * jj + 4 * half;
-            short4v dk4;
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-              const float ds = scale * p[jj * 4 + e] * (acc2[jj * 4 + e] - dta);
-              dk4[e] = (short)f2bf(ds);
-            }
-            *reinterpret_cast<short4v*>(P + sub_off<32>(ln, kv_loc)) = dk4;
-          }
-        }
-
-        // ---- dK += dS' · Q   (A = dS' tr-read, B = Q column-fragments)
-        {
-          constexpr int NB = D / 32;
-          bf16x8_t dsa_cur = ld_frag_tr<32>(P, lane, 0, 0);
-          bf16x8_t qtb_cur = ld_frag_tr<QB>(Qlds, lane, qb * 32, 0);
-          bf16x8_t dsa_nxt, qtb_nxt;
-#pragma unroll
-        for (int ks2 = 0; ks2 < 2; ++ks2) {
-#pragma unroll
-          for (int nb = 0; nb < NB; ++nb) {
-            if (nb + 1 < NB) {
-              qtb_nxt = ld_frag_tr<QB>(Qlds, lane, qb * 32 + ks2 * 16, (nb + 1) * 2);
-            } else if (ks2 == 0) {
-              dsa_nxt = ld_frag_tr<32>(P, lane, 16, 0);
-              qtb_nxt = ld_frag_tr<QB>(Qlds, lane, qb * 32 + 16, 0);
-            }
-            __builtin_amdgcn_s_setprio(1);
-            dk_acc[nb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(dsa_cur, qtb_cur, dk_acc[nb], 0, 0, 0);
-            __builtin_amdgcn_s_setprio(0);
-            qtb_cur = qtb_nxt;
-            if (nb + 1 == NB) dsa_cur = dsa_nxt;
-          }
-        }
-        }
-      }  // qb halves
-      }  // active
-
-      __syncthreads();  // all waves done with this q-tile's LDS
-      if (has_next) {
-        if (VAR != 2) {
-          qstage.store_subtiled(Qlds);
-          dostage.store_subtiled(dOlds);
-        } else {
-          stage_direct<D, QB, NTB>(Qlds, q_base, qts, qt0 + QB, Seff);
-          stage_direct<D, QB, NTB>(dOlds, do_base, do_stride, qt0 + QB, Seff);
-        }
-        if (threadIdx.x < QB) {
-          const int qr = max(min(qt0 + QB + (int)threadIdx.x, Seff - 1), 0);
-          lse_lds[threadIdx.x] = lse_base[qr];
-          dta_lds[threadIdx.x] = dta_base[qr];
-        }
-      }
-      __syncthreads();
-    }
   }
 
-  // ---- epilogue: write dK, dV (each kv row owned by exactly one block).
-  // Padded rows accumulate nothing and are written as zeros.
+  // ---- epilogue: dK, dV of the rows of this tile. Padded rows get zeros.
   const int kv_lim = VARLEN ? Seff : Sk;
-  if (kvw >= kv_lim) return;
-  unsigned short* dk_base = VARLEN ? dK + seq0 * dkts + (long)hk * D : dK + (long)b * dkbs + (long)hk * D;
-  unsigned short* dv_base = VARLEN ? dV + seq0 * dkts + (long)hk * D : dV + (long)b * dkbs + (long)hk * D;
+  const long n_part = (VARLEN ? (long)Sk : (long)B * Sk) * Hkv * D;
 #pragma unroll
   for (int j = 0; j < 16; ++j) {
-    const int r = crow(j, half);
-    const int kv_abs = kvw + r;
-    if (kv_abs < kv_lim) {
+    const int kv_abs = kvw + crow(j, half);
+    if (kv_abs >= kv_lim) continue;
+    const bool live = kv_abs < SeffK;
+    if (GS > 1) {
+      const long row = VARLEN ? seq0 + kv_abs : (long)b * Sk + kv_abs;
+      float* pk = PART + (long)part * 2 * n_part + (row * Hkv + hk) * D + ln;
 #pragma unroll
-      for (int nb = 0; nb < D / 32; ++nb) {
-        dk_base[(long)kv_abs * dkts + nb * 32 + ln] = f2bf(dk_acc[nb][j]);
-        dv_base[(long)kv_abs * dkts + nb * 32 + ln] = f2bf(dv_acc[nb][j]);
+      for (int nb = 0; nb < NB; ++nb) {
+        pk[nb * 32] = live ? dk_acc[nb][j] * scale : 0.0f;
+        pk[n_part + nb * 32] = live ? dv_acc[nb][j] : 0.0f;
+      }
+    } else {
+      const long at = (VARLEN ? seq0 * dkts : (long)b * dkbs) + (long)hk * D + (long)kv_abs * dkts + ln;
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb) {
+        dK[at + nb * 32] = live ? f2bf(dk_acc[nb][j] * scale) : 0;
+        dV[at + nb * 32] = live ? f2bf(dv_acc[nb][j]) : 0;
       }
     }
   }
 }
 
-// ===================================================== backward dQ kernel
-//
-// grid: (ceil(S/128) q-tiles, B*Hq). Each wave owns 32 q rows; kv tiles of
-// 64 staged subtiled in LDS (K serves both row-slice and column fragments,
-// V row-slice only). dS restages through a per-wave [kv 32][q 32] tile.
-// __launch_bounds__ min-waves/SIMD = 2 caps the allocation at 256 registers:
-// with the tr-read design the kernel fits (vs 441 before), doubling occupancy.
-template <int D, bool VARLEN = false>
-__global__ __launch_bounds__(fa::NTB, 2) void fa_bwd_dq_kernel(
-    const unsigned short* __restrict__ Q,
-    const unsigned short* __restrict__ K,
-    const unsigned short* __restrict__ V,
-    const unsigned short* __restrict__ dO,
-    const float* __restrict__ LSE,
-    const float* __restrict__ DELTA,
-    unsigned short* __restrict__ dQ,
-    const int* __restrict__ CU,
-    const int* __restrict__ CUK,  // padded ring pieces: kv-side valid counts
+// A block of 4 waves owns 128 query rows, 32 a wave, and streams key/value tiles of 64 rows. K serves as
+// rows (scores) and as columns (dQ), V as rows.
+template <int D, bool VARLEN>
+DEV_INLINE void bwd_dq(
+    char* smem, int f, int nblocks,
+    const unsigned short* __restrict__ Q, const unsigned short* __restrict__ K,
+    const unsigned short* __restrict__ V, const unsigned short* __restrict__ dO,
+    const float* __restrict__ LSE, const float* __restrict__ DELTA, unsigned short* __restrict__ dQ,
+    const int* __restrict__ CU, const int* __restrict__ CUK,
     long qbs, long qts, long kbs, long kts, long dqbs, long dqts,
-    int B, int S, int Sk, int Hq, int Hkv, float scale, int causal) {
+    int tiles, int B, int S, int Sk, int Hq, int Hkv, float scale, int causal) {
   using namespace fa;
-  extern __shared__ char smem[];
-  constexpr int KB_BYTES = sub_bytes<KVB, D>();
-  constexpr int PB = sub_bytes<32, 32>();  // per-wave dS tile: [kv 32][q 32]
-  // single-buffered here: double-buffering (as in the forward) pushes the
-  // block past the 80 KB needed for 2 blocks/CU and measured -13%
-  char* Klds = smem;
-  char* Vlds = smem + KB_BYTES;
-  char* Pw = smem + 2 * KB_BYTES;  // + wave*PB
-  float* lse_lds = reinterpret_cast<float*>(smem + 2 * KB_BYTES + NWB * PB);
-  float* dta_lds = lse_lds + NWB * QW;
+  constexpr int TB = tile_bytes<KVB, D>();
+  constexpr int DSL = D / 16, NB = D / 32;
+  char* Kbuf = smem;           // [2] key tiles, [2] value tiles
+  char* Vbuf = smem + 2 * TB;
 
   const int lane = threadIdx.x & 63;
   const int w = threadIdx.x >> 6;
   const int half = lane >> 5;
   const int ln = lane & 31;
 
-  int swz_x, swz_y;
-  xcd_swizzle_xy(swz_x, swz_y);  // same-bh q tiles share an XCD's L2 (K/V stream reuse)
-  const int bh = swz_y;
-  const int b = bh / Hq, h = bh % Hq;
+  f = xcd_chunk(f, nblocks);
+  const int y = f / tiles;
+  if (y >= B * Hq) return;
+  const int tile = causal ? tiles - 1 - f % tiles : f % tiles;  // late tiles see the most keys
+  const int b = VARLEN ? y % B : y / Hq, h = VARLEN ? y / B : y % Hq;
   const int hk = h / (Hq / Hkv);
-  const int q0 = swz_x * (NWB * QW);
+  const int q0 = tile * (NWB * QW);
   const int qw = q0 + w * QW;
 
   long seq0 = 0;
@@ -865,180 +703,151 @@ __global__ __launch_bounds__(fa::NTB, 2) void fa_bwd_dq_kernel(
   const unsigned short* k_base = VARLEN ? K + seq0 * kts + (long)hk * D : K + (long)b * kbs + (long)hk * D;
   const unsigned short* v_base = VARLEN ? V + seq0 * kts + (long)hk * D : V + (long)b * kbs + (long)hk * D;
 
-  constexpr int DSL = D / 16;
-  char* P = Pw + w * PB;
-
-  // lse/delta for the block's q rows
-  {
-    const float* lse_base = VARLEN ? LSE + (long)h * S + seq0 : LSE + ((long)b * Hq + h) * S;
-    const float* dta_base = VARLEN ? DELTA + (long)h * S + seq0 : DELTA + ((long)b * Hq + h) * S;
-    for (int i = threadIdx.x; i < NWB * QW; i += NTB) {
-      const int qr = max(min(q0 + i, Seff - 1), 0);
-      lse_lds[i] = lse_base[qr];
-      dta_lds[i] = dta_base[qr];
-    }
-  }
-
-  // ---- Q, dO fragments (A-operands): lane row = q (ln), d cols
+  // ---- Q, dO fragments (B operands): lane column = q (ln), d = sl*16+half*8+[0..7]
   const int q_my = max(min(qw + ln, Seff - 1), 0);
-  bf16x8_t qa[DSL], doa[DSL];
+  bf16x8_t qf[DSL], dof[DSL];
   {
     const unsigned short* qp = q_base + (long)q_my * qts + half * 8;
     const unsigned short* dop = do_base + (long)q_my * do_stride + half * 8;
 #pragma unroll
     for (int sl = 0; sl < DSL; ++sl) {
-      qa[sl] = ld_g16(qp + sl * 16);
-      doa[sl] = ld_g16(dop + sl * 16);
+      qf[sl] = ld_g16(qp + sl * 16);
+      dof[sl] = ld_g16(dop + sl * 16);
     }
   }
+  // a row that counts nothing (padding, or no visible key) has an addend of -inf
+  const long stat = (VARLEN ? (long)h * S + seq0 : ((long)b * Hq + h) * S) + q_my;
+  const float lse = qw + ln < Seff ? LSE[stat] : -INFINITY;
+  const float addend = lse == -INFINITY ? -INFINITY : -lse * 1.44269504f;
+  const float ndelta = -DELTA[stat];
+  const float scale2 = scale * 1.44269504f;
 
-  f32x16 dq_acc[D / 32];
+  f32x16 dq_acc[NB];
 #pragma unroll
-  for (int nb = 0; nb < D / 32; ++nb)
+  for (int nb = 0; nb < NB; ++nb)
 #pragma unroll
     for (int j = 0; j < 16; ++j) dq_acc[nb][j] = 0.0f;
 
   const int kv_tiles_all = (SeffK + KVB - 1) / KVB;
-  const int kv_tiles = causal ? min(kv_tiles_all, (q0 + NWB * QW + KVB - 1) / KVB) : kv_tiles_all;
+  const int kv_tiles = q0 >= Seff ? 0 : (causal ? min(kv_tiles_all, (min(q0 + NWB * QW, Seff) + KVB - 1) / KVB) : kv_tiles_all);
 
   RegStage<D, KVB, NTB> kstage, vstage;
-  // SeffK == 0 blocks skip the tile loop; the clamped loads stay in-bounds
-  kstage.load(k_base, kts, 0, SeffK);
-  vstage.load(v_base, kts, 0, SeffK);
-  kstage.store_subtiled(Klds);
-  vstage.store_subtiled(Vlds);
+  if (kv_tiles > 0) {
+    kstage.load(k_base, kts, 0, SeffK);
+    vstage.load(v_base, kts, 0, SeffK);
+    kstage.store(Kbuf);
+    vstage.store(Vbuf);
+  }
   __syncthreads();
 
   for (int t = 0; t < kv_tiles; ++t) {
-    const int k0 = t * KVB;
-    const bool has_next = (t + 1 < kv_tiles);
-    if (has_next) {
+    const int k0 = t * KVB, buf = t & 1;
+    const bool more = t + 1 < kv_tiles;
+    if (more) {
       kstage.load(k_base, kts, k0 + KVB, SeffK);
       vstage.load(v_base, kts, k0 + KVB, SeffK);
     }
-    const bool active = !(causal && k0 > qw + QW - 1) && (qw < Seff);
-    if (active) {
-
-    // 32-kv halves: live score state is p[16]+dp[16] instead of [2][16].
+    const char* Klds = Kbuf + buf * TB;
+    const char* Vlds = Vbuf + buf * TB;
+    if (!(causal && k0 > qw + QW - 1) && qw < Seff) {
 #pragma unroll
-    for (int kb = 0; kb < 2; ++kb) {
-      // ---- S[q][kv] = Q · K^T and dP[q][kv] = dO · V^T (shared loop)
-      f32x16 acc, acc2;
+      for (int kb = 0; kb < KVB / 32; ++kb) {
+        // ---- S^T[kv][q] = K · Q^T and dP^T - delta = V · dO^T - delta: column = q (ln), row = kv
+        f32x16 s, dp;
 #pragma unroll
-      for (int j = 0; j < 16; ++j) { acc[j] = 0.0f; acc2[j] = 0.0f; }
-      // software-pipelined: slice sl+1's K/V row-slice reads issue under
-      // slice sl's MFMAs (same restructure as the forward, +10% there)
-      bf16x8_t kb_cur = ld_lds16(Klds, sub_off<KVB>(kb * 32 + ln, half * 8));
-      bf16x8_t vb_cur = ld_lds16(Vlds, sub_off<KVB>(kb * 32 + ln, half * 8));
-      bf16x8_t kb_nxt, vb_nxt;
+        for (int j = 0; j < 16; ++j) { s[j] = 0.0f; dp[j] = ndelta; }
+        __builtin_amdgcn_s_setprio(1);
 #pragma unroll
-      for (int sl = 0; sl < DSL; ++sl) {
-        if (sl + 1 < DSL) {
-          kb_nxt = ld_lds16(Klds, sub_off<KVB>(kb * 32 + ln, (sl + 1) * 16 + half * 8));
-          vb_nxt = ld_lds16(Vlds, sub_off<KVB>(kb * 32 + ln, (sl + 1) * 16 + half * 8));
+        for (int sl = 0; sl < DSL; ++sl) {
+          s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ld_lds16(Klds, tile_off<KVB>(kb * 32 + ln, sl * 16 + half * 8)), qf[sl], s, 0, 0, 0);
+          dp = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ld_lds16(Vlds, tile_off<KVB>(kb * 32 + ln, sl * 16 + half * 8)), dof[sl], dp, 0, 0, 0);
         }
-        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(qa[sl], kb_cur, acc, 0, 0, 0);
-        acc2 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(doa[sl], vb_cur, acc2, 0, 0, 0);
-        kb_cur = kb_nxt;
-        vb_cur = vb_nxt;
-      }
-
-      // ---- dS = scale * P ⊙ (dP - delta[q]) with P = exp(scale*s - lse[q]);
-      // C-regs j in a 4-group are 4 consecutive q rows → packed 8 B store
-      // into the per-wave [kv 32][q 32] subtiled tile.
-      // interior kb-halves (all q/k in range, below the diagonal) take a
-      // maskless dS loop — branching at loop level keeps each path's
-      // register footprint tight
-      const bool blk_full = (k0 + kb * 32 + 32 <= SeffK) && (qw + QW <= Seff) &&
-                            (!causal || k0 + kb * 32 + 31 <= qw);
-      if (blk_full) {
+        __builtin_amdgcn_s_setprio(0);
+        // ---- dS = exp(scale s - lse) (dP - delta), its scale waits for the epilogue
+        bf16x8_t dsa[2];
+        const int kb0 = k0 + kb * 32;
+        const bool edge = kb0 + 32 > SeffK || (causal && kb0 + 31 > qw);
 #pragma unroll
-        for (int jj = 0; jj < 4; ++jj) {
-          const int q_loc0 = 8 * jj + 4 * half;
-          short4v dk4;
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            const int r = q_loc0 + e;
-            const float pv = __builtin_amdgcn_exp2f(
-                fmaf(acc[jj * 4 + e], scale * 1.44269504f, -lse_lds[w * QW + r] * 1.44269504f));
-            const float ds = scale * pv * (acc2[jj * 4 + e] - dta_lds[w * QW + r]);
-            dk4[e] = (short)f2bf(ds);
+        for (int j = 0; j < 16; ++j) {
+          float pv = __builtin_amdgcn_exp2f(fmaf(s[j], scale2, addend));
+          if (edge) {
+            const int k_abs = kb0 + crow(j, half);
+            if (k_abs >= SeffK || (causal && k_abs > qw + ln)) pv = 0.0f;
           }
-          *reinterpret_cast<short4v*>(P + sub_off<32>(ln, q_loc0)) = dk4;
+          dsa[j >> 3][j & 7] = (__bf16)(pv * dp[j]);
         }
-      } else {
+        // ---- dQ += dS · K (A: lane row = q; B: columns of K)
+        __builtin_amdgcn_s_setprio(1);
 #pragma unroll
-      for (int jj = 0; jj < 4; ++jj) {
-        const int q_loc0 = 8 * jj + 4 * half;
-        short4v dk4;
+        for (int s2 = 0; s2 < 2; ++s2)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const int r = q_loc0 + e;
-          const int q_abs = qw + r;
-          const int k_abs = k0 + kb * 32 + ln;
-          const float lse = lse_lds[w * QW + r];
-          const float dta = dta_lds[w * QW + r];
-          const bool valid = (q_abs < Seff) && (k_abs < SeffK) && (!causal || k_abs <= q_abs) && (lse != -INFINITY);
-          const float pv = valid
-              ? __builtin_amdgcn_exp2f(fmaf(acc[jj * 4 + e], scale * 1.44269504f, -lse * 1.44269504f))
-              : 0.0f;
-          const float ds = scale * pv * (acc2[jj * 4 + e] - dta);
-          dk4[e] = (short)f2bf(ds);
-        }
-        *reinterpret_cast<short4v*>(P + sub_off<32>(ln, q_loc0)) = dk4;
+          for (int nb = 0; nb < NB; ++nb)
+            dq_acc[nb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(dsa[s2], frag_born<KVB>(Klds, lane, kb * 32 + s2 * 16, nb * 2), dq_acc[nb], 0, 0, 0);
+        __builtin_amdgcn_s_setprio(0);
       }
-      }
-
-      // ---- dQ += dS · K   (A = dS tr-read: lane row = q, k = kv-local;
-      //      B = K column-fragments, k = kv-global)
-      {
-        constexpr int NB = D / 32;
-        bf16x8_t dsa_cur = ld_frag_tr<32>(P, lane, 0, 0);
-        bf16x8_t ktb_cur = ld_frag_tr<KVB>(Klds, lane, kb * 32, 0);
-        bf16x8_t dsa_nxt, ktb_nxt;
-#pragma unroll
-        for (int ks2 = 0; ks2 < 2; ++ks2) {
-#pragma unroll
-          for (int nb = 0; nb < NB; ++nb) {
-            if (nb + 1 < NB) {
-              ktb_nxt = ld_frag_tr<KVB>(Klds, lane, kb * 32 + ks2 * 16, (nb + 1) * 2);
-            } else if (ks2 == 0) {
-              dsa_nxt = ld_frag_tr<32>(P, lane, 16, 0);
-              ktb_nxt = ld_frag_tr<KVB>(Klds, lane, kb * 32 + 16, 0);
-            }
-            __builtin_amdgcn_s_setprio(1);
-            dq_acc[nb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(dsa_cur, ktb_cur, dq_acc[nb], 0, 0, 0);
-            __builtin_amdgcn_s_setprio(0);
-            ktb_cur = ktb_nxt;
-            if (nb + 1 == NB) dsa_cur = dsa_nxt;
-          }
-        }
-      }
-    }  // kb halves
-    }  // active
-
-    __syncthreads();
-    if (has_next) {
-      kstage.store_subtiled(Klds);
-      vstage.store_subtiled(Vlds);
+    }
+    if (more) {
+      kstage.store(Kbuf + (buf ^ 1) * TB);
+      vstage.store(Vbuf + (buf ^ 1) * TB);
     }
     __syncthreads();
   }
 
   // ---- epilogue: write dQ (pad rows accumulate nothing -> zeros)
   const int q_lim = VARLEN ? Seff : S;
-  if (qw >= q_lim) return;
   unsigned short* dq_base = VARLEN ? dQ + seq0 * dqts + (long)h * D : dQ + (long)b * dqbs + (long)h * D;
 #pragma unroll
   for (int j = 0; j < 16; ++j) {
-    const int r = crow(j, half);
-    const int q_abs = qw + r;
-    if (q_abs < q_lim) {
+    const int q_abs = qw + crow(j, half);
+    if (q_abs >= q_lim) continue;
 #pragma unroll
-      for (int nb = 0; nb < D / 32; ++nb) {
-        dq_base[(long)q_abs * dqts + nb * 32 + ln] = f2bf(dq_acc[nb][j]);
-      }
-    }
+    for (int nb = 0; nb < NB; ++nb) dq_base[(long)q_abs * dqts + nb * 32 + ln] = f2bf(dq_acc[nb][j] * scale);
+  }
+}
+
+template <int D>
+constexpr size_t bwd_lds() {
+  using namespace fa;
+  const size_t kv = tile_bytes<NWB * QW, D>() + 4 * tile_bytes<32, D>() + 4 * 32 * sizeof(float);
+  const size_t q = 4 * tile_bytes<KVB, D>();
+  return kv > q ? kv : q;
+}
+
+template <int D, bool VARLEN>
+__global__ __launch_bounds__(fa::NTB, 2) void fa_bwd_kernel(
+    const unsigned short* __restrict__ Q, const unsigned short* __restrict__ K,
+    const unsigned short* __restrict__ V, const unsigned short* __restrict__ dO,
+    const float* __restrict__ LSE, const float* __restrict__ DELTA,
+    unsigned short* __restrict__ dQ, unsigned short* __restrict__ dK, unsigned short* __restrict__ dV,
+    float* __restrict__ PART, int GS, const int* __restrict__ CU, const int* __restrict__ CUK,
+    long qbs, long qts, long kbs, long kts, long dqbs, long dqts, long dkbs, long dkts,
+    int n_kv, int kv_tiles, int q_tiles, int B, int S, int Sk, int Hq, int Hkv, float scale, int causal) {
+  extern __shared__ char smem[];
+  const int f = (int)blockIdx.x;
+  if (f < n_kv)
+    bwd_dkdv<D, VARLEN>(smem, f, n_kv, Q, K, V, dO, LSE, DELTA, dK, dV, PART, GS, CU, CUK, qbs, qts, kbs, kts, dkbs, dkts,
+                        kv_tiles, B, S, Sk, Hq, Hkv, scale, causal);
+  else
+    bwd_dq<D, VARLEN>(smem, f - n_kv, (int)gridDim.x - n_kv, Q, K, V, dO, LSE, DELTA, dQ, CU, CUK, qbs, qts, kbs, kts,
+                      dqbs, dqts, q_tiles, B, S, Sk, Hq, Hkv, scale, causal);
+}
+
+// dK and dV from the float32 sums of the GS blocks that shared a tile's heads: four channels a thread.
+__global__ __launch_bounds__(256) void fa_bwd_sum_kernel(unsigned short* __restrict__ dK, unsigned short* __restrict__ dV,
+                                                         const float* __restrict__ PART, int GS, long n_part, int Sk,
+                                                         int HD, long dkbs, long dkts) {
+  const long i = ((long)blockIdx.x * 256 + threadIdx.x) * 4;
+  if (i >= n_part) return;
+  const long row = i / HD;
+  const long at = row / Sk * dkbs + row % Sk * dkts + i % HD;
+#pragma unroll
+  for (int which = 0; which < 2; ++which) {
+    float4v sum = {0.0f, 0.0f, 0.0f, 0.0f};
+    for (int p = 0; p < GS; ++p) sum += *reinterpret_cast<const float4v*>(PART + (2L * p + which) * n_part + i);
+    short4v o;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) o[e] = (short)f2bf(sum[e]);
+    *reinterpret_cast<short4v*>((which ? dV : dK) + at) = o;
   }
 }
 
@@ -1051,6 +860,12 @@ void set_lds_limit(const void* kernel, size_t bytes) {
     (void)hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
   }
 }
+
+// Waves (of 32 query rows) of a forward block. Four: two blocks share a CU, and their barriers do not
+// hold each other up (8 waves in one block: 735 against 809 TFLOP/s at B4 S4096 H32 D128 causal). Two when blocks
+// of four would leave CUs empty (B2 S256 H4 D128: 10.3 against 12.4 us; B8 S197 H12 D64: 10.2 against 10.6); twice
+// the reads of K and V make them slower as soon as the chip is full (4096: 507 TFLOP/s).
+int fwd_waves(int S, long rows) { return (S + 4 * fa::QW - 1) / (4 * fa::QW) * rows < 256 ? 2 : 4; }
 
 // q/k/v are [B,S,H,D] views that may be strided in dims 0/1 (e.g. views into
 // a packed QKV GEMM output); dims 2/3 must be dense.
@@ -1099,22 +914,23 @@ std::vector<at::Tensor> flash_attn_fwd(at::Tensor q, at::Tensor k, at::Tensor v,
   auto o = at::empty({B, S, Hq, D}, q.options());
   auto lse = at::empty({B, Hq, S}, q.options().dtype(at::kFloat));
   auto stream = at::hip::getCurrentHIPStream();
-  const dim3 grid((S + NW * QW - 1) / (NW * QW), B * Hq);
   const long qbs = q.stride(0), qts = q.stride(1), kbs = k.stride(0), kts = k.stride(1);
 
-#define LAUNCH_FWD(DD)                                                                            \
+#define LAUNCH_FWD(DD, NW)                                                                            \
   do {                                                                                            \
-    const size_t lds = 4 * sub_bytes<KVB, DD>() + NW * (QW * KVB * 2);                            \
-    set_lds_limit((const void*)fa_fwd_kernel<DD, false>, lds);                                    \
-    hipLaunchKernelGGL((fa_fwd_kernel<DD, false>), grid, dim3(NT), lds, stream.stream(),          \
+    const size_t lds = 4 * tile_bytes<KVB, DD>();                                                  \
+    set_lds_limit((const void*)fa_fwd_kernel<DD, NW, false>, lds);                                \
+    hipLaunchKernelGGL((fa_fwd_kernel<DD, NW, false>), dim3((S + NW * QW - 1) / (NW * QW), B * Hq), \
+                       dim3(NW * 64), lds, stream.stream(),                                       \
                        (const unsigned short*)q.data_ptr(), (const unsigned short*)k.data_ptr(),  \
                        (const unsigned short*)v.data_ptr(), (unsigned short*)o.data_ptr(),        \
                        lse.data_ptr<float>(), cu, cuk, qbs, qts, kbs, kts,                        \
                        B, S, Sk, Hq, Hkv, (float)scale, causal ? 1 : 0);                              \
   } while (0)
 
-  if (D == 128) LAUNCH_FWD(128);
-  else LAUNCH_FWD(64);
+  const int nw = fwd_waves(S, (long)B * Hq);
+  if (D == 128) { if (nw == 4) LAUNCH_FWD(128, 4); else LAUNCH_FWD(128, 2); }
+  else { if (nw == 4) LAUNCH_FWD(64, 4); else LAUNCH_FWD(64, 2); }
 #undef LAUNCH_FWD
   HIP_CHECK_LAST();
   return {o, lse};
@@ -1138,14 +954,14 @@ std::vector<at::Tensor> flash_attn_varlen_fwd(at::Tensor q, at::Tensor k, at::Te
   auto o = at::empty({T, Hq, D}, q.options());
   auto lse = at::empty({Hq, T}, q.options().dtype(at::kFloat));
   auto stream = at::hip::getCurrentHIPStream();
-  const dim3 grid(((int)max_seqlen + NW * QW - 1) / (NW * QW), n_seq * Hq);
   const long qts = q.stride(0), kts = k.stride(0);
 
-#define LAUNCH_VFWD(DD)                                                                           \
+#define LAUNCH_VFWD(DD, NW)                                                                           \
   do {                                                                                            \
-    const size_t lds = 4 * sub_bytes<KVB, DD>() + NW * (QW * KVB * 2);                            \
-    set_lds_limit((const void*)fa_fwd_kernel<DD, true>, lds);                                     \
-    hipLaunchKernelGGL((fa_fwd_kernel<DD, true>), grid, dim3(NT), lds, stream.stream(),           \
+    const size_t lds = 4 * tile_bytes<KVB, DD>();                                                  \
+    set_lds_limit((const void*)fa_fwd_kernel<DD, NW, true>, lds);                                 \
+    hipLaunchKernelGGL((fa_fwd_kernel<DD, NW, true>),                                             \
+                       dim3(((int)max_seqlen + NW * QW - 1) / (NW * QW), n_seq * Hq), dim3(NW * 64), lds, stream.stream(), \
                        (const unsigned short*)q.data_ptr(), (const unsigned short*)k.data_ptr(),  \
                        (const unsigned short*)v.data_ptr(), (unsigned short*)o.data_ptr(),        \
                        lse.data_ptr<float>(), cu_seqlens.data_ptr<int>(), nullptr,                \
@@ -1153,8 +969,9 @@ std::vector<at::Tensor> flash_attn_varlen_fwd(at::Tensor q, at::Tensor k, at::Te
                        n_seq, T, T, Hq, Hkv, (float)scale, causal ? 1 : 0);                          \
   } while (0)
 
-  if (D == 128) LAUNCH_VFWD(128);
-  else LAUNCH_VFWD(64);
+  const int nw = fwd_waves((int)max_seqlen, (long)n_seq * Hq);
+  if (D == 128) { if (nw == 4) LAUNCH_VFWD(128, 4); else LAUNCH_VFWD(128, 2); }
+  else { if (nw == 4) LAUNCH_VFWD(64, 4); else LAUNCH_VFWD(64, 2); }
 #undef LAUNCH_VFWD
   HIP_CHECK_LAST();
   return {o, lse};
@@ -1162,27 +979,47 @@ std::vector<at::Tensor> flash_attn_varlen_fwd(at::Tensor q, at::Tensor k, at::Te
 
 namespace {
 
-hipStream_t bwd_side_stream(hipEvent_t* fork, hipEvent_t* join) {
-  static hipStream_t side_stream = nullptr;
-  static hipEvent_t ev_fork = nullptr, ev_join = nullptr;
-  if (side_stream == nullptr) {
-    (void)hipStreamCreateWithFlags(&side_stream, hipStreamNonBlocking);
-    (void)hipEventCreateWithFlags(&ev_fork, hipEventDisableTiming);
-    (void)hipEventCreateWithFlags(&ev_join, hipEventDisableTiming);
+// The backward launch of dense (VARLEN = false) and packed batches. `seqs` sequences of at most S_max queries and
+// Sk_max keys; S, Sk are the extents the kernels index with (tokens of the whole batch when packed).
+template <int D, bool VARLEN>
+void launch_bwd(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, const at::Tensor& dout, const at::Tensor& lse,
+                const at::Tensor& delta, at::Tensor& dq, at::Tensor& dk, at::Tensor& dv, const int* cu, const int* cuk,
+                long qbs, long qts, long kbs, long kts, long dqbs, long dqts, long dkbs, long dkts, int seqs, int S_max,
+                int Sk_max, int S, int Sk, int Hq, int Hkv, float scale, bool causal, hipStream_t stream) {
+  using namespace fa;
+  const int rows = NWB * QW;
+  const int kv_tiles = (Sk_max + rows - 1) / rows, q_tiles = (S_max + rows - 1) / rows;
+  const int G = Hq / Hkv;
+  // Blocks that share a tile's group of heads. All 512 blocks that fit on the chip at once start together, and
+  // under a causal mask the first tile then takes twice the average: B1 S8192, 32 over 8 heads, runs 2194 us with one
+  // block a tile (512 blocks), 2077 with two and 2110 with four (more partial sums). Without a mask the work is even
+  // and it only matters that every CU has a block. A block keeps at least 16 steps, or the sums cost more than
+  // they save.
+  const long kv_blocks = (VARLEN ? (Sk + rows - 1) / rows : (long)kv_tiles * seqs) * Hkv;
+  const bool sums_ok = dk.stride(-3) % 4 == 0 && (VARLEN || dk.stride(0) % 4 == 0) &&
+                       reinterpret_cast<uintptr_t>(dk.data_ptr()) % 8 == 0 && reinterpret_cast<uintptr_t>(dv.data_ptr()) % 8 == 0;
+  int gs = 1;
+  for (int d = 2; d <= G && sums_ok && kv_blocks * gs <= (causal ? 512 : 255); ++d)
+    if (G % d == 0 && (long)((S_max + 31) / 32) * (G / d) >= 16) gs = d;
+  const long n_part = (VARLEN ? (long)Sk : (long)seqs * Sk) * Hkv * D;
+  at::Tensor part;
+  if (gs > 1) part = at::empty({gs * 2 * n_part}, q.options().dtype(at::kFloat));
+  const int n_kv = (kv_tiles * seqs * Hkv * gs + 7) / 8 * 8, n_q = q_tiles * seqs * Hq;
+  auto kernel = fa_bwd_kernel<D, VARLEN>;
+  set_lds_limit((const void*)kernel, bwd_lds<D>());
+  hipLaunchKernelGGL(kernel, dim3(n_kv + n_q), dim3(NTB), bwd_lds<D>(), stream,
+                     (const unsigned short*)q.data_ptr(), (const unsigned short*)k.data_ptr(),
+                     (const unsigned short*)v.data_ptr(), (const unsigned short*)dout.data_ptr(), lse.data_ptr<float>(),
+                     delta.data_ptr<float>(), (unsigned short*)dq.data_ptr(), (unsigned short*)dk.data_ptr(),
+                     (unsigned short*)dv.data_ptr(), gs > 1 ? part.data_ptr<float>() : nullptr, gs, cu, cuk, qbs, qts, kbs,
+                     kts, dqbs, dqts, dkbs, dkts, n_kv, kv_tiles, q_tiles, seqs, S, Sk, Hq, Hkv, scale, causal ? 1 : 0);
+  HIP_CHECK_LAST();
+  if (gs > 1) {
+    hipLaunchKernelGGL(fa_bwd_sum_kernel, dim3((unsigned)((n_part / 4 + 255) / 256)), dim3(256), 0, stream,
+                       (unsigned short*)dk.data_ptr(), (unsigned short*)dv.data_ptr(), part.data_ptr<float>(), gs, n_part, Sk,
+                       Hkv * D, dkbs, dkts);
+    HIP_CHECK_LAST();
   }
-  *fork = ev_fork;
-  *join = ev_join;
-  return side_stream;
-}
-
-int dkdv_variant() {
-  // dkdv occupancy-variant experiment switch (docs/KERNELS.md)
-  static int dkdv_var = -1;
-  if (dkdv_var < 0) {
-    const char* e = getenv("CAI_FA_DKDV_VAR");
-    dkdv_var = e ? atoi(e) : 2;
-  }
-  return dkdv_var;
 }
 
 }  // namespace
@@ -1233,59 +1070,13 @@ std::vector<at::Tensor> flash_attn_bwd(at::Tensor dout, at::Tensor q, at::Tensor
     HIP_CHECK_LAST();
   }
 
-  const dim3 grid_kv((Sk + NWB * QW - 1) / (NWB * QW), B * Hkv);
-  const dim3 grid_q((S + NWB * QW - 1) / (NWB * QW), B * Hq);
-  const long qbs = q.stride(0), qts = q.stride(1), kbs = k.stride(0), kts = k.stride(1);
-  const long dqbs = dq.stride(0), dqts = dq.stride(1), dkbs = dk.stride(0), dkts = dk.stride(1);
-
-  // dK/dV and dQ are independent: run them on two streams so the two
-  // latency-bound kernels co-occupy the CUs.
-  hipEvent_t ev_fork, ev_join;
-  hipStream_t side_stream = bwd_side_stream(&ev_fork, &ev_join);
-  (void)hipEventRecord(ev_fork, stream.stream());
-  (void)hipStreamWaitEvent(side_stream, ev_fork, 0);
-  const int dkdv_var = dkdv_variant();
-
-#define LAUNCH_BWD(DD)                                                                              \
-  do {                                                                                              \
-    constexpr int QB = 64;                                                                          \
-    const size_t lds_kv = 2 * sub_bytes<QB, DD>() + NWB * sub_bytes<32, 32>()                       \
-                          + 2 * QB * sizeof(float);                                                 \
-    const void* dkdv_fn = dkdv_var == 0 ? (const void*)fa_bwd_dkdv_kernel<DD, 0>                    \
-                        : dkdv_var == 1 ? (const void*)fa_bwd_dkdv_kernel<DD, 1>                    \
-                        : dkdv_var == 3 ? (const void*)fa_bwd_dkdv_kernel<DD, 3>                    \
-                                        : (const void*)fa_bwd_dkdv_kernel<DD, 2>;                   \
-    set_lds_limit(dkdv_fn, lds_kv);                                                                 \
-    hipLaunchKernelGGL((dkdv_var == 0 ? fa_bwd_dkdv_kernel<DD, 0>                                   \
-                        : dkdv_var == 1 ? fa_bwd_dkdv_kernel<DD, 1>                                 \
-                        : dkdv_var == 3 ? fa_bwd_dkdv_kernel<DD, 3>                                 \
-                                        : fa_bwd_dkdv_kernel<DD, 2>),                               \
-                       grid_kv, dim3(NTB), lds_kv, stream.stream(),                                 \
-                       (const unsigned short*)q.data_ptr(), (const unsigned short*)k.data_ptr(),    \
-                       (const unsigned short*)v.data_ptr(), (const unsigned short*)dout.data_ptr(), \
-                       lse.data_ptr<float>(), delta.data_ptr<float>(),                              \
-                       (unsigned short*)dk.data_ptr(), (unsigned short*)dv.data_ptr(),              \
-                       cu, cuk, qbs, qts, kbs, kts, dkbs, dkts,                                    \
-                       B, S, Sk, Hq, Hkv, (float)scale, causal ? 1 : 0);                            \
-    HIP_CHECK_LAST();                                                                               \
-    const size_t lds_q = 2 * sub_bytes<KVB, DD>() + NWB * sub_bytes<32, 32>()                       \
-                         + 2 * NWB * QW * sizeof(float);                                            \
-    set_lds_limit((const void*)fa_bwd_dq_kernel<DD>, lds_q);                                        \
-    hipLaunchKernelGGL((fa_bwd_dq_kernel<DD>), grid_q, dim3(NTB), lds_q, side_stream,               \
-                       (const unsigned short*)q.data_ptr(), (const unsigned short*)k.data_ptr(),    \
-                       (const unsigned short*)v.data_ptr(), (const unsigned short*)dout.data_ptr(), \
-                       lse.data_ptr<float>(), delta.data_ptr<float>(),                              \
-                       (unsigned short*)dq.data_ptr(),                                              \
-                       cu, cuk, qbs, qts, kbs, kts, dqbs, dqts,                                    \
-                       B, S, Sk, Hq, Hkv, (float)scale, causal ? 1 : 0);                            \
-    HIP_CHECK_LAST();                                                                               \
-  } while (0)
-
+#define LAUNCH_BWD(DD)                                                                                               \
+  launch_bwd<DD, false>(q, k, v, dout, lse, delta, dq, dk, dv, cu, cuk, q.stride(0), q.stride(1), k.stride(0), k.stride(1), \
+                        dq.stride(0), dq.stride(1), dk.stride(0), dk.stride(1), B, S, Sk, S, Sk, Hq, Hkv, (float)scale,      \
+                        causal, stream.stream())
   if (D == 128) LAUNCH_BWD(128);
   else LAUNCH_BWD(64);
 #undef LAUNCH_BWD
-  (void)hipEventRecord(ev_join, side_stream);
-  (void)hipStreamWaitEvent(stream.stream(), ev_join, 0);
   return {dq, dk, dv};
 }
 
@@ -1313,50 +1104,13 @@ std::vector<at::Tensor> flash_attn_varlen_bwd(at::Tensor dout, at::Tensor q, at:
     HIP_CHECK_LAST();
   }
 
-  const dim3 grid_kv(((int)max_seqlen + NWB * QW - 1) / (NWB * QW), n_seq * Hkv);
-  const dim3 grid_q(((int)max_seqlen + NWB * QW - 1) / (NWB * QW), n_seq * Hq);
-  const long qts = q.stride(0), kts = k.stride(0);
-  const long dqts = dq.stride(0), dkts = dk.stride(0);
-  const int* cu = cu_seqlens.data_ptr<int>();
-
-  hipEvent_t ev_fork, ev_join;
-  hipStream_t side_stream = bwd_side_stream(&ev_fork, &ev_join);
-  (void)hipEventRecord(ev_fork, stream.stream());
-  (void)hipStreamWaitEvent(side_stream, ev_fork, 0);
-
-#define LAUNCH_VBWD(DD)                                                                             \
-  do {                                                                                              \
-    constexpr int QB = 64;                                                                          \
-    const size_t lds_kv = 2 * sub_bytes<QB, DD>() + NWB * sub_bytes<32, 32>()                       \
-                          + 2 * QB * sizeof(float);                                                 \
-    set_lds_limit((const void*)fa_bwd_dkdv_kernel<DD, 2, true>, lds_kv);                            \
-    hipLaunchKernelGGL((fa_bwd_dkdv_kernel<DD, 2, true>), grid_kv, dim3(NTB), lds_kv,               \
-                       stream.stream(),                                                             \
-                       (const unsigned short*)q.data_ptr(), (const unsigned short*)k.data_ptr(),    \
-                       (const unsigned short*)v.data_ptr(), (const unsigned short*)dout.data_ptr(), \
-                       lse.data_ptr<float>(), delta.data_ptr<float>(),                              \
-                       (unsigned short*)dk.data_ptr(), (unsigned short*)dv.data_ptr(),              \
-                       cu, nullptr, 0L, qts, 0L, kts, 0L, dkts,                                              \
-                       n_seq, T, T, Hq, Hkv, (float)scale, causal ? 1 : 0);                            \
-    HIP_CHECK_LAST();                                                                               \
-    const size_t lds_q = 2 * sub_bytes<KVB, DD>() + NWB * sub_bytes<32, 32>()                       \
-                         + 2 * NWB * QW * sizeof(float);                                            \
-    set_lds_limit((const void*)fa_bwd_dq_kernel<DD, true>, lds_q);                                  \
-    hipLaunchKernelGGL((fa_bwd_dq_kernel<DD, true>), grid_q, dim3(NTB), lds_q, side_stream,         \
-                       (const unsigned short*)q.data_ptr(), (const unsigned short*)k.data_ptr(),    \
-                       (const unsigned short*)v.data_ptr(), (const unsigned short*)dout.data_ptr(), \
-                       lse.data_ptr<float>(), delta.data_ptr<float>(),                              \
-                       (unsigned short*)dq.data_ptr(),                                              \
-                       cu, nullptr, 0L, qts, 0L, kts, 0L, dqts,                                              \
-                       n_seq, T, T, Hq, Hkv, (float)scale, causal ? 1 : 0);                            \
-    HIP_CHECK_LAST();                                                                               \
-  } while (0)
-
+#define LAUNCH_VBWD(DD)                                                                                              \
+  launch_bwd<DD, true>(q, k, v, dout, lse, delta, dq, dk, dv, cu_seqlens.data_ptr<int>(), nullptr, 0L, q.stride(0), 0L,     \
+                       k.stride(0), 0L, dq.stride(0), 0L, dk.stride(0), n_seq, (int)max_seqlen, (int)max_seqlen, T, T, Hq,  \
+                       Hkv, (float)scale, causal, stream.stream())
   if (D == 128) LAUNCH_VBWD(128);
   else LAUNCH_VBWD(64);
 #undef LAUNCH_VBWD
-  (void)hipEventRecord(ev_join, side_stream);
-  (void)hipStreamWaitEvent(stream.stream(), ev_join, 0);
   return {dq, dk, dv};
 }
 

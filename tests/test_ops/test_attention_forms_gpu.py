@@ -1,0 +1,128 @@
+"""Flash attention where its launch takes another form: forward blocks of two and four waves, tile remainders,
+key/value tiles whose heads several backward blocks share (float32 sums), strided outputs, a negative scale.
+
+The bound: outputs and gradients are rounded to bfloat16 (at most 2^-9 of a value) after products of operands
+that were rounded once themselves (probabilities or their gradients), so the 2-norm of the error is below
+3 * 2^-9 of the result's."""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+BOUND = 3 * 2.0 ** -9
+
+
+def _near(got, want, what, lone=False):
+    if lone and what in ("dq", "dk"):
+        # a softmax over one key is constant: these vanish but for dout · v and dout · out, both about sqrt(D), being
+        # rounded to bfloat16 apart
+        assert got.float().abs().max() < 2.0 ** -7 * got.shape[-1] ** 0.5, what
+        return
+    err = (got.double() - want.double()).norm() / want.double().norm().clamp_min(1e-20)
+    assert err < BOUND, f"{what}: {err:.2e}"
+
+
+def _reference(q, k, v, dout, causal, scale):
+    """Float32 outputs and gradients, one head at a time."""
+    B, S, H, D = q.shape
+    G = k.shape[2]
+    q, k, v, dout = (t.float() for t in (q, k, v, dout))
+    out, dq, dk, dv = torch.zeros_like(q), torch.zeros_like(q), torch.zeros_like(k), torch.zeros_like(v)
+    hidden = torch.ones(S, k.shape[1], dtype=torch.bool, device=q.device).triu(1) if causal else None
+    for b in range(B):
+        for h in range(H):
+            g = h // (H // G)
+            s = (q[b, :, h] @ k[b, :, g].t()) * scale
+            if causal:
+                s = s.masked_fill(hidden, float("-inf"))
+            p = torch.softmax(s, 1)
+            out[b, :, h] = p @ v[b, :, g]
+            ds = p * (dout[b, :, h] @ v[b, :, g].t() - (dout[b, :, h] * out[b, :, h]).sum(1, keepdim=True)) * scale
+            dq[b, :, h] = ds @ k[b, :, g]
+            dk[b, :, g] += ds.t() @ q[b, :, h]
+            dv[b, :, g] += p.t() @ dout[b, :, h]
+    return out, dq, dk, dv
+
+
+def _inputs(B, S, H, G, D, seed=0):
+    torch.manual_seed(seed)
+    return [torch.randn(B, S, h, D, device="cuda").bfloat16() for h in (H, G, G, H)]
+
+
+@pytest.mark.parametrize("B,S,H,G,D,causal,scale", [
+    (1, 1, 2, 1, 128, True, None),
+    (2, 31, 4, 4, 64, True, None),
+    (1, 33, 4, 2, 128, False, None),
+    (3, 129, 12, 12, 64, False, None),      # remainder rows of a block of four waves, small grid
+    (4, 300, 32, 32, 128, True, None),      # blocks of four waves
+    (1, 512, 8, 2, 128, True, None),        # four blocks share a tile's heads
+    (1, 520, 6, 2, 64, True, None),         # three do
+    (2, 640, 4, 1, 64, False, None),        # without a mask, too few blocks for the CUs
+    (1, 200, 4, 2, 64, True, -0.2),
+    (1, 130, 2, 2, 128, False, -0.1),
+])
+def test_dense(B, S, H, G, D, causal, scale):
+    from colossalai_amd.ops import flash_attention
+
+    q, k, v, dout = _inputs(B, S, H, G, D)
+    want = _reference(q, k, v, dout, causal, D ** -0.5 if scale is None else scale)
+    for t in (q, k, v):
+        t.requires_grad_()
+    out = flash_attention(q, k, v, causal=causal, scale=scale)
+    got = (out, *torch.autograd.grad(out, (q, k, v), dout))
+    for name, a, b in zip(("out", "dq", "dk", "dv"), got, want):
+        _near(a, b, name, lone=S == 1)
+
+
+def test_padded_rows_with_shared_heads():
+    from colossalai_amd.ops import flash_attention
+
+    q, k, v, dout = _inputs(2, 512, 8, 2, 128)
+    lens = [512, 333]
+    for t in (q, k, v):
+        t.requires_grad_()
+    out = flash_attention(q, k, v, causal=True, seqlens=torch.tensor(lens, dtype=torch.int32, device="cuda"))
+    got = (out, *torch.autograd.grad(out, (q, k, v), dout))
+    for b, n in enumerate(lens):
+        want = _reference(*(t[b: b + 1, :n].detach() for t in (q, k, v, dout)), True, 128 ** -0.5)
+        for name, a, w in zip(("out", "dq", "dk", "dv"), got, want):
+            _near(a[b: b + 1, :n], w, name)
+            assert (a[b, n:] == 0).all(), name
+
+
+@pytest.mark.parametrize("lens,H,G,D", [([512, 1, 0, 300], 4, 2, 128), ([700], 8, 2, 64), ([64, 128, 129, 31], 2, 2, 64)])
+def test_packed(lens, H, G, D):
+    from colossalai_amd.ops import flash_attention_varlen
+
+    total = sum(lens)
+    q, k, v, dout = (t[0] for t in _inputs(1, total, H, G, D))
+    cu = torch.tensor([0] + lens).cumsum(0).int().cuda()
+    for t in (q, k, v):
+        t.requires_grad_()
+    out = flash_attention_varlen(q, k, v, cu, max(lens), causal=True)
+    got = (out, *torch.autograd.grad(out, (q, k, v), dout))
+    at = 0
+    for n in lens:
+        if n:
+            want = _reference(*(t[None, at: at + n].detach() for t in (q, k, v, dout)), True, D ** -0.5)
+            for name, a, w in zip(("out", "dq", "dk", "dv"), got, want):
+                _near(a[None, at: at + n], w, name, lone=n == 1)
+        at += n
+
+
+def test_strided_gradients_with_shared_heads():
+    """dk/dv as views into one packed buffer, filled by the kernel that adds the partial sums."""
+    from colossalai_amd.ops import kernels
+
+    B, S, H, G, D = 1, 512, 8, 2, 64
+    q, k, v, dout = _inputs(B, S, H, G, D)
+    want = _reference(q, k, v, dout, True, D ** -0.5)
+    packed = torch.full((B, S, (H + 2 * G) * D), float("nan"), dtype=torch.bfloat16, device="cuda")
+    dq = packed[:, :, : H * D].view(B, S, H, D)
+    dk = packed[:, :, H * D: (H + G) * D].view(B, S, G, D)
+    dv = packed[:, :, (H + G) * D:].view(B, S, G, D)
+    out, lse = kernels().flash_attn_fwd(q, k, v, True, D ** -0.5)
+    kernels().flash_attn_bwd(dout, q, k, v, out, lse, True, D ** -0.5, dq, dk, dv)
+    for name, a, b in zip(("out", "dq", "dk", "dv"), (out, dq, dk, dv), want):
+        _near(a, b, name)
