@@ -26,6 +26,8 @@ namespace serving {
 
 constexpr int ATT_WAVES = 16;  // most waves of a block: they split the key blocks of one (token, kv head)
 constexpr int RC_MAX = 4;      // most query heads of a kv head's group that one block handles together
+typedef __bf16 bf16x2_v __attribute__((ext_vector_type(2)));
+
 constexpr int MFMA_TILES_PER_STEP = 2;  // 32-key tiles the matrix-core kernel stages and multiplies between two barriers
 
 // sum over the 8 adjacent lanes that share a key (quad xor 1, quad xor 2, half-row mirror)
@@ -301,7 +303,7 @@ __global__ __launch_bounds__(64 * ATT_WAVES) void paged_attention_kernel(
 // smaller (multiples of 8) is padded with zeros on its way into registers and LDS, and only its
 // own channels are stored.
 template <int DS, int VT>
-__global__ __launch_bounds__(256) void paged_attention_mfma_kernel(
+__global__ __launch_bounds__(256, 2) void paged_attention_mfma_kernel(
     bf16s* __restrict__ out, const bf16s* __restrict__ q, long q_stride, const bf16s* __restrict__ kpool,
     const bf16s* __restrict__ vpool, const int* __restrict__ block_tables, int bt_stride, const int* __restrict__ cu,
     const int* __restrict__ start, const float* __restrict__ slopes, const bf16s* __restrict__ gate, long gate_stride,
@@ -324,8 +326,11 @@ __global__ __launch_bounds__(256) void paged_attention_mfma_kernel(
 #pragma unroll
   for (int e = 0; e < 8; ++e) zero8[e] = (__bf16)0.0f;
   constexpr int KP = D + 8;            // key row pitch in LDS (elements): 16-byte reads of 16 rows hit 64 banks
-  constexpr int VP = 40;               // transposed value row pitch: 32 key slots + 8
-  constexpr int KT = 32 * KP, VTT = Dv * VP;   // elements of one staged tile
+  // Values are staged as they come, in column groups of 16 channels ([Dv / 16][32 keys][16], 32 bytes a key, 128
+  // bytes between the groups), and read as columns by transposing reads: a read takes 128 contiguous bytes
+  // from each of two neighbouring groups at a time, in different halves of the banks.
+  constexpr int VG = 32 * 16 + 64;             // elements of a group
+  constexpr int KT = 32 * KP, VTT = Dv / 16 * VG;   // elements of one staged tile
   constexpr int KCH = 32 * D / 8, VCH = 32 * Dv / 8;  // 16-byte chunks of a key / value tile
   constexpr int TP = MFMA_TILES_PER_STEP;
   extern __shared__ __align__(16) bf16s tiles[];  // [2][TP][KT + VTT], then [2][TP][32] key factors (float)
@@ -371,6 +376,11 @@ __global__ __launch_bounds__(256) void paged_attention_mfma_kernel(
 #pragma unroll
   for (int s = 0; s < DS; ++s)
     qf[s] = 16 * s + hf * 8 < Dr ? ld_g16b(q + n * q_stride + (long)h * Dr + 16 * s + hf * 8) : zero8;
+  if (scale < 0.0f) {  // exact: the largest product of a row is then its largest score
+#pragma unroll
+    for (int s = 0; s < DS; ++s) qf[s] = -qf[s];
+    scale = -scale;
+  }
 
   const int lo_min = first_visible(bp0, window, chunk);   // the staged key range is the block's
   const int lo = first_visible(pos, window, chunk);       // this token's first key
@@ -385,13 +395,14 @@ __global__ __launch_bounds__(256) void paged_attention_mfma_kernel(
   const int my_sum = (ksum != nullptr && window > 0) ? max(0, (pos - window + 1) / sum_block) : 0;  // this token's
   const float* db = dist2 != nullptr ? dist2 + (long)h * dist_rows : nullptr;
 
-  // staging: key chunk c = key c / (row chunks), 8 elements starting at 8 * (c % row chunks), stored as a row;
-  // value chunk c = key c % 32, 8 channels starting at 8 * (c / 32): the values are stored transposed, two bytes at
-  // a time, and with neighbouring threads on neighbouring keys these stores spread over the LDS banks
+  // staging: key chunk c = key c / (row chunks), 8 elements starting at 8 * (c % row chunks), stored as a row; a wave's
+  // load of values covers 16 keys of 32 channels, so that its stores spread over the LDS banks
   constexpr int KR = (KCH + 255) / 256, VR = (VCH + 255) / 256;  // chunks per thread of the 256
   // TP key tiles are staged, and multiplied, between two barriers: their loads are all in flight over the
   // products of the TP tiles before them
   bf16x8_v rk[TP][KR], rv[TP][VR];
+  auto v_key = [&](int c) { return (c / (64 * VT)) * 16 + ((c & 63) >> 2); };
+  auto v_chunk = [&](int c) { return (c >> 6) % VT * 4 + (c & 3); };
   auto tile_base = [&](int it) {
     return it < sum_tiles ? it * 32 : it < sink_tiles ? (it - sum_tiles) * 32 : wstart + (it - sink_tiles) * 32;
   };
@@ -422,7 +433,7 @@ __global__ __launch_bounds__(256) void paged_attention_mfma_kernel(
 #pragma unroll
       for (int r = 0; r < VR; ++r) {
         const int c = tid + nthreads * r;
-        const int j = kbase + (c & 31);
+        const int j = kbase + v_key(c);
         vrow[u][r] = c < VCH ? (int)(from_sum[u] ? sum_row(j) : pool_row(j)) : 0;
       }
       if (key_fac != nullptr && tid < 32) frow[u] = (int)pool_row(kbase + tid);
@@ -445,7 +456,7 @@ __global__ __launch_bounds__(256) void paged_attention_mfma_kernel(
       for (int r = 0; r < VR; ++r) {
         const int c = tid + nthreads * r;
         if (c < VCH) {
-          const int off = 8 * (c >> 5);
+          const int off = 8 * v_chunk(c);
           rv[u][r] = off < Dvr ? ld_g16b(vp + ((long)vrow[u][r] * Gv + vg) * Dvr + off) : zero8;
         }
       }
@@ -466,15 +477,8 @@ __global__ __launch_bounds__(256) void paged_attention_mfma_kernel(
       for (int r = 0; r < VR; ++r) {
         const int c = tid + nthreads * r;
         if (c < VCH) {
-          const int kk = c & 31, dv0 = 8 * (c >> 5);
-          // contraction slot of key kk: the order in which the C layout of S^T hands the weights to P^T
-          const int r16 = kk & 15;
-          const int slot = (kk & 16) + ((r16 >> 2) & 1) * 8 + (r16 >> 3) * 4 + (r16 & 3);
-#pragma unroll
-          for (int e = 0; e < 8; ++e) {
-            const __bf16 x = rv[u][r][e];
-            vt[(dv0 + e) * VP + slot] = *reinterpret_cast<const bf16s*>(&x);
-          }
+          const int ch = v_chunk(c);
+          *reinterpret_cast<bf16x8_v*>(vt + (ch >> 1) * VG + v_key(c) * 16 + (ch & 1) * 8) = rv[u][r];
         }
       }
       if (key_fac != nullptr && tid < 32) facs[(buf * TP + u) * 32 + tid] = rf[u];
@@ -493,18 +497,23 @@ __global__ __launch_bounds__(256) void paged_attention_mfma_kernel(
 #pragma unroll
     for (int i = 0; i < 16; ++i) oacc[t][i] = 0.0f;
   constexpr float LOG2E = 1.4426950408889634f;
-  const float c1 = scale * LOG2E, sl2 = slope * LOG2E;
+  const float c1 = fmaxf(scale * LOG2E, 1e-30f), sl2 = slope * LOG2E;  // a scale of 0 must not meet -inf in a product
   // soft cap in the base-2 domain: cap log2e tanh(x scale / cap), tanh(y) = 1 - 2 / (exp2(2 log2e y) + 1)
   const bool capped = softcap > 0.0f;
   const float cap2 = softcap * LOG2E, t2 = capped ? 2.0f * LOG2E * scale / softcap : 0.0f;
-  auto base2 = [&](float dot) {
-    if (!capped) return dot * c1;
+  auto cap_base2 = [&](float dot) {
     const float e = __builtin_amdgcn_exp2f(fminf(dot * t2, 64.0f));  // beyond 2^64 the quotient is 0 in float32 anyway
     return cap2 - 2.0f * cap2 * __builtin_amdgcn_rcpf(e + 1.0f);
   };
-  float row_bias[16];  // + slope log2e * (row of the C layout): the key's offset inside its tile
+  // A key's share of the distance penalty: its offset inside its tile (row of the C layout) here, the tile's per tile
+  const bool sloped = slopes != nullptr;
+  float row_bias[16];
 #pragma unroll
   for (int i = 0; i < 16; ++i) row_bias[i] = sl2 * (float)((i & 3) + 8 * (i >> 2) + 4 * hf);
+  // Without a cap, a penalty or a table the scores stay raw products and their factor enters with the fma that
+  // subtracts the reference (a negative factor has moved into the query); otherwise they are formed in the base-2 domain.
+  const bool raw = !capped && !sloped && db == nullptr;
+  const float k1 = raw ? c1 : 1.0f;
 
   const int steps_n = (tiles_n + TP - 1) / TP;
   lookup(0);
@@ -519,103 +528,144 @@ __global__ __launch_bounds__(256) void paged_attention_mfma_kernel(
       fetch();
       if (step + 2 < steps_n) lookup(step + 2);
     }
+    // The TP tiles of a step go through the softmax together: one maximum, one exchange, one look at the rescaling.
+    bool live[TP];       // this wave sees something of the tile
+    bool any = false;
 #pragma unroll
     for (int u = 0; u < TP; ++u) {
-      const int it = step * TP + u;
-      if (!head_ok || it >= tiles_n) continue;
-      const bool summ = it < sum_tiles;
-      const bool sink = it < sink_tiles;  // a tile ahead of the window's: summaries or kept first tokens
-      const int kbase = tile_base(it);
+      const int it = step * TP + u, kbase = tile_base(it);
       // (query split) a tile wholly after this wave's tokens, or wholly before what they see
-      if (!sink && (kbase > p1 || (kbase + 31 < lo_p0 && kbase >= keep_first))) continue;
-      const int klimit = sink ? n_sink : p1 + 1;  // keys of this tile at or above it are not this tile's to count
-      const bf16s* ks = tiles + (buf * TP + u) * (KT + VTT);
-      const bf16s* vt = ks + KT;
-      f32x16 sacc;
+      live[u] = head_ok && it < tiles_n && (it < sink_tiles || !(kbase > p1 || (kbase + 31 < lo_p0 && kbase >= keep_first)));
+      any = any || live[u];
+    }
+    if (any) {
+      f32x16 x[TP];
+      float off[TP];
+      __builtin_amdgcn_s_setprio(1);
 #pragma unroll
-      for (int i = 0; i < 16; ++i) sacc[i] = 0.0f;
+      for (int u = 0; u < TP; ++u)
 #pragma unroll
-      for (int s = 0; s < DS; ++s) {
-        const bf16x8_v kf = *reinterpret_cast<const bf16x8_v*>(ks + col * KP + 16 * s + hf * 8);
-        sacc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, qf[s], sacc, 0, 0, 0);
-      }
-      if (key_fac != nullptr) {
-        const float* fc = facs + (buf * TP + u) * 32 + 4 * hf;
+        for (int i = 0; i < 16; ++i) x[u][i] = 0.0f;
 #pragma unroll
-        for (int a = 0; a < 4; ++a) {
-          const float4v f4 = *reinterpret_cast<const float4v*>(fc + 8 * a);
+      for (int s = 0; s < DS; ++s)
 #pragma unroll
-          for (int c = 0; c < 4; ++c) sacc[4 * a + c] *= f4[c];
+        for (int u = 0; u < TP; ++u) {
+          const bf16x8_v kf =
+              *reinterpret_cast<const bf16x8_v*>(tiles + (buf * TP + u) * (KT + VTT) + col * KP + 16 * s + hf * 8);
+          x[u] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, qf[s], x[u], 0, 0, 0);
+        }
+      __builtin_amdgcn_s_setprio(0);
+#pragma unroll
+      for (int u = 0; u < TP; ++u) {
+        const int it = step * TP + u, kbase = tile_base(it);
+        const bool summ = it < sum_tiles;
+        const bool ahead = it < sink_tiles;  // a tile ahead of the window's: summaries or kept first tokens
+        if (key_fac != nullptr) {
+          const float* fc = facs + (buf * TP + u) * 32 + 4 * hf;
+#pragma unroll
+          for (int a = 0; a < 4; ++a) {
+            const float4v f4 = *reinterpret_cast<const float4v*>(fc + 8 * a);
+#pragma unroll
+            for (int c = 0; c < 4; ++c) x[u][4 * a + c] *= f4[c];
+          }
+        }
+        off[u] = sloped && !summ ? -sl2 * (float)(pos - kbase) : 0.0f;
+        if (!raw) {
+          if (capped) {
+#pragma unroll
+            for (int i = 0; i < 16; ++i) x[u][i] = cap_base2(x[u][i]);
+            if (sloped && !summ) {
+#pragma unroll
+              for (int i = 0; i < 16; ++i) x[u][i] += row_bias[i];
+            }
+          } else if (sloped && !summ) {
+#pragma unroll
+            for (int i = 0; i < 16; ++i) x[u][i] = fmaf(x[u][i], c1, row_bias[i]);
+          } else {
+#pragma unroll
+            for (int i = 0; i < 16; ++i) x[u][i] *= c1;
+          }
+          if (db != nullptr && !summ) {
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+              const int j = kbase + (i & 3) + 8 * (i >> 2) + 4 * hf;
+              x[u][i] += db[min(max(pos - j, 0), dist_rows - 1)];
+            }
+          }
+        }
+        // interior tile: every key is visible to every token of the wave, no masks to evaluate
+        const bool interior = live[u] && !ahead && t_off + 31 < cnt && kbase + 31 <= p0 && kbase >= lo_p1;
+        if (!interior) {
+          const int klimit = !live[u] ? 0 : ahead ? n_sink : p1 + 1;  // keys of this tile at or above it are not its to count
+#pragma unroll
+          for (int i = 0; i < 16; ++i) {
+            const int j = kbase + (i & 3) + 8 * (i >> 2) + 4 * hf;
+            const bool seen = tok_ok && (summ ? live[u] && j < my_sum : j < klimit && j <= pos && (j >= lo || j < keep_first));
+            if (!seen) x[u][i] = -INFINITY;
+          }
         }
       }
-      // scores in the base-2 domain: s2 = (q.k) scale log2e - slope log2e (pos - j), one add and one fma each
-      float sv[16];
-      const float tile_bias = -sl2 * (float)(pos - kbase);
-      // interior tile: every key is visible to every token of the tile, no masks to evaluate
-      const bool interior = !sink && t_off + 31 < cnt && kbase + 31 <= p0 && kbase >= lo_p1;
-      if (summ) {  // summaries: seen by count, no distance terms
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
-          const int j = kbase + (i & 3) + 8 * (i >> 2) + 4 * hf;
-          sv[i] = (tok_ok && j < my_sum) ? base2(sacc[i]) : -INFINITY;
-        }
-      } else if (interior) {
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
-          sv[i] = base2(sacc[i]) + (tile_bias + row_bias[i]);
-        }
-      } else {
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
-          const int j = kbase + (i & 3) + 8 * (i >> 2) + 4 * hf;
-          const bool seen = tok_ok && j < klimit && j <= pos && (j >= lo || j < keep_first);
-          sv[i] = seen ? base2(sacc[i]) + (tile_bias + row_bias[i]) : -INFINITY;
-        }
-      }
-      if (db != nullptr && !summ) {
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
-          const int j = kbase + (i & 3) + 8 * (i >> 2) + 4 * hf;
-          sv[i] += db[min(max(pos - j, 0), dist_rows - 1)];   // -inf stays -inf
-        }
-      }
-      float m_ref = 0.0f, corr = 1.0f;
+      float m_ref = 0.0f;
       if (!fixed_ref) {
         float tmax = -INFINITY;
 #pragma unroll
-        for (int i = 0; i < 16; ++i) tmax = fmaxf(tmax, sv[i]);
+        for (int u = 0; u < TP; ++u) {
+          float top = x[u][0];
+#pragma unroll
+          for (int i = 1; i < 16; ++i) top = fmaxf(top, x[u][i]);
+          tmax = fmaxf(tmax, top == -INFINITY ? -INFINITY : fmaf(top, k1, off[u]));
+        }
         tmax = fmaxf(tmax, __shfl_xor(tmax, 32));
         const float m_new = fmaxf(m, tmax);
-        m_ref = (m_new == -INFINITY) ? 0.0f : m_new;  // nothing visible yet: every weight is exp2(-inf) = 0
-        corr = (m == -INFINITY) ? 1.0f : __builtin_amdgcn_exp2f(m - m_new);  // nothing accumulated: nothing to rescale
+        if (!__all(m_new == m)) {  // otherwise the running maxima of all 32 tokens stand still: no rescaling
+          const float corr = (m == -INFINITY) ? 1.0f : __builtin_amdgcn_exp2f(m - m_new);  // nothing accumulated: nothing to rescale
+          l *= corr;
+#pragma unroll
+          for (int t = 0; t < VT; ++t)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) oacc[t][i] *= corr;
+        }
         m = m_new;
+        m_ref = (m_new == -INFINITY) ? 0.0f : m_new;  // nothing visible yet: every weight is exp2(-inf) = 0
       }
       float psum = 0.0f;
-      bf16x8_v phi[2], plo[2];
+      bf16x8_v phi[TP][2], plo[TP][2];
 #pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        const float p = __builtin_amdgcn_exp2f(sv[i] - m_ref);
-        psum += p;
-        const __bf16 hi = (__bf16)p;
-        phi[i >> 3][i & 7] = hi;
-        plo[i >> 3][i & 7] = (__bf16)(p - (float)hi);
-      }
-      l = l * corr + psum;
-      if (!fixed_ref && !__all(corr == 1.0f)) {  // the running maxima of all 32 tokens stood still: no rescaling
+      for (int u = 0; u < TP; ++u) {
+        const float base = off[u] - m_ref;
 #pragma unroll
-        for (int t = 0; t < VT; ++t)
-#pragma unroll
-          for (int i = 0; i < 16; ++i) oacc[t][i] *= corr;
-      }
-      // O^T += V^T P^T: slot hf * 8 + e of step s2 holds key kbase + 16 s2 + 8 (e >> 2) + 4 hf + (e & 3)
-#pragma unroll
-      for (int s2 = 0; s2 < 2; ++s2)
-#pragma unroll
-        for (int t = 0; t < VT; ++t) {
-          const bf16x8_v va = *reinterpret_cast<const bf16x8_v*>(vt + (t * 32 + col) * VP + 16 * s2 + hf * 8);
-          oacc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va, phi[s2], oacc[t], 0, 0, 0);
-          oacc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va, plo[s2], oacc[t], 0, 0, 0);
+        for (int i = 0; i < 16; i += 2) {  // two weights a time: one conversion packs two halves
+          const float p0 = __builtin_amdgcn_exp2f(fmaf(x[u][i], k1, base));
+          const float p1 = __builtin_amdgcn_exp2f(fmaf(x[u][i + 1], k1, base));
+          psum += p0 + p1;
+          const bf16x2_v hi = __builtin_convertvector(float2v{p0, p1}, bf16x2_v);
+          const unsigned bits = __builtin_bit_cast(unsigned, hi);
+          const bf16x2_v lo = __builtin_convertvector(float2v{p0 - __builtin_bit_cast(float, bits << 16),
+                                                              p1 - __builtin_bit_cast(float, bits & 0xffff0000u)}, bf16x2_v);
+          phi[u][i >> 3][i & 7] = hi[0];
+          phi[u][i >> 3][(i & 7) + 1] = hi[1];
+          plo[u][i >> 3][i & 7] = lo[0];
+          plo[u][i >> 3][(i & 7) + 1] = lo[1];
         }
+      }
+      l += psum;
+      // O^T += V^T P^T: slot hf * 8 + e of step s2 holds key kbase + 16 s2 + 8 (e >> 2) + 4 hf + (e & 3)
+      __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+      for (int u = 0; u < TP; ++u)
+#pragma unroll
+        for (int s2 = 0; s2 < 2; ++s2)
+#pragma unroll
+          for (int t = 0; t < VT; ++t) {
+            const bf16s* vp = tiles + (buf * TP + u) * (KT + VTT) + KT + (2 * t + ((lane >> 4) & 1)) * VG +
+                              (16 * s2 + 4 * hf + ((lane & 15) >> 2)) * 16 + (lane & 3) * 4;
+            const bf16x4_v v0 = ld_tr16(reinterpret_cast<const char*>(vp), 0);
+            const bf16x4_v v1 = ld_tr16(reinterpret_cast<const char*>(vp), 8 * 32);
+            const bf16x8_v va = __builtin_shufflevector(v0, v1, 0, 1, 2, 3, 4, 5, 6, 7);
+            oacc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va, phi[u][s2], oacc[t], 0, 0, 0);
+            oacc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va, plo[u][s2], oacc[t], 0, 0, 0);
+          }
+      __builtin_amdgcn_s_setprio(0);
     }
     if (more) stash(buf ^ 1);
     __syncthreads();
@@ -728,7 +778,7 @@ static bool launch_mfma_attention(at::Tensor& out, const at::Tensor& q, const at
     const dim3 grid((unsigned)(qsplit ? num_tiles128 : num_tiles), (unsigned)G, (unsigned)((rep + nw - 1) / nw * VC));
     const int ds = D <= 32 ? 2 : D <= 48 ? 3 : D <= 64 ? 4 : D <= 96 ? 6 : 8, vt = (Dv + 31) / 32;
     const size_t msmem = (size_t)2 * MFMA_TILES_PER_STEP *
-                         ((32 * (ds * 16 + 8) + vt * 32 * 40) * sizeof(bf16s) + (x.key_fac != nullptr ? 32 * sizeof(float) : 0));
+                         ((32 * (ds * 16 + 8) + vt * 2 * (32 * 16 + 64)) * sizeof(bf16s) + (x.key_fac != nullptr ? 32 * sizeof(float) : 0));
 #define MFMA_CASE(DS_, VT_)                                                                                        \
   do {                                                                                                             \
     auto kfn = paged_attention_mfma_kernel<DS_, VT_>;                                                              \

@@ -1,0 +1,55 @@
+"""Paged attention over the edges of its kernels: token and key tile remainders, sequences of a few tokens beside long
+ones, scales of either sign and zero, with and without the parts that put scores into the base-2 domain early.
+
+The bound: float32 scores and weights; the output is rounded to bfloat16 once (at most 2^-9 of a value) and a score
+error of a few float32 roundings of the largest score moves a weight by less than that."""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+BOUND = 2.0 ** -8
+
+
+def _batch(counts, starts, page, seed=0):
+    from colossalai_amd.ops.ragged import RaggedBatch
+
+    need = [(a + b + page - 1) // page for a, b in zip(counts, starts)]
+    order = torch.randperm(sum(need), generator=torch.Generator().manual_seed(seed)).tolist()
+    tables, at = [], 0
+    for n in need:
+        tables.append(order[at: at + n])
+        at += n
+    return RaggedBatch.build(counts, starts, list(range(len(counts))), "cuda", tables, page), sum(need)
+
+
+def _check(counts, starts, H, G, D, Dv, page, scale, **kw):
+    from colossalai_amd.ops.paged_attention import distance_slopes, paged_attention, paged_attention_ref
+
+    torch.manual_seed(1)
+    batch, pages = _batch(counts, starts, page)
+    k = torch.randn(pages, page, G, D, device="cuda").bfloat16()
+    v = torch.randn(pages, page, G, Dv, device="cuda").bfloat16()
+    q = torch.randn(sum(counts), H, D, device="cuda").bfloat16()
+    if kw.pop("slopes", False):
+        kw["slopes"] = distance_slopes(H, "cuda")
+    if kw.pop("gate", False):
+        kw["gate"] = torch.randn(sum(counts), H, device="cuda").bfloat16()
+    if kw.pop("sink_logits", False):
+        kw["sink_logits"] = torch.randn(H, device="cuda") + 2.0
+    if kw.pop("factors", False):
+        kw["key_factors"] = torch.rand(pages, page, G, device="cuda") + 0.5
+    got = paged_attention(q, k, v, batch, scale, **kw)
+    kw.setdefault("window", 0)
+    want = paged_attention_ref(q.float(), k.float(), v.float(), batch, scale, **{n: (t.float() if n == "gate" else t)
+                                                                                  for n, t in kw.items()})
+    err = (got.double() - want.double()).norm() / want.double().norm()
+    assert err < BOUND, f"{err:.2e}"
+    assert torch.isfinite(got.float()).all()
+
+
+@pytest.mark.parametrize("scale", [0.1, -0.1, 0.0])
+@pytest.mark.parametrize("kw", [{}, dict(softcap=5.0, sink=True), dict(slopes=True, window=70, keep_first=4), dict(chunk=64)])
+def test_portions_and_scales(scale, kw):
+    _check([33, 1, 96, 65], [0, 130, 31, 64], 8, 2, 128, 128, 16, scale, **dict(kw))
