@@ -8,8 +8,16 @@
 //   * every lane group runs an online softmax of its own over its keys — nothing crosses lane groups in the loop;
 //   * the weighted sum uses the values in the same lanes. Where the values are the keys (or their leading channels)
 //     they are the registers the scores were formed from: each cached row is read once.
-// The lane groups' states meet in a butterfly, the waves' states in LDS, at the end.
+// The lane groups' states meet in a butterfly, the waves' states in LDS, at the end. Few tokens with long contexts
+// have their keys cut into parts, one block each, whose states row_merge_kernel puts together.
+//
+// What bounds it: the chain of dependent loads (position, page table, rows) and the block's end, about 10 us
+// together, and beyond that the vector instructions of the products; 16 x 1024 keys of 16/4 heads of 128 run 18.9 us (29.8
+// before the base-2 scores and the halving butterfly), 1.8 TB/s; 4 x 16384 run 44 us (193 with one block per token,
+// kv head and head), 3.0 TB/s.
 #include "paged_attention.h"
+
+#include <algorithm>
 
 namespace cai {
 namespace serving {
@@ -40,6 +48,39 @@ template <> struct RowLane<float> {
   }
 };
 
+// The domain of the scores. bfloat16: base 2, so that a weight is one v_exp_f32 and the cap an exponential and a
+// reciprocal; float32 serving keeps the natural one with the library's functions.
+template <typename T> struct Dom;
+template <> struct Dom<bf16s> {
+  static constexpr float UNIT = 1.4426950408889634f;   // what one nat is here
+  DEV_INLINE static float exp_(float x) { return __builtin_amdgcn_exp2f(x); }
+  // cap tanh(x / cap) for x and cap in units of this domain: tanh(y) = 1 - 2 / (exp(2 y) + 1)
+  DEV_INLINE static float cap_(float x, float cap, float inv_cap) {
+    const float e = __builtin_amdgcn_exp2f(fminf(x * inv_cap * (2.0f * UNIT), 64.0f));
+    return cap - 2.0f * cap * __builtin_amdgcn_rcpf(e + 1.0f);
+  }
+};
+template <> struct Dom<float> {
+  static constexpr float UNIT = 1.0f;
+  DEV_INLINE static float exp_(float x) { return expf(x); }
+  DEV_INLINE static float cap_(float x, float cap, float inv_cap) { return cap * tanhf(x * inv_cap); }
+};
+
+typedef unsigned uint2v_ __attribute__((ext_vector_type(2)));
+
+// Sums of two values over the two halves of the wave (rows of 16 lanes for swap16): lanes of the lower half (even
+// rows) get a's sum, the others b's. A swap exchanges the upper half of a with the lower half of b.
+DEV_INLINE float swap32_add(float a, float b) {
+  const uint2v_ r = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(unsigned, a), __builtin_bit_cast(unsigned, b), false, false);
+  const unsigned x = r[0], y = r[1];
+  return __builtin_bit_cast(float, x) + __builtin_bit_cast(float, y);
+}
+DEV_INLINE float swap16_add(float a, float b) {
+  const uint2v_ r = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(unsigned, a), __builtin_bit_cast(unsigned, b), false, false);
+  const unsigned x = r[0], y = r[1];
+  return __builtin_bit_cast(float, x) + __builtin_bit_cast(float, y);
+}
+
 template <typename T, int RC, int NS, bool SEP>
 __global__ __launch_bounds__(64 * ROW_WAVES) void row_attention_kernel(
     T* __restrict__ out, float* __restrict__ out32, const T* __restrict__ q, long q_stride, const T* __restrict__ kpool,
@@ -47,14 +88,18 @@ __global__ __launch_bounds__(64 * ROW_WAVES) void row_attention_kernel(
     const int* __restrict__ positions, const float* __restrict__ slopes, const T* __restrict__ gate, long gate_stride,
     const float* __restrict__ sink_logits, const float* __restrict__ key_fac, int H, int G, int D, int Dv, int page_shift,
     float scale, int window, int keep_first, int chunk, float softcap, int sink, int vrep, long vrow, long vhead,
-    int lane_shift, int qvec) {
+    int lane_shift, int qvec, int splits, float* __restrict__ ws) {
   constexpr int CH = RowLane<T>::CH, HC = CH / 2;
   extern __shared__ __align__(16) float lds[];
   const int wid = threadIdx.x >> 6, lane = threadIdx.x & 63, nw = blockDim.x >> 6;
   const int R = H / G, chunks = (R + RC - 1) / RC;
-  const long n = blockIdx.x / (G * chunks);
-  const int g = (int)(blockIdx.x / chunks) % G;
-  const int h0 = g * R + (int)(blockIdx.x % chunks) * RC;
+  // Heads of a group that are other blocks' come last: those blocks read the same rows, and a multiple of 8 blocks
+  // apart they share an XCD's L2.
+  const long parts = gridDim.x / chunks, item = blockIdx.x % parts;
+  const int split = (int)(item % splits);           // which part of the keys
+  const long n = item / splits / G;
+  const int g = (int)(item / splits % G);
+  const int h0 = g * R + (int)(blockIdx.x / parts) * RC;
   const int nh = min(RC, g * R + R - h0);
   const int L = 1 << lane_shift;
   const int ch = (lane & (L - 1)) * CH;             // this lane's first channel
@@ -68,7 +113,7 @@ __global__ __launch_bounds__(64 * ROW_WAVES) void row_attention_kernel(
   float qf[RC][CH], slope[RC];
 #pragma unroll
   for (int r = 0; r < RC; ++r) {
-    slope[r] = (slopes != nullptr && r < nh) ? slopes[h0 + r] : 0.0f;
+    slope[r] = (slopes != nullptr && r < nh) ? slopes[h0 + r] * Dom<T>::UNIT : 0.0f;
     const T* qp = q + n * q_stride + (long)(h0 + r) * D + ch;
     if (qvec) {
       const int4v_ none = {0, 0, 0, 0};
@@ -79,12 +124,15 @@ __global__ __launch_bounds__(64 * ROW_WAVES) void row_attention_kernel(
       for (int c = 0; c < CH; ++c) qf[r][c] = r < nh && ch + c < D ? ldf(qp + c) : 0.0f;
     }
 #pragma unroll
-    for (int c = 0; c < CH; ++c) qf[r][c] *= scale;
+    for (int c = 0; c < CH; ++c) qf[r][c] *= scale * Dom<T>::UNIT;
   }
   const int lo = first_visible(pos, window, chunk);
   const int n_keep = window > 0 ? min(keep_first, lo) : 0;
   const int total = n_keep + (pos - lo + 1);
-  const float inv_cap = softcap > 0.0f ? 1.0f / softcap : 0.0f;
+  // this block's keys: whole key blocks of all its waves
+  const int per = splits > 1 ? ((total + splits - 1) / splits + KB - 1) / KB * KB : total;
+  const int first = split * per, last = min(total, first + per);
+  const float cap = softcap * Dom<T>::UNIT, inv_cap = softcap > 0.0f ? 1.0f / cap : 0.0f;
   const T* vbase = SEP ? vpool + (long)(g / vrep) * vhead : nullptr;
 
   float m[RC], l[RC], acc[RC][CH];
@@ -96,30 +144,34 @@ __global__ __launch_bounds__(64 * ROW_WAVES) void row_attention_kernel(
     for (int c = 0; c < CH; ++c) acc[r][c] = 0.0f;
   }
   const int4v_ zero = {0, 0, 0, 0};
-  for (int base = wid * KB; base < total; base += nw * KB) {
-    int j[NS];
-    long row[NS];
+  auto key_of = [&](int idx) { return idx < last ? (idx < n_keep ? idx : lo + (idx - n_keep)) : pos; };
+  // pool rows of a block's keys; a key past the end reads the query's own row and is masked. Looked up one block ahead.
+  int row[NS];
+  auto lookup = [&](int base) {
+#pragma unroll
+    for (int s = 0; s < NS; ++s) {
+      const int j = key_of(base + s * KPS + group);
+      row[s] = (bt[j >> page_shift] << page_shift) + (j & page_mask);
+    }
+  };
+  if (first + wid * KB < last) lookup(first + wid * KB);
+  for (int base = first + wid * KB; base < last; base += nw * KB) {
     float fac[NS];
     int4v_ kr[NS][2], vr[SEP ? NS : 1][2];
 #pragma unroll
-    for (int s = 0; s < NS; ++s) {                  // a key past the end reads the query's own row and is masked
-      const int idx = base + s * KPS + group;
-      j[s] = idx < total ? (idx < n_keep ? idx : lo + (idx - n_keep)) : pos;
-      row[s] = ((long)bt[j[s] >> page_shift] << page_shift) + (j[s] & page_mask);
-    }
-#pragma unroll
     for (int s = 0; s < NS; ++s) {
-      const bool some = base + s * KPS < total;     // the wave's step holds a key
-      const T* kp = kpool + (row[s] * G + g) * D + ch;
+      const bool some = base + s * KPS < last;      // the wave's step holds a key
+      const T* kp = kpool + ((long)row[s] * G + g) * D + ch;
       kr[s][0] = some && ch < D ? *reinterpret_cast<const int4v_*>(kp) : zero;
       kr[s][1] = some && ch + HC < D ? *reinterpret_cast<const int4v_*>(kp + HC) : zero;
-      fac[s] = key_fac != nullptr && some ? key_fac[row[s] * G + g] : 1.0f;
+      fac[s] = key_fac != nullptr && some ? key_fac[(long)row[s] * G + g] : 1.0f;
       if constexpr (SEP) {
-        const T* vp = vbase + row[s] * vrow + ch;
+        const T* vp = vbase + (long)row[s] * vrow + ch;
         vr[s][0] = some && ch < Dv ? *reinterpret_cast<const int4v_*>(vp) : zero;
         vr[s][1] = some && ch + HC < Dv ? *reinterpret_cast<const int4v_*>(vp + HC) : zero;
       }
     }
+    if (base + nw * KB < last) lookup(base + nw * KB);
     float sc[RC][NS];
 #pragma unroll
     for (int s = 0; s < NS; ++s) {
@@ -152,18 +204,18 @@ __global__ __launch_bounds__(64 * ROW_WAVES) void row_attention_kernel(
 #pragma unroll
       for (int s = 0; s < NS; ++s) {
         float v = sc[r][s] * fac[s];
-        if (softcap > 0.0f) v = softcap * tanhf(v * inv_cap);
-        v -= slope[r] * (float)(pos - j[s]);
-        sc[r][s] = base + s * KPS + group < total ? v : -INFINITY;
+        if (softcap > 0.0f) v = Dom<T>::cap_(v, cap, inv_cap);
+        v -= slope[r] * (float)(pos - key_of(base + s * KPS + group));
+        sc[r][s] = base + s * KPS + group < last ? v : -INFINITY;
         top = fmaxf(top, sc[r][s]);
       }
       const float ref = top == -INFINITY ? 0.0f : top;   // no key in this lane group yet
-      const float corr = expf(m[r] - ref);
+      const float corr = Dom<T>::exp_(m[r] - ref);
       m[r] = top;
       float sum = 0.0f;
 #pragma unroll
       for (int s = 0; s < NS; ++s) {
-        sc[r][s] = expf(sc[r][s] - ref);
+        sc[r][s] = Dom<T>::exp_(sc[r][s] - ref);
         sum += sc[r][s];
       }
       l[r] = l[r] * corr + sum;
@@ -183,26 +235,52 @@ __global__ __launch_bounds__(64 * ROW_WAVES) void row_attention_kernel(
         for (int c = 0; c < CH; ++c) acc[r][c] += sc[r][s] * vf[c];
     }
   }
+  // The lane groups' states meet. Up to 8 lanes a row, the groups are spread over the three upper bits of the lane
+  // number: each of these levels halves the channels a lane goes on with, so that 14 sums do instead of 48.
   const int PS = 2 + Dv;
 #pragma unroll
   for (int r = 0; r < RC; ++r) {
     float top = m[r];
     for (int off = L; off < 64; off <<= 1) top = fmaxf(top, __shfl_xor(top, off));
-    const float f = m[r] == -INFINITY ? 0.0f : expf(m[r] - top);
+    const float f = m[r] == -INFINITY ? 0.0f : Dom<T>::exp_(m[r] - top);
     float ll = l[r] * f;
     for (int off = L; off < 64; off <<= 1) ll += __shfl_xor(ll, off);
 #pragma unroll
     for (int c = 0; c < CH; ++c) acc[r][c] *= f;
-    for (int off = L; off < 64; off <<= 1) {
-#pragma unroll
-      for (int c = 0; c < CH; ++c) acc[r][c] += __shfl_xor(acc[r][c], off);
-    }
     float* mine = part + (wid * RC + r) * PS;
     if (lane == 0) { mine[0] = top; mine[1] = ll; }
-    if (group == 0) {
+    if (L <= 8) {
+      float a8[CH / 2], a4[CH / 4], a2[CH / 8];
 #pragma unroll
-      for (int c = 0; c < CH; ++c)
-        if (ch + c < Dv) mine[2 + ch + c] = acc[r][c];
+      for (int c = 0; c < CH / 2; ++c) a8[c] = swap32_add(acc[r][c], acc[r][c + CH / 2]);
+#pragma unroll
+      for (int c = 0; c < CH / 4; ++c) a4[c] = swap16_add(a8[c], a8[c + CH / 4]);
+      const bool up = (lane & 8) != 0;
+#pragma unroll
+      for (int c = 0; c < CH / 8; ++c) {
+        const float keep = up ? a4[c + CH / 8] : a4[c], give = up ? a4[c] : a4[c + CH / 8];
+        a2[c] = keep + __shfl_xor(give, 8);
+      }
+      for (int off = L; off < 8; off <<= 1) {
+#pragma unroll
+        for (int c = 0; c < CH / 8; ++c) a2[c] += __shfl_xor(a2[c], off);
+      }
+      if ((lane & 7) < L) {
+        const int at = ch + (lane >> 5) * (CH / 2) + (lane >> 4 & 1) * (CH / 4) + (lane >> 3 & 1) * (CH / 8);
+#pragma unroll
+        for (int c = 0; c < CH / 8; ++c)
+          if (at + c < Dv) mine[2 + at + c] = a2[c];
+      }
+    } else {
+      for (int off = L; off < 64; off <<= 1) {
+#pragma unroll
+        for (int c = 0; c < CH; ++c) acc[r][c] += __shfl_xor(acc[r][c], off);
+      }
+      if (group == 0) {
+#pragma unroll
+        for (int c = 0; c < CH; ++c)
+          if (ch + c < Dv) mine[2 + ch + c] = acc[r][c];
+      }
     }
   }
   __syncthreads();
@@ -211,14 +289,25 @@ __global__ __launch_bounds__(64 * ROW_WAVES) void row_attention_kernel(
     const float mw = lane < nw ? part[(lane * RC + r) * PS] : -INFINITY;
     const float lw = lane < nw ? part[(lane * RC + r) * PS + 1] : 0.0f;
     float top = wave_reduce_max(mw);
-    if (sink_logits != nullptr) top = fmaxf(top, sink_logits[h0 + r]);
-    const float f = mw == -INFINITY ? 0.0f : expf(mw - top);
-    float ll = wave_reduce_sum(lw * f);
-    if (sink_logits != nullptr) ll += expf(sink_logits[h0 + r] - top);
-    else if (sink) ll += expf(-top);   // the sink's score is 0
-    float c = f / ll;
-    if (gate != nullptr) c *= sigmoidf_(ldf(gate + n * gate_stride + h0 + r));
-    if (lane < nw) coef[r * ROW_WAVES + lane] = c;
+    if (splits > 1) {  // this block's state for row_merge_kernel; a part without keys has a maximum of -inf
+      const float f = mw == -INFINITY ? 0.0f : Dom<T>::exp_(mw - top);
+      const float ll = wave_reduce_sum(lw * f);
+      if (lane < nw) coef[r * ROW_WAVES + lane] = f;
+      if (lane == 0) {
+        float* state = ws + ((n * H + h0 + r) * splits + split) * (long)(2 + Dv);
+        state[0] = top;
+        state[1] = ll;
+      }
+    } else {
+      if (sink_logits != nullptr) top = fmaxf(top, sink_logits[h0 + r] * Dom<T>::UNIT);
+      const float f = mw == -INFINITY ? 0.0f : Dom<T>::exp_(mw - top);
+      float ll = wave_reduce_sum(lw * f);
+      if (sink_logits != nullptr) ll += Dom<T>::exp_(sink_logits[h0 + r] * Dom<T>::UNIT - top);
+      else if (sink) ll += Dom<T>::exp_(-top);   // the sink's score is 0
+      float c = f / ll;
+      if (gate != nullptr) c *= sigmoidf_(ldf(gate + n * gate_stride + h0 + r));
+      if (lane < nw) coef[r * ROW_WAVES + lane] = c;
+    }
   }
   __syncthreads();
   for (int i = threadIdx.x; i < nh * Dv; i += blockDim.x) {
@@ -227,8 +316,38 @@ __global__ __launch_bounds__(64 * ROW_WAVES) void row_attention_kernel(
 #pragma unroll 4
     for (int w = 0; w < nw; ++w) o += coef[r * ROW_WAVES + w] * part[(w * RC + r) * PS + 2 + dv];
     const long at = (n * H + h0 + r) * (long)Dv + dv;
-    if (out32 != nullptr) out32[at] = o;
+    if (splits > 1) ws[((n * H + h0 + r) * splits + split) * (long)(2 + Dv) + 2 + dv] = o;
+    else if (out32 != nullptr) out32[at] = o;
     else stf(out + at, o);
+  }
+}
+
+// The states of a (token, head)'s parts [splits][2 + Dv] -> its output: one wave per (token, head), the parts' weights
+// lane by lane, then channels.
+template <typename T>
+__global__ __launch_bounds__(256) void row_merge_kernel(
+    T* __restrict__ out, float* __restrict__ out32, const float* __restrict__ ws, const T* __restrict__ gate, long gate_stride,
+    const float* __restrict__ sink_logits, long rows, int H, int Dv, int sink, int splits) {
+  const long row = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
+  if (row >= rows) return;
+  const float* state = ws + row * splits * (long)(2 + Dv);
+  const int h = (int)(row % H);
+  const float m = lane < splits ? state[lane * (long)(2 + Dv)] : -INFINITY;   // splits <= 64
+  const float l = lane < splits ? state[lane * (long)(2 + Dv) + 1] : 0.0f;
+  float top = wave_reduce_max(m);
+  if (sink_logits != nullptr) top = fmaxf(top, sink_logits[h] * Dom<T>::UNIT);
+  const float f = m == -INFINITY ? 0.0f : Dom<T>::exp_(m - top);
+  float ll = wave_reduce_sum(l * f);
+  if (sink_logits != nullptr) ll += Dom<T>::exp_(sink_logits[h] * Dom<T>::UNIT - top);
+  else if (sink) ll += Dom<T>::exp_(-top);   // the sink's score is 0
+  float c = f / ll;
+  if (gate != nullptr) c *= sigmoidf_(ldf(gate + row / H * gate_stride + h));
+  for (int dv = lane; dv < Dv; dv += 64) {
+    float o = 0.0f;
+    for (int p = 0; p < splits; ++p) o += __shfl(c, p) * state[p * (long)(2 + Dv) + 2 + dv];
+    if (out32 != nullptr) out32[row * (long)Dv + dv] = o;
+    else stf(out + row * (long)Dv + dv, o);
   }
 }
 
@@ -249,22 +368,40 @@ bool launch_row_attention(at::Tensor& out, const at::Tensor& q, const at::Tensor
   int lane_shift = 0;
   while ((CH << lane_shift) < (D > Dv ? D : Dv)) ++lane_shift;
   const int R = H / G;
-  int rc = R > 1 && N * G * ((R + 1) / 2) >= 256 ? 2 : 1;   // two heads share a block's rows when enough blocks cover the CUs
+  // Most keys a token of this call can see: what its page table, window or block of positions holds.
+  long keys = block_tables.size(1) << page_shift;
+  if (window > 0) keys = std::min<long>(keys, window + keep_first);
+  if (x.chunk > 0) keys = std::min<long>(keys, x.chunk);
+  // Query heads per block and parts of the keys. Heads that share a block share its reads; heads in blocks of
+  // their own meet in L2 and cost less per key, which wins while the chip is not full and the context is short (16
+  // sequences of 1024 keys, 16/4 heads of 128: 18.9 us with one head a block, 19.7 with two and two parts; 4 x 16384: 53.9
+  // against 44.0; 16 x 6000, 32/8 heads: 221 against 113; four heads do not fit into the registers: 166).
+  // Then the keys are cut into parts while there are fewer blocks than CUs and a part still gives every wave a key
+  // block: 4 x 16384 210 -> 44 us, 8 x 2048 26.6 -> 19.1, 1 x 4096 36 -> 18. More blocks than CUs are slower again (4 x 16384
+  // with 512 blocks 76 us): a block costs about 10 us by itself.
+  int rc = R > 1 && (N * G * ((R + 1) / 2) >= 256 || keys >= 8192) ? 2 : 1;
+  int splits = 1;
+  const long blocks = N * G * ((R + rc - 1) / rc);
+  const long pass = (long)ROW_WAVES * (rc == 1 || shared ? 8 : 4) * (64 >> lane_shift);   // keys of one key block of every wave
+  while (blocks * splits * 2 <= 256 && keys > splits * pass) splits *= 2;
   auto lds_bytes = [&](int nw) { return (size_t)(rc * ROW_WAVES + nw * rc * (2 + Dv)) * sizeof(float); };
   int nwaves = ROW_WAVES;
   while (lds_bytes(nwaves) > 64 * 1024 && nwaves > 4) nwaves >>= 1;
   while (lds_bytes(nwaves) > 64 * 1024 && rc > 1) rc >>= 1;
   if (lds_bytes(nwaves) > 64 * 1024) return false;
   const int chunks = (R + rc - 1) / rc;
+  at::Tensor ws;
+  if (splits > 1) ws = at::empty({N * H * splits * (2 + Dv)}, q.options().dtype(at::kFloat));
   const int qvec = al16(q.data_ptr()) && q.stride(0) % piece == 0 ? 1 : 0;
 #define ROW_LAUNCH(RC_, NS_, SEP_)                                                                                     \
-  hipLaunchKernelGGL((row_attention_kernel<T, RC_, NS_, SEP_>), dim3((unsigned)(N * G * chunks)), dim3(64 * nwaves),    \
+  hipLaunchKernelGGL((row_attention_kernel<T, RC_, NS_, SEP_>), dim3((unsigned)(N * G * chunks * splits)), dim3(64 * nwaves), \
                      lds_bytes(nwaves), stream(), x.out32 != nullptr ? (T*)nullptr : ptr<T>(out), x.out32, ptr<T>(q),   \
                      (long)q.stride(0), ptr<T>(kpool), ptr<T>(vpool), block_tables.data_ptr<int>(),                     \
                      (int)block_tables.stride(0), tok_seq.data_ptr<int>(), positions.data_ptr<int>(), slopes,           \
                      gate.has_value() ? ptr<T>(*gate) : (const T*)nullptr, gate_stride, x.sink_logits, x.key_fac, H, G, \
                      D, Dv, page_shift, (float)scale, (int)window, (int)keep_first, x.chunk, (float)softcap,            \
-                     sink ? 1 : 0, x.vrep, vrow, vhead, lane_shift, qvec)
+                     sink ? 1 : 0, x.vrep, vrow, vhead, lane_shift, qvec, splits,                                       \
+                     splits > 1 ? ws.data_ptr<float>() : (float*)nullptr)
   SERVING_DISPATCH_ACT(q, T, {
     if (shared) {
       if (rc == 1) ROW_LAUNCH(1, 8, false);
@@ -272,6 +409,13 @@ bool launch_row_attention(at::Tensor& out, const at::Tensor& q, const at::Tensor
     } else {
       if (rc == 1) ROW_LAUNCH(1, 8, true);
       else ROW_LAUNCH(2, 4, true);
+    }
+    if (splits > 1) {
+      HIP_CHECK_LAST();
+      hipLaunchKernelGGL((row_merge_kernel<T>), dim3((unsigned)((N * H + 3) / 4)), dim3(256), 0, stream(),
+                         x.out32 != nullptr ? (T*)nullptr : ptr<T>(out), x.out32, ws.data_ptr<float>(),
+                         gate.has_value() ? ptr<T>(*gate) : (const T*)nullptr, gate_stride, x.sink_logits, N * H, H, Dv,
+                         sink ? 1 : 0, splits);
     }
   });
 #undef ROW_LAUNCH

@@ -53,3 +53,28 @@ def _check(counts, starts, H, G, D, Dv, page, scale, **kw):
 @pytest.mark.parametrize("kw", [{}, dict(softcap=5.0, sink=True), dict(slopes=True, window=70, keep_first=4), dict(chunk=64)])
 def test_portions_and_scales(scale, kw):
     _check([33, 1, 96, 65], [0, 130, 31, 64], 8, 2, 128, 128, 16, scale, **dict(kw))
+
+
+@pytest.mark.parametrize("D,Dv", [(128, 128), (64, 64), (256, 256), (72, 40), (320, 256)])
+@pytest.mark.parametrize("kw", [{}, dict(softcap=5.0, sink=True), dict(sink_logits=True, gate=True), dict(factors=True),
+                                dict(slopes=True, window=1500, keep_first=4)])
+def test_decode_with_keys_in_parts(D, Dv, kw):
+    """Long contexts beside one that leaves most parts empty, one that ends a part exactly, and a token that sees itself only."""
+    _check([1, 1, 1, 1], [4999, 0, 2047, 600], 4, 2, D, Dv, 16, 0.1, **dict(kw))
+
+
+@pytest.mark.parametrize("H,G,starts", [(16, 4, [9000]), (6, 2, [8200, 100]), (8, 8, [3000, 511, 512, 513])])
+def test_decode_heads_and_parts(H, G, starts):
+    _check([1] * len(starts), starts, H, G, 128, 128, 64, 0.09)
+
+
+def test_decode_in_float32():
+    from colossalai_amd.ops.paged_attention import paged_attention, paged_attention_ref
+
+    torch.manual_seed(2)
+    batch, pages = _batch([1, 1], [4000, 37], 16)
+    q, k, v = (torch.randn(*s, device="cuda") for s in ((2, 8, 128), (pages, 16, 2, 128), (pages, 16, 2, 128)))
+    got = paged_attention(q, k, v, batch, 0.09, softcap=7.0, sink=True)
+    want = paged_attention_ref(q, k, v, batch, 0.09, softcap=7.0, sink=True)
+    # float32 sums over 4000 weights: 4000^0.5 roundings of 2^-24 at most on average, and as much again in the reference
+    assert (got - want).norm() / want.norm() < 2 * 4000 ** 0.5 * 2.0 ** -24
