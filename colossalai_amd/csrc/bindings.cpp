@@ -29,6 +29,11 @@ std::vector<at::Tensor> rmsnorm_fused_add_fwd(at::Tensor input, at::Tensor resid
                                               double eps, bool save_inv_rms);
 std::vector<at::Tensor> rmsnorm_bwd(at::Tensor dy, at::Tensor x, at::Tensor weight, at::Tensor inv_rms);
 
+// cross_entropy.hip
+void ce_fwd(at::Tensor logits, at::Tensor labels, int64_t ignore_index, at::Tensor lse, at::Tensor nll);
+void ce_bwd(at::Tensor logits, at::Tensor labels, int64_t ignore_index, at::Tensor lse, at::Tensor grad, at::Tensor loss);
+at::Tensor ce_loss(at::Tensor nll, at::Tensor labels, int64_t ignore_index);
+
 // layernorm.hip
 std::vector<at::Tensor> layernorm_fwd(at::Tensor input, at::Tensor gamma, c10::optional<at::Tensor> beta,
                                       double eps, bool save_stats);
@@ -100,6 +105,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("rmsnorm_fwd", &cai::rmsnorm_fwd, "RMSNorm forward");
   m.def("rmsnorm_fused_add_fwd", &cai::rmsnorm_fused_add_fwd, "fused residual-add RMSNorm forward");
   m.def("rmsnorm_bwd", &cai::rmsnorm_bwd, "RMSNorm backward");
+  m.def("ce_fwd", &cai::ce_fwd, "cross entropy of bf16 logits: log-sum-exp and negative log likelihood per row");
+  m.def("ce_bwd", &cai::ce_bwd, "cross entropy backward, logits -> their gradient in place");
+  m.def("ce_loss", &cai::ce_loss, "mean negative log likelihood over the rows that are not ignored, and their number");
   m.def("layernorm_fwd", &cai::layernorm_fwd, "LayerNorm forward");
   m.def("layernorm_bwd", &cai::layernorm_bwd, "LayerNorm backward");
   m.def("rope_inplace", &cai::rope_inplace, "in-place rotary embedding (fwd/bwd)");

@@ -6,7 +6,9 @@ chunk's logits and feeds the dW/dh GEMMs directly. At the flagship bench
 size (147k tokens x 32k vocab) this replaces a ~50 GB fp32 logits+softmax
 footprint with ~1 GB of transient chunk buffers — pure HBM savings.
 
-GEMMs run through hipBLASLt (torch.matmul); softmax math is fp32.
+GEMMs run through hipBLASLt (torch.matmul); softmax math is fp32. In bfloat16 on
+the GPU a chunk's logits are read once in the forward and overwritten by their
+gradient in the backward (csrc/cross_entropy.hip).
 Reference parity: the reference materializes logits and uses torch CE (or
 DistCrossEntropy under TP); this op is our memory-optimized equivalent.
 """
@@ -14,6 +16,8 @@ DistCrossEntropy under TP); this op is our memory-optimized equivalent.
 from typing import Optional
 
 import torch
+
+from ._kernels import kernels, use_hip
 
 __all__ = ["fused_linear_cross_entropy"]
 
@@ -23,6 +27,20 @@ class _FusedLinearCE(torch.autograd.Function):
     def forward(ctx, hidden, weight, labels, ignore_index, chunk_size):
         # hidden [N, H] (bf16/fp32), weight [V, H], labels [N]
         N = hidden.shape[0]
+        ctx.chunk_size = chunk_size
+        ctx.ignore_index = ignore_index
+        ctx.hip = (hidden.dtype == weight.dtype == torch.bfloat16 and labels.dtype == torch.int64
+                   and use_hip(hidden, weight, labels))
+        if ctx.hip:
+            labels = labels.contiguous()
+            lse = torch.empty(N, dtype=torch.float32, device=hidden.device)
+            nll = torch.empty_like(lse)
+            for s in range(0, N, chunk_size):
+                e = min(s + chunk_size, N)
+                kernels().ce_fwd(hidden[s:e] @ weight.t(), labels[s:e], ignore_index, lse[s:e], nll[s:e])
+            loss = kernels().ce_loss(nll, labels, ignore_index)
+            ctx.save_for_backward(hidden, weight, labels, lse, loss)
+            return loss[0].clone()  # a tensor of its own: what is saved is not handed out
         lse = torch.empty(N, dtype=torch.float32, device=hidden.device)
         picked = torch.empty(N, dtype=torch.float32, device=hidden.device)
         valid = labels != ignore_index
@@ -35,11 +53,12 @@ class _FusedLinearCE(torch.autograd.Function):
         n_valid = valid.sum().clamp(min=1)
         loss = ((lse - picked) * valid).sum() / n_valid
         ctx.save_for_backward(hidden, weight, safe_labels, valid, lse, n_valid)
-        ctx.chunk_size = chunk_size
         return loss
 
     @staticmethod
     def backward(ctx, grad_out):
+        if ctx.hip:
+            return _backward_hip(ctx, grad_out)
         hidden, weight, safe_labels, valid, lse, n_valid = ctx.saved_tensors
         N, H = hidden.shape
         chunk_size = ctx.chunk_size
@@ -59,6 +78,28 @@ class _FusedLinearCE(torch.autograd.Function):
             dh[s:e] = ds @ weight
             dw += (ds.t() @ hidden[s:e]).float()
         return dh, dw.to(weight.dtype), None, None, None
+
+
+def _backward_hip(ctx, grad_out):
+    hidden, weight, labels, lse, loss = ctx.saved_tensors
+    N, chunk_size = hidden.shape[0], ctx.chunk_size
+    grad = grad_out.float()
+    dh = torch.empty_like(hidden)
+    dw = None
+    for s in range(0, N, chunk_size):
+        e = min(s + chunk_size, N)
+        ds = hidden[s:e] @ weight.t()
+        kernels().ce_bwd(ds, labels[s:e], ctx.ignore_index, lse[s:e], grad, loss)
+        torch.mm(ds, weight, out=dh[s:e])
+        part = ds.t() @ hidden[s:e]
+        # chunks are summed in float32; a single chunk's product is the sum already
+        if dw is None:
+            dw = part if e == N else part.float()
+        else:
+            dw += part
+    if dw is None:
+        dw = torch.zeros_like(weight)
+    return dh, dw.to(weight.dtype), None, None, None
 
 
 def fused_linear_cross_entropy(

@@ -1,9 +1,11 @@
 """Flash attention where its launch takes another form: forward blocks of two and four waves, tile remainders,
 key/value tiles whose heads several backward blocks share (float32 sums), strided outputs, a negative scale.
 
-The bound: outputs and gradients are rounded to bfloat16 (at most 2^-9 of a value) after products of operands
-that were rounded once themselves (probabilities or their gradients), so the 2-norm of the error is below
-3 * 2^-9 of the result's."""
+The bound: rounding to bfloat16 is 2^-8 of a value at most, 2^-8 / sqrt(3) of a tensor in the 2-norm. An output or a
+gradient is rounded itself and is a product of two operands of which at most two were rounded before (probabilities or
+their gradients, the output in delta): three such errors add up to 2^-8 in the 2-norm, and half as much again
+is left for their not being independent.
+"""
 
 import pytest
 import torch

@@ -1,0 +1,69 @@
+"""Cross entropy over bf16 logits and RMSNorm at the edges of their kernels, against float32 (norm) and float64 (loss)
+references of the same bfloat16 inputs."""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+ROUND = 2.0 ** -8  # of a value at most, by rounding it to bfloat16 (8 significant bits)
+
+
+def _rel(got, want):
+    return ((got.double() - want.double()).norm() / want.double().norm().clamp_min(1e-30)).item()
+
+
+@pytest.mark.parametrize("N,V,H,chunk", [(1, 8, 64, 4096), (37, 1000, 64, 4096), (130, 50257, 64, 64), (257, 32000, 128, 256),
+                                         (64, 1023, 32, 17)])
+def test_linear_cross_entropy(N, V, H, chunk):
+    from colossalai_amd.ops.fused_ce import fused_linear_cross_entropy
+
+    torch.manual_seed(0)
+    hidden = torch.randn(N, H, device="cuda").bfloat16().requires_grad_()
+    weight = (0.2 * torch.randn(V, H, device="cuda")).bfloat16().requires_grad_()
+    labels = torch.randint(0, V, (N,), device="cuda")
+    if N > 2:
+        labels[::3] = -100
+    loss = fused_linear_cross_entropy(hidden, weight, labels, chunk_size=chunk)
+    dh, dw = torch.autograd.grad(3.0 * loss, (hidden, weight))
+
+    h, w = hidden.detach().double().requires_grad_(), weight.detach().double().requires_grad_()
+    want = torch.nn.functional.cross_entropy(h @ w.t(), labels, ignore_index=-100)
+    wh, ww = torch.autograd.grad(3.0 * want, (h, w))
+    # the logits are rounded to bfloat16, at most ROUND of the largest each way, and a loss is a difference of two of them
+    top = (h @ w.t()).abs().max().item()
+    assert abs(loss.item() - want.item()) < 2 * ROUND * top
+    # a logit's rounding moves its probability by that share of it, and the gradient is rounded once more
+    assert _rel(dh, wh) < 2 * ROUND * (top + 1)
+    assert _rel(dw, ww) < 2 * ROUND * (top + 1)
+
+
+def test_cross_entropy_without_a_row_that_counts():
+    from colossalai_amd.ops.fused_ce import fused_linear_cross_entropy
+
+    hidden = torch.randn(9, 64, device="cuda").bfloat16().requires_grad_()
+    weight = torch.randn(80, 64, device="cuda").bfloat16().requires_grad_()
+    loss = fused_linear_cross_entropy(hidden, weight, torch.full((9,), -100, device="cuda"))
+    assert loss.item() == 0.0
+    assert all((g == 0).all() for g in torch.autograd.grad(loss, (hidden, weight)))
+
+
+@pytest.mark.parametrize("V", [64, 1003])
+def test_row_statistics_with_infinities(V):
+    from colossalai_amd.ops import kernels
+
+    x = torch.randn(5, V, device="cuda").bfloat16()
+    x[0, : V // 2] = float("-inf")
+    x[1, 3] = float("inf")
+    x[2] = float("-inf")
+    x[3] *= 300
+    labels = torch.tensor([V - 1, 0, 1, 2, -100], device="cuda")
+    lse, nll = torch.empty(5, device="cuda"), torch.empty(5, device="cuda")
+    kernels().ce_fwd(x, labels, -100, lse, nll)
+    want = torch.logsumexp(x.double(), 1)
+    # float32: a sum of V terms and the reference's own rounding
+    torch.testing.assert_close(lse.double(), want, rtol=V * 2.0 ** -24, atol=V * 2.0 ** -24)
+    assert nll[4] == 0 and nll[1] == float("inf") and torch.isnan(nll[2])
+    labels[0] = V  # outside the row: nothing is read there
+    kernels().ce_fwd(x, labels, -100, lse, nll)
+    assert torch.isnan(nll[0])

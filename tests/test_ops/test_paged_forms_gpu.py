@@ -1,7 +1,7 @@
 """Paged attention over the edges of its kernels: token and key tile remainders, sequences of a few tokens beside long
 ones, scales of either sign and zero, with and without the parts that put scores into the base-2 domain early.
 
-The bound: float32 scores and weights; the output is rounded to bfloat16 once (at most 2^-9 of a value) and a score
+The bound: float32 scores and weights; the output is rounded to bfloat16 once (at most 2^-8 of a value) and a score
 error of a few float32 roundings of the largest score moves a weight by less than that."""
 
 import pytest
