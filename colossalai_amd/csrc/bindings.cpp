@@ -26,8 +26,9 @@ void multi_tensor_sgd(std::vector<at::Tensor> grads, std::vector<at::Tensor> par
 // rmsnorm.hip
 std::vector<at::Tensor> rmsnorm_fwd(at::Tensor input, at::Tensor weight, double eps, bool save_inv_rms);
 std::vector<at::Tensor> rmsnorm_fused_add_fwd(at::Tensor input, at::Tensor residual, at::Tensor weight,
-                                              double eps, bool save_inv_rms);
-std::vector<at::Tensor> rmsnorm_bwd(at::Tensor dy, at::Tensor x, at::Tensor weight, at::Tensor inv_rms);
+                                              double eps, bool save_inv_rms, c10::optional<at::Tensor> res_out);
+std::vector<at::Tensor> rmsnorm_bwd(at::Tensor dy, at::Tensor x, at::Tensor weight, at::Tensor inv_rms,
+                                    c10::optional<at::Tensor> dres, bool cast_dw);
 
 // cross_entropy.hip
 void ce_fwd(at::Tensor logits, at::Tensor labels, int64_t ignore_index, at::Tensor lse, at::Tensor nll);
@@ -103,8 +104,10 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("multi_tensor_lamb", &cai::multi_tensor_lamb,
         "fused multi-tensor LAMB (two-stage: Adam update + trust-ratio scale)");
   m.def("rmsnorm_fwd", &cai::rmsnorm_fwd, "RMSNorm forward");
-  m.def("rmsnorm_fused_add_fwd", &cai::rmsnorm_fused_add_fwd, "fused residual-add RMSNorm forward");
-  m.def("rmsnorm_bwd", &cai::rmsnorm_bwd, "RMSNorm backward");
+  m.def("rmsnorm_fused_add_fwd", &cai::rmsnorm_fused_add_fwd, "fused residual-add RMSNorm forward", py::arg("input"),
+        py::arg("residual"), py::arg("weight"), py::arg("eps"), py::arg("save_inv_rms"), py::arg("res_out") = py::none());
+  m.def("rmsnorm_bwd", &cai::rmsnorm_bwd, "RMSNorm backward", py::arg("dy"), py::arg("x"), py::arg("weight"),
+        py::arg("inv_rms"), py::arg("dres") = py::none(), py::arg("cast_dw") = false);
   m.def("ce_fwd", &cai::ce_fwd, "cross entropy of bf16 logits: log-sum-exp and negative log likelihood per row");
   m.def("ce_bwd", &cai::ce_bwd, "cross entropy backward, logits -> their gradient in place");
   m.def("ce_loss", &cai::ce_loss, "mean negative log likelihood over the rows that are not ignored, and their number");

@@ -40,7 +40,7 @@ class _RMSNorm(torch.autograd.Function):
     def backward(ctx, dy):
         x, weight, inv_rms = ctx.saved_tensors
         if use_hip(x, weight, dy):
-            dx, dw = kernels().rmsnorm_bwd(dy.contiguous(), x, weight, inv_rms)
+            dx, dw = kernels().rmsnorm_bwd(dy.contiguous(), x, weight, inv_rms, None, True)
             return dx, dw.to(weight.dtype), None
         # CPU reference backward (fp32)
         xf, dyf, wf = x.float(), dy.float(), weight.float()
@@ -63,8 +63,9 @@ class _FusedAddRMSNorm(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, residual, weight, eps):
         if use_hip(x, residual, weight):
-            res = residual.contiguous().clone()  # kernel updates in place
-            out, inv_rms = kernels().rmsnorm_fused_add_fwd(x.contiguous(), res, weight.contiguous(), eps, True)
+            residual = residual.contiguous()
+            res = torch.empty_like(residual)
+            out, inv_rms = kernels().rmsnorm_fused_add_fwd(x.contiguous(), residual, weight.contiguous(), eps, True, res)
             ctx.save_for_backward(res, weight, inv_rms)
             ctx.eps = eps
             return out, res
@@ -77,8 +78,11 @@ class _FusedAddRMSNorm(torch.autograd.Function):
     def backward(ctx, dy, dres):
         h, weight, inv_rms = ctx.saved_tensors
         if use_hip(h, weight, dy):
-            dx, dw = kernels().rmsnorm_bwd(dy.contiguous(), h, weight, inv_rms)
-            dtotal = dx if dres is None else dx + dres
+            fused = dres is not None and dres.dtype == h.dtype  # the residual stream's gradient rides along
+            dtotal, dw = kernels().rmsnorm_bwd(dy.contiguous(), h, weight, inv_rms,
+                                               dres.contiguous() if fused else None, True)
+            if dres is not None and not fused:
+                dtotal = dtotal + dres
             return dtotal, dtotal, dw.to(weight.dtype), None
         hf, dyf, wf = h.float(), dy.float(), weight.float()
         H = h.shape[-1]

@@ -67,3 +67,35 @@ def test_row_statistics_with_infinities(V):
     labels[0] = V  # outside the row: nothing is read there
     kernels().ce_fwd(x, labels, -100, lse, nll)
     assert torch.isnan(nll[0])
+
+
+@pytest.mark.parametrize("rows,H", [(1, 8), (3, 512), (5, 520), (130, 768), (9, 1032), (33, 2048), (6, 2056), (7, 4104), (5, 8192),
+                                    (5000, 64)])
+def test_add_norm_and_its_gradients(rows, H):
+    from colossalai_amd.ops import fused_add_rms_norm, rms_norm
+
+    torch.manual_seed(0)
+    x, res, dy, dh = (torch.randn(rows, H, device="cuda").bfloat16() for _ in range(4))
+    w = (1 + 0.1 * torch.randn(H, device="cuda")).bfloat16()
+    for t in (x, res, w):
+        t.requires_grad_()
+    kept = res.detach().clone()
+    y, h = fused_add_rms_norm(x, res, w, 1e-5)
+    dx, dr, dw = torch.autograd.grad((y, h), (x, res, w), (dy, dh))
+    assert torch.equal(res.detach(), kept)  # the old residual stream is left alone
+
+    hf = (x.detach().float() + res.detach().float()).requires_grad_()
+    wf = w.detach().float().requires_grad_()
+    yf = hf * torch.rsqrt(hf.pow(2).mean(-1, keepdim=True) + 1e-5) * wf
+    gh, gw = torch.autograd.grad(yf, (hf, wf), dy.float())
+    assert _rel(h, hf) < ROUND and _rel(y, yf) < ROUND
+    # the backward starts from the rounded h: twice ROUND through the norm, and the result is rounded
+    assert _rel(dx, gh + dh.float()) < 3 * ROUND and torch.equal(dx, dr)
+    assert _rel(dw, gw) < 3 * ROUND
+
+    y = rms_norm(x, w, 1e-5)
+    (dx,) = torch.autograd.grad(y, (x,), dy)
+    xf = x.detach().float().requires_grad_()
+    yf = xf * torch.rsqrt(xf.pow(2).mean(-1, keepdim=True) + 1e-5) * w.detach().float()
+    (gx,) = torch.autograd.grad(yf, (xf,), dy.float())
+    assert _rel(y, yf) < ROUND and _rel(dx, gx) < 2 * ROUND
