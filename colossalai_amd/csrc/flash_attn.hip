@@ -3,12 +3,12 @@
 // MI355X-native design (not a CUDA port):
 //  - mfma_f32_32x32x16_bf16 tiles; 64-wide waves; a wave owns 32 query rows (forward,
 //    dQ) or 32 key/value rows (dK/dV); blocks of 4 waves, 2 for small forward grids.
-//  - ALL operand tiles live in LDS in ONE layout, column groups of 16 channels
+//  - ALL operand tiles live in LDS in ONE layout, planes of 8 channels
 //    (tile_off below). Row-slice fragment reads (8 consecutive d at a fixed row) are
 //    single 16 B loads; COLUMN fragment reads use gfx950's ds_read_b64_tr_b16.
 //    HW-verified semantics (mfma_selftest.hip): each lane reads 64 bits at its own
 //    address; within a 16-lane group, out[l][j] = pool[(l&15) + 16 j] where pool is
-//    the group's reads in lane order. With lane addressing row=(m>>2), byte=(m&3)*8
+//    the group's reads in lane order. With lane addressing row=(m>>2), channels (m&3)*4
 //    this delivers tile[row0+j][col m] per lane — a free 4x16 transpose.
 //  - No intermediate passes through LDS: every product whose operand is a result (P · V,
 //    P^T · dO, dS^T · Q, dS · K) is arranged so that the contracted index lies in a lane's
@@ -18,18 +18,19 @@
 //  - backward: delta preprocess, then ONE launch whose blocks take key/value tiles (dK/dV)
 //    or query tiles (dQ); both form the scores again.
 //
-// What bounds it (B2 S2048 H16/8 D128, not causal): the matrix unit is busy 41 % of the forward
-// and 43 % of the backward, the vector unit 40 %, LDS 40 % of the time. The two waves of a SIMD overlap
-// little of their products and exponentials; running them one phase apart with barriers (726 TFLOP/s),
-// forming the next tile's scores under the softmax (830 at 245 registers, 196 at D64 for want of waves) and
-// eight-wave blocks were measured against the 835 of this form.
+// What bounds it (B2 S2048 H16/8 D128, not causal): the matrix unit is busy 41 % of the forward and 43 % of the
+// backward, the vector unit 40 %. The two waves of a SIMD overlap little of their products and exponentials;
+// without the softmax the forward would run 1048 TFLOP/s, without global loads 1099, with neither 1337, at the 2.1 GHz
+// the card keeps under this load. Running the two waves one phase apart with barriers (726 TFLOP/s), forming the next
+// tile's scores under the softmax (830 at 245 registers, 196 at D64 for want of waves) and eight-wave blocks were
+// measured against the 835 of this form before the staging addresses became scalars.
 //
 // TFLOP/s, forward 2 products / backward 5 products of the visible pairs, before -> after:
-//   B4 S4096 H32 D128 causal          forward 694 -> 800, backward 498 -> 612
-//   B1 S8192 H32/8 D128 causal        forward 730 -> 917, backward 490 -> 668
-//   B8 S1024 H12 D64 causal           forward 215 -> 350, backward 225 -> 326
-//   B16 S512 H12 D64                  forward 361 -> 525, backward 294 -> 443
-//   packed, 10 sequences of 256..4096 forward 216 -> 695, backward 197 -> 573
+//   B4 S4096 H32 D128 causal          forward 694 -> 807, backward 498 -> 635
+//   B1 S8192 H32/8 D128 causal        forward 730 -> 972, backward 490 -> 686
+//   B8 S1024 H12 D64 causal           forward 215 -> 357, backward 225 -> 327
+//   B16 S512 H12 D64                  forward 361 -> 542, backward 294 -> 458
+//   packed, 10 sequences of 256..4096 forward 216 -> 714, backward 197 -> 584
 //
 // Shapes: q [B,S,Hq,D], k/v [B,S,Hkv,D] ("bshd" — no transposes in the
 // model), D in {64,128}. lse/delta are [B,Hq,S] fp32.
@@ -68,19 +69,19 @@ DEV_INLINE bf16x8_t ld_lds16(const char* lds, int byte) {
 // C-layout row for mfma_f32_32x32x16 register j (guide §3, HW-verified).
 DEV_INLINE constexpr int crow(int j, int half) { return (j & 3) + 8 * (j >> 2) + 4 * half; }
 
-// An operand tile in LDS: column groups of 16 channels, [D/16][ROWS][16], 32 bytes a row, 128 bytes
-// between the groups: a transposing read takes 128 contiguous bytes from each of two neighbouring
-// groups at a time, which then lie in different halves of the 64 banks. 16 bytes apart they collided: conflicts
-// were 49 % of the forward's active LDS cycles and are 37 % now, the rest in the row-slice reads. (Planes of 8
-// channels bring them to 16 % and no time: LDS is not what bounds these kernels.)
+// An operand tile in LDS: planes of 8 channels, [D/8][ROWS][8], 16 bytes a row, 64 bytes between the planes. Every
+// access spreads over the 64 banks: a row-slice fragment (ds_read_b128) reads 32 neighbouring rows of a plane per half-wave,
+// 512 contiguous bytes (4.3 cycles a wave; 8.5 with rows of 32 bytes); a transposing read takes 64 bytes from each
+// of four neighbouring planes at a time; a staging store writes 16 rows of four planes. Against column groups of 16
+// channels: forward 883 -> 917, backward 651 -> 656 TFLOP/s at B2 S2048 H16/8 D128.
 template <int ROWS>
-__host__ __device__ constexpr int tile_pitch() { return ROWS * 32 + 128; }
+__host__ __device__ constexpr int tile_pitch() { return ROWS * 16 + 64; }
 
 template <int ROWS>
-DEV_INLINE int tile_off(int row, int col) { return (col >> 4) * tile_pitch<ROWS>() + row * 32 + (col & 15) * 2; }
+DEV_INLINE int tile_off(int row, int col) { return (col >> 3) * tile_pitch<ROWS>() + row * 16 + (col & 7) * 2; }
 
 template <int ROWS, int COLS>
-__host__ __device__ constexpr int tile_bytes() { return (COLS / 16) * tile_pitch<ROWS>(); }
+__host__ __device__ constexpr int tile_bytes() { return (COLS / 8) * tile_pitch<ROWS>(); }
 
 // Column fragment by transposing reads, in the order in which the C layout hands out its rows: lane l
 // receives tile[k_base + 8*(e>>2) + 4*(l>>5) + (e&3)][cg_base*16 + (l&31)], e = 0..7, so
@@ -88,10 +89,10 @@ __host__ __device__ constexpr int tile_bytes() { return (COLS / 16) * tile_pitch
 template <int ROWS>
 DEV_INLINE bf16x8_t frag_born(const char* tile, int lane, int k_base, int cg_base) {
   const int m = lane & 15;
-  const int cg = cg_base + ((lane >> 4) & 1);
-  const int at = cg * tile_pitch<ROWS>() + (k_base + (lane >> 5) * 4 + (m >> 2)) * 32 + (m & 3) * 8;
+  const int plane = (cg_base + ((lane >> 4) & 1)) * 2 + ((m & 3) >> 1);
+  const int at = plane * tile_pitch<ROWS>() + (k_base + (lane >> 5) * 4 + (m >> 2)) * 16 + (m & 1) * 8;
   const bf16x4_v lo = ld_tr16(tile, at);
-  const bf16x4_v hi = ld_tr16(tile, at + 8 * 32);
+  const bf16x4_v hi = ld_tr16(tile, at + 8 * 16);
   return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
 }
 
@@ -116,45 +117,56 @@ DEV_INLINE int xcd_chunk(int f, int nblocks) {
   return (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + (f >> 3);
 }
 
-// Synchronous staging: load + store back-to-back (transient registers).
-template <int D, int ROWS, int NT_>
-DEV_INLINE void stage_direct(char* lds, const unsigned short* base, long stride, int row0, int S);
-
-// Register-staged tile for async-split staging (guide T14 / G15): global
-// loads for tile t+1 are ISSUED before tile t's compute (results land in
-// registers under the MFMAs), LDS writes happen after the barrier. NT_ must
-// divide ROWS*CPR.
+// Register-staged tile for async-split staging: global loads for tile t+1 are ISSUED before tile t's compute
+// (results land in registers under the MFMAs), LDS writes happen after it.
+//
+// A wave's instruction covers 16 rows of 64 bytes: with whole rows per instruction the stores of a row's column
+// groups met in the same LDS banks. Chunk i of a thread lies a fixed number of rows and columns from its
+// chunk 0, so that a whole tile's addresses are one offset per thread and scalars; only a tile that reaches past the last
+// row (or rows very far apart) forms an address per chunk. (Addresses of eight chunks, clamped and multiplied out for every tile, were a third of the
+// forward's vector instructions.)
 template <int D, int ROWS, int NT_>
 struct RegStage {
-  static constexpr int CPR = D / 8;
-  static constexpr int NCH = ROWS * CPR / NT_;
-  static_assert(ROWS * CPR % NT_ == 0, "RegStage: uneven chunking");
+  static constexpr int NCH = ROWS * (D / 8) / NT_;
+  static constexpr int WAVES = NT_ / 64, QUADS = D / 32;  // 64-byte pieces of a row
+  static_assert(ROWS * (D / 8) % NT_ == 0, "RegStage: uneven chunking");
+  static_assert(QUADS % WAVES == 0 || WAVES % QUADS == 0, "RegStage: chunks must lie at fixed distances");
   bf16x8_t r[NCH];
 
-  // A wave's instruction covers 16 rows of 64 bytes: with whole rows per instruction the stores
-  // of a row's column groups met in the same LDS banks.
-  DEV_INLINE static int row_of(int i) { return ((int)(threadIdx.x + i * NT_) / (CPR * 16)) * 16 + ((threadIdx.x & 63) >> 2); }
-  DEV_INLINE static int col_of(int i) {
-    return ((((int)(threadIdx.x + i * NT_) >> 6) % (CPR / 4)) * 4 + (threadIdx.x & 3)) * 8;
-  }
+  DEV_INLINE static constexpr int rows_to(int i) { return i * WAVES / QUADS * 16; }
+  DEV_INLINE static constexpr int cols_to(int i) { return i * WAVES % QUADS * 32; }
+  DEV_INLINE static int row0_of() { return (int)(threadIdx.x >> 6) / QUADS * 16 + (int)((threadIdx.x & 63) >> 2); }
+  DEV_INLINE static int col0_of() { return ((int)(threadIdx.x >> 6) % QUADS * 4 + (int)(threadIdx.x & 3)) * 8; }
 
-  DEV_INLINE void load(const unsigned short* base, long tok_stride, int row0, int S) {
+  // Bytes from a tile's first element to this thread's chunk 0, for rows less than 2^25 elements apart.
+  DEV_INLINE static unsigned offset(long tok_stride) { return (unsigned)(row0_of() * tok_stride + col0_of()) * 2u; }
+
+  DEV_INLINE void load(const unsigned short* base, long tok_stride, unsigned off, int row0, int S) {
+    if (row0 + ROWS <= S && tok_stride < (1L << 25)) {
 #pragma unroll
-    for (int i = 0; i < NCH; ++i) {
-      const int grow = max(min(row0 + row_of(i), S - 1), 0);
-      r[i] = ld_g16(base + (long)grow * tok_stride + col_of(i));
+      for (int i = 0; i < NCH; ++i)
+        r[i] = *reinterpret_cast<const bf16x8_t*>(
+            reinterpret_cast<const char*>(base + (row0 + rows_to(i)) * tok_stride + cols_to(i)) + off);
+    } else {
+#pragma unroll
+      for (int i = 0; i < NCH; ++i) {
+        const int grow = max(min(row0 + row0_of() + rows_to(i), S - 1), 0);
+        r[i] = ld_g16(base + (long)grow * tok_stride + col0_of() + cols_to(i));
+      }
     }
   }
   DEV_INLINE void store(char* lds) const {
+    char* at = lds + tile_off<ROWS>(row0_of(), col0_of());
 #pragma unroll
-    for (int i = 0; i < NCH; ++i) st_lds16(lds, tile_off<ROWS>(row_of(i), col_of(i)), r[i]);
+    for (int i = 0; i < NCH; ++i) st_lds16(at, tile_off<ROWS>(rows_to(i), cols_to(i)), r[i]);
   }
 };
 
+// Synchronous staging: load + store back-to-back (transient registers).
 template <int D, int ROWS, int NT_>
 DEV_INLINE void stage_direct(char* lds, const unsigned short* base, long stride, int row0, int S) {
   RegStage<D, ROWS, NT_> st;
-  st.load(base, stride, row0, S);
+  st.load(base, stride, st.offset(stride), row0, S);
   st.store(lds);
 }
 
@@ -345,20 +357,21 @@ __global__ __launch_bounds__(NW * 64, 2) void fa_fwd_kernel(
   };
 
   RegStage<D, KVB, NT> kstage, vstage;
+  const unsigned koff = kstage.offset(kts);
   f32x16 sc[KB];
   // async-split staging (T14): tile t+1's global loads issue before tile t's compute; their stores
   // target the OTHER buffer, so that one barrier a tile does
   // SeffK == 0 blocks skip the tile loop; the clamped loads stay in-bounds
-  kstage.load(k_base, kts, 0, SeffK);
-  vstage.load(v_base, kts, 0, SeffK);
+  kstage.load(k_base, kts, koff, 0, SeffK);
+  vstage.load(v_base, kts, koff, 0, SeffK);
   kstage.store(Kbuf);
   vstage.store(Vbuf);
   __syncthreads();
   for (int t = 0; t < kv_tiles; ++t) {
     const bool more = t + 1 < kv_tiles;
     if (more) {
-      kstage.load(k_base, kts, (t + 1) * KVB, SeffK);
-      vstage.load(v_base, kts, (t + 1) * KVB, SeffK);
+      kstage.load(k_base, kts, koff, (t + 1) * KVB, SeffK);
+      vstage.load(v_base, kts, koff, (t + 1) * KVB, SeffK);
     }
     if (t < my_tiles) {
       __builtin_amdgcn_s_setprio(1);
@@ -541,6 +554,7 @@ DEV_INLINE void bwd_dkdv(
   const float scale2 = scale * 1.44269504f;
 
   RegStage<D, QB, NTB> qstage, dostage;
+  const unsigned qoff = qstage.offset(qts), dooff = dostage.offset(do_stride);
   float lse_r = 0.0f, dta_r = 0.0f;
   auto fetch = [&](int step) {   // global loads of a step's query tile
     const int h = hk * (Hq / Hkv) + part * G + step / nq;
@@ -548,8 +562,8 @@ DEV_INLINE void bwd_dkdv(
     const unsigned short* q_base = VARLEN ? Q + seq0 * qts + (long)h * D : Q + (long)b * qbs + (long)h * D;
     const unsigned short* do_base =
         VARLEN ? dO + (seq0 * Hq + h) * D : dO + ((long)b * S * Hq + h) * D;  // dO packed
-    qstage.load(q_base, qts, qt0, Seff);
-    dostage.load(do_base, do_stride, qt0, Seff);
+    qstage.load(q_base, qts, qoff, qt0, Seff);
+    dostage.load(do_base, do_stride, dooff, qt0, Seff);
     if (threadIdx.x < QB) {
       const long at = (VARLEN ? (long)h * S + seq0 : ((long)b * Hq + h) * S) + min(qt0 + (int)threadIdx.x, Seff - 1);
       lse_r = qt0 + (int)threadIdx.x < Seff ? LSE[at] : -INFINITY;
@@ -733,9 +747,10 @@ DEV_INLINE void bwd_dq(
   const int kv_tiles = q0 >= Seff ? 0 : (causal ? min(kv_tiles_all, (min(q0 + NWB * QW, Seff) + KVB - 1) / KVB) : kv_tiles_all);
 
   RegStage<D, KVB, NTB> kstage, vstage;
+  const unsigned koff = kstage.offset(kts);
   if (kv_tiles > 0) {
-    kstage.load(k_base, kts, 0, SeffK);
-    vstage.load(v_base, kts, 0, SeffK);
+    kstage.load(k_base, kts, koff, 0, SeffK);
+    vstage.load(v_base, kts, koff, 0, SeffK);
     kstage.store(Kbuf);
     vstage.store(Vbuf);
   }
@@ -745,8 +760,8 @@ DEV_INLINE void bwd_dq(
     const int k0 = t * KVB, buf = t & 1;
     const bool more = t + 1 < kv_tiles;
     if (more) {
-      kstage.load(k_base, kts, k0 + KVB, SeffK);
-      vstage.load(v_base, kts, k0 + KVB, SeffK);
+      kstage.load(k_base, kts, koff, k0 + KVB, SeffK);
+      vstage.load(v_base, kts, koff, k0 + KVB, SeffK);
     }
     const char* Klds = Kbuf + buf * TB;
     const char* Vlds = Vbuf + buf * TB;
