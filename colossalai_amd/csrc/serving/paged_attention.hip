@@ -295,63 +295,84 @@ __global__ __launch_bounds__(64 * ATT_WAVES) void paged_attention_kernel(
 //   S^T = K Q^T   (A = key rows from LDS, B = query rows kept in registers)
 //   O^T = V^T P^T (B = the float32 weights in the C layout they were born in, split into a
 //                  high and a low bfloat16 half so that no weight loses its float32 mantissa
-//                  to the matrix unit; A = values, stored transposed in LDS in the same key
-//                  order, one 16-byte read per product)
+//                  to the matrix unit; A = values, read from LDS with the transposing
+//                  64-bit read in the same key order)
 // so column = token = lane & 31 everywhere: running max, running sum, rescaling and the gate
 // never cross lanes except for one exchange between the two half-waves.
 // The tiles are DS * 16 key channels by VT * 32 value channels; a head whose sizes Dr / Dvr are
 // smaller (multiples of 8) is padded with zeros on its way into registers and LDS, and only its
 // own channels are stored.
-template <int DS, int VT>
-__global__ __launch_bounds__(256, 2) void paged_attention_mfma_kernel(
+// What bounds it: the waits of a step. Of a wave's time 38 % are waits (LDS operands, the barrier of a step, page
+// lookups), the matrix units are busy a fifth and the vector units a quarter; registers (253 of 256 at 128 channels)
+// allow two blocks a CU and no deeper pipeline. One 4096-token prompt, 16 heads on 4 of 128, page 64:
+// 594 us with rows swizzled and a lookup for each 16 bytes, 275 with two tiles a softmax, 204 with the planes, two
+// lookups a lane and tile, and the grid by XCD (64 channels, 16 heads on 8: 654, 342, 177; a cap and a sink: 605, 302,
+// 238; 16 heads of one key head each: 631, 277, 204).
+// Reading operands six ahead of the products changed nothing (203 us), lookups through scalar loads cost (416 us: their
+// counter is the LDS reads' own).
+template <int DS, int VT, int NG>
+__global__ __launch_bounds__(256 * NG, 2) void paged_attention_mfma_kernel(
     bf16s* __restrict__ out, const bf16s* __restrict__ q, long q_stride, const bf16s* __restrict__ kpool,
     const bf16s* __restrict__ vpool, const int* __restrict__ block_tables, int bt_stride, const int* __restrict__ cu,
     const int* __restrict__ start, const float* __restrict__ slopes, const bf16s* __restrict__ gate, long gate_stride,
     int H, int G, int Dr, int Dvr, int page_shift, float scale, int window, int keep_first, float softcap, int sink,
     int qsplit, const float* __restrict__ sink2, const float* __restrict__ dist2, int dist_rows,
     const bf16s* __restrict__ ksum, const bf16s* __restrict__ vsum, int sum_shift, int sum_block,
-    float* __restrict__ cross_out, int chunk, const float* __restrict__ key_fac, int vrep, float* __restrict__ out32) {
+    float* __restrict__ cross_out, int chunk, const float* __restrict__ key_fac, int vrep, float* __restrict__ out32,
+    int num_tiles) {
   // The optional extras of the split-key kernel, in the base-2 domain: sink2 [H] = learned sink scores * log2e;
   // dist2 [H, dist_rows] = the per-distance bias * log2e, one row per head; ksum / vsum = block summaries, staged as
   // the first tiles of a block (summary idx of a sequence is seen by a token at pos when idx < (pos - window + 1) /
-  // sum_block); cross_out [N, H, G, Dv] float32: the grid's z axis then also counts the kv head whose values a block
+  // sum_block); cross_out [N, H, G, Dv] float32: a row is then also the kv head whose values a block
   // multiplies the weights with; chunk, key_fac [pool rows, G], vrep and out32 as in the split-key kernel (the factors of
   // a key tile are staged with it).
   // qsplit (kv heads with a single query head each): the four waves of a block are four consecutive 32-token tiles
-  // of that head instead of four heads, so a block covers 128 tokens, the grid's x axis counts 128-token tiles, and
+  // of that head instead of four heads, so a block covers 128 tokens, a tile is 128 tokens, and
   // the staged key/value tiles are still shared by all computing waves. The block stages the key range of all its
   // tokens; a wave skips the tiles that lie wholly after its own tokens.
   constexpr int D = DS * 16, Dv = VT * 32;
   bf16x8_v zero8;
 #pragma unroll
   for (int e = 0; e < 8; ++e) zero8[e] = (__bf16)0.0f;
-  constexpr int KP = D + 8;            // key row pitch in LDS (elements): 16-byte reads of 16 rows hit 64 banks
-  // Values are staged as they come, in column groups of 16 channels ([Dv / 16][32 keys][16], 32 bytes a key, 128
-  // bytes between the groups), and read as columns by transposing reads: a read takes 128 contiguous bytes
-  // from each of two neighbouring groups at a time, in different halves of the banks.
-  constexpr int VG = 32 * 16 + 64;             // elements of a group
-  constexpr int KT = 32 * KP, VTT = Dv / 16 * VG;   // elements of one staged tile
-  constexpr int KCH = 32 * D / 8, VCH = 32 * Dv / 8;  // 16-byte chunks of a key / value tile
-  constexpr int TP = MFMA_TILES_PER_STEP;
-  extern __shared__ __align__(16) bf16s tiles[];  // [2][TP][KT + VTT], then [2][TP][32] key factors (float)
-  float* facs = reinterpret_cast<float*>(tiles + 2 * TP * (KT + VTT));
-  constexpr int nthreads = 256;  // always four waves: those beyond the group's heads only help staging
-  const int tid = threadIdx.x;
+  // A staged tile: planes of 8 channels, [D / 8][32 keys][8], 16 bytes a key, 64 bytes between the planes, keys and
+  // values alike. Row reads take 512 contiguous bytes per half-wave, the transposing reads of the values 64 bytes
+  // from each of four planes at a time, staging stores 16 keys of four planes: none of them meets in a bank.
+  constexpr int PL = 32 * 8 + 32;              // elements of a plane
+  constexpr int KT = D / 8 * PL, VTT = Dv / 8 * PL;   // elements of one staged tile
+  constexpr int TP = MFMA_TILES_PER_STEP, TS = NG * TP;   // tiles of a step: a group's, the block's
+  extern __shared__ __align__(16) bf16s tiles[];  // [2][TS][KT + VTT], then [2][TS][32] key factors (float)
+  float* facs = reinterpret_cast<float*>(tiles + 2 * TS * (KT + VTT));
+  constexpr int nthreads = 256;  // of a group, always four waves: those beyond the kv head's group of heads only help staging
+  const int tid = threadIdx.x & 255, grp = NG > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 8) : 0;
   const int wid = tid >> 6, lane = tid & 63;
-  const int rep = H / G, g = blockIdx.y;
+  const int rep = H / G;
   const int VC = cross_out != nullptr ? G : 1;
-  const int vg = cross_out != nullptr ? (int)(blockIdx.z % VC) : g / vrep;   // kv head of the values
+  // Which (tile, row of kv head x pass) this block is. Block f runs on XCD f % 8: with rows that divide 8 or are a
+  // multiple of it a row's keys and values stay in as few L2s as possible (4 kv heads: two XCDs a head, every second
+  // tile each). Under a causal mask a late tile of a long prompt has many more key tiles than an early one: late ones
+  // start first, and where all blocks of an XCD (32 CUs, two blocks each) run at once, the second 32 go the other way, so
+  // that a CU's two blocks are a long and a short one.
+  const int f = blockIdx.x, rows = G * ((rep + 3) / 4) * VC;
+  int row, tile, b = 0;
+  if (rows <= 8 && 8 % rows == 0) {
+    const int sub = 8 / rows, xcd = f & 7, i = f >> 3, per = (num_tiles + sub - 1) / sub;   // tiles of a row on this XCD
+    const int k = per <= 64 && i >= 32 ? i - 32 : per - 1 - i;
+    row = xcd % rows;
+    tile = k * sub + xcd / rows;
+    if (tile >= num_tiles) return;
+  } else {  // a row's tiles all go one way, every second row's the other way where all blocks run at once
+    const bool by8 = rows % 8 == 0;
+    const int at = by8 ? f >> 3 : f, turn = at / num_tiles, i = at - turn * num_tiles;
+    row = by8 ? (f & 7) + 8 * turn : turn;
+    tile = num_tiles * rows <= 512 && (turn & 1) ? i : num_tiles - 1 - i;
+  }
+  const int g = row % G, zrow = row / G;
+  const int vg = cross_out != nullptr ? zrow % VC : g / vrep;   // kv head of the values
   const int Gv = G / vrep;
-  const int hl = qsplit ? 0 : (blockIdx.z / VC) * (nthreads >> 6) + wid;  // head inside the group
+  const int hl = qsplit ? 0 : (zrow / VC) * (nthreads >> 6) + wid;  // head inside the group
   const int h = g * rep + (hl < rep ? hl : 0);
   const int bshift = qsplit ? 7 : 5;                  // log2 of the tokens a block covers
-  // Under a causal mask a late tile of a long prompt has many more key tiles than an early one. Rows of the grid
-  // (kv head, pass) walk the tiles alternately from the back and from the front, switching with every 256 blocks of
-  // dispatch order, so that blocks which come to share a CU tend to pair a long tile with a short one and the
-  // longest tiles start first.
-  const bool from_back = ((gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z)) >> 8 & 1) == 0;
-  int tile = from_back ? gridDim.x - 1 - blockIdx.x : blockIdx.x, b = 0;
-  for (;; ++b) {  // the grid holds exactly sum_b ceil(count_b / tokens per block) tiles
+  for (;; ++b) {  // there are exactly sum_b ceil(count_b / tokens per block) tiles
     const int nt = (cu[b + 1] - cu[b] + (1 << bshift) - 1) >> bshift;
     if (tile < nt) break;
     tile -= nt;
@@ -395,70 +416,61 @@ __global__ __launch_bounds__(256, 2) void paged_attention_mfma_kernel(
   const int my_sum = (ksum != nullptr && window > 0) ? max(0, (pos - window + 1) / sum_block) : 0;  // this token's
   const float* db = dist2 != nullptr ? dist2 + (long)h * dist_rows : nullptr;
 
-  // staging: key chunk c = key c / (row chunks), 8 elements starting at 8 * (c % row chunks), stored as a row; a wave's
-  // load of values covers 16 keys of 32 channels, so that its stores spread over the LDS banks
-  constexpr int KR = (KCH + 255) / 256, VR = (VCH + 255) / 256;  // chunks per thread of the 256
+  // Staging: a wave's load covers 16 keys of 32 channels (4 lanes a key), load u = wave + 4 r of a tile the quad u % quads
+  // of the 16 keys u / quads, for keys and values alike: a lane looks up two keys of a tile.
+  constexpr int KQ = (D + 31) / 32, VQ = VT;               // quads of a row
+  constexpr int KR = (2 * KQ + 3) / 4, VR = (2 * VQ + 3) / 4;  // loads per wave and tile
+  const int wv = __builtin_amdgcn_readfirstlane(wid) & 3;
+  const int lkey = lane >> 2, lch = (lane & 3) * 8;        // this lane's key of the 16 and channel of the 32
   // TP key tiles are staged, and multiplied, between two barriers: their loads are all in flight over the
   // products of the TP tiles before them
   bf16x8_v rk[TP][KR], rv[TP][VR];
-  auto v_key = [&](int c) { return (c / (64 * VT)) * 16 + ((c & 63) >> 2); };
-  auto v_chunk = [&](int c) { return (c >> 6) % VT * 4 + (c & 3); };
   auto tile_base = [&](int it) {
     return it < sum_tiles ? it * 32 : it < sink_tiles ? (it - sum_tiles) * 32 : wstart + (it - sink_tiles) * 32;
   };
   auto pool_row = [&](int j) {
     const int jc = min(j, bp1);  // keys past the sequence's end are masked; read a row that exists
-    return ((long)bt[jc >> page_shift] << page_shift) + (jc & page_mask);
+    return (bt[jc >> page_shift] << page_shift) + (jc & page_mask);
   };
   auto sum_row = [&](int idx) {
     const int ic = min(idx, n_sum - 1);  // a summary tile exists only when n_sum > 0
-    return ((long)bt[ic >> sum_shift] << sum_shift) + (ic & sum_mask);
+    return (bt[ic >> sum_shift] << sum_shift) + (ic & sum_mask);
   };
-  // The page-table lookups of a tile run one tile ahead of its key/value loads (two ahead of its use), so that a
+  // The page-table lookups of a tile run one step ahead of its key/value loads (two ahead of its use), so that a
   // load's address never waits for a lookup issued in the same iteration.
-  int krow[TP][KR], vrow[TP][VR], frow[TP];
+  const bool full = Dr == D && Dvr == Dv;
+  const unsigned krs = (unsigned)(G * Dr) * 2u, vrs = (unsigned)(Gv * Dvr) * 2u;   // bytes between neighbouring keys' rows
+  int krow[TP][2], frow[TP];
   float rf[TP];
   bool from_sum[TP];  // the tiles of the last lookup that are summary tiles
   auto lookup = [&](int step) {
 #pragma unroll
     for (int u = 0; u < TP; ++u) {
-      const int kbase = tile_base(step * TP + u);  // a tile past the last one reads rows that exist and is not used
-      from_sum[u] = step * TP + u < sum_tiles;
+      const int it = step * TS + grp * TP + u, kbase = tile_base(it);  // a tile past the last one reads rows that exist and is not used
+      from_sum[u] = it < sum_tiles;
 #pragma unroll
-      for (int r = 0; r < KR; ++r) {
-        const int c = tid + nthreads * r;
-        const int j = kbase + c / (D / 8);
-        krow[u][r] = c < KCH ? (int)(from_sum[u] ? sum_row(j) : pool_row(j)) : 0;
-      }
-#pragma unroll
-      for (int r = 0; r < VR; ++r) {
-        const int c = tid + nthreads * r;
-        const int j = kbase + v_key(c);
-        vrow[u][r] = c < VCH ? (int)(from_sum[u] ? sum_row(j) : pool_row(j)) : 0;
-      }
-      if (key_fac != nullptr && tid < 32) frow[u] = (int)pool_row(kbase + tid);
+      for (int i = 0; i < 2; ++i) krow[u][i] = from_sum[u] ? sum_row(kbase + 16 * i + lkey) : pool_row(kbase + 16 * i + lkey);
+      if (key_fac != nullptr && tid < 32) frow[u] = pool_row(kbase + tid);
     }
   };
-  auto fetch = [&]() {  // the tiles whose rows the last lookup left in krow / vrow
+  auto fetch = [&]() {  // the tiles that the last lookup found
 #pragma unroll
     for (int u = 0; u < TP; ++u) {
-      const bf16s* kp = from_sum[u] ? ksum : kpool;
-      const bf16s* vp = from_sum[u] ? vsum : vpool;
+      const char* kp = reinterpret_cast<const char*>((from_sum[u] ? ksum : kpool) + (long)g * Dr + lch);
+      const char* vp = reinterpret_cast<const char*>((from_sum[u] ? vsum : vpool) + (long)vg * Dvr + lch);
 #pragma unroll
       for (int r = 0; r < KR; ++r) {
-        const int c = tid + nthreads * r;
-        if (c < KCH) {
-          const int off = 8 * (c % (D / 8));
-          rk[u][r] = off < Dr ? ld_g16b(kp + ((long)krow[u][r] * G + g) * Dr + off) : zero8;
-        }
+        const int q_ = (wv + 4 * r) % KQ, i = (wv + 4 * r) / KQ;   // quad, group of 16 keys
+        if (2 * KQ % 4 != 0 && i > 1) continue;
+        const char* at = kp + q_ * 64 + (unsigned long)(unsigned)(i ? krow[u][1] : krow[u][0]) * krs;
+        rk[u][r] = full || q_ * 32 + lch < Dr ? *reinterpret_cast<const bf16x8_v*>(at) : zero8;
       }
 #pragma unroll
       for (int r = 0; r < VR; ++r) {
-        const int c = tid + nthreads * r;
-        if (c < VCH) {
-          const int off = 8 * v_chunk(c);
-          rv[u][r] = off < Dvr ? ld_g16b(vp + ((long)vrow[u][r] * Gv + vg) * Dvr + off) : zero8;
-        }
+        const int q_ = (wv + 4 * r) % VQ, i = (wv + 4 * r) / VQ;
+        if (2 * VQ % 4 != 0 && i > 1) continue;
+        const char* at = vp + q_ * 64 + (unsigned long)(unsigned)(i ? krow[u][1] : krow[u][0]) * vrs;
+        rv[u][r] = full || q_ * 32 + lch < Dvr ? *reinterpret_cast<const bf16x8_v*>(at) : zero8;
       }
       if (key_fac != nullptr && tid < 32) rf[u] = key_fac[(long)frow[u] * G + g];
     }
@@ -466,22 +478,21 @@ __global__ __launch_bounds__(256, 2) void paged_attention_mfma_kernel(
   auto stash = [&](int buf) {
 #pragma unroll
     for (int u = 0; u < TP; ++u) {
-      bf16s* ks = tiles + (buf * TP + u) * (KT + VTT);
+      bf16s* ks = tiles + (buf * TS + grp * TP + u) * (KT + VTT);
       bf16s* vt = ks + KT;
 #pragma unroll
       for (int r = 0; r < KR; ++r) {
-        const int c = tid + nthreads * r;
-        if (c < KCH) *reinterpret_cast<bf16x8_v*>(ks + (c / (D / 8)) * KP + 8 * (c % (D / 8))) = rk[u][r];
+        const int q_ = (wv + 4 * r) % KQ, i = (wv + 4 * r) / KQ;
+        if (i > 1 || q_ * 32 + lch >= D) continue;
+        *reinterpret_cast<bf16x8_v*>(ks + (q_ * 4 + (lane & 3)) * PL + (16 * i + lkey) * 8) = rk[u][r];
       }
 #pragma unroll
       for (int r = 0; r < VR; ++r) {
-        const int c = tid + nthreads * r;
-        if (c < VCH) {
-          const int ch = v_chunk(c);
-          *reinterpret_cast<bf16x8_v*>(vt + (ch >> 1) * VG + v_key(c) * 16 + (ch & 1) * 8) = rv[u][r];
-        }
+        const int q_ = (wv + 4 * r) % VQ, i = (wv + 4 * r) / VQ;
+        if (i > 1) continue;
+        *reinterpret_cast<bf16x8_v*>(vt + (q_ * 4 + (lane & 3)) * PL + (16 * i + lkey) * 8) = rv[u][r];
       }
-      if (key_fac != nullptr && tid < 32) facs[(buf * TP + u) * 32 + tid] = rf[u];
+      if (key_fac != nullptr && tid < 32) facs[(buf * TS + grp * TP + u) * 32 + tid] = rf[u];
     }
   };
 
@@ -500,6 +511,7 @@ __global__ __launch_bounds__(256, 2) void paged_attention_mfma_kernel(
   const float c1 = fmaxf(scale * LOG2E, 1e-30f), sl2 = slope * LOG2E;  // a scale of 0 must not meet -inf in a product
   // soft cap in the base-2 domain: cap log2e tanh(x scale / cap), tanh(y) = 1 - 2 / (exp2(2 log2e y) + 1)
   const bool capped = softcap > 0.0f;
+  const float inv_cap = capped ? scale / softcap : 0.0f;
   const float cap2 = softcap * LOG2E, t2 = capped ? 2.0f * LOG2E * scale / softcap : 0.0f;
   auto cap_base2 = [&](float dot) {
     const float e = __builtin_amdgcn_exp2f(fminf(dot * t2, 64.0f));  // beyond 2^64 the quotient is 0 in float32 anyway
@@ -515,7 +527,7 @@ __global__ __launch_bounds__(256, 2) void paged_attention_mfma_kernel(
   const bool raw = !capped && !sloped && db == nullptr;
   const float k1 = raw ? c1 : 1.0f;
 
-  const int steps_n = (tiles_n + TP - 1) / TP;
+  const int steps_n = (tiles_n + TS - 1) / TS;
   lookup(0);
   fetch();
   if (steps_n > 1) lookup(1);
@@ -529,14 +541,19 @@ __global__ __launch_bounds__(256, 2) void paged_attention_mfma_kernel(
       if (step + 2 < steps_n) lookup(step + 2);
     }
     // The TP tiles of a step go through the softmax together: one maximum, one exchange, one look at the rescaling.
+    const int it0 = step * TS + grp * TP, kb0 = tile_base(it0);
+    // interior step: every key of its tiles is visible to every token of the wave, no masks to evaluate
+    const bool inner = head_ok && it0 >= sink_tiles && kb0 >= lo_p1 && kb0 + 32 * TP - 1 <= p0 && t_off + 31 < cnt;
     bool live[TP];       // this wave sees something of the tile
-    bool any = false;
+    bool any = inner;
+    if (!inner) {
 #pragma unroll
-    for (int u = 0; u < TP; ++u) {
-      const int it = step * TP + u, kbase = tile_base(it);
-      // (query split) a tile wholly after this wave's tokens, or wholly before what they see
-      live[u] = head_ok && it < tiles_n && (it < sink_tiles || !(kbase > p1 || (kbase + 31 < lo_p0 && kbase >= keep_first)));
-      any = any || live[u];
+      for (int u = 0; u < TP; ++u) {
+        const int it = it0 + u, kbase = tile_base(it);
+        // (query split) a tile wholly after this wave's tokens, or wholly before what they see
+        live[u] = head_ok && it < tiles_n && (it < sink_tiles || !(kbase > p1 || (kbase + 31 < lo_p0 && kbase >= keep_first)));
+        any = any || live[u];
+      }
     }
     if (any) {
       f32x16 x[TP];
@@ -551,17 +568,17 @@ __global__ __launch_bounds__(256, 2) void paged_attention_mfma_kernel(
 #pragma unroll
         for (int u = 0; u < TP; ++u) {
           const bf16x8_v kf =
-              *reinterpret_cast<const bf16x8_v*>(tiles + (buf * TP + u) * (KT + VTT) + col * KP + 16 * s + hf * 8);
+              *reinterpret_cast<const bf16x8_v*>(tiles + (buf * TS + grp * TP + u) * (KT + VTT) + (2 * s + hf) * PL + col * 8);
           x[u] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, qf[s], x[u], 0, 0, 0);
         }
       __builtin_amdgcn_s_setprio(0);
 #pragma unroll
       for (int u = 0; u < TP; ++u) {
-        const int it = step * TP + u, kbase = tile_base(it);
-        const bool summ = it < sum_tiles;
+        const int it = it0 + u, kbase = inner ? kb0 + 32 * u : tile_base(it);
+        const bool summ = !inner && it < sum_tiles;
         const bool ahead = it < sink_tiles;  // a tile ahead of the window's: summaries or kept first tokens
         if (key_fac != nullptr) {
-          const float* fc = facs + (buf * TP + u) * 32 + 4 * hf;
+          const float* fc = facs + (buf * TS + grp * TP + u) * 32 + 4 * hf;
 #pragma unroll
           for (int a = 0; a < 4; ++a) {
             const float4v f4 = *reinterpret_cast<const float4v*>(fc + 8 * a);
@@ -572,8 +589,21 @@ __global__ __launch_bounds__(256, 2) void paged_attention_mfma_kernel(
         off[u] = sloped && !summ ? -sl2 * (float)(pos - kbase) : 0.0f;
         if (!raw) {
           if (capped) {
+            // tanh(y) = y P(y^2) for |y| <= 1/2, P a polynomial through the Chebyshev nodes (1.3e-8 off): six fused
+            // multiplications where the general form takes an exponential and a reciprocal
+            float far = 0.0f;
 #pragma unroll
-            for (int i = 0; i < 16; ++i) x[u][i] = cap_base2(x[u][i]);
+            for (int i = 0; i < 16; ++i) far = fmaxf(far, fabsf(x[u][i]));
+            if (__all(far * inv_cap <= 0.5f)) {
+#pragma unroll
+              for (int i = 0; i < 16; ++i) {
+                const float y = x[u][i] * inv_cap, z = y * y;
+                x[u][i] = cap2 * y * fmaf(z, fmaf(z, fmaf(z, fmaf(z, 0.017131345f, -0.052984238f), 0.13324751f), -0.33333069f), 1.0f);
+              }
+            } else {
+#pragma unroll
+              for (int i = 0; i < 16; ++i) x[u][i] = cap_base2(x[u][i]);
+            }
             if (sloped && !summ) {
 #pragma unroll
               for (int i = 0; i < 16; ++i) x[u][i] += row_bias[i];
@@ -593,9 +623,7 @@ __global__ __launch_bounds__(256, 2) void paged_attention_mfma_kernel(
             }
           }
         }
-        // interior tile: every key is visible to every token of the wave, no masks to evaluate
-        const bool interior = live[u] && !ahead && t_off + 31 < cnt && kbase + 31 <= p0 && kbase >= lo_p1;
-        if (!interior) {
+        if (!inner) {
           const int klimit = !live[u] ? 0 : ahead ? n_sink : p1 + 1;  // keys of this tile at or above it are not its to count
 #pragma unroll
           for (int i = 0; i < 16; ++i) {
@@ -657,10 +685,11 @@ __global__ __launch_bounds__(256, 2) void paged_attention_mfma_kernel(
         for (int s2 = 0; s2 < 2; ++s2)
 #pragma unroll
           for (int t = 0; t < VT; ++t) {
-            const bf16s* vp = tiles + (buf * TP + u) * (KT + VTT) + KT + (2 * t + ((lane >> 4) & 1)) * VG +
-                              (16 * s2 + 4 * hf + ((lane & 15) >> 2)) * 16 + (lane & 3) * 4;
+            const bf16s* vp = tiles + (buf * TS + grp * TP + u) * (KT + VTT) + KT +
+                              (4 * t + 2 * ((lane >> 4) & 1) + ((lane & 3) >> 1)) * PL +
+                              (16 * s2 + 4 * hf + ((lane & 15) >> 2)) * 8 + (lane & 1) * 4;
             const bf16x4_v v0 = ld_tr16(reinterpret_cast<const char*>(vp), 0);
-            const bf16x4_v v1 = ld_tr16(reinterpret_cast<const char*>(vp), 8 * 32);
+            const bf16x4_v v1 = ld_tr16(reinterpret_cast<const char*>(vp), 8 * 16);
             const bf16x8_v va = __builtin_shufflevector(v0, v1, 0, 1, 2, 3, 4, 5, 6, 7);
             oacc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va, phi[u][s2], oacc[t], 0, 0, 0);
             oacc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va, plo[u][s2], oacc[t], 0, 0, 0);
@@ -669,6 +698,28 @@ __global__ __launch_bounds__(256, 2) void paged_attention_mfma_kernel(
     }
     if (more) stash(buf ^ 1);
     __syncthreads();
+  }
+  if constexpr (NG > 1) {  // the second group's states, wave by wave, through the tiles' place (all waves are past their last tile)
+    float* state = reinterpret_cast<float*>(tiles) + wid * (VT * 16 + 2) * 64 + lane;
+    if (grp == 1) {
+      state[0] = m;
+      state[64] = l;
+#pragma unroll
+      for (int t = 0; t < VT; ++t)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) state[(2 + t * 16 + i) * 64] = oacc[t][i];
+    }
+    __syncthreads();
+    if (grp == 1) return;
+    const float m1 = state[0], top = fmaxf(m, m1);
+    const float f0 = m == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m - top);
+    const float f1 = m1 == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m1 - top);
+    l = l * f0 + state[64] * f1;
+#pragma unroll
+    for (int t = 0; t < VT; ++t)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) oacc[t][i] = oacc[t][i] * f0 + state[(2 + t * 16 + i) * 64] * f1;
+    m = top;
   }
   l += __shfl_xor(l, 32);
   if (sink2 != nullptr) l += __builtin_amdgcn_exp2f(sink2[h] - m);  // a learned score; a sink far above every key: 1 / inf = 0
@@ -775,16 +826,26 @@ static bool launch_mfma_attention(at::Tensor& out, const at::Tensor& q, const at
     // one query head per kv head: the waves of a block take four consecutive token tiles instead of four heads
     const int qsplit = (rep == 1 && num_tiles128 > 0) ? 1 : 0;
     const int VC = x.cross_out != nullptr ? G : 1;
-    const dim3 grid((unsigned)(qsplit ? num_tiles128 : num_tiles), (unsigned)G, (unsigned)((rep + nw - 1) / nw * VC));
+    const int tiles = (int)(qsplit ? num_tiles128 : num_tiles), rows = G * ((rep + nw - 1) / nw) * VC;
+    const int sub = rows <= 8 && 8 % rows == 0 ? 8 / rows : 1;   // XCDs a row's tiles are spread over: whole rounds of them
+    const dim3 grid((unsigned)((tiles + sub - 1) / sub * sub * rows));
     const int ds = D <= 32 ? 2 : D <= 48 ? 3 : D <= 64 ? 4 : D <= 96 ? 6 : 8, vt = (Dv + 31) / 32;
-    const size_t msmem = (size_t)2 * MFMA_TILES_PER_STEP *
-                         ((32 * (ds * 16 + 8) + vt * 2 * (32 * 16 + 64)) * sizeof(bf16s) + (x.key_fac != nullptr ? 32 * sizeof(float) : 0));
-#define MFMA_CASE(DS_, VT_)                                                                                        \
+    // Two groups of waves take alternate key tiles where one block a CU is all there is: a second group then fills the
+    // idle half of the CU, and a lone block's chain of tiles is half as long. Measured, one group against two: 2 x 256
+    // tokens 31 -> 23 us (64 blocks), 3 x 200 after 1500 207 -> 130 (84), 100 alone 18 -> 15 (16). With 512 blocks it is mixed: 4 x 1000 117 -> 95 and
+    // 4096 tokens 205 -> 197, but 204 -> 226 with 16 key heads, 87 -> 107 with a window of 1024; beyond that it loses
+    // (16 x 1024, 2048 blocks: 175 -> 182; 4096 of 64 heads, 2048 blocks: 507 -> 572).
+    const int ng = grid.x <= 256 ? 2 : 1;
+    const size_t msmem = (size_t)2 * ng * MFMA_TILES_PER_STEP *
+                         ((ds * 2 + vt * 4) * (32 * 8 + 32) * sizeof(bf16s) + (x.key_fac != nullptr ? 32 * sizeof(float) : 0));
+#define MFMA_CASE(DS_, VT_) \
+  do { if (ng == 2) MFMA_NG(DS_, VT_, 2); else MFMA_NG(DS_, VT_, 1); } while (0)
+#define MFMA_NG(DS_, VT_, NG_)                                                                                     \
   do {                                                                                                             \
-    auto kfn = paged_attention_mfma_kernel<DS_, VT_>;                                                              \
+    auto kfn = paged_attention_mfma_kernel<DS_, VT_, NG_>;                                                         \
     if (msmem > 65536) /* more dynamic LDS than a kernel gets without asking */                                    \
       (void)hipFuncSetAttribute((const void*)kfn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)msmem);         \
-    hipLaunchKernelGGL(kfn, grid, dim3(64 * nw), msmem, stream(),                                                 \
+    hipLaunchKernelGGL(kfn, grid, dim3(64 * nw * NG_), msmem, stream(),                                            \
                        (x.cross_out != nullptr || x.out32 != nullptr) ? (bf16s*)nullptr : ptr<bf16s>(out),         \
                        ptr<bf16s>(q),                                                                              \
                        (long)q.stride(0), ptr<bf16s>(kpool), ptr<bf16s>(vpool), block_tables.data_ptr<int>(),      \
@@ -793,7 +854,7 @@ static bool launch_mfma_attention(at::Tensor& out, const at::Tensor& q, const at
                        page_shift, (float)scale, (int)window, (int)keep_first, (float)softcap, sink ? 1 : 0,       \
                        qsplit, x.sink_logits, x.dist_bias, x.dist_rows, (const bf16s*)x.ksum,                      \
                        (const bf16s*)x.vsum, x.sum_shift, x.sum_block, x.cross_out, x.chunk, x.key_fac, x.vrep,    \
-                       x.out32);                                                                                   \
+                       x.out32, tiles);                                                                            \
   } while (0)
 #define MFMA_ROW(DS_)                     \
   do {                                    \
@@ -809,6 +870,7 @@ static bool launch_mfma_attention(at::Tensor& out, const at::Tensor& q, const at
     else MFMA_ROW(8);
 #undef MFMA_ROW
 #undef MFMA_CASE
+#undef MFMA_NG
     HIP_CHECK_LAST();
     return true;
   }

@@ -78,3 +78,26 @@ def test_decode_in_float32():
     want = paged_attention_ref(q, k, v, batch, 0.09, softcap=7.0, sink=True)
     # float32 sums over 4000 weights: 4000^0.5 roundings of 2^-24 at most on average, and as much again in the reference
     assert (got - want).norm() / want.norm() < 2 * 4000 ** 0.5 * 2.0 ** -24
+
+
+@pytest.mark.parametrize("H,G,counts,starts,page", [
+    (6, 2, [40, 1, 33], [0, 70, 31], 8),     # few blocks, two groups of waves: odd and even numbers of key tiles
+    (4, 4, [300, 129], [0, 5], 16),          # a block of 128 tokens of one head
+    (24, 3, [1100], [0], 64),                # 6 rows of heads: neither a divisor nor a multiple of the XCDs
+    (16, 16, [2200, 17], [0, 0], 32),        # 16 rows, every block running at once
+    (16, 16, [4700], [0], 32),               # 16 rows, more blocks than run at once
+    (64, 8, [900], [100], 4),                # 16 rows of several heads, pages smaller than a wave's load
+    (4, 1, [2500], [0], 64),                 # one row over all XCDs
+    (8, 2, [2600, 31], [700, 0], 1),         # four XCDs a row
+])
+@pytest.mark.parametrize("D,Dv,kw", [(128, 128, {}), (64, 64, dict(softcap=5.0, sink=True)),
+                                     (72, 40, dict(slopes=True, window=200, keep_first=40))])
+def test_every_tile_is_taken_once(H, G, counts, starts, page, D, Dv, kw):
+    _check(counts, starts, H, G, D, Dv, page, 0.1, **dict(kw))
+
+
+@pytest.mark.parametrize("softcap", [0.5, 50.0])
+@pytest.mark.parametrize("scale", [1e-4, 0.03, 1.0])
+def test_soft_caps_near_and_far(softcap, scale):
+    """Scores far below the cap, about it and far above it: the two forms of tanh."""
+    _check([64, 700], [10, 0], 16, 4, 64, 64, 16, scale, softcap=softcap, sink=True)
