@@ -38,6 +38,23 @@ def test_linear_cross_entropy(N, V, H, chunk):
     assert _rel(dw, ww) < 2 * ROUND * (top + 1)
 
 
+@pytest.mark.parametrize("rows,V", [(4096, 32000), (1000, 50257), (2048, 512)])
+def test_loss_keeps_float32_precision(rows, V):
+    from colossalai_amd.ops._kernels import kernels
+
+    torch.manual_seed(1)
+    logits = torch.randn(rows, V, device="cuda").bfloat16()
+    labels = torch.randint(0, V, (rows,), device="cuda")
+    lse = torch.empty(rows, device="cuda")
+    nll = torch.empty_like(lse)
+    kernels().ce_fwd(logits, labels, -100, lse, nll)
+    loss = kernels().ce_loss(nll, labels, -100)[0].item()
+    want = torch.nn.functional.cross_entropy(logits.double(), labels).item()
+    # rows' own roundings (three of values below 16, half of 2^-20 each at most) go either way and average out; what is
+    # left is a lean of the exponentials, 1e-7 of the sum, and the rounding of the loss itself, half of 2^-20
+    assert abs(loss - want) < 2.0 ** -20
+
+
 def test_cross_entropy_without_a_row_that_counts():
     from colossalai_amd.ops.fused_ce import fused_linear_cross_entropy
 
