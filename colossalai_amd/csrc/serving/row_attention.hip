@@ -25,6 +25,7 @@ namespace serving {
 typedef int int4v_ __attribute__((ext_vector_type(4)));
 
 constexpr int ROW_WAVES = 8;
+constexpr int MAX_PARTS = WAVE;  // of a token's keys: row_merge_kernel gives each part a lane
 
 template <typename T> struct RowLane;   // CH channels = 32 bytes per lane, as two 16-byte pieces
 template <> struct RowLane<bf16s> {
@@ -333,7 +334,7 @@ __global__ __launch_bounds__(256) void row_merge_kernel(
   if (row >= rows) return;
   const float* state = ws + row * splits * (long)(2 + Dv);
   const int h = (int)(row % H);
-  const float m = lane < splits ? state[lane * (long)(2 + Dv)] : -INFINITY;   // splits <= 64
+  const float m = lane < splits ? state[lane * (long)(2 + Dv)] : -INFINITY;   // splits <= MAX_PARTS
   const float l = lane < splits ? state[lane * (long)(2 + Dv) + 1] : 0.0f;
   float top = wave_reduce_max(m);
   if (sink_logits != nullptr) top = fmaxf(top, sink_logits[h] * Dom<T>::UNIT);
@@ -378,12 +379,12 @@ bool launch_row_attention(at::Tensor& out, const at::Tensor& q, const at::Tensor
   // against 44.0; 16 x 6000, 32/8 heads: 221 against 113; four heads do not fit into the registers: 166).
   // Then the keys are cut into parts while there are fewer blocks than CUs and a part still gives every wave a key
   // block: 4 x 16384 210 -> 44 us, 8 x 2048 26.6 -> 19.1, 1 x 4096 36 -> 18. More blocks than CUs are slower again (4 x 16384
-  // with 512 blocks 76 us): a block costs about 10 us by itself.
+  // with 512 blocks 76 us): a block costs about 10 us by itself. One or two blocks stop at the parts that the merge takes.
   int rc = R > 1 && (N * G * ((R + 1) / 2) >= 256 || keys >= 8192) ? 2 : 1;
   int splits = 1;
   const long blocks = N * G * ((R + rc - 1) / rc);
   const long pass = (long)ROW_WAVES * (rc == 1 || shared ? 8 : 4) * (64 >> lane_shift);   // keys of one key block of every wave
-  while (blocks * splits * 2 <= 256 && keys > splits * pass) splits *= 2;
+  while (blocks * splits * 2 <= 256 && keys > splits * pass && splits < MAX_PARTS) splits *= 2;
   auto lds_bytes = [&](int nw) { return (size_t)(rc * ROW_WAVES + nw * rc * (2 + Dv)) * sizeof(float); };
   int nwaves = ROW_WAVES;
   while (lds_bytes(nwaves) > 64 * 1024 && nwaves > 4) nwaves >>= 1;
@@ -412,6 +413,7 @@ bool launch_row_attention(at::Tensor& out, const at::Tensor& q, const at::Tensor
     }
     if (splits > 1) {
       HIP_CHECK_LAST();
+      TORCH_CHECK(splits <= MAX_PARTS, "more parts of the keys than the merge takes");
       hipLaunchKernelGGL((row_merge_kernel<T>), dim3((unsigned)((N * H + 3) / 4)), dim3(256), 0, stream(),
                          x.out32 != nullptr ? (T*)nullptr : ptr<T>(out), x.out32, ws.data_ptr<float>(),
                          gate.has_value() ? ptr<T>(*gate) : (const T*)nullptr, gate_stride, x.sink_logits, N * H, H, Dv,

@@ -68,16 +68,41 @@ def test_decode_heads_and_parts(H, G, starts):
     _check([1] * len(starts), starts, H, G, 128, 128, 64, 0.09)
 
 
-def test_decode_in_float32():
+@pytest.mark.parametrize("H,G,starts", [(8, 2, [4000, 37]), (4, 2, [8191]), (4, 2, [8200]), (1, 1, [20000])])
+def test_decode_in_float32(H, G, starts):
+    """The last ones at and beyond the 64 parts that the merge takes."""
     from colossalai_amd.ops.paged_attention import paged_attention, paged_attention_ref
 
     torch.manual_seed(2)
-    batch, pages = _batch([1, 1], [4000, 37], 16)
-    q, k, v = (torch.randn(*s, device="cuda") for s in ((2, 8, 128), (pages, 16, 2, 128), (pages, 16, 2, 128)))
+    n = len(starts)
+    batch, pages = _batch([1] * n, starts, 16)
+    q, k, v = (torch.randn(*s, device="cuda") for s in ((n, H, 128), (pages, 16, G, 128), (pages, 16, G, 128)))
     got = paged_attention(q, k, v, batch, 0.09, softcap=7.0, sink=True)
     want = paged_attention_ref(q, k, v, batch, 0.09, softcap=7.0, sink=True)
-    # float32 sums over 4000 weights: 4000^0.5 roundings of 2^-24 at most on average, and as much again in the reference
-    assert (got - want).norm() / want.norm() < 2 * 4000 ** 0.5 * 2.0 ** -24
+    # float32 sums over the weights: keys^0.5 roundings of 2^-24 at most on average, and as much again in the reference
+    assert (got - want).norm() / want.norm() < 2 * max(starts) ** 0.5 * 2.0 ** -24
+
+
+# One sequence whose heads fill one or two blocks: its keys would go into more than the 64 parts that the merge takes from
+# 16384 keys on (32768 with a single head); one page more, twice as many and on, and shared heads.
+@pytest.mark.parametrize("H,G,start", [(4, 2, 16383), (4, 2, 16384), (4, 1, 16400), (2, 2, 40000), (1, 1, 32767), (1, 1, 33000),
+                                       (2, 1, 70000)])
+def test_decode_with_most_parts(H, G, start):
+    _check([1], [start], H, G, 128, 128, 16, 0.09)
+
+
+@pytest.mark.parametrize("start", [4095, 4096, 9000])
+def test_latent_rows_with_most_parts(start):
+    """Values that are the leading channels of wide key rows, two query heads."""
+    from colossalai_amd.ops.paged_attention import paged_attention, paged_attention_ref
+
+    torch.manual_seed(3)
+    batch, pages = _batch([1], [start], 16)
+    k = torch.randn(pages, 16, 1, 576, device="cuda").bfloat16()
+    q = torch.randn(1, 2, 576, device="cuda").bfloat16()
+    got = paged_attention(q, k, k[..., :512], batch, 0.05)
+    want = paged_attention_ref(q.float(), k.float(), k[..., :512].float(), batch, 0.05)
+    assert (got.double() - want.double()).norm() / want.double().norm() < BOUND
 
 
 @pytest.mark.parametrize("H,G,counts,starts,page", [
