@@ -438,7 +438,8 @@ __global__ __launch_bounds__(256 * NG, 2) void paged_attention_mfma_kernel(
   };
   // The page-table lookups of a tile run one step ahead of its key/value loads (two ahead of its use), so that a
   // load's address never waits for a lookup issued in the same iteration.
-  const bool full = Dr == D && Dvr == Dv;
+  // Every channel of the quads is the head's: no lane has to look. A tiling of 48 channels ends in half a quad.
+  const bool kfull = D % 32 == 0 && Dr == D, vfull = Dvr == Dv;
   const unsigned krs = (unsigned)(G * Dr) * 2u, vrs = (unsigned)(Gv * Dvr) * 2u;   // bytes between neighbouring keys' rows
   int krow[TP][2], frow[TP];
   float rf[TP];
@@ -463,14 +464,14 @@ __global__ __launch_bounds__(256 * NG, 2) void paged_attention_mfma_kernel(
         const int q_ = (wv + 4 * r) % KQ, i = (wv + 4 * r) / KQ;   // quad, group of 16 keys
         if (2 * KQ % 4 != 0 && i > 1) continue;
         const char* at = kp + q_ * 64 + (unsigned long)(unsigned)(i ? krow[u][1] : krow[u][0]) * krs;
-        rk[u][r] = full || q_ * 32 + lch < Dr ? *reinterpret_cast<const bf16x8_v*>(at) : zero8;
+        rk[u][r] = kfull || q_ * 32 + lch < Dr ? *reinterpret_cast<const bf16x8_v*>(at) : zero8;
       }
 #pragma unroll
       for (int r = 0; r < VR; ++r) {
         const int q_ = (wv + 4 * r) % VQ, i = (wv + 4 * r) / VQ;
         if (2 * VQ % 4 != 0 && i > 1) continue;
         const char* at = vp + q_ * 64 + (unsigned long)(unsigned)(i ? krow[u][1] : krow[u][0]) * vrs;
-        rv[u][r] = full || q_ * 32 + lch < Dvr ? *reinterpret_cast<const bf16x8_v*>(at) : zero8;
+        rv[u][r] = vfull || q_ * 32 + lch < Dvr ? *reinterpret_cast<const bf16x8_v*>(at) : zero8;
       }
       if (key_fac != nullptr && tid < 32) rf[u] = key_fac[(long)frow[u] * G + g];
     }

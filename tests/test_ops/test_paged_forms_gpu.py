@@ -115,7 +115,7 @@ def test_latent_rows_with_most_parts(start):
     (4, 1, [2500], [0], 64),                 # one row over all XCDs
     (8, 2, [2600, 31], [700, 0], 1),         # four XCDs a row
 ])
-@pytest.mark.parametrize("D,Dv,kw", [(128, 128, {}), (64, 64, dict(softcap=5.0, sink=True)),
+@pytest.mark.parametrize("D,Dv,kw", [(128, 128, {}), (64, 64, dict(softcap=5.0, sink=True)), (48, 64, {}),
                                      (72, 40, dict(slopes=True, window=200, keep_first=40))])
 def test_every_tile_is_taken_once(H, G, counts, starts, page, D, Dv, kw):
     _check(counts, starts, H, G, D, Dv, page, 0.1, **dict(kw))
