@@ -19,11 +19,12 @@ constexpr int CE_BLOCK = 256;
 constexpr float CE_LOG2E = 1.44269504f;
 
 // A row's running state: maximum m and s = sum exp(x - ref(m)), where an infinite maximum is no reference (a row with a
-// logit of +inf has a log-sum-exp of +inf, one of nothing but -inf has -inf).
+// logit of +inf has a log-sum-exp of +inf, one of nothing but -inf has -inf). A NaN is in s; fmaxf leaves it out of m, so
+// with a maximum of -inf s is 0 or NaN and stays as it is.
 DEV_INLINE float ce_ref(float m) { return fabsf(m) == INFINITY ? 0.0f : m; }
 
 DEV_INLINE float ce_moved(float m, float s, float ref) {
-  return m == -INFINITY ? 0.0f : s * __builtin_amdgcn_exp2f((ce_ref(m) - ref) * CE_LOG2E);
+  return m == -INFINITY ? s : s * __builtin_amdgcn_exp2f((ce_ref(m) - ref) * CE_LOG2E);
 }
 
 DEV_INLINE void ce_merge(float& m, float& s, float om, float os) {

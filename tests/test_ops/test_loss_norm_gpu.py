@@ -86,6 +86,26 @@ def test_row_statistics_with_infinities(V):
     assert torch.isnan(nll[0])
 
 
+@pytest.mark.parametrize("V", [64, 1003, 32000])
+def test_row_statistics_with_nan(V):
+    """A NaN anywhere in a row is in its statistics: the columns that a thread reads first and last, whole groups of eight, and
+    beside infinities."""
+    from colossalai_amd.ops import kernels
+
+    spots = [(0, 1), (0, 8), (V - 1, V), (V - 8, V), (V // 2, V // 2 + 1), (0, V)]
+    x = torch.randn(len(spots) + 2, V, device="cuda").bfloat16()
+    for row, (lo, hi) in enumerate(spots):
+        x[row, lo:hi] = float("nan")
+    x[-2] = float("-inf")
+    x[-2, 0] = float("nan")
+    x[-1, : V // 2] = float("-inf")
+    x[-1, 1] = float("nan")
+    labels = torch.full((len(x),), V // 4, device="cuda")
+    lse, nll = torch.empty(len(x), device="cuda"), torch.empty(len(x), device="cuda")
+    kernels().ce_fwd(x, labels, -100, lse, nll)
+    assert torch.isnan(lse).all() and torch.isnan(nll).all()
+
+
 @pytest.mark.parametrize("rows,H", [(1, 8), (3, 512), (5, 520), (130, 768), (9, 1032), (33, 2048), (6, 2056), (7, 4104), (5, 8192),
                                     (5000, 64)])
 def test_add_norm_and_its_gradients(rows, H):
