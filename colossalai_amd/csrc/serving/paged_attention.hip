@@ -515,7 +515,7 @@ __global__ __launch_bounds__(256 * NG, 2) void paged_attention_mfma_kernel(
   const float inv_cap = capped ? scale / softcap : 0.0f;
   const float cap2 = softcap * LOG2E, t2 = capped ? 2.0f * LOG2E * scale / softcap : 0.0f;
   auto cap_base2 = [&](float dot) {
-    const float e = __builtin_amdgcn_exp2f(fminf(dot * t2, 64.0f));  // beyond 2^64 the quotient is 0 in float32 anyway
+    const float e = __builtin_amdgcn_exp2f(dot * t2);  // +inf: the quotient is 0; a NaN stays one
     return cap2 - 2.0f * cap2 * __builtin_amdgcn_rcpf(e + 1.0f);
   };
   // A key's share of the distance penalty: its offset inside its tile (row of the C layout) here, the tile's per tile

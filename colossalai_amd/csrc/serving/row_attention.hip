@@ -55,9 +55,10 @@ template <typename T> struct Dom;
 template <> struct Dom<bf16s> {
   static constexpr float UNIT = 1.4426950408889634f;   // what one nat is here
   DEV_INLINE static float exp_(float x) { return __builtin_amdgcn_exp2f(x); }
-  // cap tanh(x / cap) for x and cap in units of this domain: tanh(y) = 1 - 2 / (exp(2 y) + 1)
+  // cap tanh(x / cap) for x and cap in units of this domain: tanh(y) = 1 - 2 / (exp(2 y) + 1), where an exponential of +inf
+  // is a quotient of 0 and a NaN stays one
   DEV_INLINE static float cap_(float x, float cap, float inv_cap) {
-    const float e = __builtin_amdgcn_exp2f(fminf(x * inv_cap * (2.0f * UNIT), 64.0f));
+    const float e = __builtin_amdgcn_exp2f(x * inv_cap * (2.0f * UNIT));
     return cap - 2.0f * cap * __builtin_amdgcn_rcpf(e + 1.0f);
   }
 };

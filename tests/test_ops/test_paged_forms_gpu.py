@@ -105,6 +105,28 @@ def test_latent_rows_with_most_parts(start):
     assert (got.double() - want.double()).norm() / want.double().norm() < BOUND
 
 
+@pytest.mark.parametrize("counts", [[1], [40]])
+@pytest.mark.parametrize("kw", [{}, dict(softcap=5.0), dict(softcap=5.0, sink=True)])
+def test_nan_stays_nan(counts, kw):
+    """A query or a key of NaN shows in what it touches, and nowhere else, also where a cap bounds the score. The other scores
+    reach far beyond the cap's near form."""
+    from colossalai_amd.ops.paged_attention import paged_attention
+
+    torch.manual_seed(4)
+    batch, pages = _batch(counts, [100], 16)
+    n = sum(counts)
+    k, v = (torch.randn(pages, 16, 2, 64, device="cuda").bfloat16() for _ in range(2))
+    q = torch.randn(n, 4, 64, device="cuda").bfloat16()
+    q[n - 1, 0, 5] = float("nan")          # one token's first head: of key head 0
+    k[batch.block_tables[0, 2], 3, 1, 7] = float("nan")   # position 35, which every token sees: key head 1
+    bad = torch.isnan(paged_attention(q, k, v, batch, 1.0, **kw).float()).all(-1)
+    some = torch.isnan(paged_attention(q, k, v, batch, 1.0, **kw).float()).any(-1)
+    want = torch.zeros(n, 4, dtype=torch.bool, device="cuda")
+    want[n - 1, 0] = True
+    want[:, 2:] = True
+    assert torch.equal(bad, want) and torch.equal(some, want)
+
+
 @pytest.mark.parametrize("H,G,counts,starts,page", [
     (6, 2, [40, 1, 33], [0, 70, 31], 8),     # few blocks, two groups of waves: odd and even numbers of key tiles
     (4, 4, [300, 129], [0, 5], 16),          # a block of 128 tokens of one head
