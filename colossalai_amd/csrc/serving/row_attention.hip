@@ -53,19 +53,42 @@ template <> struct RowLane<float> {
 // reciprocal; float32 serving keeps the natural one with the library's functions.
 template <typename T> struct Dom;
 template <> struct Dom<bf16s> {
-  static constexpr float UNIT = 1.4426950408889634f;   // what one nat is here
+  static constexpr double NAT = 1.4426950408889634;    // what one nat is here
+  static constexpr float UNIT = (float)NAT;
   DEV_INLINE static float exp_(float x) { return __builtin_amdgcn_exp2f(x); }
-  // cap tanh(x / cap) for x and cap in units of this domain: tanh(y) = 1 - 2 / (exp(2 y) + 1), where an exponential of +inf
-  // is a quotient of 0 and a NaN stays one
-  DEV_INLINE static float cap_(float x, float cap, float inv_cap) {
-    const float e = __builtin_amdgcn_exp2f(x * inv_cap * (2.0f * UNIT));
-    return cap - 2.0f * cap * __builtin_amdgcn_rcpf(e + 1.0f);
+  // cap tanh(x / cap) for x and cap in units of this domain, a lane's N scores. tanh(y) = y P(y^2) for |y| <= 1/2, P the polynomial
+  // through the Chebyshev nodes (1.3e-8 off); beyond, 1 - 2 / (exp(2 |y|) + 1) with y's sign, where an infinite
+  // exponential is a quotient of 0 and a NaN stays one. That form alone is off by roundings of the cap, not of the score (cap
+  // 30: 1.4e-6 at scores about 0.6 and 3, where these two are 0.9e-7 and 2.8e-7 off and the library's tanh 1.0e-7 and 3.8e-7), so a
+  // score takes the form that is its own; mostly a whole wave's are small. 16 x 1024 keys with a cap take 17.8 us either way.
+  template <int N>
+  DEV_INLINE static void cap_(float (&x)[N], float cap, float inv_cap) {
+    float far = 0.0f;
+#pragma unroll
+    for (int i = 0; i < N; ++i) far = fmaxf(far, fabsf(x[i]));
+    const bool near = __all(far * inv_cap <= 0.5f);
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      const float y = x[i] * inv_cap, z = y * y;
+      const float small = x[i] * fmaf(z, fmaf(z, fmaf(z, fmaf(z, 0.017131345f, -0.052984238f), 0.13324751f), -0.33333069f), 1.0f);
+      if (near) {
+        x[i] = small;
+      } else {
+        const float large = cap - 2.0f * cap * __builtin_amdgcn_rcpf(__builtin_amdgcn_exp2f(fabsf(y) * (2.0f * UNIT)) + 1.0f);
+        x[i] = fabsf(y) <= 0.5f ? small : copysignf(large, y);
+      }
+    }
   }
 };
 template <> struct Dom<float> {
+  static constexpr double NAT = 1.0;
   static constexpr float UNIT = 1.0f;
   DEV_INLINE static float exp_(float x) { return expf(x); }
-  DEV_INLINE static float cap_(float x, float cap, float inv_cap) { return cap * tanhf(x * inv_cap); }
+  template <int N>
+  DEV_INLINE static void cap_(float (&x)[N], float cap, float inv_cap) {
+#pragma unroll
+    for (int i = 0; i < N; ++i) x[i] = cap * tanhf(x[i] * inv_cap);
+  }
 };
 
 typedef unsigned uint2v_ __attribute__((ext_vector_type(2)));
@@ -91,6 +114,7 @@ __global__ __launch_bounds__(64 * ROW_WAVES) void row_attention_kernel(
     const float* __restrict__ sink_logits, const float* __restrict__ key_fac, int H, int G, int D, int Dv, int page_shift,
     float scale, int window, int keep_first, int chunk, float softcap, int sink, int vrep, long vrow, long vhead,
     int lane_shift, int qvec, int splits, float* __restrict__ ws) {
+  // scale: in units of the domain, rounded once (the product of two float32 factors leans a whole row's scores)
   constexpr int CH = RowLane<T>::CH, HC = CH / 2;
   extern __shared__ __align__(16) float lds[];
   const int wid = threadIdx.x >> 6, lane = threadIdx.x & 63, nw = blockDim.x >> 6;
@@ -126,7 +150,7 @@ __global__ __launch_bounds__(64 * ROW_WAVES) void row_attention_kernel(
       for (int c = 0; c < CH; ++c) qf[r][c] = r < nh && ch + c < D ? ldf(qp + c) : 0.0f;
     }
 #pragma unroll
-    for (int c = 0; c < CH; ++c) qf[r][c] *= scale * Dom<T>::UNIT;
+    for (int c = 0; c < CH; ++c) qf[r][c] *= scale;
   }
   const int lo = first_visible(pos, window, chunk);
   const int n_keep = window > 0 ? min(keep_first, lo) : 0;
@@ -204,9 +228,11 @@ __global__ __launch_bounds__(64 * ROW_WAVES) void row_attention_kernel(
     for (int r = 0; r < RC; ++r) {
       float top = m[r];
 #pragma unroll
+      for (int s = 0; s < NS; ++s) sc[r][s] *= fac[s];
+      if (softcap > 0.0f) Dom<T>::cap_(sc[r], cap, inv_cap);
+#pragma unroll
       for (int s = 0; s < NS; ++s) {
-        float v = sc[r][s] * fac[s];
-        if (softcap > 0.0f) v = Dom<T>::cap_(v, cap, inv_cap);
+        float v = sc[r][s];
         v -= slope[r] * (float)(pos - key_of(base + s * KPS + group));
         sc[r][s] = base + s * KPS + group < last ? v : -INFINITY;
         top = fmaxf(top, sc[r][s]);
@@ -401,7 +427,7 @@ bool launch_row_attention(at::Tensor& out, const at::Tensor& q, const at::Tensor
                      (long)q.stride(0), ptr<T>(kpool), ptr<T>(vpool), block_tables.data_ptr<int>(),                     \
                      (int)block_tables.stride(0), tok_seq.data_ptr<int>(), positions.data_ptr<int>(), slopes,           \
                      gate.has_value() ? ptr<T>(*gate) : (const T*)nullptr, gate_stride, x.sink_logits, x.key_fac, H, G, \
-                     D, Dv, page_shift, (float)scale, (int)window, (int)keep_first, x.chunk, (float)softcap,            \
+                     D, Dv, page_shift, (float)(scale * Dom<T>::NAT), (int)window, (int)keep_first, x.chunk, (float)softcap, \
                      sink ? 1 : 0, x.vrep, vrow, vhead, lane_shift, qvec, splits,                                       \
                      splits > 1 ? ws.data_ptr<float>() : (float*)nullptr)
   SERVING_DISPATCH_ACT(q, T, {

@@ -127,6 +127,29 @@ def test_nan_stays_nan(counts, kw):
     assert torch.equal(bad, want) and torch.equal(some, want)
 
 
+@pytest.mark.parametrize("spread", [0.02, 0.1, 0.5])
+def test_capped_scores_keep_float32_precision(spread):
+    """A decode token that sees one key and the sink returns p = 1 / (1 + exp(-s)) of its value 1: s can be read back."""
+    from colossalai_amd.ops.paged_attention import paged_attention
+
+    torch.manual_seed(5)
+    n, H, D, cap = 512, 8, 64, 30.0
+    batch, pages = _batch([1] * n, [0] * n, 1)
+    q = torch.randn(n, H, D, device="cuda").bfloat16()
+    k = torch.randn(pages, 1, H, D, device="cuda").bfloat16()
+    v = torch.ones(pages, 1, H, D, device="cuda").bfloat16()
+    dots = (q.double() * k[batch.block_tables[:, 0].long(), 0].double()).sum(-1)
+    scale = spread * cap / dots.std().item()
+    p = paged_attention(q, k, v, batch, scale, softcap=cap, sink=True, out_dtype=torch.float32)[..., 0].double()
+    s = cap * torch.tanh(dots * scale / cap)
+    mine = torch.log(p / (1 - p))
+    seen = (s < 0) & (s > -12)   # there p's own rounding is at most 2^-23 of s
+    err = (mine - s)[seen]
+    # a score's roundings are relative to it (sums of the product, scale, quotient, tanh), those of exponential, sum and quotient of p
+    # are not: four of half of 2^-23 at most either way
+    assert err.pow(2).mean().sqrt() < 4 * 2.0 ** -24 * (1 + s[seen].pow(2).mean().sqrt())
+
+
 @pytest.mark.parametrize("H,G,counts,starts,page", [
     (6, 2, [40, 1, 33], [0, 70, 31], 8),     # few blocks, two groups of waves: odd and even numbers of key tiles
     (4, 4, [300, 129], [0, 5], 16),          # a block of 128 tokens of one head
