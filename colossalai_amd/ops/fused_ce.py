@@ -57,9 +57,16 @@ class _FusedLinearCE(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, grad_out):
-        if ctx.hip:
+        # the kernel works in place and outside autograd: a backward that is part of a graph itself
+        # (create_graph) takes the general form
+        if ctx.hip and not torch.is_grad_enabled():
             return _backward_hip(ctx, grad_out)
-        hidden, weight, safe_labels, valid, lse, n_valid = ctx.saved_tensors
+        if ctx.hip:
+            hidden, weight, labels, lse, loss = ctx.saved_tensors
+            valid = labels != ctx.ignore_index
+            safe_labels, n_valid = labels.masked_fill(~valid, 0), loss[1]
+        else:
+            hidden, weight, safe_labels, valid, lse, n_valid = ctx.saved_tensors
         N, H = hidden.shape
         chunk_size = ctx.chunk_size
         dh = torch.empty_like(hidden)
