@@ -22,6 +22,12 @@ from ._kernels import kernels, use_hip
 __all__ = ["fused_linear_cross_entropy"]
 
 
+def _bf16_products(t: torch.Tensor) -> bool:
+    """Whether bfloat16 operands give a bfloat16 product here: not under autocast to another type."""
+    kind = t.device.type
+    return not torch.is_autocast_enabled(kind) or torch.get_autocast_dtype(kind) == torch.bfloat16
+
+
 class _FusedLinearCE(torch.autograd.Function):
     @staticmethod
     def forward(ctx, hidden, weight, labels, ignore_index, chunk_size):
@@ -30,7 +36,7 @@ class _FusedLinearCE(torch.autograd.Function):
         ctx.chunk_size = chunk_size
         ctx.ignore_index = ignore_index
         ctx.hip = (hidden.dtype == weight.dtype == torch.bfloat16 and labels.dtype == torch.int64
-                   and use_hip(hidden, weight, labels))
+                   and use_hip(hidden, weight, labels) and _bf16_products(hidden))
         if ctx.hip:
             labels = labels.contiguous()
             lse = torch.empty(N, dtype=torch.float32, device=hidden.device)
@@ -57,9 +63,9 @@ class _FusedLinearCE(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, grad_out):
-        # the kernel works in place and outside autograd: a backward that is part of a graph itself
-        # (create_graph) takes the general form
-        if ctx.hip and not torch.is_grad_enabled():
+        # the kernel works on bfloat16 logits, in place and outside autograd: a backward that is part of a graph itself
+        # (create_graph) or under autocast to another type takes the general form
+        if ctx.hip and not torch.is_grad_enabled() and _bf16_products(grad_out):
             return _backward_hip(ctx, grad_out)
         if ctx.hip:
             hidden, weight, labels, lse, loss = ctx.saved_tensors

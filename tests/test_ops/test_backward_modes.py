@@ -83,3 +83,30 @@ def test_loss_gradients_under_create_graph(device, chunk):
     for a, b in zip(graph, plain):
         _near(a.detach(), b)
         assert a.grad_fn is not None  # part of a graph: nothing is dropped from a second derivative in silence
+
+
+@pytest.mark.parametrize("where", ["forward", "backward", "both"])
+def test_loss_under_autocast_to_half(device, where):
+    hidden, weight, labels = _loss_inputs(device)
+    kind = hidden.device.type
+    loss = fused_ce.fused_linear_cross_entropy(hidden, weight, labels)
+    want = (loss, *torch.autograd.grad(loss, (hidden, weight)))
+    with torch.autocast(kind, dtype=torch.float16, enabled=where != "backward"):
+        loss = fused_ce.fused_linear_cross_entropy(hidden, weight, labels)
+    with torch.autocast(kind, dtype=torch.float16, enabled=where != "forward"):
+        got = (loss, *torch.autograd.grad(loss, (hidden, weight)))
+    for a, b in zip(got, want):
+        assert a.dtype == b.dtype
+        _near(a.detach(), b.detach())
+
+
+def test_loss_in_a_checkpoint(device):
+    """Saved tensors of a checkpointed segment may be taken once only."""
+    from torch.utils.checkpoint import checkpoint
+
+    hidden, weight, labels = _loss_inputs(device)
+    loss = fused_ce.fused_linear_cross_entropy(hidden, weight, labels)
+    want = torch.autograd.grad(loss, (hidden, weight))
+    loss = checkpoint(fused_ce.fused_linear_cross_entropy, hidden, weight, labels, use_reentrant=False)
+    for a, b in zip(torch.autograd.grad(loss, (hidden, weight)), want):
+        assert torch.equal(a, b)
