@@ -84,7 +84,7 @@ __global__ __launch_bounds__(CE_BLOCK) void ce_fwd_kernel(float* __restrict__ ls
   }
 }
 
-// logits -> their gradient (softmax - onehot) * valid * grad / n_valid, in place.
+// logits -> their gradient (softmax - onehot) * valid * grad / n_valid, in place (NaN for a label outside the row).
 template <bool VEC>
 __global__ __launch_bounds__(CE_BLOCK) void ce_bwd_kernel(unsigned short* __restrict__ logits, const float* __restrict__ lse,
                                                           const long* __restrict__ labels, const float* __restrict__ grad,
@@ -92,7 +92,7 @@ __global__ __launch_bounds__(CE_BLOCK) void ce_bwd_kernel(unsigned short* __rest
   const long row = blockIdx.x;
   unsigned short* x = logits + row * V;
   const long label = labels[row];
-  const float scale = label == ignore_index ? 0.0f : grad[0] / loss[1];
+  const float scale = label == ignore_index ? 0.0f : label >= 0 && label < V ? grad[0] / loss[1] : NAN;
   const float l = lse[row];
   auto one = [&](unsigned short raw, int col) {
     float p = __builtin_amdgcn_exp2f((bf2f(raw) - l) * CE_LOG2E);

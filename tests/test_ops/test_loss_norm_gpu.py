@@ -106,6 +106,20 @@ def test_row_statistics_with_nan(V):
     assert torch.isnan(lse).all() and torch.isnan(nll).all()
 
 
+@pytest.mark.parametrize("V", [80, 1003])
+@pytest.mark.parametrize("label", [-1, -7, None])
+def test_a_label_outside_the_row_spoils_its_gradient(V, label):
+    from colossalai_amd.ops.fused_ce import fused_linear_cross_entropy
+
+    hidden = torch.randn(5, 64, device="cuda").bfloat16().requires_grad_()
+    weight = torch.randn(V, 64, device="cuda").bfloat16()
+    labels = torch.tensor([1, 2, V if label is None else label, 3, -100], device="cuda")
+    loss = fused_linear_cross_entropy(hidden, weight, labels)
+    (dh,) = torch.autograd.grad(loss, hidden)
+    assert torch.isnan(loss) and torch.isnan(dh[2]).all()
+    assert torch.isfinite(dh[[0, 1, 3, 4]]).all()
+
+
 @pytest.mark.parametrize("rows,H", [(1, 8), (3, 512), (5, 520), (130, 768), (9, 1032), (33, 2048), (6, 2056), (7, 4104), (5, 8192),
                                     (5000, 64)])
 def test_add_norm_and_its_gradients(rows, H):
