@@ -33,7 +33,8 @@ DEV_INLINE void ce_merge(float& m, float& s, float om, float os) {
   m = top;
 }
 
-// lse [rows] and nll [rows] = lse - logits[label] (0 for an ignored row; NaN for a label outside the row).
+// lse [rows] and nll [rows] = lse - logits[label] (0 lse for an ignored row: what is not finite there shows, as it does in
+// the general form; NaN for a label outside the row).
 // VEC: rows of a multiple of 8 columns, 16-byte loads.
 template <bool VEC>
 __global__ __launch_bounds__(CE_BLOCK) void ce_fwd_kernel(float* __restrict__ lse, float* __restrict__ nll,
@@ -80,7 +81,7 @@ __global__ __launch_bounds__(CE_BLOCK) void ce_fwd_kernel(float* __restrict__ ls
     const long label = labels[row];
     lse[row] = ce_ref(m) + ls;
     // the difference of two logits first: it is exact or nearly so, and the sum is rounded once
-    nll[row] = label == ignore_index ? 0.0f : label >= 0 && label < V ? (ce_ref(m) - bf2f(x[label])) + ls : NAN;
+    nll[row] = label == ignore_index ? 0.0f * (ce_ref(m) + ls) : label >= 0 && label < V ? (ce_ref(m) - bf2f(x[label])) + ls : NAN;
   }
 }
 
@@ -92,7 +93,7 @@ __global__ __launch_bounds__(CE_BLOCK) void ce_bwd_kernel(unsigned short* __rest
   const long row = blockIdx.x;
   unsigned short* x = logits + row * V;
   const long label = labels[row];
-  const float scale = label == ignore_index ? 0.0f : label >= 0 && label < V ? grad[0] / loss[1] : NAN;
+  const float scale = (label == ignore_index ? 0.0f : label >= 0 && label < V ? 1.0f : NAN) * (grad[0] / loss[1]);
   const float l = lse[row];
   auto one = [&](unsigned short raw, int col) {
     float p = __builtin_amdgcn_exp2f((bf2f(raw) - l) * CE_LOG2E);

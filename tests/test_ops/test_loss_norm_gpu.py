@@ -106,6 +106,24 @@ def test_row_statistics_with_nan(V):
     assert torch.isnan(lse).all() and torch.isnan(nll).all()
 
 
+def test_ignored_rows_show_what_is_not_finite():
+    """As in the general form, where an ignored row's loss and gradient are multiplied by 0."""
+    from colossalai_amd.ops.fused_ce import fused_linear_cross_entropy
+
+    hidden = torch.randn(6, 64, device="cuda").bfloat16()
+    hidden[2] = float("nan")
+    weight = torch.randn(80, 64, device="cuda").bfloat16()
+    labels = torch.tensor([1, 2, -100, 3, -100, 4], device="cuda")
+    assert torch.isnan(fused_linear_cross_entropy(hidden, weight, labels))
+    hidden[2] = 0.0
+    hidden.requires_grad_()
+    loss = fused_linear_cross_entropy(hidden, weight, labels)
+    (dh,) = torch.autograd.grad(loss, hidden, torch.full_like(loss, float("inf")), retain_graph=True)
+    assert torch.isnan(dh[2]).all() and torch.isnan(dh[4]).all()
+    (dh,) = torch.autograd.grad(loss, hidden)
+    assert (dh[2] == 0).all() and torch.isfinite(dh).all()
+
+
 @pytest.mark.parametrize("V", [80, 1003])
 @pytest.mark.parametrize("label", [-1, -7, None])
 def test_a_label_outside_the_row_spoils_its_gradient(V, label):
