@@ -78,7 +78,9 @@ class _FusedAddRMSNorm(torch.autograd.Function):
     def backward(ctx, dy, dres):
         h, weight, inv_rms = ctx.saved_tensors
         if use_hip(h, weight, dy):
-            fused = dres is not None and dres.dtype == h.dtype  # the residual stream's gradient rides along
+            # the residual stream's gradient rides along, unless the backward is part of a graph itself (create_graph): the
+            # kernel's result would end it
+            fused = dres is not None and dres.dtype == h.dtype and not torch.is_grad_enabled()
             dtotal, dw = kernels().rmsnorm_bwd(dy.contiguous(), h, weight, inv_rms,
                                                dres.contiguous() if fused else None, True)
             if dres is not None and not fused:

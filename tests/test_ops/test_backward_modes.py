@@ -110,3 +110,16 @@ def test_loss_in_a_checkpoint(device):
     loss = checkpoint(fused_ce.fused_linear_cross_entropy, hidden, weight, labels, use_reentrant=False)
     for a, b in zip(torch.autograd.grad(loss, (hidden, weight)), want):
         assert torch.equal(a, b)
+
+
+def test_residual_gradient_keeps_its_graph(device):
+    """The gradient that flows past the norm is a function of the stream: its derivative is part of a second one."""
+    torch.manual_seed(0)
+    x, res = (torch.randn(9, 64).bfloat16().to(device) for _ in range(2))
+    w = torch.ones(64, dtype=torch.bfloat16, device=device)
+    x.requires_grad_()
+    _, h = fused_add_rms_norm(x, res, w, 1e-6)
+    (first,) = torch.autograd.grad(h.float().pow(3).sum(), x, create_graph=True)
+    _near(first.detach(), 3 * h.detach().float() ** 2)
+    (second,) = torch.autograd.grad(first.float().sum(), x)
+    _near(second, 6 * h.detach().float())
