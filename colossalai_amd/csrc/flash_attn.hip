@@ -472,7 +472,7 @@ __global__ __launch_bounds__(256) void fa_delta_kernel(
 // (32 rows, double-buffered). dK and dV stay in registers. What a query row adds (its -lse log2e and
 // -delta) enters as the accumulator the product starts from and as the exponent's addend; a row
 // that counts nothing (padding, or no visible key) has an addend of -inf.
-// GS blocks share a key/value tile's heads when there would be too few blocks otherwise; they leave
+// GS blocks share a key/value tile's heads, as evenly as they go, when there would be too few blocks otherwise; they leave
 // float32 partial sums in PART [GS][2][B * Sk * Hkv * D] for fa_bwd_sum_kernel.
 template <int D, bool VARLEN>
 DEV_INLINE void bwd_dkdv(
@@ -507,7 +507,8 @@ DEV_INLINE void bwd_dkdv(
   const int y = f / (tiles * GS);
   if (y >= B * Hkv) return;
   const int b = VARLEN ? y % B : y / Hkv, hk = VARLEN ? y / B : y % Hkv;
-  const int G = Hq / Hkv / GS;                           // heads of this block
+  const int group = Hq / Hkv, h_first = part * group / GS;
+  const int G = (part + 1) * group / GS - h_first;       // heads of this block: its share of the group, GS need not divide it
   const int kvw = kv0 + w * QW;  // this wave's first kv row
 
   long seq0 = 0;
@@ -557,7 +558,7 @@ DEV_INLINE void bwd_dkdv(
   const unsigned qoff = qstage.offset(qts), dooff = dostage.offset(do_stride);
   float lse_r = 0.0f, dta_r = 0.0f;
   auto fetch = [&](int step) {   // global loads of a step's query tile
-    const int h = hk * (Hq / Hkv) + part * G + step / nq;
+    const int h = hk * group + h_first + step / nq;
     const int qt0 = (qt_first + step % nq) * QB;
     const unsigned short* q_base = VARLEN ? Q + seq0 * qts + (long)h * D : Q + (long)b * qbs + (long)h * D;
     const unsigned short* do_base =
@@ -1006,17 +1007,25 @@ void launch_bwd(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, c
   const int rows = NWB * QW;
   const int kv_tiles = (Sk_max + rows - 1) / rows, q_tiles = (S_max + rows - 1) / rows;
   const int G = Hq / Hkv;
-  // Blocks that share a tile's group of heads. All 512 blocks that fit on the chip at once start together, and
-  // under a causal mask the first tile then takes twice the average: B1 S8192, 32 over 8 heads, runs 2194 us with one
-  // block a tile (512 blocks), 2077 with two and 2110 with four (more partial sums). Without a mask the work is even
-  // and it only matters that every CU has a block. A block keeps at least 16 steps, or the sums cost more than
-  // they save.
+  // Blocks that share a tile's group of heads (GS; the heads need not divide evenly). All 512 blocks that fit on the chip at
+  // once start together, and under a causal mask the first tile then takes twice the average: B1 S8192, 32 over 8 heads, runs
+  // 2194 us with one block a tile (512 blocks), 2077 with two and 2110 with four (more partial sums). So a block's heads
+  // are halved while there are at most 1024 blocks (71 over 1 head of 64, B1 S8192: 21.5 ms undivided, 2.57 at 15 blocks a
+  // tile, 2.66 at 71; 28 over 4 of 128, B2 S8192: 3.68, 3.54 at two, 3.59 at seven). Without a mask the work is even and it
+  // only matters that every CU has a block; a second one each pays where a block keeps 128 steps of 32 query rows (16 over 2 of
+  // 64, B1 S8192: 1413 -> 1134; 8 over 4 of 64, B16 S512: 58 -> 67). A block keeps at least 16 steps, of its heads' full length, or the
+  // sums cost more than they save. The float32 sums take 8 bytes for each channel of these blocks' 128 rows: 134 MB at most.
   const long kv_blocks = (VARLEN ? (Sk + rows - 1) / rows : (long)kv_tiles * seqs) * Hkv;
   const bool sums_ok = dk.stride(-3) % 4 == 0 && (VARLEN || dk.stride(0) % 4 == 0) &&
                        reinterpret_cast<uintptr_t>(dk.data_ptr()) % 8 == 0 && reinterpret_cast<uintptr_t>(dv.data_ptr()) % 8 == 0;
   int gs = 1;
-  for (int d = 2; d <= G && sums_ok && kv_blocks * gs <= (causal ? 512 : 255); ++d)
-    if (G % d == 0 && (long)((S_max + 31) / 32) * (G / d) >= 16) gs = d;
+  for (int most = G; most > 1 && sums_ok;) {
+    most = (most + 1) / 2;                     // heads of a block, and blocks that take
+    const int d = (G + most - 1) / most;
+    const long steps = (long)((S_max + 31) / 32) * (G / d);
+    if (steps < 16 || kv_blocks * d > (causal ? 1024 : steps >= 128 ? 512 : 510)) break;
+    gs = d;
+  }
   const long n_part = (VARLEN ? (long)Sk : (long)seqs * Sk) * Hkv * D;
   at::Tensor part;
   if (gs > 1) part = at::empty({gs * 2 * n_part}, q.options().dtype(at::kFloat));

@@ -61,6 +61,9 @@ def _inputs(B, S, H, G, D, seed=0):
     (1, 512, 8, 2, 128, True, None),        # four blocks share a tile's heads
     (1, 520, 6, 2, 64, True, None),         # three do
     (2, 640, 4, 1, 64, False, None),        # without a mask, too few blocks for the CUs
+    (1, 520, 71, 1, 64, True, None),        # a prime group: one head a block
+    (2, 1100, 71, 1, 64, True, None),       # blocks of three and of two heads
+    (1, 1100, 71, 1, 128, False, None),     # and of two and of one
     (1, 200, 4, 2, 64, True, -0.2),
     (1, 130, 2, 2, 128, False, -0.1),
     (1, 100, 2, 2, 64, True, 0.0),          # every visible key counts the same; no gradient of the scores
@@ -79,6 +82,34 @@ def test_dense(B, S, H, G, D, causal, scale):
             assert (a == 0).all(), name
         else:
             _near(a, b, name, lone=S == 1)
+
+
+@pytest.mark.parametrize("H,G,S,causal", [(71, 1, 8192, True), (28, 4, 8192, True), (71, 1, 8192, False), (8, 2, 8192, True)])
+def test_workspace_of_shared_heads_is_bounded(H, G, S, causal):
+    """The float32 sums of blocks that share a tile's heads stay below 8 bytes for each channel of 1024 tiles of 128 rows, also
+    where a group has no small divisor; every head still counts."""
+    from colossalai_amd.ops import kernels
+
+    D = 64
+    q, k, v, dout = _inputs(1, S, H, G, D)
+    out, lse = kernels().flash_attn_fwd(q, k, v, causal, D ** -0.5)
+    none = q.new_empty(0)
+    torch.cuda.synchronize()
+    torch.cuda.reset_peak_memory_stats()
+    before = torch.cuda.memory_allocated()
+    grads = kernels().flash_attn_bwd(dout, q, k, v, out, lse, causal, D ** -0.5, none, none, none)
+    kept = sum(g.nbytes for g in grads) + lse.nbytes
+    assert torch.cuda.max_memory_allocated() - before - kept <= 1024 * 128 * D * 8 + (4 << 20)
+    # a group's dV is linear in its heads' dout: all heads together are the sum of the heads one by one
+    want = torch.zeros_like(v, dtype=torch.float32)
+    for h in range(H):
+        o1, l1 = kernels().flash_attn_fwd(q[:, :, h: h + 1].contiguous(), k[:, :, h // (H // G)][:, :, None].contiguous(),
+                                          v[:, :, h // (H // G)][:, :, None].contiguous(), causal, D ** -0.5)
+        d1 = kernels().flash_attn_bwd(dout[:, :, h: h + 1].contiguous(), q[:, :, h: h + 1].contiguous(),
+                                      k[:, :, h // (H // G)][:, :, None].contiguous(),
+                                      v[:, :, h // (H // G)][:, :, None].contiguous(), o1, l1, causal, D ** -0.5, none, none, none)
+        want[:, :, h // (H // G)] += d1[2][:, :, 0].float()
+    _near(grads[2], want, "dv")
 
 
 def test_padded_rows_with_shared_heads():
