@@ -98,7 +98,7 @@ DEV_INLINE float block_reduce_max(float v, float* smem) {
 }
 
 // ------------------------------------------- subtiled LDS tiles + tr-read
-// Shared by flash_attn.hip / grouped_gemm.hip. "Subtiled row-major":
+// Tiles of grouped_gemm.hip; flash_attn.hip and the serving kernels share ld_tr16. "Subtiled row-major":
 // [COLS/16 groups][ROWS][16 bf16], 32 B row pitch, 16 B pad between groups.
 // Row-slice fragment reads (8 consecutive cols at fixed row) are single
 // 16 B vector loads; column fragments use ds_read_b64_tr_b16 (HW-verified

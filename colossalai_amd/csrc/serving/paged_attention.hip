@@ -15,8 +15,10 @@
 // lane takes the full dot product of its key with the query (query in LDS,
 // key row read with its own page lookup). Online softmax in float32 across
 // the 64-key blocks. Phase 2: lane = value channel, the block's weights and
-// pool rows are broadcast from LDS. A prompt portion and a decode token run
-// the same code, so a position's result depends on nothing but the pages.
+// pool rows are broadcast from LDS. A prompt portion and a decode token can run
+// the same code. The other forms sum the same float32 terms in an order that depends on the call as well
+// (decode: on the number of tokens and the width of the page table, which choose heads a block and parts
+// of the keys), so that a position's results agree to rounding and not bit for bit.
 // Calls without a distance table, block summaries or cross values run the form in row_attention.hip
 // where the row sizes fit it; bfloat16 prompt portions run the matrix-core kernel.
 #include "paged_attention.h"

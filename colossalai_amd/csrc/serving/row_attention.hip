@@ -12,9 +12,9 @@
 // have their keys cut into parts, one block each, whose states row_merge_kernel puts together.
 //
 // What bounds it: the chain of dependent loads (position, page table, rows) and the block's end, about 10 us
-// together, and beyond that the vector instructions of the products; 16 x 1024 keys of 16/4 heads of 128 run 18.9 us (29.8
-// before the base-2 scores and the halving butterfly), 1.8 TB/s; 4 x 16384 run 44 us (193 with one block per token,
-// kv head and head), 3.0 TB/s.
+// together, and beyond that the vector instructions of the products. 16 x 1024 keys of 16/4 heads of 128 with a cap and a sink
+// take 17.8 us (29.3 before the base-2 scores and the halving butterfly), 1.9 TB/s; 4 x 16384 take 51.5 us (242 with one
+// block per token, kv head and head), 40 of it the parts at 3.4 TB/s and 7 the merge.
 #include "paged_attention.h"
 
 #include <algorithm>
@@ -406,7 +406,7 @@ bool launch_row_attention(at::Tensor& out, const at::Tensor& q, const at::Tensor
   // against 44.0; 16 x 6000, 32/8 heads: 221 against 113; four heads do not fit into the registers: 166).
   // Then the keys are cut into parts while there are fewer blocks than CUs and a part still gives every wave a key
   // block: 4 x 16384 210 -> 44 us, 8 x 2048 26.6 -> 19.1, 1 x 4096 36 -> 18. More blocks than CUs are slower again (4 x 16384
-  // with 512 blocks 76 us): a block costs about 10 us by itself. One or two blocks stop at the parts that the merge takes.
+  // with 512 blocks 76 us): a block costs about 10 us by itself. (All repeated on the same keys.) One or two blocks stop at the parts that the merge takes.
   int rc = R > 1 && (N * G * ((R + 1) / 2) >= 256 || keys >= 8192) ? 2 : 1;
   int splits = 1;
   const long blocks = N * G * ((R + rc - 1) / rc);

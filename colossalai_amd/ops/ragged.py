@@ -4,8 +4,9 @@ One engine step runs ``N`` new tokens that belong to ``B`` live sequences:
 a prompt portion of any length next to single decode tokens. Every op that
 carries per-sequence memory (paged keys/values, recurrent matrices, the tail
 of a short convolution, the previous token of a token shift) takes this
-descriptor instead of a dense ``[B, S]`` layout, so that a result never
-depends on how a prompt was cut or on what else shares the step.
+descriptor instead of a dense ``[B, S]`` layout, so that a result does not
+depend, but for the order of float32 sums, on how a prompt was cut or on what
+else shares the step.
 """
 
 from dataclasses import dataclass
