@@ -40,6 +40,8 @@
 #include <torch/extension.h>
 #include <ATen/hip/HIPContext.h>
 
+#include <algorithm>
+
 #include "common.h"
 
 namespace cai {
@@ -838,14 +840,15 @@ __global__ __launch_bounds__(fa::NTB, 2) void fa_bwd_kernel(
     unsigned short* __restrict__ dQ, unsigned short* __restrict__ dK, unsigned short* __restrict__ dV,
     float* __restrict__ PART, int GS, const int* __restrict__ CU, const int* __restrict__ CUK,
     long qbs, long qts, long kbs, long kts, long dqbs, long dqts, long dkbs, long dkts,
-    int n_kv, int kv_tiles, int q_tiles, int B, int S, int Sk, int Hq, int Hkv, float scale, int causal) {
+    int n_kv, int n_q, int kv_tiles, int q_tiles, int B, int S, int Sk, int Hq, int Hkv, float scale, int causal) {
   extern __shared__ char smem[];
-  const int f = (int)blockIdx.x;
+  const int f = (int)(blockIdx.y * gridDim.x + blockIdx.x);   // more than one grid row only beyond 2^23 blocks
+  if (f >= n_kv + n_q) return;
   if (f < n_kv)
     bwd_dkdv<D, VARLEN>(smem, f, n_kv, Q, K, V, dO, LSE, DELTA, dK, dV, PART, GS, CU, CUK, qbs, qts, kbs, kts, dkbs, dkts,
                         kv_tiles, B, S, Sk, Hq, Hkv, scale, causal);
   else
-    bwd_dq<D, VARLEN>(smem, f - n_kv, (int)gridDim.x - n_kv, Q, K, V, dO, LSE, DELTA, dQ, CU, CUK, qbs, qts, kbs, kts,
+    bwd_dq<D, VARLEN>(smem, f - n_kv, n_q, Q, K, V, dO, LSE, DELTA, dQ, CU, CUK, qbs, qts, kbs, kts,
                       dqbs, dqts, q_tiles, B, S, Sk, Hq, Hkv, scale, causal);
 }
 
@@ -1029,15 +1032,18 @@ void launch_bwd(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, c
   const long n_part = (VARLEN ? (long)Sk : (long)seqs * Sk) * Hkv * D;
   at::Tensor part;
   if (gs > 1) part = at::empty({gs * 2 * n_part}, q.options().dtype(at::kFloat));
-  const int n_kv = (kv_tiles * seqs * Hkv * gs + 7) / 8 * 8, n_q = q_tiles * seqs * Hq;
+  const long n_kv = ((long)kv_tiles * seqs * Hkv * gs + 7) / 8 * 8, n_q = (long)q_tiles * seqs * Hq, blocks = n_kv + n_q;
+  TORCH_CHECK(blocks < (1L << 31) - (1L << 23), "flash_attn_bwd: too many tiles");
+  // a grid dimension of 2^32 threads or more is cut short without an error: packed batches of very many sequences get there
+  const long width = std::max(1L, std::min(blocks, 1L << 23));
   auto kernel = fa_bwd_kernel<D, VARLEN>;
   set_lds_limit((const void*)kernel, bwd_lds<D>());
-  hipLaunchKernelGGL(kernel, dim3(n_kv + n_q), dim3(NTB), bwd_lds<D>(), stream,
+  hipLaunchKernelGGL(kernel, dim3((unsigned)width, (unsigned)((blocks + width - 1) / width)), dim3(NTB), bwd_lds<D>(), stream,
                      (const unsigned short*)q.data_ptr(), (const unsigned short*)k.data_ptr(),
                      (const unsigned short*)v.data_ptr(), (const unsigned short*)dout.data_ptr(), lse.data_ptr<float>(),
                      delta.data_ptr<float>(), (unsigned short*)dq.data_ptr(), (unsigned short*)dk.data_ptr(),
                      (unsigned short*)dv.data_ptr(), gs > 1 ? part.data_ptr<float>() : nullptr, gs, cu, cuk, qbs, qts, kbs,
-                     kts, dqbs, dqts, dkbs, dkts, n_kv, kv_tiles, q_tiles, seqs, S, Sk, Hq, Hkv, scale, causal ? 1 : 0);
+                     kts, dqbs, dqts, dkbs, dkts, (int)n_kv, (int)n_q, kv_tiles, q_tiles, seqs, S, Sk, Hq, Hkv, scale, causal ? 1 : 0);
   HIP_CHECK_LAST();
   if (gs > 1) {
     hipLaunchKernelGGL(fa_bwd_sum_kernel, dim3((unsigned)((n_part / 4 + 255) / 256)), dim3(256), 0, stream,

@@ -148,6 +148,31 @@ def test_packed(lens, H, G, D):
         at += n
 
 
+def test_packed_backward_with_very_many_sequences():
+    """More blocks than one grid dimension holds threads for: many short sequences beside one that is long."""
+    from colossalai_amd.ops import flash_attention_varlen
+
+    lens = [1] * 65000
+    lens[30000] = 32768
+    total, D = sum(lens), 64
+    q, k, v, dout = (t[0] for t in _inputs(1, total, 1, 1, D))
+    cu = torch.tensor([0] + lens).cumsum(0).int().cuda()
+    for t in (q, k, v):
+        t.requires_grad_()
+    out = flash_attention_varlen(q, k, v, cu, max(lens), causal=True)
+    got = torch.autograd.grad(out, (q, k, v), dout)
+    # the long one by itself, through a batch of one
+    one = slice(30000, 30000 + 32768)
+    alone = [t[one].detach().requires_grad_() for t in (q, k, v)]
+    out1 = flash_attention_varlen(*alone, torch.tensor([0, 32768], dtype=torch.int32, device="cuda"), 32768, causal=True)
+    for name, a, w in zip(("dq", "dk", "dv"), got, torch.autograd.grad(out1, alone, dout[one])):
+        _near(a[one], w, name)
+    # a token that sees itself only: its value's gradient is dout
+    short = torch.ones(total, dtype=torch.bool, device="cuda")
+    short[one] = False
+    assert torch.equal(got[2][short], dout[short])
+
+
 def test_strided_gradients_with_shared_heads():
     """dk/dv as views into one packed buffer, filled by the kernel that adds the partial sums."""
     from colossalai_amd.ops import kernels
