@@ -41,9 +41,10 @@ DEV_INLINE void ce_merge(float& m, float& s, float om, float os) {
 template <bool VEC>
 __global__ __launch_bounds__(CE_BLOCK) void ce_fwd_kernel(float* __restrict__ lse, float* __restrict__ nll,
                                                           const unsigned short* __restrict__ logits,
-                                                          const long* __restrict__ labels, long ignore_index, int V) {
+                                                          const long* __restrict__ labels, long ignore_index, long rows, int V) {
   __shared__ float sm[CE_BLOCK / WAVE], ss[CE_BLOCK / WAVE];
-  const long row = blockIdx.x;
+  const long row = (long)blockIdx.y * gridDim.x + blockIdx.x;
+  if (row >= rows) return;
   const unsigned short* x = logits + row * V;
   float m = -INFINITY, s = 0.0f;
   if (VEC) {
@@ -91,8 +92,10 @@ __global__ __launch_bounds__(CE_BLOCK) void ce_fwd_kernel(float* __restrict__ ls
 template <bool VEC>
 __global__ __launch_bounds__(CE_BLOCK) void ce_bwd_kernel(unsigned short* __restrict__ logits, const float* __restrict__ lse,
                                                           const long* __restrict__ labels, const float* __restrict__ grad,
-                                                          const float* __restrict__ loss, long ignore_index, int V) {
-  const long row = blockIdx.x;
+                                                          const float* __restrict__ loss, long ignore_index, long rows,
+                                                          int V) {
+  const long row = (long)blockIdx.y * gridDim.x + blockIdx.x;
+  if (row >= rows) return;
   unsigned short* x = logits + row * V;
   const long label = labels[row];
   const float scale = (label == ignore_index ? 0.0f : label >= 0 && label < V ? 1.0f : NAN) * (grad[0] / loss[1]);
@@ -164,6 +167,12 @@ static bool ce_vec(const at::Tensor& logits) {
   return logits.size(1) % 8 == 0 && reinterpret_cast<uintptr_t>(logits.data_ptr()) % 16 == 0;
 }
 
+// A block a row. A grid dimension of 2^32 threads or more is cut short without an error: from 2^20 rows on it is two.
+static dim3 ce_grid(long rows) {
+  const long width = rows < (1L << 20) ? rows : 1L << 20;
+  return dim3((unsigned)width, (unsigned)((rows + width - 1) / width));
+}
+
 void ce_fwd(at::Tensor logits, at::Tensor labels, int64_t ignore_index, at::Tensor lse, at::Tensor nll) {
   check_ce(logits, labels, lse);
   check_ce(logits, labels, nll);
@@ -171,9 +180,9 @@ void ce_fwd(at::Tensor logits, at::Tensor labels, int64_t ignore_index, at::Tens
   if (rows == 0) return;
   auto stream = at::hip::getCurrentHIPStream();
   auto kernel = ce_vec(logits) ? ce_fwd_kernel<true> : ce_fwd_kernel<false>;
-  hipLaunchKernelGGL(kernel, dim3((unsigned)rows), dim3(CE_BLOCK), 0, stream.stream(), lse.data_ptr<float>(),
+  hipLaunchKernelGGL(kernel, ce_grid(rows), dim3(CE_BLOCK), 0, stream.stream(), lse.data_ptr<float>(),
                      nll.data_ptr<float>(), (const unsigned short*)logits.data_ptr(), (const long*)labels.data_ptr(),
-                     (long)ignore_index, (int)logits.size(1));
+                     (long)ignore_index, rows, (int)logits.size(1));
   HIP_CHECK_LAST();
 }
 
@@ -185,9 +194,9 @@ void ce_bwd(at::Tensor logits, at::Tensor labels, int64_t ignore_index, at::Tens
   if (rows == 0) return;
   auto stream = at::hip::getCurrentHIPStream();
   auto kernel = ce_vec(logits) ? ce_bwd_kernel<true> : ce_bwd_kernel<false>;
-  hipLaunchKernelGGL(kernel, dim3((unsigned)rows), dim3(CE_BLOCK), 0, stream.stream(), (unsigned short*)logits.data_ptr(),
+  hipLaunchKernelGGL(kernel, ce_grid(rows), dim3(CE_BLOCK), 0, stream.stream(), (unsigned short*)logits.data_ptr(),
                      lse.data_ptr<float>(), (const long*)labels.data_ptr(), grad.data_ptr<float>(), loss.data_ptr<float>(),
-                     (long)ignore_index, (int)logits.size(1));
+                     (long)ignore_index, rows, (int)logits.size(1));
   HIP_CHECK_LAST();
 }
 

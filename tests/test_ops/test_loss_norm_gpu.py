@@ -55,6 +55,22 @@ def test_loss_keeps_float32_precision(rows, V):
     assert abs(loss - want) < 2.0 ** -20
 
 
+def test_a_chunk_of_very_many_rows():
+    """More rows than one launch holds threads for."""
+    from colossalai_amd.ops.fused_ce import fused_linear_cross_entropy
+
+    N, V, H = (1 << 24) + 5, 8, 8
+    torch.manual_seed(0)
+    hidden = torch.randn(N, H, device="cuda").bfloat16().requires_grad_()
+    weight = torch.randn(V, H, device="cuda").bfloat16()
+    labels = torch.randint(0, V, (N,), device="cuda")
+    got = []
+    for chunk in (1 << 16, N):
+        loss = fused_linear_cross_entropy(hidden, weight, labels, chunk_size=chunk)
+        got.append((loss, torch.autograd.grad(loss * N, hidden)[0]))
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
+
+
 def test_cross_entropy_without_a_row_that_counts():
     from colossalai_amd.ops.fused_ce import fused_linear_cross_entropy
 
