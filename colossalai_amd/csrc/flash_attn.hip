@@ -254,8 +254,8 @@ __global__ __launch_bounds__(NW * 64, 2) void fa_fwd_kernel(
     }
   }
 
-  // |scale| * log2(e); a scale of 0 must not meet a masked score of -inf in a product
-  const float scale2 = fmaxf(fabsf(scale) * 1.44269504f, 1e-30f);
+  // |scale| * log2(e); a scale of 0 must not meet a masked score of -inf in a product, one of NaN stays (fmaxf drops it)
+  const float scale_abs = fabsf(scale) * 1.44269504f, scale2 = scale_abs < 1e-30f ? 1e-30f : scale_abs;
   f32x16 oacc[D / 32];                              // O^T: column = q row (ln), rows = channels
 #pragma unroll
   for (int nb = 0; nb < D / 32; ++nb)

@@ -511,7 +511,8 @@ __global__ __launch_bounds__(256 * NG, 2) void paged_attention_mfma_kernel(
 #pragma unroll
     for (int i = 0; i < 16; ++i) oacc[t][i] = 0.0f;
   constexpr float LOG2E = 1.4426950408889634f;
-  const float c1 = fmaxf(scale * LOG2E, 1e-30f), sl2 = slope * LOG2E;  // a scale of 0 must not meet -inf in a product
+  // a scale of 0 must not meet -inf in a product, one of NaN stays (fmaxf drops it)
+  const float c1 = scale * LOG2E < 1e-30f ? 1e-30f : scale * LOG2E, sl2 = slope * LOG2E;
   // soft cap in the base-2 domain: cap log2e tanh(x scale / cap), tanh(y) = 1 - 2 / (exp2(2 log2e y) + 1)
   const bool capped = softcap > 0.0f;
   const float inv_cap = capped ? scale / softcap : 0.0f;

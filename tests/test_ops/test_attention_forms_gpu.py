@@ -148,6 +148,14 @@ def test_packed(lens, H, G, D):
         at += n
 
 
+@pytest.mark.parametrize("causal", [True, False])
+def test_a_scale_of_nan_shows(causal):
+    from colossalai_amd.ops import flash_attention
+
+    q, k, v, _ = _inputs(1, 70, 2, 1, 64)
+    assert torch.isnan(flash_attention(q, k, v, causal=causal, scale=float("nan")).float()).all()
+
+
 def test_packed_backward_with_very_many_sequences():
     """More blocks than one grid dimension holds threads for: many short sequences beside one that is long."""
     from colossalai_amd.ops import flash_attention_varlen

@@ -127,6 +127,17 @@ def test_nan_stays_nan(counts, kw):
     assert torch.equal(bad, want) and torch.equal(some, want)
 
 
+@pytest.mark.parametrize("counts", [[1], [40]])
+@pytest.mark.parametrize("kw", [{}, dict(softcap=5.0, sink=True), dict(chunk=64)])
+def test_a_scale_of_nan_shows(counts, kw):
+    from colossalai_amd.ops.paged_attention import paged_attention
+
+    batch, pages = _batch(counts, [100], 16)
+    k, v = (torch.randn(pages, 16, 2, 64, device="cuda").bfloat16() for _ in range(2))
+    q = torch.randn(sum(counts), 4, 64, device="cuda").bfloat16()
+    assert torch.isnan(paged_attention(q, k, v, batch, float("nan"), **kw).float()).all()
+
+
 @pytest.mark.parametrize("spread", [0.02, 0.1, 0.5])
 def test_capped_scores_keep_float32_precision(spread):
     """A decode token that sees one key and the sink returns p = 1 / (1 + exp(-s)) of its value 1: s can be read back."""
