@@ -289,7 +289,7 @@ std::vector<at::Tensor> rmsnorm_bwd(at::Tensor dy, at::Tensor x, at::Tensor weig
   auto stream = at::hip::getCurrentHIPStream();
   at::Tensor part;
   int grid = 0;
-  // 1024 blocks are 16 waves a CU, all at once where a thread holds one or two groups (67 to 114 registers) and in two rounds
+  // 1024 blocks are 16 waves a CU, all at once where a thread holds one or two groups (67 to 114 registers) and in two turns
   // where it holds four (190 and 199: 8 waves a CU); their partial rows are 4 KB per 1024 channels each, which a block of a row's
   // width makes up for with at least four rows
   RMS_DISPATCH(H, {
