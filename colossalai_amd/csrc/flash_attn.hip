@@ -3,8 +3,8 @@
 // MI355X-native design (not a CUDA port):
 //  - mfma_f32_32x32x16_bf16 tiles; 64-wide waves; a wave owns 32 query rows (forward,
 //    dQ) or 32 key/value rows (dK/dV); blocks of 4 waves, 2 for small forward grids.
-//  - ALL operand tiles live in LDS in ONE layout, planes of 8 channels
-//    (tile_off below). Row-slice fragment reads (8 consecutive d at a fixed row) are
+//  - ALL operand tiles live in LDS in ONE layout, pieces of 16 rows of 32 channels (piece_at below), which global loads
+//    write directly. Row-slice fragment reads (8 consecutive d at a fixed row) are
 //    single 16 B loads; COLUMN fragment reads use gfx950's ds_read_b64_tr_b16.
 //    HW-verified semantics (mfma_selftest.hip): each lane reads 64 bits at its own
 //    address; within a 16-lane group, out[l][j] = pool[(l&15) + 16 j] where pool is
@@ -13,24 +13,26 @@
 //  - No intermediate passes through LDS: every product whose operand is a result (P · V,
 //    P^T · dO, dS^T · Q, dS · K) is arranged so that the contracted index lies in a lane's
 //    registers, and takes them in the order of the C layout (frag_born).
-//  - All global loads of the next tile issue before the current tile's products; two LDS
+//  - The next tile's loads are spread over the current tile's products; two LDS
 //    buffers, one barrier a tile.
+//  - What differs from wave to wave but not inside one (masks on the diagonal, the last tile) is a scalar branch
+//    with a body of its own; masks merged into the common body were half of its vector instructions.
 //  - backward: delta preprocess, then ONE launch whose blocks take key/value tiles (dK/dV)
 //    or query tiles (dQ); both form the scores again.
 //
-// What bounds it (B2 S2048 H16/8 D128, not causal): the matrix unit is busy 41 % of the forward and 43 % of the
-// backward, the vector unit 40 %. The two waves of a SIMD overlap little of their products and exponentials;
-// without the softmax the forward would run 1048 TFLOP/s, without global loads 1099, with neither 1337, at the 2.1 GHz
-// the card keeps under this load. Running the two waves one phase apart with barriers (726 TFLOP/s), forming the next
-// tile's scores under the softmax (830 at 245 registers, 196 at D64 for want of waves) and eight-wave blocks were
-// measured against the 835 of this form before the staging addresses became scalars.
+// What bounds it (B1 S8192 H32/8 D128 causal): with loads through registers and a maximum per tile, a tile took a wave 4034
+// cycles, of which 557 went into issuing the loads, 638 into storing them, 150 into the barrier; the products and the
+// softmax, 890 cycles each, overlap little between the two waves of a SIMD. The matrix unit is now busy half of the time, at
+// the 1.9 GHz that the card keeps under this load. Fragments read further ahead for P · V, other wave
+// priorities (a fixed order of a SIMD's two waves), and exponentials placed between the products changed nothing.
 //
-// TFLOP/s, forward 2 products / backward 5 products of the visible pairs, before -> after:
-//   B4 S4096 H32 D128 causal          forward 694 -> 807, backward 498 -> 635
-//   B1 S8192 H32/8 D128 causal        forward 730 -> 972, backward 490 -> 686
-//   B8 S1024 H12 D64 causal           forward 215 -> 357, backward 225 -> 327
-//   B16 S512 H12 D64                  forward 361 -> 542, backward 294 -> 458
-//   packed, 10 sequences of 256..4096 forward 216 -> 714, backward 197 -> 584
+// TFLOP/s, forward 2 products / backward 5 products of the visible pairs, with loads through registers -> now:
+//   B4 S4096 H32 D128 causal          forward 768 -> 930, backward 599 -> 693
+//   B1 S8192 H32/8 D128 causal        forward 888 -> 1040, backward 659 -> 761
+//   B2 S4096 H16/8 D128               forward 928 -> 1072, backward 699 -> 807
+//   B8 S1024 H12 D64 causal           forward 348 -> 424, backward 328 -> 395
+//   B16 S512 H12 D64                  forward 524 -> 582, backward 430 -> 501
+//   packed, 14 sequences of 256..4096, 32/8 heads   forward 608 -> 810, backward 535 -> 632
 //
 // Shapes: q [B,S,Hq,D], k/v [B,S,Hkv,D] ("bshd" — no transposes in the
 // model), D in {64,128}. lse/delta are [B,Hq,S] fp32.
@@ -41,13 +43,13 @@
 #include <ATen/hip/HIPContext.h>
 
 #include <algorithm>
+#include <type_traits>
 
 #include "common.h"
 
 namespace cai {
 
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
-typedef __bf16 bf16x4v_t __attribute__((ext_vector_type(4)));
 
 namespace fa {
 
@@ -60,41 +62,51 @@ DEV_INLINE bf16x8_t ld_g16(const unsigned short* p) {
   return *reinterpret_cast<const bf16x8_t*>(p);
 }
 
-DEV_INLINE void st_lds16(char* lds, int byte, bf16x8_t v) {
-  *reinterpret_cast<bf16x8_t*>(lds + byte) = v;
-}
-
-DEV_INLINE bf16x8_t ld_lds16(const char* lds, int byte) {
-  return *reinterpret_cast<const bf16x8_t*>(lds + byte);
-}
-
 // C-layout row for mfma_f32_32x32x16 register j (guide §3, HW-verified).
 DEV_INLINE constexpr int crow(int j, int half) { return (j & 3) + 8 * (j >> 2) + 4 * half; }
 
-// An operand tile in LDS: planes of 8 channels, [D/8][ROWS][8], 16 bytes a row, 64 bytes between the planes. Every
-// access spreads over the 64 banks: a row-slice fragment (ds_read_b128) reads 32 neighbouring rows of a plane per half-wave,
-// 512 contiguous bytes (4.3 cycles a wave; 8.5 with rows of 32 bytes); a transposing read takes 64 bytes from each
-// of four neighbouring planes at a time; a staging store writes 16 rows of four planes. Against column groups of 16
-// channels: forward 883 -> 917, backward 651 -> 656 TFLOP/s at B2 S2048 H16/8 D128.
+// An operand tile in LDS: pieces of 16 rows of 32 channels, 1024 bytes each, all row groups of a channel group one after the
+// other. In a piece the four 16-byte units of a row lie together, unit u at place u ^ (row / 4 % 4). A piece is what
+// one load instruction of a wave brings straight into LDS (16 bytes a lane in lane order, a quad of lanes 64 neighbouring bytes of a
+// row), and every access spreads over the 64 banks: a row fragment (ds_read_b128) takes one unit of 16 consecutive
+// rows, which lie in 16 different places of 16 bytes; a transposing read takes rows 0-7 or 8-15 of a piece as a whole.
 template <int ROWS>
-__host__ __device__ constexpr int tile_pitch() { return ROWS * 16 + 64; }
-
-template <int ROWS>
-DEV_INLINE int tile_off(int row, int col) { return (col >> 3) * tile_pitch<ROWS>() + row * 16 + (col & 7) * 2; }
+__host__ __device__ constexpr int piece_at(int row, int col) { return ((col >> 5) * (ROWS / 16) + (row >> 4)) * 1024; }
 
 template <int ROWS, int COLS>
-__host__ __device__ constexpr int tile_bytes() { return (COLS / 8) * tile_pitch<ROWS>(); }
+__host__ __device__ constexpr int tile_bytes() { return ROWS * COLS * 2; }
+
+// Where a lane's 8 channels 16 * sl + 8 * half of row `ln` (and every 32nd row from it) lie: `even` for even sl, `odd` for
+// odd ones, beyond which a fragment's piece is a constant.
+struct RowAt {
+  int even, odd;
+  DEV_INLINE RowAt(int ln, int half) {
+    const int place = half ^ (ln >> 2 & 3), at = (ln >> 4) * 1024 + (ln & 15) * 64;
+    even = at + place * 16;
+    odd = at + (place ^ 2) * 16;
+  }
+};
+template <int ROWS>
+DEV_INLINE bf16x8_t frag_row(const char* tile, const RowAt& at, int row0, int sl) {
+  return *reinterpret_cast<const bf16x8_t*>(tile + (sl & 1 ? at.odd : at.even) + piece_at<ROWS>(row0, sl * 16));
+}
 
 // Column fragment by transposing reads, in the order in which the C layout hands out its rows: lane l
-// receives tile[k_base + 8*(e>>2) + 4*(l>>5) + (e&3)][cg_base*16 + (l&31)], e = 0..7, so
+// receives tile[k_base + 8*(e>>2) + 4*(l>>5) + (e&3)][col + (l&31)], e = 0..7, so
 // that a packed run of eight C registers is the matching other operand.
+struct ColAt {
+  int lo, hi;
+  DEV_INLINE explicit ColAt(int lane) {
+    const int m = lane & 15, half = lane >> 5;
+    const int unit = (lane >> 4 & 1) * 2 + (m >> 1 & 1), row = half * 4 + (m >> 2);
+    lo = row * 64 + (unit ^ half) * 16 + (m & 1) * 8;
+    hi = (row + 8) * 64 + (unit ^ half ^ 2) * 16 + (m & 1) * 8;
+  }
+};
 template <int ROWS>
-DEV_INLINE bf16x8_t frag_born(const char* tile, int lane, int k_base, int cg_base) {
-  const int m = lane & 15;
-  const int plane = (cg_base + ((lane >> 4) & 1)) * 2 + ((m & 3) >> 1);
-  const int at = plane * tile_pitch<ROWS>() + (k_base + (lane >> 5) * 4 + (m >> 2)) * 16 + (m & 1) * 8;
-  const bf16x4_v lo = ld_tr16(tile, at);
-  const bf16x4_v hi = ld_tr16(tile, at + 8 * 16);
+DEV_INLINE bf16x8_t frag_born(const char* tile, const ColAt& at, int k_base, int col) {
+  const bf16x4_v lo = ld_tr16(tile, at.lo + piece_at<ROWS>(k_base, col));
+  const bf16x4_v hi = ld_tr16(tile, at.hi + piece_at<ROWS>(k_base, col));
   return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
 }
 
@@ -119,58 +131,48 @@ DEV_INLINE int xcd_chunk(int f, int nblocks) {
   return (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + (f >> 3);
 }
 
-// Register-staged tile for async-split staging: global loads for tile t+1 are ISSUED before tile t's compute
-// (results land in registers under the MFMAs), LDS writes happen after it.
-//
-// A wave's instruction covers 16 rows of 64 bytes: with whole rows per instruction the stores of a row's column
-// groups met in the same LDS banks. Chunk i of a thread lies a fixed number of rows and columns from its
-// chunk 0, so that a whole tile's addresses are one offset per thread and scalars; only a tile that reaches past the last
-// row (or rows very far apart) forms an address per chunk. (Addresses of eight chunks, clamped and multiplied out for every tile, were a third of the
-// forward's vector instructions.)
-template <int D, int ROWS, int NT_>
-struct RegStage {
-  static constexpr int NCH = ROWS * (D / 8) / NT_;
-  static constexpr int WAVES = NT_ / 64, QUADS = D / 32;  // 64-byte pieces of a row
-  static_assert(ROWS * (D / 8) % NT_ == 0, "RegStage: uneven chunking");
-  static_assert(QUADS % WAVES == 0 || WAVES % QUADS == 0, "RegStage: chunks must lie at fixed distances");
-  bf16x8_t r[NCH];
+// A tile's way from memory into LDS, without registers in between: a wave brings PER pieces, each with one load
+// instruction, which is issued wherever the caller wants it between the products of the tile before. (All of a tile's loads
+// issued together held the waves up for 557 of the 4034 cycles a tile took, at 64 bytes a cycle of address and cache
+// work, and its LDS stores, which met in the banks, for another 638: B1 S8192 H32/8 D128 causal.)
+// Rows past the matrix' end come as zeros: the buffer descriptor of a tile ends with its last row, and is made
+// anew for each tile, so that a matrix may be of any size; rows less than 2^23 elements apart (offsets stay under 2^31).
+typedef __attribute__((address_space(3))) void* lds_ptr;
 
-  DEV_INLINE static constexpr int rows_to(int i) { return i * WAVES / QUADS * 16; }
-  DEV_INLINE static constexpr int cols_to(int i) { return i * WAVES % QUADS * 32; }
-  DEV_INLINE static int row0_of() { return (int)(threadIdx.x >> 6) / QUADS * 16 + (int)((threadIdx.x & 63) >> 2); }
-  DEV_INLINE static int col0_of() { return ((int)(threadIdx.x >> 6) % QUADS * 4 + (int)(threadIdx.x & 3)) * 8; }
+template <int D, int ROWS, int WAVES>
+struct TileLoad {
+  static constexpr int RG = ROWS / 16, PIECES = RG * (D / 32), PER = PIECES / WAVES;
+  static_assert(PIECES % WAVES == 0, "TileLoad: uneven pieces");
+  const unsigned short* base;
+  long stride;
+  int rows;            // of the matrix
+  unsigned off;        // bytes from a piece's first element to this lane's
 
-  // Bytes from a tile's first element to this thread's chunk 0, for rows less than 2^25 elements apart.
-  DEV_INLINE static unsigned offset(long tok_stride) { return (unsigned)(row0_of() * tok_stride + col0_of()) * 2u; }
-
-  DEV_INLINE void load(const unsigned short* base, long tok_stride, unsigned off, int row0, int S) {
-    if (row0 + ROWS <= S && tok_stride < (1L << 25)) {
-#pragma unroll
-      for (int i = 0; i < NCH; ++i)
-        r[i] = *reinterpret_cast<const bf16x8_t*>(
-            reinterpret_cast<const char*>(base + (row0 + rows_to(i)) * tok_stride + cols_to(i)) + off);
-    } else {
-#pragma unroll
-      for (int i = 0; i < NCH; ++i) {
-        const int grow = max(min(row0 + row0_of() + rows_to(i), S - 1), 0);
-        r[i] = ld_g16(base + (long)grow * tok_stride + col0_of() + cols_to(i));
-      }
-    }
+  DEV_INLINE TileLoad(const unsigned short* base, long stride, int rows) : base(base), stride(stride), rows(rows) {
+    const int r = (threadIdx.x & 63) >> 2, unit = (threadIdx.x & 3) ^ (r >> 2 & 3);
+    off = (unsigned)(r * stride) * 2u + unit * 16;
   }
-  DEV_INLINE void store(char* lds) const {
-    char* at = lds + tile_off<ROWS>(row0_of(), col0_of());
+  // what the loads of the tile from row0 on share
+  DEV_INLINE __amdgpu_buffer_rsrc_t tile(int row0) const { return tile(base, row0); }
+  DEV_INLINE __amdgpu_buffer_rsrc_t tile(const unsigned short* base, int row0) const {   // of another matrix of these rows
+    const int left = min(rows - row0, ROWS);
+    const unsigned bytes = left > 0 ? (unsigned)((left - 1) * stride + D) * 2u : 0u;
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<unsigned short*>(base + (left > 0 ? row0 * stride : 0)), 0, (int)bytes, 0x00027000);
+  }
+  // piece i (of PER) of wave w
+  DEV_INLINE void piece(__amdgpu_buffer_rsrc_t t, char* __restrict__ lds, int w, int i) const {
+    const int c = w + WAVES * i, rg = c % RG, cg = c / RG;
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(t, (lds_ptr)(lds + c * 1024), 16, (int)off, (int)(unsigned)((rg * 16 * stride + cg * 32) * 2), 0, 0);
+  }
+  DEV_INLINE void all(int row0, char* __restrict__ lds, int w) const {
+    const auto t = tile(row0);
 #pragma unroll
-    for (int i = 0; i < NCH; ++i) st_lds16(at, tile_off<ROWS>(rows_to(i), cols_to(i)), r[i]);
+    for (int i = 0; i < PER; ++i) piece(t, lds, w, i);
   }
 };
 
-// Synchronous staging: load + store back-to-back (transient registers).
-template <int D, int ROWS, int NT_>
-DEV_INLINE void stage_direct(char* lds, const unsigned short* base, long stride, int row0, int S) {
-  RegStage<D, ROWS, NT_> st;
-  st.load(base, stride, st.offset(stride), row0, S);
-  st.store(lds);
-}
+// every load of this wave has arrived (in LDS); a barrier behind it makes that true for the block
+DEV_INLINE void loads_done() { __builtin_amdgcn_s_waitcnt(0x0f70); }   // vmcnt(0)
 
 }  // namespace fa
 
@@ -206,7 +208,7 @@ __global__ __launch_bounds__(NW * 64, 2) void fa_fwd_kernel(
   constexpr int NT = NW * 64;
   constexpr int KB_BYTES = tile_bytes<KVB, D>();
   const int lane = threadIdx.x & 63;
-  const int w = threadIdx.x >> 6;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);   // the same for a wave: what it decides is a scalar branch
   const int half = lane >> 5;
   const int ln = lane & 31;
 
@@ -262,6 +264,7 @@ __global__ __launch_bounds__(NW * 64, 2) void fa_fwd_kernel(
 #pragma unroll
     for (int j = 0; j < 16; ++j) oacc[nb][j] = 0.0f;
   float m_run = -INFINITY, l_run = 0.0f;
+  float mref = -3.0e38f;   // what the weights are taken against: m_run, and below every finite score until a row has one
 
   const int kv_tiles_all = (SeffK + KVB - 1) / KVB;
   const int kv_tiles = causal ? min(kv_tiles_all, (min(q0 + NW * QW, Seff) + KVB - 1) / KVB) : kv_tiles_all;
@@ -274,32 +277,16 @@ __global__ __launch_bounds__(NW * 64, 2) void fa_fwd_kernel(
   char* Kbuf = smem;                 // [2] key tiles, then [2] value tiles
   char* Vbuf = smem + 2 * KB_BYTES;
 
-  // ---- S^T = K · Q^T : KVB/32 32-k blocks. C: col = q (ln), row = k (crow).
-  auto scores = [&](const char* Klds, f32x16 (&s)[KB]) {
-#pragma unroll
-    for (int kb = 0; kb < KB; ++kb)
-#pragma unroll
-      for (int j = 0; j < 16; ++j) s[kb][j] = 0.0f;
-#pragma unroll
-    for (int sl = 0; sl < DSL; ++sl) {
-#pragma unroll
-      for (int kb = 0; kb < KB; ++kb)
-        s[kb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-            ld_lds16(Klds, tile_off<KVB>(kb * 32 + ln, sl * 16 + half * 8)), qf[sl], s[kb], 0, 0, 0);
-    }
-  };
   // interior tiles (every row/col in range, strictly below the causal diagonal) need no mask:
   // at S=4096 that is ~94% of tiles, and the mask chain is ~4 VALU ops per score
   auto masked = [&](int k0) { return !((k0 + KVB <= SeffK) && (qw + QW <= Seff) && (!causal || k0 + KVB - 1 <= qw)); };
+  const int last_key = q_abs >= Seff ? -1 : causal ? min(q_abs, SeffK - 1) : SeffK - 1;   // the last key this row sees
   auto mask = [&](int k0, f32x16 (&s)[KB]) {
+    const int upto = last_key - k0 - 4 * half;
 #pragma unroll
     for (int kb = 0; kb < KB; ++kb)
 #pragma unroll
-      for (int j = 0; j < 16; ++j) {
-        const int k_abs = k0 + kb * 32 + crow(j, half);
-        const bool valid = (q_abs < Seff) && (k_abs < SeffK) && (!causal || k_abs <= q_abs);
-        if (!valid) s[kb][j] = -INFINITY;
-      }
+      for (int j = 0; j < 16; ++j) s[kb][j] = kb * 32 + crow(j, 0) > upto ? -INFINITY : s[kb][j];
   };
   auto largest = [&](const f32x16 (&s)[KB]) {
     float r = s[0][0];
@@ -310,23 +297,36 @@ __global__ __launch_bounds__(NW * 64, 2) void fa_fwd_kernel(
     return r;
   };
 
-  // ---- online softmax of a tile's 64 scores of q-row (qw+ln). The running maximum is kept in the
-  // base-2 domain (v_exp_f32 is exp2); the scale enters with the fma that subtracts it.
+  // ---- online softmax of a tile's 64 scores of q-row (qw+ln), in the base-2 domain (v_exp_f32 is exp2); the scale enters
+  // with the fma that subtracts the reference m_run. m_run is a maximum the row has had, not always its newest: the
+  // weights are taken against it as it stands, and only where their sum shows that some of them passed 2^12 (a row's first
+  // finite score gives inf; NaN counts too) is the maximum formed, m_run raised and the tile's weights taken
+  // again. The sum is needed anyway, so most tiles need no maximum, no exchange between the half-waves and no
+  // rescaling; float32 and bfloat16 hold a weight of 2^12 as precisely as one of 1.
   // P in the order it was born in is the B operand of O^T += V^T · P^T: slot half*8+e of a 16-k step holds
   // key 8*(e>>2) + 4*half + (e&3) of it, and the V column fragments are read in the same key
   // order. P never passes through LDS.
   bf16x8_t pb[KB][2];
+  auto weights = [&](const f32x16 (&s)[KB]) {
+    float rowsum = 0.0f;
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+      for (int j = 0; j < 16; ++j) {
+        const float pv = __builtin_amdgcn_exp2f(fmaf(s[kb][j], scale2, -mref));
+        rowsum += pv;
+        pb[kb][j >> 3][j & 7] = (__bf16)pv;
+      }
+    return rowsum;
+  };
   auto softmax = [&](int k0, f32x16 (&s)[KB]) {
     if (masked(k0)) mask(k0, s);
-    float rowmax = largest(s);
-    rowmax = fmaxf(rowmax, __shfl_xor(rowmax, 32));
-    rowmax = rowmax == -INFINITY ? -INFINITY : rowmax * scale2;  // no 0 * inf
-    // defer-max (guide T13): if this tile's max is within 8 of the running
-    // max, keep the old max (P bounded by e^8, fine in fp32/bf16) and skip
-    // the O-rescale pass entirely when every row defers.
-    const bool defer = (m_run != -INFINITY) && (rowmax - m_run <= 11.5416f);  // 8 nats in log2
-    if (!__all(defer)) {
-      const float m_new = defer ? m_run : fmaxf(m_run, rowmax);
+    float rowsum = weights(s);
+    if (!__all(rowsum <= 4096.0f)) {
+      float rowmax = largest(s);
+      rowmax = fmaxf(rowmax, __shfl_xor(rowmax, 32));
+      rowmax = rowmax == -INFINITY ? -INFINITY : rowmax * scale2;  // no 0 * inf
+      const float m_new = fmaxf(m_run, rowmax);
       const float corr = m_run == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m_run - m_new);  // nothing summed yet: 0
 #pragma unroll
       for (int nb = 0; nb < D / 32; ++nb)
@@ -334,60 +334,74 @@ __global__ __launch_bounds__(NW * 64, 2) void fa_fwd_kernel(
         for (int j = 0; j < 16; ++j) oacc[nb][j] *= corr;
       l_run *= corr;
       m_run = m_new;
+      mref = m_run == -INFINITY ? -3.0e38f : m_run;
+      rowsum = weights(s);
     }
-    const float msafe = (m_run == -INFINITY) ? 0.0f : m_run;
-    float rowsum = 0.0f;
-#pragma unroll
-    for (int kb = 0; kb < KB; ++kb)
-#pragma unroll
-      for (int j = 0; j < 16; ++j) {
-        const float pv = __builtin_amdgcn_exp2f(fmaf(s[kb][j], scale2, -msafe));
-        rowsum += pv;
-        pb[kb][j >> 3][j & 7] = (__bf16)pv;
-      }
     l_run += rowsum;  // this lane's half of the row's keys; the halves meet at the end
   };
-  auto values = [&](const char* Vlds) {
+
+  const RowAt row_at(ln, half);
+  const ColAt col_at(lane);
+  const TileLoad<D, KVB, NW> kload(k_base, kts, SeffK), vload(v_base, kts, SeffK);
+  f32x16 sc[KB];
+  if (kv_tiles > 0) {
+    kload.all(0, Kbuf, w);
+    vload.all(0, Vbuf, w);
+  }
+  loads_done();
+  __syncthreads();
+  // A tile, while the next one arrives in the other buffers (past the last key: zeros, without a read).
+  auto step = [&](int t, const char* __restrict__ K_, const char* __restrict__ V_, char* __restrict__ Kn, char* __restrict__ Vn) __attribute__((always_inline)) {
+    const auto kt = kload.tile((t + 1) * KVB), vt = vload.tile((t + 1) * KVB);
+    constexpr int PER = TileLoad<D, KVB, NW>::PER;
+    // ---- S^T = K · Q^T : KVB/32 32-k blocks. C: col = q (ln), row = k (crow).
 #pragma unroll
     for (int kb = 0; kb < KB; ++kb)
 #pragma unroll
-      for (int s2 = 0; s2 < 2; ++s2)
+      for (int j = 0; j < 16; ++j) sc[kb][j] = 0.0f;
+    __builtin_amdgcn_s_setprio(1);
+    // the key fragments are read AHEAD products ahead of their own
+    constexpr int AHEAD = 6;
+    bf16x8_t kf[DSL * KB];
 #pragma unroll
-        for (int nb = 0; nb < D / 32; ++nb)
-          oacc[nb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-              frag_born<KVB>(Vlds, lane, kb * 32 + s2 * 16, nb * 2), pb[kb][s2], oacc[nb], 0, 0, 0);
+    for (int i = 0; i < AHEAD; ++i) kf[i] = frag_row<KVB>(K_, row_at, i % KB * 32, i / KB);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < DSL * KB; ++i) {
+      if (i + AHEAD < DSL * KB) kf[i + AHEAD] = frag_row<KVB>(K_, row_at, (i + AHEAD) % KB * 32, (i + AHEAD) / KB);
+      sc[i % KB] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[i], qf[i / KB], sc[i % KB], 0, 0, 0);
+      if (i % KB == KB - 1) {
+        const int sl = i / KB;
+#pragma unroll
+        for (int n = sl * PER / DSL; n < (sl + 1) * PER / DSL; ++n) kload.piece(kt, Kn, w, n);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    __builtin_amdgcn_s_setprio(0);
+    softmax(t * KVB, sc);
+    __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+    for (int g = 0; g < KB * 2; ++g) {
+#pragma unroll
+      for (int nb = 0; nb < D / 32; ++nb)
+        oacc[nb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(frag_born<KVB>(V_, col_at, g * 16, nb * 32), pb[g >> 1][g & 1], oacc[nb], 0, 0, 0);
+#pragma unroll
+      for (int i = g * PER / (2 * KB); i < (g + 1) * PER / (2 * KB); ++i) vload.piece(vt, Vn, w, i);
+    }
+    __builtin_amdgcn_s_setprio(0);
   };
-
-  RegStage<D, KVB, NT> kstage, vstage;
-  const unsigned koff = kstage.offset(kts);
-  f32x16 sc[KB];
-  // async-split staging (T14): tile t+1's global loads issue before tile t's compute; their stores
-  // target the OTHER buffer, so that one barrier a tile does
-  // SeffK == 0 blocks skip the tile loop; the clamped loads stay in-bounds
-  kstage.load(k_base, kts, koff, 0, SeffK);
-  vstage.load(v_base, kts, koff, 0, SeffK);
-  kstage.store(Kbuf);
-  vstage.store(Vbuf);
-  __syncthreads();
   for (int t = 0; t < kv_tiles; ++t) {
-    const bool more = t + 1 < kv_tiles;
-    if (more) {
-      kstage.load(k_base, kts, koff, (t + 1) * KVB, SeffK);
-      vstage.load(v_base, kts, koff, (t + 1) * KVB, SeffK);
-    }
+    char* K_ = Kbuf + (t & 1) * KB_BYTES;
+    char* V_ = Vbuf + (t & 1) * KB_BYTES;
+    char* Kn = Kbuf + (~t & 1) * KB_BYTES;
+    char* Vn = Vbuf + (~t & 1) * KB_BYTES;
     if (t < my_tiles) {
-      __builtin_amdgcn_s_setprio(1);
-      scores(Kbuf + (t & 1) * KB_BYTES, sc);
-      __builtin_amdgcn_s_setprio(0);
-      softmax(t * KVB, sc);
-      __builtin_amdgcn_s_setprio(1);
-      values(Vbuf + (t & 1) * KB_BYTES);
-      __builtin_amdgcn_s_setprio(0);
+      step(t, K_, V_, Kn, Vn);
+    } else {
+      kload.all((t + 1) * KVB, Kn, w);
+      vload.all((t + 1) * KVB, Vn, w);
     }
-    if (more) {
-      kstage.store(Kbuf + ((t + 1) & 1) * KB_BYTES);
-      vstage.store(Vbuf + ((t + 1) & 1) * KB_BYTES);
-    }
+    loads_done();
     __syncthreads();
   }
 
@@ -497,7 +511,7 @@ DEV_INLINE void bwd_dkdv(
   float* dta_lds = lse_lds + 2 * QB;                          // [2][32] -delta
 
   const int lane = threadIdx.x & 63;
-  const int w = threadIdx.x >> 6;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);   // the same for a wave: what it decides is a scalar branch
   const int half = lane >> 5;
   const int ln = lane & 31;
 
@@ -540,7 +554,7 @@ DEV_INLINE void bwd_dkdv(
   }
   // ---- V rows of the block (B operand of dP = dO · V^T): they do not fit into registers beside
   // the two accumulators, each wave reads its own 32 rows from LDS
-  stage_direct<D, NWB * QW, NTB>(Vlds, v_base, kts, kv0, SeffK);
+  TileLoad<D, NWB * QW, NWB>(v_base, kts, SeffK).all(kv0, Vlds, w);
 
   f32x16 dk_acc[NB], dv_acc[NB];
 #pragma unroll
@@ -556,91 +570,126 @@ DEV_INLINE void bwd_dkdv(
   const int steps = kv0 < SeffK ? nq * G : 0;
   const float scale2 = scale * 1.44269504f;
 
-  RegStage<D, QB, NTB> qstage, dostage;
-  const unsigned qoff = qstage.offset(qts), dooff = dostage.offset(do_stride);
+  const RowAt row_at(ln, half);
+  const ColAt col_at(lane);
+  typedef TileLoad<D, QB, NWB> Load;
   float lse_r = 0.0f, dta_r = 0.0f;
-  auto fetch = [&](int step) {   // global loads of a step's query tile
-    const int h = hk * group + h_first + step / nq;
-    const int qt0 = (qt_first + step % nq) * QB;
-    const unsigned short* q_base = VARLEN ? Q + seq0 * qts + (long)h * D : Q + (long)b * qbs + (long)h * D;
-    const unsigned short* do_base =
-        VARLEN ? dO + (seq0 * Hq + h) * D : dO + ((long)b * S * Hq + h) * D;  // dO packed
-    qstage.load(q_base, qts, qoff, qt0, Seff);
-    dostage.load(do_base, do_stride, dooff, qt0, Seff);
-    if (threadIdx.x < QB) {
-      const long at = (VARLEN ? (long)h * S + seq0 : ((long)b * Hq + h) * S) + min(qt0 + (int)threadIdx.x, Seff - 1);
-      lse_r = qt0 + (int)threadIdx.x < Seff ? LSE[at] : -INFINITY;
+  int f_head = 0, f_tile = 0;    // head of the block's and tile of the head that the next fetch takes
+  __amdgpu_buffer_rsrc_t q_next, do_next;
+  const Load qload(Q, qts, Seff), doload(dO, do_stride, Seff);
+  auto fetch = [&]() {           // what the loads of a step's query tile need, and its rows' statistics
+    const int h = hk * group + h_first + f_head;
+    const int qt0 = (qt_first + f_tile) * QB;
+    if (++f_tile == nq) {
+      f_tile = 0;
+      ++f_head;
+    }
+    q_next = qload.tile(VARLEN ? Q + seq0 * qts + (long)h * D : Q + (long)b * qbs + (long)h * D, qt0);
+    do_next = doload.tile(VARLEN ? dO + (seq0 * Hq + h) * D : dO + ((long)b * S * Hq + h) * D, qt0);  // dO packed
+    if (w == 0) {
+      const int row = qt0 + ln;
+      const long at = (VARLEN ? (long)h * S + seq0 : ((long)b * Hq + h) * S) + min(row, Seff - 1);
+      lse_r = row < Seff ? LSE[at] : -INFINITY;
       dta_r = DELTA[at];
     }
   };
   auto stash = [&](int buf) {
-    qstage.store(Qbuf + buf * TB);
-    dostage.store(dObuf + buf * TB);
-    if (threadIdx.x < QB) {
-      lse_lds[buf * QB + threadIdx.x] = lse_r == -INFINITY ? -INFINITY : -lse_r * 1.44269504f;
-      dta_lds[buf * QB + threadIdx.x] = -dta_r;
+    if (w == 0 && half == 0) {
+      lse_lds[buf * QB + ln] = lse_r == -INFINITY ? -INFINITY : -lse_r * 1.44269504f;
+      dta_lds[buf * QB + ln] = -dta_r;
     }
   };
   if (steps > 0) {
-    fetch(0);
+    fetch();
+#pragma unroll
+    for (int i = 0; i < Load::PER; ++i) {
+      qload.piece(q_next, Qbuf, w, i);
+      doload.piece(do_next, dObuf, w, i);
+    }
     stash(0);
   }
+  loads_done();
   __syncthreads();
 
-  for (int step = 0; step < steps; ++step) {
-    const int buf = step & 1;
-    const int qt0 = (qt_first + step % nq) * QB;
-    const bool more = step + 1 < steps;
-    if (more) fetch(step + 1);
-    const char* Qlds = Qbuf + buf * TB;
-    const char* dOlds = dObuf + buf * TB;
-    if (!(causal && qt0 + QB - 1 < kvw) && kvw < SeffK) {
-      // ---- S[q][kv] = Q · K^T and dP[q][kv] - delta[q] = dO · V^T - delta: column = kv (ln), row = q
-      f32x16 s, dp;
-      float addend[16];
+  // A query tile, while the next one arrives in the other buffers.
+  auto step = [&](int qt0, int buf, const char* __restrict__ Qlds, const char* __restrict__ dOlds, char* __restrict__ Qn,
+                  char* __restrict__ dOn) __attribute__((always_inline)) {
+    // ---- S[q][kv] = Q · K^T and dP[q][kv] - delta[q] = dO · V^T - delta: column = kv (ln), row = q
+    f32x16 s, dp;
+    float addend[16];
 #pragma unroll
-      for (int a = 0; a < 4; ++a) {
-        const float4v l4 = *reinterpret_cast<const float4v*>(lse_lds + buf * QB + 8 * a + 4 * half);
-        const float4v d4 = *reinterpret_cast<const float4v*>(dta_lds + buf * QB + 8 * a + 4 * half);
+    for (int a = 0; a < 4; ++a) {
+      const float4v l4 = *reinterpret_cast<const float4v*>(lse_lds + buf * QB + 8 * a + 4 * half);
+      const float4v d4 = *reinterpret_cast<const float4v*>(dta_lds + buf * QB + 8 * a + 4 * half);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          addend[4 * a + e] = l4[e];
-          dp[4 * a + e] = d4[e];
-          s[4 * a + e] = 0.0f;
-        }
+      for (int e = 0; e < 4; ++e) {
+        addend[4 * a + e] = l4[e];
+        dp[4 * a + e] = d4[e];
+        s[4 * a + e] = 0.0f;
       }
-      __builtin_amdgcn_s_setprio(1);
+    }
+    __builtin_amdgcn_s_setprio(1);
 #pragma unroll
-      for (int sl = 0; sl < DSL; ++sl) {
-        s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ld_lds16(Qlds, tile_off<QB>(ln, sl * 16 + half * 8)), kf[sl], s, 0, 0, 0);
-        dp = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ld_lds16(dOlds, tile_off<QB>(ln, sl * 16 + half * 8)),
-                                                     ld_lds16(Vlds, tile_off<NWB * QW>(w * QW + ln, sl * 16 + half * 8)),
-                                                     dp, 0, 0, 0);
-      }
-      __builtin_amdgcn_s_setprio(0);
-      // ---- P = exp(scale s - lse); dS = P (dP - delta), its scale waits for the epilogue
-      bf16x8_t pa[2], dsa[2];
-      const bool diagonal = causal && kvw + QW - 1 > qt0;
+    for (int sl = 0; sl < DSL; ++sl) {
+      s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(frag_row<QB>(Qlds, row_at, 0, sl), kf[sl], s, 0, 0, 0);
+      dp = __builtin_amdgcn_mfma_f32_32x32x16_bf16(frag_row<QB>(dOlds, row_at, 0, sl),
+                                                   frag_row<NWB * QW>(Vlds + w * 2048, row_at, 0, sl), dp, 0, 0, 0);
+#pragma unroll
+      for (int i = sl * Load::PER / DSL; i < (sl + 1) * Load::PER / DSL; ++i) qload.piece(q_next, Qn, w, i);
+    }
+    __builtin_amdgcn_s_setprio(0);
+    // ---- P = exp(scale s - lse); dS = P (dP - delta), its scale waits for the epilogue
+    bf16x8_t pa[2], dsa[2];
+    const int before = kvw + ln - qt0 - 4 * half;   // rows of the tile ahead of this key
+    auto grads = [&](auto diagonal) __attribute__((always_inline)) {
 #pragma unroll
       for (int j = 0; j < 16; ++j) {
         float pv = __builtin_amdgcn_exp2f(fmaf(s[j], scale2, addend[j]));
-        if (diagonal && kvw + ln > qt0 + crow(j, half)) pv = 0.0f;
+        if (diagonal) pv = before > crow(j, 0) ? 0.0f : pv;
         pa[j >> 3][j & 7] = (__bf16)pv;
         dsa[j >> 3][j & 7] = (__bf16)(pv * dp[j]);
       }
-      // ---- dV += P^T · dO, dK += dS^T · Q (A: lane row = kv; B: columns of the tiles)
-      __builtin_amdgcn_s_setprio(1);
-#pragma unroll
-      for (int s2 = 0; s2 < 2; ++s2)
-#pragma unroll
-        for (int nb = 0; nb < NB; ++nb) {
-          dv_acc[nb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(pa[s2], frag_born<QB>(dOlds, lane, s2 * 16, nb * 2), dv_acc[nb], 0, 0, 0);
-          dk_acc[nb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(dsa[s2], frag_born<QB>(Qlds, lane, s2 * 16, nb * 2), dk_acc[nb], 0, 0, 0);
-        }
-      __builtin_amdgcn_s_setprio(0);
+    };
+    // two bodies: merged into one, every tile would pay for the mask of the few on the diagonal
+    if (causal && kvw + QW - 1 > qt0) {
+      grads(std::true_type());
+      asm volatile("" ::: "memory");
+    } else {
+      grads(std::false_type());
     }
-    // the stores target the other buffer: one barrier a step
+    // ---- dV += P^T · dO, dK += dS^T · Q (A: lane row = kv; B: columns of the tiles)
+    __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+    for (int s2 = 0; s2 < 2; ++s2)
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb) {
+        dv_acc[nb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(pa[s2], frag_born<QB>(dOlds, col_at, s2 * 16, nb * 32), dv_acc[nb], 0, 0, 0);
+        dk_acc[nb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(dsa[s2], frag_born<QB>(Qlds, col_at, s2 * 16, nb * 32), dk_acc[nb], 0, 0, 0);
+        const int at = s2 * NB + nb;
+#pragma unroll
+        for (int i = at * Load::PER / (2 * NB); i < (at + 1) * Load::PER / (2 * NB); ++i) doload.piece(do_next, dOn, w, i);
+      }
+    __builtin_amdgcn_s_setprio(0);
+  };
+  for (int n = 0, c_tile = 0; n < steps; ++n) {
+    const int buf = n & 1;
+    const int qt0 = (qt_first + c_tile) * QB;
+    if (++c_tile == nq) c_tile = 0;
+    const bool more = n + 1 < steps;
+    if (more) fetch();
+    char* Qn = Qbuf + (buf ^ 1) * TB;
+    char* dOn = dObuf + (buf ^ 1) * TB;
+    if (!(causal && qt0 + QB - 1 < kvw) && kvw < SeffK) {
+      step(qt0, buf, Qbuf + buf * TB, dObuf + buf * TB, Qn, dOn);   // after the last step the loads repeat its tile
+    } else {
+#pragma unroll
+      for (int i = 0; i < Load::PER; ++i) {
+        qload.piece(q_next, Qn, w, i);
+        doload.piece(do_next, dOn, w, i);
+      }
+    }
     if (more) stash(buf ^ 1);
+    loads_done();
     __syncthreads();
   }
 
@@ -689,7 +738,7 @@ DEV_INLINE void bwd_dq(
   char* Vbuf = smem + 2 * TB;
 
   const int lane = threadIdx.x & 63;
-  const int w = threadIdx.x >> 6;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);   // the same for a wave: what it decides is a scalar branch
   const int half = lane >> 5;
   const int ln = lane & 31;
 
@@ -749,66 +798,79 @@ DEV_INLINE void bwd_dq(
   const int kv_tiles_all = (SeffK + KVB - 1) / KVB;
   const int kv_tiles = q0 >= Seff ? 0 : (causal ? min(kv_tiles_all, (min(q0 + NWB * QW, Seff) + KVB - 1) / KVB) : kv_tiles_all);
 
-  RegStage<D, KVB, NTB> kstage, vstage;
-  const unsigned koff = kstage.offset(kts);
+  const int last_key = causal ? min(qw + ln, SeffK - 1) : SeffK - 1;   // the last key this row sees
+  const RowAt row_at(ln, half);
+  const ColAt col_at(lane);
+  typedef TileLoad<D, KVB, NWB> Load;
+  const Load kload(k_base, kts, SeffK), vload(v_base, kts, SeffK);
   if (kv_tiles > 0) {
-    kstage.load(k_base, kts, koff, 0, SeffK);
-    vstage.load(v_base, kts, koff, 0, SeffK);
-    kstage.store(Kbuf);
-    vstage.store(Vbuf);
+    kload.all(0, Kbuf, w);
+    vload.all(0, Vbuf, w);
   }
+  loads_done();
   __syncthreads();
 
-  for (int t = 0; t < kv_tiles; ++t) {
-    const int k0 = t * KVB, buf = t & 1;
-    const bool more = t + 1 < kv_tiles;
-    if (more) {
-      kstage.load(k_base, kts, koff, k0 + KVB, SeffK);
-      vstage.load(v_base, kts, koff, k0 + KVB, SeffK);
-    }
-    const char* Klds = Kbuf + buf * TB;
-    const char* Vlds = Vbuf + buf * TB;
-    if (!(causal && k0 > qw + QW - 1) && qw < Seff) {
+  // A key/value tile, while the next one arrives in the other buffers (past the last key: zeros, without a read).
+  auto step = [&](int k0, const char* __restrict__ Klds, const char* __restrict__ Vlds, char* __restrict__ Kn,
+                  char* __restrict__ Vn) __attribute__((always_inline)) {
+    const auto kt = kload.tile(k0 + KVB), vt = vload.tile(k0 + KVB);
 #pragma unroll
-      for (int kb = 0; kb < KVB / 32; ++kb) {
-        // ---- S^T[kv][q] = K · Q^T and dP^T - delta = V · dO^T - delta: column = q (ln), row = kv
-        f32x16 s, dp;
+    for (int kb = 0; kb < KVB / 32; ++kb) {
+      // ---- S^T[kv][q] = K · Q^T and dP^T - delta = V · dO^T - delta: column = q (ln), row = kv
+      f32x16 s, dp;
 #pragma unroll
-        for (int j = 0; j < 16; ++j) { s[j] = 0.0f; dp[j] = ndelta; }
-        __builtin_amdgcn_s_setprio(1);
+      for (int j = 0; j < 16; ++j) { s[j] = 0.0f; dp[j] = ndelta; }
+      __builtin_amdgcn_s_setprio(1);
 #pragma unroll
-        for (int sl = 0; sl < DSL; ++sl) {
-          s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ld_lds16(Klds, tile_off<KVB>(kb * 32 + ln, sl * 16 + half * 8)), qf[sl], s, 0, 0, 0);
-          dp = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ld_lds16(Vlds, tile_off<KVB>(kb * 32 + ln, sl * 16 + half * 8)), dof[sl], dp, 0, 0, 0);
+      for (int sl = 0; sl < DSL; ++sl) {
+        s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(frag_row<KVB>(Klds, row_at, kb * 32, sl), qf[sl], s, 0, 0, 0);
+        dp = __builtin_amdgcn_mfma_f32_32x32x16_bf16(frag_row<KVB>(Vlds, row_at, kb * 32, sl), dof[sl], dp, 0, 0, 0);
+        const int at = kb * DSL + sl;
+#pragma unroll
+        for (int i = at * Load::PER / (2 * DSL); i < (at + 1) * Load::PER / (2 * DSL); ++i) {
+          kload.piece(kt, Kn, w, i);
+          vload.piece(vt, Vn, w, i);
         }
-        __builtin_amdgcn_s_setprio(0);
-        // ---- dS = exp(scale s - lse) (dP - delta), its scale waits for the epilogue
-        bf16x8_t dsa[2];
-        const int kb0 = k0 + kb * 32;
-        const bool edge = kb0 + 32 > SeffK || (causal && kb0 + 31 > qw);
+      }
+      __builtin_amdgcn_s_setprio(0);
+      // ---- dS = exp(scale s - lse) (dP - delta), its scale waits for the epilogue
+      bf16x8_t dsa[2];
+      const int kb0 = k0 + kb * 32, upto = last_key - kb0 - 4 * half;
+      auto grads = [&](auto edge) __attribute__((always_inline)) {
 #pragma unroll
         for (int j = 0; j < 16; ++j) {
           float pv = __builtin_amdgcn_exp2f(fmaf(s[j], scale2, addend));
-          if (edge) {
-            const int k_abs = kb0 + crow(j, half);
-            if (k_abs >= SeffK || (causal && k_abs > qw + ln)) pv = 0.0f;
-          }
+          if (edge) pv = crow(j, 0) > upto ? 0.0f : pv;
           dsa[j >> 3][j & 7] = (__bf16)(pv * dp[j]);
         }
-        // ---- dQ += dS · K (A: lane row = q; B: columns of K)
-        __builtin_amdgcn_s_setprio(1);
-#pragma unroll
-        for (int s2 = 0; s2 < 2; ++s2)
-#pragma unroll
-          for (int nb = 0; nb < NB; ++nb)
-            dq_acc[nb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(dsa[s2], frag_born<KVB>(Klds, lane, kb * 32 + s2 * 16, nb * 2), dq_acc[nb], 0, 0, 0);
-        __builtin_amdgcn_s_setprio(0);
+      };
+      if (kb0 + 32 > SeffK || (causal && kb0 + 31 > qw)) {
+        grads(std::true_type());
+        asm volatile("" ::: "memory");
+      } else {
+        grads(std::false_type());
       }
+      // ---- dQ += dS · K (A: lane row = q; B: columns of K)
+      __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+      for (int s2 = 0; s2 < 2; ++s2)
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb)
+          dq_acc[nb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(dsa[s2], frag_born<KVB>(Klds, col_at, kb * 32 + s2 * 16, nb * 32), dq_acc[nb], 0, 0, 0);
+      __builtin_amdgcn_s_setprio(0);
     }
-    if (more) {
-      kstage.store(Kbuf + (buf ^ 1) * TB);
-      vstage.store(Vbuf + (buf ^ 1) * TB);
+  };
+  for (int t = 0; t < kv_tiles; ++t) {
+    const int k0 = t * KVB, buf = t & 1;
+    char* Kn = Kbuf + (buf ^ 1) * TB;
+    char* Vn = Vbuf + (buf ^ 1) * TB;
+    if (!(causal && k0 > qw + QW - 1) && qw < Seff) {
+      step(k0, Kbuf + buf * TB, Vbuf + buf * TB, Kn, Vn);
+    } else {
+      kload.all(k0 + KVB, Kn, w);
+      vload.all(k0 + KVB, Vn, w);
     }
+    loads_done();
     __syncthreads();
   }
 
@@ -875,6 +937,23 @@ __global__ __launch_bounds__(256) void fa_bwd_sum_kernel(unsigned short* __restr
 
 namespace {
 
+// A tile's loads take 16 bytes at addresses of that alignment, with offsets of 32 bits inside the tile. Rows that lie
+// otherwise, or 2^23 elements apart and more, are copied together first; k and v together, which share their strides.
+bool loadable(const at::Tensor& t) {
+  const int rows = (int)t.dim() - 3;
+  return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0 &&
+         (t.size(rows) <= 1 || (t.stride(rows) % 8 == 0 && t.stride(rows) < (1L << 23))) &&
+         (rows == 0 || t.size(0) <= 1 || t.stride(0) % 8 == 0);
+}
+void make_loadable(at::Tensor& t) {
+  if (!loadable(t)) t = t.clone(at::MemoryFormat::Contiguous);
+}
+void make_loadable(at::Tensor& k, at::Tensor& v) {
+  if (loadable(k) && loadable(v)) return;
+  k = k.clone(at::MemoryFormat::Contiguous);
+  v = v.clone(at::MemoryFormat::Contiguous);
+}
+
 void set_lds_limit(const void* kernel, size_t bytes) {
   if (bytes > 65536) {
     (void)hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
@@ -916,6 +995,8 @@ std::vector<at::Tensor> flash_attn_fwd(at::Tensor q, at::Tensor k, at::Tensor v,
   at::Tensor seqlens_k = seqlens_k_opt.has_value() ? *seqlens_k_opt : at::Tensor();
   using namespace fa;
   check_fa_inputs(q, k, v);
+  make_loadable(q);
+  make_loadable(k, v);
   const int B = (int)q.size(0), S = (int)q.size(1), Hq = (int)q.size(2), D = (int)q.size(3);
   const int Hkv = (int)k.size(2);
   const int Sk = (int)k.size(1);  // kv may be a shorter ring piece
@@ -971,6 +1052,8 @@ std::vector<at::Tensor> flash_attn_varlen_fwd(at::Tensor q, at::Tensor k, at::Te
   TORCH_CHECK(D == 64 || D == 128, "flash_attn: head dim must be 64 or 128");
   TORCH_CHECK(q.stride(2) == 1 && q.stride(1) == D, "varlen: q must be dense in [H,D]");
   TORCH_CHECK(k.strides() == v.strides() && k.sizes() == v.sizes());
+  make_loadable(q);
+  make_loadable(k, v);
   auto o = at::empty({T, Hq, D}, q.options());
   auto lse = at::empty({Hq, T}, q.options().dtype(at::kFloat));
   auto stream = at::hip::getCurrentHIPStream();
@@ -1068,6 +1151,9 @@ std::vector<at::Tensor> flash_attn_bwd(at::Tensor dout, at::Tensor q, at::Tensor
   check_fa_inputs(q, k, v);
   TORCH_CHECK(dout.is_contiguous() && out.is_contiguous() && lse.is_contiguous(),
               "flash_attn_bwd: dout/out/lse must be contiguous");
+  make_loadable(q);
+  make_loadable(k, v);
+  make_loadable(dout);
   const int B = (int)q.size(0), S = (int)q.size(1), Hq = (int)q.size(2), D = (int)q.size(3);
   const int Hkv = (int)k.size(2);
   const int* cu = nullptr;
@@ -1117,6 +1203,9 @@ std::vector<at::Tensor> flash_attn_varlen_bwd(at::Tensor dout, at::Tensor q, at:
   using namespace fa;
   TORCH_CHECK(q.dim() == 3 && k.dim() == 3 && v.dim() == 3, "varlen: q/k/v must be [total,H,D]");
   TORCH_CHECK(dout.is_contiguous() && out.is_contiguous() && lse.is_contiguous());
+  make_loadable(q);
+  make_loadable(k, v);
+  make_loadable(dout);
   const int T = (int)q.size(0), Hq = (int)q.size(1), D = (int)q.size(2);
   const int Hkv = (int)k.size(1);
   const int n_seq = (int)cu_seqlens.numel() - 1;

@@ -196,3 +196,70 @@ def test_strided_gradients_with_shared_heads():
     kernels().flash_attn_bwd(dout, q, k, v, out, lse, True, D ** -0.5, dq, dk, dv)
     for name, a, b in zip(("out", "dq", "dk", "dv"), (out, dq, dk, dv), want):
         _near(a, b, name)
+
+
+@pytest.mark.parametrize("levels", [
+    (0, 9, 18, 27, 36, 45),          # every tile's weights pass the reference of the one before
+    (0, 5, 10, 15, 20, 25),          # every second one's do
+    (60, 40, 20, 0, -20, -40),       # the first tile has the largest scores
+    (-3000, 0, -3000, 4, 8, 1000),   # far below, far above
+])
+@pytest.mark.parametrize("D,causal", [(128, False), (64, False), (128, True)])
+def test_scores_that_rise_and_fall(levels, D, causal):
+    """Scores of a level of their own (in nats) in each key tile of 64: the reference that the forward takes a row's weights
+    against is left behind, raised, or stays."""
+    from colossalai_amd.ops import flash_attention
+
+    S = 64 * len(levels)
+    q, k, v, dout = _inputs(1, S, 4, 2, D)
+    scale = D ** -0.5
+    q[..., 0] = 8.0
+    k[..., 0] = torch.tensor(levels, device="cuda").repeat_interleave(64)[None, :, None] / (8.0 * scale)
+    want = _reference(q, k, v, dout, causal, scale)
+    for t in (q, k, v):
+        t.requires_grad_()
+    out = flash_attention(q, k, v, causal=causal)
+    got = (out, *torch.autograd.grad(out, (q, k, v), dout))
+    for name, a, b in zip(("out", "dq", "dk", "dv"), got, want):
+        # dq and dk: not channel 0, whose partner is as large as a level, nor rows of a single key under a mask
+        if name in ("dq", "dk"):
+            if causal:
+                continue
+            a, b = a[..., 1:], b[..., 1:]
+        _near(a, b, name)
+
+
+@pytest.mark.parametrize("place", ["odd address", "odd rows", "far rows", "one row for all"])
+@pytest.mark.parametrize("packed", [False, True])
+def test_inputs_that_tiles_cannot_be_loaded_from_as_they_lie(place, packed):
+    from colossalai_amd.ops import flash_attention, flash_attention_varlen
+
+    S, D = 150, 64
+    q, k, v, dout = _inputs(1, S, 4, 2, D, seed=3)
+
+    def lay(t):
+        n = t.shape[2] * D
+        if place == "odd address":
+            return torch.empty(S * n + 1, device="cuda", dtype=t.dtype)[1:].view(t.shape).copy_(t)
+        if place == "one row for all":
+            return t[:, :1].expand(t.shape)
+        step = n + 1 if place == "odd rows" else 1 << 23
+        room = torch.empty((S - 1) * step + n, device="cuda", dtype=t.dtype)
+        return room.as_strided(t.shape, (0, step, D, 1)).copy_(t)
+
+    laid = [lay(t).detach().requires_grad_() for t in (q, k, v)]
+    d = lay(dout) if place == "odd address" else dout
+    want = _reference(*[t.detach() for t in laid], d, True, D ** -0.5)
+    if packed:
+        cu = torch.tensor([0, S], dtype=torch.int32, device="cuda")
+        out = flash_attention_varlen(*[t[0] for t in laid], cu, S, causal=True)[None]
+    else:
+        out = flash_attention(*laid, causal=True)
+    got = (out, *torch.autograd.grad(out, laid, d))
+    for name, a, b in zip(("out", "dq", "dk", "dv"), got, want):
+        if place == "one row for all" and name in ("dq", "dk"):
+            # equal keys and values: dP - delta vanishes but for the output's rounding, 2^-9 of dout · v (4 sqrt(D) at most here),
+            # times the scale, a key or query channel (4 at most), and for dk the sum of a key's weights (ln S + 1 at most)
+            assert a.float().abs().max() < 2.0 ** -9 * 4 * 4 * (6 if name == "dk" else 1)
+        else:
+            _near(a, b, name)
