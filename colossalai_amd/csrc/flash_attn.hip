@@ -45,11 +45,11 @@
 #include <algorithm>
 #include <type_traits>
 
-#include "common.h"
+#include "lds_tiles.h"
 
 namespace cai {
 
-typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
+typedef bf16x8_v bf16x8_t;
 
 namespace fa {
 
@@ -64,51 +64,6 @@ DEV_INLINE bf16x8_t ld_g16(const unsigned short* p) {
 
 // C-layout row for mfma_f32_32x32x16 register j (guide §3, HW-verified).
 DEV_INLINE constexpr int crow(int j, int half) { return (j & 3) + 8 * (j >> 2) + 4 * half; }
-
-// An operand tile in LDS: pieces of 16 rows of 32 channels, 1024 bytes each, all row groups of a channel group one after the
-// other. In a piece the four 16-byte units of a row lie together, unit u at place u ^ (row / 4 % 4). A piece is what
-// one load instruction of a wave brings straight into LDS (16 bytes a lane in lane order, a quad of lanes 64 neighbouring bytes of a
-// row), and every access spreads over the 64 banks: a row fragment (ds_read_b128) takes one unit of 16 consecutive
-// rows, which lie in 16 different places of 16 bytes; a transposing read takes rows 0-7 or 8-15 of a piece as a whole.
-template <int ROWS>
-__host__ __device__ constexpr int piece_at(int row, int col) { return ((col >> 5) * (ROWS / 16) + (row >> 4)) * 1024; }
-
-template <int ROWS, int COLS>
-__host__ __device__ constexpr int tile_bytes() { return ROWS * COLS * 2; }
-
-// Where a lane's 8 channels 16 * sl + 8 * half of row `ln` (and every 32nd row from it) lie: `even` for even sl, `odd` for
-// odd ones, beyond which a fragment's piece is a constant.
-struct RowAt {
-  int even, odd;
-  DEV_INLINE RowAt(int ln, int half) {
-    const int place = half ^ (ln >> 2 & 3), at = (ln >> 4) * 1024 + (ln & 15) * 64;
-    even = at + place * 16;
-    odd = at + (place ^ 2) * 16;
-  }
-};
-template <int ROWS>
-DEV_INLINE bf16x8_t frag_row(const char* tile, const RowAt& at, int row0, int sl) {
-  return *reinterpret_cast<const bf16x8_t*>(tile + (sl & 1 ? at.odd : at.even) + piece_at<ROWS>(row0, sl * 16));
-}
-
-// Column fragment by transposing reads, in the order in which the C layout hands out its rows: lane l
-// receives tile[k_base + 8*(e>>2) + 4*(l>>5) + (e&3)][col + (l&31)], e = 0..7, so
-// that a packed run of eight C registers is the matching other operand.
-struct ColAt {
-  int lo, hi;
-  DEV_INLINE explicit ColAt(int lane) {
-    const int m = lane & 15, half = lane >> 5;
-    const int unit = (lane >> 4 & 1) * 2 + (m >> 1 & 1), row = half * 4 + (m >> 2);
-    lo = row * 64 + (unit ^ half) * 16 + (m & 1) * 8;
-    hi = (row + 8) * 64 + (unit ^ half ^ 2) * 16 + (m & 1) * 8;
-  }
-};
-template <int ROWS>
-DEV_INLINE bf16x8_t frag_born(const char* tile, const ColAt& at, int k_base, int col) {
-  const bf16x4_v lo = ld_tr16(tile, at.lo + piece_at<ROWS>(k_base, col));
-  const bf16x4_v hi = ld_tr16(tile, at.hi + piece_at<ROWS>(k_base, col));
-  return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
-}
 
 // Which (q tile, sequence, head) a block of the forward works on. Blocks of one (sequence, head) share an
 // XCD's L2. Packed batches run head by head, each head over all sequences: the other way round
@@ -137,8 +92,6 @@ DEV_INLINE int xcd_chunk(int f, int nblocks) {
 // work, and its LDS stores, which met in the banks, for another 638: B1 S8192 H32/8 D128 causal.)
 // Rows past the matrix' end come as zeros: the buffer descriptor of a tile ends with its last row, and is made
 // anew for each tile, so that a matrix may be of any size; rows less than 2^23 elements apart (offsets stay under 2^31).
-typedef __attribute__((address_space(3))) void* lds_ptr;
-
 template <int D, int ROWS, int WAVES>
 struct TileLoad {
   static constexpr int RG = ROWS / 16, PIECES = RG * (D / 32), PER = PIECES / WAVES;
@@ -170,9 +123,6 @@ struct TileLoad {
     for (int i = 0; i < PER; ++i) piece(t, lds, w, i);
   }
 };
-
-// every load of this wave has arrived (in LDS); a barrier behind it makes that true for the block
-DEV_INLINE void loads_done() { __builtin_amdgcn_s_waitcnt(0x0f70); }   // vmcnt(0)
 
 }  // namespace fa
 

@@ -21,6 +21,9 @@
 // of the keys), so that a position's results agree to rounding and not bit for bit.
 // Calls without a distance table, block summaries or cross values run the form in row_attention.hip
 // where the row sizes fit it; bfloat16 prompt portions run the matrix-core kernel.
+#include <type_traits>
+
+#include "../lds_tiles.h"
 #include "paged_attention.h"
 
 namespace cai {
@@ -304,21 +307,23 @@ __global__ __launch_bounds__(64 * ATT_WAVES) void paged_attention_kernel(
 // The tiles are DS * 16 key channels by VT * 32 value channels; a head whose sizes Dr / Dvr are
 // smaller (multiples of 8) is padded with zeros on its way into registers and LDS, and only its
 // own channels are stored.
-// What bounds it: the waits of a step. Of a wave's time 38 % are waits (LDS operands, the barrier of a step, page
-// lookups), the matrix units are busy a fifth and the vector units a quarter; registers (253 of 256 at 128 channels)
-// allow two blocks a CU and no deeper pipeline. One 4096-token prompt, 16 heads on 4 of 128, page 64:
-// 594 us with rows swizzled and a lookup for each 16 bytes, 275 with two tiles a softmax, 204 with the planes, two
-// lookups a lane and tile, and the grid by XCD (64 channels, 16 heads on 8: 654, 342, 177; a cap and a sink: 605, 302,
-// 238; 16 heads of one key head each: 631, 277, 204).
-// Reading operands six ahead of the products changed nothing (203 us), lookups through scalar loads cost (416 us: their
-// counter is the LDS reads' own).
-template <int DS, int VT, int NG>
+// What bounds it: a step of 64 keys took each of a SIMD's two waves 9200 cycles (16 heads on 4 of 128, a cap and a sink), of which
+// 1600 went into issuing the step's loads together, 590 into storing them, 2500 (3850 with a cap) into the softmax. With loads that
+// go straight into LDS between the products, scalar branches for what a wave has in common and no maximum it is 5250 (6640):
+// 3140 of them are products. 243 of 256 registers at 128 channels.
+// One 4096-token prompt, 16 heads on 4 of 128, page 64: 196 us before, 138 with this, 115 with two groups of waves a block; a cap and a
+// sink 228, 167, 133; 16 heads of one key head each 201, 140, 120; 16 x 1024 after 100, 16 heads on 8: 287 -> 168, and with two token tiles a
+// block; 14 decode tokens beside portions of 1000 and 963, window 1024: 141 -> 76; 2 x 256: 22.7 -> 15.1.
+// Value fragments read ahead changed nothing (138 to 140), no wave priorities cost 2 %.
+__device__ __align__(16) const bf16s zero_channels[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+
+template <int DS, int VT, int NG, bool MORE>
 __global__ __launch_bounds__(256 * NG, 2) void paged_attention_mfma_kernel(
     bf16s* __restrict__ out, const bf16s* __restrict__ q, long q_stride, const bf16s* __restrict__ kpool,
     const bf16s* __restrict__ vpool, const int* __restrict__ block_tables, int bt_stride, const int* __restrict__ cu,
     const int* __restrict__ start, const float* __restrict__ slopes, const bf16s* __restrict__ gate, long gate_stride,
     int H, int G, int Dr, int Dvr, int page_shift, float scale, int window, int keep_first, float softcap, int sink,
-    int qsplit, const float* __restrict__ sink2, const float* __restrict__ dist2, int dist_rows,
+    int tile_waves, const float* __restrict__ sink2, const float* __restrict__ dist2, int dist_rows,
     const bf16s* __restrict__ ksum, const bf16s* __restrict__ vsum, int sum_shift, int sum_block,
     float* __restrict__ cross_out, int chunk, const float* __restrict__ key_fac, int vrep, float* __restrict__ out32,
     int num_tiles) {
@@ -328,37 +333,37 @@ __global__ __launch_bounds__(256 * NG, 2) void paged_attention_mfma_kernel(
   // sum_block); cross_out [N, H, G, Dv] float32: a row is then also the kv head whose values a block
   // multiplies the weights with; chunk, key_fac [pool rows, G], vrep and out32 as in the split-key kernel (the factors of
   // a key tile are staged with it).
-  // qsplit (kv heads with a single query head each): the four waves of a block are four consecutive 32-token tiles
-  // of that head instead of four heads, so a block covers 128 tokens, a tile is 128 tokens, and
-  // the staged key/value tiles are still shared by all computing waves. The block stages the key range of all its
-  // tokens; a wave skips the tiles that lie wholly after its own tokens.
+  // tile_waves (log2; kv heads with one or two query heads): the four waves of a block are four consecutive 32-token tiles of
+  // the one head, or two tiles of the two heads, instead of four heads; a block covers 128 or 64 tokens then, which is what `num_tiles`
+  // counts, and the staged key/value tiles are still shared by all computing waves. The block stages the key range of all
+  // its tokens; a wave skips the tiles that lie wholly after its own tokens.
+  // MORE = false: no block summaries, no distance table; with their branches in it the common form has no registers left
+  if constexpr (!MORE) ksum = vsum = nullptr, dist2 = nullptr;
   constexpr int D = DS * 16, Dv = VT * 32;
   bf16x8_v zero8;
 #pragma unroll
   for (int e = 0; e < 8; ++e) zero8[e] = (__bf16)0.0f;
-  // A staged tile: planes of 8 channels, [D / 8][32 keys][8], 16 bytes a key, 64 bytes between the planes, keys and
-  // values alike. Row reads take 512 contiguous bytes per half-wave, the transposing reads of the values 64 bytes
-  // from each of four planes at a time, staging stores 16 keys of four planes: none of them meets in a bank.
-  constexpr int PL = 32 * 8 + 32;              // elements of a plane
-  constexpr int KT = D / 8 * PL, VTT = Dv / 8 * PL;   // elements of one staged tile
+  // A staged tile: 32 keys, pieces of 16 keys of 32 channels (lds_tiles.h), keys and values alike. 48 channels end in half a piece.
+  constexpr int KQ = (D + 31) / 32, VQ = VT;            // pieces side by side
+  constexpr int KT = KQ * 2048, VTT = VQ * 2048;        // bytes of one staged tile
   constexpr int TP = MFMA_TILES_PER_STEP, TS = NG * TP;   // tiles of a step: a group's, the block's
-  extern __shared__ __align__(16) bf16s tiles[];  // [2][TS][KT + VTT], then [2][TS][32] key factors (float)
+  extern __shared__ __align__(16) char tiles[];  // [2][TS][KT + VTT], then [2][TS][32] key factors (float)
   float* facs = reinterpret_cast<float*>(tiles + 2 * TS * (KT + VTT));
   constexpr int nthreads = 256;  // of a group, always four waves: those beyond the kv head's group of heads only help staging
   const int tid = threadIdx.x & 255, grp = NG > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 8) : 0;
-  const int wid = tid >> 6, lane = tid & 63;
-  const int rep = H / G;
+  const int wid = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const int rep = H / G, heads = 4 >> tile_waves;   // heads of a block
   const int VC = cross_out != nullptr ? G : 1;
   // Which (tile, row of kv head x pass) this block is. Block f runs on XCD f % 8: with rows that divide 8 or are a
   // multiple of it a row's keys and values stay in as few L2s as possible (4 kv heads: two XCDs a head, every second
   // tile each). Under a causal mask a late tile of a long prompt has many more key tiles than an early one: late ones
   // start first, and where all blocks of an XCD (32 CUs, two blocks each) run at once, the second 32 go the other way, so
   // that a CU's two blocks are a long and a short one.
-  const int f = blockIdx.x, rows = G * ((rep + 3) / 4) * VC;
+  const int f = blockIdx.x, rows = G * ((rep + heads - 1) / heads) * VC;
   int row, tile, b = 0;
   if (rows <= 8 && 8 % rows == 0) {
     const int sub = 8 / rows, xcd = f & 7, i = f >> 3, per = (num_tiles + sub - 1) / sub;   // tiles of a row on this XCD
-    const int k = per <= 64 && i >= 32 ? i - 32 : per - 1 - i;
+    const int k = NG == 1 && per <= 64 && i >= 32 ? i - 32 : per - 1 - i;
     row = xcd % rows;
     tile = k * sub + xcd / rows;
     if (tile >= num_tiles) return;
@@ -366,14 +371,14 @@ __global__ __launch_bounds__(256 * NG, 2) void paged_attention_mfma_kernel(
     const bool by8 = rows % 8 == 0;
     const int at = by8 ? f >> 3 : f, turn = at / num_tiles, i = at - turn * num_tiles;
     row = by8 ? (f & 7) + 8 * turn : turn;
-    tile = num_tiles * rows <= 512 && (turn & 1) ? i : num_tiles - 1 - i;
+    tile = NG == 1 && num_tiles * rows <= 512 && (turn & 1) ? i : num_tiles - 1 - i;
   }
   const int g = row % G, zrow = row / G;
   const int vg = cross_out != nullptr ? zrow % VC : g / vrep;   // kv head of the values
   const int Gv = G / vrep;
-  const int hl = qsplit ? 0 : (zrow / VC) * (nthreads >> 6) + wid;  // head inside the group
+  const int hl = (zrow / VC) * heads + (wid >> tile_waves);  // head inside the group
   const int h = g * rep + (hl < rep ? hl : 0);
-  const int bshift = qsplit ? 7 : 5;                  // log2 of the tokens a block covers
+  const int bshift = 5 + tile_waves;                  // log2 of the tokens a block covers
   for (;; ++b) {  // there are exactly sum_b ceil(count_b / tokens per block) tiles
     const int nt = (cu[b + 1] - cu[b] + (1 << bshift) - 1) >> bshift;
     if (tile < nt) break;
@@ -382,8 +387,8 @@ __global__ __launch_bounds__(256 * NG, 2) void paged_attention_mfma_kernel(
   const int cnt = cu[b + 1] - cu[b];
   const int col = lane & 31, hf = lane >> 5;
   const int bt_off = tile << bshift;                          // first token of the block
-  const int t_off = bt_off + (qsplit ? wid * 32 : 0);         // first token of this wave
-  const bool head_ok = qsplit ? t_off < cnt : hl < rep;       // this wave computes
+  const int t_off = bt_off + (wid & ((1 << tile_waves) - 1)) * 32;  // first token of this wave
+  const bool head_ok = hl < rep && t_off < cnt;               // this wave computes
   const bool tok_ok = t_off + col < cnt;
   const int my_i = tok_ok ? t_off + col : cnt - 1;
   const long n = cu[b] + my_i;
@@ -410,25 +415,27 @@ __global__ __launch_bounds__(256 * NG, 2) void paged_attention_mfma_kernel(
   const int lo_p0 = first_visible(p0, window, chunk), lo_p1 = first_visible(p1, window, chunk);  // the wave's
   const int wstart = lo_min & ~31;
   const int n_sink = window > 0 ? min(keep_first, wstart) : 0;  // kept keys below the window's first tile
-  const int n_sum = (ksum != nullptr && window > 0) ? max(0, (bp1 - window + 1) / sum_block) : 0;  // the block's last token's
+  const int n_sum = (MORE && ksum != nullptr && window > 0) ? max(0, (bp1 - window + 1) / sum_block) : 0;  // the block's last token's
   const int sum_tiles = (n_sum + 31) >> 5;
   const int sum_mask = (1 << sum_shift) - 1;
   const int sink_tiles = sum_tiles + ((n_sink + 31) >> 5);   // summary tiles, then kept-prefix tiles, then the window's
   const int tiles_n = sink_tiles + ((bp1 - wstart) >> 5) + 1;
-  const int my_sum = (ksum != nullptr && window > 0) ? max(0, (pos - window + 1) / sum_block) : 0;  // this token's
-  const float* db = dist2 != nullptr ? dist2 + (long)h * dist_rows : nullptr;
+  const int my_sum = (MORE && ksum != nullptr && window > 0) ? max(0, (pos - window + 1) / sum_block) : 0;  // this token's
+  const float* db = MORE && dist2 != nullptr ? dist2 + (long)h * dist_rows : nullptr;
 
-  // Staging: a wave's load covers 16 keys of 32 channels (4 lanes a key), load u = wave + 4 r of a tile the quad u % quads
-  // of the 16 keys u / quads, for keys and values alike: a lane looks up two keys of a tile.
-  constexpr int KQ = (D + 31) / 32, VQ = VT;               // quads of a row
-  constexpr int KR = (2 * KQ + 3) / 4, VR = (2 * VQ + 3) / 4;  // loads per wave and tile
-  const int wv = __builtin_amdgcn_readfirstlane(wid) & 3;
-  const int lkey = lane >> 2, lch = (lane & 3) * 8;        // this lane's key of the 16 and channel of the 32
-  // TP key tiles are staged, and multiplied, between two barriers: their loads are all in flight over the
-  // products of the TP tiles before them
-  bf16x8_v rk[TP][KR], rv[TP][VR];
+  // Staging: a wave brings every second piece of its 16 keys of a tile (wave & 1) straight into LDS, piece n the channels
+  // (wave / 2 + 2 n) * 32 of them: a lane looks up one key of a tile, for keys and values alike. A lane whose channels are
+  // beyond the head's brings zeros.
+  constexpr int KR = (KQ + 1) / 2, VR = (VQ + 1) / 2;      // pieces per wave and tile
+  const int row_group = wid & 1, quad0 = wid >> 1;
+  const int lkey = 16 * row_group + (lane >> 2);           // this lane's key of the tile
+  const int lch = ((lane & 3) ^ (lane >> 4 & 3)) * 8;      // and channel of the piece's 32
+  // TP key tiles are staged, and multiplied, between two barriers: their loads go out one by one between the products
+  // of the TP tiles before them (issued together, they held a wave up for 1600 of the 9200 cycles that a step took, and
+  // their stores for 590)
   auto tile_base = [&](int it) {
-    return it < sum_tiles ? it * 32 : it < sink_tiles ? (it - sum_tiles) * 32 : wstart + (it - sink_tiles) * 32;
+    if (MORE && it < sum_tiles) return it * 32;
+    return it < sink_tiles ? (it - sum_tiles) * 32 : wstart + (it - sink_tiles) * 32;
   };
   auto pool_row = [&](int j) {
     const int jc = min(j, bp1);  // keys past the sequence's end are masked; read a row that exists
@@ -439,64 +446,59 @@ __global__ __launch_bounds__(256 * NG, 2) void paged_attention_mfma_kernel(
     return (bt[ic >> sum_shift] << sum_shift) + (ic & sum_mask);
   };
   // The page-table lookups of a tile run one step ahead of its key/value loads (two ahead of its use), so that a
-  // load's address never waits for a lookup issued in the same iteration.
-  // Every channel of the quads is the head's: no lane has to look. A tiling of 48 channels ends in half a quad.
-  const bool kfull = D % 32 == 0 && Dr == D, vfull = Dvr == Dv;
+  // load's address never waits for a lookup issued in the same step.
   const unsigned krs = (unsigned)(G * Dr) * 2u, vrs = (unsigned)(Gv * Dvr) * 2u;   // bytes between neighbouring keys' rows
-  int krow[TP][2], frow[TP];
-  float rf[TP];
-  bool from_sum[TP];  // the tiles of the last lookup that are summary tiles
+  struct Rows {
+    int key[TP], fac[TP];
+    bool from_sum[TP];  // a summary tile
+  };
   auto lookup = [&](int step) {
+    Rows r;
 #pragma unroll
     for (int u = 0; u < TP; ++u) {
       const int it = step * TS + grp * TP + u, kbase = tile_base(it);  // a tile past the last one reads rows that exist and is not used
-      from_sum[u] = it < sum_tiles;
-#pragma unroll
-      for (int i = 0; i < 2; ++i) krow[u][i] = from_sum[u] ? sum_row(kbase + 16 * i + lkey) : pool_row(kbase + 16 * i + lkey);
-      if (key_fac != nullptr && tid < 32) frow[u] = pool_row(kbase + tid);
+      r.from_sum[u] = MORE && it < sum_tiles;
+      r.key[u] = r.from_sum[u] ? sum_row(kbase + lkey) : pool_row(kbase + lkey);
+      r.fac[u] = key_fac != nullptr && tid < 32 ? pool_row(kbase + tid) : 0;
     }
+    return r;
   };
-  auto fetch = [&]() {  // the tiles that the last lookup found
+  const char* zeros = reinterpret_cast<const char*>(zero_channels);
+  auto key_piece = [&](const Rows& r, char* __restrict__ dst, int u, int n) __attribute__((always_inline)) {
+    const int quad = quad0 + 2 * n;
+    if (KQ % 2 != 0 && quad >= KQ) return;
+    const char* at = reinterpret_cast<const char*>((r.from_sum[u] ? ksum : kpool) + (long)g * Dr + quad * 32 + lch) +
+                     (unsigned long)(unsigned)r.key[u] * krs;
+    if (quad * 32 + lch >= Dr) at = zeros;
+    __builtin_amdgcn_global_load_lds((global_ptr)at, (lds_ptr)(dst + u * (KT + VTT) + (quad * 2 + row_group) * 1024), 16, 0, 0);
+  };
+  auto value_piece = [&](const Rows& r, char* __restrict__ dst, int u, int n) __attribute__((always_inline)) {
+    const int quad = quad0 + 2 * n;
+    if (VQ % 2 != 0 && quad >= VQ) return;
+    const char* at = reinterpret_cast<const char*>((r.from_sum[u] ? vsum : vpool) + (long)vg * Dvr + quad * 32 + lch) +
+                     (unsigned long)(unsigned)r.key[u] * vrs;
+    if (quad * 32 + lch >= Dvr) at = zeros;
+    __builtin_amdgcn_global_load_lds((global_ptr)at, (lds_ptr)(dst + u * (KT + VTT) + KT + (quad * 2 + row_group) * 1024), 16, 0, 0);
+  };
+  auto all_pieces = [&](const Rows& r, char* __restrict__ dst) __attribute__((always_inline)) {
 #pragma unroll
     for (int u = 0; u < TP; ++u) {
-      const char* kp = reinterpret_cast<const char*>((from_sum[u] ? ksum : kpool) + (long)g * Dr + lch);
-      const char* vp = reinterpret_cast<const char*>((from_sum[u] ? vsum : vpool) + (long)vg * Dvr + lch);
 #pragma unroll
-      for (int r = 0; r < KR; ++r) {
-        const int q_ = (wv + 4 * r) % KQ, i = (wv + 4 * r) / KQ;   // quad, group of 16 keys
-        if (2 * KQ % 4 != 0 && i > 1) continue;
-        const char* at = kp + q_ * 64 + (unsigned long)(unsigned)(i ? krow[u][1] : krow[u][0]) * krs;
-        rk[u][r] = kfull || q_ * 32 + lch < Dr ? *reinterpret_cast<const bf16x8_v*>(at) : zero8;
-      }
+      for (int n = 0; n < KR; ++n) key_piece(r, dst, u, n);
 #pragma unroll
-      for (int r = 0; r < VR; ++r) {
-        const int q_ = (wv + 4 * r) % VQ, i = (wv + 4 * r) / VQ;
-        if (2 * VQ % 4 != 0 && i > 1) continue;
-        const char* at = vp + q_ * 64 + (unsigned long)(unsigned)(i ? krow[u][1] : krow[u][0]) * vrs;
-        rv[u][r] = vfull || q_ * 32 + lch < Dvr ? *reinterpret_cast<const bf16x8_v*>(at) : zero8;
-      }
-      if (key_fac != nullptr && tid < 32) rf[u] = key_fac[(long)frow[u] * G + g];
+      for (int n = 0; n < VR; ++n) value_piece(r, dst, u, n);
     }
   };
-  auto stash = [&](int buf) {
+  float rf[TP];
+  auto fetch_factors = [&](const Rows& r) {
 #pragma unroll
-    for (int u = 0; u < TP; ++u) {
-      bf16s* ks = tiles + (buf * TS + grp * TP + u) * (KT + VTT);
-      bf16s* vt = ks + KT;
+    for (int u = 0; u < TP; ++u)
+      if (key_fac != nullptr && tid < 32) rf[u] = key_fac[(long)r.fac[u] * G + g];
+  };
+  auto stash_factors = [&](int buf) {
 #pragma unroll
-      for (int r = 0; r < KR; ++r) {
-        const int q_ = (wv + 4 * r) % KQ, i = (wv + 4 * r) / KQ;
-        if (i > 1 || q_ * 32 + lch >= D) continue;
-        *reinterpret_cast<bf16x8_v*>(ks + (q_ * 4 + (lane & 3)) * PL + (16 * i + lkey) * 8) = rk[u][r];
-      }
-#pragma unroll
-      for (int r = 0; r < VR; ++r) {
-        const int q_ = (wv + 4 * r) % VQ, i = (wv + 4 * r) / VQ;
-        if (i > 1) continue;
-        *reinterpret_cast<bf16x8_v*>(vt + (q_ * 4 + (lane & 3)) * PL + (16 * i + lkey) * 8) = rv[u][r];
-      }
+    for (int u = 0; u < TP; ++u)
       if (key_fac != nullptr && tid < 32) facs[(buf * TS + grp * TP + u) * 32 + tid] = rf[u];
-    }
   };
 
   // With a sink and a soft cap the scores live in [-cap2, cap2] (a distance penalty only lowers them) and the
@@ -504,7 +506,11 @@ __global__ __launch_bounds__(256 * NG, 2) void paged_attention_mfma_kernel(
   // running maximum. exp2(cap2) cannot overflow for cap2 <= 96, and a weight that underflows is nothing beside the
   // sink's 1. No maximum to track, no accumulator to rescale.
   const bool fixed_ref = sink != 0 && softcap > 0.0f && softcap * 1.4426950408889634f <= 96.0f;
+  // Without one, m is a maximum the token has had, not always its newest: weights are taken against it as it stands, and
+  // only where the sum of a step's weights shows that some passed 2^12 (a token's first visible score gives inf; NaN counts
+  // too) is the maximum formed, m raised and the weights taken again. A weight of 2^12 has the mantissa of one of 1.
   float m = fixed_ref ? 0.0f : -INFINITY, l = 0.0f;  // m in the base-2 domain
+  float m_ref = fixed_ref ? 0.0f : -3.0e38f;         // m, and below every finite score until there is one
   f32x16 oacc[VT];
 #pragma unroll
   for (int t = 0; t < VT; ++t)
@@ -517,6 +523,7 @@ __global__ __launch_bounds__(256 * NG, 2) void paged_attention_mfma_kernel(
   const bool capped = softcap > 0.0f;
   const float inv_cap = capped ? scale / softcap : 0.0f;
   const float cap2 = softcap * LOG2E, t2 = capped ? 2.0f * LOG2E * scale / softcap : 0.0f;
+  const float cc0 = cap2, cc1 = cap2 * -0.33333069f, cc2 = cap2 * 0.13324751f, cc3 = cap2 * -0.052984238f, cc4 = cap2 * 0.017131345f;
   auto cap_base2 = [&](float dot) {
     const float e = __builtin_amdgcn_exp2f(dot * t2);  // +inf: the quotient is 0; a NaN stays one
     return cap2 - 2.0f * cap2 * __builtin_amdgcn_rcpf(e + 1.0f);
@@ -532,143 +539,134 @@ __global__ __launch_bounds__(256 * NG, 2) void paged_attention_mfma_kernel(
   const float k1 = raw ? c1 : 1.0f;
 
   const int steps_n = (tiles_n + TS - 1) / TS;
-  lookup(0);
-  fetch();
-  if (steps_n > 1) lookup(1);
-  stash(0);
+  const RowAt row_at(col, hf);
+  const ColAt col_at(lane);
+  Rows next = lookup(0);
+  char* mine = tiles + grp * TP * (KT + VTT);     // this group's tiles of the first buffer
+  constexpr int BUF = TS * (KT + VTT);
+  all_pieces(next, mine);
+  fetch_factors(next);
+  if (steps_n > 1) next = lookup(1);
+  stash_factors(0);
+  loads_done();
   __syncthreads();
-  for (int step = 0; step < steps_n; ++step) {
-    const int buf = step & 1;
-    const bool more = step + 1 < steps_n;
-    if (more) {
-      fetch();
-      if (step + 2 < steps_n) lookup(step + 2);
+
+  // A step's tiles of this wave, while the next step's arrive in the other buffer.
+  auto compute = [&](int it0, int kb0, bool inner, const bool (&live)[TP], int buf, const Rows& next, const char* __restrict__ cur,
+                     char* __restrict__ dst) __attribute__((always_inline)) {
+    f32x16 x[TP];
+    float off[TP];
+#pragma unroll
+    for (int u = 0; u < TP; ++u)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) x[u][i] = 0.0f;
+    // the key fragments are read AHEAD products ahead of their own
+    constexpr int AHEAD = 6, NF = DS * TP;
+    bf16x8_v kf[NF];
+    __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+    for (int i = 0; i < AHEAD && i < NF; ++i) kf[i] = frag_row<32>(cur + i % TP * (KT + VTT), row_at, 0, i / TP);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < NF; ++i) {
+      if (i + AHEAD < NF) kf[i + AHEAD] = frag_row<32>(cur + (i + AHEAD) % TP * (KT + VTT), row_at, 0, (i + AHEAD) / TP);
+      x[i % TP] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[i], qf[i / TP], x[i % TP], 0, 0, 0);
+#pragma unroll
+      for (int n = i * (TP * KR) / NF; n < (i + 1) * (TP * KR) / NF; ++n) key_piece(next, dst, n % TP, n / TP);
+      __builtin_amdgcn_sched_barrier(0);
     }
-    // The TP tiles of a step go through the softmax together: one maximum, one exchange, one look at the rescaling.
-    const int it0 = step * TS + grp * TP, kb0 = tile_base(it0);
-    // interior step: every key of its tiles is visible to every token of the wave, no masks to evaluate
-    const bool inner = head_ok && it0 >= sink_tiles && kb0 >= lo_p1 && kb0 + 32 * TP - 1 <= p0 && t_off + 31 < cnt;
-    bool live[TP];       // this wave sees something of the tile
-    bool any = inner;
+    __builtin_amdgcn_s_setprio(0);
+#pragma unroll
+    for (int u = 0; u < TP; ++u) {
+      const int it = it0 + u, kbase = inner ? kb0 + 32 * u : tile_base(it);
+      const bool summ = MORE && !inner && it < sum_tiles;
+      if (key_fac != nullptr) {
+        const float* fc = facs + (buf * TS + grp * TP + u) * 32 + 4 * hf;
+#pragma unroll
+        for (int a = 0; a < 4; ++a) {
+          const float4v f4 = *reinterpret_cast<const float4v*>(fc + 8 * a);
+#pragma unroll
+          for (int c = 0; c < 4; ++c) x[u][4 * a + c] *= f4[c];
+        }
+      }
+      off[u] = sloped && !summ ? -sl2 * (float)(pos - kbase) : 0.0f;
+    }
+    if (capped) {
+      // tanh(y) = y P(y^2) for |y| <= 1/2, P a polynomial through the Chebyshev nodes (1.3e-8 off): fused
+      // multiplications where the general form takes an exponential and a reciprocal
+      float far = 0.0f;
+#pragma unroll
+      for (int u = 0; u < TP; ++u)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) far = fmaxf(far, fabsf(x[u][i]));
+      if (__all(far * fabsf(inv_cap) <= 0.5f)) {
+#pragma unroll
+        for (int u = 0; u < TP; ++u)
+#pragma unroll
+          for (int i = 0; i < 16; ++i) {
+            const float y = x[u][i] * inv_cap, z = y * y;
+            x[u][i] = y * fmaf(z, fmaf(z, fmaf(z, fmaf(z, cc4, cc3), cc2), cc1), cc0);
+          }
+      } else {
+#pragma unroll
+        for (int u = 0; u < TP; ++u)
+#pragma unroll
+          for (int i = 0; i < 16; ++i) x[u][i] = cap_base2(x[u][i]);
+      }
+    }
+    if (!raw) {
+#pragma unroll
+      for (int u = 0; u < TP; ++u) {
+        const int it = it0 + u, kbase = inner ? kb0 + 32 * u : tile_base(it);
+        const bool summ = MORE && !inner && it < sum_tiles;
+        if (sloped && !summ) {
+          if (capped) {
+#pragma unroll
+            for (int i = 0; i < 16; ++i) x[u][i] += row_bias[i];
+          } else {
+#pragma unroll
+            for (int i = 0; i < 16; ++i) x[u][i] = fmaf(x[u][i], c1, row_bias[i]);
+          }
+        } else if (!capped) {
+#pragma unroll
+          for (int i = 0; i < 16; ++i) x[u][i] *= c1;
+        }
+        if (db != nullptr && !summ) {
+#pragma unroll
+          for (int i = 0; i < 16; ++i) {
+            const int j = kbase + (i & 3) + 8 * (i >> 2) + 4 * hf;
+            x[u][i] += db[min(max(pos - j, 0), dist_rows - 1)];
+          }
+        }
+      }
+    }
     if (!inner) {
 #pragma unroll
       for (int u = 0; u < TP; ++u) {
         const int it = it0 + u, kbase = tile_base(it);
-        // (query split) a tile wholly after this wave's tokens, or wholly before what they see
-        live[u] = head_ok && it < tiles_n && (it < sink_tiles || !(kbase > p1 || (kbase + 31 < lo_p0 && kbase >= keep_first)));
-        any = any || live[u];
-      }
-    }
-    if (any) {
-      f32x16 x[TP];
-      float off[TP];
-      __builtin_amdgcn_s_setprio(1);
-#pragma unroll
-      for (int u = 0; u < TP; ++u)
-#pragma unroll
-        for (int i = 0; i < 16; ++i) x[u][i] = 0.0f;
-#pragma unroll
-      for (int s = 0; s < DS; ++s)
-#pragma unroll
-        for (int u = 0; u < TP; ++u) {
-          const bf16x8_v kf =
-              *reinterpret_cast<const bf16x8_v*>(tiles + (buf * TS + grp * TP + u) * (KT + VTT) + (2 * s + hf) * PL + col * 8);
-          x[u] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, qf[s], x[u], 0, 0, 0);
-        }
-      __builtin_amdgcn_s_setprio(0);
-#pragma unroll
-      for (int u = 0; u < TP; ++u) {
-        const int it = it0 + u, kbase = inner ? kb0 + 32 * u : tile_base(it);
-        const bool summ = !inner && it < sum_tiles;
+        const bool summ = MORE && it < sum_tiles;
         const bool ahead = it < sink_tiles;  // a tile ahead of the window's: summaries or kept first tokens
-        if (key_fac != nullptr) {
-          const float* fc = facs + (buf * TS + grp * TP + u) * 32 + 4 * hf;
+        // the tile's keys that this token sees: those up to `last`, from `first` on or below `keep` (offsets in the tile)
+        const int last = !live[u] || !tok_ok ? -1 : summ ? my_sum - 1 - kbase : (ahead ? min(n_sink - 1, pos) : min(p1, pos)) - kbase;
+        const int first = summ ? 0 : lo - kbase, keep = summ ? 0 : keep_first - kbase;
 #pragma unroll
-          for (int a = 0; a < 4; ++a) {
-            const float4v f4 = *reinterpret_cast<const float4v*>(fc + 8 * a);
-#pragma unroll
-            for (int c = 0; c < 4; ++c) x[u][4 * a + c] *= f4[c];
-          }
-        }
-        off[u] = sloped && !summ ? -sl2 * (float)(pos - kbase) : 0.0f;
-        if (!raw) {
-          if (capped) {
-            // tanh(y) = y P(y^2) for |y| <= 1/2, P a polynomial through the Chebyshev nodes (1.3e-8 off): six fused
-            // multiplications where the general form takes an exponential and a reciprocal
-            float far = 0.0f;
-#pragma unroll
-            for (int i = 0; i < 16; ++i) far = fmaxf(far, fabsf(x[u][i]));
-            if (__all(far * inv_cap <= 0.5f)) {
-#pragma unroll
-              for (int i = 0; i < 16; ++i) {
-                const float y = x[u][i] * inv_cap, z = y * y;
-                x[u][i] = cap2 * y * fmaf(z, fmaf(z, fmaf(z, fmaf(z, 0.017131345f, -0.052984238f), 0.13324751f), -0.33333069f), 1.0f);
-              }
-            } else {
-#pragma unroll
-              for (int i = 0; i < 16; ++i) x[u][i] = cap_base2(x[u][i]);
-            }
-            if (sloped && !summ) {
-#pragma unroll
-              for (int i = 0; i < 16; ++i) x[u][i] += row_bias[i];
-            }
-          } else if (sloped && !summ) {
-#pragma unroll
-            for (int i = 0; i < 16; ++i) x[u][i] = fmaf(x[u][i], c1, row_bias[i]);
-          } else {
-#pragma unroll
-            for (int i = 0; i < 16; ++i) x[u][i] *= c1;
-          }
-          if (db != nullptr && !summ) {
-#pragma unroll
-            for (int i = 0; i < 16; ++i) {
-              const int j = kbase + (i & 3) + 8 * (i >> 2) + 4 * hf;
-              x[u][i] += db[min(max(pos - j, 0), dist_rows - 1)];
-            }
-          }
-        }
-        if (!inner) {
-          const int klimit = !live[u] ? 0 : ahead ? n_sink : p1 + 1;  // keys of this tile at or above it are not its to count
-#pragma unroll
-          for (int i = 0; i < 16; ++i) {
-            const int j = kbase + (i & 3) + 8 * (i >> 2) + 4 * hf;
-            const bool seen = tok_ok && (summ ? live[u] && j < my_sum : j < klimit && j <= pos && (j >= lo || j < keep_first));
-            if (!seen) x[u][i] = -INFINITY;
-          }
+        for (int i = 0; i < 16; ++i) {
+          const int j = (i & 3) + 8 * (i >> 2) + 4 * hf;
+          x[u][i] = (j <= last) & ((j >= first) | (j < keep)) ? x[u][i] : -INFINITY;
         }
       }
-      float m_ref = 0.0f;
-      if (!fixed_ref) {
-        float tmax = -INFINITY;
-#pragma unroll
-        for (int u = 0; u < TP; ++u) {
-          float top = x[u][0];
-#pragma unroll
-          for (int i = 1; i < 16; ++i) top = fmaxf(top, x[u][i]);
-          tmax = fmaxf(tmax, top == -INFINITY ? -INFINITY : fmaf(top, k1, off[u]));
-        }
-        tmax = fmaxf(tmax, __shfl_xor(tmax, 32));
-        const float m_new = fmaxf(m, tmax);
-        if (!__all(m_new == m)) {  // otherwise the running maxima of all 32 tokens stand still: no rescaling
-          const float corr = (m == -INFINITY) ? 1.0f : __builtin_amdgcn_exp2f(m - m_new);  // nothing accumulated: nothing to rescale
-          l *= corr;
-#pragma unroll
-          for (int t = 0; t < VT; ++t)
-#pragma unroll
-            for (int i = 0; i < 16; ++i) oacc[t][i] *= corr;
-        }
-        m = m_new;
-        m_ref = (m_new == -INFINITY) ? 0.0f : m_new;  // nothing visible yet: every weight is exp2(-inf) = 0
-      }
+      asm volatile("" ::: "memory");   // a body of its own: merged into the common one, every step would pay for it
+    }
+    bf16x8_v phi[TP][2], plo[TP][2];
+    auto weights = [&](auto plain) __attribute__((always_inline)) {
       float psum = 0.0f;
-      bf16x8_v phi[TP][2], plo[TP][2];
 #pragma unroll
       for (int u = 0; u < TP; ++u) {
         const float base = off[u] - m_ref;
 #pragma unroll
         for (int i = 0; i < 16; i += 2) {  // two weights a time: one conversion packs two halves
-          const float p0 = __builtin_amdgcn_exp2f(fmaf(x[u][i], k1, base));
-          const float p1 = __builtin_amdgcn_exp2f(fmaf(x[u][i + 1], k1, base));
+          const float p0 = __builtin_amdgcn_exp2f(plain ? x[u][i] : fmaf(x[u][i], k1, base));
+          const float p1 = __builtin_amdgcn_exp2f(plain ? x[u][i + 1] : fmaf(x[u][i + 1], k1, base));
           psum += p0 + p1;
           const bf16x2_v hi = __builtin_convertvector(float2v{p0, p1}, bf16x2_v);
           const unsigned bits = __builtin_bit_cast(unsigned, hi);
@@ -680,27 +678,77 @@ __global__ __launch_bounds__(256 * NG, 2) void paged_attention_mfma_kernel(
           plo[u][i >> 3][(i & 7) + 1] = lo[1];
         }
       }
-      l += psum;
-      // O^T += V^T P^T: slot hf * 8 + e of step s2 holds key kbase + 16 s2 + 8 (e >> 2) + 4 hf + (e & 3)
-      __builtin_amdgcn_s_setprio(1);
+      return psum;
+    };
+    float psum;
+    if (fixed_ref && !sloped) {   // scores in the base-2 domain, against 0
+      psum = weights(std::true_type());
+      asm volatile("" ::: "memory");
+    } else {
+      for (bool raised = false;; raised = true) {
+        psum = weights(std::false_type());
+        if (fixed_ref || raised || __all(psum <= 4096.0f)) break;
+        float tmax = -INFINITY;
 #pragma unroll
-      for (int u = 0; u < TP; ++u)
+        for (int u = 0; u < TP; ++u) {
+          float top = x[u][0];
 #pragma unroll
-        for (int s2 = 0; s2 < 2; ++s2)
+          for (int i = 1; i < 16; ++i) top = fmaxf(top, x[u][i]);
+          tmax = fmaxf(tmax, top == -INFINITY ? -INFINITY : fmaf(top, k1, off[u]));
+        }
+        tmax = fmaxf(tmax, __shfl_xor(tmax, 32));
+        const float m_new = fmaxf(m, tmax);
+        const float corr = (m == -INFINITY) ? 1.0f : __builtin_amdgcn_exp2f(m - m_new);  // nothing accumulated: nothing to rescale
+        l *= corr;
 #pragma unroll
-          for (int t = 0; t < VT; ++t) {
-            const bf16s* vp = tiles + (buf * TS + grp * TP + u) * (KT + VTT) + KT +
-                              (4 * t + 2 * ((lane >> 4) & 1) + ((lane & 3) >> 1)) * PL +
-                              (16 * s2 + 4 * hf + ((lane & 15) >> 2)) * 8 + (lane & 1) * 4;
-            const bf16x4_v v0 = ld_tr16(reinterpret_cast<const char*>(vp), 0);
-            const bf16x4_v v1 = ld_tr16(reinterpret_cast<const char*>(vp), 8 * 16);
-            const bf16x8_v va = __builtin_shufflevector(v0, v1, 0, 1, 2, 3, 4, 5, 6, 7);
-            oacc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va, phi[u][s2], oacc[t], 0, 0, 0);
-            oacc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va, plo[u][s2], oacc[t], 0, 0, 0);
-          }
-      __builtin_amdgcn_s_setprio(0);
+        for (int t = 0; t < VT; ++t)
+#pragma unroll
+          for (int i = 0; i < 16; ++i) oacc[t][i] *= corr;
+        m = m_new;
+        m_ref = (m_new == -INFINITY) ? -3.0e38f : m_new;  // nothing visible yet: every weight is exp2(-inf) = 0
+      }
     }
-    if (more) stash(buf ^ 1);
+    l += psum;
+    // O^T += V^T P^T: slot hf * 8 + e of step s2 holds key kbase + 16 s2 + 8 (e >> 2) + 4 hf + (e & 3)
+    __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+    for (int u = 0; u < TP; ++u)
+#pragma unroll
+      for (int s2 = 0; s2 < 2; ++s2) {
+#pragma unroll
+        for (int t = 0; t < VT; ++t) {
+          const bf16x8_v va = frag_born<32>(cur + u * (KT + VTT) + KT, col_at, 16 * s2, 32 * t);
+          oacc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va, phi[u][s2], oacc[t], 0, 0, 0);
+          oacc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va, plo[u][s2], oacc[t], 0, 0, 0);
+        }
+        const int at = u * 2 + s2;
+#pragma unroll
+        for (int n = at * (TP * VR) / (2 * TP); n < (at + 1) * (TP * VR) / (2 * TP); ++n) value_piece(next, dst, n % TP, n / TP);
+      }
+    __builtin_amdgcn_s_setprio(0);
+  };
+  for (int step = 0; step < steps_n; ++step) {
+    const int buf = step & 1;
+    const Rows now = next;          // the next step's rows; its loads repeat the last step's where there is none
+    if (step + 2 < steps_n) next = lookup(step + 2);
+    if (step + 1 < steps_n) fetch_factors(now);
+    // The TP tiles of a step go through the softmax together: one sum, one look at the reference.
+    const int it0 = step * TS + grp * TP, kb0 = tile_base(it0);
+    // interior step: every key of its tiles is visible to every token of the wave, no masks to evaluate
+    const bool inner = head_ok && it0 >= sink_tiles && kb0 >= lo_p1 && kb0 + 32 * TP - 1 <= p0 && t_off + 31 < cnt;
+    bool live[TP];       // this wave sees something of the tile
+    bool any = inner;
+#pragma unroll
+    for (int u = 0; u < TP; ++u) {
+      const int it = it0 + u, kbase = tile_base(it);
+      // (several token tiles) a tile wholly after this wave's tokens, or wholly before what they see
+      live[u] = inner || (head_ok && it < tiles_n && (it < sink_tiles || !(kbase > p1 || (kbase + 31 < lo_p0 && kbase >= keep_first))));
+      any = any || live[u];
+    }
+    if (any) compute(it0, kb0, inner, live, buf, now, mine + buf * BUF, mine + (buf ^ 1) * BUF);
+    else all_pieces(now, mine + (buf ^ 1) * BUF);
+    if (step + 1 < steps_n) stash_factors(buf ^ 1);
+    loads_done();
     __syncthreads();
   }
   if constexpr (NG > 1) {  // the second group's states, wave by wave, through the tiles' place (all waves are past their last tile)
@@ -816,37 +864,49 @@ static bool launch_mfma_attention(at::Tensor& out, const at::Tensor& q, const at
                                   const at::Tensor& block_tables, const at::Tensor& cu, const at::Tensor& start,
                                   const float* slp, const c10::optional<at::Tensor>& gate, long gstride, double scale,
                                   int64_t window, int64_t keep_first, double softcap, bool sink, int page_shift,
-                                  int64_t num_tiles, int64_t num_tiles128, const ScalarExtras& x) {
+                                  int64_t num_tiles, int64_t num_tiles128, int64_t num_tiles64, const ScalarExtras& x) {
   const int H = (int)q.size(1), D = (int)q.size(2);
   const int G = (int)kpool.size(2), Dv = (int)vpool.size(3);
   // prompt portions in bfloat16 go to the matrix cores when the head sizes fit a tiling;
   // num_tiles = sum over sequences of ceil(new tokens / 32), 0 asks for the scalar kernel
-  const bool aligned = q.stride(0) % 8 == 0 && reinterpret_cast<uintptr_t>(q.data_ptr()) % 16 == 0;
+  auto at16 = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
+  const bool aligned = q.stride(0) % 8 == 0 && at16(q.data_ptr()) && at16(kpool.data_ptr()) && at16(vpool.data_ptr()) &&
+                       at16(x.ksum) && at16(x.vsum);
   // head sizes that are multiples of 8 ride in the next larger tiling, zero-padded
   const bool mfma_shape = D % 8 == 0 && Dv % 8 == 0 && D <= 128 && Dv <= 128;
   if (!(num_tiles > 0 && is_bf16(q) && aligned && mfma_shape && vpool.is_contiguous())) return false;
   {
     const int rep = H / G, nw = 4;
-    // one query head per kv head: the waves of a block take four consecutive token tiles instead of four heads
-    const int qsplit = (rep == 1 && num_tiles128 > 0) ? 1 : 0;
+    // one query head per kv head: the waves of a block take four consecutive token tiles instead of four heads; two: two
+    const int tile_waves = rep == 1 && num_tiles128 > 0 ? 2 : rep == 2 && num_tiles64 > 0 ? 1 : 0, heads = nw >> tile_waves;
     const int VC = x.cross_out != nullptr ? G : 1;
-    const int tiles = (int)(qsplit ? num_tiles128 : num_tiles), rows = G * ((rep + nw - 1) / nw) * VC;
+    const int tiles = (int)(tile_waves == 2 ? num_tiles128 : tile_waves == 1 ? num_tiles64 : num_tiles);
+    const int rows = G * ((rep + heads - 1) / heads) * VC;
     const int sub = rows <= 8 && 8 % rows == 0 ? 8 / rows : 1;   // XCDs a row's tiles are spread over: whole rounds of them
     const dim3 grid((unsigned)((tiles + sub - 1) / sub * sub * rows));
     const int ds = D <= 32 ? 2 : D <= 48 ? 3 : D <= 64 ? 4 : D <= 96 ? 6 : 8, vt = (Dv + 31) / 32;
     // Two groups of waves take alternate key tiles where one block a CU is all there is: a second group then fills the
-    // idle half of the CU, and a lone block's chain of tiles is half as long. Measured, one group against two: 2 x 256
-    // tokens 31 -> 23 us (64 blocks), 3 x 200 after 1500 207 -> 130 (84), 100 alone 18 -> 15 (16). With 512 blocks it is mixed: 4 x 1000 117 -> 95 and
-    // 4096 tokens 205 -> 197, but 204 -> 226 with 16 key heads, 87 -> 107 with a window of 1024; beyond that it loses
-    // (16 x 1024, 2048 blocks: 175 -> 182; 4096 of 64 heads, 2048 blocks: 507 -> 572).
-    const int ng = grid.x <= 256 ? 2 : 1;
+    // idle half of the CU, and a lone block's chain of tiles is half as long (2 x 256 tokens 31 -> 23 us, 64 blocks; 3 x 200 after
+    // 1500 207 -> 130; 100 alone 18 -> 15). Up to 512 blocks of a causal prompt too: their lengths differ, a CU takes a long one and then
+    // a short one instead of both at once, of which the long one's last steps run alone (4096 tokens 138 -> 115 us, a cap and a sink
+    // 172 -> 136; 2000 of 64 channels 85 -> 59). A window makes them equally long, and two blocks at once are better (4096
+    // tokens, window 1024: 69 against 85; a mixed step of 308 blocks 77 against 90).
+    const int ng = grid.x <= (window > 0 ? 256 : 512) ? 2 : 1;
+    const bool more = x.ksum != nullptr || x.dist_bias != nullptr;
     const size_t msmem = (size_t)2 * ng * MFMA_TILES_PER_STEP *
-                         ((ds * 2 + vt * 4) * (32 * 8 + 32) * sizeof(bf16s) + (x.key_fac != nullptr ? 32 * sizeof(float) : 0));
-#define MFMA_CASE(DS_, VT_) \
-  do { if (ng == 2) MFMA_NG(DS_, VT_, 2); else MFMA_NG(DS_, VT_, 1); } while (0)
-#define MFMA_NG(DS_, VT_, NG_)                                                                                     \
+                         (((ds + 1) / 2 + vt) * 2048 + (x.key_fac != nullptr ? 32 * sizeof(float) : 0));
+// The common form exists for the sizes that serving meets most, 64 and 128 channels, and for the others with all there is.
+#define MFMA_CASE(DS_, VT_)                                                                       \
+  do {                                                                                            \
+    constexpr bool ALWAYS = !((DS_ == 4 || DS_ == 8) && (VT_ == 2 || VT_ == 4));                  \
+    if (ng == 2 && (more || ALWAYS)) MFMA_NG(DS_, VT_, 2, true);                                  \
+    else if (ng == 2) MFMA_NG(DS_, VT_, 2, ALWAYS);                                               \
+    else if (more || ALWAYS) MFMA_NG(DS_, VT_, 1, true);                                          \
+    else MFMA_NG(DS_, VT_, 1, ALWAYS);                                                            \
+  } while (0)
+#define MFMA_NG(DS_, VT_, NG_, MORE_)                                                                                     \
   do {                                                                                                             \
-    auto kfn = paged_attention_mfma_kernel<DS_, VT_, NG_>;                                                         \
+    auto kfn = paged_attention_mfma_kernel<DS_, VT_, NG_, MORE_>;                                                         \
     if (msmem > 65536) /* more dynamic LDS than a kernel gets without asking */                                    \
       (void)hipFuncSetAttribute((const void*)kfn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)msmem);         \
     hipLaunchKernelGGL(kfn, grid, dim3(64 * nw * NG_), msmem, stream(),                                            \
@@ -856,7 +916,7 @@ static bool launch_mfma_attention(at::Tensor& out, const at::Tensor& q, const at
                        (int)block_tables.stride(0), cu.data_ptr<int>(), start.data_ptr<int>(), slp,                \
                        gate.has_value() ? ptr<bf16s>(*gate) : (const bf16s*)nullptr, gstride, H, G, D, Dv,         \
                        page_shift, (float)scale, (int)window, (int)keep_first, (float)softcap, sink ? 1 : 0,       \
-                       qsplit, x.sink_logits, x.dist_bias, x.dist_rows, (const bf16s*)x.ksum,                      \
+                       tile_waves, x.sink_logits, x.dist_bias, x.dist_rows, (const bf16s*)x.ksum,                      \
                        (const bf16s*)x.vsum, x.sum_shift, x.sum_block, x.cross_out, x.chunk, x.key_fac, x.vrep,    \
                        x.out32, tiles);                                                                            \
   } while (0)
@@ -883,7 +943,7 @@ static bool launch_mfma_attention(at::Tensor& out, const at::Tensor& q, const at
 at::Tensor paged_attention(at::Tensor q, at::Tensor kpool, at::Tensor vpool, at::Tensor block_tables, at::Tensor cu,
                            at::Tensor start, at::Tensor tok_seq, at::Tensor positions, double scale, int64_t window,
                            int64_t keep_first, c10::optional<at::Tensor> slopes, c10::optional<at::Tensor> gate,
-                           int64_t num_tiles, double softcap, bool sink, int64_t num_tiles128) {
+                           int64_t num_tiles, double softcap, bool sink, int64_t num_tiles128, int64_t num_tiles64) {
   check_act(q, "q");
   TORCH_CHECK(softcap >= 0.0, "softcap must not be negative (0 = none)");
   TORCH_CHECK(q.dim() == 3 && q.stride(2) == 1 && q.stride(1) == q.size(2), "q must be [N, H, D] with dense rows");
@@ -921,7 +981,7 @@ at::Tensor paged_attention(at::Tensor q, at::Tensor kpool, at::Tensor vpool, at:
   if (N == 0) return out;
   check_i32(cu, "cu"); check_i32(start, "start");
   if (launch_mfma_attention(out, q, kpool, vpool, block_tables, cu, start, slp, gate, gstride, scale, window, keep_first,
-                            softcap, sink, page_shift, num_tiles, num_tiles128, ScalarExtras()))
+                            softcap, sink, page_shift, num_tiles, num_tiles128, num_tiles64, ScalarExtras()))
     return out;
   launch_scalar_attention(out, q, kpool, vpool, block_tables, tok_seq, positions, slp, gate, gstride, scale, window,
                           keep_first, softcap, sink, page_shift, vrow, vhead, ScalarExtras());
@@ -938,7 +998,8 @@ at::Tensor paged_attention_ext(at::Tensor q, at::Tensor kpool, at::Tensor vpool,
                                double softcap, bool sink, c10::optional<at::Tensor> sink_logits,
                                c10::optional<at::Tensor> dist_bias, c10::optional<at::Tensor> ksum,
                                c10::optional<at::Tensor> vsum, int64_t sum_block, bool cross, int64_t num_tiles,
-                               int64_t num_tiles128, int64_t chunk, c10::optional<at::Tensor> key_fac, bool out_f32) {
+                               int64_t num_tiles128, int64_t num_tiles64, int64_t chunk,
+                               c10::optional<at::Tensor> key_fac, bool out_f32) {
   check_act(q, "q");
   TORCH_CHECK(softcap >= 0.0, "softcap must not be negative (0 = none)");
   TORCH_CHECK(q.dim() == 3 && q.stride(2) == 1 && q.stride(1) == q.size(2), "q must be [N, H, D] with dense rows");
@@ -1029,7 +1090,7 @@ at::Tensor paged_attention_ext(at::Tensor q, at::Tensor kpool, at::Tensor vpool,
       x2.dist_bias = db2.data_ptr<float>();
     }
     if (launch_mfma_attention(out, q, kpool, vpool, block_tables, cu, start, slp, gate, gstride, scale, window,
-                              keep_first, softcap, sink, page_shift, num_tiles, num_tiles128, x2))
+                              keep_first, softcap, sink, page_shift, num_tiles, num_tiles128, num_tiles64, x2))
       return out;
   }
   launch_scalar_attention(out, q, kpool, vpool, block_tables, tok_seq, positions, slp, gate, gstride, scale, window,

@@ -218,8 +218,9 @@ def paged_attention(q, kpool, vpool, batch: RaggedBatch, scale: float, window: i
         o = serving_kernels().paged_attention_ext(q, kpool, vpool, batch.block_tables, batch.cu, batch.start,
                                                   batch.tok_seq, batch.positions, scale, window, keep_first, slopes,
                                                   gate, float(softcap), bool(sink), sink_logits, dist_bias, ksum, vsum,
-                                                  int(block), talk is not None, batch.num_tiles32, batch.num_tiles128, int(chunk),
-                                                  key_factors, out_dtype == torch.float32)
+                                                  int(block), talk is not None, batch.num_tiles32, batch.num_tiles128,
+                                                  batch.num_tiles64, int(chunk), key_factors,
+                                                  out_dtype == torch.float32)
         if talk is None:
             return o
         return serving_kernels().talk_mix(o, talk, q.dtype)
@@ -227,6 +228,6 @@ def paged_attention(q, kpool, vpool, batch: RaggedBatch, scale: float, window: i
         return serving_kernels().paged_attention(q, kpool, vpool, batch.block_tables, batch.cu, batch.start,
                                                  batch.tok_seq, batch.positions, scale, window, keep_first,
                                                  slopes, gate, batch.num_tiles32, float(softcap), bool(sink),
-                                                 batch.num_tiles128)
+                                                 batch.num_tiles128, batch.num_tiles64)
     return paged_attention_ref(q, kpool, vpool, batch, scale, window, keep_first, slopes, gate, softcap, sink,
                                sink_logits, dist_bias, pooled, talk, chunk, key_factors, out_dtype)

@@ -47,21 +47,28 @@ class RaggedBatch:
     def max_new(self) -> int:
         return max(self.cu_host[i + 1] - self.cu_host[i] for i in range(self.num_seqs))
 
+    def _tiles(self, tokens: int) -> int:
+        if self.max_new == 1:
+            return 0
+        return sum((self.cu_host[i + 1] - self.cu_host[i] + tokens - 1) // tokens for i in range(self.num_seqs))
+
     @property
     def num_tiles32(self) -> int:
         """32-token tiles of the prompt portions (0 for a pure decode step):
         the grid of the matrix-core attention kernel."""
-        if self.max_new == 1:
-            return 0
-        return sum((self.cu_host[i + 1] - self.cu_host[i] + 31) // 32 for i in range(self.num_seqs))
+        return self._tiles(32)
+
+    @property
+    def num_tiles64(self) -> int:
+        """64-token tiles of the prompt portions (0 for a pure decode step): the grid of the matrix-core attention
+        kernel when every key head has two query heads."""
+        return self._tiles(64)
 
     @property
     def num_tiles128(self) -> int:
         """128-token tiles of the prompt portions (0 for a pure decode step): the grid of the matrix-core attention
         kernel when every key head has a single query head."""
-        if self.max_new == 1:
-            return 0
-        return sum((self.cu_host[i + 1] - self.cu_host[i] + 127) // 128 for i in range(self.num_seqs))
+        return self._tiles(128)
 
     @property
     def max_total(self) -> int:

@@ -182,3 +182,57 @@ def test_every_tile_is_taken_once(H, G, counts, starts, page, D, Dv, kw):
 def test_soft_caps_near_and_far(softcap, scale):
     """Scores far below the cap, about it and far above it: the two forms of tanh."""
     _check([64, 700], [10, 0], 16, 4, 64, 64, 16, scale, softcap=softcap, sink=True)
+
+
+# One, two, three and four or more query heads a key head: blocks of 128, 64 and 32 tokens. Head sizes that fill the pieces of 32 channels that
+# tiles are loaded in, end inside one, or leave one of a pair out.
+@pytest.mark.parametrize("H,G,D,Dv", [(2, 2, 128, 128), (4, 2, 128, 128), (4, 2, 64, 128), (3, 1, 64, 64), (5, 1, 128, 64), (4, 2, 96, 96),
+                                      (2, 1, 48, 40), (4, 1, 24, 8), (4, 2, 72, 104)])
+@pytest.mark.parametrize("kw", [{}, dict(softcap=5.0, sink=True), dict(slopes=True, window=70, keep_first=4, gate=True),
+                                dict(factors=True, chunk=100)])
+def test_portions_of_head_counts_and_sizes(H, G, D, Dv, kw):
+    _check([33, 1, 96, 65, 64, 129], [0, 130, 31, 64, 1, 500], H, G, D, Dv, 16, 0.1, **dict(kw))
+
+
+@pytest.mark.parametrize("levels", [
+    (0, 9, 18, 27, 36, 45),          # every step's weights pass the reference of the one before
+    (60, 40, 20, 0, -20, -40),       # the first keys have the largest scores
+    (-3000, 0, -3000, 4, 8, 1000),   # far below, far above
+])
+@pytest.mark.parametrize("kw", [{}, dict(sink_logits=True), dict(window=200, keep_first=5)])
+@pytest.mark.parametrize("rows", [1, 16])
+def test_scores_that_rise_and_fall(levels, kw, rows):
+    """Keys 64 at a time have scores of a level of their own (in nats): the reference that a token's weights are taken against is left
+    behind, raised, or stays. `rows` sequences: two groups of waves a block, or one."""
+    from colossalai_amd.ops.paged_attention import paged_attention, paged_attention_ref
+
+    torch.manual_seed(6)
+    n, scale = 64 * len(levels), 128 ** -0.5
+    batch, pages = _batch([n - 10] * rows, [10] * rows, 64)
+    k, v = (torch.randn(pages, 64, 4, 128, device="cuda").bfloat16() for _ in range(2))
+    q = torch.randn(rows * (n - 10), 16, 128, device="cuda").bfloat16()
+    q[..., 0] = 8.0
+    for b in range(rows):
+        for i, level in enumerate(levels):
+            k[batch.block_tables[b, i].long(), :, :, 0] = level / (8.0 * scale)
+    kw = dict(kw)
+    if kw.pop("sink_logits", False):
+        kw["sink_logits"] = torch.randn(16, device="cuda") + 2.0
+    got = paged_attention(q, k, v, batch, scale, **kw)
+    want = paged_attention_ref(q.float(), k.float(), v.float(), batch, scale, **kw)
+    assert (got.double() - want.double()).norm() / want.double().norm() < BOUND
+
+
+@pytest.mark.parametrize("which", ["keys", "values"])
+def test_pools_at_an_odd_address(which):
+    from colossalai_amd.ops.paged_attention import paged_attention
+
+    torch.manual_seed(7)
+    batch, pages = _batch([40, 1], [100, 3], 16)
+    k, v = (torch.randn(pages, 16, 2, 64, device="cuda").bfloat16() for _ in range(2))
+    q = torch.randn(41, 4, 64, device="cuda").bfloat16()
+    want = paged_attention(q, k, v, batch, 0.1)
+    t = k if which == "keys" else v
+    odd = torch.empty(t.numel() + 1, device="cuda", dtype=t.dtype)[1:].view(t.shape).copy_(t)
+    got = paged_attention(q, odd if which == "keys" else k, odd if which == "values" else v, batch, 0.1)
+    assert (got.double() - want.double()).norm() / want.double().norm() < 2 * BOUND
