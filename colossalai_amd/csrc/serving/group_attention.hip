@@ -1,0 +1,352 @@
+// Attention of decode tokens on the matrix cores (bfloat16, head sizes 64 and 128): one block per (token, kv head, part of the
+// token's keys) with the kv head's whole group of query heads, so that every cached row is read once.
+//
+// A wave takes a tile of 32 keys by itself: its keys and values come straight into LDS of its own (lds_tiles.h), no
+// barrier until the end. As in the prompt portions' kernel the products are formed transposed,
+//   S^T = K Q^T (A = key rows, B = query rows in registers: column = head), O^T = V^T P^T (the float32 weights in the C
+//   layout they were born in, split into a high and a low bfloat16 half; A = values by transposing reads),
+// so a head is a lane and its half-wave twin. Of the 32 columns the group fills 1 to 16; the products cost a tenth of the time that
+// the tile's 16 KB take to arrive. The next tile's keys are on their way from the moment the scores are
+// formed, its values from the end of the products.
+// What bounds it: memory beyond about 8 us of dependent loads (position, page table, rows), launch and the end. Against
+// the form with a row in the registers of a few lanes (row_attention.hip), 16 heads on 4 of 128: 16 x 1024 keys with a cap
+// and a sink 18.5 -> 16.5 us, 4 x 16384 52.0 -> 38.1 (3.5 TB/s), 16 x 8192 84 -> 63 (4.3 TB/s), 8 heads on 2, 7 x 5000
+// 24.8 -> 17.5; 16 heads on 8 of 64, 16 x 3000: 41.5 -> 28.8; one head a key head, 16 x 2000: 61 -> 56; 16 x 128: 9.4 and 9.9.
+// The eight waves' states meet in LDS at the end; few tokens with long contexts have their keys cut into parts, whose
+// states row_merge_kernel puts together.
+#include "paged_attention.h"
+#include "../lds_tiles.h"
+
+#include <algorithm>
+#include <type_traits>
+
+namespace cai {
+namespace serving {
+
+namespace {
+
+constexpr int GROUP_WAVES = 8;
+constexpr size_t GROUP_LDS = 160 * 1024;   // of a CU
+constexpr int GROUP_HEADS = 16;     // most query heads of a kv head: their states must fit into a wave's tile
+typedef __bf16 bf16x2_v __attribute__((ext_vector_type(2)));
+
+// at most N vector memory operations of this wave are on their way; what follows reads what the others brought
+template <int N>
+DEV_INLINE void loads_left() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | 0x0f70);
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_sched_barrier(0);
+}
+
+template <int DS, int VT>
+__global__ __launch_bounds__(64 * GROUP_WAVES, 2) void group_attention_kernel(
+    bf16s* __restrict__ out, const bf16s* __restrict__ q, long q_stride, const bf16s* __restrict__ kpool,
+    const bf16s* __restrict__ vpool, const int* __restrict__ block_tables, int bt_stride, const int* __restrict__ tok_seq,
+    const int* __restrict__ positions, const float* __restrict__ slopes, const bf16s* __restrict__ gate, long gate_stride,
+    const float* __restrict__ sink_logits, int H, int G, int page_shift, float scale, int window, int keep_first, int chunk,
+    float softcap, int sink, int vrep, long vrow, long vhead, int splits, float* __restrict__ ws) {
+  constexpr int D = DS * 16, Dv = VT * 32, KQ = D / 32, KT = D * 64, VTT = Dv * 64;   // bytes of a tile's keys, values
+  constexpr float LOG2E = 1.4426950408889634f;
+  extern __shared__ __align__(16) char tiles[];   // [waves][KT + VTT], later the waves' states; then the pages
+  int* pages = reinterpret_cast<int*>(tiles + GROUP_WAVES * (KT + VTT));
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int col = lane & 31, hf = lane >> 5;
+  const int split = (int)(blockIdx.x % splits);
+  const long n = blockIdx.x / splits / G;
+  const int g = (int)(blockIdx.x / splits % G);
+  const int R = H / G, h0 = g * R;
+  const int pos = positions[n];
+  const int* bt = block_tables + (long)tok_seq[n] * bt_stride;
+  const int page_mask = (1 << page_shift) - 1;
+  const bool head = col < R;
+  bf16x8_v qf[DS];
+#pragma unroll
+  for (int s = 0; s < DS; ++s) qf[s] = ld_g16b(q + n * q_stride + (long)(h0 + min(col, R - 1)) * D + 16 * s + hf * 8);
+  const bool sloped = slopes != nullptr;
+  float sl2 = sloped ? slopes[h0 + min(col, R - 1)] : 0.0f;
+
+  // The token's keys: kept first ones, then those from `lo` to its own position
+  const int lo = first_visible(pos, window, chunk);
+  const int n_keep = window > 0 ? min(keep_first, lo) : 0;
+  const int total = n_keep + (pos - lo + 1);
+  const int all = (total + 31) >> 5, per = (all + splits - 1) / splits;
+  const int last = min(all, (split + 1) * per);
+  const int lkey = lane >> 2, lch = ((lane & 3) ^ (lane >> 4 & 3)) * 8;   // of a load: this lane's key of 16, channel of 32
+  // Page numbers of this block's keys in LDS: looked up in memory tile by tile, they would stand between the keys' and
+  // values' loads, and waiting for one would be waiting for all of these.
+  const int i0 = split * per * 32, i1 = min(last * 32, total);      // the block's keys, counted from the first kept one
+  const int w0 = i0 < n_keep ? lo : lo + (i0 - n_keep);             // the first one beyond the kept ones
+  const int keep_pages = i0 < n_keep ? (n_keep + page_mask) >> page_shift : 0;
+  const int num_pages = i0 < i1 ? keep_pages + ((lo + (i1 - 1 - n_keep)) >> page_shift) - (w0 >> page_shift) + 1 : 0;
+  for (int i = threadIdx.x; i < num_pages; i += 64 * GROUP_WAVES)
+    pages[i] = bt[i < keep_pages ? i : (w0 >> page_shift) + i - keep_pages];
+  __syncthreads();
+  struct Rows { int at[2]; };
+  auto lookup = [&](int t) {
+    Rows r;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int idx = min(t * 32 + i * 16 + lkey, total - 1);       // past the end: the token's own row
+      const int j = idx < n_keep ? idx : lo + (idx - n_keep);
+      const int p = idx < n_keep ? j >> page_shift : keep_pages + (j >> page_shift) - (w0 >> page_shift);
+      r.at[i] = (pages[p] << page_shift) + (j & page_mask);
+    }
+    return r;
+  };
+  const char* kbase = reinterpret_cast<const char*>(kpool + (long)g * D + lch);
+  const char* vbase = reinterpret_cast<const char*>(vpool + (long)(g / vrep) * vhead + lch);
+  const unsigned krs = (unsigned)(G * D) * 2u, vrs = (unsigned)vrow * 2u;   // bytes between neighbouring keys' rows
+  auto load_keys = [&](const Rows& r, char* __restrict__ dst) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int c = 0; c < KQ; ++c)
+        __builtin_amdgcn_global_load_lds((global_ptr)(kbase + (unsigned long)(unsigned)r.at[i] * krs + c * 64), (lds_ptr)(dst + (c * 2 + i) * 1024), 16, 0, 0);
+  };
+  auto load_values = [&](const Rows& r, char* __restrict__ dst) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int c = 0; c < VT; ++c)
+        __builtin_amdgcn_global_load_lds((global_ptr)(vbase + (unsigned long)(unsigned)r.at[i] * vrs + c * 64), (lds_ptr)(dst + (c * 2 + i) * 1024), 16, 0, 0);
+  };
+
+  int t = split * per + wid;
+  Rows first;
+  if (t < last) {
+    first = lookup(t);
+    load_keys(first, tiles + wid * (KT + VTT));
+    load_values(first, tiles + wid * (KT + VTT) + KT);
+  }
+  sl2 *= LOG2E;
+  if (scale < 0.0f) {   // exact: the largest product of a head is then its largest score
+#pragma unroll
+    for (int s = 0; s < DS; ++s) qf[s] = -qf[s];
+    scale = -scale;
+  }
+  // Scores in the base-2 domain; the reference m is raised only where a tile's sum shows that it must be, as in the prompt
+  // portions' kernel.
+  const float c1 = scale * LOG2E < 1e-30f ? 1e-30f : scale * LOG2E;   // NaN stays
+  const bool capped = softcap > 0.0f;
+  const float inv_cap = capped ? scale / softcap : 0.0f, cap2 = softcap * LOG2E, t2 = capped ? 2.0f * LOG2E * scale / softcap : 0.0f;
+  float m = -INFINITY, m_ref = -3.0e38f, l = 0.0f;
+  f32x16 oacc[VT];
+#pragma unroll
+  for (int t = 0; t < VT; ++t)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) oacc[t][i] = 0.0f;
+  const RowAt row_at(col, hf);
+  const ColAt col_at(lane);
+  char* keys = tiles + wid * (KT + VTT);
+
+  auto tile = [&](int t, auto more, const Rows& next, char* __restrict__ K_, char* __restrict__ V_) __attribute__((always_inline)) {
+    f32x16 x;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) x[i] = 0.0f;
+    constexpr int AHEAD = 4;
+    bf16x8_v kf[DS];
+#pragma unroll
+    for (int s = 0; s < AHEAD; ++s) kf[s] = frag_row<32>(K_, row_at, 0, s);
+#pragma unroll
+    for (int s = 0; s < DS; ++s) {
+      if (s + AHEAD < DS) kf[s + AHEAD] = frag_row<32>(K_, row_at, 0, s + AHEAD);
+      x = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[s], qf[s], x, 0, 0, 0);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    if (more) load_keys(next, K_);   // the key fragments are in registers
+    if (capped) {
+      float far = 0.0f;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) far = fmaxf(far, fabsf(x[i]));
+      // tanh(y) = y P(y^2) for |y| <= 1/2, P a polynomial through the Chebyshev nodes (1.3e-8 off); beyond, the exponential
+      // form, for the scores that are large themselves
+      if (__all(far * inv_cap <= 0.5f)) {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          const float y = x[i] * inv_cap, z = y * y;
+          x[i] = cap2 * y * fmaf(z, fmaf(z, fmaf(z, fmaf(z, 0.017131345f, -0.052984238f), 0.13324751f), -0.33333069f), 1.0f);
+        }
+        asm volatile("" ::: "memory");
+      } else {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          const float y = x[i] * inv_cap, z = y * y;
+          const float small = cap2 * y * fmaf(z, fmaf(z, fmaf(z, fmaf(z, 0.017131345f, -0.052984238f), 0.13324751f), -0.33333069f), 1.0f);
+          const float large = cap2 - 2.0f * cap2 * __builtin_amdgcn_rcpf(__builtin_amdgcn_exp2f(fabsf(x[i]) * t2) + 1.0f);
+          x[i] = fabsf(y) <= 0.5f ? small : copysignf(large, y);
+        }
+      }
+    }
+    const float k1 = capped ? 1.0f : c1;
+    if (sloped) {
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        const int idx = t * 32 + (i & 3) + 8 * (i >> 2) + 4 * hf;
+        const int j = idx < n_keep ? idx : lo + (idx - n_keep);
+        x[i] = x[i] * k1 - sl2 * (float)(pos - j);
+      }
+    }
+    const float k2 = sloped ? 1.0f : k1;
+    if (t * 32 + 32 > total) {
+#pragma unroll
+      for (int i = 0; i < 16; ++i) x[i] = t * 32 + (i & 3) + 8 * (i >> 2) + 4 * hf < total ? x[i] : -INFINITY;
+    }
+    bf16x8_v phi[2], plo[2];
+    float psum;
+    for (bool raised = false;; raised = true) {
+      psum = 0.0f;
+#pragma unroll
+      for (int i = 0; i < 16; i += 2) {
+        const float p0 = __builtin_amdgcn_exp2f(fmaf(x[i], k2, -m_ref)), p1 = __builtin_amdgcn_exp2f(fmaf(x[i + 1], k2, -m_ref));
+        psum += p0 + p1;
+        const bf16x2_v hi = __builtin_convertvector(float2v{p0, p1}, bf16x2_v);
+        const unsigned bits = __builtin_bit_cast(unsigned, hi);
+        const bf16x2_v low = __builtin_convertvector(float2v{p0 - __builtin_bit_cast(float, bits << 16),
+                                                             p1 - __builtin_bit_cast(float, bits & 0xffff0000u)}, bf16x2_v);
+        phi[i >> 3][i & 7] = hi[0];
+        phi[i >> 3][(i & 7) + 1] = hi[1];
+        plo[i >> 3][i & 7] = low[0];
+        plo[i >> 3][(i & 7) + 1] = low[1];
+      }
+      if (raised || __all(!head || psum <= 4096.0f)) break;
+      float top = x[0];
+#pragma unroll
+      for (int i = 1; i < 16; ++i) top = fmaxf(top, x[i]);
+      top = fmaxf(top, __shfl_xor(top, 32));
+      const float m_new = fmaxf(m, top == -INFINITY ? -INFINITY : top * k2);
+      const float corr = m == -INFINITY ? 1.0f : __builtin_amdgcn_exp2f(m - m_new);   // nothing accumulated: nothing to rescale
+      l *= corr;
+#pragma unroll
+      for (int c = 0; c < VT; ++c)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) oacc[c][i] *= corr;
+      m = m_new;
+      m_ref = m_new == -INFINITY ? -3.0e38f : m_new;
+    }
+    l += psum;
+    if (more) loads_left<2 * KQ>();   // younger than this tile's values: the next keys
+    else loads_left<0>();
+#pragma unroll
+    for (int s2 = 0; s2 < 2; ++s2)
+#pragma unroll
+      for (int c = 0; c < VT; ++c) {
+        const bf16x8_v va = frag_born<32>(V_, col_at, 16 * s2, 32 * c);
+        oacc[c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va, phi[s2], oacc[c], 0, 0, 0);
+        oacc[c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va, plo[s2], oacc[c], 0, 0, 0);
+      }
+    __builtin_amdgcn_sched_barrier(0);
+    if (more) load_values(next, V_);
+  };
+
+  if (t < last) {
+    for (; t + GROUP_WAVES < last; t += GROUP_WAVES) {
+      const Rows next = lookup(t + GROUP_WAVES);
+      loads_left<2 * VT>();          // younger than this tile's keys: its values
+      tile(t, std::true_type(), next, keys, keys + KT);
+    }
+    loads_left<2 * VT>();
+    tile(t, std::false_type(), first, keys, keys + KT);
+  }
+  // The waves' states: [head][2 + Dv] in the wave's own tiles
+  constexpr int PS = 2 + Dv;
+  l += __shfl_xor(l, 32);
+  float* mine = reinterpret_cast<float*>(keys) + col * PS;
+  if (head) {
+    if (hf == 0) {
+      mine[0] = m;
+      mine[1] = l;
+    }
+#pragma unroll
+    for (int c = 0; c < VT; ++c)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) mine[2 + c * 32 + (i & 3) + 8 * (i >> 2) + 4 * hf] = oacc[c][i];
+  }
+  __syncthreads();
+  constexpr int WS = (KT + VTT) / 4;   // floats between the waves' states
+  const float* states = reinterpret_cast<const float*>(tiles);
+  for (int i = threadIdx.x; i < R * Dv; i += 64 * GROUP_WAVES) {
+    const int r = i / Dv, dv = i % Dv;
+    float top = -INFINITY;
+#pragma unroll
+    for (int w = 0; w < GROUP_WAVES; ++w) top = fmaxf(top, states[w * WS + r * PS]);
+    if (splits == 1 && sink_logits != nullptr) top = fmaxf(top, sink_logits[h0 + r] * LOG2E);
+    float ll = 0.0f, o = 0.0f;
+#pragma unroll
+    for (int w = 0; w < GROUP_WAVES; ++w) {
+      const float mw = states[w * WS + r * PS];
+      const float f = mw == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(mw - top);
+      ll += states[w * WS + r * PS + 1] * f;     // a wave without keys: 0 * 0
+      o += states[w * WS + r * PS + 2 + dv] * f;
+    }
+    if (splits > 1) {   // a part without keys has a maximum of -inf
+      float* state = ws + ((n * H + h0 + r) * splits + split) * (long)PS;
+      state[2 + dv] = o;
+      if (dv == 0) {
+        state[0] = top;
+        state[1] = ll;
+      }
+    } else {
+      if (sink_logits != nullptr) ll += __builtin_amdgcn_exp2f(sink_logits[h0 + r] * LOG2E - top);
+      else if (sink) ll += __builtin_amdgcn_exp2f(-top);   // the sink's score is 0
+      float c = 1.0f / ll;
+      if (gate != nullptr) c *= sigmoidf_(ldf(gate + n * gate_stride + h0 + r));
+      stf(out + (n * H + h0 + r) * (long)Dv + dv, o * c);
+    }
+  }
+}
+
+}  // namespace
+
+bool launch_group_attention(at::Tensor& out, const at::Tensor& q, const at::Tensor& kpool, const at::Tensor& vpool,
+                            const at::Tensor& block_tables, const at::Tensor& tok_seq, const at::Tensor& positions,
+                            const float* slopes, const c10::optional<at::Tensor>& gate, long gate_stride, double scale,
+                            int64_t window, int64_t keep_first, double softcap, bool sink, int page_shift, long vrow,
+                            long vhead, const ScalarExtras& x) {
+  const long N = q.size(0);
+  const int H = (int)q.size(1), D = (int)q.size(2), G = (int)kpool.size(2), Dv = (int)vpool.size(3), R = H / G;
+  if (!is_bf16(q) || x.dist_bias != nullptr || x.ksum != nullptr || x.cross_out != nullptr || x.key_fac != nullptr ||
+      x.out32 != nullptr || (D != 64 && D != 128) || (Dv != 64 && Dv != 128) || R > GROUP_HEADS)
+    return false;
+  auto al16 = [](const at::Tensor& t) { return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0; };
+  if (!al16(q) || !al16(kpool) || !al16(vpool) || q.stride(0) % 8 != 0 || vrow % 8 != 0 || vrow >= (1L << 30) ||
+      vhead % 8 != 0)
+    return false;
+  long keys = block_tables.size(1) << page_shift;           // most that a token can see
+  if (window > 0) keys = std::min<long>(keys, window + keep_first);
+  if (x.chunk > 0) keys = std::min<long>(keys, x.chunk);
+  // Up to a tile a wave the other form's shorter end wins (6 x 173, 16 heads on 4 of 64: 7.9 against 8.3 us); values that are the keys
+  // stay there as well, which reads each row once.
+  if (keys <= 32 * GROUP_WAVES || vpool.data_ptr() == kpool.data_ptr()) return false;
+  // Parts of the keys while there are fewer blocks than CUs and a part keeps more than 1024 keys: parts cost a merge, about 4 us. 4 x 16384
+  // (16 heads on 4 of 128): 276 us undivided, 49 with 8 parts, 38 with 16, 42 with 32; 16 x 1024: 16.8, 16.5 with two and 15.8
+  // with four, but 5 x 700 on 2: 10.6 undivided, 12.4 with two; 1 x 8192: 16.8 with 8, 17.4 with 16, 22.4 with 32.
+  int splits = 1;
+  while (N * G * splits * 2 <= 256 && keys > splits * 1024L && splits < WAVE) splits *= 2;
+  // page numbers of a part: of its keys, rounded up to whole tiles, of a page more for where they begin, and of the kept ones
+  const long part_keys = ((keys + 31) / 32 + splits - 1) / splits * 32;
+  const size_t lds = (size_t)GROUP_WAVES * (D + Dv) * 64 + (size_t)((part_keys >> page_shift) + (keep_first >> page_shift) + 4) * sizeof(int);
+  if (lds > GROUP_LDS) return false;
+  at::Tensor ws;
+  if (splits > 1) ws = at::empty({N * H * splits * (2 + Dv)}, q.options().dtype(at::kFloat));
+#define GROUP_LAUNCH(DS_, VT_)                                                                                       \
+  do {                                                                                                             \
+    auto kernel = group_attention_kernel<DS_, VT_>;                                                                \
+    if (lds > 65536) (void)hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds); \
+    hipLaunchKernelGGL(kernel, dim3((unsigned)(N * G * splits)), dim3(64 * GROUP_WAVES), lds, stream(), ptr<bf16s>(out), \
+                       ptr<bf16s>(q), (long)q.stride(0), ptr<bf16s>(kpool), ptr<bf16s>(vpool), block_tables.data_ptr<int>(), \
+                       (int)block_tables.stride(0), tok_seq.data_ptr<int>(), positions.data_ptr<int>(), slopes,    \
+                       gate.has_value() ? ptr<bf16s>(*gate) : (const bf16s*)nullptr, gate_stride, x.sink_logits, H, G, page_shift, \
+                       (float)scale, (int)window, (int)keep_first, x.chunk, (float)softcap, sink ? 1 : 0, x.vrep, vrow, vhead, \
+                       splits, splits > 1 ? ws.data_ptr<float>() : (float*)nullptr);                              \
+  } while (0)
+  if (D == 128) { if (Dv == 128) GROUP_LAUNCH(8, 4); else GROUP_LAUNCH(8, 2); }
+  else { if (Dv == 128) GROUP_LAUNCH(4, 4); else GROUP_LAUNCH(4, 2); }
+#undef GROUP_LAUNCH
+  HIP_CHECK_LAST();
+  if (splits > 1) launch_row_merge(out, q, ws, gate, gate_stride, x, Dv, sink, splits);
+  return true;
+}
+
+}  // namespace serving
+}  // namespace cai

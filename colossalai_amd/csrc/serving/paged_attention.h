@@ -41,5 +41,16 @@ bool launch_row_attention(at::Tensor& out, const at::Tensor& q, const at::Tensor
                           int64_t window, int64_t keep_first, double softcap, bool sink, int page_shift, long vrow,
                           long vhead, const ScalarExtras& x);
 
+// The form for bfloat16 decode tokens on the matrix cores (group_attention.hip); false when the shape or the options are not its.
+bool launch_group_attention(at::Tensor& out, const at::Tensor& q, const at::Tensor& kpool, const at::Tensor& vpool,
+                            const at::Tensor& block_tables, const at::Tensor& tok_seq, const at::Tensor& positions,
+                            const float* slopes, const c10::optional<at::Tensor>& gate, long gate_stride, double scale,
+                            int64_t window, int64_t keep_first, double softcap, bool sink, int page_shift, long vrow,
+                            long vhead, const ScalarExtras& x);
+
+// The states of `splits` parts of each (token, head)'s keys in `ws` -> `out`, or x.out32; q gives the type of the call (row_attention.hip).
+void launch_row_merge(at::Tensor& out, const at::Tensor& q, const at::Tensor& ws, const c10::optional<at::Tensor>& gate,
+                      long gate_stride, const ScalarExtras& x, int Dv, bool sink, int splits);
+
 }  // namespace serving
 }  // namespace cai

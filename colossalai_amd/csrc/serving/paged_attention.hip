@@ -813,6 +813,9 @@ static void launch_scalar_attention(at::Tensor& out, const at::Tensor& q, const 
   const long N = q.size(0);
   const int H = (int)q.size(1), D = (int)q.size(2);
   const int G = (int)kpool.size(2), Dv = (int)vpool.size(3);
+  if (launch_group_attention(out, q, kpool, vpool, block_tables, tok_seq, positions, slp, gate, gstride, scale, window,
+                             keep_first, softcap, sink, page_shift, vrow, vhead, x))
+    return;
   if (launch_row_attention(out, q, kpool, vpool, block_tables, tok_seq, positions, slp, gate, gstride, scale, window,
                            keep_first, softcap, sink, page_shift, vrow, vhead, x))
     return;

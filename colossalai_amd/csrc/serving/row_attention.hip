@@ -12,9 +12,10 @@
 // have their keys cut into parts, one block each, whose states row_merge_kernel puts together.
 //
 // What bounds it: the chain of dependent loads (position, page table, rows) and the block's end, about 10 us
-// together, and beyond that the vector instructions of the products. 16 x 1024 keys of 16/4 heads of 128 with a cap and a sink
-// take 17.8 us (29.3 before the base-2 scores and the halving butterfly), 1.9 TB/s; 4 x 16384 take 51.5 us (242 with one
-// block per token, kv head and head), 40 of it the parts at 3.4 TB/s and 7 the merge.
+// together, and beyond that the vector instructions of the products. bfloat16 calls of common sizes go to
+// group_attention.hip; here are float32, shared key/value rows, key factors, float32 output and the other sizes. 16 x 1024
+// keys of 16/4 heads of 128 with a cap and a sink took 17.8 us (29.3 before the base-2 scores and the halving butterfly), 1.9
+// TB/s; 4 x 16384 took 51.5 us (242 with one block per token, kv head and head), 40 of it the parts at 3.4 TB/s and 7 the merge.
 #include "paged_attention.h"
 
 #include <algorithm>
@@ -371,12 +372,34 @@ __global__ __launch_bounds__(256) void row_merge_kernel(
   else if (sink) ll += Dom<T>::exp_(-top);   // the sink's score is 0
   float c = f / ll;
   if (gate != nullptr) c *= sigmoidf_(ldf(gate + row / H * gate_stride + h));
+  // eight parts' loads at a time: one by one, 16 parts took 7.3 us
   for (int dv = lane; dv < Dv; dv += 64) {
     float o = 0.0f;
-    for (int p = 0; p < splits; ++p) o += __shfl(c, p) * state[p * (long)(2 + Dv) + 2 + dv];
+    for (int p0 = 0; p0 < splits; p0 += 8) {
+      float v[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[e] = state[min(p0 + e, splits - 1) * (long)(2 + Dv) + 2 + dv];
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+        if (p0 + e < splits)
+          o += __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, c), p0 + e)) * v[e];
+    }
     if (out32 != nullptr) out32[row * (long)Dv + dv] = o;
     else stf(out + row * (long)Dv + dv, o);
   }
+}
+
+void launch_row_merge(at::Tensor& out, const at::Tensor& q, const at::Tensor& ws, const c10::optional<at::Tensor>& gate,
+                      long gate_stride, const ScalarExtras& x, int Dv, bool sink, int splits) {
+  const long rows = q.size(0) * q.size(1);
+  TORCH_CHECK(splits <= MAX_PARTS, "more parts of the keys than the merge takes");
+  SERVING_DISPATCH_ACT(q, T, {
+    hipLaunchKernelGGL((row_merge_kernel<T>), dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, stream(),
+                       x.out32 != nullptr ? (T*)nullptr : ptr<T>(out), x.out32, ws.data_ptr<float>(),
+                       gate.has_value() ? ptr<T>(*gate) : (const T*)nullptr, gate_stride, x.sink_logits, rows, (int)q.size(1),
+                       Dv, sink ? 1 : 0, splits);
+  });
+  HIP_CHECK_LAST();
 }
 
 bool launch_row_attention(at::Tensor& out, const at::Tensor& q, const at::Tensor& kpool, const at::Tensor& vpool,
@@ -438,17 +461,10 @@ bool launch_row_attention(at::Tensor& out, const at::Tensor& q, const at::Tensor
       if (rc == 1) ROW_LAUNCH(1, 8, true);
       else ROW_LAUNCH(2, 4, true);
     }
-    if (splits > 1) {
-      HIP_CHECK_LAST();
-      TORCH_CHECK(splits <= MAX_PARTS, "more parts of the keys than the merge takes");
-      hipLaunchKernelGGL((row_merge_kernel<T>), dim3((unsigned)((N * H + 3) / 4)), dim3(256), 0, stream(),
-                         x.out32 != nullptr ? (T*)nullptr : ptr<T>(out), x.out32, ws.data_ptr<float>(),
-                         gate.has_value() ? ptr<T>(*gate) : (const T*)nullptr, gate_stride, x.sink_logits, N * H, H, Dv,
-                         sink ? 1 : 0, splits);
-    }
   });
 #undef ROW_LAUNCH
   HIP_CHECK_LAST();
+  if (splits > 1) launch_row_merge(out, q, ws, gate, gate_stride, x, Dv, sink, splits);
   return true;
 }
 

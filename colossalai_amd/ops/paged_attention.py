@@ -211,23 +211,24 @@ def paged_attention(q, kpool, vpool, batch: RaggedBatch, scale: float, window: i
     assert out_dtype in (None, q.dtype, torch.float32)
     plain = chunk == 0 and key_factors is None and kpool.shape[2] == vpool.shape[2] and out_dtype in (None, q.dtype)
     assert plain or (pooled is None and talk is None)
-    if use_hip(q) and not (plain and sink_logits is None and dist_bias is None and pooled is None and talk is None):
+    hip = use_hip(q)
+    if hip:
+        tiles32, tiles64, tiles128 = batch.tile_counts()
+    if hip and not (plain and sink_logits is None and dist_bias is None and pooled is None and talk is None):
         # With talking heads the kernels hand back every query head's weights applied to every key/value head's
         # values, O[n, g, c] (float32): the mix is linear, so out[n, h] = sum_g talk[h, g] O[n, g, kv(h)]
         ksum, vsum, block = pooled if pooled is not None else (None, None, 0)
         o = serving_kernels().paged_attention_ext(q, kpool, vpool, batch.block_tables, batch.cu, batch.start,
                                                   batch.tok_seq, batch.positions, scale, window, keep_first, slopes,
                                                   gate, float(softcap), bool(sink), sink_logits, dist_bias, ksum, vsum,
-                                                  int(block), talk is not None, batch.num_tiles32, batch.num_tiles128,
-                                                  batch.num_tiles64, int(chunk), key_factors,
+                                                  int(block), talk is not None, tiles32, tiles128, tiles64, int(chunk), key_factors,
                                                   out_dtype == torch.float32)
         if talk is None:
             return o
         return serving_kernels().talk_mix(o, talk, q.dtype)
-    if use_hip(q):
+    if hip:
         return serving_kernels().paged_attention(q, kpool, vpool, batch.block_tables, batch.cu, batch.start,
                                                  batch.tok_seq, batch.positions, scale, window, keep_first,
-                                                 slopes, gate, batch.num_tiles32, float(softcap), bool(sink),
-                                                 batch.num_tiles128, batch.num_tiles64)
+                                                 slopes, gate, tiles32, float(softcap), bool(sink), tiles128, tiles64)
     return paged_attention_ref(q, kpool, vpool, batch, scale, window, keep_first, slopes, gate, softcap, sink,
                                sink_logits, dist_bias, pooled, talk, chunk, key_factors, out_dtype)

@@ -47,28 +47,26 @@ class RaggedBatch:
     def max_new(self) -> int:
         return max(self.cu_host[i + 1] - self.cu_host[i] for i in range(self.num_seqs))
 
-    def _tiles(self, tokens: int) -> int:
-        if self.max_new == 1:
-            return 0
-        return sum((self.cu_host[i + 1] - self.cu_host[i] + tokens - 1) // tokens for i in range(self.num_seqs))
+    def tile_counts(self):
+        """Tiles of 32, 64 and 128 tokens of the prompt portions (all 0 for a pure decode step): the grids of the matrix-core
+        attention kernel when every key head has three or more, two or a single query head."""
+        cu = self.cu_host
+        if cu[-1] == len(cu) - 1 and self.max_new == 1:
+            return 0, 0, 0
+        new = [b - a for a, b in zip(cu, cu[1:])]
+        return sum((n + 31) // 32 for n in new), sum((n + 63) // 64 for n in new), sum((n + 127) // 128 for n in new)
 
     @property
     def num_tiles32(self) -> int:
         """32-token tiles of the prompt portions (0 for a pure decode step):
         the grid of the matrix-core attention kernel."""
-        return self._tiles(32)
-
-    @property
-    def num_tiles64(self) -> int:
-        """64-token tiles of the prompt portions (0 for a pure decode step): the grid of the matrix-core attention
-        kernel when every key head has two query heads."""
-        return self._tiles(64)
+        return self.tile_counts()[0]
 
     @property
     def num_tiles128(self) -> int:
         """128-token tiles of the prompt portions (0 for a pure decode step): the grid of the matrix-core attention
         kernel when every key head has a single query head."""
-        return self._tiles(128)
+        return self.tile_counts()[2]
 
     @property
     def max_total(self) -> int:

@@ -236,3 +236,32 @@ def test_pools_at_an_odd_address(which):
     odd = torch.empty(t.numel() + 1, device="cuda", dtype=t.dtype)[1:].view(t.shape).copy_(t)
     got = paged_attention(q, odd if which == "keys" else k, odd if which == "values" else v, batch, 0.1)
     assert (got.double() - want.double()).norm() / want.double().norm() < 2 * BOUND
+
+
+# Decode tokens: groups of 1 to 16 query heads (17: another kernel), key and value sizes that differ, last tiles of one key and of 32,
+# windows and blocks that begin inside a page and a tile, kept keys that end in the middle of a page.
+@pytest.mark.parametrize("H,G,D,Dv", [(2, 2, 128, 128), (6, 2, 64, 128), (16, 1, 128, 64), (17, 1, 64, 64), (10, 2, 64, 64)])
+@pytest.mark.parametrize("page", [16, 64])
+@pytest.mark.parametrize("kw", [{}, dict(softcap=5.0), dict(sink_logits=True, gate=True), dict(chunk=1000),
+                                dict(slopes=True, window=333, keep_first=37), dict(window=2300, keep_first=5, sink=True)])
+def test_decode_of_head_counts_and_sizes(H, G, D, Dv, page, kw):
+    _check([1] * 7, [0, 30, 31, 32, 340, 1999, 4100], H, G, D, Dv, page, 0.1, **dict(kw))
+
+
+@pytest.mark.parametrize("levels", [(0, 9, 18, 27, 36, 45), (60, 40, 20, 0, -20, -40), (-3000, 0, -3000, 4, 8, 1000)])
+@pytest.mark.parametrize("parts", [False, True])
+def test_decode_scores_that_rise_and_fall(levels, parts):
+    """Levels (in nats) of 256 or 2048 keys each: inside a wave's tiles, and from part to part."""
+    from colossalai_amd.ops.paged_attention import paged_attention, paged_attention_ref
+
+    torch.manual_seed(8)
+    each, scale = 2048 if parts else 256, 128 ** -0.5
+    batch, pages = _batch([1, 1], [each * len(levels) - 1, 100], 64)
+    k, v = (torch.randn(pages, 64, 2, 128, device="cuda").bfloat16() for _ in range(2))
+    q = torch.randn(2, 8, 128, device="cuda").bfloat16()
+    q[..., 0] = 8.0
+    for i, level in enumerate(levels):
+        k[batch.block_tables[0, i * each // 64: (i + 1) * each // 64].long(), :, :, 0] = level / (8.0 * scale)
+    got = paged_attention(q, k, v, batch, scale)
+    want = paged_attention_ref(q.float(), k.float(), v.float(), batch, scale)
+    assert (got.double() - want.double()).norm() / want.double().norm() < BOUND
