@@ -35,6 +35,12 @@ void ce_fwd(at::Tensor logits, at::Tensor labels, int64_t ignore_index, at::Tens
 void ce_bwd(at::Tensor logits, at::Tensor labels, int64_t ignore_index, at::Tensor lse, at::Tensor grad, at::Tensor loss);
 at::Tensor ce_loss(at::Tensor nll, at::Tensor labels, int64_t ignore_index);
 
+// weight_grad.hip
+at::Tensor weight_grad(const at::Tensor& dy, const at::Tensor& x, const c10::optional<at::Tensor>& add, bool keep);
+
+// linear.cpp
+at::Tensor linear(const at::Tensor& x, const at::Tensor& weight);
+
 // layernorm.hip
 std::vector<at::Tensor> layernorm_fwd(at::Tensor input, at::Tensor gamma, c10::optional<at::Tensor> beta,
                                       double eps, bool save_stats);
@@ -111,6 +117,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("ce_fwd", &cai::ce_fwd, "cross entropy of bf16 logits: log-sum-exp and negative log likelihood per row");
   m.def("ce_bwd", &cai::ce_bwd, "cross entropy backward, logits -> their gradient in place");
   m.def("ce_loss", &cai::ce_loss, "mean negative log likelihood over the rows that are not ignored, and their number");
+  m.def("weight_grad", &cai::weight_grad, "dy [K, M], x [K, N] -> dy^T x (+ add) in bf16, or in float32 with keep",
+        py::arg("dy"), py::arg("x"), py::arg("add") = py::none(), py::arg("keep") = false);
+  m.def("linear", &cai::linear, "linear layer without bias, its weight gradient by weight_grad");
   m.def("layernorm_fwd", &cai::layernorm_fwd, "LayerNorm forward");
   m.def("layernorm_bwd", &cai::layernorm_bwd, "LayerNorm backward");
   m.def("rope_inplace", &cai::rope_inplace, "in-place rotary embedding (fwd/bwd)");

@@ -1,0 +1,52 @@
+// Linear layers without a bias whose weight gradient is csrc/weight_grad.hip's; the other two products are the library's.
+#include <ATen/TensorSubclassLikeUtils.h>
+#include <ATen/autocast_mode.h>
+#include <torch/csrc/jit/frontend/tracer.h>
+#include <torch/extension.h>
+
+namespace cai {
+
+at::Tensor weight_grad(const at::Tensor& dy, const at::Tensor& x, const c10::optional<at::Tensor>& add, bool keep);
+bool weight_grad_serves(const at::Tensor& dy, const at::Tensor& x);
+
+namespace {
+
+// nothing that watches or rewrites single operations stands between these tensors and a kernel
+bool plain(const at::Tensor& t) {
+  return !at::isTensorSubclassLike(t) && !at::autocast::is_autocast_enabled(at::kCUDA) && !torch::jit::tracer::isTracing()
+      && !c10::impl::tls_is_dispatch_key_included(at::DispatchKey::FuncTorchDynamicLayerFrontMode);
+}
+
+bool has_tangent(const at::Tensor& t) { return t._fw_grad(0).defined(); }
+
+struct Linear : torch::autograd::Function<Linear> {
+  static at::Tensor forward(torch::autograd::AutogradContext* ctx, const at::Tensor& x, const at::Tensor& weight) {
+    // as the built-in layer: each gradient's factor is kept only if that gradient is wanted
+    ctx->save_for_backward({x, x.requires_grad() ? weight : at::Tensor()});
+    return at::linear(x, weight);
+  }
+  static torch::autograd::variable_list backward(torch::autograd::AutogradContext* ctx, torch::autograd::variable_list grads) {
+    const auto saved = ctx->get_saved_variables();
+    const at::Tensor &x = saved[0], &weight = saved[1], &dy = grads[0];
+    if (!dy.defined()) return {at::Tensor(), at::Tensor()};
+    const at::Tensor dy2 = dy.reshape({-1, dy.size(-1)});
+    at::Tensor dx, dw;
+    if (ctx->needs_input_grad(0)) dx = at::mm(dy2, weight).view(x.sizes());
+    if (ctx->needs_input_grad(1)) {
+      const at::Tensor x2 = x.reshape({-1, x.size(-1)});
+      // a backward that is part of a graph itself (create_graph), or that something watches, takes operations it can see
+      if (!at::GradMode::is_enabled() && plain(dy2) && plain(x2) && weight_grad_serves(dy2, x2)) dw = weight_grad(dy2, x2, c10::nullopt, false);
+      else dw = at::mm(dy2.t(), x2);
+    }
+    return {dx, dw};
+  }
+};
+
+}  // namespace
+
+at::Tensor linear(const at::Tensor& x, const at::Tensor& weight) {
+  if (x.dim() < 2 || x.numel() == 0 || !plain(x) || !plain(weight) || has_tangent(x) || has_tangent(weight)) return at::linear(x, weight);
+  return Linear::apply(x, weight);
+}
+
+}  // namespace cai

@@ -26,6 +26,7 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from ..ops import build_rope_table, fused_add_rms_norm, fused_rope_attention, rms_norm, swiglu
+from ..ops.linear import project
 
 from .registry import register_model
 
@@ -142,7 +143,7 @@ class LlamaAttention(nn.Module):
                 seqlens: Optional[torch.Tensor] = None,
                 cu_seqlens: Optional[torch.Tensor] = None) -> torch.Tensor:
         B, S, _ = hidden.shape
-        qkv = self.qkv_proj(hidden)
+        qkv = project(self.qkv_proj, hidden)
         sp_mode = getattr(self, "sp_mode", None)
         if cu_seqlens is not None:
             # packed ragged batch ([1, total, ...]): per-sequence RoPE
@@ -162,7 +163,7 @@ class LlamaAttention(nn.Module):
             q, k = apply_rope(q, k, rope_table, positions)
             attn = flash_attention_varlen(q[0], k[0], v[0].contiguous(), cu_seqlens,
                                           causal=True, scale=self.scale)
-            return self.o_proj(attn.reshape(B, S, Hq * D))
+            return project(self.o_proj, attn.reshape(B, S, Hq * D))
         if sp_mode is not None:
             assert not self.qk_norm and self.pir_factor == 0, (
                 "qk-norm / partial-rotary variants are not wired into the SP "
@@ -197,7 +198,7 @@ class LlamaAttention(nn.Module):
             q, k = apply_rope(q, k, rope_table, positions)
             attn = ring_flash_attention(q, k, v, sp_group, causal=True, scale=self.scale,
                                         zigzag=zigzag, seqlens=seqlens)
-            return self.o_proj(attn.reshape(B, S, -1))
+            return project(self.o_proj, attn.reshape(B, S, -1))
         if sp_mode == "all_to_all":
             # Ulysses: scatter heads / gather sequence around attention
             import torch.distributed as dist
@@ -217,7 +218,7 @@ class LlamaAttention(nn.Module):
             q, k = apply_rope(q.contiguous(), k.contiguous(), rope_table)
             attn = flash_attention(q, k, v.contiguous(), causal=True, scale=self.scale)
             attn = all_to_all_comm(attn, sp_group, scatter_dim=1, gather_dim=2)  # back to [B, S, Hq, D]
-            return self.o_proj(attn.reshape(B, S, -1))
+            return project(self.o_proj, attn.reshape(B, S, -1))
         if self.pir_factor > 0:
             # GLM-4: partial interleaved rotary — unpack, rope, flash
             from ..ops import flash_attention
@@ -236,7 +237,7 @@ class LlamaAttention(nn.Module):
                 from ..ops.attention import attention_ref
 
                 attn = attention_ref(q, k, v, causal=True, scale=self.scale, upcast=False)
-            return self.o_proj(attn.reshape(B, S, Hq * D))
+            return project(self.o_proj, attn.reshape(B, S, Hq * D))
         if self.qk_norm:
             # Qwen3: per-head RMSNorm on q/k before RoPE — unpack, norm,
             # rope, flash (the packed fused path skips the norm)
@@ -250,14 +251,14 @@ class LlamaAttention(nn.Module):
             v = qkv[:, :, (Hq + Hkv) * D :].reshape(B, S, Hkv, D)
             q, k = apply_rope(q.contiguous(), k.contiguous(), rope_table)
             attn = flash_attention(q, k, v.contiguous(), causal=True, scale=self.scale, seqlens=seqlens)
-            return self.o_proj(attn.reshape(B, S, Hq * D))
+            return project(self.o_proj, attn.reshape(B, S, Hq * D))
         attn = fused_rope_attention(
             qkv, rope_table, self.num_heads, self.num_kv_heads, self.head_dim,
             causal=True, scale=self.scale, seqlens=seqlens,
         )
         # under split_gather SP the column-linear gathered the sequence, so
         # flatten with the attention output's own length, not the input's
-        return self.o_proj(attn.reshape(B, attn.shape[1], -1))
+        return project(self.o_proj, attn.reshape(B, attn.shape[1], -1))
 
     @torch.no_grad()
     def forward_with_cache(self, hidden, rope_table, kcache, vcache, positions, seq_lens, prefill: bool):
@@ -390,7 +391,7 @@ class LlamaMLP(nn.Module):
         self.down_proj = nn.Linear(cfg.intermediate_size, cfg.hidden_size, bias=False)
 
     def forward(self, hidden: torch.Tensor) -> torch.Tensor:
-        return self.down_proj(swiglu(self.gate_up_proj(hidden)))
+        return project(self.down_proj, swiglu(project(self.gate_up_proj, hidden)))
 
 
 class LlamaDecoderLayer(nn.Module):

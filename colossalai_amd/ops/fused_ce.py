@@ -6,7 +6,8 @@ chunk's logits and feeds the dW/dh GEMMs directly. At the flagship bench
 size (147k tokens x 32k vocab) this replaces a ~50 GB fp32 logits+softmax
 footprint with ~1 GB of transient chunk buffers — pure HBM savings.
 
-GEMMs run through hipBLASLt (torch.matmul); softmax math is fp32. In bfloat16 on
+GEMMs run through hipBLASLt (torch.matmul), the weight gradient in bfloat16 through
+csrc/weight_grad.hip; softmax math is fp32. In bfloat16 on
 the GPU a chunk's logits are read once in the forward and overwritten by their
 gradient in the backward (csrc/cross_entropy.hip).
 Reference parity: the reference materializes logits and uses torch CE (or
@@ -104,12 +105,8 @@ def _backward_hip(ctx, grad_out):
         ds = hidden[s:e] @ weight.t()
         kernels().ce_bwd(ds, labels[s:e], ctx.ignore_index, lse[s:e], grad, loss)
         torch.mm(ds, weight, out=dh[s:e])
-        part = ds.t() @ hidden[s:e]
-        # chunks are summed in float32; a single chunk's product is the sum already
-        if dw is None:
-            dw = part if e == N else part.float()
-        else:
-            dw += part
+        # chunks are summed in float32, by the product itself
+        dw = kernels().weight_grad(ds, hidden[s:e], dw, e < N)
     if dw is None:
         dw = torch.zeros_like(weight)
     return dh, dw.to(weight.dtype), None, None, None

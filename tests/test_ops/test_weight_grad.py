@@ -1,0 +1,129 @@
+"""Weight gradients of linear layers (csrc/weight_grad.hip) and the layer that uses them (csrc/linear.cpp)."""
+
+import pytest
+import torch
+import torch.nn as nn
+import torch.nn.functional as F
+
+from colossalai_amd.ops._kernels import has_kernels, kernels
+from colossalai_amd.ops.linear import project
+
+BF16 = torch.bfloat16
+needs_extension = pytest.mark.skipif(not has_kernels(), reason="extension not built")
+
+
+def _close(got, dy, x, add=None, keep=False):
+    """Within a rounding of the result's type and the float32 sums of K products, in any order."""
+    a, b = dy.double(), x.double()
+    ref, size = a.t() @ b, a.abs().t() @ b.abs()
+    if add is not None:
+        ref, size = ref + add.double(), size + add.double().abs()
+    limit = size * (dy.shape[0] + 2) * 2.0 ** -24 + (0 if keep else ref.abs() * 2.0 ** -8) + 1e-30
+    assert got.dtype == (torch.float32 if keep else BF16)
+    assert ((got.double() - ref).abs() <= limit).all()
+
+
+# edges of both tile sizes, of the steps of 32 tokens and of the parts
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(8, 8, 1), (128, 136, 31), (120, 256, 33), (264, 248, 300), (768, 768, 4100), (1032, 776, 1500),
+                                   (512, 512, 512), (4096, 4104, 65), (8, 2048, 16384), (5120, 4096, 1000)])
+def test_against_64_bits(M, N, K):
+    torch.manual_seed(M + N + K)
+    dy, x = (torch.randn(K, n, device="cuda").to(BF16) for n in (M, N))
+    _close(kernels().weight_grad(dy, x), dy, x)
+    first = kernels().weight_grad(dy, x, None, True)
+    _close(first, dy, x, None, True)
+    add = torch.randn(M, N, device="cuda")
+    before = add.clone()
+    _close(kernels().weight_grad(dy, x, add, False), dy, x, before)
+    again = kernels().weight_grad(dy, x, add, True)
+    assert again.data_ptr() == add.data_ptr()
+    _close(again, dy, x, before, True)
+
+
+@pytest.mark.gpu
+def test_strides_and_sizes_of_other_forms():
+    torch.manual_seed(0)
+    wide = torch.randn(300, 1000, device="cuda").to(BF16)
+    x = torch.randn(300, 264, device="cuda").to(BF16)
+    forms = [wide[:, 8:272], wide[:, 3:267], wide.t()[:300, :264], wide[:1, :264].expand(300, 264), wide[:, :250], wide[::2, :264]]
+    for dy in forms:
+        for a, b in ((dy, x[: dy.shape[0]]), (x[: dy.shape[0]], dy)):
+            _close(kernels().weight_grad(a, b), a, b)
+
+
+@pytest.mark.gpu
+def test_what_is_not_finite_stays_in_its_row():
+    dy, x = torch.ones(100, 264, device="cuda", dtype=BF16), torch.ones(100, 136, device="cuda", dtype=BF16)
+    dy[99, 7], x[0, 135] = float("nan"), float("inf")
+    got = kernels().weight_grad(dy, x)
+    rows = torch.arange(264, device="cuda") != 7
+    assert got[7].isnan().all() and (got[rows][:, 135] == float("inf")).all() and (got[rows][:, :135] == 100).all()
+
+
+def _step(call, x, w, g):
+    x, w = x.detach().requires_grad_(), w.detach().requires_grad_()
+    y = call(x, w)
+    y.backward(g)
+    return y.detach(), x.grad, w.grad
+
+
+@needs_extension
+@pytest.mark.parametrize("shape", [(5, 16), (2, 3, 16), (2, 2, 3, 16)])
+def test_layer_is_the_builtin_one_on_the_cpu(shape):
+    torch.manual_seed(1)
+    x, w, g = torch.randn(*shape), torch.randn(24, 16), torch.randn(*shape[:-1], 24)
+    for a, b in zip(_step(kernels().linear, x, w, g), _step(F.linear, x, w, g)):
+        torch.testing.assert_close(a, b)
+
+
+@needs_extension
+def test_layer_under_transforms():
+    torch.manual_seed(2)
+    x, w = torch.randn(4, 16, dtype=torch.float64), torch.randn(8, 16, dtype=torch.float64)
+    lin = kernels().linear
+    assert torch.autograd.gradcheck(lin, (x.requires_grad_(), w.requires_grad_()))
+    assert torch.autograd.gradgradcheck(lin, (x, w))
+    x, w = x.detach(), w.detach()
+    torch.testing.assert_close(torch.func.vmap(lin, (0, None))(x.expand(3, 4, 16), w), F.linear(x.expand(3, 4, 16), w))
+    torch.testing.assert_close(torch.func.jacrev(lin, 1)(x, w), torch.func.jacrev(F.linear, 1)(x, w))
+    torch.testing.assert_close(torch.func.jvp(lambda t: lin(t, w), (x,), (x,)), torch.func.jvp(lambda t: F.linear(t, w), (x,), (x,)))
+    with torch.autograd.forward_ad.dual_level():
+        d = torch.autograd.forward_ad.make_dual(x, x)
+        assert torch.autograd.forward_ad.unpack_dual(lin(d, w.requires_grad_())).tangent is not None
+    w, kept = w.detach().requires_grad_(), []
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: kept.append(t) or t, lambda t: t):
+        y = lin(x, w)
+    assert len(kept) == 1   # the input; the weight's own factor is not wanted
+    torch.testing.assert_close(torch.autograd.grad(y, w, torch.ones(3, 4, 8, dtype=torch.float64), is_grads_batched=True)[0],
+                               x.sum(0).expand(3, 8, 16))
+
+
+@pytest.mark.gpu
+def test_projection_takes_the_native_form_only_for_plain_layers():
+    torch.manual_seed(3)
+    layer = nn.Linear(264, 136, bias=False, device="cuda", dtype=BF16)
+    x = torch.randn(2, 50, 264, device="cuda").to(BF16).requires_grad_()
+    seen = []
+
+    assert "CppNode" in project(layer, x).grad_fn.name()
+    handle = layer.register_forward_hook(lambda *a: seen.append(1))
+    project(layer, x)
+    handle.remove()
+    assert seen == [1]
+    layer.forward = lambda t: seen.append(2) or F.linear(t, layer.weight)
+    project(layer, x)
+    del layer.forward
+    assert seen == [1, 2]
+    with torch.autocast("cuda", torch.float16):
+        assert project(layer, x).dtype == torch.float16
+    y, g = project(layer, x), torch.randn(2, 50, 136, device="cuda").to(BF16)
+    got = torch.autograd.grad(y, (x, layer.weight), g)
+    ref = torch.autograd.grad(layer(x), (x, layer.weight), g)
+    torch.testing.assert_close(got[0], ref[0], rtol=0, atol=0)
+    _close(got[1], g.view(-1, 136), x.detach().view(-1, 264))
+    graph = torch.autograd.grad(project(layer, x), layer.weight, g, create_graph=True)[0]
+    assert graph.requires_grad
+    layer.weight.requires_grad_(False)
+    project(layer, x).backward(g)
+    assert layer.weight.grad is None and x.grad is not None
