@@ -19,6 +19,7 @@ from typing import Optional
 import torch
 
 from ._kernels import kernels, use_hip
+from .linear import weight_grad
 
 __all__ = ["fused_linear_cross_entropy"]
 
@@ -106,7 +107,7 @@ def _backward_hip(ctx, grad_out):
         kernels().ce_bwd(ds, labels[s:e], ctx.ignore_index, lse[s:e], grad, loss)
         torch.mm(ds, weight, out=dh[s:e])
         # chunks are summed in float32, by the product itself
-        dw = kernels().weight_grad(ds, hidden[s:e], dw, e < N)
+        dw = weight_grad(ds, hidden[s:e], dw, e < N)
     if dw is None:
         dw = torch.zeros_like(weight)
     return dh, dw.to(weight.dtype), None, None, None

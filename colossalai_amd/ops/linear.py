@@ -4,13 +4,25 @@ The layer stays an ``nn.Linear`` that parallel policies, LoRA or the zero-bubble
 calls whatever it has become.
 """
 
+from typing import Optional
+
 import torch
 import torch.nn as nn
 from torch.nn.modules import module as _hooks
 
 from ._kernels import kernels
 
-__all__ = ["project"]
+__all__ = ["project", "weight_grad"]
+
+
+def weight_grad(dy: torch.Tensor, x: torch.Tensor, add: Optional[torch.Tensor] = None, keep: bool = False) -> torch.Tensor:
+    """dy [K, M], x [K, N] -> dy^T x (+ ``add``, float32) in their type, or in float32 with ``keep``: then in ``add`` if given."""
+    if dy.is_cuda:
+        return kernels().weight_grad(dy, x, add, keep)
+    part = dy.t() @ x
+    if add is not None:
+        part = add.add_(part) if keep else add + part
+    return part.to(torch.float32 if keep else dy.dtype)
 
 
 def _bare(layer: nn.Module) -> bool:
