@@ -32,7 +32,8 @@ std::vector<at::Tensor> rmsnorm_bwd(at::Tensor dy, at::Tensor x, at::Tensor weig
 
 // cross_entropy.hip
 void ce_fwd(at::Tensor logits, at::Tensor labels, int64_t ignore_index, at::Tensor lse, at::Tensor nll);
-void ce_bwd(at::Tensor logits, at::Tensor labels, int64_t ignore_index, at::Tensor lse, at::Tensor grad, at::Tensor loss);
+void ce_bwd(at::Tensor logits, at::Tensor labels, int64_t ignore_index, at::Tensor lse, at::Tensor grad, at::Tensor loss,
+            c10::optional<at::Tensor> into);
 at::Tensor ce_loss(at::Tensor nll, at::Tensor labels, int64_t ignore_index);
 
 // weight_grad.hip
@@ -115,7 +116,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("rmsnorm_bwd", &cai::rmsnorm_bwd, "RMSNorm backward", py::arg("dy"), py::arg("x"), py::arg("weight"),
         py::arg("inv_rms"), py::arg("dres") = py::none(), py::arg("cast_dw") = false);
   m.def("ce_fwd", &cai::ce_fwd, "cross entropy of bf16 logits: log-sum-exp and negative log likelihood per row");
-  m.def("ce_bwd", &cai::ce_bwd, "cross entropy backward, logits -> their gradient in place");
+  m.def("ce_bwd", &cai::ce_bwd, "cross entropy backward, logits -> their gradient, in place or in `into`", py::arg("logits"),
+        py::arg("labels"), py::arg("ignore_index"), py::arg("lse"), py::arg("grad"), py::arg("loss"), py::arg("into") = py::none());
   m.def("ce_loss", &cai::ce_loss, "mean negative log likelihood over the rows that are not ignored, and their number");
   m.def("weight_grad", &cai::weight_grad, "dy [K, M], x [K, N] -> dy^T x (+ add) in bf16, or in float32 with keep",
         py::arg("dy"), py::arg("x"), py::arg("add") = py::none(), py::arg("keep") = false);

@@ -2,7 +2,7 @@
 // cross entropy (ops/fused_ce.py).
 //
 // Memory-bound: the forward reads a row once (online maximum and sum of exponentials), the backward reads it
-// once and writes the gradient over it. As library passes (to float32, logsumexp; to float32, subtract, exp,
+// once and writes the gradient, over it unless the forward's logits are kept. As library passes (to float32, logsumexp; to float32, subtract, exp,
 // scatter, scale, to bf16) a chunk of 4096 x 32000 took 0.74 ms forward and 0.81 ms backward; it takes 0.05 and 0.11 ms,
 // 262 and 524 MB at 5 TB/s. A vocabulary that is no multiple of 8 has rows that no wider load fits: 4096 x 50257 took 1.11 and
 // 1.26 ms and takes 0.24 and 0.31 (50304 columns 0.07 and 0.17), bound by its two-byte accesses and, forward, three
@@ -88,15 +88,17 @@ __global__ __launch_bounds__(CE_BLOCK) void ce_fwd_kernel(float* __restrict__ ls
   }
 }
 
-// logits -> their gradient (softmax - onehot) * valid * grad / n_valid, in place (NaN for a label outside the row).
+// logits -> their gradient (softmax - onehot) * valid * grad / n_valid (NaN for a label outside the row), in place or, where
+// the logits are kept, elsewhere: a thread writes what it has read.
 template <bool VEC>
-__global__ __launch_bounds__(CE_BLOCK) void ce_bwd_kernel(unsigned short* __restrict__ logits, const float* __restrict__ lse,
+__global__ __launch_bounds__(CE_BLOCK) void ce_bwd_kernel(unsigned short* out, const unsigned short* logits, const float* __restrict__ lse,
                                                           const long* __restrict__ labels, const float* __restrict__ grad,
                                                           const float* __restrict__ loss, long ignore_index, long rows,
                                                           int V) {
   const long row = (long)blockIdx.y * gridDim.x + blockIdx.x;
   if (row >= rows) return;
-  unsigned short* x = logits + row * V;
+  const unsigned short* x = logits + row * V;
+  unsigned short* y = out + row * V;
   const long label = labels[row];
   const float scale = (label == ignore_index ? 0.0f : label >= 0 && label < V ? 1.0f : NAN) * (grad[0] / loss[1]);
   const float l = lse[row];
@@ -112,10 +114,10 @@ __global__ __launch_bounds__(CE_BLOCK) void ce_bwd_kernel(unsigned short* __rest
       short8 v = *reinterpret_cast<const short8*>(x + i * 8);
 #pragma unroll
       for (int k = 0; k < 8; ++k) v[k] = (short)one((unsigned short)v[k], i * 8 + k);
-      *reinterpret_cast<short8*>(x + i * 8) = v;
+      *reinterpret_cast<short8*>(y + i * 8) = v;
     }
   } else {
-    for (int i = threadIdx.x; i < V; i += CE_BLOCK) x[i] = one(x[i], i);
+    for (int i = threadIdx.x; i < V; i += CE_BLOCK) y[i] = one(x[i], i);
   }
 }
 
@@ -186,15 +188,19 @@ void ce_fwd(at::Tensor logits, at::Tensor labels, int64_t ignore_index, at::Tens
   HIP_CHECK_LAST();
 }
 
-void ce_bwd(at::Tensor logits, at::Tensor labels, int64_t ignore_index, at::Tensor lse, at::Tensor grad, at::Tensor loss) {
+void ce_bwd(at::Tensor logits, at::Tensor labels, int64_t ignore_index, at::Tensor lse, at::Tensor grad, at::Tensor loss,
+            c10::optional<at::Tensor> into) {
   check_ce(logits, labels, lse);
+  const at::Tensor out = into ? *into : logits;
+  check_ce(out, labels, lse);
+  TORCH_CHECK(out.sizes() == logits.sizes(), "cross_entropy: the gradient has the logits' shape");
   TORCH_CHECK(grad.is_cuda() && grad.numel() == 1 && grad.scalar_type() == at::kFloat && loss.is_cuda() && loss.numel() == 2 &&
               loss.is_contiguous() && loss.scalar_type() == at::kFloat, "cross_entropy: grad is one float32, loss two");
   const long rows = logits.size(0);
   if (rows == 0) return;
   auto stream = at::hip::getCurrentHIPStream();
-  auto kernel = ce_vec(logits) ? ce_bwd_kernel<true> : ce_bwd_kernel<false>;
-  hipLaunchKernelGGL(kernel, ce_grid(rows), dim3(CE_BLOCK), 0, stream.stream(), (unsigned short*)logits.data_ptr(),
+  auto kernel = ce_vec(logits) && ce_vec(out) ? ce_bwd_kernel<true> : ce_bwd_kernel<false>;
+  hipLaunchKernelGGL(kernel, ce_grid(rows), dim3(CE_BLOCK), 0, stream.stream(), (unsigned short*)out.data_ptr(), (const unsigned short*)logits.data_ptr(),
                      lse.data_ptr<float>(), (const long*)labels.data_ptr(), grad.data_ptr<float>(), loss.data_ptr<float>(),
                      (long)ignore_index, rows, (int)logits.size(1));
   HIP_CHECK_LAST();

@@ -4,7 +4,11 @@ Computes ``CE(hidden @ W^T, labels)`` without ever materializing the full
 [N, V] logits: tokens are processed in chunks; backward recomputes each
 chunk's logits and feeds the dW/dh GEMMs directly. At the flagship bench
 size (147k tokens x 32k vocab) this replaces a ~50 GB fp32 logits+softmax
-footprint with ~1 GB of transient chunk buffers — pure HBM savings.
+footprint with transient chunk buffers — pure HBM savings.
+On the GPU the first rows, four chunks of at most 1 GiB of logits, are one chunk whose bfloat16 logits the
+backward still finds: the activations of a decoder layer for as many tokens are larger, and forming
+them again was 5 to 7 % of a training step of 8192 to 16384 tokens (16380 x 32000 at width 4096: 2.9 ms of 51;
+its products over all rows at once take 6.9 ms for 7.7 in four chunks).
 
 GEMMs run through hipBLASLt (torch.matmul), the weight gradient in bfloat16 through
 csrc/weight_grad.hip; softmax math is fp32. In bfloat16 on
@@ -30,9 +34,22 @@ def _bf16_products(t: torch.Tensor) -> bool:
     return not torch.is_autocast_enabled(kind) or torch.get_autocast_dtype(kind) == torch.bfloat16
 
 
+_KEPT_CHUNKS, _KEPT_BYTES = 4, 1 << 30
+
+
+def _spans(rows: int, vocab: int, chunk_size: int, keep: bool):
+    """How many rows' bfloat16 logits stay for the backward, and the spans of rows that are worked on: those rows, if
+    any, then chunks."""
+    kept = 0
+    if keep:
+        fit = min(_KEPT_CHUNKS * chunk_size, _KEPT_BYTES // (2 * max(vocab, 1)))
+        kept = rows if rows <= fit else fit // chunk_size * chunk_size
+    return kept, [(0, kept)] * (kept > 0) + [(s, min(s + chunk_size, rows)) for s in range(kept, rows, chunk_size)]
+
+
 class _FusedLinearCE(torch.autograd.Function):
     @staticmethod
-    def forward(ctx, hidden, weight, labels, ignore_index, chunk_size):
+    def forward(ctx, hidden, weight, labels, ignore_index, chunk_size, recorded=False):
         # hidden [N, H] (bf16/fp32), weight [V, H], labels [N]
         N = hidden.shape[0]
         ctx.chunk_size = chunk_size
@@ -43,11 +60,15 @@ class _FusedLinearCE(torch.autograd.Function):
             labels = labels.contiguous()
             lse = torch.empty(N, dtype=torch.float32, device=hidden.device)
             nll = torch.empty_like(lse)
-            for s in range(0, N, chunk_size):
-                e = min(s + chunk_size, N)
-                kernels().ce_fwd(hidden[s:e] @ weight.t(), labels[s:e], ignore_index, lse[s:e], nll[s:e])
+            ctx.kept, spans = _spans(N, weight.shape[0], chunk_size, recorded and hidden.is_cuda)
+            kept = []
+            for s, e in spans:
+                logits = hidden[s:e] @ weight.t()
+                kernels().ce_fwd(logits, labels[s:e], ignore_index, lse[s:e], nll[s:e])
+                if e <= ctx.kept:
+                    kept.append(logits)
             loss = kernels().ce_loss(nll, labels, ignore_index)
-            ctx.save_for_backward(hidden, weight, labels, lse, loss)
+            ctx.save_for_backward(hidden, weight, labels, lse, loss, *kept)
             return loss[0].clone()  # a tensor of its own: what is saved is not handed out
         lse = torch.empty(N, dtype=torch.float32, device=hidden.device)
         picked = torch.empty(N, dtype=torch.float32, device=hidden.device)
@@ -70,7 +91,7 @@ class _FusedLinearCE(torch.autograd.Function):
         if ctx.hip and not torch.is_grad_enabled() and _bf16_products(grad_out):
             return _backward_hip(ctx, grad_out)
         if ctx.hip:
-            hidden, weight, labels, lse, loss = ctx.saved_tensors
+            hidden, weight, labels, lse, loss, *_ = ctx.saved_tensors
             valid = labels != ctx.ignore_index
             safe_labels, n_valid = labels.masked_fill(~valid, 0), loss[1]
         else:
@@ -92,25 +113,28 @@ class _FusedLinearCE(torch.autograd.Function):
             ds = ds.to(hidden.dtype)
             dh[s:e] = ds @ weight
             dw += (ds.t() @ hidden[s:e]).float()
-        return dh, dw.to(weight.dtype), None, None, None
+        return dh, dw.to(weight.dtype), None, None, None, None
 
 
 def _backward_hip(ctx, grad_out):
-    hidden, weight, labels, lse, loss = ctx.saved_tensors
-    N, chunk_size = hidden.shape[0], ctx.chunk_size
+    hidden, weight, labels, lse, loss, *kept = ctx.saved_tensors
+    N = hidden.shape[0]
     grad = grad_out.float()
     dh = torch.empty_like(hidden)
     dw = None
-    for s in range(0, N, chunk_size):
-        e = min(s + chunk_size, N)
-        ds = hidden[s:e] @ weight.t()
-        kernels().ce_bwd(ds, labels[s:e], ctx.ignore_index, lse[s:e], grad, loss)
+    for s, e in _spans(N, weight.shape[0], ctx.chunk_size, bool(kept))[1]:
+        if e <= ctx.kept:
+            ds = torch.empty_like(kept[0])  # not in the logits' place: the graph may be gone through again
+            kernels().ce_bwd(kept[0], labels[s:e], ctx.ignore_index, lse[s:e], grad, loss, ds)
+        else:
+            ds = hidden[s:e] @ weight.t()
+            kernels().ce_bwd(ds, labels[s:e], ctx.ignore_index, lse[s:e], grad, loss)
         torch.mm(ds, weight, out=dh[s:e])
         # chunks are summed in float32, by the product itself
         dw = weight_grad(ds, hidden[s:e], dw, e < N)
     if dw is None:
         dw = torch.zeros_like(weight)
-    return dh, dw.to(weight.dtype), None, None, None
+    return dh, dw.to(weight.dtype), None, None, None, None
 
 
 def fused_linear_cross_entropy(
@@ -122,4 +146,5 @@ def fused_linear_cross_entropy(
 ) -> torch.Tensor:
     """hidden [.., H], weight [V, H], labels [..] -> mean CE over valid tokens."""
     H = hidden.shape[-1]
-    return _FusedLinearCE.apply(hidden.reshape(-1, H), weight, labels.reshape(-1), ignore_index, chunk_size)
+    recorded = torch.is_grad_enabled() and (hidden.requires_grad or weight.requires_grad)
+    return _FusedLinearCE.apply(hidden.reshape(-1, H), weight, labels.reshape(-1), ignore_index, chunk_size, recorded)

@@ -184,3 +184,28 @@ def test_add_norm_and_its_gradients(rows, H):
     yf = xf * torch.rsqrt(xf.pow(2).mean(-1, keepdim=True) + 1e-5) * w.detach().float()
     (gx,) = torch.autograd.grad(yf, (xf,), dy.float())
     assert _rel(y, yf) < ROUND and _rel(dx, gx) < 2 * ROUND
+
+
+# rows in the kept part, in it and beyond it, and logits of which none fit
+@pytest.mark.parametrize("N,V,chunk,kept_bytes,kept", [(37, 1000, 64, 1 << 30, 37), (300, 1024, 64, 1 << 30, 256),
+                                                       (300, 1024, 64, 300000, 128), (300, 1003, 64, 100000, 0)])
+def test_linear_cross_entropy_with_kept_logits(monkeypatch, N, V, chunk, kept_bytes, kept):
+    from colossalai_amd.ops import fused_ce
+
+    monkeypatch.setattr(fused_ce, "_KEPT_BYTES", kept_bytes)
+    assert fused_ce._spans(N, V, chunk, True)[0] == kept
+    torch.manual_seed(5)
+    hidden = torch.randn(N, 64, device="cuda").bfloat16().requires_grad_()
+    weight = (0.2 * torch.randn(V, 64, device="cuda")).bfloat16().requires_grad_()
+    labels = torch.randint(0, V, (N,), device="cuda")
+    loss = fused_ce.fused_linear_cross_entropy(hidden, weight, labels, chunk_size=chunk)
+    first = torch.autograd.grad(loss, (hidden, weight), retain_graph=True)
+    again = torch.autograd.grad(loss, (hidden, weight))
+    assert all(torch.equal(a, b) for a, b in zip(first, again))
+    h, w = hidden.detach().double().requires_grad_(), weight.detach().double().requires_grad_()
+    want = torch.nn.functional.cross_entropy(h @ w.t(), labels)
+    top = (h @ w.t()).abs().max().item()
+    for got, ref in zip(first, torch.autograd.grad(want, (h, w))):
+        assert _rel(got, ref) < 2 * ROUND * (top + 1)
+    with torch.no_grad():
+        assert abs(fused_ce.fused_linear_cross_entropy(hidden, weight, labels, chunk_size=chunk).item() - want.item()) < 2 * ROUND * top
