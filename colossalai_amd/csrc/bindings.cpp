@@ -36,7 +36,8 @@ void ce_bwd(at::Tensor logits, at::Tensor labels, int64_t ignore_index, at::Tens
             c10::optional<at::Tensor> into);
 at::Tensor ce_loss(at::Tensor nll, at::Tensor labels, int64_t ignore_index);
 
-// weight_grad.hip
+// products.hip
+at::Tensor multiply(const at::Tensor& x, const at::Tensor& w, bool slow);
 at::Tensor weight_grad(const at::Tensor& dy, const at::Tensor& x, const c10::optional<at::Tensor>& add, bool keep);
 
 // linear.cpp
@@ -121,6 +122,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("ce_loss", &cai::ce_loss, "mean negative log likelihood over the rows that are not ignored, and their number");
   m.def("weight_grad", &cai::weight_grad, "dy [K, M], x [K, N] -> dy^T x (+ add) in bf16, or in float32 with keep",
         py::arg("dy"), py::arg("x"), py::arg("add") = py::none(), py::arg("keep") = false);
+  m.def("multiply", &cai::multiply, "x [M, K] times w [N, K]^T, or with `slow` times w [K, N]");
   m.def("linear", &cai::linear, "linear layer without bias, its weight gradient by weight_grad");
   m.def("layernorm_fwd", &cai::layernorm_fwd, "LayerNorm forward");
   m.def("layernorm_bwd", &cai::layernorm_bwd, "LayerNorm backward");

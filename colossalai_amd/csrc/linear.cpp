@@ -1,4 +1,4 @@
-// Linear layers without a bias whose weight gradient is csrc/weight_grad.hip's; the other two products are the library's.
+// Linear layers without a bias: weight gradients and small products are csrc/products.hip's, the others the library's.
 #include <ATen/TensorSubclassLikeUtils.h>
 #include <ATen/autocast_mode.h>
 #include <torch/csrc/jit/frontend/tracer.h>
@@ -8,6 +8,7 @@ namespace cai {
 
 at::Tensor weight_grad(const at::Tensor& dy, const at::Tensor& x, const c10::optional<at::Tensor>& add, bool keep);
 bool weight_grad_serves(const at::Tensor& dy, const at::Tensor& x);
+at::Tensor multiply(const at::Tensor& x, const at::Tensor& w, bool slow);
 
 namespace {
 
@@ -23,7 +24,10 @@ struct Linear : torch::autograd::Function<Linear> {
   static at::Tensor forward(torch::autograd::AutogradContext* ctx, const at::Tensor& x, const at::Tensor& weight) {
     // as the built-in layer: each gradient's factor is kept only if that gradient is wanted
     ctx->save_for_backward({x, x.requires_grad() ? weight : at::Tensor()});
-    return at::linear(x, weight);
+    if (x.size(-1) != weight.size(1) || weight.dim() != 2) return at::linear(x, weight);   // which says what is wrong
+    auto sizes = x.sizes().vec();
+    sizes.back() = weight.size(0);
+    return multiply(x.reshape({-1, x.size(-1)}), weight, false).view(sizes);
   }
   static torch::autograd::variable_list backward(torch::autograd::AutogradContext* ctx, torch::autograd::variable_list grads) {
     const auto saved = ctx->get_saved_variables();
@@ -31,11 +35,12 @@ struct Linear : torch::autograd::Function<Linear> {
     if (!dy.defined()) return {at::Tensor(), at::Tensor()};
     const at::Tensor dy2 = dy.reshape({-1, dy.size(-1)});
     at::Tensor dx, dw;
-    if (ctx->needs_input_grad(0)) dx = at::mm(dy2, weight).view(x.sizes());
+    // a backward that is part of a graph itself (create_graph), or that something watches, takes operations it can see
+    const bool closed = !at::GradMode::is_enabled() && plain(dy2);
+    if (ctx->needs_input_grad(0)) dx = (closed && plain(weight) ? multiply(dy2, weight, true) : at::mm(dy2, weight)).view(x.sizes());
     if (ctx->needs_input_grad(1)) {
       const at::Tensor x2 = x.reshape({-1, x.size(-1)});
-      // a backward that is part of a graph itself (create_graph), or that something watches, takes operations it can see
-      if (!at::GradMode::is_enabled() && plain(dy2) && plain(x2) && weight_grad_serves(dy2, x2)) dw = weight_grad(dy2, x2, c10::nullopt, false);
+      if (closed && plain(x2) && weight_grad_serves(dy2, x2)) dw = weight_grad(dy2, x2, c10::nullopt, false);
       else dw = at::mm(dy2.t(), x2);
     }
     return {dx, dw};

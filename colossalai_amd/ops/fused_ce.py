@@ -10,8 +10,8 @@ backward still finds: the activations of a decoder layer for as many tokens are 
 them again was 5 to 7 % of a training step of 8192 to 16384 tokens (16380 x 32000 at width 4096: 2.9 ms of 51;
 its products over all rows at once take 6.9 ms for 7.7 in four chunks).
 
-GEMMs run through hipBLASLt (torch.matmul), the weight gradient in bfloat16 through
-csrc/weight_grad.hip; softmax math is fp32. In bfloat16 on
+GEMMs run through hipBLASLt (torch.matmul), the weight gradient and small products in bfloat16
+through csrc/products.hip; softmax math is fp32. In bfloat16 on
 the GPU a chunk's logits are read once in the forward and overwritten by their
 gradient in the backward (csrc/cross_entropy.hip).
 Reference parity: the reference materializes logits and uses torch CE (or
@@ -23,7 +23,7 @@ from typing import Optional
 import torch
 
 from ._kernels import kernels, use_hip
-from .linear import weight_grad
+from .linear import multiply, weight_grad
 
 __all__ = ["fused_linear_cross_entropy"]
 
@@ -63,7 +63,7 @@ class _FusedLinearCE(torch.autograd.Function):
             ctx.kept, spans = _spans(N, weight.shape[0], chunk_size, recorded and hidden.is_cuda)
             kept = []
             for s, e in spans:
-                logits = hidden[s:e] @ weight.t()
+                logits = multiply(hidden[s:e], weight)
                 kernels().ce_fwd(logits, labels[s:e], ignore_index, lse[s:e], nll[s:e])
                 if e <= ctx.kept:
                     kept.append(logits)
@@ -127,9 +127,12 @@ def _backward_hip(ctx, grad_out):
             ds = torch.empty_like(kept[0])  # not in the logits' place: the graph may be gone through again
             kernels().ce_bwd(kept[0], labels[s:e], ctx.ignore_index, lse[s:e], grad, loss, ds)
         else:
-            ds = hidden[s:e] @ weight.t()
+            ds = multiply(hidden[s:e], weight)
             kernels().ce_bwd(ds, labels[s:e], ctx.ignore_index, lse[s:e], grad, loss)
-        torch.mm(ds, weight, out=dh[s:e])
+        if e - s == N:
+            dh = multiply(ds, weight, True)
+        else:
+            torch.mm(ds, weight, out=dh[s:e])
         # chunks are summed in float32, by the product itself
         dw = weight_grad(ds, hidden[s:e], dw, e < N)
     if dw is None:

@@ -1,4 +1,5 @@
-"""Linear layers in training: the weight gradient of a plain bfloat16 ``nn.Linear`` by csrc/weight_grad.hip.
+"""Linear layers in training: the weight gradient and small products of a plain bfloat16 ``nn.Linear`` by
+csrc/products.hip.
 
 The layer stays an ``nn.Linear`` that parallel policies, LoRA or the zero-bubble schedule replace or change; ``project``
 calls whatever it has become.
@@ -12,7 +13,14 @@ from torch.nn.modules import module as _hooks
 
 from ._kernels import kernels
 
-__all__ = ["project", "weight_grad"]
+__all__ = ["multiply", "project", "weight_grad"]
+
+
+def multiply(x: torch.Tensor, w: torch.Tensor, slow: bool = False) -> torch.Tensor:
+    """x [M, K] times w [N, K]^T, or with ``slow`` times w [K, N]; outside autograd."""
+    if x.is_cuda:
+        return kernels().multiply(x, w, slow)
+    return x @ (w if slow else w.t())
 
 
 def weight_grad(dy: torch.Tensor, x: torch.Tensor, add: Optional[torch.Tensor] = None, keep: bool = False) -> torch.Tensor:

@@ -1,4 +1,4 @@
-"""Weight gradients of linear layers (csrc/weight_grad.hip) and the layer that uses them (csrc/linear.cpp)."""
+"""Weight gradients and small products of linear layers (csrc/products.hip) and the layer that uses them (csrc/linear.cpp)."""
 
 import pytest
 import torch
@@ -59,6 +59,20 @@ def test_what_is_not_finite_stays_in_its_row():
     got = kernels().weight_grad(dy, x)
     rows = torch.arange(264, device="cuda") != 7
     assert got[7].isnan().all() and (got[rows][:, 135] == float("inf")).all() and (got[rows][:, :135] == 100).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(1, 8, 32), (127, 136, 64), (129, 128, 96), (510, 1024, 512), (300, 264, 1056), (512, 512, 2048),
+                                   (2048, 2048, 512), (33, 40, 40), (8192, 512, 64)])
+def test_products_against_64_bits(M, N, K):
+    torch.manual_seed(M + N + K)
+    x, w = torch.randn(M, K, device="cuda").to(BF16), torch.randn(N, K, device="cuda").to(BF16)
+    for a in (x, torch.randn(M, 2 * K + 8, device="cuda").to(BF16)[:, 8: K + 8]):
+        _close(kernels().multiply(a, w, False), a.t(), w.t())
+        _close(kernels().multiply(a, w.t().contiguous(), True), a.t(), w.t())
+    x[M // 2, K - 1] = float("nan")
+    got = kernels().multiply(x, w, False)
+    assert got[M // 2].isnan().all() and got.isnan().sum() == N
 
 
 def _step(call, x, w, g):
