@@ -43,6 +43,20 @@ at::Tensor weight_grad(const at::Tensor& dy, const at::Tensor& x, const c10::opt
 // linear.cpp
 at::Tensor linear(const at::Tensor& x, const at::Tensor& weight);
 
+// functions.cpp
+c10::optional<at::Tensor> native_rms_norm(const at::Tensor& x, const at::Tensor& weight, double eps);
+c10::optional<std::tuple<at::Tensor, at::Tensor>> native_fused_add_rms_norm(const at::Tensor& x, const at::Tensor& residual,
+                                                                           const at::Tensor& weight, double eps);
+c10::optional<at::Tensor> native_swiglu(const at::Tensor& gate_up);
+c10::optional<at::Tensor> native_flash_attention(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, bool causal,
+                                                 double scale, const c10::optional<at::Tensor>& seqlens,
+                                                 const c10::optional<at::Tensor>& seqlens_k);
+c10::optional<at::Tensor> native_flash_attention_varlen(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v,
+                                                        const at::Tensor& cu, int64_t longest, bool causal, double scale);
+c10::optional<at::Tensor> native_fused_rope_attention(const at::Tensor& qkv, const at::Tensor& table,
+                                                      const c10::optional<at::Tensor>& positions, int64_t Hq, int64_t Hkv,
+                                                      int64_t D, bool causal, double scale, const c10::optional<at::Tensor>& seqlens);
+
 // layernorm.hip
 std::vector<at::Tensor> layernorm_fwd(at::Tensor input, at::Tensor gamma, c10::optional<at::Tensor> beta,
                                       double eps, bool save_stats);
@@ -124,6 +138,12 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("dy"), py::arg("x"), py::arg("add") = py::none(), py::arg("keep") = false);
   m.def("multiply", &cai::multiply, "x [M, K] times w [N, K]^T, or with `slow` times w [K, N]");
   m.def("linear", &cai::linear, "linear layer without bias, its weight gradient by weight_grad");
+  m.def("native_rms_norm", &cai::native_rms_norm, "autograd functions of the kernels above and below; None: use the Python one");
+  m.def("native_fused_add_rms_norm", &cai::native_fused_add_rms_norm);
+  m.def("native_swiglu", &cai::native_swiglu);
+  m.def("native_flash_attention", &cai::native_flash_attention);
+  m.def("native_flash_attention_varlen", &cai::native_flash_attention_varlen);
+  m.def("native_fused_rope_attention", &cai::native_fused_rope_attention);
   m.def("layernorm_fwd", &cai::layernorm_fwd, "LayerNorm forward");
   m.def("layernorm_bwd", &cai::layernorm_bwd, "LayerNorm backward");
   m.def("rope_inplace", &cai::rope_inplace, "in-place rotary embedding (fwd/bwd)");

@@ -1,8 +1,8 @@
 // Linear layers without a bias: weight gradients and small products are csrc/products.hip's, the others the library's.
-#include <ATen/TensorSubclassLikeUtils.h>
 #include <ATen/autocast_mode.h>
-#include <torch/csrc/jit/frontend/tracer.h>
 #include <torch/extension.h>
+
+#include "plain.h"
 
 namespace cai {
 
@@ -12,13 +12,8 @@ at::Tensor multiply(const at::Tensor& x, const at::Tensor& w, bool slow);
 
 namespace {
 
-// nothing that watches or rewrites single operations stands between these tensors and a kernel
-bool plain(const at::Tensor& t) {
-  return !at::isTensorSubclassLike(t) && !at::autocast::is_autocast_enabled(at::kCUDA) && !torch::jit::tracer::isTracing()
-      && !c10::impl::tls_is_dispatch_key_included(at::DispatchKey::FuncTorchDynamicLayerFrontMode);
-}
-
-bool has_tangent(const at::Tensor& t) { return t._fw_grad(0).defined(); }
+// not under autocast either, which casts the operands of the library's products
+bool plain_here(const at::Tensor& t) { return plain(t) && !at::autocast::is_autocast_enabled(at::kCUDA); }
 
 struct Linear : torch::autograd::Function<Linear> {
   static at::Tensor forward(torch::autograd::AutogradContext* ctx, const at::Tensor& x, const at::Tensor& weight) {
@@ -36,11 +31,11 @@ struct Linear : torch::autograd::Function<Linear> {
     const at::Tensor dy2 = dy.reshape({-1, dy.size(-1)});
     at::Tensor dx, dw;
     // a backward that is part of a graph itself (create_graph), or that something watches, takes operations it can see
-    const bool closed = !at::GradMode::is_enabled() && plain(dy2);
-    if (ctx->needs_input_grad(0)) dx = (closed && plain(weight) ? multiply(dy2, weight, true) : at::mm(dy2, weight)).view(x.sizes());
+    const bool closed = !at::GradMode::is_enabled() && plain_here(dy2);
+    if (ctx->needs_input_grad(0)) dx = (closed && plain_here(weight) ? multiply(dy2, weight, true) : at::mm(dy2, weight)).view(x.sizes());
     if (ctx->needs_input_grad(1)) {
       const at::Tensor x2 = x.reshape({-1, x.size(-1)});
-      if (closed && plain(x2) && weight_grad_serves(dy2, x2)) dw = weight_grad(dy2, x2, c10::nullopt, false);
+      if (closed && plain_here(x2) && weight_grad_serves(dy2, x2)) dw = weight_grad(dy2, x2, c10::nullopt, false);
       else dw = at::mm(dy2.t(), x2);
     }
     return {dx, dw};
@@ -50,7 +45,7 @@ struct Linear : torch::autograd::Function<Linear> {
 }  // namespace
 
 at::Tensor linear(const at::Tensor& x, const at::Tensor& weight) {
-  if (x.dim() < 2 || x.numel() == 0 || !plain(x) || !plain(weight) || has_tangent(x) || has_tangent(weight)) return at::linear(x, weight);
+  if (x.dim() < 2 || x.numel() == 0 || !plain_here(x) || !plain_here(weight) || has_tangent(x) || has_tangent(weight)) return at::linear(x, weight);
   return Linear::apply(x, weight);
 }
 

@@ -45,6 +45,14 @@ def use_hip(*tensors: torch.Tensor) -> bool:
     return True
 
 
+def native_function(name: str, first: torch.Tensor):
+    """An autograd function of csrc/functions.cpp for GPU tensors, outside compilation, else None. It returns None itself where
+    something stands between the tensors and a kernel; the Python function then does what it does."""
+    if not first.is_cuda or _C is None or torch.compiler.is_compiling():
+        return None
+    return getattr(_C, name)
+
+
 # ---------------------------------------------------------------------------
 # The ragged serving kernels are two small extensions of their own, so that a
 # fresh checkout that only serves a model compiles the few files that model

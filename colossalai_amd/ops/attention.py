@@ -16,7 +16,7 @@ from typing import Optional, Tuple
 
 import torch
 
-from ._kernels import kernels, use_hip
+from ._kernels import kernels, native_function, use_hip
 from .rope import apply_rope_ref
 
 __all__ = ["flash_attention", "flash_attention_varlen", "fused_rope_attention", "attention_ref",
@@ -135,6 +135,11 @@ def flash_attention(
     """
     if seqlens is None and attention_mask is not None:
         seqlens = seqlens_from_attention_mask(attention_mask).to(q.device)
+    native = native_function("native_flash_attention", q)
+    if native:
+        out = native(q, k, v, causal, 1.0 / math.sqrt(q.shape[-1]) if scale is None else scale, seqlens, seqlens_k)
+        if out is not None:
+            return out
     return _FlashAttention.apply(q, k, v, causal, scale, seqlens, seqlens_k)
 
 
@@ -187,7 +192,13 @@ def flash_attention_varlen(
     if max_seqlen is None:
         cs = cu_seqlens.to("cpu")
         max_seqlen = int((cs[1:] - cs[:-1]).max())
-    return _FlashAttentionVarlen.apply(q, k, v, cu_seqlens.to(torch.int32), max_seqlen, causal, scale)
+    cu_seqlens = cu_seqlens.to(torch.int32)
+    native = native_function("native_flash_attention_varlen", q)
+    if native:
+        out = native(q, k, v, cu_seqlens, int(max_seqlen), causal, 1.0 / math.sqrt(q.shape[-1]) if scale is None else scale)
+        if out is not None:
+            return out
+    return _FlashAttentionVarlen.apply(q, k, v, cu_seqlens, max_seqlen, causal, scale)
 
 
 def _qkv_views(qkv: torch.Tensor, Hq: int, Hkv: int, D: int):
@@ -260,4 +271,9 @@ def fused_rope_attention(
     seqlens: Optional[torch.Tensor] = None,
 ) -> torch.Tensor:
     """qkv [B,S,(Hq+2Hkv)*D] bf16 -> out [B,S,Hq,D]. Mutates qkv (RoPE)."""
+    native = native_function("native_fused_rope_attention", qkv)
+    if native:
+        out = native(qkv, rope_table, positions, Hq, Hkv, D, causal, 1.0 / math.sqrt(D) if scale is None else scale, seqlens)
+        if out is not None:
+            return out
     return _FusedRopeAttention.apply(qkv, rope_table, positions, Hq, Hkv, D, causal, scale, seqlens)

@@ -11,7 +11,7 @@ from typing import Tuple
 
 import torch
 
-from ._kernels import kernels, use_hip
+from ._kernels import kernels, native_function, use_hip
 
 __all__ = ["rms_norm", "fused_add_rms_norm", "rms_norm_ref"]
 
@@ -98,10 +98,14 @@ class _FusedAddRMSNorm(torch.autograd.Function):
 
 
 def rms_norm(x: torch.Tensor, weight: torch.Tensor, eps: float = 1e-6) -> torch.Tensor:
-    return _RMSNorm.apply(x, weight, eps)
+    native = native_function("native_rms_norm", x)
+    out = native(x, weight, eps) if native else None
+    return _RMSNorm.apply(x, weight, eps) if out is None else out
 
 
 def fused_add_rms_norm(
     x: torch.Tensor, residual: torch.Tensor, weight: torch.Tensor, eps: float = 1e-6
 ) -> Tuple[torch.Tensor, torch.Tensor]:
-    return _FusedAddRMSNorm.apply(x, residual, weight, eps)
+    native = native_function("native_fused_add_rms_norm", x)
+    out = native(x, residual, weight, eps) if native else None
+    return _FusedAddRMSNorm.apply(x, residual, weight, eps) if out is None else out

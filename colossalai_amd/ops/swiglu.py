@@ -2,7 +2,7 @@
 
 import torch
 
-from ._kernels import kernels, use_hip
+from ._kernels import kernels, native_function, use_hip
 
 __all__ = ["swiglu", "swiglu_ref"]
 
@@ -38,4 +38,6 @@ class _SwiGLU(torch.autograd.Function):
 
 
 def swiglu(gate_up: torch.Tensor) -> torch.Tensor:
-    return _SwiGLU.apply(gate_up)
+    native = native_function("native_swiglu", gate_up)
+    out = native(gate_up) if native else None
+    return _SwiGLU.apply(gate_up) if out is None else out
