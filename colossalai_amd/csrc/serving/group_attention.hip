@@ -13,7 +13,7 @@
 // and a sink 18.5 -> 16.5 us, 4 x 16384 52.0 -> 38.1 (3.5 TB/s), 16 x 8192 84 -> 63 (4.3 TB/s), 8 heads on 2, 7 x 5000
 // 24.8 -> 17.5; 16 heads on 8 of 64, 16 x 3000: 41.5 -> 28.8; one head a key head, 16 x 2000: 61 -> 56; 16 x 128: 9.4 and 9.9.
 // The eight waves' states meet in LDS at the end; few tokens with long contexts have their keys cut into parts, whose
-// states row_merge_kernel puts together.
+// states row_merge_kernel puts together. Beside prompt portions it may serve just the sequences that bring one token.
 #include "paged_attention.h"
 #include "../lds_tiles.h"
 
@@ -45,7 +45,7 @@ __global__ __launch_bounds__(64 * GROUP_WAVES, 2) void group_attention_kernel(
     const bf16s* __restrict__ vpool, const int* __restrict__ block_tables, int bt_stride, const int* __restrict__ tok_seq,
     const int* __restrict__ positions, const float* __restrict__ slopes, const bf16s* __restrict__ gate, long gate_stride,
     const float* __restrict__ sink_logits, int H, int G, int page_shift, float scale, int window, int keep_first, int chunk,
-    float softcap, int sink, int vrep, long vrow, long vhead, int splits, float* __restrict__ ws) {
+    float softcap, int sink, int vrep, long vrow, long vhead, int splits, float* __restrict__ ws, const int* __restrict__ cu) {
   constexpr int D = DS * 16, Dv = VT * 32, KQ = D / 32, KT = D * 64, VTT = Dv * 64;   // bytes of a tile's keys, values
   constexpr float LOG2E = 1.4426950408889634f;
   extern __shared__ __align__(16) char tiles[];   // [waves][KT + VTT], later the waves' states; then the pages
@@ -53,7 +53,12 @@ __global__ __launch_bounds__(64 * GROUP_WAVES, 2) void group_attention_kernel(
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int col = lane & 31, hf = lane >> 5;
   const int split = (int)(blockIdx.x % splits);
-  const long n = blockIdx.x / splits / G;
+  const long unit = blockIdx.x / splits / G;   // a token, or with `cu` a sequence
+  long n = unit;
+  if (cu != nullptr) {
+    if (cu[unit + 1] - cu[unit] != 1) return;
+    n = cu[unit];
+  }
   const int g = (int)(blockIdx.x / splits % G);
   const int R = H / G, h0 = g * R;
   const int pos = positions[n];
@@ -280,7 +285,7 @@ __global__ __launch_bounds__(64 * GROUP_WAVES, 2) void group_attention_kernel(
       o += states[w * WS + r * PS + 2 + dv] * f;
     }
     if (splits > 1) {   // a part without keys has a maximum of -inf
-      float* state = ws + ((n * H + h0 + r) * splits + split) * (long)PS;
+      float* state = ws + ((unit * H + h0 + r) * splits + split) * (long)PS;
       state[2 + dv] = o;
       if (dv == 0) {
         state[0] = top;
@@ -302,8 +307,9 @@ bool launch_group_attention(at::Tensor& out, const at::Tensor& q, const at::Tens
                             const at::Tensor& block_tables, const at::Tensor& tok_seq, const at::Tensor& positions,
                             const float* slopes, const c10::optional<at::Tensor>& gate, long gate_stride, double scale,
                             int64_t window, int64_t keep_first, double softcap, bool sink, int page_shift, long vrow,
-                            long vhead, const ScalarExtras& x) {
-  const long N = q.size(0);
+                            long vhead, const ScalarExtras& x, const SingleTokens& only) {
+  const bool some = only.cu != nullptr;
+  const long N = some ? only.count : q.size(0), units = some ? only.seqs : N;   // tokens, and what takes their place
   const int H = (int)q.size(1), D = (int)q.size(2), G = (int)kpool.size(2), Dv = (int)vpool.size(3), R = H / G;
   if (!is_bf16(q) || x.dist_bias != nullptr || x.ksum != nullptr || x.cross_out != nullptr || x.key_fac != nullptr ||
       x.out32 != nullptr || (D != 64 && D != 128) || (Dv != 64 && Dv != 128) || R > GROUP_HEADS)
@@ -328,23 +334,23 @@ bool launch_group_attention(at::Tensor& out, const at::Tensor& q, const at::Tens
   const size_t lds = (size_t)GROUP_WAVES * (D + Dv) * 64 + (size_t)((part_keys >> page_shift) + (keep_first >> page_shift) + 4) * sizeof(int);
   if (lds > GROUP_LDS) return false;
   at::Tensor ws;
-  if (splits > 1) ws = at::empty({N * H * splits * (2 + Dv)}, q.options().dtype(at::kFloat));
+  if (splits > 1) ws = at::empty({units * H * splits * (2 + Dv)}, q.options().dtype(at::kFloat));
 #define GROUP_LAUNCH(DS_, VT_)                                                                                       \
   do {                                                                                                             \
     auto kernel = group_attention_kernel<DS_, VT_>;                                                                \
     if (lds > 65536) (void)hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds); \
-    hipLaunchKernelGGL(kernel, dim3((unsigned)(N * G * splits)), dim3(64 * GROUP_WAVES), lds, stream(), ptr<bf16s>(out), \
+    hipLaunchKernelGGL(kernel, dim3((unsigned)(units * G * splits)), dim3(64 * GROUP_WAVES), lds, stream(), ptr<bf16s>(out), \
                        ptr<bf16s>(q), (long)q.stride(0), ptr<bf16s>(kpool), ptr<bf16s>(vpool), block_tables.data_ptr<int>(), \
                        (int)block_tables.stride(0), tok_seq.data_ptr<int>(), positions.data_ptr<int>(), slopes,    \
                        gate.has_value() ? ptr<bf16s>(*gate) : (const bf16s*)nullptr, gate_stride, x.sink_logits, H, G, page_shift, \
                        (float)scale, (int)window, (int)keep_first, x.chunk, (float)softcap, sink ? 1 : 0, x.vrep, vrow, vhead, \
-                       splits, splits > 1 ? ws.data_ptr<float>() : (float*)nullptr);                              \
+                       splits, splits > 1 ? ws.data_ptr<float>() : (float*)nullptr, only.cu);                            \
   } while (0)
   if (D == 128) { if (Dv == 128) GROUP_LAUNCH(8, 4); else GROUP_LAUNCH(8, 2); }
   else { if (Dv == 128) GROUP_LAUNCH(4, 4); else GROUP_LAUNCH(4, 2); }
 #undef GROUP_LAUNCH
   HIP_CHECK_LAST();
-  if (splits > 1) launch_row_merge(out, q, ws, gate, gate_stride, x, Dv, sink, splits);
+  if (splits > 1) launch_row_merge(out, q, ws, gate, gate_stride, x, Dv, sink, splits, only);
   return true;
 }
 

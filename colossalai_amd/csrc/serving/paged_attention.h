@@ -21,6 +21,13 @@ struct ScalarExtras {
   float* out32 = nullptr;
 };
 
+// The decode tokens of a mixed step for kernels that otherwise take every token of the call: those of the `seqs` sequences whose
+// offsets in `cu` are one apart, `count` of them. A sequence takes a token's place then; others end at once.
+struct SingleTokens {
+  const int* cu = nullptr;
+  long seqs = 0, count = 0;
+};
+
 template <int CTRL>
 DEV_INLINE float dpp_add(float v) {
   const int moved = __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, false);
@@ -46,11 +53,11 @@ bool launch_group_attention(at::Tensor& out, const at::Tensor& q, const at::Tens
                             const at::Tensor& block_tables, const at::Tensor& tok_seq, const at::Tensor& positions,
                             const float* slopes, const c10::optional<at::Tensor>& gate, long gate_stride, double scale,
                             int64_t window, int64_t keep_first, double softcap, bool sink, int page_shift, long vrow,
-                            long vhead, const ScalarExtras& x);
+                            long vhead, const ScalarExtras& x, const SingleTokens& only = SingleTokens());
 
 // The states of `splits` parts of each (token, head)'s keys in `ws` -> `out`, or x.out32; q gives the type of the call (row_attention.hip).
 void launch_row_merge(at::Tensor& out, const at::Tensor& q, const at::Tensor& ws, const c10::optional<at::Tensor>& gate,
-                      long gate_stride, const ScalarExtras& x, int Dv, bool sink, int splits);
+                      long gate_stride, const ScalarExtras& x, int Dv, bool sink, int splits, const SingleTokens& only = SingleTokens());
 
 }  // namespace serving
 }  // namespace cai

@@ -326,7 +326,7 @@ __global__ __launch_bounds__(256 * NG, 2) void paged_attention_mfma_kernel(
     int tile_waves, const float* __restrict__ sink2, const float* __restrict__ dist2, int dist_rows,
     const bf16s* __restrict__ ksum, const bf16s* __restrict__ vsum, int sum_shift, int sum_block,
     float* __restrict__ cross_out, int chunk, const float* __restrict__ key_fac, int vrep, float* __restrict__ out32,
-    int num_tiles) {
+    int num_tiles, int fewest) {
   // The optional extras of the split-key kernel, in the base-2 domain: sink2 [H] = learned sink scores * log2e;
   // dist2 [H, dist_rows] = the per-distance bias * log2e, one row per head; ksum / vsum = block summaries, staged as
   // the first tiles of a block (summary idx of a sequence is seen by a token at pos when idx < (pos - window + 1) /
@@ -379,8 +379,8 @@ __global__ __launch_bounds__(256 * NG, 2) void paged_attention_mfma_kernel(
   const int hl = (zrow / VC) * heads + (wid >> tile_waves);  // head inside the group
   const int h = g * rep + (hl < rep ? hl : 0);
   const int bshift = 5 + tile_waves;                  // log2 of the tokens a block covers
-  for (;; ++b) {  // there are exactly sum_b ceil(count_b / tokens per block) tiles
-    const int nt = (cu[b + 1] - cu[b] + (1 << bshift) - 1) >> bshift;
+  for (;; ++b) {  // there are exactly sum_b ceil(count_b / tokens per block) tiles, of the sequences of `fewest` tokens or more
+    const int count = cu[b + 1] - cu[b], nt = count < fewest ? 0 : (count + (1 << bshift) - 1) >> bshift;
     if (tile < nt) break;
     tile -= nt;
   }
@@ -867,7 +867,7 @@ static bool launch_mfma_attention(at::Tensor& out, const at::Tensor& q, const at
                                   const at::Tensor& block_tables, const at::Tensor& cu, const at::Tensor& start,
                                   const float* slp, const c10::optional<at::Tensor>& gate, long gstride, double scale,
                                   int64_t window, int64_t keep_first, double softcap, bool sink, int page_shift,
-                                  int64_t num_tiles, int64_t num_tiles128, int64_t num_tiles64, const ScalarExtras& x) {
+                                  int64_t num_tiles, int64_t num_tiles128, int64_t num_tiles64, const ScalarExtras& x, int fewest = 1) {
   const int H = (int)q.size(1), D = (int)q.size(2);
   const int G = (int)kpool.size(2), Dv = (int)vpool.size(3);
   // prompt portions in bfloat16 go to the matrix cores when the head sizes fit a tiling;
@@ -921,7 +921,7 @@ static bool launch_mfma_attention(at::Tensor& out, const at::Tensor& q, const at
                        page_shift, (float)scale, (int)window, (int)keep_first, (float)softcap, sink ? 1 : 0,       \
                        tile_waves, x.sink_logits, x.dist_bias, x.dist_rows, (const bf16s*)x.ksum,                      \
                        (const bf16s*)x.vsum, x.sum_shift, x.sum_block, x.cross_out, x.chunk, x.key_fac, x.vrep,    \
-                       x.out32, tiles);                                                                            \
+                       x.out32, tiles, fewest);                                                                         \
   } while (0)
 #define MFMA_ROW(DS_)                     \
   do {                                    \
@@ -946,7 +946,8 @@ static bool launch_mfma_attention(at::Tensor& out, const at::Tensor& q, const at
 at::Tensor paged_attention(at::Tensor q, at::Tensor kpool, at::Tensor vpool, at::Tensor block_tables, at::Tensor cu,
                            at::Tensor start, at::Tensor tok_seq, at::Tensor positions, double scale, int64_t window,
                            int64_t keep_first, c10::optional<at::Tensor> slopes, c10::optional<at::Tensor> gate,
-                           int64_t num_tiles, double softcap, bool sink, int64_t num_tiles128, int64_t num_tiles64) {
+                           int64_t num_tiles, double softcap, bool sink, int64_t num_tiles128, int64_t num_tiles64, int64_t singles,
+                           bool singles_see_half) {
   check_act(q, "q");
   TORCH_CHECK(softcap >= 0.0, "softcap must not be negative (0 = none)");
   TORCH_CHECK(q.dim() == 3 && q.stride(2) == 1 && q.stride(1) == q.size(2), "q must be [N, H, D] with dense rows");
@@ -983,8 +984,27 @@ at::Tensor paged_attention(at::Tensor q, at::Tensor kpool, at::Tensor vpool, at:
   at::Tensor out = at::empty({N, H, Dv}, q.options());
   if (N == 0) return out;
   check_i32(cu, "cu"); check_i32(start, "start");
+  // A decode token beside prompt portions is a tile of its own in their kernel, 4 waves over all its keys, and costs little as
+  // long as its blocks fit beside the others; a launch of its own stands in line (10 to 15 us). It goes apart where its blocks
+  // would be the first beyond one, or two, for each CU and it sees half as many keys as a portion or more: 14 beside portions
+  // of 1000 and 963, window 1024: 80 us together, 70 apart (32 heads on 8: 123, 96), without a window 2100 keys 150, 133, 16000 keys 1427, 1110.
+  // Otherwise: 15 of 400 beside 4000, 8 heads on 4 of 64: 76 together, 86 apart; 15 beside 512 after 2000, window 512: 29, 40.
+  int fewest = 1;
+  if (singles > 0 && num_tiles > singles && vpool.is_contiguous()) {
+    const int rep = H / G;
+    const long tiles = rep == 1 && num_tiles128 > 0 ? num_tiles128 : rep == 2 && num_tiles64 > 0 ? num_tiles64 : num_tiles;
+    const long rows = (long)G * (rep <= 4 ? 1 : (rep + 3) / 4), portions = (tiles - singles) * rows, both = tiles * rows;
+    if (portions <= 512 && (both + 255) / 256 > (portions + 255) / 256 && singles_see_half &&
+        launch_group_attention(out, q, kpool, vpool, block_tables, tok_seq, positions, slp, gate, gstride, scale, window, keep_first,
+                               softcap, sink, page_shift, vrow, vhead, ScalarExtras(), SingleTokens{cu.data_ptr<int>(), cu.numel() - 1, singles})) {
+      fewest = 2;
+      num_tiles -= singles;
+      num_tiles128 -= singles;
+      num_tiles64 -= singles;
+    }
+  }
   if (launch_mfma_attention(out, q, kpool, vpool, block_tables, cu, start, slp, gate, gstride, scale, window, keep_first,
-                            softcap, sink, page_shift, num_tiles, num_tiles128, num_tiles64, ScalarExtras()))
+                            softcap, sink, page_shift, num_tiles, num_tiles128, num_tiles64, ScalarExtras(), fewest))
     return out;
   launch_scalar_attention(out, q, kpool, vpool, block_tables, tok_seq, positions, slp, gate, gstride, scale, window,
                           keep_first, softcap, sink, page_shift, vrow, vhead, ScalarExtras());

@@ -229,6 +229,7 @@ def paged_attention(q, kpool, vpool, batch: RaggedBatch, scale: float, window: i
     if hip:
         return serving_kernels().paged_attention(q, kpool, vpool, batch.block_tables, batch.cu, batch.start,
                                                  batch.tok_seq, batch.positions, scale, window, keep_first,
-                                                 slopes, gate, tiles32, float(softcap), bool(sink), tiles128, tiles64)
+                                                 slopes, gate, tiles32, float(softcap), bool(sink), tiles128, tiles64,
+                                                 *(batch.single_tokens(window) if tiles32 else (0, False)))
     return paged_attention_ref(q, kpool, vpool, batch, scale, window, keep_first, slopes, gate, softcap, sink,
                                sink_logits, dist_bias, pooled, talk, chunk, key_factors, out_dtype)

@@ -34,6 +34,7 @@ class RaggedBatch:
     page_size: int = 0
     _dense: Optional[dict] = None  # memo of dense_context(), by window
     _chunk_tables: Optional[dict] = None  # memo of chunk_tables(), by chunk size
+    _singles: Optional[tuple] = None  # memo of single_tokens()
 
     @property
     def num_seqs(self) -> int:
@@ -55,6 +56,18 @@ class RaggedBatch:
             return 0, 0, 0
         new = [b - a for a, b in zip(cu, cu[1:])]
         return sum((n + 31) // 32 for n in new), sum((n + 63) // 64 for n in new), sum((n + 127) // 128 for n in new)
+
+    def single_tokens(self, window: int = 0):
+        """Of a step with prompt portions: how many sequences bring one token, and whether the longest of them sees at least
+        half as many keys as the longest portion's last token."""
+        if self._singles is None:
+            new = [b - a for a, b in zip(self.cu_host, self.cu_host[1:])]
+            single = [s + 1 for n, s in zip(new, self.start_host) if n == 1]
+            self._singles = len(single), max(single, default=0), max((s + n for n, s in zip(new, self.start_host) if n > 1), default=0)
+        count, short, long = self._singles
+        if window > 0:
+            short, long = min(short, window), min(long, window)
+        return count, 2 * short >= long
 
     @property
     def num_tiles32(self) -> int:

@@ -265,3 +265,13 @@ def test_decode_scores_that_rise_and_fall(levels, parts):
     got = paged_attention(q, k, v, batch, scale)
     want = paged_attention_ref(q.float(), k.float(), v.float(), batch, scale)
     assert (got.double() - want.double()).norm() / want.double().norm() < BOUND
+
+
+# decode tokens beside portions that fill the chip alone, first, last and between them: they go to the decode kernel, whole and
+# in parts; in the last two cases they stay (short contexts, few enough blocks)
+@pytest.mark.parametrize("counts,starts", [([1, 1000, 1, 990, 1], [900, 40, 1500, 0, 3]), ([1, 1, 1, 1990], [2100, 1025, 0, 3]),
+                                           ([1, 1000, 1, 990], [300, 40, 100, 0]), ([1, 500, 1], [700, 0, 600])])
+@pytest.mark.parametrize("H,G,D,Dv", [(16, 4, 128, 128), (16, 8, 64, 64), (16, 4, 64, 128)])
+@pytest.mark.parametrize("kw", [dict(window=1024, keep_first=4, slopes=True, gate=True), dict(softcap=5.0, sink=True)])
+def test_decode_tokens_beside_long_portions(counts, starts, H, G, D, Dv, kw):
+    _check(counts, starts, H, G, D, Dv, 16, D ** -0.5, **dict(kw))
