@@ -128,7 +128,8 @@ def test_padded_rows_with_shared_heads():
             assert (a[b, n:] == 0).all(), name
 
 
-@pytest.mark.parametrize("lens,H,G,D", [([512, 1, 0, 300], 4, 2, 128), ([700], 8, 2, 64), ([64, 128, 129, 31], 2, 2, 64)])
+@pytest.mark.parametrize("lens,H,G,D", [([512, 1, 0, 300], 4, 2, 128), ([700], 8, 2, 64), ([64, 128, 129, 31], 2, 2, 64),
+                                        ([300 - 7 * i for i in range(40)], 8, 2, 128)])  # the last by tile
 def test_packed(lens, H, G, D):
     from colossalai_amd.ops import flash_attention_varlen
 
