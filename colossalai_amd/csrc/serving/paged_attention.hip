@@ -313,7 +313,7 @@ __global__ __launch_bounds__(64 * ATT_WAVES) void paged_attention_kernel(
 // 3140 of them are products. 243 of 256 registers at 128 channels.
 // One 4096-token prompt, 16 heads on 4 of 128, page 64: 196 us before, 138 with this, 115 with two groups of waves a block; a cap and a
 // sink 228, 167, 133; 16 heads of one key head each 201, 140, 120; 16 x 1024 after 100, 16 heads on 8: 287 -> 168, and with two token tiles a
-// block; 14 decode tokens beside portions of 1000 and 963, window 1024: 141 -> 76; 2 x 256: 22.7 -> 15.1.
+// block; 14 decode tokens beside portions of 1000 and 963, window 1024: 141 -> 76, and 65 with what has changed since; 2 x 256: 22.7 -> 15.1.
 // Value fragments read ahead changed nothing (138 to 140), no wave priorities cost 2 %.
 __device__ __align__(16) const bf16s zero_channels[8] = {0, 0, 0, 0, 0, 0, 0, 0};
 
@@ -452,11 +452,18 @@ __global__ __launch_bounds__(256 * NG, 2) void paged_attention_mfma_kernel(
     int key[TP], fac[TP];
     bool from_sum[TP];  // a summary tile
   };
-  auto lookup = [&](int step) {
+  // Steps go from the nearest keys to the farthest. The other way round the scores of a head with a steep distance penalty rise by
+  // more than 12 from step to step, so that every step raises the reference and takes its weights twice (4000 tokens, window 1024:
+  // 83 us, 75 this way; 14 decode tokens beside portions of 1000 and 963: 72, 65). Without a penalty it is all the same (4096
+  // tokens 125 and 125 us), but a way that depends on the call costs 2 to 3 %.
+  const int steps_n = (tiles_n + TS - 1) / TS;
+  constexpr int way = -TS;
+  const int first_tile = (steps_n - 1) * TS;
+  auto lookup = [&](int tile0) {   // of the step whose first tile this is
     Rows r;
 #pragma unroll
     for (int u = 0; u < TP; ++u) {
-      const int it = step * TS + grp * TP + u, kbase = tile_base(it);  // a tile past the last one reads rows that exist and is not used
+      const int it = tile0 + grp * TP + u, kbase = tile_base(it);  // a tile past the last one reads rows that exist and is not used
       r.from_sum[u] = MORE && it < sum_tiles;
       r.key[u] = r.from_sum[u] ? sum_row(kbase + lkey) : pool_row(kbase + lkey);
       r.fac[u] = key_fac != nullptr && tid < 32 ? pool_row(kbase + tid) : 0;
@@ -538,15 +545,14 @@ __global__ __launch_bounds__(256 * NG, 2) void paged_attention_mfma_kernel(
   const bool raw = !capped && !sloped && db == nullptr;
   const float k1 = raw ? c1 : 1.0f;
 
-  const int steps_n = (tiles_n + TS - 1) / TS;
   const RowAt row_at(col, hf);
   const ColAt col_at(lane);
-  Rows next = lookup(0);
+  Rows next = lookup(first_tile);
   char* mine = tiles + grp * TP * (KT + VTT);     // this group's tiles of the first buffer
   constexpr int BUF = TS * (KT + VTT);
   all_pieces(next, mine);
   fetch_factors(next);
-  if (steps_n > 1) next = lookup(1);
+  if (steps_n > 1) next = lookup(first_tile + way);
   stash_factors(0);
   loads_done();
   __syncthreads();
@@ -727,13 +733,14 @@ __global__ __launch_bounds__(256 * NG, 2) void paged_attention_mfma_kernel(
       }
     __builtin_amdgcn_s_setprio(0);
   };
-  for (int step = 0; step < steps_n; ++step) {
+  int tile0 = first_tile;
+  for (int step = 0; step < steps_n; ++step, tile0 += way) {
     const int buf = step & 1;
     const Rows now = next;          // the next step's rows; its loads repeat the last step's where there is none
-    if (step + 2 < steps_n) next = lookup(step + 2);
+    if (step + 2 < steps_n) next = lookup(tile0 + 2 * way);
     if (step + 1 < steps_n) fetch_factors(now);
     // The TP tiles of a step go through the softmax together: one sum, one look at the reference.
-    const int it0 = step * TS + grp * TP, kb0 = tile_base(it0);
+    const int it0 = tile0 + grp * TP, kb0 = tile_base(it0);
     // interior step: every key of its tiles is visible to every token of the wave, no masks to evaluate
     const bool inner = head_ok && it0 >= sink_tiles && kb0 >= lo_p1 && kb0 + 32 * TP - 1 <= p0 && t_off + 31 < cnt;
     bool live[TP];       // this wave sees something of the tile
