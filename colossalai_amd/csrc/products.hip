@@ -4,7 +4,7 @@
 // Operands lie as they come: with the contracted index fast, fragments are plain LDS reads, with it slow (both of a weight
 // gradient) transposing ones (ds_read_b64_tr_b16, see flash_attn.hip). Four waves hold a tile's sums in registers, one
 // quarter each: 256 x 256 where there is enough of them, which is the least LDS and memory traffic a product has here (a
-// wave's 128 x 128 sums are 256 registers, one wave a SIMD), else 128 x 128 with two blocks a CU. Four steps of 32
+// wave's 128 x 128 sums are 256 registers, one wave a SIMD), else 256 x 128 or 128 x 128 with two blocks a CU. Four steps of 32
 // contracted indices lie in LDS: while one is multiplied the next is there and two are on their way, so that a step waits for
 // loads that are two steps old (s_waitcnt vmcnt, never 0) and for one barrier. A wave reads the fragments of the next 16
 // indices and issues its loads one by one between the products of the 16 before.
@@ -14,8 +14,8 @@
 //
 // Weight gradients M, N, K; us with the library's product -> here:
 //   22016, 4096, 16384   2785 -> 2214     4096, 11008, 16384   1536 -> 1132     4096, 4096, 16384   470 -> 404
-//   32000, 4096, 4096     952 -> 859      32000, 768, 4096      223 -> 191      4096, 768, 8192      84 -> 65
-//   768, 2048, 8192        65 -> 40       768, 768, 8192         49 -> 22       2048, 512, 512       21 -> 10
+//   32000, 4096, 4096     952 -> 859      32000, 768, 4096      223 -> 191      4096, 768, 8192      84 -> 61
+//   768, 2048, 8192        65 -> 38       768, 768, 8192         49 -> 22       2048, 512, 512       21 -> 10
 // Small others, back to back (the library's call takes the host 19 to 20 us, its kernels 8 to 11):
 //   x W^T: 512, 1536, 512   19.2 -> 9.0   512, 512, 1024   19.7 -> 11.4     dy W: 512, 512, 2048   19.2 -> 13.9
 // Large ones stay with the library: 16384, 12288, 4096   1080 us there, 1468 here; dy W 16384, 4096, 12288   1224, 1377.
@@ -272,29 +272,33 @@ void launch(const Args& a, hipStream_t stream) {
 }
 
 struct Plan {
-  int tile, full, parts;
+  int tm, tn, full, parts;
   double us;
 };
 
-// Tile size and parts by the time that they should take. A round of blocks over the 256 CUs takes a step in 0.79 us with large tiles
-// (1.36 PFLOP/s) and in 0.25 us with small ones (1.07; two blocks share a CU, each then at half the speed), 5 us
+// Tile size and parts by the time that they should take. A round of blocks over the 256 CUs takes a step in 0.79 us with 256 x 256 tiles
+// (1.36 PFLOP/s) and in 0.25 us with 128 x 128 ones (1.07; two blocks share a CU, each then at half the speed), 5 us
 // around its steps; what is left after whole rounds of tiles may be cut into parts of at least 256 contracted indices, whose sums
-// travel at about 5 TB/s both ways and take another launch. A cut has to promise 2 %. Measured, weight gradients, large
-// tiles whole / cut, small ones whole / cut, us: 22016 x 4096 x 16384: 2370 / 2214; 4096 x 11008 x 16384: 1132 / 1181,
-// 1927 / 1656; 4096 x 768 x 8192: 140 / 65, 69 / 68; 768 x 768 x 8192: 138 / 31, 62 / 22; 512 x 512 x 512: 19 / 18, 8.3 / 10.5.
-Plan plan(long M, long N, long K, int largest) {
-  Plan best{0, 0, 1, 0.0};
-  for (int t = largest; t >= 128; t -= 128) {
-    const long tiles = ((M + t - 1) / t) * ((N + t - 1) / t), steps = (K + KT - 1) / KT, slots = t == 256 ? 256 : 512;
-    const double c = t == 256 ? 0.79 : 0.25;
+// travel at about 5 TB/s both ways and take another launch. Tiles of 256 x 128 take 0.36 us as long as one round is all; over
+// several the clock falls, and they are no better than 128 x 128. A change has to promise 2 %. Measured, weight
+// gradients, 256 x 256 whole / cut, 256 x 128 cut, 128 x 128 whole / cut, us: 22016 x 4096 x 16384: 2370 / 2214, 2731, -;
+// 4096 x 11008 x 16384: 1132 / 1181, -, 1927 / 1656; 4096 x 768 x 8192: 140 / 63, 61, 69 / 66; 768 x 2048 x 8192: 146 / 44, 38, 68 / 39;
+// 768 x 768 x 8192: 138 / 31, 25, 62 / 22; 512 x 512 x 512: 19 / 18, 14, 8.3 / 10.5.
+Plan plan(long M, long N, long K, bool small_only) {
+  struct { int tm, tn; double step; long slots; bool one_round; } forms[] = {{256, 256, 0.79, 256, false}, {256, 128, 0.36, 256, true}, {128, 128, 0.25, 512, false}};
+  Plan best{0, 0, 0, 1, 0.0};
+  for (const auto& form : forms) {
+    if (small_only && form.tm != 128) continue;
+    const long tiles = ((M + form.tm - 1) / form.tm) * ((N + form.tn - 1) / form.tn), steps = (K + KT - 1) / KT;
+    if (form.one_round && tiles > 256) continue;
     auto take = [&](long full, long parts, double us) {
-      if (best.tile == 0 || us < 0.98 * best.us) best = Plan{t, (int)full, (int)parts, us};
+      if (best.tm == 0 || us < 0.98 * best.us) best = Plan{form.tm, form.tn, (int)full, (int)parts, us};
     };
-    auto round = [&](long blocks, long n) { return (double)((blocks + 255) / 256) * (n * c + 5.0); };
+    auto round = [&](long blocks, long n) { return (double)((blocks + 255) / 256) * (n * form.step + 5.0); };
     take(tiles, 1, round(tiles, steps));
-    const long full = tiles / slots * slots, rest = tiles - full;
-    for (long p = 2; rest && p * rest <= 512 && p * 8 <= steps; ++p)
-      take(full, p, round(full, steps) + round(rest * p, (steps + p - 1) / p) + 3.0 + rest * p * t * t * 8 / 5e6);
+    const long full = tiles / form.slots * form.slots, rest = tiles - full;
+    for (long p = 2; rest && p * rest <= (form.one_round ? 256 : 512) && p * 8 <= steps; ++p)
+      take(full, p, round(full, steps) + round(rest * p, (steps + p - 1) / p) + 3.0 + rest * p * form.tm * form.tn * 8 / 5e6);
   }
   return best;
 }
@@ -316,8 +320,8 @@ at::Tensor run(const at::Tensor& p, const at::Tensor& q, Plan plan, const c10::o
   a.K = (int)p.size(PC ? 0 : 1);
   a.M = (int)p.size(PC ? 1 : 0);
   a.N = (int)q.size(QC ? 1 : 0);
-  a.tiles_m = (a.M + plan.tile - 1) / plan.tile;
-  a.tiles_n = (a.N + plan.tile - 1) / plan.tile;
+  a.tiles_m = (a.M + plan.tm - 1) / plan.tm;
+  a.tiles_n = (a.N + plan.tn - 1) / plan.tn;
   a.full = plan.full;
   a.part_k = ((a.K + plan.parts - 1) / plan.parts + KT - 1) / KT * KT;
   a.parts = (a.K + a.part_k - 1) / a.part_k;
@@ -328,12 +332,13 @@ at::Tensor run(const at::Tensor& p, const at::Tensor& q, Plan plan, const c10::o
   at::Tensor ws;
   const long rest = (long)a.tiles_m * a.tiles_n - a.full;
   if (rest) {
-    ws = at::empty({rest * a.parts * plan.tile * plan.tile}, p.options().dtype(at::kFloat));
+    ws = at::empty({rest * a.parts * plan.tm * plan.tn}, p.options().dtype(at::kFloat));
     a.ws = ws.data_ptr<float>();
   }
   const auto stream = at::hip::getCurrentHIPStream();
   if constexpr (PC) {
-    if (plan.tile == 256) launch<PC, QC, 256, 256, 4>(a, stream);
+    if (plan.tn == 256) launch<PC, QC, 256, 256, 4>(a, stream);
+    else if (plan.tm == 256) launch<PC, QC, 256, 128, 4>(a, stream);
     else launch<PC, QC, 128, 128, 4>(a, stream);
   } else {
     launch<PC, QC, 128, 128, 4>(a, stream);
@@ -367,7 +372,7 @@ at::Tensor weight_grad(const at::Tensor& dy, const at::Tensor& x, const c10::opt
     return r.to(keep ? at::kFloat : dy.scalar_type());
   }
   return pr::run<true, true>(pr::loadable(dy) ? dy : dy.clone(at::MemoryFormat::Contiguous),
-                             pr::loadable(x) ? x : x.clone(at::MemoryFormat::Contiguous), pr::plan(dy.size(1), x.size(1), dy.size(0), 256), add, keep);
+                             pr::loadable(x) ? x : x.clone(at::MemoryFormat::Contiguous), pr::plan(dy.size(1), x.size(1), dy.size(0), false), add, keep);
 }
 
 // x [M, K] times w [N, K]^T, or with `slow` times w [K, N]. Products that should take at most 14 us, about what the
@@ -377,7 +382,7 @@ at::Tensor multiply(const at::Tensor& x, const at::Tensor& w, bool slow) {
       && pr::loadable(x) && pr::loadable(w)) {
     const long M = x.size(0), N = w.size(slow ? 1 : 0), K = x.size(1);
     if (((M + 127) / 128) * ((N + 127) / 128) <= 256) {
-      const pr::Plan plan = pr::plan(M, N, K, 128);
+      const pr::Plan plan = pr::plan(M, N, K, true);
       if (plan.us <= 14.0) return slow ? pr::run<false, true>(x, w, plan, c10::nullopt, false) : pr::run<false, false>(x, w, plan, c10::nullopt, false);
     }
   }

@@ -26,7 +26,8 @@ def _close(got, dy, x, add=None, keep=False):
 # edges of both tile sizes, of the steps of 32 tokens and of the parts
 @pytest.mark.gpu
 @pytest.mark.parametrize("M,N,K", [(8, 8, 1), (128, 136, 31), (120, 256, 33), (264, 248, 300), (768, 768, 4100), (1032, 776, 1500),
-                                   (512, 512, 512), (4096, 4104, 65), (8, 2048, 16384), (5120, 4096, 1000)])
+                                   (512, 512, 512), (4096, 4104, 65), (8, 2048, 16384), (5120, 4096, 1000),
+                                   (4096, 768, 8190), (760, 2056, 8192), (2312, 776, 4100)])
 def test_against_64_bits(M, N, K):
     torch.manual_seed(M + N + K)
     dy, x = (torch.randn(K, n, device="cuda").to(BF16) for n in (M, N))
