@@ -4,7 +4,7 @@
 // A wave takes a tile of 32 keys by itself: its keys and values come straight into LDS of its own (lds_tiles.h), no
 // barrier until the end. As in the prompt portions' kernel the products are formed transposed,
 //   S^T = K Q^T (A = key rows, B = query rows in registers: column = head), O^T = V^T P^T (the float32 weights in the C
-//   layout they were born in, split into a high and a low bfloat16 half; A = values by transposing reads),
+//   layout they were born in, each as three bfloat16 pieces, which hold all of its 24 bits; A = values by transposing reads),
 // so a head is a lane and its half-wave twin. Of the 32 columns the group fills 1 to 16; the products cost a tenth of the time that
 // the tile's 16 KB take to arrive. The next tile's keys are on their way from the moment the scores are
 // formed, its values from the end of the products.
@@ -197,7 +197,7 @@ __global__ __launch_bounds__(64 * GROUP_WAVES, 2) void group_attention_kernel(
 #pragma unroll
       for (int i = 0; i < 16; ++i) x[i] = t * 32 + (i & 3) + 8 * (i >> 2) + 4 * hf < total ? x[i] : -INFINITY;
     }
-    bf16x8_v phi[2], plo[2];
+    bf16x8_v pw[3][2];
     float psum;
     for (bool raised = false;; raised = true) {
       psum = 0.0f;
@@ -205,14 +205,16 @@ __global__ __launch_bounds__(64 * GROUP_WAVES, 2) void group_attention_kernel(
       for (int i = 0; i < 16; i += 2) {
         const float p0 = __builtin_amdgcn_exp2f(fmaf(x[i], k2, -m_ref)), p1 = __builtin_amdgcn_exp2f(fmaf(x[i + 1], k2, -m_ref));
         psum += p0 + p1;
-        const bf16x2_v hi = __builtin_convertvector(float2v{p0, p1}, bf16x2_v);
-        const unsigned bits = __builtin_bit_cast(unsigned, hi);
-        const bf16x2_v low = __builtin_convertvector(float2v{p0 - __builtin_bit_cast(float, bits << 16),
-                                                             p1 - __builtin_bit_cast(float, bits & 0xffff0000u)}, bf16x2_v);
-        phi[i >> 3][i & 7] = hi[0];
-        phi[i >> 3][(i & 7) + 1] = hi[1];
-        plo[i >> 3][i & 7] = low[0];
-        plo[i >> 3][(i & 7) + 1] = low[1];
+        float2v rest = {p0, p1};
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {   // one conversion packs two pieces; what it leaves is exact
+          const bf16x2_v piece = __builtin_convertvector(rest, bf16x2_v);
+          const unsigned bits = __builtin_bit_cast(unsigned, piece);
+          rest[0] -= __builtin_bit_cast(float, bits << 16);
+          rest[1] -= __builtin_bit_cast(float, bits & 0xffff0000u);
+          pw[k][i >> 3][i & 7] = piece[0];
+          pw[k][i >> 3][(i & 7) + 1] = piece[1];
+        }
       }
       if (raised || __all(!head || psum <= 4096.0f)) break;
       float top = x[0];
@@ -237,8 +239,8 @@ __global__ __launch_bounds__(64 * GROUP_WAVES, 2) void group_attention_kernel(
 #pragma unroll
       for (int c = 0; c < VT; ++c) {
         const bf16x8_v va = frag_born<32>(V_, col_at, 16 * s2, 32 * c);
-        oacc[c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va, phi[s2], oacc[c], 0, 0, 0);
-        oacc[c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va, plo[s2], oacc[c], 0, 0, 0);
+#pragma unroll
+        for (int k = 0; k < 3; ++k) oacc[c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va, pw[k][s2], oacc[c], 0, 0, 0);
       }
     __builtin_amdgcn_sched_barrier(0);
     if (more) load_values(next, V_);

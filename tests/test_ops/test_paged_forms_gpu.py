@@ -275,3 +275,31 @@ def test_decode_scores_that_rise_and_fall(levels, parts):
 @pytest.mark.parametrize("kw", [dict(window=1024, keep_first=4, slopes=True, gate=True), dict(softcap=5.0, sink=True)])
 def test_decode_tokens_beside_long_portions(counts, starts, H, G, D, Dv, kw):
     _check(counts, starts, H, G, D, Dv, 16, D ** -0.5, **dict(kw))
+
+
+@pytest.mark.parametrize("D", [64, 128])
+def test_decode_weights_are_whole(D):
+    """256 keys of value v_a and 256 of -1, whose weights p differ from head to head and whose sums nearly cancel: 2^-13 of them is
+    left. A weight's error of 2^-18, what two bfloat16 halves leave, would be up to a twentieth of the result; weights of 24 bits,
+    their exponential (2^-22) and the result's own rounding make less than 2^-7 of it."""
+    from colossalai_amd.ops.paged_attention import paged_attention
+
+    heads, n, page = 32, 512, 16
+    batch, pages = _batch([1], [n - 1], page)
+    k, v = torch.zeros(n, heads, D), torch.zeros(n, heads, D)
+    q = torch.zeros(1, heads, D)
+    q[0, :, 3] = 1.0
+    below = -(0.05 + torch.arange(heads) / 50.0).bfloat16().double()      # scores of the second half; those of the first are 0
+    k[n // 2:, :, 3] = below.float()
+    v[n // 2:] = -1.0
+    p = torch.exp(below)
+    v[: n // 2] = p.bfloat16().float()[:, None]
+    for i in range(3):   # the first keys' values bring the sums together
+        gap = (n // 2) * (p * (1 + 2.0 ** -13)) - v[: n // 2, :, 0].double().sum(0)
+        v[i] = (v[i, :, 0].double() + gap).bfloat16().float()[:, None]
+    want = (v[: n // 2, :, 0].double().sum(0) - (n // 2) * p) / ((n // 2) * (1 + p))
+    assert (want.abs() / p).max() < 2.0 ** -12 and want.abs().min() > 0
+    order = batch.block_tables[0].long().cpu()
+    pool = lambda t: t.view(pages, page, heads, D)[torch.argsort(order)].cuda().bfloat16()
+    got = paged_attention(q.cuda().bfloat16(), pool(k), pool(v), batch, 1.0)[0, :, 0].double().cpu()
+    assert ((got - want).abs() <= 2.0 ** -6 * want.abs().max()).all()
