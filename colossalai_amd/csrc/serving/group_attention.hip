@@ -6,7 +6,9 @@
 //   S^T = K Q^T (A = key rows, B = query rows in registers: column = head), O^T = V^T P^T (the float32 weights in the C
 //   layout they were born in, each as three bfloat16 pieces, which hold all of its 24 bits; A = values by transposing reads),
 // so a head is a lane and its half-wave twin. Of the 32 columns the group fills 1 to 16; the products cost a tenth of the time that
-// the tile's 16 KB take to arrive. The next tile's keys are on their way from the moment the scores are
+// the tile's 16 KB take to arrive. Up to 10 heads stand three times in the columns, once for each piece of their weights: one
+// product then does for three (16 x 1024 keys with a cap and a sink, 16 heads on 4 of 128: 17.5 us with three, 16.9 with one). The pieces' sums
+// meet at the end; where the first one's is infinite, it is the result (0 and negative rests of a weight times infinity). The next tile's keys are on their way from the moment the scores are
 // formed, its values from the end of the products.
 // What bounds it: memory beyond about 8 us of dependent loads (position, page table, rows), launch and the end. Against
 // the form with a row in the registers of a few lanes (row_attention.hip), 16 heads on 4 of 128: 16 x 1024 keys with a cap
@@ -28,6 +30,7 @@ namespace {
 constexpr int GROUP_WAVES = 8;
 constexpr size_t GROUP_LDS = 160 * 1024;   // of a CU
 constexpr int GROUP_HEADS = 16;     // most query heads of a kv head: their states must fit into a wave's tile
+constexpr int PIECE_HEADS = 10;     // that stand three times in 32 columns
 typedef __bf16 bf16x2_v __attribute__((ext_vector_type(2)));
 
 // at most N vector memory operations of this wave are on their way; what follows reads what the others brought
@@ -39,7 +42,9 @@ DEV_INLINE void loads_left() {
   __builtin_amdgcn_sched_barrier(0);
 }
 
-template <int DS, int VT>
+__device__ __align__(16) const bf16s no_values[128] = {};   // a key's past the end
+
+template <int DS, int VT, bool COLS>
 __global__ __launch_bounds__(64 * GROUP_WAVES, 2) void group_attention_kernel(
     bf16s* __restrict__ out, const bf16s* __restrict__ q, long q_stride, const bf16s* __restrict__ kpool,
     const bf16s* __restrict__ vpool, const int* __restrict__ block_tables, int bt_stride, const int* __restrict__ tok_seq,
@@ -64,12 +69,13 @@ __global__ __launch_bounds__(64 * GROUP_WAVES, 2) void group_attention_kernel(
   const int pos = positions[n];
   const int* bt = block_tables + (long)tok_seq[n] * bt_stride;
   const int page_mask = (1 << page_shift) - 1;
-  const bool head = col < R;
+  const int piece = COLS ? col / PIECE_HEADS : 0, hcol = col - piece * PIECE_HEADS;   // of the weights, head of the group
+  const bool head = hcol < R;
   bf16x8_v qf[DS];
 #pragma unroll
-  for (int s = 0; s < DS; ++s) qf[s] = ld_g16b(q + n * q_stride + (long)(h0 + min(col, R - 1)) * D + 16 * s + hf * 8);
+  for (int s = 0; s < DS; ++s) qf[s] = ld_g16b(q + n * q_stride + (long)(h0 + min(hcol, R - 1)) * D + 16 * s + hf * 8);
   const bool sloped = slopes != nullptr;
-  float sl2 = sloped ? slopes[h0 + min(col, R - 1)] : 0.0f;
+  float sl2 = sloped ? slopes[h0 + min(hcol, R - 1)] : 0.0f;
 
   // The token's keys: kept first ones, then those from `lo` to its own position
   const int lo = first_visible(pos, window, chunk);
@@ -87,12 +93,16 @@ __global__ __launch_bounds__(64 * GROUP_WAVES, 2) void group_attention_kernel(
   for (int i = threadIdx.x; i < num_pages; i += 64 * GROUP_WAVES)
     pages[i] = bt[i < keep_pages ? i : (w0 >> page_shift) + i - keep_pages];
   __syncthreads();
-  struct Rows { int at[2]; };
+  struct Rows {
+    int at[2];
+    bool past[2];
+  };
   auto lookup = [&](int t) {
     Rows r;
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
-      const int idx = min(t * 32 + i * 16 + lkey, total - 1);       // past the end: the token's own row
+      const int key = t * 32 + i * 16 + lkey, idx = min(key, total - 1);   // past the end: the token's own row
+      r.past[i] = key >= total;
       const int j = idx < n_keep ? idx : lo + (idx - n_keep);
       const int p = idx < n_keep ? j >> page_shift : keep_pages + (j >> page_shift) - (w0 >> page_shift);
       r.at[i] = (pages[p] << page_shift) + (j & page_mask);
@@ -101,6 +111,7 @@ __global__ __launch_bounds__(64 * GROUP_WAVES, 2) void group_attention_kernel(
   };
   const char* kbase = reinterpret_cast<const char*>(kpool + (long)g * D + lch);
   const char* vbase = reinterpret_cast<const char*>(vpool + (long)(g / vrep) * vhead + lch);
+  const char* none = reinterpret_cast<const char*>(no_values + lch);
   const unsigned krs = (unsigned)(G * D) * 2u, vrs = (unsigned)vrow * 2u;   // bytes between neighbouring keys' rows
   auto load_keys = [&](const Rows& r, char* __restrict__ dst) __attribute__((always_inline)) {
 #pragma unroll
@@ -111,10 +122,12 @@ __global__ __launch_bounds__(64 * GROUP_WAVES, 2) void group_attention_kernel(
   };
   auto load_values = [&](const Rows& r, char* __restrict__ dst) __attribute__((always_inline)) {
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < 2; ++i) {
+      const char* at = r.past[i] ? none : vbase + (unsigned long)(unsigned)r.at[i] * vrs;   // a weight of 0 times a value that may be infinite
 #pragma unroll
       for (int c = 0; c < VT; ++c)
-        __builtin_amdgcn_global_load_lds((global_ptr)(vbase + (unsigned long)(unsigned)r.at[i] * vrs + c * 64), (lds_ptr)(dst + (c * 2 + i) * 1024), 16, 0, 0);
+        __builtin_amdgcn_global_load_lds((global_ptr)(at + c * 64), (lds_ptr)(dst + (c * 2 + i) * 1024), 16, 0, 0);
+    }
   };
 
   int t = split * per + wid;
@@ -136,11 +149,15 @@ __global__ __launch_bounds__(64 * GROUP_WAVES, 2) void group_attention_kernel(
   const bool capped = softcap > 0.0f;
   const float inv_cap = capped ? scale / softcap : 0.0f, cap2 = softcap * LOG2E, t2 = capped ? 2.0f * LOG2E * scale / softcap : 0.0f;
   float m = -INFINITY, m_ref = -3.0e38f, l = 0.0f;
-  f32x16 oacc[VT];
+  f32x16 oacc[VT], orest[COLS ? 1 : VT];   // the first pieces' sums apart from the others', or with COLS a piece a column
 #pragma unroll
   for (int t = 0; t < VT; ++t)
 #pragma unroll
-    for (int i = 0; i < 16; ++i) oacc[t][i] = 0.0f;
+    for (int i = 0; i < 16; ++i) {
+      oacc[t][i] = 0.0f;
+      if (!COLS) orest[t][i] = 0.0f;
+    }
+  const float sel[2] = {piece >= 1 ? -1.0f : 0.0f, piece >= 2 ? -1.0f : 0.0f};
   const RowAt row_at(col, hf);
   const ColAt col_at(lane);
   char* keys = tiles + wid * (KT + VTT);
@@ -197,7 +214,7 @@ __global__ __launch_bounds__(64 * GROUP_WAVES, 2) void group_attention_kernel(
 #pragma unroll
       for (int i = 0; i < 16; ++i) x[i] = t * 32 + (i & 3) + 8 * (i >> 2) + 4 * hf < total ? x[i] : -INFINITY;
     }
-    bf16x8_v pw[3][2];
+    bf16x8_v pw[COLS ? 1 : 3][2];
     float psum;
     for (bool raised = false;; raised = true) {
       psum = 0.0f;
@@ -208,12 +225,16 @@ __global__ __launch_bounds__(64 * GROUP_WAVES, 2) void group_attention_kernel(
         float2v rest = {p0, p1};
 #pragma unroll
         for (int k = 0; k < 3; ++k) {   // one conversion packs two pieces; what it leaves is exact
-          const bf16x2_v piece = __builtin_convertvector(rest, bf16x2_v);
-          const unsigned bits = __builtin_bit_cast(unsigned, piece);
-          rest[0] -= __builtin_bit_cast(float, bits << 16);
-          rest[1] -= __builtin_bit_cast(float, bits & 0xffff0000u);
-          pw[k][i >> 3][i & 7] = piece[0];
-          pw[k][i >> 3][(i & 7) + 1] = piece[1];
+          const bf16x2_v two = __builtin_convertvector(rest, bf16x2_v);
+          const unsigned bits = __builtin_bit_cast(unsigned, two);
+          if (!COLS || k == 2) {
+            pw[COLS ? 0 : k][i >> 3][i & 7] = two[0];
+            pw[COLS ? 0 : k][i >> 3][(i & 7) + 1] = two[1];
+          }
+          if (k < 2) {
+            rest[0] = fmaf(__builtin_bit_cast(float, bits << 16), COLS ? sel[k] : -1.0f, rest[0]);
+            rest[1] = fmaf(__builtin_bit_cast(float, bits & 0xffff0000u), COLS ? sel[k] : -1.0f, rest[1]);
+          }
         }
       }
       if (raised || __all(!head || psum <= 4096.0f)) break;
@@ -227,7 +248,10 @@ __global__ __launch_bounds__(64 * GROUP_WAVES, 2) void group_attention_kernel(
 #pragma unroll
       for (int c = 0; c < VT; ++c)
 #pragma unroll
-        for (int i = 0; i < 16; ++i) oacc[c][i] *= corr;
+        for (int i = 0; i < 16; ++i) {
+          oacc[c][i] *= corr;
+          if (!COLS) orest[c][i] *= corr;
+        }
       m = m_new;
       m_ref = m_new == -INFINITY ? -3.0e38f : m_new;
     }
@@ -239,8 +263,11 @@ __global__ __launch_bounds__(64 * GROUP_WAVES, 2) void group_attention_kernel(
 #pragma unroll
       for (int c = 0; c < VT; ++c) {
         const bf16x8_v va = frag_born<32>(V_, col_at, 16 * s2, 32 * c);
-#pragma unroll
-        for (int k = 0; k < 3; ++k) oacc[c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va, pw[k][s2], oacc[c], 0, 0, 0);
+        oacc[c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va, pw[0][s2], oacc[c], 0, 0, 0);
+        if constexpr (!COLS) {
+          orest[c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va, pw[1][s2], orest[c], 0, 0, 0);
+          orest[c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va, pw[2][s2], orest[c], 0, 0, 0);
+        }
       }
     __builtin_amdgcn_sched_barrier(0);
     if (more) load_values(next, V_);
@@ -255,11 +282,12 @@ __global__ __launch_bounds__(64 * GROUP_WAVES, 2) void group_attention_kernel(
     loads_left<2 * VT>();
     tile(t, std::false_type(), first, keys, keys + KT);
   }
-  // The waves' states: [head][2 + Dv] in the wave's own tiles
+  // The waves' states: [head][2 + Dv] in the wave's own tiles, with COLS [piece][head][2 + Dv]
   constexpr int PS = 2 + Dv;
+  auto whole = [](float first, float rest) { return fabsf(first) < INFINITY ? first + rest : first; };
   l += __shfl_xor(l, 32);
-  float* mine = reinterpret_cast<float*>(keys) + col * PS;
-  if (head) {
+  float* mine = reinterpret_cast<float*>(keys) + (piece * R + hcol) * PS;
+  if (head && piece < 3) {
     if (hf == 0) {
       mine[0] = m;
       mine[1] = l;
@@ -267,7 +295,7 @@ __global__ __launch_bounds__(64 * GROUP_WAVES, 2) void group_attention_kernel(
 #pragma unroll
     for (int c = 0; c < VT; ++c)
 #pragma unroll
-      for (int i = 0; i < 16; ++i) mine[2 + c * 32 + (i & 3) + 8 * (i >> 2) + 4 * hf] = oacc[c][i];
+      for (int i = 0; i < 16; ++i) mine[2 + c * 32 + (i & 3) + 8 * (i >> 2) + 4 * hf] = COLS ? oacc[c][i] : whole(oacc[c][i], orest[c][i]);
   }
   __syncthreads();
   constexpr int WS = (KT + VTT) / 4;   // floats between the waves' states
@@ -284,7 +312,8 @@ __global__ __launch_bounds__(64 * GROUP_WAVES, 2) void group_attention_kernel(
       const float mw = states[w * WS + r * PS];
       const float f = mw == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(mw - top);
       ll += states[w * WS + r * PS + 1] * f;     // a wave without keys: 0 * 0
-      o += states[w * WS + r * PS + 2 + dv] * f;
+      const float* sums = states + w * WS + r * PS + 2 + dv;
+      o += (COLS ? whole(sums[0], sums[R * PS] + sums[2 * R * PS]) : sums[0]) * f;
     }
     if (splits > 1) {   // a part without keys has a maximum of -inf
       float* state = ws + ((unit * H + h0 + r) * splits + split) * (long)PS;
@@ -337,9 +366,11 @@ bool launch_group_attention(at::Tensor& out, const at::Tensor& q, const at::Tens
   if (lds > GROUP_LDS) return false;
   at::Tensor ws;
   if (splits > 1) ws = at::empty({units * H * splits * (2 + Dv)}, q.options().dtype(at::kFloat));
+  // every piece's sums of a head must fit into a wave's tile as well
+  const bool cols = R <= PIECE_HEADS && 3 * R * (2 + Dv) * 4 <= (D + Dv) * 64;
 #define GROUP_LAUNCH(DS_, VT_)                                                                                       \
   do {                                                                                                             \
-    auto kernel = group_attention_kernel<DS_, VT_>;                                                                \
+    auto kernel = cols ? group_attention_kernel<DS_, VT_, true> : group_attention_kernel<DS_, VT_, false>;          \
     if (lds > 65536) (void)hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds); \
     hipLaunchKernelGGL(kernel, dim3((unsigned)(units * G * splits)), dim3(64 * GROUP_WAVES), lds, stream(), ptr<bf16s>(out), \
                        ptr<bf16s>(q), (long)q.stride(0), ptr<bf16s>(kpool), ptr<bf16s>(vpool), block_tables.data_ptr<int>(), \

@@ -303,3 +303,31 @@ def test_decode_weights_are_whole(D):
     pool = lambda t: t.view(pages, page, heads, D)[torch.argsort(order)].cuda().bfloat16()
     got = paged_attention(q.cuda().bfloat16(), pool(k), pool(v), batch, 1.0)[0, :, 0].double().cpu()
     assert ((got - want).abs() <= 2.0 ** -6 * want.abs().max()).all()
+
+
+@pytest.mark.parametrize("H,G,D,Dv", [(4, 2, 128, 128), (8, 1, 64, 128), (16, 1, 64, 64), (2, 2, 64, 64)])
+@pytest.mark.parametrize("start", [300, 335, 3000])
+@pytest.mark.parametrize("kw", [{}, dict(window=290, keep_first=3), dict(sink=True, softcap=5.0)])
+def test_decode_values_that_are_infinite(H, G, D, Dv, start, kw):
+    """A visible value of inf is the result of its channel, one of each sign or a NaN give NaN; the other channels, and keys that are
+    not seen, keep theirs."""
+    from colossalai_amd.ops.paged_attention import paged_attention
+
+    torch.manual_seed(9)
+    batch, pages = _batch([1, 1], [start, start - 7], 16)
+    k, v = torch.randn(pages, 16, G, D, device="cuda").bfloat16(), torch.randn(pages, 16, G, Dv, device="cuda").bfloat16()
+    q = torch.randn(2, H, D, device="cuda").bfloat16()
+    want = paged_attention(q, k, v, batch, 0.1, **kw)
+    row = lambda pos: (batch.block_tables[0, pos // 16].long(), pos % 16)
+    inf = float("inf")
+    for pos, channel, value in [(start, 1, inf), (start - 40, 2, -inf), (start - 280, 3, inf), (start - 280, 4, inf),
+                                (start, 4, -inf), (start - 1, 5, float("nan"))]:
+        v[row(pos)][G - 1, channel] = value
+    hidden = row(start + 1 if (start + 1) % 16 else 5)   # behind the token, or ahead of the window if there is one
+    if (start + 1) % 16 or "window" in kw:
+        v[hidden][:, 6] = inf
+    got = paged_attention(q, k, v, batch, 0.1, **kw)
+    last = got[0, -1]
+    assert last[1] == inf and last[2] == -inf and last[3] == inf and last[4].isnan() and last[5].isnan()
+    want[0, (G - 1) * (H // G):, 1:6] = got[0, (G - 1) * (H // G):, 1:6]
+    torch.testing.assert_close(got, want, rtol=0, atol=0, equal_nan=True)
