@@ -22,7 +22,7 @@ struct Linear : torch::autograd::Function<Linear> {
     if (x.size(-1) != weight.size(1) || weight.dim() != 2) return at::linear(x, weight);   // which says what is wrong
     auto sizes = x.sizes().vec();
     sizes.back() = weight.size(0);
-    return multiply(x.reshape({-1, x.size(-1)}), weight, false).view(sizes);
+    return at::_unsafe_view(multiply(x.reshape({-1, x.size(-1)}), weight, false), sizes);   // no view, which may not be changed in place
   }
   static torch::autograd::variable_list backward(torch::autograd::AutogradContext* ctx, torch::autograd::variable_list grads) {
     const auto saved = ctx->get_saved_variables();

@@ -93,6 +93,24 @@ def test_layer_is_the_builtin_one_on_the_cpu(shape):
 
 
 @needs_extension
+@pytest.mark.parametrize("shape", [(5, 16), (2, 3, 16)])
+@pytest.mark.parametrize("change", [lambda y: y.add_(1.0), lambda y: y[..., :4].mul_(2.0), lambda y: y.relu_()])
+def test_result_may_be_changed_in_place(shape, change):
+    torch.manual_seed(4)
+    x, w, g = torch.randn(*shape), torch.randn(24, 16), torch.randn(*shape[:-1], 24)
+
+    def changed(lin):
+        def call(x, w):
+            y = lin(x, w)
+            change(y)
+            return y
+        return call
+
+    for a, b in zip(_step(changed(kernels().linear), x, w, g), _step(changed(F.linear), x, w, g)):
+        torch.testing.assert_close(a, b)
+
+
+@needs_extension
 def test_layer_under_transforms():
     torch.manual_seed(2)
     x, w = torch.randn(4, 16, dtype=torch.float64), torch.randn(8, 16, dtype=torch.float64)
