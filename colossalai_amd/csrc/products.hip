@@ -26,6 +26,7 @@
 #include <algorithm>
 
 #include "lds_tiles.h"
+#include "plain.h"
 
 namespace cai {
 
@@ -347,8 +348,9 @@ at::Tensor run(const at::Tensor& p, const at::Tensor& q, Plan plan, const c10::o
   return out;
 }
 
+// bfloat16 matrices on one device that nothing watches: a mode that counts or rewrites operations is to see the library's products
 bool bf16_pair(const at::Tensor& p, const at::Tensor& q) {
-  return p.is_cuda() && q.device() == p.device() && p.scalar_type() == at::kBFloat16 && q.scalar_type() == at::kBFloat16
+  return plain(p) && plain(q) && p.is_cuda() && q.device() == p.device() && p.scalar_type() == at::kBFloat16 && q.scalar_type() == at::kBFloat16
       && p.dim() == 2 && q.dim() == 2 && p.size(0) < (1L << 30) && p.numel() > 0 && q.numel() > 0;
 }
 

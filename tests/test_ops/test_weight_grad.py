@@ -160,3 +160,19 @@ def test_projection_takes_the_native_form_only_for_plain_layers():
     layer.weight.requires_grad_(False)
     project(layer, x).backward(g)
     assert layer.weight.grad is None and x.grad is not None
+
+
+@pytest.mark.gpu
+def test_a_mode_that_counts_operations_sees_every_product():
+    from torch.utils.flop_counter import FlopCounterMode
+
+    from colossalai_amd.ops.fused_ce import fused_linear_cross_entropy
+
+    x, w = torch.randn(96, 64, device="cuda").to(BF16).requires_grad_(), torch.randn(136, 64, device="cuda").to(BF16).requires_grad_()
+    labels = torch.arange(96, device="cuda")
+    layer = nn.Linear(64, 136, bias=False, device="cuda", dtype=BF16)
+    for call, rows in ((lambda: fused_linear_cross_entropy(x, w, labels), 3 * 96), (lambda: project(layer, x).sum(), 3 * 96),
+                       (lambda: fused_linear_cross_entropy(x, w, labels, chunk_size=20), 3 * 96 + 16)):   # 16 rows' logits twice
+        with FlopCounterMode(display=False) as counter:
+            call().backward()
+        assert counter.get_total_flops() == 2 * rows * 64 * 136
