@@ -368,6 +368,11 @@ at::Tensor weight_grad(const at::Tensor& dy, const at::Tensor& x, const c10::opt
   if (add)
     TORCH_CHECK(add->device() == dy.device() && add->scalar_type() == at::kFloat && add->is_contiguous() && add->dim() == 2
                 && add->size(0) == dy.size(1) && add->size(1) == x.size(1), "weight_grad: add is not a float32 [M, N] matrix");
+  // the kernels read and write sums 16 bytes at a time
+  if (add && reinterpret_cast<uintptr_t>(add->data_ptr()) % 16 != 0) {
+    const at::Tensor r = weight_grad(dy, x, c10::nullopt, true);
+    return keep ? add->add_(r) : at::add(*add, r).to(dy.scalar_type());
+  }
   if (!weight_grad_serves(dy, x)) {
     at::Tensor r = at::mm(dy.t(), x);
     if (add) r = keep ? add->add_(r) : at::add(*add, r);

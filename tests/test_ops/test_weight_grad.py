@@ -43,6 +43,27 @@ def test_against_64_bits(M, N, K):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(128, 136, 31), (264, 248, 300), (768, 768, 4100), (12, 20, 33)])
+@pytest.mark.parametrize("offset", [1, 2, 3, 5])
+@pytest.mark.parametrize("keep", [False, True])
+def test_sums_at_odd_addresses(M, N, K, offset, keep):
+    torch.manual_seed(offset)
+    dy, x = (torch.randn(K, n, device="cuda").to(BF16) for n in (M, N))
+    flat = torch.randn(M * N + 16, device="cuda")
+    add = flat[offset: offset + M * N].view(M, N)
+    before = flat.clone()
+    got = kernels().weight_grad(dy, x, add, keep)
+    if keep:
+        assert got.data_ptr() == add.data_ptr()
+    # sizes that the library multiplies round the product to bfloat16 before it is added
+    wide = 0 if M % 8 == 0 else (dy.double().t() @ x.double()).abs() * 2.0 ** -8
+    ref = before[offset: offset + M * N].view(M, N).double() + dy.double().t() @ x.double()
+    size = before.abs().max() + dy.double().abs().t() @ x.double().abs()
+    assert ((got.double() - ref).abs() <= size * (K + 2) * 2.0 ** -24 + wide + (0 if keep else ref.abs() * 2.0 ** -8 + 1e-30)).all()
+    assert torch.equal(flat[:offset], before[:offset]) and torch.equal(flat[offset + M * N:], before[offset + M * N:])
+
+
+@pytest.mark.gpu
 def test_strides_and_sizes_of_other_forms():
     torch.manual_seed(0)
     wide = torch.randn(300, 1000, device="cuda").to(BF16)
