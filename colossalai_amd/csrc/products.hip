@@ -16,7 +16,7 @@
 //   22016, 4096, 16384   2785 -> 2214     4096, 11008, 16384   1536 -> 1132     4096, 4096, 16384   470 -> 404
 //   32000, 4096, 4096     952 -> 859      32000, 768, 4096      223 -> 191      4096, 768, 8192      84 -> 61
 //   768, 2048, 8192        65 -> 38       768, 768, 8192         49 -> 22       2048, 512, 512       21 -> 10
-// Small others, back to back (the library's call takes the host 19 to 20 us, its kernels 8 to 11):
+// Small others, back to back (the library's call takes the host 19 to 20 us, its kernels 5 to 11):
 //   x W^T: 512, 1536, 512   19.2 -> 9.0   512, 512, 1024   19.7 -> 11.4     dy W: 512, 512, 2048   19.2 -> 13.9
 // Large ones stay with the library: 16384, 12288, 4096   1080 us there, 1468 here; dy W 16384, 4096, 12288   1224, 1377.
 #include <torch/extension.h>
@@ -277,16 +277,17 @@ struct Plan {
   double us;
 };
 
-// Tile size and parts by the time that they should take. A round of blocks over the 256 CUs takes a step in 0.79 us with 256 x 256 tiles
-// (1.36 PFLOP/s) and in 0.25 us with 128 x 128 ones (1.07; two blocks share a CU, each then at half the speed), 5 us
-// around its steps; what is left after whole rounds of tiles may be cut into parts of at least 256 contracted indices, whose sums
-// travel at about 5 TB/s both ways and take another launch. Tiles of 256 x 128 take 0.36 us as long as one round is all; over
-// several the clock falls, and they are no better than 128 x 128. A change has to promise 2 %. Measured, weight
+// Tile size and parts by the time that they should take. A round of blocks over the 256 CUs takes a step in 0.76 us with 256 x 256 tiles
+// (1.41 PFLOP/s) and in 0.25 us with 128 x 128 ones (1.07; two blocks share a CU, each then at half the speed), 14 and 5 us
+// around its steps (the first loads, the stores); what is left after whole rounds of tiles may be cut into parts of at least 256
+// contracted indices, whose sums travel at about 5 TB/s both ways and take another launch. Tiles of 256 x 128 take 0.36 us and 9 around them as long as one round
+// is all; over several the clock falls, and they are no better than 128 x 128. A change has to promise 2 %. Measured, weight
 // gradients, 256 x 256 whole / cut, 256 x 128 cut, 128 x 128 whole / cut, us: 22016 x 4096 x 16384: 2370 / 2214, 2731, -;
 // 4096 x 11008 x 16384: 1132 / 1181, -, 1927 / 1656; 4096 x 768 x 8192: 140 / 63, 61, 69 / 66; 768 x 2048 x 8192: 146 / 44, 38, 68 / 39;
 // 768 x 768 x 8192: 138 / 31, 25, 62 / 22; 512 x 512 x 512: 19 / 18, 14, 8.3 / 10.5.
 Plan plan(long M, long N, long K, bool small_only) {
-  struct { int tm, tn; double step; long slots; bool one_round; } forms[] = {{256, 256, 0.79, 256, false}, {256, 128, 0.36, 256, true}, {128, 128, 0.25, 512, false}};
+  struct { int tm, tn; double step, around; long slots; bool one_round; } forms[] = {
+      {256, 256, 0.76, 14.0, 256, false}, {256, 128, 0.36, 9.0, 256, true}, {128, 128, 0.25, 5.0, 512, false}};
   Plan best{0, 0, 0, 1, 0.0};
   for (const auto& form : forms) {
     if (small_only && form.tm != 128) continue;
@@ -295,7 +296,7 @@ Plan plan(long M, long N, long K, bool small_only) {
     auto take = [&](long full, long parts, double us) {
       if (best.tm == 0 || us < 0.98 * best.us) best = Plan{form.tm, form.tn, (int)full, (int)parts, us};
     };
-    auto round = [&](long blocks, long n) { return (double)((blocks + 255) / 256) * (n * form.step + 5.0); };
+    auto round = [&](long blocks, long n) { return (double)((blocks + 255) / 256) * (n * form.step + form.around); };
     take(tiles, 1, round(tiles, steps));
     const long full = tiles / form.slots * form.slots, rest = tiles - full;
     for (long p = 2; rest && p * rest <= (form.one_round ? 256 : 512) && p * 8 <= steps; ++p)
@@ -356,7 +357,7 @@ bool bf16_pair(const at::Tensor& p, const at::Tensor& q) {
 
 }  // namespace pr
 
-// what the kernel multiplies; everything else takes the library's product
+// what the kernel can multiply; everything else takes the library's product
 bool weight_grad_serves(const at::Tensor& dy, const at::Tensor& x) {
   const long most = 1L << 22;
   return pr::bf16_pair(dy, x) && dy.size(0) == x.size(0) && dy.size(1) <= most && x.size(1) <= most && dy.size(1) % 8 == 0
@@ -373,17 +374,25 @@ at::Tensor weight_grad(const at::Tensor& dy, const at::Tensor& x, const c10::opt
     const at::Tensor r = weight_grad(dy, x, c10::nullopt, true);
     return keep ? add->add_(r) : at::add(*add, r).to(dy.scalar_type());
   }
-  if (!weight_grad_serves(dy, x)) {
+  const bool serves = weight_grad_serves(dy, x);
+  const pr::Plan plan = serves ? pr::plan(dy.size(1), x.size(1), dy.size(0), false) : pr::Plan{};
+  // Over few tokens storing the result is most of it, which the library does faster: 22016 x 4096 over 64, 256, 512, 1024 and 2048
+  // tokens 63, 103, 126, 213 and 404 us there, 112, 143, 176, 241 and 373 here; 4096 x 4096: 12, 18, 26, 40 and 71 there, 23, 27, 33,
+  // 45 and 70 here. It multiplies those, unless the host is what a call waits for (see multiply); a float32 result it does not have.
+  if (!serves || (!add && !keep && dy.size(0) < 2048 && plan.us > 14.0)) {
     at::Tensor r = at::mm(dy.t(), x);
     if (add) r = keep ? add->add_(r) : at::add(*add, r);
     return r.to(keep ? at::kFloat : dy.scalar_type());
   }
   return pr::run<true, true>(pr::loadable(dy) ? dy : dy.clone(at::MemoryFormat::Contiguous),
-                             pr::loadable(x) ? x : x.clone(at::MemoryFormat::Contiguous), pr::plan(dy.size(1), x.size(1), dy.size(0), false), add, keep);
+                             pr::loadable(x) ? x : x.clone(at::MemoryFormat::Contiguous), plan, add, keep);
 }
 
-// x [M, K] times w [N, K]^T, or with `slow` times w [K, N]. Products that should take at most 14 us, about what the
-// library's call takes the host in a chain of them, are formed here; where the time is known, 512 x 512 x 2048 is the longest.
+// x [M, K] times w [N, K]^T, or with `slow` times w [K, N]. Products that should take at most 14 us are formed here, because the host
+// takes 19 to 20 us for the library's call and 9 for this one, and a chain of such products waits for it. On the device they
+// are no faster, 6 to 13 us where the library's kernels take 4 to 11. Steps of two layers, us, library and here: width 512, 512 tokens 1320
+// and 1050 (kernels 490 and 525); 1024, 512 tokens 1130 and 900; where the device is the bound nothing shows: 512, 4096 tokens 1316 and
+// 1301, 1024, 2048 tokens 1343 and 1347.
 at::Tensor multiply(const at::Tensor& x, const at::Tensor& w, bool slow) {
   if (pr::bf16_pair(x, w) && x.size(1) == w.size(slow ? 0 : 1) && x.size(1) % pr::KT == 0 && w.size(slow ? 1 : 0) % 8 == 0
       && pr::loadable(x) && pr::loadable(w)) {

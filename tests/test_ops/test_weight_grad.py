@@ -63,6 +63,27 @@ def test_sums_at_odd_addresses(M, N, K, offset, keep):
     assert torch.equal(flat[:offset], before[:offset]) and torch.equal(flat[offset + M * N:], before[offset + M * N:])
 
 
+def _formed_here(call):
+    from torch.profiler import ProfilerActivity, profile
+
+    with profile(activities=[ProfilerActivity.CUDA]) as seen:
+        call()
+        torch.cuda.synchronize()
+    return any("product_kernel" in e.key for e in seen.key_averages())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K,here", [(4096, 4096, 64, False), (4096, 2048, 1024, False), (2304, 4096, 2047, False),
+                                        (2304, 4096, 2048, True), (512, 512, 512, True)])
+def test_few_tokens_are_the_librarys(M, N, K, here):
+    """Storing is most of such a product, which the library does faster; small ones are the host's time, and a float32 sum is formed here."""
+    torch.manual_seed(K)
+    dy, x = (torch.randn(K, n, device="cuda").to(BF16) for n in (M, N))
+    _close(kernels().weight_grad(dy, x), dy, x)
+    assert _formed_here(lambda: kernels().weight_grad(dy, x)) == here
+    assert _formed_here(lambda: kernels().weight_grad(dy, x, None, True))
+
+
 @pytest.mark.gpu
 def test_strides_and_sizes_of_other_forms():
     torch.manual_seed(0)
