@@ -4,11 +4,12 @@ Computes ``CE(hidden @ W^T, labels)`` without ever materializing the full
 [N, V] logits: tokens are processed in chunks; backward recomputes each
 chunk's logits and feeds the dW/dh GEMMs directly. At the flagship bench
 size (147k tokens x 32k vocab) this replaces a ~50 GB fp32 logits+softmax
-footprint with transient chunk buffers — pure HBM savings.
+footprint with chunk buffers.
 On the GPU the first rows, four chunks of at most 1 GiB of logits, are one chunk whose bfloat16 logits the
 backward still finds: the activations of a decoder layer for as many tokens are larger, and forming
 them again was 5 to 7 % of a training step of 8192 to 16384 tokens (16380 x 32000 at width 4096: 2.9 ms of 51;
-its products over all rows at once take 6.9 ms for 7.7 in four chunks).
+its products over all rows at once take 6.9 ms for 7.7 in four chunks). They are held from the forward to the backward,
+which takes as much again for their gradient; ``kept_bytes`` bounds them, or with 0 leaves one chunk at a time.
 
 GEMMs run through hipBLASLt (torch.matmul), the weight gradient and small products in bfloat16
 through csrc/products.hip; softmax math is fp32. In bfloat16 on
@@ -37,19 +38,20 @@ def _bf16_products(t: torch.Tensor) -> bool:
 _KEPT_CHUNKS, _KEPT_BYTES = 4, 1 << 30
 
 
-def _spans(rows: int, vocab: int, chunk_size: int, keep: bool):
+def _spans(rows: int, vocab: int, chunk_size: int, keep: bool, kept_bytes: Optional[int] = None):
     """How many rows' bfloat16 logits stay for the backward, and the spans of rows that are worked on: those rows, if
     any, then chunks."""
     kept = 0
     if keep:
-        fit = min(_KEPT_CHUNKS * chunk_size, _KEPT_BYTES // (2 * max(vocab, 1)))
+        most = _KEPT_BYTES if kept_bytes is None else max(kept_bytes, 0)
+        fit = min(_KEPT_CHUNKS * chunk_size, most // (2 * max(vocab, 1)))
         kept = rows if rows <= fit else fit // chunk_size * chunk_size
     return kept, [(0, kept)] * (kept > 0) + [(s, min(s + chunk_size, rows)) for s in range(kept, rows, chunk_size)]
 
 
 class _FusedLinearCE(torch.autograd.Function):
     @staticmethod
-    def forward(ctx, hidden, weight, labels, ignore_index, chunk_size, recorded=False):
+    def forward(ctx, hidden, weight, labels, ignore_index, chunk_size, recorded=False, kept_bytes=None):
         # hidden [N, H] (bf16/fp32), weight [V, H], labels [N]
         N = hidden.shape[0]
         ctx.chunk_size = chunk_size
@@ -60,9 +62,9 @@ class _FusedLinearCE(torch.autograd.Function):
             labels = labels.contiguous()
             lse = torch.empty(N, dtype=torch.float32, device=hidden.device)
             nll = torch.empty_like(lse)
-            ctx.kept, spans = _spans(N, weight.shape[0], chunk_size, recorded and hidden.is_cuda)
+            ctx.kept, ctx.spans = _spans(N, weight.shape[0], chunk_size, recorded and hidden.is_cuda, kept_bytes)
             kept = []
-            for s, e in spans:
+            for s, e in ctx.spans:
                 logits = multiply(hidden[s:e], weight)
                 kernels().ce_fwd(logits, labels[s:e], ignore_index, lse[s:e], nll[s:e])
                 if e <= ctx.kept:
@@ -113,7 +115,7 @@ class _FusedLinearCE(torch.autograd.Function):
             ds = ds.to(hidden.dtype)
             dh[s:e] = ds @ weight
             dw += (ds.t() @ hidden[s:e]).float()
-        return dh, dw.to(weight.dtype), None, None, None, None
+        return dh, dw.to(weight.dtype), None, None, None, None, None
 
 
 def _backward_hip(ctx, grad_out):
@@ -122,7 +124,7 @@ def _backward_hip(ctx, grad_out):
     grad = grad_out.float()
     dh = torch.empty_like(hidden)
     dw = None
-    for s, e in _spans(N, weight.shape[0], ctx.chunk_size, bool(kept))[1]:
+    for s, e in ctx.spans:
         if e <= ctx.kept:
             ds = torch.empty_like(kept[0])  # not in the logits' place: the graph may be gone through again
             kernels().ce_bwd(kept[0], labels[s:e], ctx.ignore_index, lse[s:e], grad, loss, ds)
@@ -137,7 +139,7 @@ def _backward_hip(ctx, grad_out):
         dw = weight_grad(ds, hidden[s:e], dw, e < N)
     if dw is None:
         dw = torch.zeros_like(weight)
-    return dh, dw.to(weight.dtype), None, None, None, None
+    return dh, dw.to(weight.dtype), None, None, None, None, None
 
 
 def fused_linear_cross_entropy(
@@ -146,8 +148,14 @@ def fused_linear_cross_entropy(
     labels: torch.Tensor,
     ignore_index: int = -100,
     chunk_size: int = 4096,
+    kept_bytes: Optional[int] = None,
 ) -> torch.Tensor:
-    """hidden [.., H], weight [V, H], labels [..] -> mean CE over valid tokens."""
+    """hidden [.., H], weight [V, H], labels [..] -> mean CE over valid tokens.
+
+    Memory beyond the inputs and gradients, in bfloat16 on the GPU: the logits of ``chunk_size`` rows at a time, and, where a
+    gradient is recorded, those of the first rows (four chunks, ``kept_bytes`` at most, 1 GiB if it is None) from the
+    forward to the backward and as much again during the backward. Losses that are summed before one backward hold theirs
+    each. ``kept_bytes=0`` keeps none: the backward forms every chunk's logits again."""
     H = hidden.shape[-1]
     recorded = torch.is_grad_enabled() and (hidden.requires_grad or weight.requires_grad)
-    return _FusedLinearCE.apply(hidden.reshape(-1, H), weight, labels.reshape(-1), ignore_index, chunk_size, recorded)
+    return _FusedLinearCE.apply(hidden.reshape(-1, H), weight, labels.reshape(-1), ignore_index, chunk_size, recorded, kept_bytes)

@@ -209,3 +209,28 @@ def test_linear_cross_entropy_with_kept_logits(monkeypatch, N, V, chunk, kept_by
         assert _rel(got, ref) < 2 * ROUND * (top + 1)
     with torch.no_grad():
         assert abs(fused_ce.fused_linear_cross_entropy(hidden, weight, labels, chunk_size=chunk).item() - want.item()) < 2 * ROUND * top
+
+
+@pytest.mark.parametrize("kept_bytes,chunks", [(0, 0), (1 << 24, 2), (None, 4)])
+def test_memory_of_kept_logits(kept_bytes, chunks):
+    """What a loss holds until its backward, and the backward's peak, are bounded by what the caller allows."""
+    from colossalai_amd.ops.fused_ce import fused_linear_cross_entropy
+
+    N, V, H, chunk = 8192, 4096, 64, 1024
+    a_chunk = chunk * V * 2
+    torch.manual_seed(6)
+    hidden = torch.randn(N, H, device="cuda").bfloat16().requires_grad_()
+    weight = (0.2 * torch.randn(V, H, device="cuda")).bfloat16().requires_grad_()
+    labels = torch.randint(0, V, (N,), device="cuda")
+    want = torch.autograd.grad(fused_linear_cross_entropy(hidden, weight, labels), (hidden, weight))
+    torch.cuda.synchronize()
+    before = torch.cuda.memory_allocated()
+    loss = fused_linear_cross_entropy(hidden, weight, labels, chunk_size=chunk, kept_bytes=kept_bytes)
+    few = 4 << 20   # statistics, gradients and the sums of the weight's
+    assert torch.cuda.memory_allocated() - before <= chunks * a_chunk + few
+    torch.cuda.reset_peak_memory_stats()
+    got = torch.autograd.grad(loss, (hidden, weight))
+    # the kept logits and their gradient, and two chunks: one is let go when the next is formed
+    assert torch.cuda.max_memory_allocated() - before <= (2 * chunks + 2) * a_chunk + few
+    for a, b in zip(got, want):
+        assert _rel(a, b) < 2 * ROUND
