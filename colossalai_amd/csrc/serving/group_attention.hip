@@ -7,7 +7,7 @@
 //   layout they were born in, each as three bfloat16 pieces, which hold all of its 24 bits; A = values by transposing reads),
 // so a head is a lane and its half-wave twin. Of the 32 columns the group fills 1 to 16; the products cost a tenth of the time that
 // the tile's 16 KB take to arrive. Up to 10 heads stand three times in the columns, once for each piece of their weights: one
-// product then does for three (16 x 1024 keys with a cap and a sink, 16 heads on 4 of 128: 17.5 us with three, 16.9 with one). The pieces' sums
+// product then does for three (16 x 1024 keys with a cap and a sink, 16 heads on 4 of 128: 17.5 us with three, 16.6 with one). The pieces' sums
 // meet at the end; where the first one's is infinite, it is the result (0 and negative rests of a weight times infinity). The next tile's keys are on their way from the moment the scores are
 // formed, its values from the end of the products.
 // What bounds it: memory beyond about 8 us of dependent loads (position, page table, rows), launch and the end. Against
@@ -32,6 +32,11 @@ constexpr size_t GROUP_LDS = 160 * 1024;   // of a CU
 constexpr int GROUP_HEADS = 16;     // most query heads of a kv head: their states must fit into a wave's tile
 constexpr int PIECE_HEADS = 10;     // that stand three times in 32 columns
 typedef __bf16 bf16x2_v __attribute__((ext_vector_type(2)));
+
+DEV_INLINE float rounded_product(float a, float b) {
+#pragma clang fp contract(off)
+  return a * b;
+}
 
 // at most N vector memory operations of this wave are on their way; what follows reads what the others brought
 template <int N>
@@ -130,7 +135,8 @@ __global__ __launch_bounds__(64 * GROUP_WAVES, 2) void group_attention_kernel(
     }
   };
 
-  int t = split * per + wid;
+  const int t0 = split * per + wid;
+  int t = t0;
   Rows first;
   if (t < last) {
     first = lookup(t);
@@ -144,7 +150,7 @@ __global__ __launch_bounds__(64 * GROUP_WAVES, 2) void group_attention_kernel(
     scale = -scale;
   }
   // Scores in the base-2 domain; the reference m is raised only where a tile's sum shows that it must be, as in the prompt
-  // portions' kernel.
+  // portions' kernel, and in the wave's first tile, which has a key that counts.
   const float c1 = scale * LOG2E < 1e-30f ? 1e-30f : scale * LOG2E;   // NaN stays
   const bool capped = softcap > 0.0f;
   const float inv_cap = capped ? scale / softcap : 0.0f, cap2 = softcap * LOG2E, t2 = capped ? 2.0f * LOG2E * scale / softcap : 0.0f;
@@ -200,16 +206,19 @@ __global__ __launch_bounds__(64 * GROUP_WAVES, 2) void group_attention_kernel(
         }
       }
     }
-    const float k1 = capped ? 1.0f : c1;
+    // rounded once for the weights and the largest of them: fused into the difference below, a score of 4e9 would miss itself by 2^8
+    if (!capped) {
+#pragma unroll
+      for (int i = 0; i < 16; ++i) x[i] = rounded_product(x[i], c1);
+    }
     if (sloped) {
 #pragma unroll
       for (int i = 0; i < 16; ++i) {
         const int idx = t * 32 + (i & 3) + 8 * (i >> 2) + 4 * hf;
         const int j = idx < n_keep ? idx : lo + (idx - n_keep);
-        x[i] = x[i] * k1 - sl2 * (float)(pos - j);
+        x[i] = x[i] - sl2 * (float)(pos - j);
       }
     }
-    const float k2 = sloped ? 1.0f : k1;
     if (t * 32 + 32 > total) {
 #pragma unroll
       for (int i = 0; i < 16; ++i) x[i] = t * 32 + (i & 3) + 8 * (i >> 2) + 4 * hf < total ? x[i] : -INFINITY;
@@ -220,7 +229,7 @@ __global__ __launch_bounds__(64 * GROUP_WAVES, 2) void group_attention_kernel(
       psum = 0.0f;
 #pragma unroll
       for (int i = 0; i < 16; i += 2) {
-        const float p0 = __builtin_amdgcn_exp2f(fmaf(x[i], k2, -m_ref)), p1 = __builtin_amdgcn_exp2f(fmaf(x[i + 1], k2, -m_ref));
+        const float p0 = __builtin_amdgcn_exp2f(x[i] - m_ref), p1 = __builtin_amdgcn_exp2f(x[i + 1] - m_ref);
         psum += p0 + p1;
         float2v rest = {p0, p1};
 #pragma unroll
@@ -237,12 +246,12 @@ __global__ __launch_bounds__(64 * GROUP_WAVES, 2) void group_attention_kernel(
           }
         }
       }
-      if (raised || __all(!head || psum <= 4096.0f)) break;
+      if (raised || (t != t0 && __all(!head || psum <= 4096.0f))) break;
       float top = x[0];
 #pragma unroll
       for (int i = 1; i < 16; ++i) top = fmaxf(top, x[i]);
       top = fmaxf(top, __shfl_xor(top, 32));
-      const float m_new = fmaxf(m, top == -INFINITY ? -INFINITY : top * k2);
+      const float m_new = fmaxf(m, top);
       const float corr = m == -INFINITY ? 1.0f : __builtin_amdgcn_exp2f(m - m_new);   // nothing accumulated: nothing to rescale
       l *= corr;
 #pragma unroll

@@ -331,3 +331,26 @@ def test_decode_values_that_are_infinite(H, G, D, Dv, start, kw):
     assert last[1] == inf and last[2] == -inf and last[3] == inf and last[4].isnan() and last[5].isnan()
     want[0, (G - 1) * (H // G):, 1:6] = got[0, (G - 1) * (H // G):, 1:6]
     torch.testing.assert_close(got, want, rtol=0, atol=0, equal_nan=True)
+
+
+@pytest.mark.parametrize("start", [100, 299, 3000])
+@pytest.mark.parametrize("size", [1.2e19, 3e9, -1.5e10])
+@pytest.mark.parametrize("kw", [{}, dict(window=290), dict(slopes=True)])
+def test_decode_scores_of_any_size(start, size, kw):
+    """Equal scores as large as float32 holds them (-3.2e38 in base 2), or so large that a rounding of theirs is more than the exponential
+    can take: a token is the mean of the values that it sees."""
+    from colossalai_amd.ops.paged_attention import paged_attention, paged_attention_ref
+
+    torch.manual_seed(10)
+    batch, pages = _batch([1], [start], 16)
+    q, k = torch.zeros(1, 4, 64, device="cuda"), torch.zeros(pages, 16, 2, 64, device="cuda")
+    q[..., 0] = 2.0 ** 64 if size > 1e15 else 1.0
+    k[..., 0] = -size
+    v = torch.randn(pages, 16, 2, 64, device="cuda").bfloat16()
+    kw = dict(kw)
+    if kw.pop("slopes", False):
+        kw["slopes"] = torch.full((4,), 2.0 ** -60, device="cuda")   # nothing beside such a score
+    got = paged_attention(q.bfloat16(), k.bfloat16(), v, batch, 1.0, **kw)
+    kw.setdefault("window", 0)
+    want = paged_attention_ref(q * 0, k, v.float(), batch, 1.0, **kw)   # equal scores, of any size
+    assert (got.double() - want.double()).norm() / want.double().norm() < BOUND
