@@ -264,3 +264,17 @@ def test_inputs_that_tiles_cannot_be_loaded_from_as_they_lie(place, packed):
             assert a.float().abs().max() < 2.0 ** -9 * 4 * 4 * (6 if name == "dk" else 1)
         else:
             _near(a, b, name)
+
+
+def test_a_score_of_nan_is_not_lost():
+    """The forward looks at a tile's sum to see whether its reference must be raised; NaN makes the rows that meet it NaN."""
+    from colossalai_amd.ops import flash_attention
+
+    q, k, v, _ = _inputs(1, 300, 4, 2, 64)
+    k[0, 200, 1, 5] = float("nan")     # key head 1, seen from row 200 on
+    q[0, 100, 0, 3] = float("nan")
+    bad = flash_attention(q, k, v, causal=True)[0].isnan()
+    want = torch.zeros_like(bad)
+    want[200:, 2:] = True
+    want[100, 0] = True
+    assert torch.equal(bad, want)

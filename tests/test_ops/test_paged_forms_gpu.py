@@ -354,3 +354,59 @@ def test_decode_scores_of_any_size(start, size, kw):
     kw.setdefault("window", 0)
     want = paged_attention_ref(q * 0, k, v.float(), batch, 1.0, **kw)   # equal scores, of any size
     assert (got.double() - want.double()).norm() / want.double().norm() < BOUND
+
+
+@pytest.mark.parametrize("start", [299, 3000])
+@pytest.mark.parametrize("H,D", [(4, 64), (32, 128)])
+@pytest.mark.parametrize("kw", [{}, dict(softcap=5.0), dict(softcap=5.0, sink=True), dict(sink_logits=True), dict(slopes=True, window=280)])
+def test_decode_nan_stays_nan(start, H, D, kw):
+    """As test_nan_stays_nan, over more keys than the form for short contexts takes, whole and in parts: a query, a key that one wave
+    of many meets, a slope, and a scale of NaN."""
+    from colossalai_amd.ops.paged_attention import distance_slopes, paged_attention
+
+    torch.manual_seed(4)
+    batch, pages = _batch([1, 1], [start, start - 20], 16)
+    k, v = (torch.randn(pages, 16, 2, D, device="cuda").bfloat16() for _ in range(2))
+    q = torch.randn(2, H, D, device="cuda").bfloat16()
+    kw = dict(kw)
+    if kw.pop("sink_logits", False):
+        kw["sink_logits"] = torch.randn(H, device="cuda")
+    if kw.pop("slopes", False):
+        kw["slopes"] = distance_slopes(H, "cuda")
+        kw["slopes"][1] = float("nan")
+    clean = paged_attention(q, k, v, batch, 1.0, **kw)
+    q[1, 0, 5] = float("nan")
+    k[batch.block_tables[0, (start - 200) // 16], (start - 200) % 16, 1, 7] = float("nan")
+    got = paged_attention(q, k, v, batch, 1.0, **kw)
+    bad = torch.zeros(2, H, dtype=torch.bool, device="cuda")
+    bad[1, 0] = True
+    bad[0, H // 2:] = True
+    if "slopes" in kw:
+        bad[:, 1] = True
+    assert torch.equal(got.isnan().all(-1), bad) and torch.equal(got.isnan().any(-1), bad)
+    # heads of a block raise their references together: roundings of the others may differ
+    assert (got[~bad].double() - clean[~bad].double()).norm() < BOUND * clean[~bad].double().norm()
+    assert paged_attention(q, k, v, batch, float("nan"), **kw).isnan().all()
+
+
+@pytest.mark.parametrize("starts", [[299, 700], [3000]])
+@pytest.mark.parametrize("H,G,D,Dv", [(8, 4, 64, 128), (16, 2, 128, 64), (12, 12, 128, 128)])
+@pytest.mark.parametrize("kw", [{}, dict(chunk=600), dict(sink_logits=True, gate=True)])
+def test_decode_with_shared_value_heads(starts, H, G, D, Dv, kw):
+    """Two key heads (all of them where there are two) read the same values."""
+    from colossalai_amd.ops.paged_attention import paged_attention, paged_attention_ref
+
+    torch.manual_seed(11)
+    n = len(starts)
+    batch, pages = _batch([1] * n, starts, 16)
+    k, v = torch.randn(pages, 16, G, D, device="cuda").bfloat16(), torch.randn(pages, 16, G // 2, Dv, device="cuda").bfloat16()
+    q = torch.randn(n, H, D, device="cuda").bfloat16()
+    kw = dict(kw)
+    if kw.pop("gate", False):
+        kw["gate"] = torch.randn(n, H, device="cuda").bfloat16()
+    if kw.pop("sink_logits", False):
+        kw["sink_logits"] = torch.randn(H, device="cuda") + 2.0
+    got = paged_attention(q, k, v, batch, 0.1, **kw)
+    want = paged_attention_ref(q.float(), k.float(), v.float(), batch, 0.1, 0, **{a: (t.float() if a == "gate" else t)
+                                                                                for a, t in kw.items()})
+    assert (got.double() - want.double()).norm() / want.double().norm() < BOUND
