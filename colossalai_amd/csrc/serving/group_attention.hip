@@ -364,19 +364,25 @@ bool launch_group_attention(at::Tensor& out, const at::Tensor& q, const at::Tens
   // Up to a tile a wave the other form's shorter end wins (6 x 173, 16 heads on 4 of 64: 7.9 against 8.3 us); values that are the keys
   // stay there as well, which reads each row once.
   if (keys <= 32 * GROUP_WAVES || vpool.data_ptr() == kpool.data_ptr()) return false;
-  // Parts of the keys while there are fewer blocks than CUs and a part keeps more than 1024 keys: parts cost a merge, about 4 us. 4 x 16384
-  // (16 heads on 4 of 128): 276 us undivided, 49 with 8 parts, 38 with 16, 42 with 32; 16 x 1024: 16.8, 16.5 with two and 15.8
-  // with four, but 5 x 700 on 2: 10.6 undivided, 12.4 with two; 1 x 8192: 16.8 with 8, 17.4 with 16, 22.4 with 32.
+  // every piece's sums of a head must fit into a wave's tile as well
+  const bool cols = R <= PIECE_HEADS && 3 * R * (2 + Dv) * 4 <= (D + Dv) * 64;
+  // Little work goes to the other form too, where a wave's own chain is longer there than the row's: with three products a tile (16 heads on 1
+  // of 128, that form and this: 1 x 512 8.8, 10.6, 4 x 2048 14.0, 18.6, but 32 x 300 10.3, 9.8, 16 x 1300 17.5, 16.5, 1 x 8192 26.5,
+  // 18.9 us), and over up to 512 keys with a distance penalty (4 x 512, 16 heads on 4 of 128: 8.9, 10.5; 64 x 512: 32, 17.5).
+  const long blocks = N * G;
+  if (!cols && blocks < 32 && keys < 8192 && blocks * keys < 20000) return false;
+  if (slopes != nullptr && blocks <= 64 && keys <= 512) return false;
+  // Parts of more than 1024 keys while there are fewer blocks than CUs and a part keeps 512: parts cost a merge, about 4 us. 4 x 16384
+  // (16 heads on 4 of 128): 276 us undivided, 49 with 8 parts, 38 with 16, 42 with 32; 1 x 2048: 17.7, 15.2 with two, 12.4 with four; but
+  // 5 x 700 on 2: 10.6 undivided, 12.4 with two; 1 x 8192: 16.8 with 8, 17.4 with 16, 22.4 with 32.
   int splits = 1;
-  while (N * G * splits * 2 <= 256 && keys > splits * 1024L && splits < WAVE) splits *= 2;
+  while (blocks * splits * 2 <= 256 && keys > 1024 && keys >= splits * 1024L && splits < WAVE) splits *= 2;
   // page numbers of a part: of its keys, rounded up to whole tiles, of a page more for where they begin, and of the kept ones
   const long part_keys = ((keys + 31) / 32 + splits - 1) / splits * 32;
   const size_t lds = (size_t)GROUP_WAVES * (D + Dv) * 64 + (size_t)((part_keys >> page_shift) + (keep_first >> page_shift) + 4) * sizeof(int);
   if (lds > GROUP_LDS) return false;
   at::Tensor ws;
   if (splits > 1) ws = at::empty({units * H * splits * (2 + Dv)}, q.options().dtype(at::kFloat));
-  // every piece's sums of a head must fit into a wave's tile as well
-  const bool cols = R <= PIECE_HEADS && 3 * R * (2 + Dv) * 4 <= (D + Dv) * 64;
 #define GROUP_LAUNCH(DS_, VT_)                                                                                       \
   do {                                                                                                             \
     auto kernel = cols ? group_attention_kernel<DS_, VT_, true> : group_attention_kernel<DS_, VT_, false>;          \

@@ -277,8 +277,8 @@ def test_decode_tokens_beside_long_portions(counts, starts, H, G, D, Dv, kw):
     _check(counts, starts, H, G, D, Dv, 16, D ** -0.5, **dict(kw))
 
 
-@pytest.mark.parametrize("D", [64, 128])
-def test_decode_weights_are_whole(D):
+@pytest.mark.parametrize("D,group", [(64, 1), (128, 1), (64, 16), (128, 4)])
+def test_decode_weights_are_whole(D, group):
     """256 keys of value v_a and 256 of -1, whose weights p differ from head to head and whose sums nearly cancel: 2^-13 of them is
     left. A weight's error of 2^-18, what two bfloat16 halves leave, would be up to a twentieth of the result; weights of 24 bits,
     their exponential (2^-22) and the result's own rounding make less than 2^-7 of it."""
@@ -301,8 +301,9 @@ def test_decode_weights_are_whole(D):
     assert (want.abs() / p).max() < 2.0 ** -12 and want.abs().min() > 0
     order = batch.block_tables[0].long().cpu()
     pool = lambda t: t.view(pages, page, heads, D)[torch.argsort(order)].cuda().bfloat16()
-    got = paged_attention(q.cuda().bfloat16(), pool(k), pool(v), batch, 1.0)[0, :, 0].double().cpu()
-    assert ((got - want).abs() <= 2.0 ** -6 * want.abs().max()).all()
+    q = q.repeat_interleave(group, 1).cuda().bfloat16()   # all heads of a key head alike
+    got = paged_attention(q, pool(k), pool(v), batch, 1.0)[0, :, 0].double().cpu().view(heads, group)
+    assert ((got - want[:, None]).abs() <= 2.0 ** -6 * want.abs().max()).all()
 
 
 @pytest.mark.parametrize("H,G,D,Dv", [(4, 2, 128, 128), (8, 1, 64, 128), (16, 1, 64, 64), (2, 2, 64, 64)])
@@ -314,9 +315,10 @@ def test_decode_values_that_are_infinite(H, G, D, Dv, start, kw):
     from colossalai_amd.ops.paged_attention import paged_attention
 
     torch.manual_seed(9)
-    batch, pages = _batch([1, 1], [start, start - 7], 16)
+    n = 34   # enough for groups of any size
+    batch, pages = _batch([1] * n, [start] + [start - 7] * (n - 1), 16)
     k, v = torch.randn(pages, 16, G, D, device="cuda").bfloat16(), torch.randn(pages, 16, G, Dv, device="cuda").bfloat16()
-    q = torch.randn(2, H, D, device="cuda").bfloat16()
+    q = torch.randn(n, H, D, device="cuda").bfloat16()
     want = paged_attention(q, k, v, batch, 0.1, **kw)
     row = lambda pos: (batch.block_tables[0, pos // 16].long(), pos % 16)
     inf = float("inf")
@@ -365,9 +367,10 @@ def test_decode_nan_stays_nan(start, H, D, kw):
     from colossalai_amd.ops.paged_attention import distance_slopes, paged_attention
 
     torch.manual_seed(4)
-    batch, pages = _batch([1, 1], [start, start - 20], 16)
+    n = 17   # enough for groups of 16 heads
+    batch, pages = _batch([1] * n, [start] + [start - 20] * (n - 1), 16)
     k, v = (torch.randn(pages, 16, 2, D, device="cuda").bfloat16() for _ in range(2))
-    q = torch.randn(2, H, D, device="cuda").bfloat16()
+    q = torch.randn(n, H, D, device="cuda").bfloat16()
     kw = dict(kw)
     if kw.pop("sink_logits", False):
         kw["sink_logits"] = torch.randn(H, device="cuda")
@@ -378,7 +381,7 @@ def test_decode_nan_stays_nan(start, H, D, kw):
     q[1, 0, 5] = float("nan")
     k[batch.block_tables[0, (start - 200) // 16], (start - 200) % 16, 1, 7] = float("nan")
     got = paged_attention(q, k, v, batch, 1.0, **kw)
-    bad = torch.zeros(2, H, dtype=torch.bool, device="cuda")
+    bad = torch.zeros(n, H, dtype=torch.bool, device="cuda")
     bad[1, 0] = True
     bad[0, H // 2:] = True
     if "slopes" in kw:
