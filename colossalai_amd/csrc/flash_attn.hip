@@ -579,14 +579,11 @@ DEV_INLINE void bwd_dkdv(
                   char* __restrict__ dOn) __attribute__((always_inline)) {
     // ---- S[q][kv] = Q · K^T and dP[q][kv] - delta[q] = dO · V^T - delta: column = kv (ln), row = q
     f32x16 s, dp;
-    float addend[16];
 #pragma unroll
     for (int a = 0; a < 4; ++a) {
-      const float4v l4 = *reinterpret_cast<const float4v*>(lse_lds + buf * QB + 8 * a + 4 * half);
       const float4v d4 = *reinterpret_cast<const float4v*>(dta_lds + buf * QB + 8 * a + 4 * half);
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        addend[4 * a + e] = l4[e];
         dp[4 * a + e] = d4[e];
         s[4 * a + e] = 0.0f;
       }
@@ -606,11 +603,16 @@ DEV_INLINE void bwd_dkdv(
     const int before = kvw + ln - qt0 - 4 * half;   // rows of the tile ahead of this key
     auto grads = [&](auto diagonal) __attribute__((always_inline)) {
 #pragma unroll
-      for (int j = 0; j < 16; ++j) {
-        float pv = __builtin_amdgcn_exp2f(fmaf(s[j], scale2, addend[j]));
-        if (diagonal) pv = before > crow(j, 0) ? 0.0f : pv;
-        pa[j >> 3][j & 7] = (__bf16)pv;
-        dsa[j >> 3][j & 7] = (__bf16)(pv * dp[j]);
+      for (int a = 0; a < 4; ++a) {   // read here, the statistics take 4 registers and not 16 over the products
+        const float4v l4 = *reinterpret_cast<const float4v*>(lse_lds + buf * QB + 8 * a + 4 * half);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int j = 4 * a + e;
+          float pv = __builtin_amdgcn_exp2f(fmaf(s[j], scale2, l4[e]));
+          if (diagonal) pv = before > crow(j, 0) ? 0.0f : pv;
+          pa[j >> 3][j & 7] = (__bf16)pv;
+          dsa[j >> 3][j & 7] = (__bf16)(pv * dp[j]);
+        }
       }
     };
     // two bodies: merged into one, every tile would pay for the mask of the few on the diagonal
@@ -863,8 +865,9 @@ constexpr size_t bwd_lds() {
   return kv > q ? kv : q;
 }
 
+// Three waves a SIMD with 64 channels, 168 registers; left to itself the packed form took 174 and had two.
 template <int D, bool VARLEN>
-__global__ __launch_bounds__(fa::NTB, 2) void fa_bwd_kernel(
+__global__ __launch_bounds__(fa::NTB, D == 64 ? 3 : 2) void fa_bwd_kernel(
     const unsigned short* __restrict__ Q, const unsigned short* __restrict__ K,
     const unsigned short* __restrict__ V, const unsigned short* __restrict__ dO,
     const float* __restrict__ LSE, const float* __restrict__ DELTA,
