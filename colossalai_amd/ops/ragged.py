@@ -34,6 +34,7 @@ class RaggedBatch:
     page_size: int = 0
     _dense: Optional[dict] = None  # memo of dense_context(), by window
     _chunk_tables: Optional[dict] = None  # memo of chunk_tables(), by chunk size
+    _tiles: Optional[tuple] = None  # memo of tile_counts()
     _singles: Optional[tuple] = None  # memo of single_tokens()
 
     @property
@@ -51,11 +52,12 @@ class RaggedBatch:
     def tile_counts(self):
         """Tiles of 32, 64 and 128 tokens of the prompt portions (all 0 for a pure decode step): the grids of the matrix-core
         attention kernel when every key head has three or more, two or a single query head."""
-        cu = self.cu_host
-        if cu[-1] == len(cu) - 1 and self.max_new == 1:
-            return 0, 0, 0
-        new = [b - a for a, b in zip(cu, cu[1:])]
-        return sum((n + 31) // 32 for n in new), sum((n + 63) // 64 for n in new), sum((n + 127) // 128 for n in new)
+        if self._tiles is None:
+            cu = self.cu_host
+            new = [b - a for a, b in zip(cu, cu[1:])]
+            decode = cu[-1] == len(new)   # every sequence brings a token
+            self._tiles = tuple(0 if decode else sum((n + size - 1) // size for n in new) for size in (32, 64, 128))
+        return self._tiles
 
     def single_tokens(self, window: int = 0):
         """Of a step with prompt portions: how many sequences bring one token, and whether the longest of them sees at least
@@ -74,12 +76,6 @@ class RaggedBatch:
         """32-token tiles of the prompt portions (0 for a pure decode step):
         the grid of the matrix-core attention kernel."""
         return self.tile_counts()[0]
-
-    @property
-    def num_tiles128(self) -> int:
-        """128-token tiles of the prompt portions (0 for a pure decode step): the grid of the matrix-core attention
-        kernel when every key head has a single query head."""
-        return self.tile_counts()[2]
 
     @property
     def max_total(self) -> int:
