@@ -21,6 +21,7 @@
 // of the keys), so that a position's results agree to rounding and not bit for bit.
 // Calls without a distance table, block summaries or cross values run the form in row_attention.hip
 // where the row sizes fit it; bfloat16 prompt portions run the matrix-core kernel.
+#include <algorithm>
 #include <type_traits>
 
 #include "../lds_tiles.h"
@@ -880,11 +881,21 @@ static bool launch_mfma_attention(at::Tensor& out, const at::Tensor& q, const at
   // prompt portions in bfloat16 go to the matrix cores when the head sizes fit a tiling;
   // num_tiles = sum over sequences of ceil(new tokens / 32), 0 asks for the scalar kernel
   auto at16 = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
-  const bool aligned = q.stride(0) % 8 == 0 && at16(q.data_ptr()) && at16(kpool.data_ptr()) && at16(vpool.data_ptr()) &&
-                       at16(x.ksum) && at16(x.vsum);
+  const bool aligned = q.stride(0) % 8 == 0 && at16(q.data_ptr()) && at16(x.ksum) && at16(x.vsum);
   // head sizes that are multiples of 8 ride in the next larger tiling, zero-padded
   const bool mfma_shape = D % 8 == 0 && Dv % 8 == 0 && D <= 128 && Dv <= 128;
   if (!(num_tiles > 0 && is_bf16(q) && aligned && mfma_shape && vpool.is_contiguous())) return false;
+  if (!at16(kpool.data_ptr()) || !at16(vpool.data_ptr())) {
+    // Loads go straight into LDS from addresses of 16 bytes. Pools that lie otherwise lend the pages of the call's sequences to copies, which
+    // the tables then number (4096 tokens of 16 heads on 4 of 128: 154 us, 135 without the copies, 5000 in the general kernel); not with data that is
+    // numbered by page as well, nor beyond 1 GiB.
+    const long pages = block_tables.numel(), per_page = (kpool.numel() + vpool.numel()) / std::max<long>(kpool.size(0), 1) * 2;
+    if (x.ksum != nullptr || x.key_fac != nullptr || pages * per_page > (1L << 30)) return false;
+    const at::Tensor ids = block_tables.reshape({-1}).clamp(0, kpool.size(0) - 1);   // places past a sequence's end hold anything
+    return launch_mfma_attention(out, q, kpool.index_select(0, ids), vpool.index_select(0, ids),
+                                 at::arange(pages, block_tables.options()).view(block_tables.sizes()), cu, start, slp, gate, gstride, scale,
+                                 window, keep_first, softcap, sink, page_shift, num_tiles, num_tiles128, num_tiles64, x, fewest);
+  }
   {
     const int rep = H / G, nw = 4;
     // one query head per kv head: the waves of a block take four consecutive token tiles instead of four heads; two: two

@@ -238,6 +238,27 @@ def test_pools_at_an_odd_address(which):
     assert (got.double() - want.double()).norm() / want.double().norm() < 2 * BOUND
 
 
+@pytest.mark.parametrize("counts,starts", [([40, 1], [100, 3]), ([200], [0]), ([33, 1, 96], [0, 130, 31])])
+@pytest.mark.parametrize("kw", [{}, dict(window=70, keep_first=4), dict(sink_logits=True)])
+@pytest.mark.parametrize("offset", [1, 4])
+def test_portions_of_pools_at_odd_addresses_take_the_same_kernel(counts, starts, kw, offset):
+    """The same bits; the pages beside a sequence's own may be numbered anyhow."""
+    from colossalai_amd.ops.paged_attention import paged_attention
+
+    torch.manual_seed(12)
+    batch, pages = _batch(counts, starts, 16)
+    k, v = (torch.randn(pages, 16, 2, 64, device="cuda").bfloat16() for _ in range(2))
+    q = torch.randn(sum(counts), 4, 64, device="cuda").bfloat16()
+    kw = dict(kw)
+    if kw.pop("sink_logits", False):
+        kw["sink_logits"] = torch.randn(4, device="cuda")
+    odd = [torch.empty(t.numel() + offset, device="cuda", dtype=t.dtype)[offset:].view(t.shape).copy_(t) for t in (k, v)]
+    want = paged_attention(q, k, v, batch, 0.1, **kw)
+    own = torch.tensor([(a + b + 15) // 16 for a, b in zip(counts, starts)], device="cuda")
+    batch.block_tables[torch.arange(batch.block_tables.shape[1], device="cuda") >= own[:, None]] = 1 << 20
+    assert torch.equal(paged_attention(q, *odd, batch, 0.1, **kw), want)
+
+
 # Decode tokens: groups of 1 to 16 query heads (17: another kernel), key and value sizes that differ, last tiles of one key and of 32,
 # windows and blocks that begin inside a page and a tile, kept keys that end in the middle of a page.
 @pytest.mark.parametrize("H,G,D,Dv", [(2, 2, 128, 128), (6, 2, 64, 128), (16, 1, 128, 64), (17, 1, 64, 64), (10, 2, 64, 64)])
