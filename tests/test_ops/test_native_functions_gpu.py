@@ -60,6 +60,56 @@ def test_same_bits_as_the_python_function(name, kept):
         assert a.dtype == b.dtype and torch.equal(a, b)
 
 
+NAMES = ["rms_norm", "add_norm", "swiglu", "dense", "padded", "packed", "rope", "rope_at"]
+
+
+def _backward(call, inputs, form):
+    inputs = [t.detach().requires_grad_() for t in inputs]
+    out = call(*inputs)
+    out = out if isinstance(out, tuple) else (out,)
+    if form == "last result":
+        return torch.autograd.grad(out[-1], inputs, torch.ones_like(out[-1]), allow_unused=True)
+    douts = [torch.ones((), device="cuda", dtype=t.dtype).expand_as(t) if form == "one for all" else torch.ones_like(t).cumsum(-1) for t in out]
+    if form == "some inputs":
+        return torch.autograd.grad(out, inputs[-1:], douts)
+    if form == "twice":
+        torch.autograd.grad(out, inputs, douts, retain_graph=True)
+    return torch.autograd.grad(out, inputs, douts, create_graph=form == "graph", retain_graph=True)
+
+
+@pytest.mark.parametrize("name", NAMES)
+@pytest.mark.parametrize("form", ["one for all", "last result", "some inputs", "twice", "graph"])
+def test_backward_forms_of_both(name, form):
+    native, python, inputs = _calls()[name]
+    for a, b in zip(_backward(native, inputs, form), _backward(python, inputs, form)):
+        if b is None:
+            assert a is None
+            continue
+        assert a.dtype == b.dtype and a.requires_grad == b.requires_grad and torch.equal(a, b)
+
+
+@pytest.mark.parametrize("name", NAMES)
+def test_results_are_changed_in_place_alike(name):
+    """Accepted or refused, forward and backward."""
+    def told(call, inputs):
+        inputs = [t.detach().requires_grad_() for t in inputs]
+        try:
+            out = call(*inputs)
+            out = out if isinstance(out, tuple) else (out,)
+            for t in out:
+                t.mul_(2.0)
+            return torch.autograd.grad(out, inputs, [torch.ones_like(t) for t in out])
+        except RuntimeError as e:
+            return "in place" in str(e) or "inplace" in str(e)
+
+    native, python, inputs = _calls()[name]
+    a, b = told(native, inputs), told(python, inputs)
+    if isinstance(b, bool):
+        assert a is b is True
+    else:
+        assert all(torch.equal(x, y) for x, y in zip(a, b))
+
+
 def test_what_watches_or_rewrites_goes_to_python():
     class Watch(TorchDispatchMode):
         def __torch_dispatch__(self, func, types, args=(), kwargs=None):
