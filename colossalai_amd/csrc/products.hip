@@ -4,7 +4,8 @@
 // Operands lie as they come: with the contracted index fast, fragments are plain LDS reads, with it slow (both of a weight
 // gradient) transposing ones (ds_read_b64_tr_b16, see flash_attn.hip). Four waves hold a tile's sums in registers, one
 // quarter each: 256 x 256 where there is enough of them, which is the least LDS and memory traffic a product has here (a
-// wave's 128 x 128 sums are 256 registers, one wave a SIMD), else 256 x 128 or 128 x 128 with two blocks a CU. Four steps of 32
+// wave's 128 x 128 sums are 256 registers, one wave a SIMD), else 256 x 128, also one block a CU (96 KB of LDS), or 128 x 128 with
+// two. Four steps of 32
 // contracted indices lie in LDS: while one is multiplied the next is there and two are on their way, so that a step waits for
 // loads that are two steps old (s_waitcnt vmcnt, never 0) and for one barrier. A wave reads the fragments of the next 16
 // indices and issues its loads one by one between the products of the 16 before.
@@ -134,7 +135,7 @@ DEV_INLINE void put(const Args& a, long at, float4v v) {
 
 // STEPS steps lie in LDS: one in use, one arrived, the others on their way.
 template <bool PC, bool QC, int TM, int TN, int STEPS>
-__global__ __launch_bounds__(256, TM == 256 && TN == 256 ? 1 : 2) void product_kernel(const Args a) {
+__global__ __launch_bounds__(256, TM == 256 ? 1 : 2) void product_kernel(const Args a) {
   extern __shared__ char smem[];
   constexpr int FA = TN / 64, FB = TM / 64;
   constexpr int YB = Operand<PC, TM>::BYTES, SB = YB + Operand<QC, TN>::BYTES;
