@@ -377,10 +377,12 @@ at::Tensor weight_grad(const at::Tensor& dy, const at::Tensor& x, const c10::opt
   }
   const bool serves = weight_grad_serves(dy, x);
   const pr::Plan plan = serves ? pr::plan(dy.size(1), x.size(1), dy.size(0), false) : pr::Plan{};
-  // Over few tokens storing the result is most of it, which the library does faster: 22016 x 4096 over 64, 256, 512, 1024 and 2048
-  // tokens 63, 103, 126, 213 and 404 us there, 112, 143, 176, 241 and 373 here; 4096 x 4096: 12, 18, 26, 40 and 71 there, 23, 27, 33,
-  // 45 and 70 here. It multiplies those, unless the host is what a call waits for (see multiply); a float32 result it does not have.
-  if (!serves || (!add && !keep && dy.size(0) < 2048 && plan.us > 14.0)) {
+  // Over few tokens storing a large result is most of the work, which the library does faster. Its time and the kernel's, us: 22016 x 4096 over
+  // 64, 256, 512, 1024 and 2048 tokens 63, 103, 126, 213, 404 and 112, 143, 176, 241, 373; 4096 x 4096 12, 18, 26, 40, 71 and 23, 27,
+  // 33, 45, 70. Over results of 9 to 131 million elements the kernel takes 1.5 times the library's at 100 tokens, 1.2 at 500, 1.06 from 1000 to
+  // 1500 (1.2 at 1536) and 1 at 1700 to 2000; below 2^23 elements it is ahead or, up to 10 us, bound by the host (see multiply). A
+  // float32 result the library does not have.
+  if (!serves || (!add && !keep && dy.size(0) < 1600 && dy.size(1) * x.size(1) > (1L << 23))) {
     at::Tensor r = at::mm(dy.t(), x);
     if (add) r = keep ? add->add_(r) : at::add(*add, r);
     return r.to(keep ? at::kFloat : dy.scalar_type());

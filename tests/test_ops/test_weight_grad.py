@@ -73,10 +73,10 @@ def _formed_here(call):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("M,N,K,here", [(4096, 4096, 64, False), (4096, 2048, 1024, False), (2304, 4096, 2047, False),
-                                        (2304, 4096, 2048, True), (512, 512, 512, True)])
+@pytest.mark.parametrize("M,N,K,here", [(4096, 4096, 64, False), (4096, 2056, 1024, False), (2304, 4096, 1599, False),
+                                        (2304, 4096, 1600, True), (4096, 2048, 100, True), (512, 512, 512, True)])
 def test_few_tokens_are_the_librarys(M, N, K, here):
-    """Storing is most of such a product, which the library does faster; small ones are the host's time, and a float32 sum is formed here."""
+    """Storing a large result is most of such a product, which the library does faster; a float32 sum is formed here in any case."""
     torch.manual_seed(K)
     dy, x = (torch.randn(K, n, device="cuda").to(BF16) for n in (M, N))
     _close(kernels().weight_grad(dy, x), dy, x)
