@@ -7,13 +7,14 @@
 //   layout they were born in, each as three bfloat16 pieces, which hold all of its 24 bits; A = values by transposing reads),
 // so a head is a lane and its half-wave twin. Of the 32 columns the group fills 1 to 16; the products cost a tenth of the time that
 // the tile's 16 KB take to arrive. Up to 10 heads stand three times in the columns, once for each piece of their weights: one
-// product then does for three (16 x 1024 keys with a cap and a sink, 16 heads on 4 of 128: 17.5 us with three, 16.6 with one). The pieces' sums
-// meet at the end; where the first one's is infinite, it is the result (0 and negative rests of a weight times infinity). The next tile's keys are on their way from the moment the scores are
-// formed, its values from the end of the products.
-// What bounds it: memory beyond about 8 us of dependent loads (position, page table, rows), launch and the end. Against
-// the form with a row in the registers of a few lanes (row_attention.hip), 16 heads on 4 of 128: 16 x 1024 keys with a cap
-// and a sink 18.5 -> 16.5 us, 4 x 16384 52.0 -> 38.1 (3.5 TB/s), 16 x 8192 84 -> 63 (4.3 TB/s), 8 heads on 2, 7 x 5000
-// 24.8 -> 17.5; 16 heads on 8 of 64, 16 x 3000: 41.5 -> 28.8; one head a key head, 16 x 2000: 61 -> 56; 16 x 128: 9.4 and 9.9.
+// product then does for three (16 x 1024 keys with a cap and a sink, 16 heads on 4 of 128: 17.5 us with three, 16.6 with one). The
+// pieces' sums meet at the end; where the first one's is infinite it is the result, as the rests of a weight, 0 or negative, times infinity
+// are not its part. The next tile's keys are on their way from the moment the scores are formed, its values from the end of the
+// products.
+// What bounds it: memory beyond about 8 us of dependent loads (position, page table, rows), launch and the end. The form with a
+// row in the registers of a few lanes (row_attention.hip) and this one, us, replayed from a graph: 16 heads on 4 of 128: 16 x 1024 keys with a
+// cap and a sink 15.6, 15.5, 4 x 16384 38.6, 30.9 (4.3 TB/s), 16 x 8192 56.2, 47.7 (5.6 TB/s); 8 on 2 of 128, 7 x 5000 20.2, 15.0; 16
+// on 8 of 64, 16 x 3000 25.6, 23.0; one head a key head, 16 x 2000 45.7, 43.1; 16 on 1 of 128, 16 x 2000 21.0, 16.0.
 // The eight waves' states meet in LDS at the end; few tokens with long contexts have their keys cut into parts, whose
 // states row_merge_kernel puts together. Beside prompt portions it may serve just the sequences that bring one token.
 #include "paged_attention.h"

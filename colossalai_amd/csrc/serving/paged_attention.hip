@@ -300,8 +300,8 @@ __global__ __launch_bounds__(64 * ATT_WAVES) void paged_attention_kernel(
 // lane-local because the products are formed transposed:
 //   S^T = K Q^T   (A = key rows from LDS, B = query rows kept in registers)
 //   O^T = V^T P^T (B = the float32 weights in the C layout they were born in, split into a
-//                  high and a low bfloat16 half so that no weight loses its float32 mantissa
-//                  to the matrix unit; A = values, read from LDS with the transposing
+//                  high and a low bfloat16 half, 16 to 17 of a weight's 24 bits, twice what
+//                  the matrix unit takes at once; A = values, read from LDS with the transposing
 //                  64-bit read in the same key order)
 // so column = token = lane & 31 everywhere: running max, running sum, rescaling and the gate
 // never cross lanes except for one exchange between the two half-waves.
