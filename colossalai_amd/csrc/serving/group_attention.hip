@@ -15,12 +15,20 @@
 // row in the registers of a few lanes (row_attention.hip) and this one, us, replayed from a graph: 16 heads on 4 of 128: 16 x 1024 keys with a
 // cap and a sink 15.6, 15.5, 4 x 16384 38.6, 30.9 (4.3 TB/s), 16 x 8192 56.2, 47.7 (5.6 TB/s); 8 on 2 of 128, 7 x 5000 20.2, 15.0; 16
 // on 8 of 64, 16 x 3000 25.6, 23.0; one head a key head, 16 x 2000 45.7, 43.1; 16 on 1 of 128, 16 x 2000 21.0, 16.0.
-// The eight waves' states meet in LDS at the end; few tokens with long contexts have their keys cut into parts, whose
-// states row_merge_kernel puts together. Beside prompt portions it may serve just the sequences that bring one token.
+// The eight waves' states meet in LDS at the end; few tokens have their keys cut into parts, whose states the block that ends last puts
+// together (a launch for that took 4 to 6 us, and the host as long as the first one's). Which one that is needs no memory that somebody has cleared: a part
+// leaves its states, then a mark that belongs to this launch alone, then looks at all marks of its token and key head. The last
+// one to look finds them all; if two do, both write the same. What passes between the blocks goes around the L2 caches, which
+// the XCDs do not share, word by word: fences at the scope of the device, which write back and empty these caches, took up to 100 us of a launch.
+// 16 x 1024 keys with a cap and a sink 20.2 -> 16.0 us, 1 x 8192 16.6 -> 13.4, 4 x 16384 39.2 -> 36.5 (other keys and values in every
+// call). Beside prompt portions the kernel may serve just the sequences that bring one token.
 #include "paged_attention.h"
 #include "../lds_tiles.h"
 
 #include <algorithm>
+#include <atomic>
+#include <cmath>
+#include <random>
 #include <type_traits>
 
 namespace cai {
@@ -50,13 +58,22 @@ DEV_INLINE void loads_left() {
 
 __device__ __align__(16) const bf16s no_values[128] = {};   // a key's past the end
 
+// A part's state, for a block on any XCD to read: every access is one of its own at the scope of the device, past the L2 caches.
+DEV_INLINE void put_state(float* p, float v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+DEV_INLINE float get_state(float* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+// this wave's stores and atomics have been performed where every XCD sees them
+DEV_INLINE void stores_done() { asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory"); }
+// floats of a part's states of a group of R heads, in cache lines of its own
+__host__ __device__ constexpr long part_floats(int R, int Dv) { return (R * (2 + Dv) + 63L) / 64 * 64; }
+
 template <int DS, int VT, bool COLS>
 __global__ __launch_bounds__(64 * GROUP_WAVES, 2) void group_attention_kernel(
     bf16s* __restrict__ out, const bf16s* __restrict__ q, long q_stride, const bf16s* __restrict__ kpool,
     const bf16s* __restrict__ vpool, const int* __restrict__ block_tables, int bt_stride, const int* __restrict__ tok_seq,
     const int* __restrict__ positions, const float* __restrict__ slopes, const bf16s* __restrict__ gate, long gate_stride,
     const float* __restrict__ sink_logits, int H, int G, int page_shift, float scale, int window, int keep_first, int chunk,
-    float softcap, int sink, int vrep, long vrow, long vhead, int splits, float* __restrict__ ws, const int* __restrict__ cu) {
+    float softcap, int sink, int vrep, long vrow, long vhead, int splits, float* __restrict__ ws, const int* __restrict__ cu,
+    unsigned long long* __restrict__ marks, unsigned long long mark) {
   constexpr int D = DS * 16, Dv = VT * 32, KQ = D / 32, KT = D * 64, VTT = Dv * 64;   // bytes of a tile's keys, values
   constexpr float LOG2E = 1.4426950408889634f;
   extern __shared__ __align__(16) char tiles[];   // [waves][KT + VTT], later the waves' states; then the pages
@@ -326,11 +343,11 @@ __global__ __launch_bounds__(64 * GROUP_WAVES, 2) void group_attention_kernel(
       o += (COLS ? whole(sums[0], sums[R * PS] + sums[2 * R * PS]) : sums[0]) * f;
     }
     if (splits > 1) {   // a part without keys has a maximum of -inf
-      float* state = ws + ((unit * H + h0 + r) * splits + split) * (long)PS;
-      state[2 + dv] = o;
+      float* state = ws + ((unit * G + g) * splits + split) * part_floats(R, Dv) + r * PS;
+      put_state(state + 2 + dv, o);
       if (dv == 0) {
-        state[0] = top;
-        state[1] = ll;
+        put_state(state, top);
+        put_state(state + 1, ll);
       }
     } else {
       if (sink_logits != nullptr) ll += __builtin_amdgcn_exp2f(sink_logits[h0 + r] * LOG2E - top);
@@ -340,6 +357,75 @@ __global__ __launch_bounds__(64 * GROUP_WAVES, 2) void group_attention_kernel(
       stf(out + (n * H + h0 + r) * (long)Dv + dv, o * c);
     }
   }
+  if (splits == 1) return;
+
+  // The part that finds all marks of its token and kv head set puts the states together.
+  int* all_there = pages;   // the page numbers are done with
+  stores_done();
+  __syncthreads();
+  marks += (unit * G + g) * splits;
+  if (wid == 0) {
+    if (lane == split) (void)__hip_atomic_exchange(marks + lane, mark, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    stores_done();                   // own mark first: of two parts that look at the same time one sees the other's
+    unsigned long long none = 0;
+    asm volatile("" : "+v"(none));   // an addition to where the marks are ordered, not a load
+    const int there = __all(lane >= splits || __hip_atomic_fetch_add(marks + lane, none, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == mark);
+    if (lane == 0) *all_there = there;
+  }
+  __syncthreads();
+  if (!*all_there) return;
+  float* coef = reinterpret_cast<float*>(tiles);   // [R][WAVE]
+  const long step = part_floats(R, Dv);
+  float* parts = ws + (unit * G + g) * splits * step;
+  constexpr int AHEAD = 8;
+  float v[AHEAD];
+  auto fetch = [&](int i, int p0) {
+    float* sums = parts + i / Dv * PS + 2 + i % Dv;
+#pragma unroll
+    for (int e = 0; e < AHEAD; ++e) v[e] = get_state(sums + min(p0 + e, splits - 1) * step);
+  };
+  if ((int)threadIdx.x < R * Dv) fetch(threadIdx.x, 0);
+  for (int r = wid; r < R; r += GROUP_WAVES) {
+    float* state = parts + min(lane, splits - 1) * step + r * PS;
+    const float m_at = get_state(state), l_at = get_state(state + 1);
+    const float mp = lane < splits ? m_at : -INFINITY, lp = lane < splits ? l_at : 0.0f;
+    float top = wave_reduce_max(mp);
+    if (sink_logits != nullptr) top = fmaxf(top, sink_logits[h0 + r] * LOG2E);
+    const float f = mp == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(mp - top);
+    float ll = wave_reduce_sum(lp * f);
+    if (sink_logits != nullptr) ll += __builtin_amdgcn_exp2f(sink_logits[h0 + r] * LOG2E - top);
+    else if (sink) ll += __builtin_amdgcn_exp2f(-top);   // the sink's score is 0
+    float c = f / ll;
+    if (gate != nullptr) c *= sigmoidf_(ldf(gate + n * gate_stride + h0 + r));
+    coef[r * WAVE + lane] = c;
+  }
+  __syncthreads();
+  for (int i = threadIdx.x; i < R * Dv; i += 64 * GROUP_WAVES) {
+    const float* c = coef + i / Dv * WAVE;
+    float o = 0.0f;
+    for (int p0 = 0; p0 < splits; p0 += AHEAD) {
+      if (i != (int)threadIdx.x || p0 > 0) fetch(i, p0);
+#pragma unroll
+      for (int e = 0; e < AHEAD; ++e)
+        if (p0 + e < splits) o += c[p0 + e] * v[e];
+    }
+    stf(out + (n * H + h0 + i / Dv) * (long)Dv + i % Dv, o);
+  }
+  // a launch that a graph repeats has the same mark each time (whoever looks now finds too little, and is not needed)
+  if (wid == 0 && lane < splits) __hip_atomic_store(marks + lane, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// A number that no launch of this process had before and that memory does not hold by chance.
+unsigned long long new_mark() {
+  static const unsigned long long seed = [] {
+    std::random_device r;
+    return (unsigned long long)r() << 32 | r();
+  }();
+  static std::atomic<unsigned long long> count{0};
+  unsigned long long z = seed + ++count * 0x9e3779b97f4a7c15ull;   // splitmix64, one to one
+  z = (z ^ z >> 30) * 0xbf58476d1ce4e5b9ull;
+  z = (z ^ z >> 27) * 0x94d049bb133111ebull;
+  return z ^ z >> 31;
 }
 
 }  // namespace
@@ -362,28 +448,40 @@ bool launch_group_attention(at::Tensor& out, const at::Tensor& q, const at::Tens
   long keys = block_tables.size(1) << page_shift;           // most that a token can see
   if (window > 0) keys = std::min<long>(keys, window + keep_first);
   if (x.chunk > 0) keys = std::min<long>(keys, x.chunk);
-  // Up to a tile a wave the other form's shorter end wins (6 x 173, 16 heads on 4 of 64: 7.9 against 8.3 us); values that are the keys
-  // stay there as well, which reads each row once.
-  if (keys <= 32 * GROUP_WAVES || vpool.data_ptr() == kpool.data_ptr()) return false;
+  // Values that are the keys stay in the other form, which reads each row once.
+  if (vpool.data_ptr() == kpool.data_ptr()) return false;
+  const long blocks = N * G;
+  // Up to a tile a wave: few tokens with many heads a key head go to the other form, whose end is shorter (that form and this, us: 8 x 200 keys,
+  // 8 heads on 1 of 128: 7.1, 7.8; 16 on 1 7.3, 8.9; but 48 x 200 14.1, 9.0; 16 on 4, 1 x 200 7.1, 6.6, 128 x 200 43.0, 20.8; 64 channels 8 x 200
+  // 7.2, 5.0), and so do tokens beside prompt portions, which then ride with these.
+  if (keys <= 32 * GROUP_WAVES && (some || (D + Dv > 128 && R > 4 && blocks < 48))) return false;
   // every piece's sums of a head must fit into a wave's tile as well
   const bool cols = R <= PIECE_HEADS && 3 * R * (2 + Dv) * 4 <= (D + Dv) * 64;
-  // Little work goes to the other form too, where a wave's own chain is longer there than the row's: with three products a tile (16 heads on 1
-  // of 128, that form and this: 1 x 512 8.8, 10.6, 4 x 2048 14.0, 18.6, but 32 x 300 10.3, 9.8, 16 x 1300 17.5, 16.5, 1 x 8192 26.5,
-  // 18.9 us), and over up to 512 keys with a distance penalty (4 x 512, 16 heads on 4 of 128: 8.9, 10.5; 64 x 512: 32, 17.5).
-  const long blocks = N * G;
-  if (!cols && blocks < 32 && keys < 8192 && blocks * keys < 20000) return false;
-  if (slopes != nullptr && blocks <= 64 && keys <= 512) return false;
-  // Parts of more than 1024 keys while there are fewer blocks than CUs and a part keeps 512: parts cost a merge, about 4 us. 4 x 16384
-  // (16 heads on 4 of 128): 276 us undivided, 49 with 8 parts, 38 with 16, 42 with 32; 1 x 2048: 17.7, 15.2 with two, 12.4 with four; but
-  // 5 x 700 on 2: 10.6 undivided, 12.4 with two; 1 x 8192: 16.8 with 8, 17.4 with 16, 22.4 with 32.
-  int splits = 1;
-  while (blocks * splits * 2 <= 256 && keys > 1024 && keys >= splits * 1024L && splits < WAVE) splits *= 2;
+  // Little work goes to the other form too, where a wave's own chain is longer here than the row's: with three products a tile (16 heads on 1
+  // of 128, that form and this: 1 x 512 11.7, 13.2, 4 x 2048 16.4, 17.5, 16 x 600 12.3, 14.4, but 16 x 1300 17.9, 17.5, 1 x 8192 26.5,
+  // 18.9 us), and over 257 to 512 keys with a distance penalty (4 x 300, 16 heads on 4 of 128: 9.1, 9.4; 16 x 400 11.0, 12.0; 64 x 512: 32, 17.5).
+  if (keys > 32 * GROUP_WAVES) {
+    if (!cols && blocks < 32 && keys < 8192 && blocks * keys < 20000) return false;
+    if (slopes != nullptr && blocks <= 64 && keys <= 512) return false;
+  }
+  // Parts of the keys while there are fewer blocks than CUs. A tile of 32 keys takes a wave 1.75 us at 128 channels, of which eight run side by side;
+  // parts cost about 2 us, a store and three round trips to memory, and 0.1 each for reading their states. Whole, and in parts: 16 x 1024 (16 heads on
+  // 4 of 128) 22.8 us, 2: 19.0, 4: 16.0, 8 (512 blocks): 22.8; 4 x 16384 277, 8: 48.4, 16: 36.6, 32: 41.4; 1 x 8192 66, 8: 17.4, 16: 14.4, 24:
+  // 13.4, 64: 16.1; 1 x 2048 20.8, 4: 12.9, 12: 11.3, 16: 10.8; 16 x 300 (8 on 4) 9.3, 2: 10.6, 4: 9.9; 3 x 1500 (4 on 2 of 64) 12.3, 8: 8.2.
+  const double whole = (double)((keys + 31) / 32) * 0.22 * (D + Dv) / 256;
+  int splits = (int)std::max<long>(1, std::min<long>({256 / blocks, WAVE, std::lround(std::sqrt(whole * 10.0))}));
+  if (whole <= whole / splits + 2.0 + 0.1 * splits) splits = 1;
   // page numbers of a part: of its keys, rounded up to whole tiles, of a page more for where they begin, and of the kept ones
   const long part_keys = ((keys + 31) / 32 + splits - 1) / splits * 32;
   const size_t lds = (size_t)GROUP_WAVES * (D + Dv) * 64 + (size_t)((part_keys >> page_shift) + (keep_first >> page_shift) + 4) * sizeof(int);
   if (lds > GROUP_LDS) return false;
   at::Tensor ws;
-  if (splits > 1) ws = at::empty({units * H * splits * (2 + Dv)}, q.options().dtype(at::kFloat));
+  unsigned long long* marks = nullptr;
+  if (splits > 1) {   // states, then marks
+    const long states = units * G * splits * part_floats(R, Dv);
+    ws = at::empty({states + units * G * splits * 2}, q.options().dtype(at::kFloat));
+    marks = reinterpret_cast<unsigned long long*>(ws.data_ptr<float>() + states);
+  }
 #define GROUP_LAUNCH(DS_, VT_)                                                                                       \
   do {                                                                                                             \
     auto kernel = cols ? group_attention_kernel<DS_, VT_, true> : group_attention_kernel<DS_, VT_, false>;          \
@@ -393,13 +491,12 @@ bool launch_group_attention(at::Tensor& out, const at::Tensor& q, const at::Tens
                        (int)block_tables.stride(0), tok_seq.data_ptr<int>(), positions.data_ptr<int>(), slopes,    \
                        gate.has_value() ? ptr<bf16s>(*gate) : (const bf16s*)nullptr, gate_stride, x.sink_logits, H, G, page_shift, \
                        (float)scale, (int)window, (int)keep_first, x.chunk, (float)softcap, sink ? 1 : 0, x.vrep, vrow, vhead, \
-                       splits, splits > 1 ? ws.data_ptr<float>() : (float*)nullptr, only.cu);                            \
+                       splits, splits > 1 ? ws.data_ptr<float>() : (float*)nullptr, only.cu, marks, splits > 1 ? new_mark() : 0ull);                            \
   } while (0)
   if (D == 128) { if (Dv == 128) GROUP_LAUNCH(8, 4); else GROUP_LAUNCH(8, 2); }
   else { if (Dv == 128) GROUP_LAUNCH(4, 4); else GROUP_LAUNCH(4, 2); }
 #undef GROUP_LAUNCH
   HIP_CHECK_LAST();
-  if (splits > 1) launch_row_merge(out, q, ws, gate, gate_stride, x, Dv, sink, splits, only);
   return true;
 }
 

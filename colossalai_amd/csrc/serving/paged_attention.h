@@ -55,9 +55,5 @@ bool launch_group_attention(at::Tensor& out, const at::Tensor& q, const at::Tens
                             int64_t window, int64_t keep_first, double softcap, bool sink, int page_shift, long vrow,
                             long vhead, const ScalarExtras& x, const SingleTokens& only = SingleTokens());
 
-// The states of `splits` parts of each (token, head)'s keys in `ws` -> `out`, or x.out32; q gives the type of the call (row_attention.hip).
-void launch_row_merge(at::Tensor& out, const at::Tensor& q, const at::Tensor& ws, const c10::optional<at::Tensor>& gate,
-                      long gate_stride, const ScalarExtras& x, int Dv, bool sink, int splits, const SingleTokens& only = SingleTokens());
-
 }  // namespace serving
 }  // namespace cai

@@ -356,16 +356,11 @@ __global__ __launch_bounds__(64 * ROW_WAVES) void row_attention_kernel(
 template <typename T>
 __global__ __launch_bounds__(256) void row_merge_kernel(
     T* __restrict__ out, float* __restrict__ out32, const float* __restrict__ ws, const T* __restrict__ gate, long gate_stride,
-    const float* __restrict__ sink_logits, const int* __restrict__ cu, long rows, int H, int Dv, int sink, int splits) {
-  long row = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
+    const float* __restrict__ sink_logits, long rows, int H, int Dv, int sink, int splits) {
+  const long row = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
   if (row >= rows) return;
   const float* state = ws + row * splits * (long)(2 + Dv);
-  if (cu != nullptr) {   // rows are sequences' heads so far
-    const int b = (int)(row / H);
-    if (cu[b + 1] - cu[b] != 1) return;
-    row += (long)(cu[b] - b) * H;
-  }
   const int h = (int)(row % H);
   const float m = lane < splits ? state[lane * (long)(2 + Dv)] : -INFINITY;   // splits <= MAX_PARTS
   const float l = lane < splits ? state[lane * (long)(2 + Dv) + 1] : 0.0f;
@@ -394,15 +389,15 @@ __global__ __launch_bounds__(256) void row_merge_kernel(
   }
 }
 
-void launch_row_merge(at::Tensor& out, const at::Tensor& q, const at::Tensor& ws, const c10::optional<at::Tensor>& gate,
-                      long gate_stride, const ScalarExtras& x, int Dv, bool sink, int splits, const SingleTokens& only) {
-  const long rows = (only.cu != nullptr ? only.seqs : q.size(0)) * q.size(1);
+static void launch_row_merge(at::Tensor& out, const at::Tensor& q, const at::Tensor& ws, const c10::optional<at::Tensor>& gate,
+                             long gate_stride, const ScalarExtras& x, int Dv, bool sink, int splits) {
+  const long rows = q.size(0) * q.size(1);
   TORCH_CHECK(splits <= MAX_PARTS, "more parts of the keys than the merge takes");
   SERVING_DISPATCH_ACT(q, T, {
     hipLaunchKernelGGL((row_merge_kernel<T>), dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, stream(),
                        x.out32 != nullptr ? (T*)nullptr : ptr<T>(out), x.out32, ws.data_ptr<float>(),
-                       gate.has_value() ? ptr<T>(*gate) : (const T*)nullptr, gate_stride, x.sink_logits, only.cu, rows, (int)q.size(1),
-                       Dv, sink ? 1 : 0, splits);
+                       gate.has_value() ? ptr<T>(*gate) : (const T*)nullptr, gate_stride, x.sink_logits, rows, (int)q.size(1), Dv,
+                       sink ? 1 : 0, splits);
   });
   HIP_CHECK_LAST();
 }

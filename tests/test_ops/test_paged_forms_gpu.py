@@ -434,3 +434,38 @@ def test_decode_with_shared_value_heads(starts, H, G, D, Dv, kw):
     want = paged_attention_ref(q.float(), k.float(), v.float(), batch, 0.1, 0, **{a: (t.float() if a == "gate" else t)
                                                                                 for a, t in kw.items()})
     assert (got.double() - want.double()).norm() / want.double().norm() < BOUND
+
+
+@pytest.mark.parametrize("H,G,D,Dv", [(16, 4, 128, 128), (16, 1, 64, 128), (4, 4, 64, 64)])
+@pytest.mark.parametrize("starts", [[20, 0], [255, 100, 31], [700] * 5, [1300, 900] * 8, [9000], [30000, 3]])
+def test_decode_parts_meet_whoever_ends_last(H, G, D, Dv, starts):
+    """The parts of a token's keys are put together by one of their own blocks, in an order that does not depend on which: every
+    repetition has the same bits, also from a graph, whose launches repeat themselves over memory that others have used."""
+    from colossalai_amd.ops.paged_attention import paged_attention, paged_attention_ref
+
+    torch.manual_seed(6)
+    n = len(starts)
+    batch, pages = _batch([1] * n, starts, 16)
+    k, v = (torch.randn(pages, 16, G, d, device="cuda").bfloat16() for d in (D, Dv))
+    gate = torch.randn(n, H, device="cuda").bfloat16()
+    qs = [torch.randn(n, H, D, device="cuda").bfloat16() for _ in range(3)]
+
+    def call(q):
+        return paged_attention(q, k, v, batch, D ** -0.5, gate=gate, softcap=20.0, sink=True)
+
+    want = [call(q) for q in qs]
+    for q, w in zip(qs, want):
+        ref = paged_attention_ref(q.float(), k.float(), v.float(), batch, D ** -0.5, gate=gate.float(), softcap=20.0, sink=True)
+        assert (w.double() - ref.double()).norm() / ref.double().norm() < BOUND
+    torch.cuda.synchronize()
+    q = qs[0].clone()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        first, second = call(q), call(q)
+    for i in range(30):
+        q.copy_(qs[i % 3])
+        first.zero_()
+        second.zero_()
+        graph.replay()
+        assert torch.equal(first, want[i % 3]) and torch.equal(second, want[i % 3])
+        assert torch.equal(call(q), want[i % 3])
