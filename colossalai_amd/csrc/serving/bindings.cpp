@@ -8,6 +8,8 @@ namespace serving {
 
 at::Tensor token_shift(at::Tensor x, at::Tensor mu, at::Tensor prev, at::Tensor cu, at::Tensor start,
                        at::Tensor slots, at::Tensor tok_seq, at::ScalarType out_dtype);
+void ragged_index(at::Tensor buf, int64_t B, int64_t N, int64_t width, int64_t page_size);
+void dense_context(at::Tensor rows, at::Tensor tables, at::Tensor block_tables, at::Tensor of, int64_t page_size);
 at::Tensor relu_squared(at::Tensor x);
 at::Tensor softcap(at::Tensor x, double cap);
 void paged_kv_write(at::Tensor k, at::Tensor v, at::Tensor kpool, at::Tensor vpool, at::Tensor rows);
@@ -80,6 +82,8 @@ at::Tensor expert_grouped_gemm(at::Tensor a, c10::optional<at::Tensor> a_rows, a
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   namespace s = cai::serving;
   m.def("token_shift", &s::token_shift, "token shift over a ragged batch with a carried previous row");
+  m.def("ragged_index", &s::ragged_index, "sequence, position and pool row of every token of a ragged step");
+  m.def("dense_context", &s::dense_context, "pool rows and page tables of a step's contexts laid out densely");
   m.def("relu_squared", &s::relu_squared, "max(x, 0)^2");
   m.def("softcap", &s::softcap, "cap * tanh(x / cap), float32");
   m.def("paged_kv_write", &s::paged_kv_write, "scatter a ragged batch's keys/values into pool rows");

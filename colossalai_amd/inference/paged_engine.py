@@ -27,7 +27,7 @@ from .engine import LLMEngine
 from .kv_cache import KVCacheManager
 from .request_manager import Request, RequestManager
 from .state_cache import StateCacheManager
-from ..ops.ragged import RaggedBatch
+from ..ops.ragged import RaggedBatch, to_device
 
 __all__ = ["ContinuousBatchEngine"]
 
@@ -121,8 +121,7 @@ class ContinuousBatchEngine:
         if vocab is not None and flat and not 0 <= min(flat) <= max(flat) < vocab:
             raise ValueError(f"token ids must lie in 0 .. {vocab - 1}")
         batch = RaggedBatch.build(counts, starts, slots, self.device, tables, self.kv.block_size)
-        tokens = torch.tensor(flat, dtype=torch.long, device=self.device)
-        widx = torch.tensor(want, dtype=torch.long, device=self.device)
+        tokens, widx = to_device(flat + want, torch.long, self.device).split([len(flat), len(want)])
         logits = self.model.forward_ragged(tokens, batch, self.kv, self.state, widx)
         for (seq_id, toks, _), s0 in zip(items, starts):
             self._cached[seq_id] = s0 + len(toks)

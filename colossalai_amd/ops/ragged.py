@@ -14,7 +14,19 @@ from typing import List, Optional, Sequence
 
 import torch
 
-__all__ = ["RaggedBatch"]
+from ._kernels import serving_kernels
+
+__all__ = ["RaggedBatch", "to_device"]
+
+LISTED_TOKENS = 32  # up to here a step's per-token vectors are made on the host: a launch takes as long
+
+
+def to_device(values: Sequence, dtype, device) -> torch.Tensor:
+    """A tensor of host numbers on `device`. To a GPU it goes from pinned memory and the host does not wait: a copy from pageable
+    memory waits for all the work ahead of it, so that the GPU then waits for what the host does next."""
+    if torch.device(device).type != "cuda":
+        return torch.tensor(values, dtype=dtype).to(device)
+    return torch.tensor(values, dtype=dtype, pin_memory=True).to(device, non_blocking=True)
 
 
 @dataclass
@@ -104,9 +116,15 @@ class RaggedBatch:
                 first.append(total_pages)
                 total_pages += n
             width = max(n + k for n, k in zip(pages, skip))
-            host = torch.tensor([first, pages, lens, skip], dtype=torch.int32).to(dev)   # one copy
-            first_d, pages_d, lens_d, skip_d = (host[i].long() for i in range(4))
+            host = to_device([first, pages, lens, skip], torch.int32, dev)   # one copy
             total = total_pages * ps
+            if self.block_tables.is_cuda:
+                rows = torch.empty(total, dtype=torch.long, device=dev)
+                tables = torch.empty(self.num_seqs, width, dtype=torch.int32, device=dev)
+                serving_kernels().dense_context(rows, tables, self.block_tables, host, ps)
+                self._dense[window] = (rows, tables, total)
+                return self._dense[window]
+            first_d, pages_d, lens_d, skip_d = (host[i].long() for i in range(4))
             seq = torch.repeat_interleave(torch.arange(self.num_seqs, device=dev), pages_d * ps, output_size=total)
             pos = torch.arange(total, device=dev) - (first_d - skip_d)[seq] * ps
             pos = torch.minimum(pos, lens_d[seq] - 1)
@@ -129,9 +147,16 @@ class RaggedBatch:
                 for t in range(lo, hi, size):
                     rows += [b, t, min(t + size, hi), 0]
                 ranges.append(len(rows) // 4)
-            buf = torch.tensor(rows + ranges, dtype=torch.int32).to(self.cu.device)
+            buf = to_device(rows + ranges, torch.int32, self.cu.device)
             self._chunk_tables[size] = (buf[: len(rows)].view(-1, 4), buf[len(rows):])
         return self._chunk_tables[size]
+
+    @staticmethod
+    def _fit_int32(starts, new_counts, pages, page_size) -> bool:
+        """Whether positions and pool rows are numbers that the device's 32-bit arithmetic makes, as they nearly always are; the
+        host's lists refuse others."""
+        return (min(starts) >= 0 and max(s + n for s, n in zip(starts, new_counts)) < 2 ** 31
+                and (not pages or (min(pages) >= 0 and (max(pages) + 1) * page_size <= 2 ** 31)))
 
     @classmethod
     def build(cls, new_counts: Sequence[int], starts: Sequence[int], slots: Sequence[int], device,
@@ -140,31 +165,33 @@ class RaggedBatch:
         for n in new_counts:
             assert n > 0, "a sequence in a step brings at least one token"
             cu.append(cu[-1] + n)
-        tok_seq, pos, rows = [], [], []
-        for i, n in enumerate(new_counts):
-            tok_seq += [i] * n
-            pos += list(range(starts[i], starts[i] + n))
-            if tables is not None:
-                t = tables[i]
-                assert len(t) * page_size >= starts[i] + n, "block table does not cover the new tokens"
-                rows += [t[p // page_size] * page_size + p % page_size for p in range(starts[i], starts[i] + n)]
-        # one host-to-device copy for all index vectors of the step; the fields are views into it
-        B = len(new_counts)
-        parts = [cu, list(starts), list(slots), tok_seq, pos]
-        width = 0
+        B, N, width = len(new_counts), cu[-1], 0
         if tables is not None:
+            for i, n in enumerate(new_counts):
+                assert len(tables[i]) * page_size >= starts[i] + n, "block table does not cover the new tokens"
             width = max(len(t) for t in tables)
-            parts += [[p for t in tables for p in list(t) + [0] * (width - len(t))], rows]
-        flat = [v for part in parts for v in part]
-        buf = torch.tensor(flat, dtype=torch.int32).to(device)
-        sizes = [len(part) for part in parts]
-        views, at = [], 0
-        for n in sizes:
-            views.append(buf[at : at + n])
-            at += n
+        # one host-to-device copy for all index vectors of the step; the fields are views into it
+        parts = [cu, list(starts), list(slots), [p for t in tables or () for p in list(t) + [0] * (width - len(t))]]
+        sizes = [B + 1, B, B, B * width, N, N, N if tables is not None else 0]
+        if torch.device(device).type == "cuda" and N > LISTED_TOKENS and cls._fit_int32(starts, new_counts, parts[3], page_size):
+            # a token's own entries are filled in on the device
+            buf = torch.empty(sum(sizes), dtype=torch.int32, device=device)
+            head = torch.tensor([v for part in parts for v in part], dtype=torch.int32, pin_memory=True)
+            buf[: head.numel()].copy_(head, non_blocking=True)
+            serving_kernels().ragged_index(buf, B, N, width, page_size)
+        else:
+            tok_seq, pos, rows = [], [], []
+            for i, n in enumerate(new_counts):
+                tok_seq += [i] * n
+                pos += list(range(starts[i], starts[i] + n))
+                if tables is not None:
+                    t = tables[i]
+                    rows += [t[p // page_size] * page_size + p % page_size for p in range(starts[i], starts[i] + n)]
+            buf = to_device([v for part in parts + [tok_seq, pos, rows] for v in part], torch.int32, device)
+        cu_d, start_d, slots_d, tables_d, tok_seq_d, pos_d, rows_d = buf.split(sizes)
         return cls(
-            cu=views[0], start=views[1], slots=views[2], tok_seq=views[3], positions=views[4],
-            block_tables=views[5].view(B, width) if tables is not None else None,
-            kv_rows=views[6] if tables is not None else None,
+            cu=cu_d, start=start_d, slots=slots_d, tok_seq=tok_seq_d, positions=pos_d,
+            block_tables=tables_d.view(B, width) if tables is not None else None,
+            kv_rows=rows_d if tables is not None else None,
             cu_host=cu, start_host=list(starts), slots_host=list(slots), page_size=page_size,
         )

@@ -386,3 +386,26 @@ def test_expert_sort(N, top, E):
     assert offsets.tolist() == offsets_ref.tolist()
     assert src.tolist() == (order // top).tolist()
     assert inv.reshape(-1).tolist() == inv_ref.tolist()
+
+
+@pytest.mark.parametrize("counts,starts", [([33], [0]), ([1] * 40, list(range(0, 800, 20))), ([1, 300, 1, 257, 5], [70, 0, 1, 513, 16]),
+                                           ([256, 256], [64, 0]), ([4096], [1])])
+@pytest.mark.parametrize("page", [1, 16, 64])
+def test_index_vectors_of_a_step(counts, starts, page):
+    """Those made on the device are those made on the host, also of the dense layout of whole contexts."""
+    from colossalai_amd.ops.ragged import RaggedBatch
+
+    tables, at = [], 3
+    for i, (n, s) in enumerate(zip(counts, starts)):
+        need = (n + s + page - 1) // page + i % 2
+        tables.append(list(range(at + need, at, -1)))
+        at += need
+    slots = list(range(len(counts)))[::-1]
+    for paged in (True, False):
+        gpu, cpu = (RaggedBatch.build(counts, starts, slots, d, tables if paged else None, page if paged else 0) for d in ("cuda", "cpu"))
+        for name in ("cu", "start", "slots", "tok_seq", "positions", "block_tables", "kv_rows"):
+            a, b = getattr(gpu, name), getattr(cpu, name)
+            assert (a is None and b is None) or (a.dtype == b.dtype and torch.equal(a.cpu(), b)), name
+        for window in (0, 50, 5000) if paged else ():
+            for a, b in zip(gpu.dense_context(window), cpu.dense_context(window)):
+                assert a == b if isinstance(a, int) else a.dtype == b.dtype and torch.equal(a.cpu(), b)
