@@ -56,4 +56,13 @@ typedef const __attribute__((address_space(1))) void* global_ptr;
 // every load of this wave has arrived (in LDS); a barrier behind it makes that true for the block
 DEV_INLINE void loads_done() { __builtin_amdgcn_s_waitcnt(0x0f70); }   // vmcnt(0)
 
+// at most N vector memory operations of this wave are on their way; what follows reads what the others brought
+template <int N>
+DEV_INLINE void loads_left() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | 0x0f70);
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_sched_barrier(0);
+}
+
 }  // namespace cai

@@ -47,15 +47,6 @@ DEV_INLINE float rounded_product(float a, float b) {
   return a * b;
 }
 
-// at most N vector memory operations of this wave are on their way; what follows reads what the others brought
-template <int N>
-DEV_INLINE void loads_left() {
-  asm volatile("" ::: "memory");
-  __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | 0x0f70);
-  asm volatile("" ::: "memory");
-  __builtin_amdgcn_sched_barrier(0);
-}
-
 __device__ __align__(16) const bf16s no_values[128] = {};   // a key's past the end
 
 // A part's state, for a block on any XCD to read: every access is one of its own at the scope of the device, past the L2 caches.
@@ -465,12 +456,12 @@ bool launch_group_attention(at::Tensor& out, const at::Tensor& q, const at::Tens
     if (slopes != nullptr && blocks <= 64 && keys <= 512) return false;
   }
   // Parts of the keys while there are fewer blocks than CUs. A tile of 32 keys takes a wave 1.75 us at 128 channels, of which eight run side by side;
-  // parts cost about 2 us, a store and three round trips to memory, and 0.1 each for reading their states. Whole, and in parts: 16 x 1024 (16 heads on
+  // parts cost 2 to 2.5 us, a store and three round trips to memory, and 0.1 each for reading their states. Whole, and in parts: 16 x 1024 (16 heads on
   // 4 of 128) 22.8 us, 2: 19.0, 4: 16.0, 8 (512 blocks): 22.8; 4 x 16384 277, 8: 48.4, 16: 36.6, 32: 41.4; 1 x 8192 66, 8: 17.4, 16: 14.4, 24:
   // 13.4, 64: 16.1; 1 x 2048 20.8, 4: 12.9, 12: 11.3, 16: 10.8; 16 x 300 (8 on 4) 9.3, 2: 10.6, 4: 9.9; 3 x 1500 (4 on 2 of 64) 12.3, 8: 8.2.
   const double whole = (double)((keys + 31) / 32) * 0.22 * (D + Dv) / 256;
   int splits = (int)std::max<long>(1, std::min<long>({256 / blocks, WAVE, std::lround(std::sqrt(whole * 10.0))}));
-  if (whole <= whole / splits + 2.0 + 0.1 * splits) splits = 1;
+  if (whole <= whole / splits + 2.5 + 0.1 * splits) splits = 1;
   // page numbers of a part: of its keys, rounded up to whole tiles, of a page more for where they begin, and of the kept ones
   const long part_keys = ((keys + 31) / 32 + splits - 1) / splits * 32;
   const size_t lds = (size_t)GROUP_WAVES * (D + Dv) * 64 + (size_t)((part_keys >> page_shift) + (keep_first >> page_shift) + 4) * sizeof(int);

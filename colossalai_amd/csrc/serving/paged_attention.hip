@@ -308,17 +308,18 @@ __global__ __launch_bounds__(64 * ATT_WAVES) void paged_attention_kernel(
 // The tiles are DS * 16 key channels by VT * 32 value channels; a head whose sizes Dr / Dvr are
 // smaller (multiples of 8) is padded with zeros on its way into registers and LDS, and only its
 // own channels are stored.
-// What bounds it: a step of 64 keys took each of a SIMD's two waves 9200 cycles (16 heads on 4 of 128, a cap and a sink), of which
-// 1600 went into issuing the step's loads together, 590 into storing them, 2500 (3850 with a cap) into the softmax. With loads that
-// go straight into LDS between the products, scalar branches for what a wave has in common and no maximum it is 5250 (6640):
-// 3140 of them are products. 243 of 256 registers at 128 channels.
-// One 4096-token prompt, 16 heads on 4 of 128, page 64: 196 us before, 138 with this, 115 with two groups of waves a block; a cap and a
-// sink 228, 167, 133; 16 heads of one key head each 201, 140, 120; 16 x 1024 after 100, 16 heads on 8: 287 -> 168, and with two token tiles a
-// block; 14 decode tokens beside portions of 1000 and 963, window 1024: 141 -> 76, and 65 with what has changed since; 2 x 256: 22.7 -> 15.1.
-// Value fragments read ahead changed nothing (138 to 140), no wave priorities cost 2 %.
+// What bounds it: the vector unit's issue. A product occupies the matrix unit for 32 cycles and the issue for 11, another instruction the issue for 4
+// to 5 (an exponential 8), for a SIMD's waves together; the halves of the weights, a cap and a penalty make 5 to 9 of these a product. In
+// phases (scores, weights, values) a wave's times for both add up, and two waves that meet at a barrier each step have the same phase; so
+// a wave's instructions alternate between the products of two tiles and the weights of a third (`turn`). 256 registers at 128 channels, a few spilled
+// around the loop; with the branches of several forms in one loop it was 60.
+// One 4096-token prompt, 16 heads on 4 of 128, page 64, us, in phases -> now: 131 -> 122, a cap and a sink 140 -> 127; 2000 tokens 64 -> 48, with a
+// cap 71 -> 54 (lanes past a sequence's last token repeat it, and its tiles need no masks for them); 3 x 200 after 1500 54 -> 42; 14
+// decode tokens beside portions of 1000 and 963, window 1024: 58 -> 53. A lone prompt of 40 or 100 tokens has one turn more in its chain, 11.1 -> 11.3
+// to 11.9. Weights' low halves by dot products with (-1, 0) instead of a shift, a mask and two differences: the same or slower.
 __device__ __align__(16) const bf16s zero_channels[8] = {0, 0, 0, 0, 0, 0, 0, 0};
 
-template <int DS, int VT, int NG, bool MORE>
+template <int DS, int VT, int NG, int FORM>
 __global__ __launch_bounds__(256 * NG, 2) void paged_attention_mfma_kernel(
     bf16s* __restrict__ out, const bf16s* __restrict__ q, long q_stride, const bf16s* __restrict__ kpool,
     const bf16s* __restrict__ vpool, const int* __restrict__ block_tables, int bt_stride, const int* __restrict__ cu,
@@ -327,7 +328,7 @@ __global__ __launch_bounds__(256 * NG, 2) void paged_attention_mfma_kernel(
     int tile_waves, const float* __restrict__ sink2, const float* __restrict__ dist2, int dist_rows,
     const bf16s* __restrict__ ksum, const bf16s* __restrict__ vsum, int sum_shift, int sum_block,
     float* __restrict__ cross_out, int chunk, const float* __restrict__ key_fac, int vrep, float* __restrict__ out32,
-    int num_tiles, int fewest) {
+    int num_tiles, int fewest, int seqs) {
   // The optional extras of the split-key kernel, in the base-2 domain: sink2 [H] = learned sink scores * log2e;
   // dist2 [H, dist_rows] = the per-distance bias * log2e, one row per head; ksum / vsum = block summaries, staged as
   // the first tiles of a block (summary idx of a sequence is seen by a token at pos when idx < (pos - window + 1) /
@@ -338,7 +339,9 @@ __global__ __launch_bounds__(256 * NG, 2) void paged_attention_mfma_kernel(
   // the one head, or two tiles of the two heads, instead of four heads; a block covers 128 or 64 tokens then, which is what `num_tiles`
   // counts, and the staged key/value tiles are still shared by all computing waves. The block stages the key range of all
   // its tokens; a wave skips the tiles that lie wholly after its own tokens.
-  // MORE = false: no block summaries, no distance table; with their branches in it the common form has no registers left
+  // FORM 0: no block summaries, no distance table; with their branches in it the common form has no registers left. 1: all there is. 2: capped
+  // scores and a sink, against the fixed reference (see below), and nothing else on the scores
+  constexpr bool MORE = FORM == 1, CAPPED = FORM == 2;
   if constexpr (!MORE) ksum = vsum = nullptr, dist2 = nullptr;
   constexpr int D = DS * 16, Dv = VT * 32;
   bf16x8_v zero8;
@@ -348,7 +351,7 @@ __global__ __launch_bounds__(256 * NG, 2) void paged_attention_mfma_kernel(
   constexpr int KQ = (D + 31) / 32, VQ = VT;            // pieces side by side
   constexpr int KT = KQ * 2048, VTT = VQ * 2048;        // bytes of one staged tile
   constexpr int TP = MFMA_TILES_PER_STEP, TS = NG * TP;   // tiles of a step: a group's, the block's
-  extern __shared__ __align__(16) char tiles[];  // [2][TS][KT + VTT], then [2][TS][32] key factors (float)
+  extern __shared__ __align__(16) char tiles[];  // [NG][2][TP] key tiles and [2][TP] value tiles, then [3][TS][32] key factors (float)
   float* facs = reinterpret_cast<float*>(tiles + 2 * TS * (KT + VTT));
   constexpr int nthreads = 256;  // of a group, always four waves: those beyond the kv head's group of heads only help staging
   const int tid = threadIdx.x & 255, grp = NG > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 8) : 0;
@@ -380,20 +383,38 @@ __global__ __launch_bounds__(256 * NG, 2) void paged_attention_mfma_kernel(
   const int hl = (zrow / VC) * heads + (wid >> tile_waves);  // head inside the group
   const int h = g * rep + (hl < rep ? hl : 0);
   const int bshift = 5 + tile_waves;                  // log2 of the tokens a block covers
-  for (;; ++b) {  // there are exactly sum_b ceil(count_b / tokens per block) tiles, of the sequences of `fewest` tokens or more
-    const int count = cu[b + 1] - cu[b], nt = count < fewest ? 0 : (count + (1 << bshift) - 1) >> bshift;
-    if (tile < nt) break;
-    tile -= nt;
+  // The block's sequence, 64 a time: there are exactly sum_b ceil(count_b / tokens per block) tiles, of the sequences of `fewest` tokens or more.
+  // (One by one a step of 16 sequences took 4700 cycles here.)
+  int first, cnt, s0;   // its first token, number of tokens, of tokens before them
+  for (int b0 = 0;; b0 += 64) {
+    const int at = min(b0 + lane, seqs - 1), from = cu[at], count = cu[at + 1] - from, held = start[at];
+    const int own = b0 + lane >= seqs || count < fewest ? 0 : (count + (1 << bshift) - 1) >> bshift;
+    int upto = own;   // summed over the lanes up to this one: inside rows of 16, then over the rows
+    upto += __builtin_amdgcn_update_dpp(0, upto, 0x111, 0xf, 0xf, false);
+    upto += __builtin_amdgcn_update_dpp(0, upto, 0x112, 0xf, 0xf, false);
+    upto += __builtin_amdgcn_update_dpp(0, upto, 0x114, 0xf, 0xf, false);
+    upto += __builtin_amdgcn_update_dpp(0, upto, 0x118, 0xf, 0xf, false);
+    upto += __builtin_amdgcn_update_dpp(0, upto, 0x142, 0xa, 0xf, false);
+    upto += __builtin_amdgcn_update_dpp(0, upto, 0x143, 0xc, 0xf, false);
+    const unsigned long long past = __ballot(tile < upto);
+    if (past != 0 || b0 + 64 >= seqs) {
+      const int at_lane = past != 0 ? __builtin_ctzll(past) : 63;
+      b = b0 + at_lane;
+      first = __builtin_amdgcn_readlane(from, at_lane);
+      cnt = __builtin_amdgcn_readlane(count, at_lane);
+      s0 = __builtin_amdgcn_readlane(held, at_lane);
+      tile -= __builtin_amdgcn_readlane(upto - own, at_lane);
+      break;
+    }
+    tile -= __builtin_amdgcn_readlane(upto, 63);
   }
-  const int cnt = cu[b + 1] - cu[b];
   const int col = lane & 31, hf = lane >> 5;
   const int bt_off = tile << bshift;                          // first token of the block
   const int t_off = bt_off + (wid & ((1 << tile_waves) - 1)) * 32;  // first token of this wave
   const bool head_ok = hl < rep && t_off < cnt;               // this wave computes
   const bool tok_ok = t_off + col < cnt;
   const int my_i = tok_ok ? t_off + col : cnt - 1;
-  const long n = cu[b] + my_i;
-  const int s0 = start[b];
+  const long n = first + my_i;
   const int pos = s0 + my_i;
   const int p0 = s0 + t_off, p1 = s0 + min(t_off + 31, cnt - 1);              // this wave's positions
   const int bp0 = s0 + bt_off, bp1 = s0 + min(bt_off + (1 << bshift) - 1, cnt - 1);  // the block's
@@ -454,7 +475,7 @@ __global__ __launch_bounds__(256 * NG, 2) void paged_attention_mfma_kernel(
     bool from_sum[TP];  // a summary tile
   };
   // Steps go from the nearest keys to the farthest. The other way round the scores of a head with a steep distance penalty rise by
-  // more than 12 from step to step, so that every step raises the reference and takes its weights twice (4000 tokens, window 1024:
+  // more than 30 from step to step, so that many steps raise the reference and take their weights twice (with 12: 4000 tokens, window 1024:
   // 83 us, 75 this way; 14 decode tokens beside portions of 1000 and 963: 72, 65). Without a penalty it is all the same (4096
   // tokens 125 and 125 us), but a way that depends on the call costs 2 to 3 %.
   const int steps_n = (tiles_n + TS - 1) / TS;
@@ -472,30 +493,27 @@ __global__ __launch_bounds__(256 * NG, 2) void paged_attention_mfma_kernel(
     return r;
   };
   const char* zeros = reinterpret_cast<const char*>(zero_channels);
-  auto key_piece = [&](const Rows& r, char* __restrict__ dst, int u, int n) __attribute__((always_inline)) {
-    const int quad = quad0 + 2 * n;
-    if (KQ % 2 != 0 && quad >= KQ) return;
-    const char* at = reinterpret_cast<const char*>((r.from_sum[u] ? ksum : kpool) + (long)g * Dr + quad * 32 + lch) +
-                     (unsigned long)(unsigned)r.key[u] * krs;
-    if (quad * 32 + lch >= Dr) at = zeros;
-    __builtin_amdgcn_global_load_lds((global_ptr)at, (lds_ptr)(dst + u * (KT + VTT) + (quad * 2 + row_group) * 1024), 16, 0, 0);
+  // Pieces of a step's keys (to the step's place among the two of them) and values, n of the wave's TP * KR and TP * VR. Head sizes that fill the
+  // tiles, as nearly all do, need no look at the channel.
+  auto piece = [&](const char* row, int n, int channels, char* __restrict__ dst) __attribute__((always_inline)) {
+    const int quad = quad0 + 2 * (n / TP);
+    const char* at = row + (n / TP) * 128;
+    if (channels % 64 != 0 && quad * 32 + lch >= channels) at = zeros;
+    __builtin_amdgcn_global_load_lds((global_ptr)at, (lds_ptr)(dst + (quad * 2 + row_group) * 1024), 16, 0, 0);
   };
-  auto value_piece = [&](const Rows& r, char* __restrict__ dst, int u, int n) __attribute__((always_inline)) {
-    const int quad = quad0 + 2 * n;
-    if (VQ % 2 != 0 && quad >= VQ) return;
-    const char* at = reinterpret_cast<const char*>((r.from_sum[u] ? vsum : vpool) + (long)vg * Dvr + quad * 32 + lch) +
-                     (unsigned long)(unsigned)r.key[u] * vrs;
-    if (quad * 32 + lch >= Dvr) at = zeros;
-    __builtin_amdgcn_global_load_lds((global_ptr)at, (lds_ptr)(dst + u * (KT + VTT) + KT + (quad * 2 + row_group) * 1024), 16, 0, 0);
+  auto key_row = [&](const Rows& r, int u) {
+    return reinterpret_cast<const char*>((r.from_sum[u] ? ksum : kpool) + (long)g * Dr + quad0 * 32 + lch) + (unsigned long)(unsigned)r.key[u] * krs;
   };
-  auto all_pieces = [&](const Rows& r, char* __restrict__ dst) __attribute__((always_inline)) {
-#pragma unroll
-    for (int u = 0; u < TP; ++u) {
-#pragma unroll
-      for (int n = 0; n < KR; ++n) key_piece(r, dst, u, n);
-#pragma unroll
-      for (int n = 0; n < VR; ++n) value_piece(r, dst, u, n);
-    }
+  auto value_row = [&](const Rows& r, int u) {
+    return reinterpret_cast<const char*>((r.from_sum[u] ? vsum : vpool) + (long)vg * Dvr + quad0 * 32 + lch) + (unsigned long)(unsigned)r.key[u] * vrs;
+  };
+  auto key_piece = [&](const char* const (&row)[TP], char* __restrict__ dst, int n) __attribute__((always_inline)) {
+    if (KQ % 2 != 0 && quad0 + 2 * (n / TP) >= KQ) return;
+    piece(row[n % TP], n, Dr, dst + n % TP * KT);
+  };
+  auto value_piece = [&](const char* const (&row)[TP], char* __restrict__ dst, int n) __attribute__((always_inline)) {
+    if (VQ % 2 != 0 && quad0 + 2 * (n / TP) >= VQ) return;
+    piece(row[n % TP], n, Dvr, dst + n % TP * VTT);
   };
   float rf[TP];
   auto fetch_factors = [&](const Rows& r) {
@@ -503,20 +521,21 @@ __global__ __launch_bounds__(256 * NG, 2) void paged_attention_mfma_kernel(
     for (int u = 0; u < TP; ++u)
       if (key_fac != nullptr && tid < 32) rf[u] = key_fac[(long)r.fac[u] * G + g];
   };
-  auto stash_factors = [&](int buf) {
+  // of a step among three: a step's last tile is weighted in the next one, when the factors of the one after that arrive
+  auto stash_factors = [&](int at) {
 #pragma unroll
     for (int u = 0; u < TP; ++u)
-      if (key_fac != nullptr && tid < 32) facs[(buf * TS + grp * TP + u) * 32 + tid] = rf[u];
+      if (key_fac != nullptr && tid < 32) facs[(at * TS + grp * TP + u) * 32 + tid] = rf[u];
   };
 
   // With a sink and a soft cap the scores live in [-cap2, cap2] (a distance penalty only lowers them) and the
   // denominator holds the sink's exp2(0) = 1: the weights can be taken against the fixed reference 0 instead of a
   // running maximum. exp2(cap2) cannot overflow for cap2 <= 96, and a weight that underflows is nothing beside the
   // sink's 1. No maximum to track, no accumulator to rescale.
-  const bool fixed_ref = sink != 0 && softcap > 0.0f && softcap * 1.4426950408889634f <= 96.0f;
+  const bool fixed_ref = CAPPED || (sink != 0 && softcap > 0.0f && softcap * 1.4426950408889634f <= 96.0f);
   // Without one, m is a maximum the token has had, not always its newest: weights are taken against it as it stands, and
-  // only where the sum of a step's weights shows that some passed 2^12 (a token's first visible score gives inf; NaN counts
-  // too) is the maximum formed, m raised and the weights taken again. A weight of 2^12 has the mantissa of one of 1.
+  // only where the sum of a tile's weights shows that some passed 2^30 (a token's first visible score gives inf; NaN counts
+  // too) is the maximum formed, m raised and the weights taken again. A weight of 2^30 has the mantissa of one of 1.
   float m = fixed_ref ? 0.0f : -INFINITY, l = 0.0f;  // m in the base-2 domain
   float m_ref = fixed_ref ? 0.0f : -3.0e38f;         // m, and below every finite score until there is one
   f32x16 oacc[VT];
@@ -528,19 +547,20 @@ __global__ __launch_bounds__(256 * NG, 2) void paged_attention_mfma_kernel(
   // a scale of 0 must not meet -inf in a product, one of NaN stays (fmaxf drops it)
   const float c1 = scale * LOG2E < 1e-30f ? 1e-30f : scale * LOG2E, sl2 = slope * LOG2E;
   // soft cap in the base-2 domain: cap log2e tanh(x scale / cap), tanh(y) = 1 - 2 / (exp2(2 log2e y) + 1)
-  const bool capped = softcap > 0.0f;
+  const bool capped = CAPPED || softcap > 0.0f;
   const float inv_cap = capped ? scale / softcap : 0.0f;
   const float cap2 = softcap * LOG2E, t2 = capped ? 2.0f * LOG2E * scale / softcap : 0.0f;
-  const float cc0 = cap2, cc1 = cap2 * -0.33333069f, cc2 = cap2 * 0.13324751f, cc3 = cap2 * -0.052984238f, cc4 = cap2 * 0.017131345f;
+  // of the polynomial in x^2
+  struct Poly {
+    float c0, c1, c2, c3, c4;
+  };
+  const float ic2 = inv_cap * inv_cap, ic4 = ic2 * ic2, cx = cap2 * inv_cap;
+  const Poly cap_poly{cx, cx * ic2 * -0.33333069f, cx * ic4 * 0.13324751f, cx * ic4 * ic2 * -0.052984238f, cx * ic4 * ic4 * 0.017131345f};
   auto cap_base2 = [&](float dot) {
     const float e = __builtin_amdgcn_exp2f(dot * t2);  // +inf: the quotient is 0; a NaN stays one
     return cap2 - 2.0f * cap2 * __builtin_amdgcn_rcpf(e + 1.0f);
   };
-  // A key's share of the distance penalty: its offset inside its tile (row of the C layout) here, the tile's per tile
-  const bool sloped = slopes != nullptr;
-  float row_bias[16];
-#pragma unroll
-  for (int i = 0; i < 16; ++i) row_bias[i] = sl2 * (float)((i & 3) + 8 * (i >> 2) + 4 * hf);
+  const bool sloped = !CAPPED && slopes != nullptr;
   // Without a cap, a penalty or a table the scores stay raw products and their factor enters with the fma that
   // subtracts the reference (a negative factor has moved into the query); otherwise they are formed in the base-2 domain.
   const bool raw = !capped && !sloped && db == nullptr;
@@ -549,225 +569,335 @@ __global__ __launch_bounds__(256 * NG, 2) void paged_attention_mfma_kernel(
   const RowAt row_at(col, hf);
   const ColAt col_at(lane);
   Rows next = lookup(first_tile);
-  char* mine = tiles + grp * TP * (KT + VTT);     // this group's tiles of the first buffer
-  constexpr int BUF = TS * (KT + VTT);
-  all_pieces(next, mine);
+  // this group's place: [2] steps' keys, [2] steps' values
+  constexpr int KS = TP * KT, VS = TP * VTT;
+  char* keys = tiles + grp * (2 * KS + 2 * VS);
+  char* values = keys + 2 * KS;
+  const char *krow[TP], *vrow[TP];
+#pragma unroll
+  for (int u = 0; u < TP; ++u) krow[u] = key_row(next, u);
+#pragma unroll
+  for (int n = 0; n < TP * KR; ++n) key_piece(krow, keys, n);
   fetch_factors(next);
+#pragma unroll
+  for (int u = 0; u < TP; ++u) vrow[u] = value_row(next, u);
+  Rows of_values = next;
   if (steps_n > 1) next = lookup(first_tile + way);
   stash_factors(0);
-  loads_done();
+  __builtin_amdgcn_sched_barrier(0);
+  // the first step's values behind its keys: they are not waited for yet
+#pragma unroll
+  for (int n = 0; n < TP * VR; ++n) value_piece(vrow, values, n);
+  if (quad0 == 0) loads_left<TP * VR>();
+  else loads_left<TP * (VQ / 2)>();
   __syncthreads();
 
-  // A step's tiles of this wave, while the next step's arrive in the other buffer.
-  auto compute = [&](int it0, int kb0, bool inner, const bool (&live)[TP], int buf, const Rows& next, const char* __restrict__ cur,
-                     char* __restrict__ dst) __attribute__((always_inline)) {
-    f32x16 x[TP];
-    float off[TP];
+  // What a tile's scores go through before they are weights: factors, the cap, a penalty or a table, masks. `it` is the tile, `fc` its keys' factors.
+  struct Tile {
+    int it, kbase;
+    bool summ, inner, live;
+  };
+  auto tile_of = [&](int it) {
+    Tile t;
+    t.it = it;
+    t.kbase = tile_base(it);
+    t.summ = MORE && it < sum_tiles;
+    // inner: every key is visible to every token of the wave (lanes past the last one repeat it), no masks to evaluate
+    t.inner = head_ok && it >= sink_tiles && t.kbase >= lo_p1 && t.kbase + 31 <= p0;
+    // (several token tiles) a tile wholly after this wave's tokens, or wholly before what they see, is not live
+    t.live = t.inner || (head_ok && it < tiles_n && (it < sink_tiles || !(t.kbase > p1 || (t.kbase + 31 < lo_p0 && t.kbase >= keep_first))));
+    return t;
+  };
+  auto factors = [&](f32x16& x, int place) __attribute__((always_inline)) {
+    if (key_fac != nullptr) {
+      const float* fc = facs + place * 32 + 4 * hf;
 #pragma unroll
-    for (int u = 0; u < TP; ++u)
+      for (int a = 0; a < 4; ++a) {
+        const float4v f4 = *reinterpret_cast<const float4v*>(fc + 8 * a);
 #pragma unroll
-      for (int i = 0; i < 16; ++i) x[u][i] = 0.0f;
-    // the key fragments are read AHEAD products ahead of their own
-    constexpr int AHEAD = 6, NF = DS * TP;
-    bf16x8_v kf[NF];
-    __builtin_amdgcn_s_setprio(1);
-#pragma unroll
-    for (int i = 0; i < AHEAD && i < NF; ++i) kf[i] = frag_row<32>(cur + i % TP * (KT + VTT), row_at, 0, i / TP);
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int i = 0; i < NF; ++i) {
-      if (i + AHEAD < NF) kf[i + AHEAD] = frag_row<32>(cur + (i + AHEAD) % TP * (KT + VTT), row_at, 0, (i + AHEAD) / TP);
-      x[i % TP] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[i], qf[i / TP], x[i % TP], 0, 0, 0);
-#pragma unroll
-      for (int n = i * (TP * KR) / NF; n < (i + 1) * (TP * KR) / NF; ++n) key_piece(next, dst, n % TP, n / TP);
-      __builtin_amdgcn_sched_barrier(0);
-    }
-    __builtin_amdgcn_s_setprio(0);
-#pragma unroll
-    for (int u = 0; u < TP; ++u) {
-      const int it = it0 + u, kbase = inner ? kb0 + 32 * u : tile_base(it);
-      const bool summ = MORE && !inner && it < sum_tiles;
-      if (key_fac != nullptr) {
-        const float* fc = facs + (buf * TS + grp * TP + u) * 32 + 4 * hf;
-#pragma unroll
-        for (int a = 0; a < 4; ++a) {
-          const float4v f4 = *reinterpret_cast<const float4v*>(fc + 8 * a);
-#pragma unroll
-          for (int c = 0; c < 4; ++c) x[u][4 * a + c] *= f4[c];
-        }
+        for (int c = 0; c < 4; ++c) x[4 * a + c] *= f4[c];
       }
-      off[u] = sloped && !summ ? -sl2 * (float)(pos - kbase) : 0.0f;
     }
+  };
+  // tanh(y) = y P(y^2) for |y| <= 1/2, P a polynomial through the Chebyshev nodes (1.3e-8 off): fused
+  // multiplications where the general form takes an exponential and a reciprocal
+  auto near = [&](const f32x16& x) __attribute__((always_inline)) {
+    float far = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 16; i += 2) asm("v_max3_f32 %0, %0, |%1|, |%2|" : "+v"(far) : "v"(x[i]), "v"(x[i + 1]));   // fmaxf makes two and a half of it
+    return __all(far * fabsf(inv_cap) <= 0.5f);
+  };
+  auto near_cap = [&](f32x16& x) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const float z = x[i] * x[i];
+      x[i] *= fmaf(z, fmaf(z, fmaf(z, fmaf(z, cap_poly.c4, cap_poly.c3), cap_poly.c2), cap_poly.c1), cap_poly.c0);
+    }
+  };
+  auto prepare = [&](const Tile& t, f32x16& x) __attribute__((always_inline)) {
     if (capped) {
-      // tanh(y) = y P(y^2) for |y| <= 1/2, P a polynomial through the Chebyshev nodes (1.3e-8 off): fused
-      // multiplications where the general form takes an exponential and a reciprocal
-      float far = 0.0f;
-#pragma unroll
-      for (int u = 0; u < TP; ++u)
-#pragma unroll
-        for (int i = 0; i < 16; ++i) far = fmaxf(far, fabsf(x[u][i]));
-      if (__all(far * fabsf(inv_cap) <= 0.5f)) {
-#pragma unroll
-        for (int u = 0; u < TP; ++u)
-#pragma unroll
-          for (int i = 0; i < 16; ++i) {
-            const float y = x[u][i] * inv_cap, z = y * y;
-            x[u][i] = y * fmaf(z, fmaf(z, fmaf(z, fmaf(z, cc4, cc3), cc2), cc1), cc0);
-          }
+      if (near(x)) {
+        near_cap(x);
       } else {
 #pragma unroll
-        for (int u = 0; u < TP; ++u)
-#pragma unroll
-          for (int i = 0; i < 16; ++i) x[u][i] = cap_base2(x[u][i]);
+        for (int i = 0; i < 16; ++i) x[i] = cap_base2(x[i]);
       }
     }
     if (!raw) {
+      if (sloped && !t.summ) {
+        // a key's share of the distance penalty, its offset inside the tile (row of the C layout); the tile's own comes with the reference
 #pragma unroll
-      for (int u = 0; u < TP; ++u) {
-        const int it = it0 + u, kbase = inner ? kb0 + 32 * u : tile_base(it);
-        const bool summ = MORE && !inner && it < sum_tiles;
-        if (sloped && !summ) {
-          if (capped) {
+        for (int i = 0; i < 16; ++i) x[i] = fmaf(sl2, (float)((i & 3) + 8 * (i >> 2)), capped ? x[i] : x[i] * c1);
+      } else if (!capped) {
 #pragma unroll
-            for (int i = 0; i < 16; ++i) x[u][i] += row_bias[i];
-          } else {
-#pragma unroll
-            for (int i = 0; i < 16; ++i) x[u][i] = fmaf(x[u][i], c1, row_bias[i]);
-          }
-        } else if (!capped) {
-#pragma unroll
-          for (int i = 0; i < 16; ++i) x[u][i] *= c1;
-        }
-        if (db != nullptr && !summ) {
-#pragma unroll
-          for (int i = 0; i < 16; ++i) {
-            const int j = kbase + (i & 3) + 8 * (i >> 2) + 4 * hf;
-            x[u][i] += db[min(max(pos - j, 0), dist_rows - 1)];
-          }
-        }
+        for (int i = 0; i < 16; ++i) x[i] *= c1;
       }
-    }
-    if (!inner) {
-#pragma unroll
-      for (int u = 0; u < TP; ++u) {
-        const int it = it0 + u, kbase = tile_base(it);
-        const bool summ = MORE && it < sum_tiles;
-        const bool ahead = it < sink_tiles;  // a tile ahead of the window's: summaries or kept first tokens
-        // the tile's keys that this token sees: those up to `last`, from `first` on or below `keep` (offsets in the tile)
-        const int last = !live[u] || !tok_ok ? -1 : summ ? my_sum - 1 - kbase : (ahead ? min(n_sink - 1, pos) : min(p1, pos)) - kbase;
-        const int first = summ ? 0 : lo - kbase, keep = summ ? 0 : keep_first - kbase;
+      if (db != nullptr && !t.summ) {
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
-          const int j = (i & 3) + 8 * (i >> 2) + 4 * hf;
-          x[u][i] = (j <= last) & ((j >= first) | (j < keep)) ? x[u][i] : -INFINITY;
+          const int j = t.kbase + (i & 3) + 8 * (i >> 2) + 4 * hf;
+          x[i] += db[min(max(pos - j, 0), dist_rows - 1)];
         }
       }
-      asm volatile("" ::: "memory");   // a body of its own: merged into the common one, every step would pay for it
     }
-    bf16x8_v phi[TP][2], plo[TP][2];
-    auto weights = [&](auto plain) __attribute__((always_inline)) {
-      float psum = 0.0f;
+    if (!t.inner) {
+      const bool ahead = t.it < sink_tiles;  // a tile ahead of the window's: summaries or kept first tokens
+      // the tile's keys that this token sees: those up to `last`, from `first` on or below `keep` (offsets in the tile)
+      const int last = !t.live ? -1 : t.summ ? my_sum - 1 - t.kbase : (ahead ? min(n_sink - 1, pos) : min(p1, pos)) - t.kbase;
+      const int first = t.summ ? 0 : lo - t.kbase, keep = t.summ ? 0 : keep_first - t.kbase;
 #pragma unroll
-      for (int u = 0; u < TP; ++u) {
-        const float base = off[u] - m_ref;
-#pragma unroll
-        for (int i = 0; i < 16; i += 2) {  // two weights a time: one conversion packs two halves
-          const float p0 = __builtin_amdgcn_exp2f(plain ? x[u][i] : fmaf(x[u][i], k1, base));
-          const float p1 = __builtin_amdgcn_exp2f(plain ? x[u][i + 1] : fmaf(x[u][i + 1], k1, base));
-          psum += p0 + p1;
-          const bf16x2_v hi = __builtin_convertvector(float2v{p0, p1}, bf16x2_v);
-          const unsigned bits = __builtin_bit_cast(unsigned, hi);
-          const bf16x2_v lo = __builtin_convertvector(float2v{p0 - __builtin_bit_cast(float, bits << 16),
-                                                              p1 - __builtin_bit_cast(float, bits & 0xffff0000u)}, bf16x2_v);
-          phi[u][i >> 3][i & 7] = hi[0];
-          phi[u][i >> 3][(i & 7) + 1] = hi[1];
-          plo[u][i >> 3][i & 7] = lo[0];
-          plo[u][i >> 3][(i & 7) + 1] = lo[1];
-        }
+      for (int i = 0; i < 16; ++i) {
+        const int j = (i & 3) + 8 * (i >> 2) + 4 * hf;
+        x[i] = (j <= last) & ((j >= first) | (j < keep)) ? x[i] : CAPPED ? -1e18f : -INFINITY;   // finite where its square meets 0
       }
-      return psum;
-    };
-    float psum;
-    if (fixed_ref && !sloped) {   // scores in the base-2 domain, against 0
-      psum = weights(std::true_type());
-      asm volatile("" ::: "memory");
+      asm volatile("" ::: "memory");   // a body of its own: merged into the common one, every tile would pay for it
+    }
+  };
+  constexpr std::true_type yes{};
+  constexpr std::false_type no{};
+  struct Weights {
+    bf16x8_v hi[2], lo[2];
+  };
+  // Two weights in stages: (0) with CAPPED, where the near form of the cap is a part of them, and (1) the exponentials, (2) sum and high halves, (3)
+  // low halves; one conversion packs two. A tile that has been through `prepare` takes the polynomial 1.
+  struct Pair {
+    float a, b, za, zb;
+    unsigned bits;
+  };
+  auto stage = [&](int k, const Poly& c, const f32x16& x, float base, int i, Pair& s, float& psum, Weights& p) __attribute__((always_inline)) {
+    if (k == 0) {
+      s.za = x[i] * x[i];
+      s.zb = x[i + 1] * x[i + 1];
+      s.a = fmaf(s.za, c.c4, c.c3);
+      s.b = fmaf(s.zb, c.c4, c.c3);
+      s.a = fmaf(s.za, s.a, c.c2);
+      s.b = fmaf(s.zb, s.b, c.c2);
+    } else if (k == 1) {
+      if (CAPPED) {
+        s.a = fmaf(s.za, fmaf(s.za, s.a, c.c1), c.c0);
+        s.b = fmaf(s.zb, fmaf(s.zb, s.b, c.c1), c.c0);
+        s.a = __builtin_amdgcn_exp2f(x[i] * s.a);
+        s.b = __builtin_amdgcn_exp2f(x[i + 1] * s.b);
+      } else {
+        s.a = __builtin_amdgcn_exp2f(fmaf(x[i], k1, base));
+        s.b = __builtin_amdgcn_exp2f(fmaf(x[i + 1], k1, base));
+      }
+    } else if (k == 2) {
+      psum += s.a;
+      psum += s.b;
+      const bf16x2_v hi = __builtin_convertvector(float2v{s.a, s.b}, bf16x2_v);
+      s.bits = __builtin_bit_cast(unsigned, hi);
+      p.hi[i >> 3][i & 7] = hi[0];
+      p.hi[i >> 3][(i & 7) + 1] = hi[1];
     } else {
-      for (bool raised = false;; raised = true) {
-        psum = weights(std::false_type());
-        if (fixed_ref || raised || __all(psum <= 4096.0f)) break;
-        float tmax = -INFINITY;
+      const bf16x2_v lo = __builtin_convertvector(float2v{s.a - __builtin_bit_cast(float, s.bits << 16),
+                                                          s.b - __builtin_bit_cast(float, s.bits & 0xffff0000u)}, bf16x2_v);
+      p.lo[i >> 3][i & 7] = lo[0];
+      p.lo[i >> 3][(i & 7) + 1] = lo[1];
+    }
+  };
+  // where the sum of a tile's weights shows that some passed 2^30: the maximum, and the weights again
+  auto raise = [&](const f32x16& x, float off, float psum, Weights& p) __attribute__((always_inline)) {
+    if (!fixed_ref && !__all(psum <= 0x1p30f)) {
+      Pair again;
+      float top = x[0];
 #pragma unroll
-        for (int u = 0; u < TP; ++u) {
-          float top = x[u][0];
+      for (int i = 1; i < 16; ++i) top = fmaxf(top, x[i]);
+      float tmax = top == -INFINITY ? -INFINITY : fmaf(top, k1, off);
+      tmax = fmaxf(tmax, __shfl_xor(tmax, 32));
+      const float m_new = fmaxf(m, tmax);
+      const float corr = (m == -INFINITY) ? 1.0f : __builtin_amdgcn_exp2f(m - m_new);  // nothing accumulated: nothing to rescale
+      l *= corr;
 #pragma unroll
-          for (int i = 1; i < 16; ++i) top = fmaxf(top, x[u][i]);
-          tmax = fmaxf(tmax, top == -INFINITY ? -INFINITY : fmaf(top, k1, off[u]));
-        }
-        tmax = fmaxf(tmax, __shfl_xor(tmax, 32));
-        const float m_new = fmaxf(m, tmax);
-        const float corr = (m == -INFINITY) ? 1.0f : __builtin_amdgcn_exp2f(m - m_new);  // nothing accumulated: nothing to rescale
-        l *= corr;
+      for (int t = 0; t < VT; ++t)
 #pragma unroll
-        for (int t = 0; t < VT; ++t)
+        for (int i = 0; i < 16; ++i) oacc[t][i] *= corr;
+      m = m_new;
+      m_ref = (m_new == -INFINITY) ? -3.0e38f : m_new;  // nothing visible yet: every weight is exp2(-inf) = 0
+      psum = 0.0f;
 #pragma unroll
-          for (int i = 0; i < 16; ++i) oacc[t][i] *= corr;
-        m = m_new;
-        m_ref = (m_new == -INFINITY) ? -3.0e38f : m_new;  // nothing visible yet: every weight is exp2(-inf) = 0
-      }
+      for (int i = 0; i < 16; i += 2)
+#pragma unroll
+        for (int k = 1; k < 4; ++k) stage(k, cap_poly, x, off - m_ref, i, again, psum, p);
     }
     l += psum;
-    // O^T += V^T P^T: slot hf * 8 + e of step s2 holds key kbase + 16 s2 + 8 (e >> 2) + 4 hf + (e & 3)
-    __builtin_amdgcn_s_setprio(1);
-#pragma unroll
-    for (int u = 0; u < TP; ++u)
-#pragma unroll
-      for (int s2 = 0; s2 < 2; ++s2) {
-#pragma unroll
-        for (int t = 0; t < VT; ++t) {
-          const bf16x8_v va = frag_born<32>(cur + u * (KT + VTT) + KT, col_at, 16 * s2, 32 * t);
-          oacc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va, phi[u][s2], oacc[t], 0, 0, 0);
-          oacc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va, plo[u][s2], oacc[t], 0, 0, 0);
-        }
-        const int at = u * 2 + s2;
-#pragma unroll
-        for (int n = at * (TP * VR) / (2 * TP); n < (at + 1) * (TP * VR) / (2 * TP); ++n) value_piece(next, dst, n % TP, n / TP);
-      }
-    __builtin_amdgcn_s_setprio(0);
   };
-  int tile0 = first_tile;
-  for (int step = 0; step < steps_n; ++step, tile0 += way) {
-    const int buf = step & 1;
-    const Rows now = next;          // the next step's rows; its loads repeat the last step's where there is none
-    if (step + 2 < steps_n) next = lookup(tile0 + 2 * way);
-    if (step + 1 < steps_n) fetch_factors(now);
-    // The TP tiles of a step go through the softmax together: one sum, one look at the reference.
-    const int it0 = tile0 + grp * TP, kb0 = tile_base(it0);
-    // interior step: every key of its tiles is visible to every token of the wave, no masks to evaluate
-    const bool inner = head_ok && it0 >= sink_tiles && kb0 >= lo_p1 && kb0 + 32 * TP - 1 <= p0 && t_off + 31 < cnt;
-    bool live[TP];       // this wave sees something of the tile
-    bool any = inner;
+  auto offset = [&](const Tile& t) { return sloped && !t.summ ? -sl2 * (float)(pos - t.kbase - 4 * hf) : 0.0f; };
+
+  // One tile's turn: the scores of the tile after it (keys at `K_`) into `xn`, the weights of this one's scores `x` into `p`, and what the tile
+  // before it adds, its weights `pp` times the values at `V_`, none of which waits for another. A wave's instructions alternate between them, so that
+  // the matrix unit has work while the exponentials are formed.
+  // O^T += V^T P^T: slot hf * 8 + e of half s2 holds key 16 s2 + 8 (e >> 2) + 4 hf + (e & 3)
+  constexpr int GROUPS = DS > 2 * VT ? DS : 2 * VT, AHEAD = 2;
+  auto turn = [&](auto with_scores, auto with_weights, auto with_values, const Poly& poly, const char* __restrict__ K_, const char* __restrict__ V_,
+                  f32x16& xn, const f32x16& x, float off, Weights& p, const Weights& pp, auto load) __attribute__((always_inline)) {
+    bf16x8_v kf[DS], vf[2 * VT];
+    const float base = off - m_ref;
+    float psum = 0.0f;
+    Pair s[8];
+    auto read = [&](int i) __attribute__((always_inline)) {
+      if (with_scores && i < DS) kf[i] = frag_row<32>(K_, row_at, 0, i);
+      if (with_values && i < 2 * VT) vf[i] = frag_born<32>(V_, col_at, 16 * (i / VT), 32 * (i % VT));
+    };
+    // after product n of all: its share of the weights' stages. One product's time is that of eight other instructions, of which a wave issues
+    // none while its next product waits for the unit: they have to stand between the products.
+    constexpr int PRODUCTS = (decltype(with_scores)::value ? DS : 0) + (decltype(with_values)::value ? 4 * VT : 0);
+    auto weigh = [&](int n) __attribute__((always_inline)) {
+      constexpr int FROM = CAPPED ? 0 : 1, STAGES = 4 - FROM;
+      if (with_weights) {
+#pragma unroll
+        for (int k = n * 8 * STAGES / PRODUCTS; k < (n + 1) * 8 * STAGES / PRODUCTS; ++k)
+          stage(FROM + k % STAGES, poly, x, base, k / STAGES * 2, s[k / STAGES], psum, p);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    if (with_scores) {
+#pragma unroll
+      for (int i = 0; i < 16; ++i) xn[i] = 0.0f;
+    }
+#pragma unroll
+    for (int i = 0; i < AHEAD; ++i) read(i);
+    __builtin_amdgcn_sched_barrier(0);
+    int n = 0;
+#pragma unroll
+    for (int i = 0; i < GROUPS; ++i) {
+      read(i + AHEAD);
+      if (with_scores && i < DS) {
+        xn = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[i], qf[i], xn, 0, 0, 0);
+        weigh(n++);
+      }
+      if (with_values && i < 2 * VT) {
+        oacc[i % VT] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[i], pp.hi[i / VT], oacc[i % VT], 0, 0, 0);
+        weigh(n++);
+        oacc[i % VT] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[i], pp.lo[i / VT], oacc[i % VT], 0, 0, 0);
+        weigh(n++);
+      }
+      load(i);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    if (with_weights) {
+      // formed here: the compiler moves them to where they are used, behind the products
+#pragma unroll
+      for (int e = 0; e < 2; ++e) asm volatile("" : "+v"(p.hi[e]), "+v"(p.lo[e]));
+      raise(x, off, psum, p);
+    }
+  };
+  // the weights' turn of a tile, by what its scores need ahead of it
+  auto weights_turn = [&](auto with_scores, auto with_values, const Tile& t, int place, const char* __restrict__ K_, const char* __restrict__ V_,
+                          f32x16& xn, f32x16& x, Weights& p, const Weights& pp, auto load) __attribute__((always_inline)) {
+    factors(x, place);
+    Poly poly = cap_poly;
+    if (!CAPPED || !t.inner || !near(x)) {
+      prepare(t, x);
+      poly = Poly{1.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+    }
+    turn(with_scores, yes, with_values, poly, K_, V_, xn, x, offset(t), p, pp, load);
+  };
+  // Keys are a step ahead of values. In step s a wave forms the scores of the step's two tiles, the weights of the tile before them and
+  // of the first one, and adds what the two tiles of the step before are worth; the next step's keys and this step's values are on their way.
+  // Steps in which a wave has nothing to do yet (several token tiles) only load; one without tokens or a head does no other.
+  int tile0 = first_tile, step = 0, third = 0;   // third: the step's place among three
+  auto begin = [&]() __attribute__((always_inline)) {   // the next step's keys and this step's values; past the last step the loads repeat rows
+    const Rows now = next;
 #pragma unroll
     for (int u = 0; u < TP; ++u) {
-      const int it = it0 + u, kbase = tile_base(it);
-      // (several token tiles) a tile wholly after this wave's tokens, or wholly before what they see
-      live[u] = inner || (head_ok && it < tiles_n && (it < sink_tiles || !(kbase > p1 || (kbase + 31 < lo_p0 && kbase >= keep_first))));
-      any = any || live[u];
+      krow[u] = key_row(next, u);
+      vrow[u] = value_row(of_values, u);
     }
-    if (any) compute(it0, kb0, inner, live, buf, now, mine + buf * BUF, mine + (buf ^ 1) * BUF);
-    else all_pieces(now, mine + (buf ^ 1) * BUF);
-    if (step + 1 < steps_n) stash_factors(buf ^ 1);
+    of_values = next;
+    if (step + 2 < steps_n) next = lookup(tile0 + 2 * way);
+    if (step + 1 < steps_n) fetch_factors(now);
+  };
+  auto end = [&]() __attribute__((always_inline)) {
+    third = third == 2 ? 0 : third + 1;
+    if (step + 1 < steps_n) stash_factors(third);
     loads_done();
     __syncthreads();
+    ++step;
+    tile0 += way;
+  };
+  // all of them in the first of a step's two turns: those that go out last have to arrive before the step ends
+  auto load_keys = [&](int i) __attribute__((always_inline)) {
+#pragma unroll
+    for (int n = i * (TP * KR) / GROUPS; n < (i + 1) * (TP * KR) / GROUPS; ++n) key_piece(krow, keys + (~step & 1) * KS, n);
+  };
+  auto load_values = [&](int i) __attribute__((always_inline)) {
+#pragma unroll
+    for (int n = i * (TP * VR) / GROUPS; n < (i + 1) * (TP * VR) / GROUPS; ++n) value_piece(vrow, values + (step & 1) * VS, n);
+  };
+  auto load = [&](int i) __attribute__((always_inline)) {
+    load_keys(i);
+    load_values(i);
+  };
+  auto load_first = [&](int i) __attribute__((always_inline)) {   // the values of step 0 are on their way; a lone step waits for nothing more
+    if (step + 1 < steps_n) load_keys(i);
+    if (step > 0) load_values(i);
+  };
+  auto nothing = [](int) {};
+  auto idle = [&]() __attribute__((always_inline)) {
+    begin();
+#pragma unroll
+    for (int i = 0; i < GROUPS; ++i) load_first(i);
+    end();
+  };
+  auto mine_of = [&](int u) { return tile_of(tile0 + grp * TP + u); };
+  while (step < steps_n && !mine_of(0).live && !mine_of(1).live) idle();
+  if (step < steps_n) {
+    f32x16 xe, xo;            // scores of an even and an odd tile of the wave's
+    Weights pe, po;
+    {
+      begin();
+      const char* K_ = keys + (step & 1) * KS;
+      turn(yes, no, no, cap_poly, K_, K_, xe, xo, 0.0f, po, pe, load_first);
+      weights_turn(yes, no, mine_of(0), third * TS + grp * TP, K_ + KT, K_, xo, xe, pe, po, nothing);
+      end();
+    }
+    while (step < steps_n) {
+      const Tile odd = tile_of(tile0 - way + grp * TP + 1), even = mine_of(0);
+      begin();
+      const char* K_ = keys + (step & 1) * KS;
+      const char* V_ = values + (~step & 1) * VS;
+      weights_turn(yes, yes, odd, (third == 0 ? 2 : third - 1) * TS + grp * TP + 1, K_, V_, xe, xo, po, pe, load);
+      weights_turn(yes, yes, even, third * TS + grp * TP, K_ + KT, V_ + VTT, xo, xe, pe, po, nothing);
+      end();
+    }
+    const Tile odd = tile_of(tile0 - way + grp * TP + 1);
+    const char* V_ = values + (~step & 1) * VS;
+    weights_turn(no, yes, odd, (third == 0 ? 2 : third - 1) * TS + grp * TP + 1, V_, V_, xe, xo, po, pe, nothing);
+    turn(no, no, yes, cap_poly, V_, V_ + VTT, xo, xe, 0.0f, pe, po, nothing);
   }
-  if constexpr (NG > 1) {  // the second group's states, wave by wave, through the tiles' place (all waves are past their last tile)
-    float* state = reinterpret_cast<float*>(tiles) + wid * (VT * 16 + 2) * 64 + lane;
+  if constexpr (NG > 1) {  // the second group's states, wave by wave, through the tiles' place
+    __syncthreads();         // all waves are past their last tile
+    float4v* sums = reinterpret_cast<float4v*>(tiles) + wid * (VT * 4 * 64 + 32) + lane;   // 16 bytes an access
+    float* state = reinterpret_cast<float*>(sums - lane + VT * 4 * 64) + lane;
     if (grp == 1) {
       state[0] = m;
       state[64] = l;
 #pragma unroll
       for (int t = 0; t < VT; ++t)
 #pragma unroll
-        for (int i = 0; i < 16; ++i) state[(2 + t * 16 + i) * 64] = oacc[t][i];
+        for (int a = 0; a < 4; ++a)
+          sums[(t * 4 + a) * 64] = float4v{oacc[t][4 * a], oacc[t][4 * a + 1], oacc[t][4 * a + 2], oacc[t][4 * a + 3]};
     }
     __syncthreads();
     if (grp == 1) return;
@@ -778,7 +908,11 @@ __global__ __launch_bounds__(256 * NG, 2) void paged_attention_mfma_kernel(
 #pragma unroll
     for (int t = 0; t < VT; ++t)
 #pragma unroll
-      for (int i = 0; i < 16; ++i) oacc[t][i] = oacc[t][i] * f0 + state[(2 + t * 16 + i) * 64] * f1;
+      for (int a = 0; a < 4; ++a) {
+        const float4v other = sums[(t * 4 + a) * 64];
+#pragma unroll
+        for (int c = 0; c < 4; ++c) oacc[t][4 * a + c] = oacc[t][4 * a + c] * f0 + other[c] * f1;
+      }
     m = top;
   }
   l += __shfl_xor(l, 32);
@@ -914,20 +1048,27 @@ static bool launch_mfma_attention(at::Tensor& out, const at::Tensor& q, const at
     // tokens, window 1024: 69 against 85; a mixed step of 308 blocks 77 against 90).
     const int ng = grid.x <= (window > 0 ? 256 : 512) ? 2 : 1;
     const bool more = x.ksum != nullptr || x.dist_bias != nullptr;
-    const size_t msmem = (size_t)2 * ng * MFMA_TILES_PER_STEP *
-                         (((ds + 1) / 2 + vt) * 2048 + (x.key_fac != nullptr ? 32 * sizeof(float) : 0));
+    // a sink, a cap that needs no running maximum and whose powers are ordinary numbers
+    const double near = std::abs(scale) / softcap;
+    const bool capped = sink && softcap > 0.0 && softcap * 1.4427 <= 96.0 && slp == nullptr && near > 1e-4 && near < 1e3;
+    const size_t msmem = (size_t)ng * MFMA_TILES_PER_STEP *
+                         (((ds + 1) / 2 + vt) * 4096 + (x.key_fac != nullptr ? 3 * 32 * sizeof(float) : 0));
 // The common form exists for the sizes that serving meets most, 64 and 128 channels, and for the others with all there is.
 #define MFMA_CASE(DS_, VT_)                                                                       \
   do {                                                                                            \
     constexpr bool ALWAYS = !((DS_ == 4 || DS_ == 8) && (VT_ == 2 || VT_ == 4));                  \
-    if (ng == 2 && (more || ALWAYS)) MFMA_NG(DS_, VT_, 2, true);                                  \
-    else if (ng == 2) MFMA_NG(DS_, VT_, 2, ALWAYS);                                               \
-    else if (more || ALWAYS) MFMA_NG(DS_, VT_, 1, true);                                          \
-    else MFMA_NG(DS_, VT_, 1, ALWAYS);                                                            \
+    if (ng == 2) MFMA_FORM(DS_, VT_, 2, ALWAYS);                                                  \
+    else MFMA_FORM(DS_, VT_, 1, ALWAYS);                                                          \
   } while (0)
-#define MFMA_NG(DS_, VT_, NG_, MORE_)                                                                                     \
+#define MFMA_FORM(DS_, VT_, NG_, ALWAYS_)                                                         \
+  do {                                                                                            \
+    if (more || ALWAYS_) MFMA_NG(DS_, VT_, NG_, 1);                                               \
+    else if (capped) MFMA_NG(DS_, VT_, NG_, ALWAYS_ ? 1 : 2);                                     \
+    else MFMA_NG(DS_, VT_, NG_, ALWAYS_ ? 1 : 0);                                                 \
+  } while (0)
+#define MFMA_NG(DS_, VT_, NG_, FORM_)                                                                                     \
   do {                                                                                                             \
-    auto kfn = paged_attention_mfma_kernel<DS_, VT_, NG_, MORE_>;                                                         \
+    auto kfn = paged_attention_mfma_kernel<DS_, VT_, NG_, FORM_>;                                                         \
     if (msmem > 65536) /* more dynamic LDS than a kernel gets without asking */                                    \
       (void)hipFuncSetAttribute((const void*)kfn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)msmem);         \
     hipLaunchKernelGGL(kfn, grid, dim3(64 * nw * NG_), msmem, stream(),                                            \
@@ -939,7 +1080,7 @@ static bool launch_mfma_attention(at::Tensor& out, const at::Tensor& q, const at
                        page_shift, (float)scale, (int)window, (int)keep_first, (float)softcap, sink ? 1 : 0,       \
                        tile_waves, x.sink_logits, x.dist_bias, x.dist_rows, (const bf16s*)x.ksum,                      \
                        (const bf16s*)x.vsum, x.sum_shift, x.sum_block, x.cross_out, x.chunk, x.key_fac, x.vrep,    \
-                       x.out32, tiles, fewest);                                                                         \
+                       x.out32, tiles, fewest, (int)cu.numel() - 1);                                                                         \
   } while (0)
 #define MFMA_ROW(DS_)                     \
   do {                                    \
@@ -955,6 +1096,7 @@ static bool launch_mfma_attention(at::Tensor& out, const at::Tensor& q, const at
     else MFMA_ROW(8);
 #undef MFMA_ROW
 #undef MFMA_CASE
+#undef MFMA_FORM
 #undef MFMA_NG
     HIP_CHECK_LAST();
     return true;

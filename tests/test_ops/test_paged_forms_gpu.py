@@ -469,3 +469,10 @@ def test_decode_parts_meet_whoever_ends_last(H, G, D, Dv, starts):
         graph.replay()
         assert torch.equal(first, want[i % 3]) and torch.equal(second, want[i % 3])
         assert torch.equal(call(q), want[i % 3])
+
+
+@pytest.mark.parametrize("seqs", [17, 64, 65, 130])
+def test_portions_of_many_sequences_find_theirs(seqs):
+    """A block looks for its sequence 64 at a time: decode tokens, short and longer portions on either side of that."""
+    counts = [1 if i % 5 else 33 + i % 40 for i in range(seqs)]
+    _check(counts, [(7 * i) % 90 for i in range(seqs)], 8, 2, 64, 64, 16, 0.1, window=64, keep_first=3)
