@@ -235,58 +235,52 @@ __global__ __launch_bounds__(NW * 64, 2) void fa_fwd_kernel(
   // tiles this wave computes: those above its diagonal produce nothing (barriers stay uniform)
   const int my_tiles = qw >= Seff ? 0 : (causal ? min(kv_tiles, (qw + QW - 1) / KVB + 1) : kv_tiles);
 
-  constexpr int KB = KVB / 32;
   const int q_abs = qw + ln;
   char* Kbuf = smem;                 // [2] key tiles, then [2] value tiles
   char* Vbuf = smem + 2 * KB_BYTES;
 
-  // interior tiles (every row/col in range, strictly below the causal diagonal) need no mask:
-  // at S=4096 that is ~94% of tiles, and the mask chain is ~4 VALU ops per score
-  auto masked = [&](int k0) { return !((k0 + KVB <= SeffK) && (qw + QW <= Seff) && (!causal || k0 + KVB - 1 <= qw)); };
-  const int last_key = q_abs >= Seff ? -1 : causal ? min(q_abs, SeffK - 1) : SeffK - 1;   // the last key this row sees
-  auto mask = [&](int k0, f32x16 (&s)[KB]) {
-    const int upto = last_key - k0 - 4 * half;
+  // The mask of 32 keys, of the few that need one: at the diagonal and at the end of the keys. Rows past the sequence's last one repeat it, or
+  // see what keys there are; what becomes of them is overwritten at the end.
+  const int last_key = causal ? min(q_abs, SeffK - 1) : SeffK - 1;   // the last key this row sees
+  auto mask = [&](int k0, f32x16& s) __attribute__((always_inline)) {
+    if (k0 + 32 > SeffK || (causal && k0 + 31 > qw)) {
+      const int upto = last_key - k0 - 4 * half;
 #pragma unroll
-    for (int kb = 0; kb < KB; ++kb)
-#pragma unroll
-      for (int j = 0; j < 16; ++j) s[kb][j] = kb * 32 + crow(j, 0) > upto ? -INFINITY : s[kb][j];
-  };
-  auto largest = [&](const f32x16 (&s)[KB]) {
-    float r = s[0][0];
-#pragma unroll
-    for (int kb = 0; kb < KB; ++kb)
-#pragma unroll
-      for (int j = 0; j < 16; ++j) r = fmaxf(r, s[kb][j]);
-    return r;
+      for (int j = 0; j < 16; ++j) s[j] = crow(j, 0) > upto ? -INFINITY : s[j];
+      asm volatile("" ::: "memory");   // a body of its own: merged into the common one, every tile would pay for it
+    }
   };
 
-  // ---- online softmax of a tile's 64 scores of q-row (qw+ln), in the base-2 domain (v_exp_f32 is exp2); the scale enters
+  // ---- online softmax of 32 scores of q-row (qw+ln), half of them in this lane, in the base-2 domain (v_exp_f32 is exp2); the scale enters
   // with the fma that subtracts the reference m_run. m_run is a maximum the row has had, not always its newest: the
-  // weights are taken against it as it stands, and only where their sum shows that some of them passed 2^12 (a row's first
-  // finite score gives inf; NaN counts too) is the maximum formed, m_run raised and the tile's weights taken
+  // weights are taken against it as it stands, and only where their sum shows that some of them passed 2^30 (a row's first
+  // finite score gives inf; NaN counts too) is the maximum formed, m_run raised and the weights taken
   // again. The sum is needed anyway, so most tiles need no maximum, no exchange between the half-waves and no
-  // rescaling; float32 and bfloat16 hold a weight of 2^12 as precisely as one of 1.
+  // rescaling; float32 and bfloat16 hold a weight of 2^30 as precisely as one of 1.
   // P in the order it was born in is the B operand of O^T += V^T · P^T: slot half*8+e of a 16-k step holds
   // key 8*(e>>2) + 4*half + (e&3) of it, and the V column fragments are read in the same key
   // order. P never passes through LDS.
-  bf16x8_t pb[KB][2];
-  auto weights = [&](const f32x16 (&s)[KB]) {
-    float rowsum = 0.0f;
-#pragma unroll
-    for (int kb = 0; kb < KB; ++kb)
-#pragma unroll
-      for (int j = 0; j < 16; ++j) {
-        const float pv = __builtin_amdgcn_exp2f(fmaf(s[kb][j], scale2, -mref));
-        rowsum += pv;
-        pb[kb][j >> 3][j & 7] = (__bf16)pv;
-      }
-    return rowsum;
+  struct Weights {
+    bf16x8_t p[2];
   };
-  auto softmax = [&](int k0, f32x16 (&s)[KB]) {
-    if (masked(k0)) mask(k0, s);
-    float rowsum = weights(s);
-    if (!__all(rowsum <= 4096.0f)) {
-      float rowmax = largest(s);
+  // Two weights in two stages: the exponentials, then their sum and rounding.
+  auto stage = [&](int k, const f32x16& s, int i, float (&w)[2], float& sum, Weights& p) __attribute__((always_inline)) {
+    if (k == 0) {
+#pragma unroll
+      for (int e = 0; e < 2; ++e) w[e] = __builtin_amdgcn_exp2f(fmaf(s[i + e], scale2, -mref));
+    } else {
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        sum += w[e];
+        p.p[i >> 3][(i & 7) + e] = (__bf16)w[e];
+      }
+    }
+  };
+  auto raise = [&](const f32x16& s, float rowsum, Weights& p) __attribute__((always_inline)) {
+    if (!__all(rowsum <= 0x1p30f)) {
+      float rowmax = s[0];
+#pragma unroll
+      for (int j = 1; j < 16; ++j) rowmax = fmaxf(rowmax, s[j]);
       rowmax = fmaxf(rowmax, __shfl_xor(rowmax, 32));
       rowmax = rowmax == -INFINITY ? -INFINITY : rowmax * scale2;  // no 0 * inf
       const float m_new = fmaxf(m_run, rowmax);
@@ -298,7 +292,13 @@ __global__ __launch_bounds__(NW * 64, 2) void fa_fwd_kernel(
       l_run *= corr;
       m_run = m_new;
       mref = m_run == -INFINITY ? -3.0e38f : m_run;
-      rowsum = weights(s);
+      rowsum = 0.0f;
+#pragma unroll
+      for (int i = 0; i < 16; i += 2) {
+        float w[2];
+        stage(0, s, i, w, rowsum, p);
+        stage(1, s, i, w, rowsum, p);
+      }
     }
     l_run += rowsum;  // this lane's half of the row's keys; the halves meet at the end
   };
@@ -306,74 +306,139 @@ __global__ __launch_bounds__(NW * 64, 2) void fa_fwd_kernel(
   const RowAt row_at(ln, half);
   const ColAt col_at(lane);
   const TileLoad<D, KVB, NW> kload(k_base, kts, SeffK), vload(v_base, kts, SeffK);
-  f32x16 sc[KB];
+  constexpr int PER = TileLoad<D, KVB, NW>::PER;
+
+  // The turn of 32 keys: the scores of the 32 after them into `sn` (keys from row kr of the tile at `K_`), their own weights from `s` into `p`, and what
+  // the 32 ahead of them add, weights `pp` times the values from row vr at `V_`; none of these waits for another, and a
+  // wave's instructions alternate between them. A product takes the matrix unit 32 cycles and the SIMD's issue 11; whatever else the SIMD's
+  // waves issue (4 to 5 cycles, an exponential 8) fits beside it only if it stands between the products.
+  constexpr int GROUPS = DSL > D / 16 ? DSL : D / 16, AHEAD = 2;
+  auto turn = [&](auto with_scores, auto with_weights, auto with_values, const char* __restrict__ K_, int kr, const char* __restrict__ V_, int vr,
+                  f32x16& sn, const f32x16& s, Weights& p, const Weights& pp, auto load) __attribute__((always_inline)) {
+    constexpr int NB = D / 32;
+    bf16x8_t kf[DSL], vf[2 * NB];
+    float w[8][2], sum = 0.0f;
+    auto read = [&](int i) __attribute__((always_inline)) {
+      if (with_scores && i < DSL) kf[i] = frag_row<KVB>(K_, row_at, kr, i);
+      if (with_values && i < 2 * NB) vf[i] = frag_born<KVB>(V_, col_at, vr + i / NB * 16, i % NB * 32);
+    };
+    constexpr int PRODUCTS = (decltype(with_scores)::value ? DSL : 0) + (decltype(with_values)::value ? 2 * NB : 0);
+    auto weigh = [&](int n) __attribute__((always_inline)) {
+      if (with_weights) {
+#pragma unroll
+        for (int k = n * 16 / PRODUCTS; k < (n + 1) * 16 / PRODUCTS; ++k) stage(k & 1, s, (k >> 1) * 2, w[k >> 1], sum, p);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    if (with_scores) {
+#pragma unroll
+      for (int j = 0; j < 16; ++j) sn[j] = 0.0f;
+    }
+#pragma unroll
+    for (int i = 0; i < AHEAD; ++i) read(i);
+    __builtin_amdgcn_sched_barrier(0);
+    int n = 0;
+#pragma unroll
+    for (int i = 0; i < GROUPS; ++i) {
+      read(i + AHEAD);
+      if (with_scores && i < DSL) {
+        sn = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[i], qf[i], sn, 0, 0, 0);
+        weigh(n++);
+      }
+      if (with_values && i < 2 * NB) {
+        oacc[i % NB] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[i], pp.p[i / NB], oacc[i % NB], 0, 0, 0);
+        weigh(n++);
+      }
+      load(i);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    if (with_weights) {
+      // formed here: the compiler moves them to where they are used, behind the products
+      asm volatile("" : "+v"(p.p[0]), "+v"(p.p[1]));
+      raise(s, sum, p);
+    }
+  };
+  constexpr std::true_type yes{};
+  constexpr std::false_type no{};
+
+  // Keys are a tile ahead of values: in step t a wave forms the scores of the tile's two halves, the weights of the half ahead of them and of the
+  // first one, and adds what the halves of the tile before are worth; the next keys and this tile's values are on their way, all
+  // issued in the first half of the step, so that they have arrived at its end (past the last key: zeros, without a read).
   if (kv_tiles > 0) {
     kload.all(0, Kbuf, w);
     vload.all(0, Vbuf, w);
   }
-  loads_done();
+  loads_left<PER>();
   __syncthreads();
-  // A tile, while the next one arrives in the other buffers (past the last key: zeros, without a read).
-  auto step = [&](int t, const char* __restrict__ K_, const char* __restrict__ V_, char* __restrict__ Kn, char* __restrict__ Vn) __attribute__((always_inline)) {
-    const auto kt = kload.tile((t + 1) * KVB), vt = vload.tile((t + 1) * KVB);
-    constexpr int PER = TileLoad<D, KVB, NW>::PER;
-    // ---- S^T = K · Q^T : KVB/32 32-k blocks. C: col = q (ln), row = k (crow).
-#pragma unroll
-    for (int kb = 0; kb < KB; ++kb)
-#pragma unroll
-      for (int j = 0; j < 16; ++j) sc[kb][j] = 0.0f;
-    __builtin_amdgcn_s_setprio(1);
-    // the key fragments are read AHEAD products ahead of their own
-    constexpr int AHEAD = 6;
-    bf16x8_t kf[DSL * KB];
-#pragma unroll
-    for (int i = 0; i < AHEAD; ++i) kf[i] = frag_row<KVB>(K_, row_at, i % KB * 32, i / KB);
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int i = 0; i < DSL * KB; ++i) {
-      if (i + AHEAD < DSL * KB) kf[i + AHEAD] = frag_row<KVB>(K_, row_at, (i + AHEAD) % KB * 32, (i + AHEAD) / KB);
-      sc[i % KB] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[i], qf[i / KB], sc[i % KB], 0, 0, 0);
-      if (i % KB == KB - 1) {
-        const int sl = i / KB;
-#pragma unroll
-        for (int n = sl * PER / DSL; n < (sl + 1) * PER / DSL; ++n) kload.piece(kt, Kn, w, n);
-      }
-      __builtin_amdgcn_sched_barrier(0);
-    }
-    __builtin_amdgcn_s_setprio(0);
-    softmax(t * KVB, sc);
-    __builtin_amdgcn_s_setprio(1);
-#pragma unroll
-    for (int g = 0; g < KB * 2; ++g) {
-#pragma unroll
-      for (int nb = 0; nb < D / 32; ++nb)
-        oacc[nb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(frag_born<KVB>(V_, col_at, g * 16, nb * 32), pb[g >> 1][g & 1], oacc[nb], 0, 0, 0);
-#pragma unroll
-      for (int i = g * PER / (2 * KB); i < (g + 1) * PER / (2 * KB); ++i) vload.piece(vt, Vn, w, i);
-    }
-    __builtin_amdgcn_s_setprio(0);
+  int t = 0;
+  __amdgpu_buffer_rsrc_t kt, vt;
+  auto begin = [&]() __attribute__((always_inline)) {
+    kt = kload.tile((t + 1) * KVB);
+    vt = vload.tile(t * KVB);
   };
-  for (int t = 0; t < kv_tiles; ++t) {
-    char* K_ = Kbuf + (t & 1) * KB_BYTES;
-    char* V_ = Vbuf + (t & 1) * KB_BYTES;
-    char* Kn = Kbuf + (~t & 1) * KB_BYTES;
-    char* Vn = Vbuf + (~t & 1) * KB_BYTES;
-    if (t < my_tiles) {
-      step(t, K_, V_, Kn, Vn);
-    } else {
-      kload.all((t + 1) * KVB, Kn, w);
-      vload.all((t + 1) * KVB, Vn, w);
-    }
+  auto end = [&]() __attribute__((always_inline)) {
     loads_done();
     __syncthreads();
+    ++t;
+  };
+  auto load_keys = [&](int i) __attribute__((always_inline)) {
+#pragma unroll
+    for (int n = i * PER / GROUPS; n < (i + 1) * PER / GROUPS; ++n) kload.piece(kt, Kbuf + (~t & 1) * KB_BYTES, w, n);
+  };
+  auto load = [&](int i) __attribute__((always_inline)) {
+    load_keys(i);
+#pragma unroll
+    for (int n = i * PER / GROUPS; n < (i + 1) * PER / GROUPS; ++n) vload.piece(vt, Vbuf + (t & 1) * KB_BYTES, w, n);
+  };
+  auto nothing = [](int) {};
+  if (my_tiles > 0) {
+    f32x16 se, so;            // scores of an even and an odd half
+    Weights pe, po;
+    {
+      begin();
+      turn(yes, no, no, Kbuf, 0, Kbuf, 0, se, so, po, pe, load_keys);   // the first values are on their way
+      mask(0, se);
+      turn(yes, yes, no, Kbuf, 32, Kbuf, 0, so, se, pe, po, nothing);
+      end();
+    }
+    while (t < my_tiles) {
+      begin();
+      const char* K_ = Kbuf + (t & 1) * KB_BYTES;
+      const char* V_ = Vbuf + (~t & 1) * KB_BYTES;
+      mask(t * KVB - 32, so);
+      turn(yes, yes, yes, K_, 0, V_, 0, se, so, po, pe, load);
+      mask(t * KVB, se);
+      turn(yes, yes, yes, K_, 32, V_, 32, so, se, pe, po, nothing);
+      end();
+    }
+    const char* V_ = Vbuf + (~t & 1) * KB_BYTES;
+    const int k0 = t * KVB - 32;
+    if (k0 < SeffK && !(causal && k0 > qw + QW - 1)) {   // the last half shows something to the wave
+      mask(k0, so);
+      turn(no, yes, yes, V_, 0, V_, 0, se, so, po, pe, nothing);
+      turn(no, no, yes, V_, 0, V_, 32, se, so, po, po, nothing);
+    } else {
+      turn(no, no, yes, V_, 0, V_, 0, se, so, po, pe, nothing);
+    }
+  }
+  while (t < kv_tiles) {
+    begin();
+#pragma unroll
+    for (int i = 0; i < GROUPS; ++i) {
+      if (t > 0) load(i);
+      else load_keys(i);
+    }
+    end();
   }
 
   // ---- epilogue: O /= l, store O and LSE. Rows beyond Seff (right-padded
-  // batches) have l_run == 0 -> O = 0, LSE = -inf, which the backward uses
+  // batches) become O = 0, LSE = -inf, which the backward uses
   // to mask them; the buffer extent S is still fully written.
   const int row_lim = VARLEN ? Seff : S;
   l_run += __shfl_xor(l_run, 32);
   if (q_abs >= row_lim) return;
+  const bool pad = q_abs >= Seff;
+  if (pad) l_run = 0.0f;
   unsigned short* o_base = VARLEN ? O + (seq0 * Hq + h) * D : O + ((long)b * S * Hq + h) * D;
   float* lse_base = VARLEN ? LSE + (long)h * S + seq0 : LSE + ((long)b * Hq + h) * S;
   const float inv_l = (l_run > 0.0f) ? 1.0f / l_run : 0.0f;
@@ -383,7 +448,7 @@ __global__ __launch_bounds__(NW * 64, 2) void fa_fwd_kernel(
     for (int jj = 0; jj < 4; ++jj) {
       short4v pk;
 #pragma unroll
-      for (int e = 0; e < 4; ++e) pk[e] = (short)f2bf(oacc[nb][jj * 4 + e] * inv_l);
+      for (int e = 0; e < 4; ++e) pk[e] = pad ? 0 : (short)f2bf(oacc[nb][jj * 4 + e] * inv_l);
       *reinterpret_cast<short4v*>(o_base + (long)q_abs * o_stride + nb * 32 + 8 * jj + 4 * half) = pk;
     }
   if (half == 0) {
