@@ -64,7 +64,7 @@ __global__ __launch_bounds__(64 * GROUP_WAVES, 2) void group_attention_kernel(
     const int* __restrict__ positions, const float* __restrict__ slopes, const bf16s* __restrict__ gate, long gate_stride,
     const float* __restrict__ sink_logits, int H, int G, int page_shift, float scale, int window, int keep_first, int chunk,
     float softcap, int sink, int vrep, long vrow, long vhead, int splits, float* __restrict__ ws, const int* __restrict__ cu,
-    unsigned long long* __restrict__ marks, unsigned long long mark) {
+    unsigned long long* __restrict__ marks, unsigned long long mark, int seqs, int width) {
   constexpr int D = DS * 16, Dv = VT * 32, KQ = D / 32, KT = D * 64, VTT = Dv * 64;   // bytes of a tile's keys, values
   constexpr float LOG2E = 1.4426950408889634f;
   extern __shared__ __align__(16) char tiles[];   // [waves][KT + VTT], later the waves' states; then the pages
@@ -80,8 +80,11 @@ __global__ __launch_bounds__(64 * GROUP_WAVES, 2) void group_attention_kernel(
   }
   const int g = (int)(blockIdx.x / splits % G);
   const int R = H / G, h0 = g * R;
-  const int pos = positions[n];
-  const int* bt = block_tables + (long)tok_seq[n] * bt_stride;
+  // A page table of few pages (width > 0) is read whole, into registers, beside the token's position and sequence and not after them: on the guess that
+  // token n is of sequence n, as in a step of decode tokens alone it is.
+  const int guess = width > 0 ? block_tables[min(unit, seqs - 1L) * bt_stride + min((int)threadIdx.x, width - 1)] : 0;
+  const int pos = positions[n], seq = tok_seq[n];
+  const int* bt = block_tables + (long)seq * bt_stride;
   const int page_mask = (1 << page_shift) - 1;
   const int piece = COLS ? col / PIECE_HEADS : 0, hcol = col - piece * PIECE_HEADS;   // of the weights, head of the group
   const bool head = hcol < R;
@@ -104,8 +107,12 @@ __global__ __launch_bounds__(64 * GROUP_WAVES, 2) void group_attention_kernel(
   const int w0 = i0 < n_keep ? lo : lo + (i0 - n_keep);             // the first one beyond the kept ones
   const int keep_pages = i0 < n_keep ? (n_keep + page_mask) >> page_shift : 0;
   const int num_pages = i0 < i1 ? keep_pages + ((lo + (i1 - 1 - n_keep)) >> page_shift) - (w0 >> page_shift) + 1 : 0;
-  for (int i = threadIdx.x; i < num_pages; i += 64 * GROUP_WAVES)
-    pages[i] = bt[i < keep_pages ? i : (w0 >> page_shift) + i - keep_pages];
+  const int skip = width > 0 ? 0 : keep_pages - (w0 >> page_shift);   // from a page's number in the table to its place in LDS, beyond the kept ones
+  if (width > 0) {
+    if ((int)threadIdx.x < width) pages[threadIdx.x] = seq == unit ? guess : bt[threadIdx.x];
+  } else {
+    for (int i = threadIdx.x; i < num_pages; i += 64 * GROUP_WAVES) pages[i] = bt[i < keep_pages ? i : i - skip];
+  }
   __syncthreads();
   struct Rows {
     int at[2];
@@ -118,7 +125,7 @@ __global__ __launch_bounds__(64 * GROUP_WAVES, 2) void group_attention_kernel(
       const int key = t * 32 + i * 16 + lkey, idx = min(key, total - 1);   // past the end: the token's own row
       r.past[i] = key >= total;
       const int j = idx < n_keep ? idx : lo + (idx - n_keep);
-      const int p = idx < n_keep ? j >> page_shift : keep_pages + (j >> page_shift) - (w0 >> page_shift);
+      const int p = (j >> page_shift) + (idx < n_keep ? 0 : skip);
       r.at[i] = (pages[p] << page_shift) + (j & page_mask);
     }
     return r;
@@ -456,15 +463,18 @@ bool launch_group_attention(at::Tensor& out, const at::Tensor& q, const at::Tens
     if (slopes != nullptr && blocks <= 64 && keys <= 512) return false;
   }
   // Parts of the keys while there are fewer blocks than CUs. A tile of 32 keys takes a wave 1.75 us at 128 channels, of which eight run side by side;
-  // parts cost 2 to 2.5 us, a store and three round trips to memory, and 0.1 each for reading their states. Whole, and in parts: 16 x 1024 (16 heads on
+  // parts cost 2 us (2.5 over 500 keys that are in L2), a store and three round trips to memory, and 0.1 each for reading their states. Whole, and in parts: 16 x 1024 (16 heads on
   // 4 of 128) 22.8 us, 2: 19.0, 4: 16.0, 8 (512 blocks): 22.8; 4 x 16384 277, 8: 48.4, 16: 36.6, 32: 41.4; 1 x 8192 66, 8: 17.4, 16: 14.4, 24:
   // 13.4, 64: 16.1; 1 x 2048 20.8, 4: 12.9, 12: 11.3, 16: 10.8; 16 x 300 (8 on 4) 9.3, 2: 10.6, 4: 9.9; 3 x 1500 (4 on 2 of 64) 12.3, 8: 8.2.
   const double whole = (double)((keys + 31) / 32) * 0.22 * (D + Dv) / 256;
   int splits = (int)std::max<long>(1, std::min<long>({256 / blocks, WAVE, std::lround(std::sqrt(whole * 10.0))}));
-  if (whole <= whole / splits + 2.5 + 0.1 * splits) splits = 1;
+  if (whole < 4.2 || whole <= whole / splits + 2.0 + 0.1 * splits) splits = 1;
   // page numbers of a part: of its keys, rounded up to whole tiles, of a page more for where they begin, and of the kept ones
   const long part_keys = ((keys + 31) / 32 + splits - 1) / splits * 32;
-  const size_t lds = (size_t)GROUP_WAVES * (D + Dv) * 64 + (size_t)((part_keys >> page_shift) + (keep_first >> page_shift) + 4) * sizeof(int);
+  const long table = block_tables.size(1);
+  const int width = table <= 64 * GROUP_WAVES ? (int)table : 0;   // a page a thread
+  const size_t lds = (size_t)GROUP_WAVES * (D + Dv) * 64 +
+                     (size_t)(width > 0 ? width : (part_keys >> page_shift) + (keep_first >> page_shift) + 4) * sizeof(int);
   if (lds > GROUP_LDS) return false;
   at::Tensor ws;
   unsigned long long* marks = nullptr;
@@ -482,7 +492,8 @@ bool launch_group_attention(at::Tensor& out, const at::Tensor& q, const at::Tens
                        (int)block_tables.stride(0), tok_seq.data_ptr<int>(), positions.data_ptr<int>(), slopes,    \
                        gate.has_value() ? ptr<bf16s>(*gate) : (const bf16s*)nullptr, gate_stride, x.sink_logits, H, G, page_shift, \
                        (float)scale, (int)window, (int)keep_first, x.chunk, (float)softcap, sink ? 1 : 0, x.vrep, vrow, vhead, \
-                       splits, splits > 1 ? ws.data_ptr<float>() : (float*)nullptr, only.cu, marks, splits > 1 ? new_mark() : 0ull);                            \
+                       splits, splits > 1 ? ws.data_ptr<float>() : (float*)nullptr, only.cu, marks, splits > 1 ? new_mark() : 0ull, \
+                       (int)block_tables.size(0), width);                            \
   } while (0)
   if (D == 128) { if (Dv == 128) GROUP_LAUNCH(8, 4); else GROUP_LAUNCH(8, 2); }
   else { if (Dv == 128) GROUP_LAUNCH(4, 4); else GROUP_LAUNCH(4, 2); }
