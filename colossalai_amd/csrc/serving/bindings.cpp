@@ -58,7 +58,12 @@ at::Tensor query_norm_key_write(at::Tensor q, at::Tensor k, at::Tensor weight, d
                                 at::Tensor positions, at::Tensor kpool, at::Tensor kfac, at::Tensor rows);
 at::Tensor difference_norm(at::Tensor o, int64_t kv_heads, double lam, double mult, double eps, at::ScalarType out_dtype);
 std::vector<at::Tensor> streams_start(at::Tensor table, at::Tensor tokens, int64_t streams, at::Tensor w_in,
-                                      at::Tensor weight, double eps, double scale);
+                                      at::Tensor weight, double eps, double scale, bool fill);
+bool streams_pairs(int64_t S, int64_t W);
+c10::optional<at::Tensor> streams_pass(c10::optional<at::Tensor> x, c10::optional<at::Tensor> table, c10::optional<at::Tensor> tokens,
+                                       c10::optional<at::Tensor> y1, c10::optional<at::Tensor> mix1, c10::optional<at::Tensor> out1, at::Tensor y,
+                                       at::Tensor mix, at::Tensor w_out, c10::optional<at::Tensor> w_in, at::Tensor weight, double eps,
+                                       at::ScalarType out_dtype);
 c10::optional<at::Tensor> streams_update(at::Tensor x, at::Tensor y, at::Tensor mix, at::Tensor w_out,
                                          c10::optional<at::Tensor> w_in, c10::optional<at::Tensor> weight, double eps,
                                          at::ScalarType out_dtype);
@@ -109,7 +114,11 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("query_norm_key_write", &s::query_norm_key_write,
         "RMS norm + position growth of queries; raw keys and their 1 / rms into the pool");
   m.def("difference_norm", &s::difference_norm, "unit RMS of the difference of two attention maps' outputs, scaled");
-  m.def("streams_start", &s::streams_start, "embedding rows as parallel residual streams, and the first sublayer's input");
+  m.def("streams_start", &s::streams_start, "embedding rows as parallel residual streams, and the first sublayer's input",
+        py::arg("table"), py::arg("tokens"), py::arg("streams"), py::arg("w_in"), py::arg("weight"), py::arg("eps"), py::arg("scale"),
+        py::arg("fill") = true);
+  m.def("streams_pairs", &s::streams_pairs, "whether streams_pass serves this many streams of this width");
+  m.def("streams_pass", &s::streams_pass, "the read and norm after a sublayer's write without it, or after two sublayers' writes");
   m.def("streams_update", &s::streams_update, "write a sublayer's output into the streams, read and norm the next input");
   m.def("gated_grouped_rms_norm", &s::gated_grouped_rms_norm, "x * silu(gate), then grouped RMS norm");
   m.def("add_layer_norm", &s::add_layer_norm,

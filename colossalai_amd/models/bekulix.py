@@ -40,7 +40,7 @@ from ..ops.latent_attention import latent_attention, latent_kv_write
 from ..ops.normed_keys import query_norm_key_write
 from ..ops.paged_attention import paged_attention, paged_kv_write
 from ..ops.ragged import RaggedBatch
-from ..ops.streams import streams_start, streams_update
+from ..ops.streams import Rows, streams_begin, streams_pairs, streams_read, streams_update, streams_update_two
 from .looped import layer_runs, parse_loop
 from .packed import PackedLinear
 from .registry import register_model
@@ -273,17 +273,26 @@ class BekulixForCausalLM(nn.Module):
         every layer run."""
         eps, act = self.config.norm_eps, self.act_dtype
         layers = [self.layers[i] for i in self.runs]
-        x, h = streams_start(self.embed.weight, tokens, self.config.streams, layers[0].hc1.read, layers[0].norm1, eps)
+        x, h = streams_begin(self.embed.weight, tokens, self.config.streams, layers[0].hc1.read, layers[0].norm1, eps)
         for r, layer in enumerate(layers):
             last = r + 1 == len(layers)
             after = (None, self.final_norm) if last else (layers[r + 1].hc1.read, layers[r + 1].norm1)
-            y, hc = layer.mix(h, batch, kv, r), layer.hc1
+            y, hc, first = layer.mix(h, batch, kv, r), layer.hc1, None
             if layer.mlp is not None:
-                h = streams_update(x, y, hc.mix, hc.write, layer.hc2.read, layer.norm2, eps, act)
+                if streams_pairs(y, self.config.streams):
+                    first = (y, hc.mix, hc.write)
+                    h = streams_read(x, *first, layer.hc2.read, layer.norm2, eps, act)
+                else:
+                    h = streams_update(x, y, hc.mix, hc.write, layer.hc2.read, layer.norm2, eps, act)
                 y, hc = layer.mlp(h), layer.hc2
-            if last and want is not None and residuals is None:  # the last write is per row: the wanted rows only
-                x, y = x.index_select(0, want), y.index_select(0, want)
-            h = streams_update(x, y, hc.mix, hc.write, *after, eps, act)
+            if last and want is not None and residuals is None:  # the last writes are per row: the wanted rows only
+                x, y = x.select(want) if isinstance(x, Rows) else x.index_select(0, want), y.index_select(0, want)
+                first = None if first is None else (first[0].index_select(0, want),) + first[1:]
+            if first is not None:
+                x, h = streams_update_two(x, first, y, hc.mix, hc.write, *after, eps, act)
+            else:
+                x = x.filled() if isinstance(x, Rows) else x
+                h = streams_update(x, y, hc.mix, hc.write, *after, eps, act)
             if residuals is not None:
                 residuals.append(x.sum(1))
         if want is not None and residuals is not None:

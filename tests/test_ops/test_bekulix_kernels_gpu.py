@@ -165,3 +165,28 @@ def test_shapes_the_kernels_do_not_take_are_refused():
         paged_attention(q, kp, kp, bg, 1.0, key_factors=torch.zeros(pages + 1, 16, 2, device="cuda"))
     with pytest.raises(AssertionError):
         paged_attention(q, kp, kp, bg, 1.0, window=3, chunk=4)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("S,W", [(1, 4), (2, 260), (3, 1024), (4, 1028), (4, 2048), (4, 4096), (5, 64), (4, 4100), (2, 6)])
+@pytest.mark.parametrize("N", [1, 37])
+def test_streams_written_once_a_layer(dtype, S, W, N):
+    """Two sublayers' writes at once, from streams and from the tokens' rows, have the bits of one update after the other, and what the second one
+    reads too; sizes without kernels for it go one by one."""
+    torch.manual_seed(S * W + N)
+    table = torch.randn(50, W).to(dtype).cuda()
+    toks = torch.randint(0, 50, (N,)).cuda()
+    y1, y2 = (torch.randn(N, W).to(dtype).cuda() for _ in range(2))
+    m1, m2 = (torch.randn(S, S).cuda() for _ in range(2))
+    o1, o2, r1, r2 = (torch.randn(S).cuda() for _ in range(4))
+    w = torch.rand(W).cuda() + 0.5
+    x, h0 = streams.streams_start(table, toks, S, r1, w, 1e-5)
+    rows, g0 = streams.streams_begin(table, toks, S, r1, w, 1e-5)
+    assert torch.equal(h0, g0) and isinstance(rows, streams.Rows) == streams.streams_pairs(table, S)
+    for base in (rows, x.clone()):
+        want = x.clone()
+        a = streams.streams_update(want, y1, m1, o1, r2, w, 1e-5, dtype)
+        assert torch.equal(streams.streams_read(base, y1, m1, o1, r2, w, 1e-5, dtype), a)
+        b = streams.streams_update(want, y2, m2, o2, None, w, 1e-5, dtype)
+        got, h = streams.streams_update_two(base, (y1, m1, o1), y2, m2, o2, None, w, 1e-5, dtype)
+        assert torch.equal(h, b) and torch.equal(got, want)
