@@ -328,7 +328,7 @@ __global__ __launch_bounds__(256 * NG, 2) void paged_attention_mfma_kernel(
     int tile_waves, const float* __restrict__ sink2, const float* __restrict__ dist2, int dist_rows,
     const bf16s* __restrict__ ksum, const bf16s* __restrict__ vsum, int sum_shift, int sum_block,
     float* __restrict__ cross_out, int chunk, const float* __restrict__ key_fac, int vrep, float* __restrict__ out32,
-    int num_tiles, int fewest, int seqs) {
+    int num_tiles, int fewest, int seqs, int sorted) {
   // The optional extras of the split-key kernel, in the base-2 domain: sink2 [H] = learned sink scores * log2e;
   // dist2 [H, dist_rows] = the per-distance bias * log2e, one row per head; ksum / vsum = block summaries, staged as
   // the first tiles of a block (summary idx of a sequence is seen by a token at pos when idx < (pos - window + 1) /
@@ -389,13 +389,45 @@ __global__ __launch_bounds__(256 * NG, 2) void paged_attention_mfma_kernel(
   for (int b0 = 0;; b0 += 64) {
     const int at = min(b0 + lane, seqs - 1), from = cu[at], count = cu[at + 1] - from, held = start[at];
     const int own = b0 + lane >= seqs || count < fewest ? 0 : (count + (1 << bshift) - 1) >> bshift;
-    int upto = own;   // summed over the lanes up to this one: inside rows of 16, then over the rows
-    upto += __builtin_amdgcn_update_dpp(0, upto, 0x111, 0xf, 0xf, false);
-    upto += __builtin_amdgcn_update_dpp(0, upto, 0x112, 0xf, 0xf, false);
-    upto += __builtin_amdgcn_update_dpp(0, upto, 0x114, 0xf, 0xf, false);
-    upto += __builtin_amdgcn_update_dpp(0, upto, 0x118, 0xf, 0xf, false);
-    upto += __builtin_amdgcn_update_dpp(0, upto, 0x142, 0xa, 0xf, false);
-    upto += __builtin_amdgcn_update_dpp(0, upto, 0x143, 0xc, 0xf, false);
+    // over the lanes up to this one: inside rows of 16, then over the rows
+    auto summed = [](int v) {
+      v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);
+      v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);
+      v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);
+      v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);
+      v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);
+      v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);
+      return v;
+    };
+    if (sorted) {
+      // The tiles of up to 64 sequences by the position they end at (in tiles): those that end after `past`, found by halving, go ahead of this
+      // one. In the sequences' order the long tiles of the last one would start when half of the time is over (4 x 1000 tokens, two groups of waves: 53 us).
+      const int before = held >> bshift, rank = num_tiles - 1 - tile;
+      auto ending = [&](int end) {   // tiles that end there or later
+        return __builtin_amdgcn_readlane(summed(max(0, min(before + own - end + 1, own))), 63); };
+      int lo = 1, hi = (int)wave_reduce_max((float)(before + own)) + 1, ahead = 0;
+      lo = __builtin_amdgcn_readfirstlane(lo);
+      hi = __builtin_amdgcn_readfirstlane(hi);
+      while (hi - lo > 1) {   // ending(lo) > rank >= ending(hi) = ahead
+        const int mid = (lo + hi) >> 1, n = ending(mid);
+        if (n > rank) {
+          lo = mid;
+        } else {
+          hi = mid;
+          ahead = n;
+        }
+      }
+      unsigned long long same = __ballot(lo > before && lo <= before + own);
+      for (int skip = rank - ahead; skip > 0; --skip) same &= same - 1;
+      const int at_lane = same != 0 ? __builtin_ctzll(same) : 0;
+      b = at_lane;
+      first = __builtin_amdgcn_readlane(from, at_lane);
+      cnt = __builtin_amdgcn_readlane(count, at_lane);
+      s0 = __builtin_amdgcn_readlane(held, at_lane);
+      tile = lo - 1 - __builtin_amdgcn_readlane(before, at_lane);
+      break;
+    }
+    const int upto = summed(own);
     const unsigned long long past = __ballot(tile < upto);
     if (past != 0 || b0 + 64 >= seqs) {
       const int at_lane = past != 0 ? __builtin_ctzll(past) : 63;
@@ -1009,7 +1041,7 @@ static bool launch_mfma_attention(at::Tensor& out, const at::Tensor& q, const at
                                   const at::Tensor& block_tables, const at::Tensor& cu, const at::Tensor& start,
                                   const float* slp, const c10::optional<at::Tensor>& gate, long gstride, double scale,
                                   int64_t window, int64_t keep_first, double softcap, bool sink, int page_shift,
-                                  int64_t num_tiles, int64_t num_tiles128, int64_t num_tiles64, const ScalarExtras& x, int fewest = 1) {
+                                  int64_t num_tiles, int64_t num_tiles128, int64_t num_tiles64, const ScalarExtras& x, double even, int64_t longest, int fewest = 1) {
   const int H = (int)q.size(1), D = (int)q.size(2);
   const int G = (int)kpool.size(2), Dv = (int)vpool.size(3);
   // prompt portions in bfloat16 go to the matrix cores when the head sizes fit a tiling;
@@ -1028,7 +1060,7 @@ static bool launch_mfma_attention(at::Tensor& out, const at::Tensor& q, const at
     const at::Tensor ids = block_tables.reshape({-1}).clamp(0, kpool.size(0) - 1);   // places past a sequence's end hold anything
     return launch_mfma_attention(out, q, kpool.index_select(0, ids), vpool.index_select(0, ids),
                                  at::arange(pages, block_tables.options()).view(block_tables.sizes()), cu, start, slp, gate, gstride, scale,
-                                 window, keep_first, softcap, sink, page_shift, num_tiles, num_tiles128, num_tiles64, x, fewest);
+                                 window, keep_first, softcap, sink, page_shift, num_tiles, num_tiles128, num_tiles64, x, even, longest, fewest);
   }
   {
     const int rep = H / G, nw = 4;
@@ -1041,12 +1073,16 @@ static bool launch_mfma_attention(at::Tensor& out, const at::Tensor& q, const at
     const dim3 grid((unsigned)((tiles + sub - 1) / sub * sub * rows));
     const int ds = D <= 32 ? 2 : D <= 48 ? 3 : D <= 64 ? 4 : D <= 96 ? 6 : 8, vt = (Dv + 31) / 32;
     // Two groups of waves take alternate key tiles where one block a CU is all there is: a second group then fills the
-    // idle half of the CU, and a lone block's chain of tiles is half as long (2 x 256 tokens 31 -> 23 us, 64 blocks; 3 x 200 after
-    // 1500 207 -> 130; 100 alone 18 -> 15). Up to 512 blocks of a causal prompt too: their lengths differ, a CU takes a long one and then
-    // a short one instead of both at once, of which the long one's last steps run alone (4096 tokens 138 -> 115 us, a cap and a sink
-    // 172 -> 136; 2000 of 64 channels 85 -> 59). A window makes them equally long, and two blocks at once are better (4096
-    // tokens, window 1024: 69 against 85; a mixed step of 308 blocks 77 against 90).
-    const int ng = grid.x <= (window > 0 ? 256 : 512) ? 2 : 1;
+    // idle half of the CU, and a lone block's chain of tiles is half as long (2000 tokens, 16 heads on 4 of 128: 55 us with one group, 46 with two). Up to
+    // 512 blocks it is a question of how even they are: a CU takes two after the other, and where long and short ones alternate, as in one long
+    // prompt, that is better than both at once, of which the long one's last steps run alone; blocks of about one length, by a window or
+    // many cached tokens, hide each other's waits when they run together. `even` is their mean length over the longest; one group and two: 4096 tokens 129,
+    // 114 (0.5), with a window of 1024 63, 71 (0.9); 3000 with the window (376 blocks, 0.84) 53, 64; 2200 with it (276, 0.8) 41, 35; 8 x 512
+    // after 1000 73, 82 (0.83); 16 x 200 after 1500 (448, 0.95) 82, 92; 2 x 1200 with the window (304) 43, 36. Short blocks wait for their
+    // first loads a good part of their time, and sooner run together: 4 x 1000 (512, 0.5) 39, 44, 3 x 1000 (384) 37, 38.
+    const int ng = grid.x <= 256 || (grid.x <= 512 && even * grid.x <= (longest < 1536 ? 230 : 300)) ? 2 : 1;
+    // the order of tiles matters where some wait for others, or share a CU with them
+    const int sorted = cu.numel() > 2 && cu.numel() <= 65 && grid.x > 256;
     const bool more = x.ksum != nullptr || x.dist_bias != nullptr;
     // a sink, a cap that needs no running maximum and whose powers are ordinary numbers
     const double near = std::abs(scale) / softcap;
@@ -1080,7 +1116,7 @@ static bool launch_mfma_attention(at::Tensor& out, const at::Tensor& q, const at
                        page_shift, (float)scale, (int)window, (int)keep_first, (float)softcap, sink ? 1 : 0,       \
                        tile_waves, x.sink_logits, x.dist_bias, x.dist_rows, (const bf16s*)x.ksum,                      \
                        (const bf16s*)x.vsum, x.sum_shift, x.sum_block, x.cross_out, x.chunk, x.key_fac, x.vrep,    \
-                       x.out32, tiles, fewest, (int)cu.numel() - 1);                                                                         \
+                       x.out32, tiles, fewest, (int)cu.numel() - 1, sorted);                                                                         \
   } while (0)
 #define MFMA_ROW(DS_)                     \
   do {                                    \
@@ -1107,7 +1143,7 @@ at::Tensor paged_attention(at::Tensor q, at::Tensor kpool, at::Tensor vpool, at:
                            at::Tensor start, at::Tensor tok_seq, at::Tensor positions, double scale, int64_t window,
                            int64_t keep_first, c10::optional<at::Tensor> slopes, c10::optional<at::Tensor> gate,
                            int64_t num_tiles, double softcap, bool sink, int64_t num_tiles128, int64_t num_tiles64, int64_t singles,
-                           bool singles_see_half) {
+                           bool singles_see_half, double even, int64_t longest) {
   check_act(q, "q");
   TORCH_CHECK(softcap >= 0.0, "softcap must not be negative (0 = none)");
   TORCH_CHECK(q.dim() == 3 && q.stride(2) == 1 && q.stride(1) == q.size(2), "q must be [N, H, D] with dense rows");
@@ -1164,7 +1200,7 @@ at::Tensor paged_attention(at::Tensor q, at::Tensor kpool, at::Tensor vpool, at:
     }
   }
   if (launch_mfma_attention(out, q, kpool, vpool, block_tables, cu, start, slp, gate, gstride, scale, window, keep_first,
-                            softcap, sink, page_shift, num_tiles, num_tiles128, num_tiles64, ScalarExtras(), fewest))
+                            softcap, sink, page_shift, num_tiles, num_tiles128, num_tiles64, ScalarExtras(), even, longest, fewest))
     return out;
   launch_scalar_attention(out, q, kpool, vpool, block_tables, tok_seq, positions, slp, gate, gstride, scale, window,
                           keep_first, softcap, sink, page_shift, vrow, vhead, ScalarExtras());
@@ -1182,7 +1218,7 @@ at::Tensor paged_attention_ext(at::Tensor q, at::Tensor kpool, at::Tensor vpool,
                                c10::optional<at::Tensor> dist_bias, c10::optional<at::Tensor> ksum,
                                c10::optional<at::Tensor> vsum, int64_t sum_block, bool cross, int64_t num_tiles,
                                int64_t num_tiles128, int64_t num_tiles64, int64_t chunk,
-                               c10::optional<at::Tensor> key_fac, bool out_f32) {
+                               c10::optional<at::Tensor> key_fac, bool out_f32, double even, int64_t longest) {
   check_act(q, "q");
   TORCH_CHECK(softcap >= 0.0, "softcap must not be negative (0 = none)");
   TORCH_CHECK(q.dim() == 3 && q.stride(2) == 1 && q.stride(1) == q.size(2), "q must be [N, H, D] with dense rows");
@@ -1273,7 +1309,7 @@ at::Tensor paged_attention_ext(at::Tensor q, at::Tensor kpool, at::Tensor vpool,
       x2.dist_bias = db2.data_ptr<float>();
     }
     if (launch_mfma_attention(out, q, kpool, vpool, block_tables, cu, start, slp, gate, gstride, scale, window,
-                              keep_first, softcap, sink, page_shift, num_tiles, num_tiles128, num_tiles64, x2))
+                              keep_first, softcap, sink, page_shift, num_tiles, num_tiles128, num_tiles64, x2, even, longest))
       return out;
   }
   launch_scalar_attention(out, q, kpool, vpool, block_tables, tok_seq, positions, slp, gate, gstride, scale, window,

@@ -48,6 +48,7 @@ class RaggedBatch:
     _chunk_tables: Optional[dict] = None  # memo of chunk_tables(), by chunk size
     _tiles: Optional[tuple] = None  # memo of tile_counts()
     _singles: Optional[tuple] = None  # memo of single_tokens()
+    _even: Optional[dict] = None  # memo of key_lengths(), by window
 
     @property
     def num_seqs(self) -> int:
@@ -82,6 +83,26 @@ class RaggedBatch:
         if window > 0:
             short, long = min(short, window), min(long, window)
         return count, 2 * short >= long
+
+    def key_lengths(self, window: int = 0):
+        """How many keys the tiles of 32 new tokens see on average, over the most that one sees; and these."""
+        if self._even is None:
+            self._even = {}
+        if window not in self._even:
+            total = most = tiles = 0.0
+            for a, b, s in zip(self.cu_host, self.cu_host[1:], self.start_host):
+                lo, hi, n = s + min(32, b - a), s + b - a, (b - a + 31) // 32
+                if window <= 0 or hi <= window:
+                    mean = (lo + hi) / 2
+                elif lo >= window:
+                    mean = window
+                else:   # grows up to the window, then stays
+                    mean = ((lo + window) / 2 * (window - lo) + window * (hi - window)) / (hi - lo)
+                total += mean * n
+                tiles += n
+                most = max(most, min(hi, window) if window > 0 else hi)
+            self._even[window] = total / (tiles * most), int(most)
+        return self._even[window]
 
     @property
     def num_tiles32(self) -> int:

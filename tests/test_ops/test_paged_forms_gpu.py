@@ -476,3 +476,11 @@ def test_portions_of_many_sequences_find_theirs(seqs):
     """A block looks for its sequence 64 at a time: decode tokens, short and longer portions on either side of that."""
     counts = [1 if i % 5 else 33 + i % 40 for i in range(seqs)]
     _check(counts, [(7 * i) % 90 for i in range(seqs)], 8, 2, 64, 64, 16, 0.1, window=64, keep_first=3)
+
+
+@pytest.mark.parametrize("counts,starts", [([1000] * 4, [0] * 4), ([700, 33, 1, 1100, 150, 1], [0, 900, 700, 100, 1500, 0]), ([300] * 9, list(range(0, 1800, 200))),
+                                           ([65] * 40, [31 * i for i in range(40)]), ([40] * 70, [0] * 70)])
+@pytest.mark.parametrize("H,G,kw", [(16, 4, {}), (8, 8, dict(window=300, keep_first=5)), (16, 8, dict(softcap=5.0, sink=True))])
+def test_tiles_by_length_are_all_taken(counts, starts, H, G, kw):
+    """More blocks than CUs: the longest tiles of all sequences start first, of up to 64 sequences."""
+    _check(counts, starts, H, G, 64, 64, 16, 0.1, **dict(kw))
