@@ -22,17 +22,23 @@
 //
 // What bounds it (B1 S8192 H32/8 D128 causal): with loads through registers and a maximum per tile, a tile took a wave 4034
 // cycles, of which 557 went into issuing the loads, 638 into storing them, 150 into the barrier; the products and the
-// softmax, 890 cycles each, overlap little between the two waves of a SIMD. The matrix unit is now busy half of the time, at
-// the 1.9 GHz that the card keeps under this load. Fragments read further ahead for P · V, other wave
-// priorities (a fixed order of a SIMD's two waves), and exponentials placed between the products changed nothing.
+// softmax, 890 cycles each, overlapped little between the two waves of a SIMD, since it issues one instruction of all its waves
+// at a time: 11 cycles for a product, 4 to 5 for a vector instruction, 8 for an exponential. The forward therefore places
+// a half tile's exponentials between the products of its neighbours. A full chip is held by power then (1.9 GHz under this load);
+// the backward has no registers for the same. Fragments read further ahead for P · V and other wave
+// priorities (a fixed order of a SIMD's two waves) changed nothing.
 //
-// TFLOP/s, forward 2 products / backward 5 products of the visible pairs, with loads through registers -> now:
+// TFLOP/s, forward 2 products / backward 5 products of the visible pairs, loads through registers -> into LDS directly:
 //   B4 S4096 H32 D128 causal          forward 768 -> 930, backward 599 -> 693
 //   B1 S8192 H32/8 D128 causal        forward 888 -> 1040, backward 659 -> 761
 //   B2 S4096 H16/8 D128               forward 928 -> 1072, backward 699 -> 807
 //   B8 S1024 H12 D64 causal           forward 348 -> 424, backward 328 -> 395
 //   B16 S512 H12 D64                  forward 524 -> 582, backward 430 -> 501
 //   packed, 14 sequences of 256..4096, 32/8 heads   forward 608 -> 810, backward 535 -> 632
+// and the forward with products and weights in turns, us (another card):
+//   B4 S4096 H32/8 D128 causal 570 -> 550, B1 S8192 H32/8 514 -> 500, H4 159 -> 128 (half the chip); B8 S1024 H12 D64 32.0 -> 31.2,
+//   packed, 16384 tokens of up to 4096, 32/8 of 128 384 -> 367, 12 of 64 102 -> 95, 8192 of up to 2048, 32/8 113 -> 103;
+//   B1 S4096 H8/2 D64 unmasked 56.9 -> 53.3, but B1 S8192 H12 D64 causal 168 -> 171
 //
 // Shapes: q [B,S,Hq,D], k/v [B,S,Hkv,D] ("bshd" — no transposes in the
 // model), D in {64,128}. lse/delta are [B,Hq,S] fp32.
