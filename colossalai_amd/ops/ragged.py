@@ -23,7 +23,8 @@ LISTED_TOKENS = 32  # up to here a step's per-token vectors are made on the host
 
 def to_device(values: Sequence, dtype, device) -> torch.Tensor:
     """A tensor of host numbers on `device`. To a GPU it goes from pinned memory and the host does not wait: a copy from pageable
-    memory waits for all the work ahead of it, so that the GPU then waits for what the host does next."""
+    memory waits for all the work ahead of it, so that the GPU then waits for what the host does next. As with any work of the device, the result
+    is for the current stream; another one has to wait for it."""
     if torch.device(device).type != "cuda":
         return torch.tensor(values, dtype=dtype).to(device)
     return torch.tensor(values, dtype=dtype, pin_memory=True).to(device, non_blocking=True)
