@@ -582,11 +582,12 @@ __global__ __launch_bounds__(256 * NG, 2) void paged_attention_mfma_kernel(
   const bool capped = CAPPED || softcap > 0.0f;
   const float inv_cap = capped ? scale / softcap : 0.0f;
   const float cap2 = softcap * LOG2E, t2 = capped ? 2.0f * LOG2E * scale / softcap : 0.0f;
-  // of the polynomial in x^2
+  // of the polynomial of tanh(y) / y in y^2; with CAPPED in the raw product's square, for which the host bounds the ratio of scale and cap, whose
+  // eighth power is one of its factors
   struct Poly {
     float c0, c1, c2, c3, c4;
   };
-  const float ic2 = inv_cap * inv_cap, ic4 = ic2 * ic2, cx = cap2 * inv_cap;
+  const float ic = CAPPED ? inv_cap : 1.0f, ic2 = ic * ic, ic4 = ic2 * ic2, cx = cap2 * ic;
   const Poly cap_poly{cx, cx * ic2 * -0.33333069f, cx * ic4 * 0.13324751f, cx * ic4 * ic2 * -0.052984238f, cx * ic4 * ic4 * 0.017131345f};
   auto cap_base2 = [&](float dot) {
     const float e = __builtin_amdgcn_exp2f(dot * t2);  // +inf: the quotient is 0; a NaN stays one
@@ -662,8 +663,8 @@ __global__ __launch_bounds__(256 * NG, 2) void paged_attention_mfma_kernel(
   auto near_cap = [&](f32x16& x) __attribute__((always_inline)) {
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
-      const float z = x[i] * x[i];
-      x[i] *= fmaf(z, fmaf(z, fmaf(z, fmaf(z, cap_poly.c4, cap_poly.c3), cap_poly.c2), cap_poly.c1), cap_poly.c0);
+      const float y = CAPPED ? x[i] : x[i] * inv_cap, z = y * y;
+      x[i] = y * fmaf(z, fmaf(z, fmaf(z, fmaf(z, cap_poly.c4, cap_poly.c3), cap_poly.c2), cap_poly.c1), cap_poly.c0);
     }
   };
   auto prepare = [&](const Tile& t, f32x16& x) __attribute__((always_inline)) {

@@ -4,6 +4,8 @@ ones, scales of either sign and zero, with and without the parts that put scores
 The bound: float32 scores and weights; the output is rounded to bfloat16 once (at most 2^-8 of a value) and a score
 error of a few float32 roundings of the largest score moves a weight by less than that."""
 
+import math
+
 import pytest
 import torch
 
@@ -182,6 +184,37 @@ def test_every_tile_is_taken_once(H, G, counts, starts, page, D, Dv, kw):
 def test_soft_caps_near_and_far(softcap, scale):
     """Scores far below the cap, about it and far above it: the two forms of tanh."""
     _check([64, 700], [10, 0], 16, 4, 64, 64, 16, scale, softcap=softcap, sink=True)
+
+
+@pytest.mark.parametrize("ratio", [1e-9, 1e-6, 1e-5, 0.9e-4, 1.1e-4, 3e-3, 0.9e3, 1.1e3, 1e5, 1e6])
+@pytest.mark.parametrize("D", [64, 128, 72])
+@pytest.mark.parametrize("kw", [dict(sink=True), {}, dict(sink=True, slopes=True)])
+def test_soft_caps_of_any_ratio(ratio, D, kw):
+    """Scores up to half the cap, whatever product of a scale and of queries they come from; queries of 0 are among them."""
+    from colossalai_amd.ops.paged_attention import distance_slopes, paged_attention
+
+    torch.manual_seed(12)
+    n, start, H, G, cap = 70, 40, 8, 2, 30.0
+    batch, pages = _batch([n], [start], 16)
+    k, v = (torch.randn(pages, 16, G, D, device="cuda").bfloat16() for _ in range(2))
+    q = torch.randn(n, H, D, device="cuda").bfloat16()
+    q[5] = 0.0
+    kk, vv = (t[batch.block_tables[0].long()].flatten(0, 1)[: n + start].double().repeat_interleave(H // G, 1) for t in (k, v))
+    most = torch.einsum("nhd,mhd->hnm", q.double(), kk).abs().max().item()
+    q *= 2.0 ** math.floor(math.log2(0.5 / ratio / most))    # exact
+    slopes = distance_slopes(H, "cuda") if kw.get("slopes") else None
+    got = paged_attention(q, k, v, batch, ratio * cap, softcap=cap, sink=kw.get("sink", False), slopes=slopes, out_dtype=torch.float32)
+    s = cap * torch.tanh(torch.einsum("nhd,mhd->hnm", q.double(), kk) * ratio)
+    far = torch.arange(start, start + n, device="cuda")[:, None] - torch.arange(start + n, device="cuda")
+    if slopes is not None:
+        s -= slopes.double()[:, None, None] * far
+    s = s.masked_fill(far < 0, float("-inf"))
+    if kw.get("sink"):
+        s = torch.cat([s, torch.zeros_like(s[..., :1])], -1)
+    want = torch.einsum("hnm,mhd->nhd", torch.softmax(s, -1)[..., : n + start], vv)
+    # weights have 16 bits or more (two bfloat16 halves), and a score of up to 15 nats some ten roundings of 2^-24
+    err = (got - want).norm() / want.norm()
+    assert err < 2.0 ** -16 + 15 * 10 * 2.0 ** -24, f"{err:.2e}"
 
 
 # One, two, three and four or more query heads a key head: blocks of 128, 64 and 32 tokens. Head sizes that fill the pieces of 32 channels that
