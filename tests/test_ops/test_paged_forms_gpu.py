@@ -190,7 +190,7 @@ def test_soft_caps_near_and_far(softcap, scale):
 @pytest.mark.parametrize("D", [64, 128, 72])
 @pytest.mark.parametrize("kw", [dict(sink=True), {}, dict(sink=True, slopes=True)])
 def test_soft_caps_of_any_ratio(ratio, D, kw):
-    """Scores up to half the cap, whatever product of a scale and of queries they come from; queries of 0 are among them."""
+    """Scores about half the cap, whatever product of a scale and of queries they come from; queries of 0 are among them."""
     from colossalai_amd.ops.paged_attention import distance_slopes, paged_attention
 
     torch.manual_seed(12)
@@ -198,10 +198,12 @@ def test_soft_caps_of_any_ratio(ratio, D, kw):
     batch, pages = _batch([n], [start], 16)
     k, v = (torch.randn(pages, 16, G, D, device="cuda").bfloat16() for _ in range(2))
     q = torch.randn(n, H, D, device="cuda").bfloat16()
-    q[5] = 0.0
+    q[..., 0], q[5] = 64.0, 0.0
+    k[..., 0] = (2.0 + 2.0 * torch.rand(pages, 16, G, device="cuda")) * (-1.0 if kw else 1.0)   # a sink shows scores far below it
     kk, vv = (t[batch.block_tables[0].long()].flatten(0, 1)[: n + start].double().repeat_interleave(H // G, 1) for t in (k, v))
     most = torch.einsum("nhd,mhd->hnm", q.double(), kk).abs().max().item()
-    q *= 2.0 ** math.floor(math.log2(0.5 / ratio / most))    # exact
+    up = 2.0 ** math.floor(math.log2(0.5 / ratio / most))    # exact
+    q, ratio = q * up, 0.499 / (most * up)
     slopes = distance_slopes(H, "cuda") if kw.get("slopes") else None
     got = paged_attention(q, k, v, batch, ratio * cap, softcap=cap, sink=kw.get("sink", False), slopes=slopes, out_dtype=torch.float32)
     s = cap * torch.tanh(torch.einsum("nhd,mhd->hnm", q.double(), kk) * ratio)
