@@ -655,9 +655,11 @@ __global__ __launch_bounds__(256 * NG, 2) void paged_attention_mfma_kernel(
   // tanh(y) = y P(y^2) for |y| <= 1/2, P a polynomial through the Chebyshev nodes (1.3e-8 off): fused
   // multiplications where the general form takes an exponential and a reciprocal
   auto near = [&](const f32x16& x) __attribute__((always_inline)) {
+    // A NaN is the largest, and takes the general form. One instruction for two scores, which the compiler knows to read a product's result: as
+    // inline assembly it could stand behind the product without the wait that this takes.
     float far = 0.0f;
 #pragma unroll
-    for (int i = 0; i < 16; i += 2) asm("v_max3_f32 %0, %0, |%1|, |%2|" : "+v"(far) : "v"(x[i]), "v"(x[i + 1]));   // fmaxf makes two and a half of it
+    for (int i = 0; i < 16; i += 2) far = __builtin_elementwise_maximum(__builtin_elementwise_maximum(far, fabsf(x[i])), fabsf(x[i + 1]));
     return __all(far * fabsf(inv_cap) <= 0.5f);
   };
   auto near_cap = [&](f32x16& x) __attribute__((always_inline)) {
