@@ -259,10 +259,10 @@ __global__ __launch_bounds__(NW * 64, 2) void fa_fwd_kernel(
 
   // ---- online softmax of 32 scores of q-row (qw+ln), half of them in this lane, in the base-2 domain (v_exp_f32 is exp2); the scale enters
   // with the fma that subtracts the reference m_run. m_run is a maximum the row has had, not always its newest: the
-  // weights are taken against it as it stands, and only where their sum shows that some of them passed 2^30 (a row's first
+  // weights are taken against it as it stands, and only where their sum shows that some of them passed 2^12 (a row's first
   // finite score gives inf; NaN counts too) is the maximum formed, m_run raised and the weights taken
   // again. The sum is needed anyway, so most tiles need no maximum, no exchange between the half-waves and no
-  // rescaling; float32 and bfloat16 hold a weight of 2^30 as precisely as one of 1.
+  // rescaling; float32 and bfloat16 hold a weight of 2^12 as precisely as one of 1, and its products with values of up to 2^100 are finite in any number.
   // P in the order it was born in is the B operand of O^T += V^T · P^T: slot half*8+e of a 16-k step holds
   // key 8*(e>>2) + 4*half + (e&3) of it, and the V column fragments are read in the same key
   // order. P never passes through LDS.
@@ -283,7 +283,7 @@ __global__ __launch_bounds__(NW * 64, 2) void fa_fwd_kernel(
     }
   };
   auto raise = [&](const f32x16& s, float rowsum, Weights& p) __attribute__((always_inline)) {
-    if (!__all(rowsum <= 0x1p30f)) {
+    if (!__all(rowsum <= 4096.0f)) {
       float rowmax = s[0];
 #pragma unroll
       for (int j = 1; j < 16; ++j) rowmax = fmaxf(rowmax, s[j]);

@@ -230,6 +230,26 @@ def test_scores_that_rise_and_fall(levels, D, causal):
         _near(a, b, name)
 
 
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("packed", [False, True])
+def test_large_values_of_rising_scores(D, packed):
+    """Values of about 2^104: a weight is taken again before it passes 2^12, so that its product stays below 2^128."""
+    from colossalai_amd.ops import flash_attention, flash_attention_varlen
+
+    S = 192
+    q, k, v, dout = _inputs(1, S, 4, 2, D)
+    q[..., 0] = 8.0
+    k[:, :, :, 0] = torch.where(torch.arange(S, device="cuda") < 64, 0.0, 16.0)[None, :, None] / (8.0 * D ** -0.5)
+    v = v * 2.0 ** 104
+    want = _reference(q, k, v, dout, packed, D ** -0.5)[0]
+    if packed:
+        cu = torch.tensor([0, S], dtype=torch.int32, device="cuda")
+        got = flash_attention_varlen(q[0], k[0], v[0], cu, S, causal=True)[None]
+    else:
+        got = flash_attention(q, k, v, causal=False)
+    _near(got, want, "out")
+
+
 @pytest.mark.parametrize("place", ["odd address", "odd rows", "far rows", "one row for all"])
 @pytest.mark.parametrize("packed", [False, True])
 def test_inputs_that_tiles_cannot_be_loaded_from_as_they_lie(place, packed):
