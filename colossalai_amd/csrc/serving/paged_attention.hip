@@ -566,8 +566,9 @@ __global__ __launch_bounds__(256 * NG, 2) void paged_attention_mfma_kernel(
   // sink's 1. No maximum to track, no accumulator to rescale.
   const bool fixed_ref = CAPPED || (sink != 0 && softcap > 0.0f && softcap * 1.4426950408889634f <= 96.0f);
   // Without one, m is a maximum the token has had, not always its newest: weights are taken against it as it stands, and
-  // only where the sum of a tile's weights shows that some passed 2^30 (a token's first visible score gives inf; NaN counts
-  // too) is the maximum formed, m raised and the weights taken again. A weight of 2^30 has the mantissa of one of 1.
+  // only where the sum of a tile's weights shows that some passed 2^12 (a token's first visible score gives inf; NaN counts
+  // too) is the maximum formed, m raised and the weights taken again. A weight of 2^12 has the mantissa of one of 1, and its
+  // products with values of up to 2^100 are finite in any number.
   float m = fixed_ref ? 0.0f : -INFINITY, l = 0.0f;  // m in the base-2 domain
   float m_ref = fixed_ref ? 0.0f : -3.0e38f;         // m, and below every finite score until there is one
   f32x16 oacc[VT];
@@ -751,9 +752,9 @@ __global__ __launch_bounds__(256 * NG, 2) void paged_attention_mfma_kernel(
       p.lo[i >> 3][(i & 7) + 1] = lo[1];
     }
   };
-  // where the sum of a tile's weights shows that some passed 2^30: the maximum, and the weights again
+  // where the sum of a tile's weights shows that some passed 2^12: the maximum, and the weights again
   auto raise = [&](const f32x16& x, float off, float psum, Weights& p) __attribute__((always_inline)) {
-    if (!fixed_ref && !__all(psum <= 0x1p30f)) {
+    if (!fixed_ref && !__all(psum <= 4096.0f)) {
       Pair again;
       float top = x[0];
 #pragma unroll

@@ -258,6 +258,26 @@ def test_scores_that_rise_and_fall(levels, kw, rows):
     assert (got.double() - want.double()).norm() / want.double().norm() < BOUND
 
 
+@pytest.mark.parametrize("D", [64, 128, 72])
+@pytest.mark.parametrize("rows", [1, 40])
+def test_large_values_of_rising_scores(D, rows):
+    """Values of about 2^104: a weight is taken again before it passes 2^12, so that its product stays below 2^128."""
+    from colossalai_amd.ops.paged_attention import paged_attention, paged_attention_ref
+
+    torch.manual_seed(14)
+    n, scale = 256, D ** -0.5
+    batch, pages = _batch([n] * rows, [0] * rows, 64)
+    k, v = (torch.randn(pages, 64, 4, D, device="cuda").bfloat16() for _ in range(2))
+    q = torch.randn(rows * n, 16, D, device="cuda").bfloat16()
+    q[..., 0] = 8.0
+    for i, level in enumerate((16, 16, 16, 0)):   # the nearest keys are taken first
+        k[batch.block_tables[:, i].long(), :, :, 0] = level / (8.0 * scale)
+    v = v * 2.0 ** 104
+    got = paged_attention(q, k, v, batch, scale)
+    want = paged_attention_ref(q.float(), k.float(), v.float(), batch, scale)
+    assert (got.double() - want.double()).norm() / want.double().norm() < BOUND
+
+
 @pytest.mark.parametrize("which", ["keys", "values"])
 def test_pools_at_an_odd_address(which):
     from colossalai_amd.ops.paged_attention import paged_attention
