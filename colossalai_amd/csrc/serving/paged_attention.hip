@@ -622,6 +622,18 @@ __global__ __launch_bounds__(256 * NG, 2) void paged_attention_mfma_kernel(
   // the first step's values behind its keys: they are not waited for yet
 #pragma unroll
   for (int n = 0; n < TP * VR; ++n) value_piece(vrow, values, n);
+  // The steps in which the wave sees something: from `from` up to `stop` in its window, then, where the kept first keys or summaries lie apart, from
+  // `again` on. Numbers, and not a look at each step's tiles, which as a condition of the loop cost up to 470 spilled registers.
+  const int mine0 = first_tile + grp * TP;      // the group's first tile of step 0
+  const int w_lo = keep_first > wstart ? sink_tiles : sink_tiles + (max(0, lo_p0 - wstart) >> 5);   // lowest and highest tile of the wave's window
+  const int w_hi = min(tiles_n - 1, sink_tiles + ((p1 - wstart) >> 5));
+  const int again = head_ok ? (max(0, mine0 - sink_tiles + 1) + TS - 1) / TS : steps_n;
+  int from = head_ok ? (max(0, mine0 - w_hi) + TS - 1) / TS : steps_n, stop = (mine0 + 1 - w_lo + TS) / TS;
+  if (again <= stop) stop = steps_n;
+  if (from >= stop) {   // the group's tiles lie beside a short window
+    from = again;
+    stop = steps_n;
+  }
   if (quad0 == 0) loads_left<TP * VR>();
   else loads_left<TP * (VQ / 2)>();
   __syncthreads();
@@ -851,7 +863,8 @@ __global__ __launch_bounds__(256 * NG, 2) void paged_attention_mfma_kernel(
   };
   // Keys are a step ahead of values. In step s a wave forms the scores of the step's two tiles, the weights of the tile before them and
   // of the first one, and adds what the two tiles of the step before are worth; the next step's keys and this step's values are on their way.
-  // Steps in which a wave has nothing to do yet (several token tiles) only load; one without tokens or a head does no other.
+  // Steps in which a wave sees nothing (several token tiles) only load, and nothing they hold meets a weight of 0; a wave without tokens or a head
+  // does no other.
   int tile0 = first_tile, step = 0, third = 0;   // third: the step's place among three
   auto begin = [&]() __attribute__((always_inline)) {   // the next step's keys and this step's values; past the last step the loads repeat rows
     const Rows now = next;
@@ -897,8 +910,9 @@ __global__ __launch_bounds__(256 * NG, 2) void paged_attention_mfma_kernel(
     end();
   };
   auto mine_of = [&](int u) { return tile_of(tile0 + grp * TP + u); };
-  while (step < steps_n && !mine_of(0).live && !mine_of(1).live) idle();
-  if (step < steps_n) {
+  do {
+    while (step < from) idle();
+    if (step >= steps_n) break;
     f32x16 xe, xo;            // scores of an even and an odd tile of the wave's
     Weights pe, po;
     {
@@ -908,7 +922,7 @@ __global__ __launch_bounds__(256 * NG, 2) void paged_attention_mfma_kernel(
       weights_turn(yes, no, mine_of(0), third * TS + grp * TP, K_ + KT, K_, xo, xe, pe, po, nothing);
       end();
     }
-    while (step < steps_n) {
+    while (step < stop) {
       const Tile odd = tile_of(tile0 - way + grp * TP + 1), even = mine_of(0);
       begin();
       const char* K_ = keys + (step & 1) * KS;
@@ -917,11 +931,14 @@ __global__ __launch_bounds__(256 * NG, 2) void paged_attention_mfma_kernel(
       weights_turn(yes, yes, even, third * TS + grp * TP, K_ + KT, V_ + VTT, xo, xe, pe, po, nothing);
       end();
     }
+    // the tiles that are left, while other waves' loads go to the other places
     const Tile odd = tile_of(tile0 - way + grp * TP + 1);
     const char* V_ = values + (~step & 1) * VS;
     weights_turn(no, yes, odd, (third == 0 ? 2 : third - 1) * TS + grp * TP + 1, V_, V_, xe, xo, po, pe, nothing);
     turn(no, no, yes, cap_poly, V_, V_ + VTT, xo, xe, 0.0f, pe, po, nothing);
-  }
+    from = max(step, again);
+    stop = steps_n;
+  } while (step < steps_n);
   if constexpr (NG > 1) {  // the second group's states, wave by wave, through the tiles' place
     __syncthreads();         // all waves are past their last tile
     float4v* sums = reinterpret_cast<float4v*>(tiles) + wid * (VT * 4 * 64 + 32) + lane;   // 16 bytes an access

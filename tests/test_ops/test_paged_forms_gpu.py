@@ -278,6 +278,26 @@ def test_large_values_of_rising_scores(D, rows):
     assert (got.double() - want.double()).norm() / want.double().norm() < BOUND
 
 
+@pytest.mark.parametrize("bad", [float("inf"), float("nan")])
+@pytest.mark.parametrize("rows,H", [(1, 2), (40, 16)])
+@pytest.mark.parametrize("keep_first,key,clean", [(0, 270, 364), (4, 290, 396)])
+def test_values_outside_a_window_of_several_token_tiles(bad, rows, H, keep_first, key, clean):
+    """Blocks of 128 tokens: a step whose keys all lie before a wave's window adds nothing to it, whatever they hold, and the kept first keys
+    behind it are seen again. One and two groups of waves."""
+    from colossalai_amd.ops.paged_attention import paged_attention
+
+    torch.manual_seed(15)
+    batch, pages = _batch([128] * rows, [300] * rows, 16)
+    k, v = (torch.randn(pages, 16, H, 64, device="cuda").bfloat16() for _ in range(2))
+    q = torch.randn(128 * rows, H, 64, device="cuda").bfloat16()
+    want = paged_attention(q, k, v, batch, 0.1, 40, keep_first)
+    v[batch.block_tables[:, key // 16].long(), key % 16] = bad
+    got = paged_attention(q, k, v, batch, 0.1, 40, keep_first)
+    sees = (batch.positions >= key) & (batch.positions < key + 40)
+    assert not torch.isfinite(got[sees].float()).any()
+    assert torch.equal(got[batch.positions >= clean], want[batch.positions >= clean])
+
+
 @pytest.mark.parametrize("which", ["keys", "values"])
 def test_pools_at_an_odd_address(which):
     from colossalai_amd.ops.paged_attention import paged_attention
