@@ -101,7 +101,7 @@ class ContinuousBatchEngine:
         the next tokens of open sequences (a prompt portion or one decode
         token each) and the places among them whose logits are wanted. Returns
         float32 logits ``[sum(len(want)), vocab]`` in item order; the caches
-        then hold the new tokens."""
+        then hold the new tokens. What the model is given is ready on the current stream, like what the step before left there."""
         counts, starts, slots, tables, flat, want = [], [], [], [], [], []
         at = 0
         for seq_id, toks, w in items:
@@ -120,8 +120,8 @@ class ContinuousBatchEngine:
         vocab = getattr(self.model.config, "vocab", None)
         if vocab is not None and flat and not 0 <= min(flat) <= max(flat) < vocab:
             raise ValueError(f"token ids must lie in 0 .. {vocab - 1}")
-        batch = RaggedBatch.build(counts, starts, slots, self.device, tables, self.kv.block_size)
-        tokens, widx = to_device(flat + want, torch.long, self.device).split([len(flat), len(want)])
+        batch = RaggedBatch.build(counts, starts, slots, self.device, tables, self.kv.block_size, ordered=True)
+        tokens, widx = to_device(flat + want, torch.long, self.device, ordered=True).split([len(flat), len(want)])
         logits = self.model.forward_ragged(tokens, batch, self.kv, self.state, widx)
         for (seq_id, toks, _), s0 in zip(items, starts):
             self._cached[seq_id] = s0 + len(toks)

@@ -241,7 +241,7 @@ class MubutarForCausalLM(nn.Module):
                             dtype=self.act_dtype, layer_shapes=self.kv_layer_shapes(),
                             layer_sources=self.kv_layer_sources())
         tables = [list(range(b * pages, (b + 1) * pages)) for b in range(B)]
-        batch = RaggedBatch.build([S] * B, [0] * B, list(range(B)), dev, tables, page)
+        batch = RaggedBatch.build([S] * B, [0] * B, list(range(B)), dev, tables, page, ordered=True)
         with torch.no_grad():
             return self.forward_ragged(input_ids.reshape(-1), batch, kv).view(B, S, -1)
 

@@ -312,7 +312,7 @@ class VitinexForCausalLM(nn.Module):
                             dtype=self.act_dtype, layer_shapes=self.kv_layer_shapes())
         state = StateCacheManager(self.state_layer_buffers(), B, device=dev)
         tables = [list(range(b * pages, (b + 1) * pages)) for b in range(B)]
-        batch = RaggedBatch.build([S] * B, [0] * B, list(range(B)), dev, tables, page)
+        batch = RaggedBatch.build([S] * B, [0] * B, list(range(B)), dev, tables, page, ordered=True)
         with torch.no_grad():
             return self.forward_ragged(input_ids.reshape(-1), batch, kv, state).view(B, S, -1)
 

@@ -21,13 +21,35 @@ __all__ = ["RaggedBatch", "to_device"]
 LISTED_TOKENS = 32  # up to here a step's per-token vectors are made on the host: a launch takes as long
 
 
-def to_device(values: Sequence, dtype, device) -> torch.Tensor:
-    """A tensor of host numbers on `device`. To a GPU it goes from pinned memory and the host does not wait: a copy from pageable
-    memory waits for all the work ahead of it, so that the GPU then waits for what the host does next. As with any work of the device, the result
-    is for the current stream; another one has to wait for it."""
+_COPIES = {}  # device index -> the stream of complete()
+
+
+def complete(make, device) -> torch.Tensor:
+    """The tensor that ``make()`` fills on a GPU from host numbers, complete for every stream when this returns, as one copied from pageable
+    memory is. Such a copy waits for all the work ahead of it, so that the GPU then waits for what the host does next; this one has a
+    stream of its own, and the host waits for nothing else."""
+    index = torch.device(device).index
+    index = torch.cuda.current_device() if index is None else index
+    if index not in _COPIES:
+        _COPIES[index] = torch.cuda.Stream(index)
+    current, copies = torch.cuda.current_stream(index), _COPIES[index]
+    with torch.cuda.stream(copies):
+        made = make()
+    made.record_stream(current)  # the memory is of the other stream's: not to be used again before this one's work is done
+    copies.synchronize()
+    return made
+
+
+def to_device(values: Sequence, dtype, device, ordered: bool = False) -> torch.Tensor:
+    """A tensor of host numbers on `device`, complete for every stream; `ordered`: for the current one, as any work of the device, with nothing
+    that the host waits for (15 to 20 us)."""
     if torch.device(device).type != "cuda":
         return torch.tensor(values, dtype=dtype).to(device)
-    return torch.tensor(values, dtype=dtype, pin_memory=True).to(device, non_blocking=True)
+
+    def copy():
+        return torch.tensor(values, dtype=dtype, pin_memory=True).to(device, non_blocking=True)
+
+    return copy() if ordered else complete(copy, device)
 
 
 @dataclass
@@ -45,6 +67,7 @@ class RaggedBatch:
     start_host: List[int]
     slots_host: List[int]
     page_size: int = 0
+    ordered: bool = False  # vectors are for the stream they were made on
     _dense: Optional[dict] = None  # memo of dense_context(), by window
     _chunk_tables: Optional[dict] = None  # memo of chunk_tables(), by chunk size
     _tiles: Optional[tuple] = None  # memo of tile_counts()
@@ -123,7 +146,7 @@ class RaggedBatch:
         table of the dense layout itself (consecutive pages, sequence after sequence). With a sliding ``window`` the
         layout of a sequence starts with the page (and 32-key tile) of the first key that its first new token still
         sees; table entries ahead of it are not meant to be read. Built on the device from the step's own index
-        vectors, once per step and window."""
+        vectors, once per step and window, on the stream that is the current one then."""
         if self._dense is None:
             self._dense = {}
         if window not in self._dense:
@@ -138,7 +161,7 @@ class RaggedBatch:
                 first.append(total_pages)
                 total_pages += n
             width = max(n + k for n, k in zip(pages, skip))
-            host = to_device([first, pages, lens, skip], torch.int32, dev)   # one copy
+            host = to_device([first, pages, lens, skip], torch.int32, dev, self.ordered)   # one copy
             total = total_pages * ps
             if self.block_tables.is_cuda:
                 rows = torch.empty(total, dtype=torch.long, device=dev)
@@ -169,7 +192,7 @@ class RaggedBatch:
                 for t in range(lo, hi, size):
                     rows += [b, t, min(t + size, hi), 0]
                 ranges.append(len(rows) // 4)
-            buf = to_device(rows + ranges, torch.int32, self.cu.device)
+            buf = to_device(rows + ranges, torch.int32, self.cu.device, self.ordered)
             self._chunk_tables[size] = (buf[: len(rows)].view(-1, 4), buf[len(rows):])
         return self._chunk_tables[size]
 
@@ -182,7 +205,9 @@ class RaggedBatch:
 
     @classmethod
     def build(cls, new_counts: Sequence[int], starts: Sequence[int], slots: Sequence[int], device,
-              tables: Optional[Sequence[Sequence[int]]] = None, page_size: int = 0) -> "RaggedBatch":
+              tables: Optional[Sequence[Sequence[int]]] = None, page_size: int = 0, *, ordered: bool = False) -> "RaggedBatch":
+        """The vectors are complete for every stream when this returns; with `ordered` for the current one, and so are those made later
+        from host numbers: for a step that is used there and nowhere else."""
         cu = [0]
         for n in new_counts:
             assert n > 0, "a sequence in a step brings at least one token"
@@ -196,11 +221,14 @@ class RaggedBatch:
         parts = [cu, list(starts), list(slots), [p for t in tables or () for p in list(t) + [0] * (width - len(t))]]
         sizes = [B + 1, B, B, B * width, N, N, N if tables is not None else 0]
         if torch.device(device).type == "cuda" and N > LISTED_TOKENS and cls._fit_int32(starts, new_counts, parts[3], page_size):
-            # a token's own entries are filled in on the device
-            buf = torch.empty(sum(sizes), dtype=torch.int32, device=device)
-            head = torch.tensor([v for part in parts for v in part], dtype=torch.int32, pin_memory=True)
-            buf[: head.numel()].copy_(head, non_blocking=True)
-            serving_kernels().ragged_index(buf, B, N, width, page_size)
+            def fill():   # a token's own entries on the device
+                buf = torch.empty(sum(sizes), dtype=torch.int32, device=device)
+                head = torch.tensor([v for part in parts for v in part], dtype=torch.int32, pin_memory=True)
+                buf[: head.numel()].copy_(head, non_blocking=True)
+                serving_kernels().ragged_index(buf, B, N, width, page_size)
+                return buf
+
+            buf = fill() if ordered else complete(fill, device)
         else:
             tok_seq, pos, rows = [], [], []
             for i, n in enumerate(new_counts):
@@ -209,11 +237,11 @@ class RaggedBatch:
                 if tables is not None:
                     t = tables[i]
                     rows += [t[p // page_size] * page_size + p % page_size for p in range(starts[i], starts[i] + n)]
-            buf = to_device([v for part in parts + [tok_seq, pos, rows] for v in part], torch.int32, device)
+            buf = to_device([v for part in parts + [tok_seq, pos, rows] for v in part], torch.int32, device, ordered)
         cu_d, start_d, slots_d, tables_d, tok_seq_d, pos_d, rows_d = buf.split(sizes)
         return cls(
             cu=cu_d, start=start_d, slots=slots_d, tok_seq=tok_seq_d, positions=pos_d,
             block_tables=tables_d.view(B, width) if tables is not None else None,
             kv_rows=rows_d if tables is not None else None,
-            cu_host=cu, start_host=list(starts), slots_host=list(slots), page_size=page_size,
+            cu_host=cu, start_host=list(starts), slots_host=list(slots), page_size=page_size, ordered=ordered,
         )

@@ -409,3 +409,53 @@ def test_index_vectors_of_a_step(counts, starts, page):
         for window in (0, 50, 5000) if paged else ():
             for a, b in zip(gpu.dense_context(window), cpu.dense_context(window)):
                 assert a == b if isinstance(a, int) else a.dtype == b.dtype and torch.equal(a.cpu(), b)
+
+
+def _busy(stream):
+    x = torch.randn(8192, 8192, device="cuda").bfloat16()
+    stream.wait_stream(torch.cuda.default_stream())
+    with torch.cuda.stream(stream):
+        for _ in range(20):
+            x = (x @ x).clamp_(-1, 1)
+
+
+def _step(count, device):
+    tables = [list(range(40, 10, -1)), list(range(50, 80))]
+    return RaggedBatch.build([count, 3], [5, 40], [1, 0], device, tables, 16)
+
+
+VECTORS = ("cu", "start", "slots", "tok_seq", "positions", "block_tables", "kv_rows")
+
+
+@pytest.mark.parametrize("count", [4, 300])
+def test_a_steps_vectors_are_complete_for_every_stream(count):
+    """Made behind work of one stream, read by another that waits for nothing: listed on the host, filled in on the device."""
+    one, other = torch.cuda.Stream(), torch.cuda.Stream()
+    want = _step(count, "cpu")
+    _step(count, "cuda")
+    _busy(one)
+    with torch.cuda.stream(one):
+        batch = _step(count, "cuda")
+        rows, ranges = batch.chunk_tables(64)
+    with torch.cuda.stream(other):
+        got = [getattr(batch, name).cpu() for name in VECTORS] + [rows.cpu(), ranges.cpu()]
+    torch.cuda.synchronize()
+    for a, b in zip(got, [getattr(want, name) for name in VECTORS] + list(want.chunk_tables(64))):
+        assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("count", [4, 300])
+def test_a_steps_vectors_last_as_long_as_work_that_reads_them(count):
+    """The next step's are made while a stream is still busy ahead of reading the last one's, which nothing holds any more."""
+    one = torch.cuda.Stream()
+    want = _step(count, "cpu")
+    _busy(one)
+    with torch.cuda.stream(one):
+        batch = _step(count, "cuda")
+        got = [getattr(batch, name).clone() for name in VECTORS]
+        del batch
+        for shift in range(1, 9):
+            RaggedBatch.build([count, 3], [5 + shift, 40 - shift], [0, 1], "cuda", [list(range(80, 110)), list(range(110, 140))], 16)
+    torch.cuda.synchronize()
+    for a, name in zip(got, VECTORS):
+        assert torch.equal(a.cpu(), getattr(want, name)), name
