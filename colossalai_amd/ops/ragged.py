@@ -40,11 +40,18 @@ def complete(make, device) -> torch.Tensor:
     return made
 
 
+def refuse_capture() -> None:
+    """A captured copy from pinned memory would be repeated by every replay, from memory that holds something else by then."""
+    if torch.cuda.is_current_stream_capturing():
+        raise RuntimeError("tensors of host numbers cannot be made while a graph is captured")
+
+
 def to_device(values: Sequence, dtype, device, ordered: bool = False) -> torch.Tensor:
     """A tensor of host numbers on `device`, complete for every stream; `ordered`: for the current one, as any work of the device, with nothing
-    that the host waits for (15 to 20 us)."""
+    that the host waits for (15 to 20 us). Not while a graph is captured."""
     if torch.device(device).type != "cuda":
         return torch.tensor(values, dtype=dtype).to(device)
+    refuse_capture()
 
     def copy():
         return torch.tensor(values, dtype=dtype, pin_memory=True).to(device, non_blocking=True)
@@ -221,6 +228,8 @@ class RaggedBatch:
         parts = [cu, list(starts), list(slots), [p for t in tables or () for p in list(t) + [0] * (width - len(t))]]
         sizes = [B + 1, B, B, B * width, N, N, N if tables is not None else 0]
         if torch.device(device).type == "cuda" and N > LISTED_TOKENS and cls._fit_int32(starts, new_counts, parts[3], page_size):
+            refuse_capture()
+
             def fill():   # a token's own entries on the device
                 buf = torch.empty(sum(sizes), dtype=torch.int32, device=device)
                 head = torch.tensor([v for part in parts for v in part], dtype=torch.int32, pin_memory=True)

@@ -459,3 +459,15 @@ def test_a_steps_vectors_last_as_long_as_work_that_reads_them(count):
     torch.cuda.synchronize()
     for a, name in zip(got, VECTORS):
         assert torch.equal(a.cpu(), getattr(want, name)), name
+
+
+@pytest.mark.parametrize("count", [4, 300])
+def test_no_vectors_from_host_numbers_in_a_graph(count):
+    """A replay would read what the host has long used for something else."""
+    _step(count, "cuda")
+    graph = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph):
+        with pytest.raises(RuntimeError, match="captured"):
+            _step(count, "cuda")
+    assert torch.equal(_step(count, "cuda").positions.cpu(), _step(count, "cpu").positions)
