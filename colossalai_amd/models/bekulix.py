@@ -40,12 +40,17 @@ from ..ops.latent_attention import latent_attention, latent_kv_write
 from ..ops.normed_keys import query_norm_key_write
 from ..ops.paged_attention import paged_attention, paged_kv_write
 from ..ops.ragged import RaggedBatch
-from ..ops.streams import Rows, streams_begin, streams_pairs, streams_read, streams_update, streams_update_two
+from ..ops.streams import Rows, streams_begin, streams_pairs, streams_read, streams_start, streams_update, streams_update_two
 from .looped import layer_runs, parse_loop
 from .packed import PackedLinear
 from .registry import register_model
 
 __all__ = ["BekulixConfig", "BekulixForCausalLM"]
+
+# From here on (tokens x width) the residual streams are written once a layer. Below, the host bounds a step, and one update after the other is less of its
+# work: a step of three layers, us, one after the other and once: one token 618 and 639, 1024 wide, 512 tokens 728, 751, 1536 768, 786, 2048 809, 810; 2048
+# wide, 768 tokens 766, 779, 1024 838, 820, 2048 1230, 1195.
+WRITE_ONCE_ELEMENTS = 1 << 21
 
 
 @dataclass
@@ -273,13 +278,15 @@ class BekulixForCausalLM(nn.Module):
         every layer run."""
         eps, act = self.config.norm_eps, self.act_dtype
         layers = [self.layers[i] for i in self.runs]
-        x, h = streams_begin(self.embed.weight, tokens, self.config.streams, layers[0].hc1.read, layers[0].norm1, eps)
+        once = tokens.numel() * self.config.width >= WRITE_ONCE_ELEMENTS and streams_pairs(self.embed.weight, self.config.streams)
+        begin = streams_begin if once else streams_start
+        x, h = begin(self.embed.weight, tokens, self.config.streams, layers[0].hc1.read, layers[0].norm1, eps)
         for r, layer in enumerate(layers):
             last = r + 1 == len(layers)
             after = (None, self.final_norm) if last else (layers[r + 1].hc1.read, layers[r + 1].norm1)
             y, hc, first = layer.mix(h, batch, kv, r), layer.hc1, None
             if layer.mlp is not None:
-                if streams_pairs(y, self.config.streams):
+                if once:
                     first = (y, hc.mix, hc.write)
                     h = streams_read(x, *first, layer.hc2.read, layer.norm2, eps, act)
                 else:

@@ -93,3 +93,22 @@ def test_random_configuration(seed):
                 assert err.max().item() < 3e-4, (cfg, err.max().item())
             else:
                 assert err.median().item() < 0.03 and (err > 0.1).float().mean().item() < 0.05, (cfg, err.median().item())
+
+
+@pytest.mark.parametrize("seed", range(6))
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_streams_written_once_a_layer_have_the_same_bits(seed, dtype, monkeypatch):
+    """Small steps write the streams after every sublayer, large ones once a layer: either way for every step."""
+    import colossalai_amd.models.bekulix as bekulix
+
+    rng = random.Random(seed)
+    cfg = random_config(rng)
+    cfg.update(streams=rng.choice([2, 4]), width=rng.choice([64, 160]))
+    P = {k: v.float() for k, v in O.random_checkpoint(cfg, seed).items()}
+    toks = {"a": [(7 * i) % cfg["vocab"] for i in range(90)], "b": [(5 * i) % cfg["vocab"] for i in range(33)]}
+    plan = [[("a", 60), ("b", 20)], [("a", 1), ("b", 10)], [("a", 10 ** 6), ("b", 1)], [("b", 10 ** 6)]]
+    got = []
+    for elements in (0, 1 << 40):
+        monkeypatch.setattr(bekulix, "WRITE_ONCE_ELEMENTS", elements)
+        got.append(run(cfg, P, toks, dtype, plan))
+    assert all(torch.equal(got[0][k], got[1][k]) for k in toks)
