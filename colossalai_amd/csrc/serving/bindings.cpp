@@ -23,7 +23,7 @@ at::Tensor paged_attention(at::Tensor q, at::Tensor kpool, at::Tensor vpool, at:
                            at::Tensor start, at::Tensor tok_seq, at::Tensor positions, double scale, int64_t window,
                            int64_t keep_first, c10::optional<at::Tensor> slopes, c10::optional<at::Tensor> gate,
                            int64_t num_tiles, double softcap, bool sink, int64_t num_tiles128, int64_t num_tiles64, int64_t singles,
-                           bool singles_see_half, double even, int64_t longest);
+                           bool singles_see_half, double even, int64_t longest, double even_apart, int64_t longest_apart);
 at::Tensor paged_attention_ext(at::Tensor q, at::Tensor kpool, at::Tensor vpool, at::Tensor block_tables, at::Tensor cu,
                                at::Tensor start, at::Tensor tok_seq, at::Tensor positions, double scale, int64_t window,
                                int64_t keep_first, c10::optional<at::Tensor> slopes, c10::optional<at::Tensor> gate,

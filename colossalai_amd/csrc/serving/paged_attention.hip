@@ -1097,7 +1097,8 @@ static bool launch_mfma_attention(at::Tensor& out, const at::Tensor& q, const at
     // idle half of the CU, and a lone block's chain of tiles is half as long (2000 tokens, 16 heads on 4 of 128: 55 us with one group, 46 with two). Up to
     // 512 blocks it is a question of how even they are: a CU takes two after the other, and where long and short ones alternate, as in one long
     // prompt, that is better than both at once, of which the long one's last steps run alone; blocks of about one length, by a window or
-    // many cached tokens, hide each other's waits when they run together. `even` is their mean length over the longest; one group and two: 4096 tokens 129,
+    // many cached tokens, hide each other's waits when they run together. `even` is the mean length of their sequences' tiles of 32 tokens over
+    // the longest; one group and two: 4096 tokens 129,
     // 114 (0.5), with a window of 1024 63, 71 (0.9); 3000 with the window (376 blocks, 0.84) 53, 64; 2200 with it (276, 0.8) 41, 35; 8 x 512
     // after 1000 73, 82 (0.83); 16 x 200 after 1500 (448, 0.95) 82, 92; 2 x 1200 with the window (304) 43, 36. Short blocks wait for their
     // first loads a good part of their time, and sooner run together: 4 x 1000 (512, 0.5) 39, 44, 3 x 1000 (384) 37, 38.
@@ -1164,7 +1165,7 @@ at::Tensor paged_attention(at::Tensor q, at::Tensor kpool, at::Tensor vpool, at:
                            at::Tensor start, at::Tensor tok_seq, at::Tensor positions, double scale, int64_t window,
                            int64_t keep_first, c10::optional<at::Tensor> slopes, c10::optional<at::Tensor> gate,
                            int64_t num_tiles, double softcap, bool sink, int64_t num_tiles128, int64_t num_tiles64, int64_t singles,
-                           bool singles_see_half, double even, int64_t longest) {
+                           bool singles_see_half, double even, int64_t longest, double even_apart, int64_t longest_apart) {
   check_act(q, "q");
   TORCH_CHECK(softcap >= 0.0, "softcap must not be negative (0 = none)");
   TORCH_CHECK(q.dim() == 3 && q.stride(2) == 1 && q.stride(1) == q.size(2), "q must be [N, H, D] with dense rows");
@@ -1205,6 +1206,7 @@ at::Tensor paged_attention(at::Tensor q, at::Tensor kpool, at::Tensor vpool, at:
   // long as its blocks fit beside the others; a launch of its own stands in line (10 to 15 us). It goes apart where its blocks
   // would be the first beyond one, or two, for each CU and it sees half as many keys as a portion or more: 14 beside portions
   // of 1000 and 963, window 1024: 80 us together, 70 apart (32 heads on 8: 123, 96), without a window 2100 keys 150, 133, 16000 keys 1427, 1110.
+  // `even` and `longest` then are those of the portions alone (`even_apart`, `longest_apart`).
   // Otherwise: 15 of 400 beside 4000, 8 heads on 4 of 64: 76 together, 86 apart; 15 beside 512 after 2000, window 512: 29, 40.
   int fewest = 1;
   if (singles > 0 && num_tiles > singles && vpool.is_contiguous()) {
@@ -1218,6 +1220,8 @@ at::Tensor paged_attention(at::Tensor q, at::Tensor kpool, at::Tensor vpool, at:
       num_tiles -= singles;
       num_tiles128 -= singles;
       num_tiles64 -= singles;
+      even = even_apart;
+      longest = longest_apart;
     }
   }
   if (launch_mfma_attention(out, q, kpool, vpool, block_tables, cu, start, slp, gate, gstride, scale, window, keep_first,

@@ -222,14 +222,17 @@ def paged_attention(q, kpool, vpool, batch: RaggedBatch, scale: float, window: i
                                                   batch.tok_seq, batch.positions, scale, window, keep_first, slopes,
                                                   gate, float(softcap), bool(sink), sink_logits, dist_bias, ksum, vsum,
                                                   int(block), talk is not None, tiles32, tiles128, tiles64, int(chunk), key_factors,
-                                                  out_dtype == torch.float32, *((0.5, chunk) if chunk > 0 else batch.key_lengths(window)))
+                                                  out_dtype == torch.float32, *((0.5, chunk) if chunk > 0 or not tiles32 else batch.key_lengths(window)))
         if talk is None:
             return o
         return serving_kernels().talk_mix(o, talk, q.dtype)
     if hip:
+        told = (0, False, 0.5, 0, 0.5, 0)
+        if tiles32:
+            count, half = batch.single_tokens(window)
+            told = (count, half, *batch.key_lengths(window), *batch.key_lengths(window, 2 if count else 1))
         return serving_kernels().paged_attention(q, kpool, vpool, batch.block_tables, batch.cu, batch.start,
                                                  batch.tok_seq, batch.positions, scale, window, keep_first,
-                                                 slopes, gate, tiles32, float(softcap), bool(sink), tiles128, tiles64,
-                                                 *(batch.single_tokens(window) + batch.key_lengths(window) if tiles32 else (0, False, 0.5, 0)))
+                                                 slopes, gate, tiles32, float(softcap), bool(sink), tiles128, tiles64, *told)
     return paged_attention_ref(q, kpool, vpool, batch, scale, window, keep_first, slopes, gate, softcap, sink,
                                sink_logits, dist_bias, pooled, talk, chunk, key_factors, out_dtype)

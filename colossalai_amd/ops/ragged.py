@@ -79,7 +79,7 @@ class RaggedBatch:
     _chunk_tables: Optional[dict] = None  # memo of chunk_tables(), by chunk size
     _tiles: Optional[tuple] = None  # memo of tile_counts()
     _singles: Optional[tuple] = None  # memo of single_tokens()
-    _even: Optional[dict] = None  # memo of key_lengths(), by window
+    _even: Optional[dict] = None  # memo of key_lengths(), by window and fewest
 
     @property
     def num_seqs(self) -> int:
@@ -115,13 +115,16 @@ class RaggedBatch:
             short, long = min(short, window), min(long, window)
         return count, 2 * short >= long
 
-    def key_lengths(self, window: int = 0):
-        """How many keys the tiles of 32 new tokens see on average, over the most that one sees; and these."""
+    def key_lengths(self, window: int = 0, fewest: int = 1):
+        """Of the tiles of 32 new tokens of the sequences that bring `fewest` or more: ``(mean / most, most)`` of the keys that a tile's last token
+        sees, about (a sequence's tiles count as its first and last one's mean), and the most that one sees."""
         if self._even is None:
             self._even = {}
-        if window not in self._even:
+        if (window, fewest) not in self._even:
             total = most = tiles = 0.0
             for a, b, s in zip(self.cu_host, self.cu_host[1:], self.start_host):
+                if b - a < fewest:
+                    continue
                 lo, hi, n = s + min(32, b - a), s + b - a, (b - a + 31) // 32
                 if window <= 0 or hi <= window:
                     mean = (lo + hi) / 2
@@ -132,8 +135,8 @@ class RaggedBatch:
                 total += mean * n
                 tiles += n
                 most = max(most, min(hi, window) if window > 0 else hi)
-            self._even[window] = total / (tiles * most), int(most)
-        return self._even[window]
+            self._even[window, fewest] = (total / (tiles * most), int(most)) if tiles else (0.5, 0)
+        return self._even[window, fewest]
 
     @property
     def num_tiles32(self) -> int:
