@@ -230,6 +230,25 @@ def test_scores_that_rise_and_fall(levels, D, causal):
         _near(a, b, name)
 
 
+# Levels of 32 keys: every half tile, every odd one, every even one passes the reference of those before it, or the first has the largest scores.
+LEVELS_32 = [(0, 9, 18, 27, 36, 45, 54, 63), (0, 25, 50, 75, 100, 125), (0, 14, 14, 28, 28, 42, 42, 56), (0, 0, 14, 14, 28, 28, 42), (63, 45, 54, 36, 27, 0, 9)]
+
+
+@pytest.mark.parametrize("levels", LEVELS_32)
+@pytest.mark.parametrize("S", [None, 160, 200])
+@pytest.mark.parametrize("D,causal", [(128, False), (64, False), (128, True)])
+def test_half_tiles_that_rise(levels, S, D, causal):
+    """The reference is raised after either half of a tile, while the weights of the half before it are on their way to the values."""
+    from colossalai_amd.ops import flash_attention
+
+    S = S or 32 * len(levels)
+    q, k, v, dout = _inputs(1, S, 4, 2, D)
+    q[..., 0] = 8.0
+    level = torch.tensor(levels, device="cuda").repeat_interleave(32)[:S]
+    k[..., 0] = torch.nn.functional.pad(level, (0, max(0, S - len(level))))[None, :, None] / (8.0 * D ** -0.5)
+    _near(flash_attention(q, k, v, causal=causal), _reference(q, k, v, dout, causal, D ** -0.5)[0], "out")
+
+
 @pytest.mark.parametrize("D", [64, 128])
 @pytest.mark.parametrize("packed", [False, True])
 def test_large_values_of_rising_scores(D, packed):
@@ -248,6 +267,27 @@ def test_large_values_of_rising_scores(D, packed):
     else:
         got = flash_attention(q, k, v, causal=False)
     _near(got, want, "out")
+
+
+@pytest.mark.parametrize("bad", [float("nan"), float("inf")])
+@pytest.mark.parametrize("D,causal", [(128, False), (64, False), (64, True)])
+def test_rows_past_a_padded_sequence_may_hold_anything(bad, D, causal):
+    """Ends in the first and in the second half of a tile and of a wave's rows; the rows past them are 0, and so are their gradients."""
+    from colossalai_amd.ops import flash_attention
+
+    lens = [130, 1, 33, 64, 95, 160, 97]
+    q, k, v, dout = _inputs(len(lens), 160, 4, 2, D)
+    past = torch.arange(160, device="cuda") >= torch.tensor(lens, device="cuda")[:, None]
+    want = [torch.zeros_like(t, dtype=torch.float32) for t in (q, q, k, v)]
+    for b, n in enumerate(lens):
+        for t, r in zip(want, _reference(*[t[b: b + 1, :n] for t in (q, k, v, dout)], causal, D ** -0.5)):
+            t[b, :n] = r[0]
+    q, k, v = (t.masked_fill(past[..., None, None], bad).requires_grad_() for t in (q, k, v))
+    out = flash_attention(q, k, v, causal=causal, seqlens=torch.tensor(lens, dtype=torch.int32, device="cuda"))
+    got = (out, *torch.autograd.grad(out, (q, k, v), dout))
+    for name, a, b in zip(("out", "dq", "dk", "dv"), got, want):
+        _near(a, b, name)
+        assert not a[past].any(), name
 
 
 @pytest.mark.parametrize("place", ["odd address", "odd rows", "far rows", "one row for all"])

@@ -230,8 +230,8 @@ def test_portions_of_head_counts_and_sizes(H, G, D, Dv, kw):
 
 
 @pytest.mark.parametrize("levels", [
-    (0, 9, 18, 27, 36, 45),          # every step's weights pass the reference of the one before
-    (60, 40, 20, 0, -20, -40),       # the first keys have the largest scores
+    (0, 9, 18, 27, 36, 45),          # the nearest keys, which are taken first, have the largest scores
+    (60, 40, 20, 0, -20, -40),       # every 64 keys' weights pass the reference of those before
     (-3000, 0, -3000, 4, 8, 1000),   # far below, far above
 ])
 @pytest.mark.parametrize("kw", [{}, dict(sink_logits=True), dict(window=200, keep_first=5)])
@@ -250,6 +250,37 @@ def test_scores_that_rise_and_fall(levels, kw, rows):
     for b in range(rows):
         for i, level in enumerate(levels):
             k[batch.block_tables[b, i].long(), :, :, 0] = level / (8.0 * scale)
+    kw = dict(kw)
+    if kw.pop("sink_logits", False):
+        kw["sink_logits"] = torch.randn(16, device="cuda") + 2.0
+    got = paged_attention(q, k, v, batch, scale, **kw)
+    want = paged_attention_ref(q.float(), k.float(), v.float(), batch, scale, **kw)
+    assert (got.double() - want.double()).norm() / want.double().norm() < BOUND
+
+
+@pytest.mark.parametrize("levels", [
+    (0, 9, 18, 27, 36, 45, 54, 63),  # from the farthest tile of 32 keys to the nearest, which is taken first
+    (63, 54, 45, 36, 27, 18, 9, 0),  # every tile passes the reference of those before it
+    (125, 100, 75, 50, 25, 0),
+    (56, 42, 42, 28, 28, 14, 14, 0),   # every second one does
+    (42, 42, 28, 28, 14, 14, 0),
+    (9, 0, 27, 36, 54, 45, 63),
+])
+@pytest.mark.parametrize("kw", [{}, dict(sink_logits=True), dict(window=150, keep_first=40)])
+@pytest.mark.parametrize("rows", [1, 32])
+def test_tiles_that_rise(levels, kw, rows):
+    """Keys 32 at a time have scores of a level of their own: the reference is raised after the first or the second of a step's two
+    tiles, while the other's weights are on their way to the values. `rows` sequences: two groups of waves a block, or one."""
+    from colossalai_amd.ops.paged_attention import paged_attention, paged_attention_ref
+
+    torch.manual_seed(13)
+    n, scale = 32 * len(levels), 128 ** -0.5
+    batch, pages = _batch([n - 10] * rows, [10] * rows, 32)
+    k, v = (torch.randn(pages, 32, 4, 128, device="cuda").bfloat16() for _ in range(2))
+    q = torch.randn(rows * (n - 10), 16, 128, device="cuda").bfloat16()
+    q[..., 0] = 8.0
+    for i, level in enumerate(levels):
+        k[batch.block_tables[:, i].long(), :, :, 0] = level / (8.0 * scale)
     kw = dict(kw)
     if kw.pop("sink_logits", False):
         kw["sink_logits"] = torch.randn(16, device="cuda") + 2.0
