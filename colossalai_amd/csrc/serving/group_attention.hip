@@ -13,8 +13,8 @@
 // products.
 // What bounds it: memory beyond about 8 us of dependent loads (position, page table, rows), launch and the end. The form with a
 // row in the registers of a few lanes (row_attention.hip) and this one, us, replayed from a graph: 16 heads on 4 of 128: 16 x 1024 keys with a
-// cap and a sink 15.6, 15.5, 4 x 16384 38.6, 30.9 (4.3 TB/s), 16 x 8192 56.2, 47.7 (5.6 TB/s); 8 on 2 of 128, 7 x 5000 20.2, 15.0; 16
-// on 8 of 64, 16 x 3000 25.6, 23.0; one head a key head, 16 x 2000 45.7, 43.1; 16 on 1 of 128, 16 x 2000 21.0, 16.0.
+// cap and a sink 15.6, 11.7, 4 x 16384 38.6, 28.1 (4.8 TB/s), 16 x 8192 56.2, 47.0 (5.7 TB/s); 8 on 2 of 128, 7 x 5000 20.2, 13.0; 16
+// on 8 of 64, 16 x 3000 25.6, 23.0; one head a key head, 16 x 2000 45.7, 43.5; 16 on 1 of 128, 16 x 2000 21.0, 14.8.
 // The eight waves' states meet in LDS at the end; few tokens have their keys cut into parts, whose states the block that ends last puts
 // together (a launch for that took 4 to 6 us, and the host as long as the first one's). Which one that is needs no memory that somebody has cleared: a part
 // leaves its states, then a mark that belongs to this launch alone, then looks at all marks of its token and key head. The last
@@ -462,13 +462,19 @@ bool launch_group_attention(at::Tensor& out, const at::Tensor& q, const at::Tens
     if (!cols && blocks < 32 && keys < 8192 && blocks * keys < 20000) return false;
     if (slopes != nullptr && blocks <= 64 && keys <= 512) return false;
   }
-  // Parts of the keys while there are fewer blocks than CUs. A tile of 32 keys takes a wave 1.75 us at 128 channels, of which eight run side by side;
-  // parts cost 2 us (2.5 over 500 keys that are in L2), a store and three round trips to memory, and 0.1 each for reading their states. Whole, and in parts: 16 x 1024 (16 heads on
-  // 4 of 128) 22.8 us, 2: 19.0, 4: 16.0, 8 (512 blocks): 22.8; 4 x 16384 277, 8: 48.4, 16: 36.6, 32: 41.4; 1 x 8192 66, 8: 17.4, 16: 14.4, 24:
-  // 13.4, 64: 16.1; 1 x 2048 20.8, 4: 12.9, 12: 11.3, 16: 10.8; 16 x 300 (8 on 4) 9.3, 2: 10.6, 4: 9.9; 3 x 1500 (4 on 2 of 64) 12.3, 8: 8.2.
-  const double whole = (double)((keys + 31) / 32) * 0.22 * (D + Dv) / 256;
-  int splits = (int)std::max<long>(1, std::min<long>({256 / blocks, WAVE, std::lround(std::sqrt(whole * 10.0))}));
-  if (whole < 4.2 || whole <= whole / splits + 2.0 + 0.1 * splits) splits = 1;
+  // Parts of the keys while there are fewer blocks than CUs. A tile of 32 keys takes a wave 1.75 us at 128 channels, and eight waves run
+  // side by side; parts cost 2.4 us (64 channels) to 3.6 for a store and three round trips to memory, and each of them
+  // 0.08 and more for the reading of its states, which one block does for all heads of the group, eight parts at a time. Whole and in
+  // parts, other keys and values in every call, us: 16 heads on 4 of 128, 16 x 1000 14.5, 2: 13.8, 4: 13.4; 4 x 600 8.6, 2: 9.9, 8: 9.2; 1 x 2000 18.3,
+  // 4: 11.0, 8: 10.5, 16: 9.8; 1 x 8000 64, 8: 16.9, 24: 13.2, 64: 16.0; 4 x 16000 223, 8: 40.9, 16: 33.2; 16 on 1 of 128, 16 x 2000 23.7, 4: 17.2, 8: 15.9,
+  // 12: 18.0; 8 x 16000 132, 8: 31.0, 16: 26.1, 24: 27.9, 32: 29.8; 8 on 8 of 128, 16 x 800 13.9, 2: 16.6; 8 on 4 of 64, 8 x 1000 9.4, 4: 8.7,
+  // 8: 8.2. Over 1219 such sizes the rule's choice takes 0.6 % more than the best one on average.
+  const double whole = (double)((keys + 31) / 32) * 0.22 * (D + Dv) / 256, each = std::max(0.08, 0.02 * R * Dv / 128);
+  const long most = std::max<long>(1, std::min<long>(256 / blocks, WAVE));
+  long parts = std::min(most, std::lround(std::sqrt(whole / each)));
+  if (parts >= 6) parts = std::min(most, (parts + 4) / 8 * 8);
+  if (parts > 8) parts = parts / 8 * 8;
+  const int splits = parts < 2 || whole <= whole / parts + 1.2 + 2.4 * (D + Dv) / 256 + each * parts ? 1 : (int)parts;
   // page numbers of a part: of its keys, rounded up to whole tiles, of a page more for where they begin, and of the kept ones
   const long part_keys = ((keys + 31) / 32 + splits - 1) / splits * 32;
   const long table = block_tables.size(1);
