@@ -622,18 +622,6 @@ __global__ __launch_bounds__(256 * NG, 2) void paged_attention_mfma_kernel(
   // the first step's values behind its keys: they are not waited for yet
 #pragma unroll
   for (int n = 0; n < TP * VR; ++n) value_piece(vrow, values, n);
-  // The steps in which the wave sees something: from `from` up to `stop` in its window, then, where the kept first keys or summaries lie apart, from
-  // `again` on. Numbers, and not a look at each step's tiles, which as a condition of the loop cost up to 470 spilled registers.
-  const int mine0 = first_tile + grp * TP;      // the group's first tile of step 0
-  const int w_lo = keep_first > wstart ? sink_tiles : sink_tiles + (max(0, lo_p0 - wstart) >> 5);   // lowest and highest tile of the wave's window
-  const int w_hi = min(tiles_n - 1, sink_tiles + ((p1 - wstart) >> 5));
-  const int again = head_ok ? (max(0, mine0 - sink_tiles + 1) + TS - 1) / TS : steps_n;
-  int from = head_ok ? (max(0, mine0 - w_hi) + TS - 1) / TS : steps_n, stop = (mine0 + 1 - w_lo + TS) / TS;
-  if (again <= stop) stop = steps_n;
-  if (from >= stop) {   // the group's tiles lie beside a short window
-    from = again;
-    stop = steps_n;
-  }
   if (quad0 == 0) loads_left<TP * VR>();
   else loads_left<TP * (VQ / 2)>();
   __syncthreads();
@@ -909,10 +897,17 @@ __global__ __launch_bounds__(256 * NG, 2) void paged_attention_mfma_kernel(
     for (int i = 0; i < GROUPS; ++i) load_first(i);
     end();
   };
+  // A wave that has begun goes on up to `stop`, the first step with nothing of its window, and where kept first keys or summaries lie apart, from `again` on:
+  // numbers, as a look at each step's tiles in the loop cost up to 470 spilled registers. A loop around both parts is slower too (decode tokens two
+  // by two, 16 heads on 8, 1000 keys 27.9 us for 26.9).
+  const int mine0 = first_tile + grp * TP;      // the group's first tile of step 0
+  const int w_lo = keep_first > wstart ? sink_tiles : sink_tiles + (max(0, lo_p0 - wstart) >> 5);   // lowest tile of the wave's window
+  const int again = head_ok ? (max(0, mine0 - sink_tiles + 1) + TS - 1) / TS : steps_n;
+  int stop = (mine0 + 1 - w_lo + TS) / TS;
+  if (again <= stop) stop = steps_n;
   auto mine_of = [&](int u) { return tile_of(tile0 + grp * TP + u); };
-  do {
-    while (step < from) idle();
-    if (step >= steps_n) break;
+  while (step < steps_n && !mine_of(0).live && !mine_of(1).live) idle();
+  if (step < steps_n) {
     f32x16 xe, xo;            // scores of an even and an odd tile of the wave's
     Weights pe, po;
     {
@@ -936,9 +931,22 @@ __global__ __launch_bounds__(256 * NG, 2) void paged_attention_mfma_kernel(
     const char* V_ = values + (~step & 1) * VS;
     weights_turn(no, yes, odd, (third == 0 ? 2 : third - 1) * TS + grp * TP + 1, V_, V_, xe, xo, po, pe, nothing);
     turn(no, no, yes, cap_poly, V_, V_ + VTT, xo, xe, 0.0f, pe, po, nothing);
-    from = max(step, again);
-    stop = steps_n;
-  } while (step < steps_n);
+  }
+  while (step < again) idle();
+#pragma clang loop unroll(disable)
+  while (step < steps_n) {   // the tiles ahead of the window, few and seldom apart: step by step
+    f32x16 xe, xo;
+    Weights pe, po;
+    const Tile even = mine_of(0), odd = mine_of(1);
+    begin();
+    const char* K_ = keys + (step & 1) * KS;
+    turn(yes, no, no, cap_poly, K_, K_, xe, xo, 0.0f, po, pe, load_first);
+    weights_turn(yes, no, even, third * TS + grp * TP, K_ + KT, K_, xo, xe, pe, po, nothing);
+    end();
+    const char* V_ = values + (~step & 1) * VS;
+    weights_turn(no, yes, odd, (third == 0 ? 2 : third - 1) * TS + grp * TP + 1, V_, V_, xe, xo, po, pe, nothing);
+    turn(no, no, yes, cap_poly, V_, V_ + VTT, xo, xe, 0.0f, pe, po, nothing);
+  }
   if constexpr (NG > 1) {  // the second group's states, wave by wave, through the tiles' place
     __syncthreads();         // all waves are past their last tile
     float4v* sums = reinterpret_cast<float4v*>(tiles) + wid * (VT * 4 * 64 + 32) + lane;   // 16 bytes an access
