@@ -1004,10 +1004,10 @@ void set_lds_limit(const void* kernel, size_t bytes) {
 }
 
 // Waves (of 32 query rows) of a forward block. Four: two blocks share a CU, and their barriers do not
-// hold each other up (8 waves in one block: 735 against 809 TFLOP/s at B4 S4096 H32 D128 causal). Two when blocks
-// of four would leave CUs empty (B2 S256 H4 D128: 10.3 against 12.4 us; B8 S197 H12 D64: 10.2 against 10.6); twice
-// the reads of K and V make them slower as soon as the chip is full (4096: 507 TFLOP/s).
-int fwd_waves(int S, long rows) { return (S + 4 * fa::QW - 1) / (4 * fa::QW) * rows < 256 ? 2 : 4; }
+// hold each other up (8 waves in one block: 735 against 809 TFLOP/s at B4 S4096 H32 D128 causal). Two as long as blocks of two have a CU each, up to
+// 128 of four: a wave has fewer neighbours to wait for, 8 to 20 % at 128 and 256 tokens, nothing at 2048. Beyond, two blocks of two share a CU
+// and its loads are twice those of one block of four: 4/2 waves at 144 to 252 blocks 0.93 (128 tokens), 0.84 (512), 0.76 (2048); with a mask 0.9, 0.83, 0.98.
+int fwd_waves(long blocks) { return blocks <= 128 ? 2 : 4; }
 
 // q/k/v are [B,S,H,D] views that may be strided in dims 0/1 (e.g. views into
 // a packed QKV GEMM output); dims 2/3 must be dense.
@@ -1072,7 +1072,7 @@ std::vector<at::Tensor> flash_attn_fwd(at::Tensor q, at::Tensor k, at::Tensor v,
                        B, S, Sk, Hq, Hkv, (float)scale, causal ? 1 : 0);                              \
   } while (0)
 
-  const int nw = fwd_waves(S, (long)B * Hq);
+  const int nw = fwd_waves((S + 4 * QW - 1L) / (4 * QW) * B * Hq);
   if (D == 128) { if (nw == 4) LAUNCH_FWD(128, 4); else LAUNCH_FWD(128, 2); }
   else { if (nw == 4) LAUNCH_FWD(64, 4); else LAUNCH_FWD(64, 2); }
 #undef LAUNCH_FWD
@@ -1115,7 +1115,9 @@ std::vector<at::Tensor> flash_attn_varlen_fwd(at::Tensor q, at::Tensor k, at::Te
                        n_seq, T, T, Hq, Hkv, (float)scale, causal ? 1 : 0);                          \
   } while (0)
 
-  const int nw = fwd_waves((int)max_seqlen, (long)n_seq * Hq);
+  // blocks' worth of waves that have tokens, a sequence's last wave half of them (8 heads on 2 of 128, 23 samples of 8 to 128 tokens: 6.8 us, blocks of four 7.3)
+  const long whole = (max_seqlen + 4 * QW - 1) / (4 * QW) * n_seq, some = T / (4 * QW) + n_seq / 8;
+  const int nw = fwd_waves(std::min(whole, some) * Hq);
   if (D == 128) { if (nw == 4) LAUNCH_VFWD(128, 4); else LAUNCH_VFWD(128, 2); }
   else { if (nw == 4) LAUNCH_VFWD(64, 4); else LAUNCH_VFWD(64, 2); }
 #undef LAUNCH_VFWD

@@ -199,6 +199,23 @@ def test_strided_gradients_with_shared_heads():
         _near(a, b, name)
 
 
+@pytest.mark.parametrize("H", [31, 32, 33])
+@pytest.mark.parametrize("D,causal", [(64, True), (128, False)])
+@pytest.mark.parametrize("packed", [False, True])
+def test_on_either_side_of_blocks_of_two_waves(H, D, causal, packed):
+    """Four tiles of 128 rows a head: up to 128 blocks of four waves they are cut into blocks of two."""
+    from colossalai_amd.ops import flash_attention, flash_attention_varlen
+
+    q, k, v, dout = _inputs(1, 500, H, H, D)
+    want = _reference(q, k, v, dout, causal, D ** -0.5)[0]
+    if packed:
+        cu = torch.tensor([0, 500], dtype=torch.int32, device="cuda")
+        got = flash_attention_varlen(q[0], k[0], v[0], cu, 500, causal=causal)[None]
+    else:
+        got = flash_attention(q, k, v, causal=causal)
+    _near(got, want, "out")
+
+
 @pytest.mark.parametrize("levels", [
     (0, 9, 18, 27, 36, 45),          # every tile's weights pass the reference of the one before
     (0, 5, 10, 15, 20, 25),          # every second one's do
