@@ -5,11 +5,12 @@
 //                    rms_norm(u) * w is formed in the same launch;
 //   streams_update : the write of one sublayer, in place, and the read + norm of the next one
 //                    (or of the output, with in = 1 everywhere) in one pass over the streams;
-//   streams_read   : what an update would read and norm, without the write;
-//   streams_update_two : the writes of two sublayers, the second formed over the first in registers.
-// A layer of two sublayers reads the streams twice and writes them once with the last two, where two updates write them twice: 4096 tokens, four
-// streams of 2048, 47 + 47 -> 30 + 51 us. Ahead of the first write every stream is the token's embedding row, which is read instead
-// of them (`table`, `tokens`), so that they need not be written at the start (37 -> 15 us).
+//   streams_pass   : either what an update would read and norm, without the write, or the writes of two sublayers, the second formed
+//                    over the first in registers, with the read and norm after them.
+// A layer of two sublayers then reads the streams twice and writes them once with the last two, where two updates write them twice: 4096 tokens, four
+// streams of 2048, 47 + 47 -> 30 + 51 us. Ahead of the first write every stream is the token's embedding row, which streams_pass reads in the
+// place of them (`table`, `tokens`), so that they need not be written at the start (37 -> 15 us). It serves up to 4 streams of a
+// width that is a multiple of 4 up to 4096; others are updated one sublayer at a time.
 #include "serving_common.h"
 
 namespace cai {
@@ -230,7 +231,7 @@ c10::optional<at::Tensor> streams_update(at::Tensor x, at::Tensor y, at::Tensor 
   return h;
 }
 
-// streams_read (no y1; nothing is written) and streams_update_two (x: [N, S, W], or with `table` to be filled). The old streams are x or, with `table`
+// Without y1 nothing is written; with it both sublayers' writes go to x [N, S, W], with `table` to be filled. The old streams are x or, with `table`
 // [vocab, W] of y's type and `tokens` [N], S times the token's row. For up to 4 streams of a width that is a multiple of 4 up to
 // 4096, everything at addresses of 16 bytes (streams_pairs says so); returns nothing otherwise, having done nothing.
 bool streams_pairs(int64_t S, int64_t W) { return S >= 1 && S <= 4 && W % 4 == 0 && W <= 4096; }
