@@ -5,21 +5,23 @@
 // gradient) transposing ones (ds_read_b64_tr_b16, see flash_attn.hip). Four waves hold a tile's sums in registers, one
 // quarter each: 256 x 256 where there is enough of them, which is the least LDS and memory traffic a product has here (a
 // wave's 128 x 128 sums are 256 registers, one wave a SIMD), else 256 x 128, also one block a CU (96 KB of LDS), or 128 x 128 with
-// two. Four steps of 32
-// contracted indices lie in LDS: while one is multiplied the next is there and two are on their way, so that a step waits for
-// loads that are two steps old (s_waitcnt vmcnt, never 0) and for one barrier. A wave reads the fragments of the next 16
-// indices and issues its loads one by one between the products of the 16 before.
+// two. Four steps of 32 contracted indices lie in LDS. A wave reads each fragment again, from the next step, as soon as its last product of this
+// one is done; loads go to a step's place half a step after all of its fragments are read, so that they are two and a half to three
+// steps old when they are waited for (s_waitcnt vmcnt, never 0), at one barrier a step.
 //
-// What bounds it: a step of the large tile takes 1203 cycles of which the products are 1024; the clock falls to 1.4 to 1.6
-// GHz under it (M 4096 and 12288, N 4096, K 16384). The small tile takes 725 cycles for two blocks, 512 of them products.
+// What bounds it: power, and the issue of one wave a SIMD. Matrix instructions of 16 x 16 x 32 instead of 32 x 32 x 16 touch the sums half as
+// often: a loop of nothing else runs at 2060 TFLOP/s on the full chip for 1775. They leave room for two to three other instructions
+// each (a third one costs 4 cycles of 16), so that reads and loads stand one by one between them, nothing else is computed in the loop, and the ring
+// is unrolled. M 12288, N 4096, K 16384: 32 x 32 x 16 74 % of the cycles are products, at 1.44 GHz; 16 x 16 x 32 in the same order 61 %, 1.71 GHz; as
+// it is now 78 %, 1.50 GHz.
 //
-// Weight gradients M, N, K; us with the library's product -> here:
-//   22016, 4096, 16384   2785 -> 2214     4096, 11008, 16384   1536 -> 1132     4096, 4096, 16384   470 -> 404
-//   32000, 4096, 4096     952 -> 859      32000, 768, 4096      223 -> 191      4096, 768, 8192      84 -> 61
-//   768, 2048, 8192        65 -> 38       768, 768, 8192         49 -> 22       2048, 512, 512       21 -> 10
-// Small others, back to back (the library's call takes the host 19 to 20 us, its kernels 5 to 11):
+// Weight gradients M, N, K; us with the library's product -> 32 x 32 x 16 -> here:
+//   22016, 4096, 16384   2800 -> 2270 -> 2060     4096, 11008, 16384   1540 -> 1140 -> 1040     4096, 4096, 16384   460 -> 403 -> 375
+//   32000, 4096, 4096     940 -> 893 -> 806       32000, 768, 8192     462 -> 347 -> 320        4096, 768, 8192      77 -> 59 -> 56
+//   768, 2048, 8192        62 -> 36 -> 34         768, 768, 8192        48 -> 21 -> 19          3072, 1024, 2048     24 -> 22 -> 19
+// Small others, back to back (the library's call takes the host 19 to 20 us, its kernels 5 to 11), with the products of 32 x 32 x 16:
 //   x W^T: 512, 1536, 512   19.2 -> 9.0   512, 512, 1024   19.7 -> 11.4     dy W: 512, 512, 2048   19.2 -> 13.9
-// Large ones stay with the library: 16384, 12288, 4096   1080 us there, 1468 here; dy W 16384, 4096, 12288   1224, 1377.
+// Large ones stay with the library: 16384, 12288, 4096   1048 us there, 1490 here (its rows are read 64 bytes at a time); dy W 16384, 4096, 12288   1265, 1310.
 #include <torch/extension.h>
 #include <ATen/hip/HIPContext.h>
 #include <c10/hip/HIPGuard.h>
@@ -35,13 +37,13 @@ namespace pr {
 
 constexpr int KT = 32;       // contracted indices of a step
 
-// One operand of a product: how a step of it comes into LDS and how the matrix unit's fragments are read from there. A step is pieces
-// of 1024 bytes, each brought by one load of a wave straight into LDS, 16 bytes a lane; 32 free indices are
-// 2048 bytes. Either form spreads every access over the 64 banks, and both hand out the contracted indices in the same order.
+// One operand of a product: how a step of it comes into LDS and how the matrix unit's fragments (16 free by 32 contracted indices, eight of the
+// contracted ones a lane) are read from there. A step is pieces of 1024 bytes, each brought by one load of a wave straight into LDS, 16 bytes a lane.
+// Either form spreads every access over the 64 banks, and both hand out the contracted indices in the same order.
 //
 // COLS: the free index is the fast one ([K, free] in memory). Pieces of 8 contracted by 64 free indices, the four pieces of 64 free
-// indices one after the other, 128 neighbouring bytes a row. A row's 16-byte unit u lies at place u ^ 4 * (row / 2 % 2),
-// so that the four rows of 32 columns that half a wave's transposing read takes are in different banks. The descriptor of a
+// indices one after the other, 128 neighbouring bytes a row. A row's 16-byte unit u lies at place u ^ 4 * (row / 2 % 2) ^ 2 * (piece % 2),
+// so that the eight rows of 16 columns that half a wave's transposing read takes, four of either piece, are in different banks. The descriptor of a
 // step ends with the last row: rows past it come as zeros; columns past the last one bring what follows, into results
 // that are not stored.
 // Rows otherwise ([free, K] in memory). Pieces of 16 free by 32 contracted indices as in lds_tiles.h; free indices past the last
@@ -49,51 +51,60 @@ constexpr int KT = 32;       // contracted indices of a step
 template <bool COLS, int T>
 struct Operand {
   static constexpr int PER = T / 64, BYTES = T * KT * 2;   // pieces of a wave, bytes of a step
-  const unsigned short* base;
+  const unsigned short* base;   // of the next step to be brought
   long stride;
-  int left, end;                // free indices left from the tile's first one, contracted ones
+  int whole, last;              // bytes of a step, of the last one
   unsigned off;
-  int even, odd;                // where a lane reads: free indices 0-31 and 32-63 of 64, or contracted ones 0-15 and 16-31
+  int at[COLS ? 4 : 1];         // where a lane reads, by which 16 of 64 free indices
 
-  DEV_INLINE Operand(const unsigned short* p, long stride, int first, int all, int end) : stride(stride), left(all - first), end(end) {
-    const int lane = threadIdx.x & 63, half = lane >> 5;
+  // the operand's free indices from `first` on, of `all`, contracted ones from k0 up to k1
+  DEV_INLINE Operand(const unsigned short* p, long stride, int first, int all, int k0, int k1, int w) : stride(stride) {
+    const int lane = threadIdx.x & 63, m = lane & 15, g = lane >> 4, left = all - first;
     if (COLS) {
-      base = p + first;
-      const int row = lane >> 3, m = lane & 15;
-      off = (unsigned)(row * stride) * 2u + (((lane & 7) ^ ((row >> 1 & 1) << 2)) * 16);
-      even = half * 1024 + (m >> 2) * 128 + (m >> 3 & 1) * 64 + (lane >> 4 & 1) * 32 + (m & 3) * 8;
-      odd = even ^ 64;
+      base = p + first + k0 * stride;
+      whole = (int)(((unsigned)(KT - 1) * (unsigned)stride + (unsigned)left) * 2u);
+      last = (int)(((unsigned)((k1 - k0 - 1) % KT) * (unsigned)stride + (unsigned)left) * 2u);
+      const int row = lane >> 3;
+      off = (unsigned)(row * stride) * 2u + (((lane & 7) ^ ((row >> 1 & 1) << 2) ^ ((w & 1) << 1)) * 16);
+#pragma unroll
+      for (int b = 0; b < 4; ++b)
+        at[COLS ? b : 0] = g * 1024 + (m >> 2) * 128 + ((b * 2) ^ (m >> 1 & 1) ^ ((m >> 3 & 1) << 2) ^ ((g & 1) << 1)) * 16 + (m & 1) * 8;
     } else {
-      base = p + (long)first * stride;
+      base = p + (long)first * stride + k0;
+      whole = last = (int)(((unsigned)(min(left, T) - 1) * (unsigned)stride + KT) * 2u);
       const int row = lane >> 2;
       off = (unsigned)(row * stride) * 2u + (((lane & 3) ^ (row >> 2 & 3)) * 16);
-      const RowAt at(lane & 31, half);
-      even = at.even;
-      odd = at.odd;
+      at[0] = m * 64 + (g ^ (m >> 2)) * 16;
     }
   }
-  DEV_INLINE __amdgpu_buffer_rsrc_t step(int k) const {
-    const int rows = COLS ? min(end - k, KT) : min(left, T);
-    const unsigned bytes = ((unsigned)(rows - 1) * (unsigned)stride + (unsigned)(COLS ? left : end - k)) * 2u;
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<unsigned short*>(base + (COLS ? k * stride : (long)k)), 0, k < end ? (int)bytes : 0, 0x00027000);
+  // the next step, `left` of them with it
+  DEV_INLINE __amdgpu_buffer_rsrc_t step(int left) {
+    const auto t = __builtin_amdgcn_make_buffer_rsrc(const_cast<unsigned short*>(base), 0, left > 1 ? whole : left == 1 ? last : 0, 0x00027000);
+    base += COLS ? KT * stride : (long)KT;
+    return t;
   }
   // piece i of wave w
   DEV_INLINE void piece(__amdgpu_buffer_rsrc_t t, char* __restrict__ lds, int w, int i) const {
     const int c = i * 4 + w;
-    const unsigned at = COLS ? (unsigned)(w * 8 * stride + i * 64) * 2u : (unsigned)(c * 16 * stride) * 2u;
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(t, (lds_ptr)(lds + c * 1024), 16, (int)off, (int)at, 0, 0);
+    const unsigned from = COLS ? (unsigned)(w * 8 * stride + i * 64) * 2u : (unsigned)(c * 16 * stride) * 2u;
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(t, (lds_ptr)(lds + c * 1024), 16, (int)off, (int)from, 0, 0);
   }
-  // contracted indices 16 ks .. of free ones 32 b ..
-  DEV_INLINE bf16x8_v frag(const char* __restrict__ lds, int ks, int b) const {
-    if (!COLS) return *reinterpret_cast<const bf16x8_v*>(lds + (ks ? odd : even) + b * 2048);
-    const int o = (b & 1 ? odd : even) + (b >> 1) * 4096 + ks * 2048;
-    const bf16x4_v lo = ld_tr16(lds, o), hi = ld_tr16(lds, o + 512);
-    return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+  // A step's contracted indices of free ones 16 b ..: lane l has those from 8 * (l / 16) on of free index l % 16. Read r of READS.
+  static constexpr int READS = COLS ? 2 : 1;
+  struct Frag {
+    bf16x4_v lo, hi;
+    bf16x8_v row;
+    DEV_INLINE bf16x8_v all() const { return COLS ? __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7) : row; }
+  };
+  DEV_INLINE void read(const char* __restrict__ lds, int b, int r, Frag& f) const {
+    if constexpr (COLS) (r ? f.hi : f.lo) = ld_tr16(lds, at[b & 3] + (b >> 2) * 4096 + r * 512);
+    else f.row = *reinterpret_cast<const bf16x8_v*>(lds + at[0] + b * 1024);
   }
 };
 
+// every wave's loads but the last N have arrived, and what it has read from LDS too
 template <int N>
-DEV_INLINE void arrived_but() { asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(N) : "memory"); }
+DEV_INLINE void arrived_but() { asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory"); }
 
 struct Args {
   const unsigned short *p, *q;  // C[m, n] = sum over k of P(m, k) Q(n, k)
@@ -119,9 +130,6 @@ DEV_INLINE int xcd_chunk(int f, int n) {
   return (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + (f >> 3);
 }
 
-// four neighbouring sums of a fragment
-DEV_INLINE float4v sums(const f32x16& c, int jj) { return float4v{c[jj * 4], c[jj * 4 + 1], c[jj * 4 + 2], c[jj * 4 + 3]}; }
-
 DEV_INLINE void put(const Args& a, long at, float4v v) {
   if (a.sum) {
     *reinterpret_cast<float4v*>(a.sum + at) = v;
@@ -133,14 +141,62 @@ DEV_INLINE void put(const Args& a, long at, float4v v) {
   *reinterpret_cast<short4v*>(a.out + at) = pk;
 }
 
+// c += x y. The compiler copies sums that are loop-carried in accumulation registers to other ones and back around each product of this size (128 moves and 50
+// waits in a loop of 32 products), so it is told the register. What the compiler would otherwise look after: settled() stands between these products and
+// any other use of the sums, ahead of them and behind them.
+template <bool ACC>
+DEV_INLINE void mac(float4v& c, bf16x8_v x, bf16x8_v y) {
+  if constexpr (ACC) asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(x), "v"(y));
+  else c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x, y, c, 0, 0, 0);
+}
+// A product's result may be read 7 cycles of issue after it, and a product may read what another instruction wrote 2 after that.
+template <int FA, int FB>
+DEV_INLINE void settled(float4v (&c)[FA][FB]) {
+  auto each = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < FA; ++i)
+#pragma unroll
+      for (int j = 0; j < FB; ++j) asm volatile("" : "+a"(c[i][j]));
+  };
+  each();
+  asm volatile("s_nop 15");
+  each();
+}
+
+// Behind which of a half step's N products its reads and loads stand: of `reads` those from `at` on are each not before a product of their own
+// (`each` reads every `every` products), loads where no read is, as long as there is room.
+template <int N, int READS, int LOADS>
+struct Places {
+  int read[READS] = {}, load[LOADS] = {};
+  constexpr Places(int at, int each, int every) {
+    constexpr int MOST = (READS + LOADS + N - 1) / N;   // between two products
+    int used[N] = {};
+    for (int r = 0, n = 0; r < READS; ++r) {
+      const int first = r < at ? 0 : ((r - at) / each + 1) * every;
+      if (n < first) n = first;
+      while (n < N - 1 && used[n] >= MOST) ++n;
+      read[r] = n;
+      ++used[n];
+    }
+    for (int l = 0, n = 0; l < LOADS; ++l) {
+      const int even = (2 * l + 1) * N / (2 * LOADS);
+      if (n < even) n = even;
+      while (n < N - 1 && used[n] >= MOST) ++n;
+      if (used[n] >= MOST) n = even;
+      load[l] = n;
+      ++used[n];
+    }
+  }
+};
+
 // STEPS steps lie in LDS: one in use, one arrived, the others on their way.
 template <bool PC, bool QC, int TM, int TN, int STEPS>
 __global__ __launch_bounds__(256, TM == 256 ? 1 : 2) void product_kernel(const Args a) {
   extern __shared__ char smem[];
-  constexpr int FA = TN / 64, FB = TM / 64;
+  constexpr int FA = TN / 32, FB = TM / 32;      // fragments of a wave
   constexpr int YB = Operand<PC, TM>::BYTES, SB = YB + Operand<QC, TN>::BYTES;
-  constexpr int PER = FA + FB;
-  const int lane = threadIdx.x & 63, half = lane >> 5, ln = lane & 31;
+  constexpr int PY = Operand<PC, TM>::PER, PER = PY + Operand<QC, TN>::PER;
+  const int lane = threadIdx.x & 63, quarter = lane >> 4, ln = lane & 15;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wm = w & 1, wn = w >> 1;
 
@@ -158,91 +214,114 @@ __global__ __launch_bounds__(256, TM == 256 ? 1 : 2) void product_kernel(const A
   int tm, tn;
   where(a, tile, tm, tn);
   const int m0 = tm * TM, n0 = tn * TN;
-  const Operand<PC, TM> P(a.p, a.ldp, m0, a.M, k1);
-  const Operand<QC, TN> Q(a.q, a.ldq, n0, a.N, k1);
+  Operand<PC, TM> P(a.p, a.ldp, m0, a.M, k0, k1, w);
+  Operand<QC, TN> Q(a.q, a.ldq, n0, a.N, k0, k1, w);
 
-  f32x16 acc[FA][FB];
+  float4v acc[FA][FB];
 #pragma unroll
   for (int i = 0; i < FA; ++i)
 #pragma unroll
-    for (int j = 0; j < FB; ++j)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
+    for (int j = 0; j < FB; ++j) acc[i][j] = float4v{0.0f, 0.0f, 0.0f, 0.0f};
 
   const int steps = (k1 - k0 + KT - 1) / KT;
-  auto bring = [&](int s, char* __restrict__ to, int i, __amdgpu_buffer_rsrc_t yt, __amdgpu_buffer_rsrc_t xt) __attribute__((always_inline)) {
-    if (i < FB) P.piece(yt, to, w, i);
-    else Q.piece(xt, to + YB, w, i - FB);
+  auto bring = [&](char* __restrict__ to, int i, __amdgpu_buffer_rsrc_t yt, __amdgpu_buffer_rsrc_t xt) __attribute__((always_inline)) {
+    if (i < PY) P.piece(yt, to, w, i);
+    else Q.piece(xt, to + YB, w, i - PY);
   };
 #pragma unroll
   for (int s = 0; s < STEPS - 1; ++s) {
-    const auto yt = P.step(k0 + s * KT), xt = Q.step(k0 + s * KT);
+    const auto yt = P.step(steps - s), xt = Q.step(steps - s);
 #pragma unroll
-    for (int i = 0; i < PER; ++i) bring(s, smem + s * SB, i, yt, xt);
+    for (int i = 0; i < PER; ++i) bring(smem + s * SB, i, yt, xt);
   }
-  bf16x8_v fx[2][FA], fy[2][FB];
-  // fragments in the order of their use
-  auto read = [&](const char* __restrict__ st, int ks, int r, bf16x8_v (&px)[FA], bf16x8_v (&py)[FB]) __attribute__((always_inline)) {
-    if (r == 0) px[0] = Q.frag(st + YB, ks, wn * FA);
-    else if (r <= FB) py[r - 1] = P.frag(st, ks, wm * FB + r - 1);
-    else px[r - FB] = Q.frag(st + YB, ks, wn * FA + r - FB);
-  };
-  arrived_but<(STEPS - 2) * PER>();
+  // A step multiplies the first half of P's fragments with all of Q's, then the second half. Each fragment is read again as soon as its last product
+  // is done, in the same registers: Q's and the first half of P's in a step's second half, from the next step, the others in the first half. Between the
+  // halves every wave has read all of the step, and the step that is STEPS ahead goes to its place: half of its loads in this second half, half in
+  // the next first one. One read or load stands between two products, where there is time for three instructions.
+  constexpr int H = FB / 2, NM = FA * H, LH = PER / 2;
+  constexpr bool ACC = TM == 256;
+  typename Operand<PC, TM>::Frag fy[FB];
+  typename Operand<QC, TN>::Frag fx[FA];
+  constexpr int RP = Operand<PC, TM>::READS, RQ = Operand<QC, TN>::READS;
+  auto read_x = [&](const char* __restrict__ st, int i, int r) __attribute__((always_inline)) { Q.read(st + YB, wn * FA + i, r, fx[i]); };
+  auto read_y = [&](const char* __restrict__ st, int j, int r) __attribute__((always_inline)) { P.read(st, wm * FB + j, r, fy[j]); };
+  __amdgpu_buffer_rsrc_t yt = P.step(steps - (STEPS - 1)), xt = Q.step(steps - (STEPS - 1));
 #pragma unroll
-  for (int r = 0; r < PER; ++r) read(smem, 0, r, fx[0], fy[0]);
+  for (int i = 0; i < LH; ++i) bring(smem + (STEPS - 1) * SB, i, yt, xt);
+  arrived_but<(STEPS - 2) * PER + LH>();
+#pragma unroll
+  for (int j = 0; j < H * RP; ++j) read_y(smem, j / RP, j % RP);
+#pragma unroll
+  for (int i = 0; i < (FA - 1) * RQ; ++i) read_x(smem, i / RQ, i % RQ);
 
-  constexpr int NM = FA * FB;
-  auto step = [&](int s, const char* __restrict__ cur, const char* __restrict__ nxt, char* __restrict__ to) __attribute__((always_inline)) {
-    __amdgpu_buffer_rsrc_t yt, xt;
-    const int row = k0 + (s + STEPS - 1) * KT;
+  constexpr Places<NM, RQ + H * RP, LH> one(RQ + H * RP, 1, 1);
+  constexpr Places<NM, H * RP + (FA - 1) * RQ, LH> two(H * RP, RQ, H);
+  auto step = [&](int left, const char* __restrict__ cur, const char* __restrict__ nxt, char* __restrict__ before) __attribute__((always_inline)) {
 #pragma unroll
-    for (int i = 0; i < NM; ++i) {
+    for (int n = 0; n < NM; ++n) {
+      mac<ACC>(acc[n / H][n % H], fx[n / H].all(), fy[n % H].all());
 #pragma unroll
-      for (int r = i * PER / NM; r < (i + 1) * PER / NM; ++r) read(cur, 1, r, fx[1], fy[1]);
-      if (i == NM / 2 - 1) yt = P.step(row);
-      if (i == NM / 2) xt = Q.step(row);
-      acc[i / FB][i % FB] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fx[0][i / FB], fy[0][i % FB], acc[i / FB][i % FB], 0, 0, 0);
+      for (int r = 0; r < RQ + H * RP; ++r)
+        if (one.read[r] == n) {
+          if (r < RQ) read_x(cur, FA - 1, r);
+          else read_y(cur, H + (r - RQ) / RP, (r - RQ) % RP);
+        }
+#pragma unroll
+      for (int l = 0; l < LH; ++l)
+        if (one.load[l] == n) bring(before, LH + l, yt, xt);
+      if (n == (one.load[LH - 1] > NM - 2 ? one.load[LH - 1] : NM - 2)) yt = P.step(left - STEPS);   // behind the last load that takes it
       __builtin_amdgcn_sched_barrier(0);
     }
-    arrived_but<(STEPS - 3) * PER>();
+    arrived_but<(STEPS - 2) * PER>();
 #pragma unroll
-    for (int i = 0; i < NM; ++i) {
+    for (int n = 0; n < NM; ++n) {
+      mac<ACC>(acc[n / H][H + n % H], fx[n / H].all(), fy[H + n % H].all());
 #pragma unroll
-      for (int r = i * PER / NM; r < (i + 1) * PER / NM; ++r) {
-        read(nxt, 0, r, fx[0], fy[0]);
-        bring(s, to, r, yt, xt);
-      }
-      acc[i / FB][i % FB] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fx[1][i / FB], fy[1][i % FB], acc[i / FB][i % FB], 0, 0, 0);
+      for (int r = 0; r < H * RP + (FA - 1) * RQ; ++r)
+        if (two.read[r] == n) {
+          if (r < H * RP) read_y(nxt, r / RP, r % RP);
+          else read_x(nxt, (r - H * RP) / RQ, (r - H * RP) % RQ);
+        }
+#pragma unroll
+      for (int l = 0; l < LH; ++l)
+        if (two.load[l] == n) bring(const_cast<char*>(cur), l, yt, xt);
+      if (n == NM - 2) xt = Q.step(left - STEPS);
       __builtin_amdgcn_sched_barrier(0);
     }
   };
-  int at = 0;   // the step's place in the ring
-  for (int s = 0; s < steps; ++s) {
-    const int next = at + SB == STEPS * SB ? 0 : at + SB, last = at == 0 ? (STEPS - 1) * SB : at - SB;
-    step(s, smem + at, smem + next, smem + last);
-    at = next;
+  if (ACC) settled(acc);
+  auto turn = [&](int left, int at) __attribute__((always_inline)) {
+    step(left, smem + at * SB, smem + (at + 1) % STEPS * SB, smem + (at + STEPS - 1) % STEPS * SB);
+  };
+  for (int left = steps; left > 0;) {   // around the ring
+#pragma unroll
+    for (int at = 0; at < STEPS; ++at) {
+      turn(left, at);
+      if (--left == 0) break;
+    }
   }
+  if (ACC) settled(acc);
 
   loads_done();   // what is still on its way has no bytes
 #pragma unroll
-  for (int ib = 0; ib < FB; ++ib) {
-    const int ml = (wm * FB + ib) * 32 + ln, m = m0 + ml;
-    const int nl = wn * FA * 32 + 4 * half;
+  for (int j = 0; j < FB; ++j) {
+    const int ml = (wm * FB + j) * 16 + ln, m = m0 + ml;
+    const int nl = wn * FA * 16 + 4 * quarter;
     if (part >= 0) {
       float* p = a.ws + ((long)(tile - a.full) * a.parts + part) * TM * TN + ml * TN + nl;
 #pragma unroll
-      for (int i = 0; i < FA * 4; ++i) *reinterpret_cast<float4v*>(p + i * 8) = sums(acc[i / 4][ib], i % 4);
+      for (int i = 0; i < FA; ++i) *reinterpret_cast<float4v*>(p + i * 16) = acc[i][j];
       continue;
     }
     if (m >= a.M) continue;
     const long at_out = (long)m * a.N + n0 + nl;
     const int left = a.N - n0 - nl;
-    float4v add[FA * 4];   // read together: the result may lie in the same place
+    float4v add[FA];   // read together: the result may lie in the same place
 #pragma unroll
-    for (int i = 0; i < FA * 4; ++i) add[i] = a.add && i * 8 < left ? *reinterpret_cast<const float4v*>(a.add + at_out + i * 8) : float4v{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int i = 0; i < FA; ++i) add[i] = a.add && i * 16 < left ? *reinterpret_cast<const float4v*>(a.add + at_out + i * 16) : float4v{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-    for (int i = 0; i < FA * 4; ++i)
-      if (i * 8 < left) put(a, at_out + i * 8, sums(acc[i / 4][ib], i % 4) + add[i]);
+    for (int i = 0; i < FA; ++i)
+      if (i * 16 < left) put(a, at_out + i * 16, acc[i][j] + add[i]);
   }
 }
 
@@ -278,17 +357,18 @@ struct Plan {
   double us;
 };
 
-// Tile size and parts by the time that they should take. A round of blocks over the 256 CUs takes a step in 0.76 us with 256 x 256 tiles
-// (1.41 PFLOP/s) and in 0.25 us with 128 x 128 ones (1.07; two blocks share a CU, each then at half the speed), 14 and 5 us
-// around its steps (the first loads, the stores); what is left after whole rounds of tiles may be cut into parts of at least 256
-// contracted indices, whose sums travel at about 5 TB/s both ways and take another launch. Tiles of 256 x 128 take 0.36 us and 9 around them as long as one round
-// is all; over several the clock falls, and they are no better than 128 x 128. A change has to promise 2 %. Measured, weight
-// gradients, 256 x 256 whole / cut, 256 x 128 cut, 128 x 128 whole / cut, us: 22016 x 4096 x 16384: 2370 / 2214, 2731, -;
-// 4096 x 11008 x 16384: 1132 / 1181, -, 1927 / 1656; 4096 x 768 x 8192: 140 / 63, 61, 69 / 66; 768 x 2048 x 8192: 146 / 44, 38, 68 / 39;
-// 768 x 768 x 8192: 138 / 31, 25, 62 / 22; 512 x 512 x 512: 19 / 18, 14, 8.3 / 10.5.
+// Tile size and parts by the time that they should take. A round of blocks over the 256 CUs takes a step in 0.705 us with 256 x 256 tiles
+// (1.52 PFLOP/s), in 0.40 us with 256 x 128 and in 0.27 us with 128 x 128 ones (0.21 where the operands come from near; two blocks share a CU, each
+// then at half the speed), and 16, 11 and 6 us around its steps (the first loads, the stores); what is left after whole rounds of tiles may be cut into
+// parts of at least 256 contracted indices, whose sums travel at about 10 TB/s both ways and take another launch. Tiles of 256 x 128 pay as long as
+// one round is all; over several they are no better than 128 x 128. A change has to promise 2 %. Measured, weight gradients, 256 x 256 whole / cut,
+// 256 x 128 cut, 128 x 128 whole / cut, us, operands from memory: 4096 x 768 x 8192: 174 / 66, 84, 91 / 86; 2304 x 768 x 8192: 167 / 52, 50, 84 / 56;
+// 768 x 2048 x 8192: 161 / 46, 43, 83 / 50; 768 x 768 x 8192: 161 / 35, 28, 78 / 26; 32000 x 768 x 8184: 377 / 342, 410 (whole), 498; 3072 x 1024 x
+// 2048: 60 / 37, 32, 28 / 33; 6144 x 2048 x 4096: 106 / 127, 130 (whole), 121 / 133; and the same product over and over: 22016 x 4096 x 16384:
+// 2174 / 2056, 2746, 3237; 4096 x 11008 x 16384: 1050 / 1105, 1217 (whole), 1969 / 1708.
 Plan plan(long M, long N, long K, bool small_only) {
   struct { int tm, tn; double step, around; long slots; bool one_round; } forms[] = {
-      {256, 256, 0.76, 14.0, 256, false}, {256, 128, 0.36, 9.0, 256, true}, {128, 128, 0.25, 5.0, 512, false}};
+      {256, 256, 0.705, 16.0, 256, false}, {256, 128, 0.40, 11.0, 256, true}, {128, 128, 0.27, 6.0, 512, false}};
   Plan best{0, 0, 0, 1, 0.0};
   for (const auto& form : forms) {
     if (small_only && form.tm != 128) continue;
@@ -301,7 +381,7 @@ Plan plan(long M, long N, long K, bool small_only) {
     take(tiles, 1, round(tiles, steps));
     const long full = tiles / form.slots * form.slots, rest = tiles - full;
     for (long p = 2; rest && p * rest <= (form.one_round ? 256 : 512) && p * 8 <= steps; ++p)
-      take(full, p, round(full, steps) + round(rest * p, (steps + p - 1) / p) + 3.0 + rest * p * form.tm * form.tn * 8 / 5e6);
+      take(full, p, round(full, steps) + round(rest * p, (steps + p - 1) / p) + 3.0 + rest * p * form.tm * form.tn * 8 / 10e6);
   }
   return best;
 }
@@ -391,7 +471,7 @@ at::Tensor weight_grad(const at::Tensor& dy, const at::Tensor& x, const c10::opt
                              pr::loadable(x) ? x : x.clone(at::MemoryFormat::Contiguous), plan, add, keep);
 }
 
-// x [M, K] times w [N, K]^T, or with `slow` times w [K, N]. Products that should take at most 14 us are formed here, because the host
+// x [M, K] times w [N, K]^T, or with `slow` times w [K, N]. Products that should take at most 15 us by the plan are formed here, because the host
 // takes 19 to 20 us for the library's call and 9 for this one, and a chain of such products waits for it. On the device they
 // are no faster, 6 to 13 us where the library's kernels take 4 to 11. Steps of two layers, us, library and here: width 512, 512 tokens 1320
 // and 1050 (kernels 490 and 525); 1024, 512 tokens 1130 and 900; where the device is the bound nothing shows: 512, 4096 tokens 1316 and
@@ -402,7 +482,7 @@ at::Tensor multiply(const at::Tensor& x, const at::Tensor& w, bool slow) {
     const long M = x.size(0), N = w.size(slow ? 1 : 0), K = x.size(1);
     if (((M + 127) / 128) * ((N + 127) / 128) <= 256) {
       const pr::Plan plan = pr::plan(M, N, K, true);
-      if (plan.us <= 14.0) return slow ? pr::run<false, true>(x, w, plan, c10::nullopt, false) : pr::run<false, false>(x, w, plan, c10::nullopt, false);
+      if (plan.us <= 15.0) return slow ? pr::run<false, true>(x, w, plan, c10::nullopt, false) : pr::run<false, false>(x, w, plan, c10::nullopt, false);
     }
   }
   return slow ? at::mm(x, w) : at::mm(x, w.t());

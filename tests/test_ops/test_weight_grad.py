@@ -42,6 +42,16 @@ def test_against_64_bits(M, N, K):
     _close(again, dy, x, before, True)
 
 
+# one round of the tiles of 256 x 256 and of 256 x 128, whose ring of four steps is left behind each of them
+@pytest.mark.gpu
+@pytest.mark.parametrize("N", [4088, 2040])
+@pytest.mark.parametrize("K", [1, 33, 65, 97, 129, 160, 192, 223, 256, 261])
+def test_large_tiles_over_few_steps(N, K):
+    torch.manual_seed(N + K)
+    dy, x = (torch.randn(K, n, device="cuda").to(BF16) for n in (4088, N))
+    _close(kernels().weight_grad(dy, x, None, True), dy, x, None, True)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("M,N,K", [(128, 136, 31), (264, 248, 300), (768, 768, 4100), (12, 20, 33)])
 @pytest.mark.parametrize("offset", [1, 2, 3, 5])
