@@ -39,6 +39,9 @@
 //   B4 S4096 H32/8 D128 causal 570 -> 550, B1 S8192 H32/8 514 -> 500, H4 159 -> 128 (half the chip); B8 S1024 H12 D64 32.0 -> 31.2,
 //   packed, 16384 tokens of up to 4096, 32/8 of 128 384 -> 367, 12 of 64 102 -> 95, 8192 of up to 2048, 32/8 113 -> 103;
 //   B1 S4096 H8/2 D64 unmasked 56.9 -> 53.3, but B1 S8192 H12 D64 causal 168 -> 171
+// and with a quarter of its instructions taken out, waits and scalar ones (a step of 64 keys 380 -> 273; they were 25 % of what a SIMD issues), us:
+//   B1 S8192 H4/1 D128 causal 126 -> 116, H12 D64 167 -> 162; B1 S2048 H12 D64 27.1 -> 24.8; B1 S4096 H8/2 D64 54 -> 50; B4 S4096 H32 D128 582 -> 572,
+//   H32/8 at a full chip the same: power. Slower there: products of 16 x 16 x 32 (542 for 532, H4/1 148 for 127: more instructions), 64 rows a wave (610).
 //
 // Shapes: q [B,S,Hq,D], k/v [B,S,Hkv,D] ("bshd" — no transposes in the
 // model), D in {64,128}. lse/delta are [B,Hq,S] fp32.
@@ -141,6 +144,28 @@ struct TileLoad {
 #pragma unroll
     for (int i = 0; i < PER; ++i) piece(t, lds, w, i);
   }
+};
+
+// A matrix' tiles one after the other, through a descriptor that is advanced instead of formed anew (six scalar instructions for some 20).
+template <int D, int ROWS, int WAVES>
+struct TileStream : TileLoad<D, ROWS, WAVES> {
+  typedef TileLoad<D, ROWS, WAVES> Base;
+  const unsigned short* at;    // of the next tile
+  int left, whole, last;       // rows from there on; bytes of a tile, of the last one
+  __amdgpu_buffer_rsrc_t now;
+  DEV_INLINE TileStream(const unsigned short* base, long stride, int rows) : Base(base, stride, rows), at(base), left(rows) {
+    whole = (int)((unsigned)((ROWS - 1) * stride + D) * 2u);
+    last = (int)((unsigned)(((max(rows, 1) - 1) % ROWS) * stride + D) * 2u);
+  }
+  DEV_INLINE void skip(int tiles) {
+    at += tiles * ROWS * Base::stride;
+    left -= tiles * ROWS;
+  }
+  DEV_INLINE void next() {
+    now = __builtin_amdgcn_make_buffer_rsrc(const_cast<unsigned short*>(at), 0, left > ROWS ? whole : left > 0 ? last : 0, 0x00027000);
+    skip(1);
+  }
+  DEV_INLINE void piece(char* __restrict__ lds, int w, int i) const { Base::piece(now, lds, w, i); }
 };
 
 }  // namespace fa
@@ -283,7 +308,7 @@ __global__ __launch_bounds__(NW * 64, 2) void fa_fwd_kernel(
     }
   };
   auto raise = [&](const f32x16& s, float rowsum, Weights& p) __attribute__((always_inline)) {
-    if (!__all(rowsum <= 4096.0f)) {
+    if (__builtin_expect(!__all(rowsum <= 4096.0f), 0)) {
       float rowmax = s[0];
 #pragma unroll
       for (int j = 1; j < 16; ++j) rowmax = fmaxf(rowmax, s[j]);
@@ -311,23 +336,28 @@ __global__ __launch_bounds__(NW * 64, 2) void fa_fwd_kernel(
 
   const RowAt row_at(ln, half);
   const ColAt col_at(lane);
-  const TileLoad<D, KVB, NW> kload(k_base, kts, SeffK), vload(v_base, kts, SeffK);
+  TileStream<D, KVB, NW> kload(k_base, kts, SeffK), vload(v_base, kts, SeffK);
   constexpr int PER = TileLoad<D, KVB, NW>::PER;
 
   // The turn of 32 keys: the scores of the 32 after them into `sn` (keys from row kr of the tile at `K_`), their own weights from `s` into `p`, and what
   // the 32 ahead of them add, weights `pp` times the values from row vr at `V_`; none of these waits for another, and a
   // wave's instructions alternate between them. A product takes the matrix unit 32 cycles and the SIMD's issue 11; whatever else the SIMD's
   // waves issue (4 to 5 cycles, an exponential 8) fits beside it only if it stands between the products.
-  constexpr int GROUPS = DSL > D / 16 ? DSL : D / 16, AHEAD = 2;
+  // Fragments are read a group ahead of the products that take them, with one wait a group (a wait for each was 16 of a turn's 190 instructions).
+  constexpr int NB = D / 32, GROUPS = D / 32;   // a group: two fragments of keys, two of values
   auto turn = [&](auto with_scores, auto with_weights, auto with_values, const char* __restrict__ K_, int kr, const char* __restrict__ V_, int vr,
                   f32x16& sn, const f32x16& s, Weights& p, const Weights& pp, auto load) __attribute__((always_inline)) {
-    constexpr int NB = D / 32;
     bf16x8_t kf[DSL], vf[2 * NB];
     float w[8][2], sum = 0.0f;
-    auto read = [&](int i) __attribute__((always_inline)) {
-      if (with_scores && i < DSL) kf[i] = frag_row<KVB>(K_, row_at, kr, i);
-      if (with_values && i < 2 * NB) vf[i] = frag_born<KVB>(V_, col_at, vr + i / NB * 16, i % NB * 32);
+    auto read = [&](int g) __attribute__((always_inline)) {
+      if (g >= GROUPS) return;
+#pragma unroll
+      for (int i = 2 * g; i < 2 * g + 2; ++i) {
+        if (with_scores) kf[i] = frag_row<KVB>(K_, row_at, kr, i);
+        if (with_values) vf[i] = frag_born<KVB>(V_, col_at, vr + i / NB * 16, i % NB * 32);
+      }
     };
+    constexpr int READS = (decltype(with_scores)::value ? 2 : 0) + (decltype(with_values)::value ? 4 : 0);   // LDS instructions of a group
     constexpr int PRODUCTS = (decltype(with_scores)::value ? DSL : 0) + (decltype(with_values)::value ? 2 * NB : 0);
     auto weigh = [&](int n) __attribute__((always_inline)) {
       if (with_weights) {
@@ -340,23 +370,27 @@ __global__ __launch_bounds__(NW * 64, 2) void fa_fwd_kernel(
 #pragma unroll
       for (int j = 0; j < 16; ++j) sn[j] = 0.0f;
     }
-#pragma unroll
-    for (int i = 0; i < AHEAD; ++i) read(i);
+    read(0);
     __builtin_amdgcn_sched_barrier(0);
     int n = 0;
 #pragma unroll
-    for (int i = 0; i < GROUPS; ++i) {
-      read(i + AHEAD);
-      if (with_scores && i < DSL) {
-        sn = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[i], qf[i], sn, 0, 0, 0);
-        weigh(n++);
-      }
-      if (with_values && i < 2 * NB) {
-        oacc[i % NB] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[i], pp.p[i / NB], oacc[i % NB], 0, 0, 0);
-        weigh(n++);
-      }
-      load(i);
+    for (int g = 0; g < GROUPS; ++g) {
+      read(g + 1);
       __builtin_amdgcn_sched_barrier(0);
+      reads_left<READS>(g + 1 < GROUPS);
+#pragma unroll
+      for (int i = 2 * g; i < 2 * g + 2; ++i) {
+        if (with_scores) {
+          sn = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[i], qf[i], sn, 0, 0, 0);
+          weigh(n++);
+        }
+        if (with_values) {
+          oacc[i % NB] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[i], pp.p[i / NB], oacc[i % NB], 0, 0, 0);
+          weigh(n++);
+        }
+        load(i);
+        __builtin_amdgcn_sched_barrier(0);
+      }
     }
     if (with_weights) {
       // formed here: the compiler moves them to where they are used, behind the products
@@ -377,24 +411,25 @@ __global__ __launch_bounds__(NW * 64, 2) void fa_fwd_kernel(
   loads_left<PER>();
   __syncthreads();
   int t = 0;
-  __amdgpu_buffer_rsrc_t kt, vt;
+  kload.skip(1);
   auto begin = [&]() __attribute__((always_inline)) {
-    kt = kload.tile((t + 1) * KVB);
-    vt = vload.tile(t * KVB);
+    kload.next();
+    vload.next();
   };
   auto end = [&]() __attribute__((always_inline)) {
     loads_done();
     __syncthreads();
     ++t;
   };
-  auto load_keys = [&](int i) __attribute__((always_inline)) {
+  constexpr int PARTS = 2 * GROUPS;   // of the loads of a step, in its first turn
+  auto load_keys = [&](char* __restrict__ K_, int i) __attribute__((always_inline)) {
 #pragma unroll
-    for (int n = i * PER / GROUPS; n < (i + 1) * PER / GROUPS; ++n) kload.piece(kt, Kbuf + (~t & 1) * KB_BYTES, w, n);
+    for (int n = i * PER / PARTS; n < (i + 1) * PER / PARTS; ++n) kload.piece(K_, w, n);
   };
-  auto load = [&](int i) __attribute__((always_inline)) {
-    load_keys(i);
+  auto load = [&](char* __restrict__ K_, char* __restrict__ V_, int i) __attribute__((always_inline)) {
+    load_keys(K_, i);
 #pragma unroll
-    for (int n = i * PER / GROUPS; n < (i + 1) * PER / GROUPS; ++n) vload.piece(vt, Vbuf + (t & 1) * KB_BYTES, w, n);
+    for (int n = i * PER / PARTS; n < (i + 1) * PER / PARTS; ++n) vload.piece(V_, w, n);
   };
   auto nothing = [](int) {};
   if (my_tiles > 0) {
@@ -402,21 +437,28 @@ __global__ __launch_bounds__(NW * 64, 2) void fa_fwd_kernel(
     Weights pe, po;
     {
       begin();
-      turn(yes, no, no, Kbuf, 0, Kbuf, 0, se, so, po, pe, load_keys);   // the first values are on their way
+      turn(yes, no, no, Kbuf, 0, Kbuf, 0, se, so, po, pe, [&](int i) __attribute__((always_inline)) { load_keys(Kbuf + KB_BYTES, i); });   // the first values are on their way
       mask(0, se);
       turn(yes, yes, no, Kbuf, 32, Kbuf, 0, so, se, pe, po, nothing);
       end();
     }
-    while (t < my_tiles) {
+    // step t in buffer t % 2
+    auto step = [&](auto masked, int odd) __attribute__((always_inline)) {
+      char* K_ = Kbuf + odd * KB_BYTES;
+      char* V_ = Vbuf + odd * KB_BYTES;
+      char* Kn = Kbuf + (1 - odd) * KB_BYTES;
+      char* Vn = Vbuf + (1 - odd) * KB_BYTES;   // of the step before
       begin();
-      const char* K_ = Kbuf + (t & 1) * KB_BYTES;
-      const char* V_ = Vbuf + (~t & 1) * KB_BYTES;
-      mask(t * KVB - 32, so);
-      turn(yes, yes, yes, K_, 0, V_, 0, se, so, po, pe, load);
-      mask(t * KVB, se);
-      turn(yes, yes, yes, K_, 32, V_, 32, so, se, pe, po, nothing);
+      if (masked) mask(t * KVB - 32, so);
+      turn(yes, yes, yes, K_, 0, Vn, 0, se, so, po, pe, [&](int i) __attribute__((always_inline)) { load(Kn, V_, i); });
+      if (masked) mask(t * KVB, se);
+      turn(yes, yes, yes, K_, 32, Vn, 32, so, se, pe, po, nothing);
       end();
-    }
+    };
+    // most steps meet no mask: they do not look for one either
+    const int plain = min(my_tiles, min(SeffK >= 32 ? (SeffK + 32) / KVB : 0, causal ? (qw + KVB - 31) / KVB : my_tiles));
+    while (t < plain) step(no, t & 1);
+    while (t < my_tiles) step(yes, t & 1);
     const char* V_ = Vbuf + (~t & 1) * KB_BYTES;
     const int k0 = t * KVB - 32;
     if (k0 < SeffK && !(causal && k0 > qw + QW - 1)) {   // the last half shows something to the wave
@@ -429,10 +471,11 @@ __global__ __launch_bounds__(NW * 64, 2) void fa_fwd_kernel(
   }
   while (t < kv_tiles) {
     begin();
+    char* K_ = Kbuf + (~t & 1) * KB_BYTES;
 #pragma unroll
-    for (int i = 0; i < GROUPS; ++i) {
-      if (t > 0) load(i);
-      else load_keys(i);
+    for (int i = 0; i < PARTS; ++i) {
+      if (t > 0) load(K_, Vbuf + (t & 1) * KB_BYTES, i);
+      else load_keys(K_, i);
     }
     end();
   }

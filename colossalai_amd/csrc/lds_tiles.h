@@ -65,4 +65,12 @@ DEV_INLINE void loads_left() {
   __builtin_amdgcn_sched_barrier(0);
 }
 
+// At most N of this wave's LDS reads (where `ahead`, else none) are on their way.
+template <int N>
+DEV_INLINE void reads_left(bool ahead) {
+  if (ahead) __builtin_amdgcn_s_waitcnt(0xc07f | N << 8);
+  else __builtin_amdgcn_s_waitcnt(0xc07f);
+  __builtin_amdgcn_sched_barrier(0);
+}
+
 }  // namespace cai

@@ -199,6 +199,25 @@ def test_strided_gradients_with_shared_heads():
         _near(a, b, name)
 
 
+@pytest.mark.parametrize("S", [31, 32, 33, 63, 64, 65, 95, 96, 97, 159, 160, 161, 223, 225, 257])
+@pytest.mark.parametrize("D,causal", [(64, True), (128, True), (128, False)])
+def test_where_steps_without_a_mask_end(S, D, causal):
+    """Steps of 64 keys do not look for a mask until the diagonal or the end of the keys is near: odd halves on either side of it,
+    with whole sequences and with padded ones."""
+    from colossalai_amd.ops import flash_attention
+
+    q, k, v, dout = _inputs(2, S, 2, 1, D, S)
+    lens = [S, max(1, S - 33)]
+    for padded in (False, True):
+        a = [t.clone().requires_grad_() for t in (q, k, v)]
+        o = flash_attention(*a, causal=causal, seqlens=torch.tensor(lens, dtype=torch.int32, device="cuda") if padded else None)
+        got = [o] + list(torch.autograd.grad(o, a, dout))
+        for b, n in enumerate(lens if padded else [S, S]):
+            one = [t[b: b + 1, :n] for t in (q, k, v, dout)]
+            for name, x, y in zip(("out", "dq", "dk", "dv"), got, _reference(*one, causal, D ** -0.5)):
+                _near(x[b: b + 1, :n], y, f"{name} {padded} {b}", False)
+
+
 @pytest.mark.parametrize("H", [31, 32, 33])
 @pytest.mark.parametrize("D,causal", [(64, True), (128, False)])
 @pytest.mark.parametrize("packed", [False, True])
