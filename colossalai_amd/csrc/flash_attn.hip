@@ -52,6 +52,7 @@
 #include <ATen/hip/HIPContext.h>
 
 #include <algorithm>
+#include <climits>
 #include <type_traits>
 
 #include "lds_tiles.h"
@@ -160,6 +161,10 @@ struct TileStream : TileLoad<D, ROWS, WAVES> {
   DEV_INLINE void skip(int tiles) {
     at += tiles * ROWS * Base::stride;
     left -= tiles * ROWS;
+  }
+  DEV_INLINE void next(bool all) {
+    now = __builtin_amdgcn_make_buffer_rsrc(const_cast<unsigned short*>(at), 0, all ? whole : last, 0x00027000);
+    at += ROWS * Base::stride;
   }
   DEV_INLINE void next() {
     now = __builtin_amdgcn_make_buffer_rsrc(const_cast<unsigned short*>(at), 0, left > ROWS ? whole : left > 0 ? last : 0, 0x00027000);
@@ -506,11 +511,14 @@ __global__ __launch_bounds__(NW * 64, 2) void fa_fwd_kernel(
   }
 }
 
-// ==================================================== delta = rowsum(dO ⊙ O)
+// ==================================================== what a query row adds in the backward: -lse log2(e) and -rowsum(dO ⊙ O)
+// One beside the other, so that one load of a wave brings those of 32 rows; a row that counts nothing (padding, or no
+// visible key) has an addend of -inf.
 __global__ __launch_bounds__(256) void fa_delta_kernel(
     const unsigned short* __restrict__ dO,
     const unsigned short* __restrict__ Oin,
-    float* __restrict__ delta,  // [B, H, S]
+    const float* __restrict__ LSE,
+    float2v* __restrict__ stats,  // [B, H, S]
     long rows,  // B*S*H
     int S, int H, int D) {
   const int lane = threadIdx.x & 63;
@@ -545,7 +553,9 @@ __global__ __launch_bounds__(256) void fa_delta_kernel(
       const long rem = row % ((long)S * H);
       const long s = rem / H;
       const long hh = rem % H;
-      delta[(bidx * H + hh) * S + s] = acc;
+      const long at = (bidx * H + hh) * S + s;
+      const float lse = LSE[at];
+      stats[at] = float2v{lse == -INFINITY ? -INFINITY : -lse * 1.44269504f, -acc};
     }
   }
 }
@@ -560,6 +570,14 @@ __global__ __launch_bounds__(256) void fa_delta_kernel(
 // over in the registers of a lane (the C layout's rows), so a packed run of eight registers is an
 // operand of the next product as it stands and neither passes through LDS (frag_born reads the other
 // operand's columns in the same order).
+//
+// What bounds it: the SIMDs' issue, 66 % of all cycles at 32 over 8 heads of 128, 8192 tokens, 30 % of that scalar instructions (78 for each 32 x 32
+// scores), and waits for LDS reads right behind them; with the chip full then power (1.7 GHz). So descriptors are advanced, statistics come by one load
+// into LDS, what a wave does not see is a loop of its own, and fragments are read a product pair ahead with one wait for each pair. us, before -> now:
+//   B1 S8192 H32/8 D128 causal 1745 -> 1625, H4/1 362 -> 294, H12 D64 430 -> 394     B4 S4096 H32 D128 1900 -> 1738     B1 S2048 H12 D64 68 -> 53
+//   B2 S4096 H16/8 D128 804 -> 752     B1 S4096 H8/2 D64 144 -> 127     B16 S512 H12 D64 63.5 -> 61     B2 S256 H4 D128 19 -> 16
+//   packed, 16384 tokens of up to 4096, 32/8 of 128 1215 -> 1105, 12 of 64 278 -> 250; of up to 512, 16/4 of 64 145 -> 135
+// Column fragments read ahead of the exponentials: nothing at 128 channels, 64 spill two registers by it in the first part (81 -> 78 us without, B8 S1024 H12).
 
 // A block of 4 waves owns 128 key/value rows, 32 a wave, and streams the query tiles of its group's heads
 // (32 rows, double-buffered). dK and dV stay in registers. What a query row adds (its -lse log2e and
@@ -571,8 +589,7 @@ template <int D, bool VARLEN>
 DEV_INLINE void bwd_dkdv(
     char* smem, int f, int nblocks,
     const unsigned short* __restrict__ Q, const unsigned short* __restrict__ K,
-    const unsigned short* __restrict__ V, const unsigned short* __restrict__ dO,
-    const float* __restrict__ LSE, const float* __restrict__ DELTA,
+    const unsigned short* __restrict__ V, const unsigned short* __restrict__ dO, const float2v* __restrict__ STATS,
     unsigned short* __restrict__ dK, unsigned short* __restrict__ dV, float* __restrict__ PART, int GS,
     const int* __restrict__ CU, const int* __restrict__ CUK,
     long qbs, long qts, long kbs, long kts, long dkbs, long dkts,
@@ -584,8 +601,7 @@ DEV_INLINE void bwd_dkdv(
   char* Vlds = smem;                                     // [128 rows]
   char* Qbuf = smem + tile_bytes<NWB * QW, D>();         // [2] query tiles, [2] dO tiles
   char* dObuf = Qbuf + 2 * TB;
-  float* lse_lds = reinterpret_cast<float*>(dObuf + 2 * TB);  // [2][32] -lse log2e
-  float* dta_lds = lse_lds + 2 * QB;                          // [2][32] -delta
+  char* stats_lds = dObuf + 2 * TB;                      // [2][32 of -lse log2e, 32 of -delta]
 
   const int lane = threadIdx.x & 63;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);   // the same for a wave: what it decides is a scalar branch
@@ -649,41 +665,44 @@ DEV_INLINE void bwd_dkdv(
 
   const RowAt row_at(ln, half);
   const ColAt col_at(lane);
+  const int first = qt_first * QB, last = first + nq * QB;   // query rows of a head, in tiles
+  int f_head = -1;               // head of the block's that is fetched from
+  TileStream<D, QB, NWB> qs(Q, qts, Seff), dos(dO, do_stride, Seff);
+  const float2v* stats = STATS;
+  int stats_whole = QB * 8, stats_last = ((max(Seff, 1) - 1) % QB + 1) * 8;
+  __amdgpu_buffer_rsrc_t stats_now;
+  const unsigned stats_off = ln * 8 + half * 4;
+  // what the loads of the tile behind the one at `qt0` need, and of its rows' statistics; behind the last head's last one they bring zeros
+  auto fetch = [&](int qt0) __attribute__((always_inline)) {
+    bool all = qt0 + 2 * QB < last;
+    if (__builtin_expect(qt0 + QB >= last, 0)) {
+      all = nq > 1;
+      if (++f_head < G) {
+        const int h = hk * group + h_first + f_head;
+        qs.at = (VARLEN ? Q + seq0 * qts + (long)h * D : Q + (long)b * qbs + (long)h * D) + (long)first * qts;
+        dos.at = (VARLEN ? dO + (seq0 * Hq + h) * D : dO + ((long)b * S * Hq + h) * D) + (long)first * do_stride;   // dO packed
+        stats = STATS + (VARLEN ? (long)h * S + seq0 : ((long)b * Hq + h) * S) + first;
+      } else {
+        qs.whole = qs.last = dos.whole = dos.last = stats_whole = stats_last = 0;
+      }
+    }
+    qs.next(all);
+    dos.next(all);
+    stats_now = __builtin_amdgcn_make_buffer_rsrc(const_cast<float2v*>(stats), 0, all ? stats_whole : stats_last, 0x00027000);
+    stats += QB;
+  };
+  auto bring_stats = [&](int buf) __attribute__((always_inline)) {
+    if (w == 0) __builtin_amdgcn_raw_ptr_buffer_load_lds(stats_now, (lds_ptr)(stats_lds + buf * 256), 4, (int)stats_off, 0, 0, 0);
+  };
   typedef TileLoad<D, QB, NWB> Load;
-  float lse_r = 0.0f, dta_r = 0.0f;
-  int f_head = 0, f_tile = 0;    // head of the block's and tile of the head that the next fetch takes
-  __amdgpu_buffer_rsrc_t q_next, do_next;
-  const Load qload(Q, qts, Seff), doload(dO, do_stride, Seff);
-  auto fetch = [&]() {           // what the loads of a step's query tile need, and its rows' statistics
-    const int h = hk * group + h_first + f_head;
-    const int qt0 = (qt_first + f_tile) * QB;
-    if (++f_tile == nq) {
-      f_tile = 0;
-      ++f_head;
-    }
-    q_next = qload.tile(VARLEN ? Q + seq0 * qts + (long)h * D : Q + (long)b * qbs + (long)h * D, qt0);
-    do_next = doload.tile(VARLEN ? dO + (seq0 * Hq + h) * D : dO + ((long)b * S * Hq + h) * D, qt0);  // dO packed
-    if (w == 0) {
-      const int row = qt0 + ln;
-      const long at = (VARLEN ? (long)h * S + seq0 : ((long)b * Hq + h) * S) + min(row, Seff - 1);
-      lse_r = row < Seff ? LSE[at] : -INFINITY;
-      dta_r = DELTA[at];
-    }
-  };
-  auto stash = [&](int buf) {
-    if (w == 0 && half == 0) {
-      lse_lds[buf * QB + ln] = lse_r == -INFINITY ? -INFINITY : -lse_r * 1.44269504f;
-      dta_lds[buf * QB + ln] = -dta_r;
-    }
-  };
   if (steps > 0) {
-    fetch();
+    fetch(last);
 #pragma unroll
     for (int i = 0; i < Load::PER; ++i) {
-      qload.piece(q_next, Qbuf, w, i);
-      doload.piece(do_next, dObuf, w, i);
+      qs.piece(Qbuf, w, i);
+      dos.piece(dObuf, w, i);
     }
-    stash(0);
+    bring_stats(0);
   }
   loads_done();
   __syncthreads();
@@ -691,11 +710,12 @@ DEV_INLINE void bwd_dkdv(
   // A query tile, while the next one arrives in the other buffers.
   auto step = [&](int qt0, int buf, const char* __restrict__ Qlds, const char* __restrict__ dOlds, char* __restrict__ Qn,
                   char* __restrict__ dOn) __attribute__((always_inline)) {
+    const float* stats = reinterpret_cast<const float*>(stats_lds + buf * 256) + 4 * half;
     // ---- S[q][kv] = Q · K^T and dP[q][kv] - delta[q] = dO · V^T - delta: column = kv (ln), row = q
     f32x16 s, dp;
 #pragma unroll
     for (int a = 0; a < 4; ++a) {
-      const float4v d4 = *reinterpret_cast<const float4v*>(dta_lds + buf * QB + 8 * a + 4 * half);
+      const float4v d4 = *reinterpret_cast<const float4v*>(stats + QB + 8 * a);
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         dp[4 * a + e] = d4[e];
@@ -703,22 +723,38 @@ DEV_INLINE void bwd_dkdv(
       }
     }
     __builtin_amdgcn_s_setprio(1);
+    bf16x8_t qr[DSL], dor[DSL], vr[DSL], doc[2 * NB], qc[2 * NB];   // fragments, read ahead of their products with one wait for each pair of these
+    auto rows = [&](int i) __attribute__((always_inline)) {
+      if (i >= DSL) return;
+      qr[i] = frag_row<QB>(Qlds, row_at, 0, i);
+      dor[i] = frag_row<QB>(dOlds, row_at, 0, i);
+      vr[i] = frag_row<NWB * QW>(Vlds + w * 2048, row_at, 0, i);
+    };
+    auto columns = [&](int i) __attribute__((always_inline)) {
+      if (i >= 2 * NB) return;
+      doc[i] = frag_born<QB>(dOlds, col_at, i / NB * 16, i % NB * 32);
+      qc[i] = frag_born<QB>(Qlds, col_at, i / NB * 16, i % NB * 32);
+    };
+    rows(0);
 #pragma unroll
     for (int sl = 0; sl < DSL; ++sl) {
-      s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(frag_row<QB>(Qlds, row_at, 0, sl), kf[sl], s, 0, 0, 0);
-      dp = __builtin_amdgcn_mfma_f32_32x32x16_bf16(frag_row<QB>(dOlds, row_at, 0, sl),
-                                                   frag_row<NWB * QW>(Vlds + w * 2048, row_at, 0, sl), dp, 0, 0, 0);
+      rows(sl + 1);
+      __builtin_amdgcn_sched_barrier(0);
+      reads_left<3>(sl + 1 < DSL);
+      s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(qr[sl], kf[sl], s, 0, 0, 0);
+      dp = __builtin_amdgcn_mfma_f32_32x32x16_bf16(dor[sl], vr[sl], dp, 0, 0, 0);
 #pragma unroll
-      for (int i = sl * Load::PER / DSL; i < (sl + 1) * Load::PER / DSL; ++i) qload.piece(q_next, Qn, w, i);
+      for (int i = sl * Load::PER / DSL; i < (sl + 1) * Load::PER / DSL; ++i) qs.piece(Qn, w, i);
     }
     __builtin_amdgcn_s_setprio(0);
+    if (D == 128) columns(0);   // ahead of the exponentials; 64 channels have no registers for them there
     // ---- P = exp(scale s - lse); dS = P (dP - delta), its scale waits for the epilogue
     bf16x8_t pa[2], dsa[2];
     const int before = kvw + ln - qt0 - 4 * half;   // rows of the tile ahead of this key
     auto grads = [&](auto diagonal) __attribute__((always_inline)) {
 #pragma unroll
       for (int a = 0; a < 4; ++a) {   // read here, the statistics take 4 registers and not 16 over the products
-        const float4v l4 = *reinterpret_cast<const float4v*>(lse_lds + buf * QB + 8 * a + 4 * half);
+        const float4v l4 = *reinterpret_cast<const float4v*>(stats + 8 * a);
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           const int j = 4 * a + e;
@@ -730,46 +766,58 @@ DEV_INLINE void bwd_dkdv(
       }
     };
     // two bodies: merged into one, every tile would pay for the mask of the few on the diagonal
-    if (causal && kvw + QW - 1 > qt0) {
+    if (causal && qt0 < kvw + QW - 1) {
       grads(std::true_type());
       asm volatile("" ::: "memory");
     } else {
       grads(std::false_type());
     }
     // ---- dV += P^T · dO, dK += dS^T · Q (A: lane row = kv; B: columns of the tiles)
+    if (D != 128) columns(0);
     __builtin_amdgcn_s_setprio(1);
 #pragma unroll
-    for (int s2 = 0; s2 < 2; ++s2)
+    for (int at = 0; at < 2 * NB; ++at) {
+      columns(at + 1);
+      __builtin_amdgcn_sched_barrier(0);
+      reads_left<4>(at + 1 < 2 * NB);
+      dv_acc[at % NB] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(pa[at / NB], doc[at], dv_acc[at % NB], 0, 0, 0);
+      dk_acc[at % NB] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(dsa[at / NB], qc[at], dk_acc[at % NB], 0, 0, 0);
 #pragma unroll
-      for (int nb = 0; nb < NB; ++nb) {
-        dv_acc[nb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(pa[s2], frag_born<QB>(dOlds, col_at, s2 * 16, nb * 32), dv_acc[nb], 0, 0, 0);
-        dk_acc[nb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(dsa[s2], frag_born<QB>(Qlds, col_at, s2 * 16, nb * 32), dk_acc[nb], 0, 0, 0);
-        const int at = s2 * NB + nb;
-#pragma unroll
-        for (int i = at * Load::PER / (2 * NB); i < (at + 1) * Load::PER / (2 * NB); ++i) doload.piece(do_next, dOn, w, i);
-      }
+      for (int i = at * Load::PER / (2 * NB); i < (at + 1) * Load::PER / (2 * NB); ++i) dos.piece(dOn, w, i);
+    }
     __builtin_amdgcn_s_setprio(0);
   };
-  for (int n = 0, c_tile = 0; n < steps; ++n) {
-    const int buf = n & 1;
-    const int qt0 = (qt_first + c_tile) * QB;
-    if (++c_tile == nq) c_tile = 0;
-    const bool more = n + 1 < steps;
-    if (more) fetch();
-    char* Qn = Qbuf + (buf ^ 1) * TB;
-    char* dOn = dObuf + (buf ^ 1) * TB;
-    if (!(causal && qt0 + QB - 1 < kvw) && kvw < SeffK) {
-      step(qt0, buf, Qbuf + buf * TB, dObuf + buf * TB, Qn, dOn);   // after the last step the loads repeat its tile
-    } else {
-#pragma unroll
-      for (int i = 0; i < Load::PER; ++i) {
-        qload.piece(q_next, Qn, w, i);
-        doload.piece(do_next, dOn, w, i);
-      }
-    }
-    if (more) stash(buf ^ 1);
+  // A head's first tiles show some waves nothing: they only bring the next one's rows, in a loop of its own, ahead of which the sums stay in their registers.
+  int buf = 0;
+  char *Qn, *dOn;
+  auto begin = [&](int qt0) __attribute__((always_inline)) {
+    fetch(qt0);
+    Qn = Qbuf + (buf ^ 1) * TB;
+    dOn = dObuf + (buf ^ 1) * TB;
+    bring_stats(buf ^ 1);
+  };
+  auto finish = [&]() __attribute__((always_inline)) {
+    buf ^= 1;
     loads_done();
     __syncthreads();
+  };
+  const int from = kvw >= SeffK ? last : causal ? min(kvw, last) : 0;
+  for (int head = 0; head < (steps > 0 ? G : 0); ++head) {
+    int qt0 = first;
+    for (; qt0 < from; qt0 += QB) {
+      begin(qt0);
+#pragma unroll
+      for (int i = 0; i < Load::PER; ++i) {
+        qs.piece(Qn, w, i);
+        dos.piece(dOn, w, i);
+      }
+      finish();
+    }
+    for (; qt0 < last; qt0 += QB) {
+      begin(qt0);
+      step(qt0, buf, Qbuf + buf * TB, dObuf + buf * TB, Qn, dOn);
+      finish();
+    }
   }
 
   // ---- epilogue: dK, dV of the rows of this tile. Padded rows get zeros.
@@ -806,7 +854,7 @@ DEV_INLINE void bwd_dq(
     char* smem, int f, int nblocks,
     const unsigned short* __restrict__ Q, const unsigned short* __restrict__ K,
     const unsigned short* __restrict__ V, const unsigned short* __restrict__ dO,
-    const float* __restrict__ LSE, const float* __restrict__ DELTA, unsigned short* __restrict__ dQ,
+    const float2v* __restrict__ STATS, unsigned short* __restrict__ dQ,
     const int* __restrict__ CU, const int* __restrict__ CUK,
     long qbs, long qts, long kbs, long kts, long dqbs, long dqts,
     int tiles, int B, int S, int Sk, int Hq, int Hkv, float scale, int causal) {
@@ -867,11 +915,9 @@ DEV_INLINE void bwd_dq(
       dof[sl] = ld_g16(dop + sl * 16);
     }
   }
-  // a row that counts nothing (padding, or no visible key) has an addend of -inf
   const long stat = (VARLEN ? (long)h * S + seq0 : ((long)b * Hq + h) * S) + q_my;
-  const float lse = qw + ln < Seff ? LSE[stat] : -INFINITY;
-  const float addend = lse == -INFINITY ? -INFINITY : -lse * 1.44269504f;
-  const float ndelta = -DELTA[stat];
+  const float2v own = STATS[stat];
+  const float addend = qw + ln < Seff ? own[0] : -INFINITY, ndelta = own[1];
   const float scale2 = scale * 1.44269504f;
 
   f32x16 dq_acc[NB];
@@ -887,18 +933,24 @@ DEV_INLINE void bwd_dq(
   const RowAt row_at(ln, half);
   const ColAt col_at(lane);
   typedef TileLoad<D, KVB, NWB> Load;
-  const Load kload(k_base, kts, SeffK), vload(v_base, kts, SeffK);
+  TileStream<D, KVB, NWB> kload(k_base, kts, SeffK), vload(v_base, kts, SeffK);
   if (kv_tiles > 0) {
     kload.all(0, Kbuf, w);
     vload.all(0, Vbuf, w);
+    kload.skip(1);
+    vload.skip(1);
   }
+  // keys from which on a wave's rows do not see all of 32, tiles of which they see something
+  const int edge = min(SeffK - 31, causal ? qw - 30 : INT_MAX);
+  const int my_tiles = qw >= Seff ? 0 : causal ? min(kv_tiles, (qw + QW - 1) / KVB + 1) : kv_tiles;
   loads_done();
   __syncthreads();
 
   // A key/value tile, while the next one arrives in the other buffers (past the last key: zeros, without a read).
   auto step = [&](int k0, const char* __restrict__ Klds, const char* __restrict__ Vlds, char* __restrict__ Kn,
                   char* __restrict__ Vn) __attribute__((always_inline)) {
-    const auto kt = kload.tile(k0 + KVB), vt = vload.tile(k0 + KVB);
+    kload.next();
+    vload.next();
 #pragma unroll
     for (int kb = 0; kb < KVB / 32; ++kb) {
       // ---- S^T[kv][q] = K · Q^T and dP^T - delta = V · dO^T - delta: column = q (ln), row = kv
@@ -906,18 +958,34 @@ DEV_INLINE void bwd_dq(
 #pragma unroll
       for (int j = 0; j < 16; ++j) { s[j] = 0.0f; dp[j] = ndelta; }
       __builtin_amdgcn_s_setprio(1);
+      bf16x8_t kr[DSL], vr[DSL], kc[2 * NB];
+      auto rows = [&](int i) __attribute__((always_inline)) {
+        if (i >= DSL) return;
+        kr[i] = frag_row<KVB>(Klds, row_at, kb * 32, i);
+        vr[i] = frag_row<KVB>(Vlds, row_at, kb * 32, i);
+      };
+      auto columns = [&](int g) __attribute__((always_inline)) {   // two fragments
+        if (g >= NB) return;
+#pragma unroll
+        for (int i = 2 * g; i < 2 * g + 2; ++i) kc[i] = frag_born<KVB>(Klds, col_at, kb * 32 + i / NB * 16, i % NB * 32);
+      };
+      rows(0);
 #pragma unroll
       for (int sl = 0; sl < DSL; ++sl) {
-        s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(frag_row<KVB>(Klds, row_at, kb * 32, sl), qf[sl], s, 0, 0, 0);
-        dp = __builtin_amdgcn_mfma_f32_32x32x16_bf16(frag_row<KVB>(Vlds, row_at, kb * 32, sl), dof[sl], dp, 0, 0, 0);
+        rows(sl + 1);
+        __builtin_amdgcn_sched_barrier(0);
+        reads_left<2>(sl + 1 < DSL);
+        s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kr[sl], qf[sl], s, 0, 0, 0);
+        dp = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vr[sl], dof[sl], dp, 0, 0, 0);
         const int at = kb * DSL + sl;
 #pragma unroll
         for (int i = at * Load::PER / (2 * DSL); i < (at + 1) * Load::PER / (2 * DSL); ++i) {
-          kload.piece(kt, Kn, w, i);
-          vload.piece(vt, Vn, w, i);
+          kload.piece(Kn, w, i);
+          vload.piece(Vn, w, i);
         }
       }
       __builtin_amdgcn_s_setprio(0);
+      columns(0);
       // ---- dS = exp(scale s - lse) (dP - delta), its scale waits for the epilogue
       bf16x8_t dsa[2];
       const int kb0 = k0 + kb * 32, upto = last_key - kb0 - 4 * half;
@@ -929,7 +997,7 @@ DEV_INLINE void bwd_dq(
           dsa[j >> 3][j & 7] = (__bf16)(pv * dp[j]);
         }
       };
-      if (kb0 + 32 > SeffK || (causal && kb0 + 31 > qw)) {
+      if (kb0 >= edge) {
         grads(std::true_type());
         asm volatile("" ::: "memory");
       } else {
@@ -938,10 +1006,14 @@ DEV_INLINE void bwd_dq(
       // ---- dQ += dS · K (A: lane row = q; B: columns of K)
       __builtin_amdgcn_s_setprio(1);
 #pragma unroll
-      for (int s2 = 0; s2 < 2; ++s2)
+      for (int g = 0; g < NB; ++g) {
+        columns(g + 1);
+        __builtin_amdgcn_sched_barrier(0);
+        reads_left<4>(g + 1 < NB);
 #pragma unroll
-        for (int nb = 0; nb < NB; ++nb)
-          dq_acc[nb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(dsa[s2], frag_born<KVB>(Klds, col_at, kb * 32 + s2 * 16, nb * 32), dq_acc[nb], 0, 0, 0);
+        for (int i = 2 * g; i < 2 * g + 2; ++i)
+          dq_acc[i % NB] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(dsa[i / NB], kc[i], dq_acc[i % NB], 0, 0, 0);
+      }
       __builtin_amdgcn_s_setprio(0);
     }
   };
@@ -949,11 +1021,16 @@ DEV_INLINE void bwd_dq(
     const int k0 = t * KVB, buf = t & 1;
     char* Kn = Kbuf + (buf ^ 1) * TB;
     char* Vn = Vbuf + (buf ^ 1) * TB;
-    if (!(causal && k0 > qw + QW - 1) && qw < Seff) {
+    if (t < my_tiles) {
       step(k0, Kbuf + buf * TB, Vbuf + buf * TB, Kn, Vn);
     } else {
-      kload.all(k0 + KVB, Kn, w);
-      vload.all(k0 + KVB, Vn, w);
+      kload.next();
+      vload.next();
+#pragma unroll
+      for (int i = 0; i < Load::PER; ++i) {
+        kload.piece(Kn, w, i);
+        vload.piece(Vn, w, i);
+      }
     }
     loads_done();
     __syncthreads();
@@ -984,7 +1061,7 @@ template <int D, bool VARLEN>
 __global__ __launch_bounds__(fa::NTB, D == 64 ? 3 : 2) void fa_bwd_kernel(
     const unsigned short* __restrict__ Q, const unsigned short* __restrict__ K,
     const unsigned short* __restrict__ V, const unsigned short* __restrict__ dO,
-    const float* __restrict__ LSE, const float* __restrict__ DELTA,
+    const float2v* __restrict__ STATS,
     unsigned short* __restrict__ dQ, unsigned short* __restrict__ dK, unsigned short* __restrict__ dV,
     float* __restrict__ PART, int GS, const int* __restrict__ CU, const int* __restrict__ CUK,
     long qbs, long qts, long kbs, long kts, long dqbs, long dqts, long dkbs, long dkts,
@@ -993,10 +1070,10 @@ __global__ __launch_bounds__(fa::NTB, D == 64 ? 3 : 2) void fa_bwd_kernel(
   const int f = (int)(blockIdx.y * gridDim.x + blockIdx.x);   // more than one grid row only beyond 2^23 blocks
   if (f >= n_kv + n_q) return;
   if (f < n_kv)
-    bwd_dkdv<D, VARLEN>(smem, f, n_kv, Q, K, V, dO, LSE, DELTA, dK, dV, PART, GS, CU, CUK, qbs, qts, kbs, kts, dkbs, dkts,
+    bwd_dkdv<D, VARLEN>(smem, f, n_kv, Q, K, V, dO, STATS, dK, dV, PART, GS, CU, CUK, qbs, qts, kbs, kts, dkbs, dkts,
                         kv_tiles, B, S, Sk, Hq, Hkv, scale, causal);
   else
-    bwd_dq<D, VARLEN>(smem, f - n_kv, n_q, Q, K, V, dO, LSE, DELTA, dQ, CU, CUK, qbs, qts, kbs, kts,
+    bwd_dq<D, VARLEN>(smem, f - n_kv, n_q, Q, K, V, dO, STATS, dQ, CU, CUK, qbs, qts, kbs, kts,
                       dqbs, dqts, q_tiles, B, S, Sk, Hq, Hkv, scale, causal);
 }
 
@@ -1173,8 +1250,8 @@ namespace {
 // The backward launch of dense (VARLEN = false) and packed batches. `seqs` sequences of at most S_max queries and
 // Sk_max keys; S, Sk are the extents the kernels index with (tokens of the whole batch when packed).
 template <int D, bool VARLEN>
-void launch_bwd(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, const at::Tensor& dout, const at::Tensor& lse,
-                const at::Tensor& delta, at::Tensor& dq, at::Tensor& dk, at::Tensor& dv, const int* cu, const int* cuk,
+void launch_bwd(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, const at::Tensor& dout, const at::Tensor& stats,
+                at::Tensor& dq, at::Tensor& dk, at::Tensor& dv, const int* cu, const int* cuk,
                 long qbs, long qts, long kbs, long kts, long dqbs, long dqts, long dkbs, long dkts, int seqs, int S_max,
                 int Sk_max, int S, int Sk, int Hq, int Hkv, float scale, bool causal, hipStream_t stream) {
   using namespace fa;
@@ -1211,8 +1288,8 @@ void launch_bwd(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, c
   set_lds_limit((const void*)kernel, bwd_lds<D>());
   hipLaunchKernelGGL(kernel, dim3((unsigned)width, (unsigned)((blocks + width - 1) / width)), dim3(NTB), bwd_lds<D>(), stream,
                      (const unsigned short*)q.data_ptr(), (const unsigned short*)k.data_ptr(),
-                     (const unsigned short*)v.data_ptr(), (const unsigned short*)dout.data_ptr(), lse.data_ptr<float>(),
-                     delta.data_ptr<float>(), (unsigned short*)dq.data_ptr(), (unsigned short*)dk.data_ptr(),
+                     (const unsigned short*)v.data_ptr(), (const unsigned short*)dout.data_ptr(),
+                     (const float2v*)stats.data_ptr(), (unsigned short*)dq.data_ptr(), (unsigned short*)dk.data_ptr(),
                      (unsigned short*)dv.data_ptr(), gs > 1 ? part.data_ptr<float>() : nullptr, gs, cu, cuk, qbs, qts, kbs,
                      kts, dqbs, dqts, dkbs, dkts, (int)n_kv, (int)n_q, kv_tiles, q_tiles, seqs, S, Sk, Hq, Hkv, scale, causal ? 1 : 0);
   HIP_CHECK_LAST();
@@ -1263,20 +1340,20 @@ std::vector<at::Tensor> flash_attn_bwd(at::Tensor dout, at::Tensor q, at::Tensor
   check_fa_view(dq, "dq");
   check_fa_view(dk, "dk");
   TORCH_CHECK(dk.strides() == dv.strides(), "flash_attn_bwd: dk/dv strides must match");
-  auto delta = at::empty({B, Hq, S}, q.options().dtype(at::kFloat));
+  auto stats = at::empty({B, Hq, S, 2}, q.options().dtype(at::kFloat));
   auto stream = at::hip::getCurrentHIPStream();
 
-  {  // delta preprocess (pad rows of O are zero -> delta 0)
+  {  // what the rows add (pad rows of O are zero -> delta 0)
     const long rows = (long)B * S * Hq;
     const int grid = capped_grid((rows + 15) / 16, 4096);
     hipLaunchKernelGGL(fa_delta_kernel, dim3(grid), dim3(256), 0, stream.stream(),
                        (const unsigned short*)dout.data_ptr(), (const unsigned short*)out.data_ptr(),
-                       delta.data_ptr<float>(), rows, S, Hq, D);
+                       lse.data_ptr<float>(), (float2v*)stats.data_ptr(), rows, S, Hq, D);
     HIP_CHECK_LAST();
   }
 
 #define LAUNCH_BWD(DD)                                                                                               \
-  launch_bwd<DD, false>(q, k, v, dout, lse, delta, dq, dk, dv, cu, cuk, q.stride(0), q.stride(1), k.stride(0), k.stride(1), \
+  launch_bwd<DD, false>(q, k, v, dout, stats, dq, dk, dv, cu, cuk, q.stride(0), q.stride(1), k.stride(0), k.stride(1), \
                         dq.stride(0), dq.stride(1), dk.stride(0), dk.stride(1), B, S, Sk, S, Sk, Hq, Hkv, (float)scale,      \
                         causal, stream.stream())
   if (D == 128) LAUNCH_BWD(128);
@@ -1300,20 +1377,20 @@ std::vector<at::Tensor> flash_attn_varlen_bwd(at::Tensor dout, at::Tensor q, at:
   auto dq = at::empty({T, Hq, D}, q.options());
   auto dk = at::empty({T, Hkv, D}, k.options());
   auto dv = at::empty({T, Hkv, D}, v.options());
-  auto delta = at::empty({Hq, T}, q.options().dtype(at::kFloat));
+  auto stats = at::empty({Hq, T, 2}, q.options().dtype(at::kFloat));
   auto stream = at::hip::getCurrentHIPStream();
 
-  {  // delta preprocess over packed rows ([1, Hq, T] layout == [Hq, T])
+  {  // what the rows add ([1, Hq, T] layout == [Hq, T])
     const long rows = (long)T * Hq;
     const int grid = capped_grid((rows + 15) / 16, 4096);
     hipLaunchKernelGGL(fa_delta_kernel, dim3(grid), dim3(256), 0, stream.stream(),
                        (const unsigned short*)dout.data_ptr(), (const unsigned short*)out.data_ptr(),
-                       delta.data_ptr<float>(), rows, T, Hq, D);
+                       lse.data_ptr<float>(), (float2v*)stats.data_ptr(), rows, T, Hq, D);
     HIP_CHECK_LAST();
   }
 
 #define LAUNCH_VBWD(DD)                                                                                              \
-  launch_bwd<DD, true>(q, k, v, dout, lse, delta, dq, dk, dv, cu_seqlens.data_ptr<int>(), nullptr, 0L, q.stride(0), 0L,     \
+  launch_bwd<DD, true>(q, k, v, dout, stats, dq, dk, dv, cu_seqlens.data_ptr<int>(), nullptr, 0L, q.stride(0), 0L,     \
                        k.stride(0), 0L, dq.stride(0), 0L, dk.stride(0), n_seq, (int)max_seqlen, (int)max_seqlen, T, T, Hq,  \
                        Hkv, (float)scale, causal, stream.stream())
   if (D == 128) LAUNCH_VBWD(128);

@@ -207,7 +207,7 @@ def test_where_steps_without_a_mask_end(S, D, causal):
     from colossalai_amd.ops import flash_attention
 
     q, k, v, dout = _inputs(2, S, 2, 1, D, S)
-    lens = [S, max(1, S - 33)]
+    lens = [S, S - 17]
     for padded in (False, True):
         a = [t.clone().requires_grad_() for t in (q, k, v)]
         o = flash_attention(*a, causal=causal, seqlens=torch.tensor(lens, dtype=torch.int32, device="cuda") if padded else None)
@@ -215,7 +215,7 @@ def test_where_steps_without_a_mask_end(S, D, causal):
         for b, n in enumerate(lens if padded else [S, S]):
             one = [t[b: b + 1, :n] for t in (q, k, v, dout)]
             for name, x, y in zip(("out", "dq", "dk", "dv"), got, _reference(*one, causal, D ** -0.5)):
-                _near(x[b: b + 1, :n], y, f"{name} {padded} {b}", False)
+                _near(x[b: b + 1, :n], y, f"{name} {padded} {b}")
 
 
 @pytest.mark.parametrize("H", [31, 32, 33])
