@@ -317,6 +317,9 @@ __global__ __launch_bounds__(64 * ATT_WAVES) void paged_attention_kernel(
 // cap 71 -> 54 (lanes past a sequence's last token repeat it, and its tiles need no masks for them); 3 x 200 after 1500 54 -> 42; 14
 // decode tokens beside portions of 1000 and 963, window 1024: 58 -> 53. A lone prompt of 40 or 100 tokens has one turn more in its chain, 11.1 -> 11.3
 // to 11.9. Weights' low halves by dot products with (-1, 0) instead of a shift, a mask and two differences: the same or slower.
+// A page number is left as it comes until its row is needed, a step later: formed behind the lookup the row waited for it in every step. With that, and
+// fewer scalar instructions about masks (18 % of what a SIMD issued), us: 4096 tokens 121.5 -> 116.5, a cap and a sink 125 -> 121; 2000 49.0 -> 47.3,
+// with a cap 54.5 -> 52.2; 3 x 200 after 1500 44.8 -> 42.9; 8 x 512 after 512, window 512 42.9 -> 41.1. While its waves run, 87 % of the cycles issue.
 __device__ __align__(16) const bf16s zero_channels[8] = {0, 0, 0, 0, 0, 0, 0, 0};
 
 template <int DS, int VT, int NG, int FORM>
@@ -491,21 +494,18 @@ __global__ __launch_bounds__(256 * NG, 2) void paged_attention_mfma_kernel(
     if (MORE && it < sum_tiles) return it * 32;
     return it < sink_tiles ? (it - sum_tiles) * 32 : wstart + (it - sink_tiles) * 32;
   };
-  auto pool_row = [&](int j) {
-    const int jc = min(j, bp1);  // keys past the sequence's end are masked; read a row that exists
-    return (bt[jc >> page_shift] << page_shift) + (jc & page_mask);
-  };
-  auto sum_row = [&](int idx) {
-    const int ic = min(idx, n_sum - 1);  // a summary tile exists only when n_sum > 0
-    return (bt[ic >> sum_shift] << sum_shift) + (ic & sum_mask);
-  };
+  // The key of the sequence, or the summary, that a lane brings. Keys past the sequence's end are masked, those of a step past the last (below 0) not
+  // used: the block's last token stands for them, whose page exists.
+  auto pool_key = [&](int j) { return (int)min((unsigned)j, (unsigned)bp1); };
+  auto sum_key = [&](int idx) { return min(idx, n_sum - 1); };   // a summary tile exists only when n_sum > 0
   // The page-table lookups of a tile run one step ahead of its key/value loads (two ahead of its use), so that a
   // load's address never waits for a lookup issued in the same step.
   const unsigned krs = (unsigned)(G * Dr) * 2u, vrs = (unsigned)(Gv * Dvr) * 2u;   // bytes between neighbouring keys' rows
-  struct Rows {
+  // Page numbers stay as they come until their rows are needed: what they go through would be waited for right behind the lookup, in every step.
+  struct Pages {
     int key[TP], fac[TP];
-    bool from_sum[TP];  // a summary tile
   };
+  auto summed_tile = [&](int it) { return MORE && it >= 0 && it < sum_tiles; };
   // Steps go from the nearest keys to the farthest. The other way round the scores of a head with a steep distance penalty rise by
   // more than 30 from step to step, so that many steps raise the reference and take their weights twice (with 12: 4000 tokens, window 1024:
   // 83 us, 75 this way; 14 decode tokens beside portions of 1000 and 963: 72, 65). Without a penalty it is all the same (4096
@@ -514,44 +514,57 @@ __global__ __launch_bounds__(256 * NG, 2) void paged_attention_mfma_kernel(
   constexpr int way = -TS;
   const int first_tile = (steps_n - 1) * TS;
   auto lookup = [&](int tile0) {   // of the step whose first tile this is
-    Rows r;
+    Pages r;
 #pragma unroll
     for (int u = 0; u < TP; ++u) {
       const int it = tile0 + grp * TP + u, kbase = tile_base(it);  // a tile past the last one reads rows that exist and is not used
-      r.from_sum[u] = MORE && it < sum_tiles;
-      r.key[u] = r.from_sum[u] ? sum_row(kbase + lkey) : pool_row(kbase + lkey);
-      r.fac[u] = key_fac != nullptr && tid < 32 ? pool_row(kbase + tid) : 0;
+      r.key[u] = bt[summed_tile(it) ? sum_key(kbase + lkey) >> sum_shift : pool_key(kbase + lkey) >> page_shift];
+      if (key_fac != nullptr && tid < 32) r.fac[u] = bt[pool_key(kbase + tid) >> page_shift];
+    }
+    return r;
+  };
+  struct Rows {
+    int key[TP];
+  };
+  auto rows_of = [&](const Pages& p, int tile0) {
+    Rows r;
+#pragma unroll
+    for (int u = 0; u < TP; ++u) {
+      const int it = tile0 + grp * TP + u, kbase = tile_base(it);
+      r.key[u] = summed_tile(it) ? (p.key[u] << sum_shift) + (sum_key(kbase + lkey) & sum_mask)
+                                 : (p.key[u] << page_shift) + (pool_key(kbase + lkey) & page_mask);
     }
     return r;
   };
   const char* zeros = reinterpret_cast<const char*>(zero_channels);
   // Pieces of a step's keys (to the step's place among the two of them) and values, n of the wave's TP * KR and TP * VR. Head sizes that fill the
   // tiles, as nearly all do, need no look at the channel.
-  auto piece = [&](const char* row, int n, int channels, char* __restrict__ dst) __attribute__((always_inline)) {
+  auto piece = [&](const char* row, int n, int channels, int fewest_channels, char* __restrict__ dst) __attribute__((always_inline)) {
     const int quad = quad0 + 2 * (n / TP);
     const char* at = row + (n / TP) * 128;
-    if (channels % 64 != 0 && quad * 32 + lch >= channels) at = zeros;
+    if (64 * (n / TP + 1) > fewest_channels && channels % 64 != 0 && quad * 32 + lch >= channels) at = zeros;
     __builtin_amdgcn_global_load_lds((global_ptr)at, (lds_ptr)(dst + (quad * 2 + row_group) * 1024), 16, 0, 0);
   };
-  auto key_row = [&](const Rows& r, int u) {
-    return reinterpret_cast<const char*>((r.from_sum[u] ? ksum : kpool) + (long)g * Dr + quad0 * 32 + lch) + (unsigned long)(unsigned)r.key[u] * krs;
+  auto key_row = [&](const Rows& r, int tile0, int u) {
+    return reinterpret_cast<const char*>((summed_tile(tile0 + grp * TP + u) ? ksum : kpool) + (long)g * Dr + quad0 * 32 + lch) + (unsigned long)(unsigned)r.key[u] * krs;
   };
-  auto value_row = [&](const Rows& r, int u) {
-    return reinterpret_cast<const char*>((r.from_sum[u] ? vsum : vpool) + (long)vg * Dvr + quad0 * 32 + lch) + (unsigned long)(unsigned)r.key[u] * vrs;
+  auto value_row = [&](const Rows& r, int tile0, int u) {
+    return reinterpret_cast<const char*>((summed_tile(tile0 + grp * TP + u) ? vsum : vpool) + (long)vg * Dvr + quad0 * 32 + lch) + (unsigned long)(unsigned)r.key[u] * vrs;
   };
   auto key_piece = [&](const char* const (&row)[TP], char* __restrict__ dst, int n) __attribute__((always_inline)) {
     if (KQ % 2 != 0 && quad0 + 2 * (n / TP) >= KQ) return;
-    piece(row[n % TP], n, Dr, dst + n % TP * KT);
+    piece(row[n % TP], n, Dr, DS == 8 ? 97 : DS == 6 ? 65 : D - 15, dst + n % TP * KT);
   };
   auto value_piece = [&](const char* const (&row)[TP], char* __restrict__ dst, int n) __attribute__((always_inline)) {
     if (VQ % 2 != 0 && quad0 + 2 * (n / TP) >= VQ) return;
-    piece(row[n % TP], n, Dvr, dst + n % TP * VTT);
+    piece(row[n % TP], n, Dvr, Dv - 31, dst + n % TP * VTT);
   };
   float rf[TP];
-  auto fetch_factors = [&](const Rows& r) {
+  auto fetch_factors = [&](const Pages& p, int tile0) {
 #pragma unroll
     for (int u = 0; u < TP; ++u)
-      if (key_fac != nullptr && tid < 32) rf[u] = key_fac[(long)r.fac[u] * G + g];
+      if (key_fac != nullptr && tid < 32)
+        rf[u] = key_fac[(long)((p.fac[u] << page_shift) + (pool_key(tile_base(tile0 + grp * TP + u) + tid) & page_mask)) * G + g];
   };
   // of a step among three: a step's last tile is weighted in the next one, when the factors of the one after that arrive
   auto stash_factors = [&](int at) {
@@ -602,20 +615,20 @@ __global__ __launch_bounds__(256 * NG, 2) void paged_attention_mfma_kernel(
 
   const RowAt row_at(col, hf);
   const ColAt col_at(lane);
-  Rows next = lookup(first_tile);
+  Pages next = lookup(first_tile);
   // this group's place: [2] steps' keys, [2] steps' values
   constexpr int KS = TP * KT, VS = TP * VTT;
   char* keys = tiles + grp * (2 * KS + 2 * VS);
   char* values = keys + 2 * KS;
   const char *krow[TP], *vrow[TP];
+  Rows of_values = rows_of(next, first_tile);
 #pragma unroll
-  for (int u = 0; u < TP; ++u) krow[u] = key_row(next, u);
+  for (int u = 0; u < TP; ++u) krow[u] = key_row(of_values, first_tile, u);
 #pragma unroll
   for (int n = 0; n < TP * KR; ++n) key_piece(krow, keys, n);
-  fetch_factors(next);
+  fetch_factors(next, first_tile);
 #pragma unroll
-  for (int u = 0; u < TP; ++u) vrow[u] = value_row(next, u);
-  Rows of_values = next;
+  for (int u = 0; u < TP; ++u) vrow[u] = value_row(of_values, first_tile, u);
   if (steps_n > 1) next = lookup(first_tile + way);
   stash_factors(0);
   __builtin_amdgcn_sched_barrier(0);
@@ -629,18 +642,23 @@ __global__ __launch_bounds__(256 * NG, 2) void paged_attention_mfma_kernel(
   // What a tile's scores go through before they are weights: factors, the cap, a penalty or a table, masks. `it` is the tile, `fc` its keys' factors.
   struct Tile {
     int it, kbase;
-    bool summ, inner, live;
+    bool summ, inner;
   };
+  // inner: every key is visible to every token of the wave (lanes past the last one repeat it), no masks to evaluate: the tiles of the window from
+  // in_lo on, inner_n of them
+  const int in_lo = sink_tiles + ((lo_p1 - wstart + 31) >> 5);
+  const unsigned inner_n = head_ok ? (unsigned)max(0, sink_tiles + ((p0 - 31 - wstart) >> 5) - in_lo + 1) : 0u;
   auto tile_of = [&](int it) {
     Tile t;
     t.it = it;
     t.kbase = tile_base(it);
     t.summ = MORE && it < sum_tiles;
-    // inner: every key is visible to every token of the wave (lanes past the last one repeat it), no masks to evaluate
-    t.inner = head_ok && it >= sink_tiles && t.kbase >= lo_p1 && t.kbase + 31 <= p0;
-    // (several token tiles) a tile wholly after this wave's tokens, or wholly before what they see, is not live
-    t.live = t.inner || (head_ok && it < tiles_n && (it < sink_tiles || !(t.kbase > p1 || (t.kbase + 31 < lo_p0 && t.kbase >= keep_first))));
+    t.inner = (unsigned)(it - in_lo) < inner_n;
     return t;
+  };
+  // (several token tiles) a tile wholly after this wave's tokens, or wholly before what they see, is not live
+  auto live = [&](const Tile& t) {
+    return t.inner || (head_ok && t.it < tiles_n && (t.it < sink_tiles || !(t.kbase > p1 || (t.kbase + 31 < lo_p0 && t.kbase >= keep_first))));
   };
   auto factors = [&](f32x16& x, int place) __attribute__((always_inline)) {
     if (key_fac != nullptr) {
@@ -699,7 +717,7 @@ __global__ __launch_bounds__(256 * NG, 2) void paged_attention_mfma_kernel(
     if (!t.inner) {
       const bool ahead = t.it < sink_tiles;  // a tile ahead of the window's: summaries or kept first tokens
       // the tile's keys that this token sees: those up to `last`, from `first` on or below `keep` (offsets in the tile)
-      const int last = !t.live ? -1 : t.summ ? my_sum - 1 - t.kbase : (ahead ? min(n_sink - 1, pos) : min(p1, pos)) - t.kbase;
+      const int last = !live(t) ? -1 : t.summ ? my_sum - 1 - t.kbase : (ahead ? min(n_sink - 1, pos) : min(p1, pos)) - t.kbase;
       const int first = t.summ ? 0 : lo - t.kbase, keep = t.summ ? 0 : keep_first - t.kbase;
 #pragma unroll
       for (int i = 0; i < 16; ++i) {
@@ -754,7 +772,7 @@ __global__ __launch_bounds__(256 * NG, 2) void paged_attention_mfma_kernel(
   };
   // where the sum of a tile's weights shows that some passed 2^12: the maximum, and the weights again
   auto raise = [&](const f32x16& x, float off, float psum, Weights& p) __attribute__((always_inline)) {
-    if (!fixed_ref && !__all(psum <= 4096.0f)) {
+    if (!fixed_ref && __builtin_expect(!__all(psum <= 4096.0f), 0)) {
       Pair again;
       float top = x[0];
 #pragma unroll
@@ -855,15 +873,16 @@ __global__ __launch_bounds__(256 * NG, 2) void paged_attention_mfma_kernel(
   // does no other.
   int tile0 = first_tile, step = 0, third = 0;   // third: the step's place among three
   auto begin = [&]() __attribute__((always_inline)) {   // the next step's keys and this step's values; past the last step the loads repeat rows
-    const Rows now = next;
+    const Pages now = next;
+    const Rows rows = rows_of(now, tile0 + way);
 #pragma unroll
     for (int u = 0; u < TP; ++u) {
-      krow[u] = key_row(next, u);
-      vrow[u] = value_row(of_values, u);
+      krow[u] = key_row(rows, tile0 + way, u);
+      vrow[u] = value_row(of_values, tile0, u);
     }
-    of_values = next;
-    if (step + 2 < steps_n) next = lookup(tile0 + 2 * way);
-    if (step + 1 < steps_n) fetch_factors(now);
+    of_values = rows;
+    next = lookup(tile0 + 2 * way);
+    if (step + 1 < steps_n) fetch_factors(now, tile0 + way);
   };
   auto end = [&]() __attribute__((always_inline)) {
     third = third == 2 ? 0 : third + 1;
@@ -906,7 +925,7 @@ __global__ __launch_bounds__(256 * NG, 2) void paged_attention_mfma_kernel(
   int stop = (mine0 + 1 - w_lo + TS) / TS;
   if (again <= stop) stop = steps_n;
   auto mine_of = [&](int u) { return tile_of(tile0 + grp * TP + u); };
-  while (step < steps_n && !mine_of(0).live && !mine_of(1).live) idle();
+  while (step < steps_n && !live(mine_of(0)) && !live(mine_of(1))) idle();
   if (step < steps_n) {
     f32x16 xe, xo;            // scores of an even and an odd tile of the wave's
     Weights pe, po;
