@@ -38,7 +38,7 @@
 // and the forward with products and weights in turns, us (another card):
 //   B4 S4096 H32/8 D128 causal 570 -> 550, B1 S8192 H32/8 514 -> 500, H4 159 -> 128 (half the chip); B8 S1024 H12 D64 32.0 -> 31.2,
 //   packed, 16384 tokens of up to 4096, 32/8 of 128 384 -> 367, 12 of 64 102 -> 95, 8192 of up to 2048, 32/8 113 -> 103;
-//   B1 S4096 H8/2 D64 unmasked 56.9 -> 53.3, but B1 S8192 H12 D64 causal 168 -> 171
+//   B1 S4096 H8/2 D64 unmasked 56.9 -> 53.3
 // and with a quarter of its instructions taken out, waits and scalar ones (a step of 64 keys 380 -> 273; they were 25 % of what a SIMD issues), us:
 //   B1 S8192 H4/1 D128 causal 126 -> 116, H12 D64 167 -> 162; B1 S2048 H12 D64 27.1 -> 24.8; B1 S4096 H8/2 D64 54 -> 50; B4 S4096 H32 D128 582 -> 572,
 //   H32/8 at a full chip the same: power. Slower there: products of 16 x 16 x 32 (542 for 532, H4/1 148 for 127: more instructions), 64 rows a wave (610).
@@ -75,32 +75,115 @@ DEV_INLINE bf16x8_t ld_g16(const unsigned short* p) {
 // C-layout row for mfma_f32_32x32x16 register j (guide §3, HW-verified).
 DEV_INLINE constexpr int crow(int j, int half) { return (j & 3) + 8 * (j >> 2) + 4 * half; }
 
-// Whether a head's blocks of a causal packed batch go by tile, late ones of all sequences first, and not sequence by sequence.
+// Whether a head's blocks of a causal packed batch that they do not look up (packed_tile) go by tile, late ones of all sequences first, and not sequence by sequence.
 // Short sequences leave many tiles empty and end unevenly; keys and values of long ones, and of heads that share none, are
 // met in L2 by the tiles that run together. By sequence / by tile, us, forward and backward: 186 sequences of up to 256 tokens, 16/4
 // heads of 64: 48 / 39, 151 / 141; 54 of 900, 8/2 of 128: 58 / 49, 210 / 200; 46 of 1024, 32/8: 193 / 179, 534 / 531 (41: 188 / 185,
 // 541 / 554); but 14 of 4096: 406 / 437, 1108 / 1147; 81 of 600, 12 heads of 64: 39 / 45, 110 / 116; 20 of 300, 8 heads: 9.3 / 10.4.
 DEV_INLINE bool by_tile(int tiles, long blocks, int group) { return tiles <= 8 && blocks > 512 && group > 1; }
 
-// Which (q tile, sequence, head) a block of the forward works on. Blocks of one (sequence, head) share an
+// XCDs that share a row of tiles, so that all of them get as much: 1, 2, 4 or 8
+__host__ __device__ __forceinline__ int row_parts(int n_y) { return n_y % 8 == 0 ? 1 : n_y % 4 == 0 ? 2 : n_y % 2 == 0 ? 4 : 8; }
+// Blocks that deal() takes for n_y rows of n_x tiles: whole rounds of the XCDs
+__host__ __device__ __forceinline__ long dealt_blocks(long n_x, int n_y) {
+  const int parts = row_parts(n_y);
+  return (n_x + parts - 1) / parts * parts * n_y;
+}
+// Tile x and row y of block f, false if it has none; x goes from a row's longest tile to its shortest. An XCD (f % 8) has whole rows, or every
+// second, fourth or eighth tile of them, and takes W rows at a time, tile by tile, so that it ends with short tiles of many rows. With `pairs` the
+// blocks are all there are: where two share a CU (32 on an XCD) they are a long one and a short one.
+DEV_INLINE bool deal(int f, int n_x, int n_y, int W, bool pairs, int& x, int& y) {
+  const int parts = row_parts(n_y), rows = n_y * parts / 8, tiles = (n_x + parts - 1) / parts, all = rows * tiles;
+  int i = f >> 3;
+  if (i >= all) return false;
+  if (pairs && all <= 64 && i >= 32) i = all - 1 - (i - 32);
+  const int first = i / (W * tiles) * W, wide = min(W, rows - first);
+  i -= first * tiles;
+  const int row = (f & 7) * rows + first + i % wide;
+  x = i / wide * parts + row % parts;
+  y = row / parts;
+  return x < n_x;
+}
+
+// Tile i of a packed batch of up to MOST_PACKED sequences of at most `most` tiles of `rows` rows, those of more tiles first; false past the last one. Every
+// lane has four sequences; how many tiles those of at least c tiles have is a sum over the lanes, and the c of tile i found by halving.
+constexpr int MOST_PACKED = 256;
+DEV_INLINE bool packed_tile(const int* __restrict__ CU, int B, int rows, int most, int i, int& b, int& tile, int& tiles) {
+  const int lane = threadIdx.x & 63;
+  int own[MOST_PACKED / 64];
+#pragma unroll
+  for (int k = 0; k < MOST_PACKED / 64; ++k) {
+    const int at = 64 * k + lane;
+    own[k] = 64 * k < B && at < B ? min((CU[at + 1] - CU[at] + rows - 1) / rows, most) : 0;
+  }
+  auto at_least = [&](int c) {
+    int v = own[0] >= c ? own[0] : 0;
+#pragma unroll
+    for (int k = 1; k < MOST_PACKED / 64; ++k)
+      if (64 * k < B) v += own[k] >= c ? own[k] : 0;
+    // summed inside rows of 16 lanes, then over the rows
+    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);
+    return __builtin_amdgcn_readlane(v, 63);
+  };
+  int ahead = 0, hi = most + 1;   // at_least(tiles) > i >= at_least(hi) = ahead
+  tiles = 1;
+  if (at_least(1) <= i) return false;
+  while (hi - tiles > 1) {
+    const int mid = (tiles + hi) >> 1, n = at_least(mid);
+    if (n > i) {
+      tiles = mid;
+    } else {
+      hi = mid;
+      ahead = n;
+    }
+  }
+  int nth = (i - ahead) / tiles;   // of the sequences of as many tiles
+  tile = i - ahead - nth * tiles;
+#pragma unroll
+  for (int k = 0; k < MOST_PACKED / 64; ++k) {
+    const unsigned long long same = __ballot(own[k] == tiles);
+    const int here = __builtin_popcountll(same);
+    if (nth >= 0 && nth < here) {
+      const int order = __builtin_amdgcn_mbcnt_hi((unsigned)(same >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)same, 0));
+      b = 64 * k + __builtin_ctzll(__ballot(own[k] == tiles && order == nth));
+    }
+    nth -= here;
+  }
+  return true;
+}
+
+// Which (q tile, sequence, head) a block of the forward works on, false if on none. Blocks of one (sequence, head) share an
 // XCD's L2. Packed batches run head by head, each head over all sequences: the other way round
 // the longest sequence is one XCD's work (10 sequences of 256..4096 tokens: 1488 against 463 us). Under a causal
-// mask the late tiles see the most keys: they start first. A grid that fits on the chip at once (two blocks a
-// CU) runs every second head the other way, so that a CU's two blocks are a long and a short one.
+// mask the late tiles see the most keys: they start first. `dealt`: tiles of a row that deal() takes, of the packed batch or of a causal sequence.
 template <bool VARLEN>
-DEV_INLINE void q_block(int B, int Hq, int group, int causal, int& tile, int& b, int& h) {
+DEV_INLINE bool q_block(const int* __restrict__ CU, int rows, int B, int Hq, int group, int causal, int W, int dealt, int most, int& tile, int& b, int& h) {
   int y;
+  if (dealt) {
+    if (!deal((int)(blockIdx.y * gridDim.x + blockIdx.x), dealt, (VARLEN ? 1 : B) * Hq, W, true, tile, y)) return false;
+    b = VARLEN ? 0 : y / Hq;
+    h = VARLEN ? y : y % Hq;
+    int tiles = dealt;
+    if (VARLEN && !packed_tile(CU, B, rows, most, tile, b, tile, tiles)) return false;
+    if (causal) tile = tiles - 1 - tile;
+    return true;
+  }
   xcd_swizzle_xy(tile, y);
-  const bool once = (int)(gridDim.x * gridDim.y) <= 512 && (y & 1);
   b = VARLEN ? y % B : y / Hq;
   h = VARLEN ? y / B : y % Hq;
   if (VARLEN && causal && by_tile((int)gridDim.x, (long)gridDim.x * gridDim.y, group)) {
     const int i = b * (int)gridDim.x + tile;
     tile = (int)gridDim.x - 1 - i / B;
     b = i % B;
-  } else if (causal && !once) {
+  } else if (causal) {
     tile = (int)gridDim.x - 1 - tile;
   }
+  return true;
 }
 
 // Logical index of block f of nblocks so that every XCD (block f runs on XCD f % 8) gets a contiguous range.
@@ -201,7 +284,7 @@ __global__ __launch_bounds__(NW * 64, 2) void fa_fwd_kernel(
     const int* __restrict__ CU,
     const int* __restrict__ CUK,
     long qbs, long qts, long kbs, long kts,
-    int B, int S, int Sk, int Hq, int Hkv, float scale, int causal) {
+    int B, int S, int Sk, int Hq, int Hkv, float scale, int causal, int W, int dealt, int most) {
   using namespace fa;
   extern __shared__ char smem[];
   constexpr int NT = NW * 64;
@@ -212,7 +295,7 @@ __global__ __launch_bounds__(NW * 64, 2) void fa_fwd_kernel(
   const int ln = lane & 31;
 
   int tile, b, h;
-  q_block<VARLEN>(B, Hq, Hq / Hkv, causal, tile, b, h);
+  if (!q_block<VARLEN>(CU, NW * QW, B, Hq, Hq / Hkv, causal, W, dealt, most, tile, b, h)) return;
   const int hk = h / (Hq / Hkv);
   const int q0 = tile * (NW * QW);
   const int qw = q0 + w * QW;  // this wave's first q row
@@ -593,7 +676,7 @@ DEV_INLINE void bwd_dkdv(
     unsigned short* __restrict__ dK, unsigned short* __restrict__ dV, float* __restrict__ PART, int GS,
     const int* __restrict__ CU, const int* __restrict__ CUK,
     long qbs, long qts, long kbs, long kts, long dkbs, long dkts,
-    int tiles, int B, int S, int Sk, int Hq, int Hkv, float scale, int causal) {
+    int tiles, int B, int S, int Sk, int Hq, int Hkv, float scale, int causal, int W, int dealt) {
   using namespace fa;
   constexpr int QB = 32;
   constexpr int TB = tile_bytes<QB, D>();
@@ -608,14 +691,26 @@ DEV_INLINE void bwd_dkdv(
   const int half = lane >> 5;
   const int ln = lane & 31;
 
-  f = xcd_chunk(f, nblocks);
   // key/value tile fastest, then the part of the group's heads, then (sequence, kv head): their
   // Q/dO streams meet in one XCD's L2. Under a causal mask the first tiles see the most queries.
-  const int kv0 = (f % tiles) * (NWB * QW);
-  const int part = (f / tiles) % GS;
-  const int y = f / (tiles * GS);
-  if (y >= B * Hkv) return;
-  const int b = VARLEN ? y % B : y / Hkv, hk = VARLEN ? y / B : y % Hkv;
+  int tile, part, b, hk;
+  if (dealt) {
+    int y, all;
+    if (!deal(f, dealt, (VARLEN ? 1 : B) * Hkv * GS, W, false, tile, y)) return;
+    part = y % GS;
+    b = VARLEN ? 0 : y / GS / Hkv;
+    hk = VARLEN ? y / GS : y / GS % Hkv;
+    if (VARLEN && !packed_tile(CU, B, NWB * QW, tiles, tile, b, tile, all)) return;
+  } else {
+    f = xcd_chunk(f, nblocks);
+    tile = f % tiles;
+    part = (f / tiles) % GS;
+    const int y = f / (tiles * GS);
+    if (y >= B * Hkv) return;
+    b = VARLEN ? y % B : y / Hkv;
+    hk = VARLEN ? y / B : y % Hkv;
+  }
+  const int kv0 = tile * (NWB * QW);
   const int group = Hq / Hkv, h_first = part * group / GS;
   const int G = (part + 1) * group / GS - h_first;       // heads of this block: its share of the group, GS need not divide it
   const int kvw = kv0 + w * QW;  // this wave's first kv row
@@ -857,7 +952,7 @@ DEV_INLINE void bwd_dq(
     const float2v* __restrict__ STATS, unsigned short* __restrict__ dQ,
     const int* __restrict__ CU, const int* __restrict__ CUK,
     long qbs, long qts, long kbs, long kts, long dqbs, long dqts,
-    int tiles, int B, int S, int Sk, int Hq, int Hkv, float scale, int causal) {
+    int tiles, int B, int S, int Sk, int Hq, int Hkv, float scale, int causal, int W, int dealt) {
   using namespace fa;
   constexpr int TB = tile_bytes<KVB, D>();
   constexpr int DSL = D / 16, NB = D / 32;
@@ -869,16 +964,28 @@ DEV_INLINE void bwd_dq(
   const int half = lane >> 5;
   const int ln = lane & 31;
 
-  f = xcd_chunk(f, nblocks);
-  const int y = f / tiles;
-  if (y >= B * Hq) return;
-  int tile = causal ? tiles - 1 - f % tiles : f % tiles;  // late tiles see the most keys
-  int b = VARLEN ? y % B : y / Hq;
-  const int h = VARLEN ? y / B : y % Hq;
-  if (VARLEN && causal && by_tile(tiles, nblocks, Hq / Hkv)) {
-    const int i = f - h * B * tiles;
-    tile = tiles - 1 - i / B;
-    b = i % B;
+  int y, tile, b, h;
+  if (dealt) {
+    int all = dealt;
+    if (!deal(f, dealt, (VARLEN ? 1 : B) * Hq, W, false, tile, y)) return;
+    b = VARLEN ? 0 : y / Hq;
+    h = VARLEN ? y : y % Hq;
+    if (VARLEN && !packed_tile(CU, B, NWB * QW, tiles, tile, b, tile, all)) return;
+    if (causal) tile = all - 1 - tile;  // late tiles see the most keys
+  } else {
+    f = xcd_chunk(f, nblocks);
+    y = f / tiles;
+    tile = f % tiles;
+    if (y >= B * Hq) return;
+    b = VARLEN ? y % B : y / Hq;
+    h = VARLEN ? y / B : y % Hq;
+    if (VARLEN && causal && by_tile(tiles, nblocks, Hq / Hkv)) {
+      const int i = b * tiles + tile;
+      tile = tiles - 1 - i / B;
+      b = i % B;
+    } else if (causal) {
+      tile = tiles - 1 - tile;
+    }
   }
   const int hk = h / (Hq / Hkv);
   const int q0 = tile * (NWB * QW);
@@ -1065,16 +1172,16 @@ __global__ __launch_bounds__(fa::NTB, D == 64 ? 3 : 2) void fa_bwd_kernel(
     unsigned short* __restrict__ dQ, unsigned short* __restrict__ dK, unsigned short* __restrict__ dV,
     float* __restrict__ PART, int GS, const int* __restrict__ CU, const int* __restrict__ CUK,
     long qbs, long qts, long kbs, long kts, long dqbs, long dqts, long dkbs, long dkts,
-    int n_kv, int n_q, int kv_tiles, int q_tiles, int B, int S, int Sk, int Hq, int Hkv, float scale, int causal) {
+    int n_kv, int n_q, int kv_tiles, int q_tiles, int B, int S, int Sk, int Hq, int Hkv, float scale, int causal, int W, int dealt) {
   extern __shared__ char smem[];
   const int f = (int)(blockIdx.y * gridDim.x + blockIdx.x);   // more than one grid row only beyond 2^23 blocks
   if (f >= n_kv + n_q) return;
   if (f < n_kv)
     bwd_dkdv<D, VARLEN>(smem, f, n_kv, Q, K, V, dO, STATS, dK, dV, PART, GS, CU, CUK, qbs, qts, kbs, kts, dkbs, dkts,
-                        kv_tiles, B, S, Sk, Hq, Hkv, scale, causal);
+                        kv_tiles, B, S, Sk, Hq, Hkv, scale, causal, W, dealt);
   else
     bwd_dq<D, VARLEN>(smem, f - n_kv, n_q, Q, K, V, dO, STATS, dQ, CU, CUK, qbs, qts, kbs, kts,
-                      dqbs, dqts, q_tiles, B, S, Sk, Hq, Hkv, scale, causal);
+                      dqbs, dqts, q_tiles, B, S, Sk, Hq, Hkv, scale, causal, W, dealt);
 }
 
 // dK and dV from the float32 sums of the GS blocks that shared a tile's heads: four channels a thread.
@@ -1129,6 +1236,27 @@ void set_lds_limit(const void* kernel, size_t bytes) {
 // and its loads are twice those of one block of four: 4/2 waves at 144 to 252 blocks 0.93 (128 tokens), 0.84 (512), 0.76 (2048); with a mask 0.9, 0.83, 0.98.
 int fwd_waves(long blocks) { return blocks <= 128 ? 2 : 4; }
 
+// Rows (heads of sequences) whose tiles an XCD takes side by side (deal): as many as end evenly and whose keys and values, of kv_bytes a kv head,
+// still meet in its L2 (4 MB; twice that, as not all are in the same place). us, forward and backward, one row, four, eight, sixteen: B8 S1024 H12 D64 31
+// and 81, 31 and 73, 30 and 73, 25 and 67; B4 S4096 H32 D128 568 and 1778, 548 and 1714, 555 and 1723, 571 and 1773; B4 S2048 H16/4 D128 91 and 288, 78
+// and 276, 74 and 269, 74 and 272; B1 S8192 H12 D64 (two of three rows an XCD) 175 and 386, 123 and 338; B1 S8192 H32/8 D128 554 and 1645, 527 and 1579.
+int rows_together(int group, long kv_bytes) { return (int)std::max(4L, group * std::min(16L, (8L << 20) / std::max(1L, kv_bytes))); }
+
+// Tiles of a packed batch that its blocks look up (packed_tile), an upper bound; 0: sequence by sequence or tile by tile. Sequences of one tile need no
+// order, and small grids run at once in any. us, forward and backward, before and by lookup: 16384 tokens of up to 4096 in 12 sequences, 32/8 heads of
+// 128 363 and 1110, 346 and 1072; 12 of 64 96 and 257, 80 and 235; 64 sequences of up to 900, 8/2 of 128 54 and 187, 37 and 138; 46 of 1024, 32/8 of 128 169
+// and 493, 161 and 443; 56 of 500, 16/2 of 64 22 and 88, 22 and 62; 47 of 256, 16/4 of 64 12.3 and 37.1, 12.4 and 35.3; 39 of 128, 32/8 of 64 11.4, 12.8.
+long packed_tiles(long T, int n_seq, long tiles, int rows, int H) {
+  const long all = std::min(T / rows + n_seq, tiles * n_seq);
+  return n_seq <= fa::MOST_PACKED && tiles > 1 && all * H > 512 ? all : 0;
+}
+
+// a grid dimension of 2^32 threads or more is cut short without an error
+dim3 wide_grid(long blocks) {
+  const long width = std::max(1L, std::min(blocks, 1L << 23));
+  return dim3((unsigned)width, (unsigned)((blocks + width - 1) / width));
+}
+
 // q/k/v are [B,S,H,D] views that may be strided in dims 0/1 (e.g. views into
 // a packed QKV GEMM output); dims 2/3 must be dense.
 void check_fa_view(const at::Tensor& t, const char* name) {
@@ -1182,14 +1310,15 @@ std::vector<at::Tensor> flash_attn_fwd(at::Tensor q, at::Tensor k, at::Tensor v,
 
 #define LAUNCH_FWD(DD, NW)                                                                            \
   do {                                                                                            \
+    const int tiles = (S + NW * QW - 1) / (NW * QW), dealt = causal && (long)tiles * B * Hq > 256 ? tiles : 0;  \
     const size_t lds = 4 * tile_bytes<KVB, DD>();                                                  \
     set_lds_limit((const void*)fa_fwd_kernel<DD, NW, false>, lds);                                \
-    hipLaunchKernelGGL((fa_fwd_kernel<DD, NW, false>), dim3((S + NW * QW - 1) / (NW * QW), B * Hq), \
+    hipLaunchKernelGGL((fa_fwd_kernel<DD, NW, false>), dealt ? wide_grid(dealt_blocks(tiles, B * Hq)) : dim3((unsigned)tiles, B * Hq), \
                        dim3(NW * 64), lds, stream.stream(),                                       \
                        (const unsigned short*)q.data_ptr(), (const unsigned short*)k.data_ptr(),  \
                        (const unsigned short*)v.data_ptr(), (unsigned short*)o.data_ptr(),        \
                        lse.data_ptr<float>(), cu, cuk, qbs, qts, kbs, kts,                        \
-                       B, S, Sk, Hq, Hkv, (float)scale, causal ? 1 : 0);                              \
+                       B, S, Sk, Hq, Hkv, (float)scale, causal ? 1 : 0, rows_together(Hq / Hkv, Sk * DD * 4L), dealt, 0);  \
   } while (0)
 
   const int nw = fwd_waves((S + 4 * QW - 1L) / (4 * QW) * B * Hq);
@@ -1225,14 +1354,15 @@ std::vector<at::Tensor> flash_attn_varlen_fwd(at::Tensor q, at::Tensor k, at::Te
 #define LAUNCH_VFWD(DD, NW)                                                                           \
   do {                                                                                            \
     const size_t lds = 4 * tile_bytes<KVB, DD>();                                                  \
+    const long tiles = (max_seqlen + NW * QW - 1) / (NW * QW), packed = packed_tiles(T, n_seq, tiles, NW * QW, Hq);  \
     set_lds_limit((const void*)fa_fwd_kernel<DD, NW, true>, lds);                                 \
     hipLaunchKernelGGL((fa_fwd_kernel<DD, NW, true>),                                             \
-                       dim3(((int)max_seqlen + NW * QW - 1) / (NW * QW), n_seq * Hq), dim3(NW * 64), lds, stream.stream(), \
+                       packed ? wide_grid(dealt_blocks(packed, Hq)) : dim3((unsigned)tiles, n_seq * Hq), dim3(NW * 64), lds, stream.stream(), \
                        (const unsigned short*)q.data_ptr(), (const unsigned short*)k.data_ptr(),  \
                        (const unsigned short*)v.data_ptr(), (unsigned short*)o.data_ptr(),        \
                        lse.data_ptr<float>(), cu_seqlens.data_ptr<int>(), nullptr,                \
                        0L, qts, 0L, kts,                                                          \
-                       n_seq, T, T, Hq, Hkv, (float)scale, causal ? 1 : 0);                          \
+                       n_seq, T, T, Hq, Hkv, (float)scale, causal ? 1 : 0, rows_together(Hq / Hkv, max_seqlen * DD * 4L), (int)packed, (int)tiles);  \
   } while (0)
 
   // blocks' worth of waves that have tokens, a sequence's last wave half of them (8 heads on 2 of 128, 23 samples of 8 to 128 tokens: 6.8 us, blocks of four 7.3)
@@ -1280,18 +1410,20 @@ void launch_bwd(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, c
   const long n_part = (VARLEN ? (long)Sk : (long)seqs * Sk) * Hkv * D;
   at::Tensor part;
   if (gs > 1) part = at::empty({gs * 2 * n_part}, q.options().dtype(at::kFloat));
-  const long n_kv = ((long)kv_tiles * seqs * Hkv * gs + 7) / 8 * 8, n_q = (long)q_tiles * seqs * Hq, blocks = n_kv + n_q;
+  const long dealt = VARLEN ? packed_tiles(S, seqs, q_tiles, rows, Hq) : causal && S_max == Sk_max ? q_tiles : 0;
+  const int each = VARLEN ? 1 : seqs;
+  const long n_kv = dealt ? (dealt_blocks(dealt, each * Hkv * gs) + 7) / 8 * 8 : ((long)kv_tiles * seqs * Hkv * gs + 7) / 8 * 8;
+  const long n_q = dealt ? dealt_blocks(dealt, each * Hq) : (long)q_tiles * seqs * Hq, blocks = n_kv + n_q;
   TORCH_CHECK(blocks < (1L << 31) - (1L << 23), "flash_attn_bwd: too many tiles");
-  // a grid dimension of 2^32 threads or more is cut short without an error: packed batches of very many sequences get there
-  const long width = std::max(1L, std::min(blocks, 1L << 23));
   auto kernel = fa_bwd_kernel<D, VARLEN>;
   set_lds_limit((const void*)kernel, bwd_lds<D>());
-  hipLaunchKernelGGL(kernel, dim3((unsigned)width, (unsigned)((blocks + width - 1) / width)), dim3(NTB), bwd_lds<D>(), stream,
+  hipLaunchKernelGGL(kernel, wide_grid(blocks), dim3(NTB), bwd_lds<D>(), stream,
                      (const unsigned short*)q.data_ptr(), (const unsigned short*)k.data_ptr(),
                      (const unsigned short*)v.data_ptr(), (const unsigned short*)dout.data_ptr(),
                      (const float2v*)stats.data_ptr(), (unsigned short*)dq.data_ptr(), (unsigned short*)dk.data_ptr(),
                      (unsigned short*)dv.data_ptr(), gs > 1 ? part.data_ptr<float>() : nullptr, gs, cu, cuk, qbs, qts, kbs,
-                     kts, dqbs, dqts, dkbs, dkts, (int)n_kv, (int)n_q, kv_tiles, q_tiles, seqs, S, Sk, Hq, Hkv, scale, causal ? 1 : 0);
+                     kts, dqbs, dqts, dkbs, dkts, (int)n_kv, (int)n_q, kv_tiles, q_tiles, seqs, S, Sk, Hq, Hkv, scale, causal ? 1 : 0,
+                     rows_together(G, Sk_max * D * 4L), (int)dealt);
   HIP_CHECK_LAST();
   if (gs > 1) {
     hipLaunchKernelGGL(fa_bwd_sum_kernel, dim3((unsigned)((n_part / 4 + 255) / 256)), dim3(256), 0, stream,

@@ -218,6 +218,46 @@ def test_where_steps_without_a_mask_end(S, D, causal):
                 _near(x[b: b + 1, :n], y, f"{name} {padded} {b}")
 
 
+@pytest.mark.parametrize("B,S,H,G", [(1, 700, 12, 12), (3, 300, 5, 5), (2, 1100, 7, 1), (1, 130, 20, 4), (1, 3000, 6, 2), (5, 257, 16, 16)])
+def test_rows_dealt_to_the_chips_parts(B, S, H, G):
+    """Causal rows, of numbers that eight parts of the chip share evenly or not, several side by side; remainders of either."""
+    q, k, v, dout = _inputs(B, S, H, G, 64, S)
+    a = [t.clone().requires_grad_() for t in (q, k, v)]
+    from colossalai_amd.ops import flash_attention
+
+    o = flash_attention(*a, causal=True)
+    for name, x, y in zip(("out", "dq", "dk", "dv"), [o] + list(torch.autograd.grad(o, a, dout)), _reference(q, k, v, dout, True, 0.125)):
+        _near(x, y, name)
+
+
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("lens,H,G", [
+    ([900, 1, 0, 900, 129, 1500, 128, 640], 12, 12),               # equal lengths, an empty one, tiles that are just full
+    ([5000], 16, 4), ([40, 300] * 32 + [1100], 6, 2),              # one; two a lane
+    ([20] * 255 + [900], 9, 3), ([20] * 256 + [900], 9, 3),        # the most that are looked up, and one more
+    ([300 + 37 * i for i in range(20)], 5, 5),
+])
+def test_packed_tiles_by_lookup(lens, H, G, causal):
+    """Packed batches of more blocks than run at once: their blocks look their tiles up, longest sequences first."""
+    from colossalai_amd.ops import flash_attention_varlen
+
+    T, D = sum(lens), 64
+    q, k, v, dout = (t[0] for t in _inputs(1, T, H, G, D, T))
+    a = [t.clone().requires_grad_() for t in (q, k, v)]
+    cu = torch.tensor([0] + lens).cumsum(0).int().cuda()
+    o = flash_attention_varlen(*a, cu, max(lens), causal=causal)
+    got = [o] + list(torch.autograd.grad(o, a, dout))
+    want = [torch.zeros_like(t, dtype=torch.float32) for t in (q, q, k, v)]
+    at = 0
+    for n in lens:
+        if n:
+            for w, r in zip(want, _reference(*(t[None, at: at + n] for t in (q, k, v, dout)), causal, D ** -0.5)):
+                w[at: at + n] = r[0]
+        at += n
+    for name, x, y in zip(("out", "dq", "dk", "dv"), got, want):
+        _near(x, y, name)
+
+
 @pytest.mark.parametrize("H", [31, 32, 33])
 @pytest.mark.parametrize("D,causal", [(64, True), (128, False)])
 @pytest.mark.parametrize("packed", [False, True])
