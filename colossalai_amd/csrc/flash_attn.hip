@@ -643,6 +643,11 @@ __global__ __launch_bounds__(256) void fa_delta_kernel(
   }
 }
 
+// Query tiles, of all of a block's heads, whose rows' statistics a block of the backward can form itself, instead of a kernel ahead of it.
+constexpr int OWN_TILES = 8;
+template <int D, bool VARLEN>
+constexpr bool CAN_OWN = D == 64 && !VARLEN;
+
 // ============================================================ backward kernel
 //
 // One launch for dK/dV and dQ: the first n_kv blocks (a multiple of 8) take key/value tiles, the
@@ -673,7 +678,7 @@ DEV_INLINE void bwd_dkdv(
     char* smem, int f, int nblocks,
     const unsigned short* __restrict__ Q, const unsigned short* __restrict__ K,
     const unsigned short* __restrict__ V, const unsigned short* __restrict__ dO, const float2v* __restrict__ STATS,
-    unsigned short* __restrict__ dK, unsigned short* __restrict__ dV, float* __restrict__ PART, int GS,
+    const unsigned short* __restrict__ O, const float* __restrict__ LSE, unsigned short* __restrict__ dK, unsigned short* __restrict__ dV, float* __restrict__ PART, int GS,
     const int* __restrict__ CU, const int* __restrict__ CUK,
     long qbs, long qts, long kbs, long kts, long dkbs, long dkts,
     int tiles, int B, int S, int Sk, int Hq, int Hkv, float scale, int causal, int W, int dealt) {
@@ -684,7 +689,8 @@ DEV_INLINE void bwd_dkdv(
   char* Vlds = smem;                                     // [128 rows]
   char* Qbuf = smem + tile_bytes<NWB * QW, D>();         // [2] query tiles, [2] dO tiles
   char* dObuf = Qbuf + 2 * TB;
-  char* stats_lds = dObuf + 2 * TB;                      // [2][32 of -lse log2e, 32 of -delta]
+  char* stats_lds = dObuf + 2 * TB;                      // [2, or OWN_TILES][32 of -lse log2e, 32 of -delta]
+  const bool own = CAN_OWN<D, VARLEN> && STATS == nullptr;   // no kernel ahead has formed them: all of the block's, in the order of its steps
 
   const int lane = threadIdx.x & 63;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);   // the same for a wave: what it decides is a scalar branch
@@ -786,8 +792,9 @@ DEV_INLINE void bwd_dkdv(
     stats_now = __builtin_amdgcn_make_buffer_rsrc(const_cast<float2v*>(stats), 0, all ? stats_whole : stats_last, 0x00027000);
     stats += QB;
   };
+  const int stats_wave = own ? -1 : 0;
   auto bring_stats = [&](int buf) __attribute__((always_inline)) {
-    if (w == 0) __builtin_amdgcn_raw_ptr_buffer_load_lds(stats_now, (lds_ptr)(stats_lds + buf * 256), 4, (int)stats_off, 0, 0, 0);
+    if (w == stats_wave) __builtin_amdgcn_raw_ptr_buffer_load_lds(stats_now, (lds_ptr)(stats_lds + buf * 256), 4, (int)stats_off, 0, 0, 0);
   };
   typedef TileLoad<D, QB, NWB> Load;
   if (steps > 0) {
@@ -798,14 +805,39 @@ DEV_INLINE void bwd_dkdv(
       dos.piece(dObuf, w, i);
     }
     bring_stats(0);
+    if (own) {
+      constexpr int TPR = D / 8, AT_ONCE = NTB / TPR;   // threads of a row, rows
+      const int c = threadIdx.x % TPR, sub = threadIdx.x / TPR;
+#pragma unroll 4
+      for (int at = 0; at < min(steps, OWN_TILES) * QB; at += AT_ONCE) {
+        const int step = at / QB, head = step / nq, in = at % QB + sub, row = first + (step - head * nq) * QB + in;
+        float dot = 0.0f, lse = -INFINITY;
+        if (row < Seff) {
+          const int h = hk * group + h_first + head;
+          const long from = ((long)b * S + row) * do_stride + (long)h * D + c * 8;
+          const bf16x8_t x = ld_g16(dO + from), y = ld_g16(O + from);
+#pragma unroll
+          for (int e = 0; e < 8; ++e) dot = fmaf((float)x[e], (float)y[e], dot);
+          lse = LSE[((long)b * Hq + h) * S + row];
+        }
+#pragma unroll
+        for (int o = 1; o < TPR; o <<= 1) dot += __shfl_xor(dot, o);
+        if (c == 0) {
+          float* to = reinterpret_cast<float*>(stats_lds + step * 256) + in;
+          to[0] = lse == -INFINITY ? -INFINITY : -lse * 1.44269504f;
+          to[QB] = -dot;
+        }
+      }
+    }
   }
   loads_done();
   __syncthreads();
 
+  int stats_at = 0;
   // A query tile, while the next one arrives in the other buffers.
   auto step = [&](int qt0, int buf, const char* __restrict__ Qlds, const char* __restrict__ dOlds, char* __restrict__ Qn,
                   char* __restrict__ dOn) __attribute__((always_inline)) {
-    const float* stats = reinterpret_cast<const float*>(stats_lds + buf * 256) + 4 * half;
+    const float* stats = reinterpret_cast<const float*>(stats_lds + stats_at) + 4 * half;
     // ---- S[q][kv] = Q · K^T and dP[q][kv] - delta[q] = dO · V^T - delta: column = kv (ln), row = q
     f32x16 s, dp;
 #pragma unroll
@@ -893,6 +925,7 @@ DEV_INLINE void bwd_dkdv(
   };
   auto finish = [&]() __attribute__((always_inline)) {
     buf ^= 1;
+    stats_at = own ? stats_at + 256 : buf * 256;
     loads_done();
     __syncthreads();
   };
@@ -949,7 +982,7 @@ DEV_INLINE void bwd_dq(
     char* smem, int f, int nblocks,
     const unsigned short* __restrict__ Q, const unsigned short* __restrict__ K,
     const unsigned short* __restrict__ V, const unsigned short* __restrict__ dO,
-    const float2v* __restrict__ STATS, unsigned short* __restrict__ dQ,
+    const float2v* __restrict__ STATS, const unsigned short* __restrict__ O, const float* __restrict__ LSE, unsigned short* __restrict__ dQ,
     const int* __restrict__ CU, const int* __restrict__ CUK,
     long qbs, long qts, long kbs, long kts, long dqbs, long dqts,
     int tiles, int B, int S, int Sk, int Hq, int Hkv, float scale, int causal, int W, int dealt) {
@@ -1023,7 +1056,21 @@ DEV_INLINE void bwd_dq(
     }
   }
   const long stat = (VARLEN ? (long)h * S + seq0 : ((long)b * Hq + h) * S) + q_my;
-  const float2v own = STATS[stat];
+  float2v own;
+  if (!CAN_OWN<D, VARLEN> || STATS != nullptr) {
+    own = STATS[stat];
+  } else {   // a lane has half of its row's channels
+    const unsigned short* op = O + (do_base - dO) + (long)q_my * do_stride + half * 8;
+    float dot = 0.0f;
+#pragma unroll
+    for (int sl = 0; sl < DSL; ++sl) {
+      const bf16x8_t y = ld_g16(op + sl * 16);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) dot = fmaf((float)dof[sl][e], (float)y[e], dot);
+    }
+    const float lse = LSE[stat];
+    own = float2v{lse == -INFINITY ? -INFINITY : -lse * 1.44269504f, -(dot + __shfl_xor(dot, 32))};
+  }
   const float addend = qw + ln < Seff ? own[0] : -INFINITY, ndelta = own[1];
   const float scale2 = scale * 1.44269504f;
 
@@ -1168,7 +1215,7 @@ template <int D, bool VARLEN>
 __global__ __launch_bounds__(fa::NTB, D == 64 ? 3 : 2) void fa_bwd_kernel(
     const unsigned short* __restrict__ Q, const unsigned short* __restrict__ K,
     const unsigned short* __restrict__ V, const unsigned short* __restrict__ dO,
-    const float2v* __restrict__ STATS,
+    const float2v* __restrict__ STATS, const unsigned short* __restrict__ O, const float* __restrict__ LSE,
     unsigned short* __restrict__ dQ, unsigned short* __restrict__ dK, unsigned short* __restrict__ dV,
     float* __restrict__ PART, int GS, const int* __restrict__ CU, const int* __restrict__ CUK,
     long qbs, long qts, long kbs, long kts, long dqbs, long dqts, long dkbs, long dkts,
@@ -1177,10 +1224,10 @@ __global__ __launch_bounds__(fa::NTB, D == 64 ? 3 : 2) void fa_bwd_kernel(
   const int f = (int)(blockIdx.y * gridDim.x + blockIdx.x);   // more than one grid row only beyond 2^23 blocks
   if (f >= n_kv + n_q) return;
   if (f < n_kv)
-    bwd_dkdv<D, VARLEN>(smem, f, n_kv, Q, K, V, dO, STATS, dK, dV, PART, GS, CU, CUK, qbs, qts, kbs, kts, dkbs, dkts,
+    bwd_dkdv<D, VARLEN>(smem, f, n_kv, Q, K, V, dO, STATS, O, LSE, dK, dV, PART, GS, CU, CUK, qbs, qts, kbs, kts, dkbs, dkts,
                         kv_tiles, B, S, Sk, Hq, Hkv, scale, causal, W, dealt);
   else
-    bwd_dq<D, VARLEN>(smem, f - n_kv, n_q, Q, K, V, dO, STATS, dQ, CU, CUK, qbs, qts, kbs, kts,
+    bwd_dq<D, VARLEN>(smem, f - n_kv, n_q, Q, K, V, dO, STATS, O, LSE, dQ, CU, CUK, qbs, qts, kbs, kts,
                       dqbs, dqts, q_tiles, B, S, Sk, Hq, Hkv, scale, causal, W, dealt);
 }
 
@@ -1380,8 +1427,8 @@ namespace {
 // The backward launch of dense (VARLEN = false) and packed batches. `seqs` sequences of at most S_max queries and
 // Sk_max keys; S, Sk are the extents the kernels index with (tokens of the whole batch when packed).
 template <int D, bool VARLEN>
-void launch_bwd(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, const at::Tensor& dout, const at::Tensor& stats,
-                at::Tensor& dq, at::Tensor& dk, at::Tensor& dv, const int* cu, const int* cuk,
+void launch_bwd(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, const at::Tensor& dout, const at::Tensor& out,
+                const at::Tensor& lse, at::Tensor& dq, at::Tensor& dk, at::Tensor& dv, const int* cu, const int* cuk,
                 long qbs, long qts, long kbs, long kts, long dqbs, long dqts, long dkbs, long dkts, int seqs, int S_max,
                 int Sk_max, int S, int Sk, int Hq, int Hkv, float scale, bool causal, hipStream_t stream) {
   using namespace fa;
@@ -1415,12 +1462,27 @@ void launch_bwd(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, c
   const long n_kv = dealt ? (dealt_blocks(dealt, each * Hkv * gs) + 7) / 8 * 8 : ((long)kv_tiles * seqs * Hkv * gs + 7) / 8 * 8;
   const long n_q = dealt ? dealt_blocks(dealt, each * Hq) : (long)q_tiles * seqs * Hq, blocks = n_kv + n_q;
   TORCH_CHECK(blocks < (1L << 31) - (1L << 23), "flash_attn_bwd: too many tiles");
+  // Where all blocks run at once and have few query tiles they form the rows' statistics themselves: one launch and one tensor less for the host, which
+  // bounds such calls (B8 S197 H12 D64, forward and backward through autograd: 75.9 -> 69.3 us); on the device B8 S197 H12 15.5 -> 14.7, B8 S250 H8 14.6 -> 14.5,
+  // B4 S128 H12 10.7 -> 9.6, but B2 S512 H8 (16 tiles) 19 -> 22. With 128 channels B2 S256 H4 16.2 -> 19.9, B3 S100 H6/3 16.2 -> 19.4.
+  const bool own = CAN_OWN<D, VARLEN> && blocks <= 512 && (long)((S_max + 31) / 32) * ((G + gs - 1) / gs) <= OWN_TILES &&
+                   reinterpret_cast<uintptr_t>(out.data_ptr()) % 16 == 0;
+  at::Tensor stats;
+  if (!own) {   // (pad rows of O are zero -> delta 0)
+    stats = at::empty({lse.numel(), 2}, lse.options());
+    const long all = out.numel() / D;
+    hipLaunchKernelGGL(fa_delta_kernel, dim3(capped_grid((all + 15) / 16, 4096)), dim3(256), 0, stream,
+                       (const unsigned short*)dout.data_ptr(), (const unsigned short*)out.data_ptr(),
+                       lse.data_ptr<float>(), (float2v*)stats.data_ptr(), all, S, Hq, D);
+    HIP_CHECK_LAST();
+  }
   auto kernel = fa_bwd_kernel<D, VARLEN>;
-  set_lds_limit((const void*)kernel, bwd_lds<D>());
-  hipLaunchKernelGGL(kernel, wide_grid(blocks), dim3(NTB), bwd_lds<D>(), stream,
+  const size_t lds = bwd_lds<D>() + (own ? OWN_TILES * 256 : 0);
+  set_lds_limit((const void*)kernel, lds);
+  hipLaunchKernelGGL(kernel, wide_grid(blocks), dim3(NTB), lds, stream,
                      (const unsigned short*)q.data_ptr(), (const unsigned short*)k.data_ptr(),
                      (const unsigned short*)v.data_ptr(), (const unsigned short*)dout.data_ptr(),
-                     (const float2v*)stats.data_ptr(), (unsigned short*)dq.data_ptr(), (unsigned short*)dk.data_ptr(),
+                     own ? nullptr : (const float2v*)stats.data_ptr(), (const unsigned short*)out.data_ptr(), lse.data_ptr<float>(), (unsigned short*)dq.data_ptr(), (unsigned short*)dk.data_ptr(),
                      (unsigned short*)dv.data_ptr(), gs > 1 ? part.data_ptr<float>() : nullptr, gs, cu, cuk, qbs, qts, kbs,
                      kts, dqbs, dqts, dkbs, dkts, (int)n_kv, (int)n_q, kv_tiles, q_tiles, seqs, S, Sk, Hq, Hkv, scale, causal ? 1 : 0,
                      rows_together(G, Sk_max * D * 4L), (int)dealt);
@@ -1472,20 +1534,10 @@ std::vector<at::Tensor> flash_attn_bwd(at::Tensor dout, at::Tensor q, at::Tensor
   check_fa_view(dq, "dq");
   check_fa_view(dk, "dk");
   TORCH_CHECK(dk.strides() == dv.strides(), "flash_attn_bwd: dk/dv strides must match");
-  auto stats = at::empty({B, Hq, S, 2}, q.options().dtype(at::kFloat));
   auto stream = at::hip::getCurrentHIPStream();
 
-  {  // what the rows add (pad rows of O are zero -> delta 0)
-    const long rows = (long)B * S * Hq;
-    const int grid = capped_grid((rows + 15) / 16, 4096);
-    hipLaunchKernelGGL(fa_delta_kernel, dim3(grid), dim3(256), 0, stream.stream(),
-                       (const unsigned short*)dout.data_ptr(), (const unsigned short*)out.data_ptr(),
-                       lse.data_ptr<float>(), (float2v*)stats.data_ptr(), rows, S, Hq, D);
-    HIP_CHECK_LAST();
-  }
-
 #define LAUNCH_BWD(DD)                                                                                               \
-  launch_bwd<DD, false>(q, k, v, dout, stats, dq, dk, dv, cu, cuk, q.stride(0), q.stride(1), k.stride(0), k.stride(1), \
+  launch_bwd<DD, false>(q, k, v, dout, out, lse, dq, dk, dv, cu, cuk, q.stride(0), q.stride(1), k.stride(0), k.stride(1), \
                         dq.stride(0), dq.stride(1), dk.stride(0), dk.stride(1), B, S, Sk, S, Sk, Hq, Hkv, (float)scale,      \
                         causal, stream.stream())
   if (D == 128) LAUNCH_BWD(128);
@@ -1509,20 +1561,10 @@ std::vector<at::Tensor> flash_attn_varlen_bwd(at::Tensor dout, at::Tensor q, at:
   auto dq = at::empty({T, Hq, D}, q.options());
   auto dk = at::empty({T, Hkv, D}, k.options());
   auto dv = at::empty({T, Hkv, D}, v.options());
-  auto stats = at::empty({Hq, T, 2}, q.options().dtype(at::kFloat));
   auto stream = at::hip::getCurrentHIPStream();
 
-  {  // what the rows add ([1, Hq, T] layout == [Hq, T])
-    const long rows = (long)T * Hq;
-    const int grid = capped_grid((rows + 15) / 16, 4096);
-    hipLaunchKernelGGL(fa_delta_kernel, dim3(grid), dim3(256), 0, stream.stream(),
-                       (const unsigned short*)dout.data_ptr(), (const unsigned short*)out.data_ptr(),
-                       lse.data_ptr<float>(), (float2v*)stats.data_ptr(), rows, T, Hq, D);
-    HIP_CHECK_LAST();
-  }
-
 #define LAUNCH_VBWD(DD)                                                                                              \
-  launch_bwd<DD, true>(q, k, v, dout, stats, dq, dk, dv, cu_seqlens.data_ptr<int>(), nullptr, 0L, q.stride(0), 0L,     \
+  launch_bwd<DD, true>(q, k, v, dout, out, lse, dq, dk, dv, cu_seqlens.data_ptr<int>(), nullptr, 0L, q.stride(0), 0L,     \
                        k.stride(0), 0L, dq.stride(0), 0L, dk.stride(0), n_seq, (int)max_seqlen, (int)max_seqlen, T, T, Hq,  \
                        Hkv, (float)scale, causal, stream.stream())
   if (D == 128) LAUNCH_VBWD(128);

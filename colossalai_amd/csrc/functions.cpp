@@ -90,9 +90,8 @@ struct FlashAttention : torch::autograd::Function<FlashAttention> {
   }
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
     const auto s = ctx->get_saved_variables();
-    const at::Tensor fresh = at::empty({0}, s[0].options());
     auto r = flash_attn_bwd(grads[0].contiguous(), s[0], s[1], s[2], s[3], s[4], ctx->saved_data["causal"].toBool(),
-                            ctx->saved_data["scale"].toDouble(), fresh, fresh, fresh, maybe(s[5]), maybe(s[6]));
+                            ctx->saved_data["scale"].toDouble(), none, none, none, maybe(s[5]), maybe(s[6]));
     return {r[0], r[1], r[2], none, none, none, none};
   }
 };

@@ -258,6 +258,27 @@ def test_packed_tiles_by_lookup(lens, H, G, causal):
         _near(x, y, name)
 
 
+@pytest.mark.parametrize("causal", [True, False])
+# at least 20 keys: of two, a row's dq is one difference of dout · v and dout · out, whose roundings (2^-9 of about sqrt(D) each) are not small beside it
+@pytest.mark.parametrize("S,H,G", [(20, 2, 2), (63, 4, 1), (64, 4, 1), (65, 4, 1), (255, 3, 3), (256, 2, 2), (257, 2, 2)])
+def test_statistics_of_few_rows(S, H, G, causal):
+    """64 channels, up to 8 tiles of 32 query rows a block: the backward's blocks form -lse and -delta themselves. Padded sequences too, one of them empty."""
+    from colossalai_amd.ops import flash_attention
+
+    q, k, v, dout = _inputs(3, S, H, G, 64, S)
+    lens = [S, max(20, S - 40), 0]
+    a = [t.clone().requires_grad_() for t in (q, k, v)]
+    o = flash_attention(*a, causal=causal, seqlens=torch.tensor(lens, dtype=torch.int32, device="cuda"))
+    got = [o] + list(torch.autograd.grad(o, a, dout))
+    for b, n in enumerate(lens):
+        for x in got:
+            assert not x[b, n:].any()
+        if n:
+            want = _reference(*(t[b: b + 1, :n] for t in (q, k, v, dout)), causal, 0.125)
+            for name, x, y in zip(("out", "dq", "dk", "dv"), got, want):
+                _near(x[b: b + 1, :n], y, name)
+
+
 @pytest.mark.parametrize("H", [31, 32, 33])
 @pytest.mark.parametrize("D,causal", [(64, True), (128, False)])
 @pytest.mark.parametrize("packed", [False, True])
