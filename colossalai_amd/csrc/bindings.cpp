@@ -38,6 +38,7 @@ at::Tensor ce_loss(at::Tensor nll, at::Tensor labels, int64_t ignore_index);
 
 // products.hip
 at::Tensor multiply(const at::Tensor& x, const at::Tensor& w, bool slow);
+at::Tensor embedding(const at::Tensor& tokens, const at::Tensor& weight);
 at::Tensor weight_grad(const at::Tensor& dy, const at::Tensor& x, const c10::optional<at::Tensor>& add, bool keep);
 
 // linear.cpp
@@ -138,6 +139,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("dy"), py::arg("x"), py::arg("add") = py::none(), py::arg("keep") = false);
   m.def("multiply", &cai::multiply, "x [M, K] times w [N, K]^T, or with `slow` times w [K, N]");
   m.def("linear", &cai::linear, "linear layer without bias, its weight gradient by weight_grad");
+  m.def("embedding", &cai::embedding, "rows of a table by tokens, with the table's gradient from embedding.hip");
   m.def("native_rms_norm", &cai::native_rms_norm, "autograd functions of the kernels above and below; None: use the Python one");
   m.def("native_fused_add_rms_norm", &cai::native_fused_add_rms_norm);
   m.def("native_swiglu", &cai::native_swiglu);

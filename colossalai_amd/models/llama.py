@@ -26,7 +26,7 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from ..ops import build_rope_table, fused_add_rms_norm, fused_rope_attention, rms_norm, swiglu
-from ..ops.linear import project
+from ..ops.linear import embed, project
 
 from .registry import register_model
 
@@ -457,7 +457,7 @@ class LlamaModel(nn.Module):
         is_last = end == len(self.layers)
         if is_first:
             assert input_ids is not None
-            residual = self.embed_tokens(input_ids)
+            residual = embed(self.embed_tokens, input_ids)
             device = input_ids.device
             if getattr(self, "sp_split_gather_group", None) is not None:
                 # Megatron-style SP: the residual stream lives on seq shards;

@@ -1,5 +1,5 @@
 """Linear layers in training: the weight gradient and small products of a plain bfloat16 ``nn.Linear`` by
-csrc/products.hip.
+csrc/products.hip, the table's gradient of a plain ``nn.Embedding`` by csrc/embedding.hip.
 
 The layer stays an ``nn.Linear`` that parallel policies, LoRA or the zero-bubble schedule replace or change; ``project``
 calls whatever it has become.
@@ -13,7 +13,7 @@ from torch.nn.modules import module as _hooks
 
 from ._kernels import kernels
 
-__all__ = ["multiply", "project", "weight_grad"]
+__all__ = ["embed", "multiply", "project", "weight_grad"]
 
 
 def multiply(x: torch.Tensor, w: torch.Tensor, slow: bool = False) -> torch.Tensor:
@@ -50,3 +50,16 @@ def project(layer: nn.Module, x: torch.Tensor) -> torch.Tensor:
                 and weight.device == x.device and _bare(layer) and not torch._C._len_torch_function_stack()):
             return kernels().linear(x, weight)
     return layer(x)
+
+
+def embed(layer: nn.Module, tokens: torch.Tensor) -> torch.Tensor:
+    """``layer(tokens)``. Plain bfloat16 tables that are trained take the native form, others are called, as in ``project``; so are
+    tables of less than 2^20 elements, whose gradients the host bounds either way (1024 rows of 512, 512 tokens: 41 us both)."""
+    if (type(layer) is nn.Embedding and type(tokens) is torch.Tensor and tokens.is_cuda and tokens.dtype is torch.int64
+            and not torch.compiler.is_compiling() and torch.is_grad_enabled()):
+        weight = layer.weight
+        if (layer.padding_idx is None and layer.max_norm is None and not layer.scale_grad_by_freq and not layer.sparse
+                and type(weight) is nn.Parameter and weight.numel() >= 1 << 20 and weight.requires_grad and weight.dtype is torch.bfloat16
+                and weight.device == tokens.device and _bare(layer) and not torch._C._len_torch_function_stack()):
+            return kernels().embedding(tokens, weight)
+    return layer(tokens)
