@@ -1452,23 +1452,38 @@ void launch_bwd(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, c
   const int rows = NWB * QW;
   const int kv_tiles = (Sk_max + rows - 1) / rows, q_tiles = (S_max + rows - 1) / rows;
   const int G = Hq / Hkv;
-  // Blocks that share a tile's group of heads (GS; the heads need not divide evenly). All 512 blocks that fit on the chip at
-  // once start together, and under a causal mask the first tile then takes twice the average: B1 S8192, 32 over 8 heads, runs
-  // 2194 us with one block a tile (512 blocks), 2077 with two and 2110 with four (more partial sums). So a block's heads
-  // are halved while there are at most 1024 blocks (71 over 1 head of 64, B1 S8192: 21.5 ms undivided, 2.57 at 15 blocks a
-  // tile, 2.66 at 71; 28 over 4 of 128, B2 S8192: 3.68, 3.54 at two, 3.59 at seven). Without a mask the work is even and it
-  // only matters that every CU has a block; a second one each pays where a block keeps 128 steps of 32 query rows (16 over 2 of
+  // Blocks that share a tile's group of heads (GS; the heads need not divide evenly).
+  // Under a causal mask the first tile takes twice the average, and what is left of it when all else is done runs almost alone. The time by GS, in steps
+  // of 32 query rows by 128 keys: all blocks' over the 512 that run at once (768 with 64 channels), the dQ part's 3/4 of a step included and 6 steps around
+  // each block, at 1.75 us (1.65); what the longest takes beyond that at 1.12; the partial sums, written and read at 4.8 TB/s, and their launch. Packed
+  // batches are taken to be half as long as their longest on average, or T / sequences. us, GS 1, 2, 4, * chosen: B1 S8192 H32/8 D128 1748, 1731 *, -;
+  // B1 S4096 635, 462 *, 472; B2 S4096 894 *, 914, 952; B4 S2048 H16/4 332, 259 *, 272; D64 B1 S8192 H16/4 821, 564, 501 *; B2 S4096 H32/8 582, 508 *, 522;
+  // packed 43 of up to 1024, H8/2 D128 175, 122 *, 146; 64 of 900 158, 116 *, 141; 85 of 512, H16/4 D64 96 *, 114, 139; 12 of 2048, H32/8 374, 364 *, 415.
+  // Without a mask the work is even and it only matters that every CU has a block; a second one each pays where a block keeps 128 steps (16 over 2 of
   // 64, B1 S8192: 1413 -> 1134; 8 over 4 of 64, B16 S512: 58 -> 67). A block keeps at least 16 steps, of its heads' full length, or the
   // sums cost more than they save. The float32 sums take 8 bytes for each channel of these blocks' 128 rows: 134 MB at most.
   const long kv_blocks = (VARLEN ? (Sk + rows - 1) / rows : (long)kv_tiles * seqs) * Hkv;
   const bool sums_ok = dk.stride(-3) % 4 == 0 && (VARLEN || dk.stride(0) % 4 == 0) &&
                        reinterpret_cast<uintptr_t>(dk.data_ptr()) % 8 == 0 && reinterpret_cast<uintptr_t>(dv.data_ptr()) % 8 == 0;
+  const double tokens = VARLEN ? S : (double)seqs * S, length = VARLEN ? std::max(tokens / std::max(seqs, 1), 0.5 * S_max) : S_max;
+  const double tiles = VARLEN ? tokens / rows + 0.5 * seqs : (double)q_tiles * seqs;
+  auto causal_us = [&](int d) {
+    const double all = (1.75 * Hq * tokens / rows * (length / 64 + 2) + 6 * tiles * (Hq + (double)Hkv * d)) / (D == 64 ? 768 : 512);
+    const double longest = (double)((S_max + 31) / 32) * ((G + d - 1) / d) + 6;
+    return (D == 64 ? 1.65 : 1.75) * all + 1.12 * std::max(0.0, longest - all) + (d > 1 ? 3 + 16.0 * d * tokens * Hkv * D / 4.8e6 : 0.0);
+  };
   int gs = 1;
+  double us = causal ? causal_us(1) : 0.0;
   for (int most = G; most > 1 && sums_ok;) {
     most = (most + 1) / 2;                     // heads of a block, and blocks that take
     const int d = (G + most - 1) / most;
     const long steps = (long)((S_max + 31) / 32) * (G / d);
     if (steps < 16 || kv_blocks * d > (causal ? 1024 : steps >= 128 ? 512 : 510)) break;
+    if (causal) {
+      const double by_d = causal_us(d);
+      if (by_d >= us) continue;
+      us = by_d;
+    }
     gs = d;
   }
   const long n_part = (VARLEN ? (long)Sk : (long)seqs * Sk) * Hkv * D;
