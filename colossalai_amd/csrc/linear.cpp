@@ -9,6 +9,7 @@ namespace cai {
 at::Tensor weight_grad(const at::Tensor& dy, const at::Tensor& x, const c10::optional<at::Tensor>& add, bool keep);
 bool weight_grad_serves(const at::Tensor& dy, const at::Tensor& x);
 at::Tensor multiply(const at::Tensor& x, const at::Tensor& w, bool slow);
+std::vector<at::Tensor> linear_grads(const at::Tensor& dy, const at::Tensor& w, const at::Tensor& x);
 
 namespace {
 
@@ -32,6 +33,10 @@ struct Linear : torch::autograd::Function<Linear> {
     at::Tensor dx, dw;
     // a backward that is part of a graph itself (create_graph), or that something watches, takes operations it can see
     const bool closed = !at::GradMode::is_enabled() && plain_here(dy2);
+    if (closed && ctx->needs_input_grad(0) && ctx->needs_input_grad(1) && plain_here(weight) && plain_here(x)) {
+      const auto both = linear_grads(dy2, weight, x.reshape({-1, x.size(-1)}));
+      if (!both.empty()) return {both[0].view(x.sizes()), both[1]};
+    }
     if (ctx->needs_input_grad(0)) dx = (closed && plain_here(weight) ? multiply(dy2, weight, true) : at::mm(dy2, weight)).view(x.sizes());
     if (ctx->needs_input_grad(1)) {
       const at::Tensor x2 = x.reshape({-1, x.size(-1)});

@@ -20,8 +20,9 @@
 //   32000, 4096, 4096     940 -> 893 -> 806       32000, 768, 8192     462 -> 347 -> 320        4096, 768, 8192      77 -> 59 -> 56
 //   768, 2048, 8192        62 -> 36 -> 34         768, 768, 8192        48 -> 21 -> 19          3072, 1024, 2048     24 -> 22 -> 19
 // Small others, back to back (the library's call takes the host 19 to 20 us, its kernels 5 to 11), with the products of 32 x 32 x 16:
-//   x W^T: 512, 1536, 512   19.2 -> 9.0   512, 512, 1024   19.7 -> 11.4     dy W: 512, 512, 2048   19.2 -> 13.9
-// Large ones stay with the library: 16384, 12288, 4096   1048 us there, 1490 here (its rows are read 64 bytes at a time); dy W 16384, 4096, 12288   1265, 1310.
+//   x W^T: 512, 1536, 512   19.2 -> 9.0   512, 512, 1024   19.7 -> 11.4     dy W: 512, 512, 2048   19.2 -> 13.9 (with the weight gradient: linear_grads)
+// Large ones stay with the library: 16384, 12288, 4096   1048 us there, 1490 here (its rows are read 64 bytes at a time); dy W 16384, 4096, 12288   1181 there, 1255
+// here with the present products, 16384, 4096, 22016   2122, 2130, 16384, 11008, 4096   1192, 1144, 8192, 768, 4096   59, 59.
 #include <torch/extension.h>
 #include <ATen/hip/HIPContext.h>
 #include <c10/hip/HIPGuard.h>
@@ -189,10 +190,9 @@ struct Places {
   }
 };
 
-// STEPS steps lie in LDS: one in use, one arrived, the others on their way.
+// Block f of `blocks`. STEPS steps lie in LDS: one in use, one arrived, the others on their way.
 template <bool PC, bool QC, int TM, int TN, int STEPS>
-__global__ __launch_bounds__(256, TM == 256 ? 1 : 2) void product_kernel(const Args a) {
-  extern __shared__ char smem[];
+DEV_INLINE void product_block(const Args& a, char* smem, int f, int blocks) {
   constexpr int FA = TN / 32, FB = TM / 32;      // fragments of a wave
   constexpr int YB = Operand<PC, TM>::BYTES, SB = YB + Operand<QC, TN>::BYTES;
   constexpr int PY = Operand<PC, TM>::PER, PER = PY + Operand<QC, TN>::PER;
@@ -200,11 +200,11 @@ __global__ __launch_bounds__(256, TM == 256 ? 1 : 2) void product_kernel(const A
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wm = w & 1, wn = w >> 1;
 
-  int f = blockIdx.x, tile, part = -1, k0 = 0, k1 = a.K;
+  int tile, part = -1, k0 = 0, k1 = a.K;
   if (f < a.full) {
     tile = xcd_chunk(f, a.full);
   } else {
-    f = xcd_chunk(f - a.full, (int)gridDim.x - a.full);
+    f = xcd_chunk(f - a.full, blocks - a.full);
     const int rest = a.tiles_m * a.tiles_n - a.full;
     part = f / rest;
     tile = a.full + f % rest;
@@ -325,6 +325,20 @@ __global__ __launch_bounds__(256, TM == 256 ? 1 : 2) void product_kernel(const A
   }
 }
 
+template <bool PC, bool QC, int TM, int TN, int STEPS>
+__global__ __launch_bounds__(256, TM == 256 ? 1 : 2) void product_kernel(const Args a) {
+  extern __shared__ char smem[];
+  product_block<PC, QC, TM, TN, STEPS>(a, smem, blockIdx.x, gridDim.x);
+}
+
+// dY W (n blocks) and a weight gradient (the others) together
+__global__ __launch_bounds__(256, 2) void product_pair_kernel(const Args dx, const Args dw, int n) {
+  extern __shared__ char smem[];
+  const int f = blockIdx.x;
+  if (f < n) product_block<false, true, 128, 128, 4>(dx, smem, f, n);
+  else product_block<true, true, 128, 128, 4>(dw, smem, f - n, (int)gridDim.x - n);
+}
+
 // sums the parts of the tiles that were cut
 template <int TM, int TN>
 __global__ __launch_bounds__(256) void product_sum_kernel(const Args a) {
@@ -392,10 +406,18 @@ bool loadable(const at::Tensor& t) {
       && reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0;
 }
 
-template <bool PC, bool QC>
-at::Tensor run(const at::Tensor& p, const at::Tensor& q, Plan plan, const c10::optional<at::Tensor>& add, bool keep) {
-  const c10::hip::HIPGuard guard(p.device().index());
+// what a launch takes, with its result and the sums' place
+struct Call {
   Args a{};
+  at::Tensor out, ws;
+  int rest;
+  int blocks() const { return a.full + rest * a.parts; }
+};
+
+template <bool PC, bool QC>
+Call call(const at::Tensor& p, const at::Tensor& q, const Plan& plan, const c10::optional<at::Tensor>& add, bool keep) {
+  Call c;
+  Args& a = c.a;
   a.p = reinterpret_cast<const unsigned short*>(p.data_ptr());
   a.q = reinterpret_cast<const unsigned short*>(q.data_ptr());
   a.ldp = p.stride(0);
@@ -409,15 +431,22 @@ at::Tensor run(const at::Tensor& p, const at::Tensor& q, Plan plan, const c10::o
   a.part_k = ((a.K + plan.parts - 1) / plan.parts + KT - 1) / KT * KT;
   a.parts = (a.K + a.part_k - 1) / a.part_k;
   if (add) a.add = add->data_ptr<float>();
-  at::Tensor out = keep && add ? *add : at::empty({a.M, a.N}, p.options().dtype(keep ? at::kFloat : at::kBFloat16));
-  if (keep) a.sum = out.data_ptr<float>();
-  else a.out = reinterpret_cast<unsigned short*>(out.data_ptr());
-  at::Tensor ws;
-  const long rest = (long)a.tiles_m * a.tiles_n - a.full;
-  if (rest) {
-    ws = at::empty({rest * a.parts * plan.tm * plan.tn}, p.options().dtype(at::kFloat));
-    a.ws = ws.data_ptr<float>();
+  c.out = keep && add ? *add : at::empty({a.M, a.N}, p.options().dtype(keep ? at::kFloat : at::kBFloat16));
+  if (keep) a.sum = c.out.data_ptr<float>();
+  else a.out = reinterpret_cast<unsigned short*>(c.out.data_ptr());
+  c.rest = a.tiles_m * a.tiles_n - a.full;
+  if (c.rest) {
+    c.ws = at::empty({(long)c.rest * a.parts * plan.tm * plan.tn}, p.options().dtype(at::kFloat));
+    a.ws = c.ws.data_ptr<float>();
   }
+  return c;
+}
+
+template <bool PC, bool QC>
+at::Tensor run(const at::Tensor& p, const at::Tensor& q, Plan plan, const c10::optional<at::Tensor>& add, bool keep) {
+  const c10::hip::HIPGuard guard(p.device().index());
+  const Call c = call<PC, QC>(p, q, plan, add, keep);
+  const Args& a = c.a;
   const auto stream = at::hip::getCurrentHIPStream();
   if constexpr (PC) {
     if (plan.tn == 256) launch<PC, QC, 256, 256, 4>(a, stream);
@@ -427,7 +456,7 @@ at::Tensor run(const at::Tensor& p, const at::Tensor& q, Plan plan, const c10::o
     launch<PC, QC, 128, 128, 4>(a, stream);
   }
   HIP_CHECK_LAST();
-  return out;
+  return c.out;
 }
 
 // bfloat16 matrices on one device that nothing watches: a mode that counts or rewrites operations is to see the library's products
@@ -476,16 +505,42 @@ at::Tensor weight_grad(const at::Tensor& dy, const at::Tensor& x, const c10::opt
 // are no faster, 6 to 13 us where the library's kernels take 4 to 11. Steps of two layers, us, library and here: width 512, 512 tokens 1320
 // and 1050 (kernels 490 and 525); 1024, 512 tokens 1130 and 900; where the device is the bound nothing shows: 512, 4096 tokens 1316 and
 // 1301, 1024, 2048 tokens 1343 and 1347.
-at::Tensor multiply(const at::Tensor& x, const at::Tensor& w, bool slow) {
+static bool small_product(const at::Tensor& x, const at::Tensor& w, bool slow, pr::Plan& plan) {
   if (pr::bf16_pair(x, w) && x.size(1) == w.size(slow ? 0 : 1) && x.size(1) % pr::KT == 0 && w.size(slow ? 1 : 0) % 8 == 0
       && pr::loadable(x) && pr::loadable(w)) {
     const long M = x.size(0), N = w.size(slow ? 1 : 0), K = x.size(1);
     if (((M + 127) / 128) * ((N + 127) / 128) <= 256) {
-      const pr::Plan plan = pr::plan(M, N, K, true);
-      if (plan.us <= 15.0) return slow ? pr::run<false, true>(x, w, plan, c10::nullopt, false) : pr::run<false, false>(x, w, plan, c10::nullopt, false);
+      plan = pr::plan(M, N, K, true);
+      return plan.us <= 15.0;
     }
   }
+  return false;
+}
+
+at::Tensor multiply(const at::Tensor& x, const at::Tensor& w, bool slow) {
+  pr::Plan plan;
+  if (small_product(x, w, slow, plan)) return slow ? pr::run<false, true>(x, w, plan, c10::nullopt, false) : pr::run<false, false>(x, w, plan, c10::nullopt, false);
   return slow ? at::mm(x, w) : at::mm(x, w.t());
+}
+
+// Both gradients of a small linear layer, dy [K, M] times w [M, N] and dy^T x with x [K, N], by one launch; empty where one of them is not small. Neither
+// fills the chip, and the host takes some 4 us for a launch, of which a step of two layers has eight less. Such steps' kernels, us: width 512, 512 tokens
+// 504 -> 441; 256, 2000 tokens 608 -> 553; 512, 2800 tokens 748 -> 720; 1024, 600 tokens 682 -> 654.
+std::vector<at::Tensor> linear_grads(const at::Tensor& dy, const at::Tensor& w, const at::Tensor& x) {
+  pr::Plan dx_plan;
+  if (!small_product(dy, w, true, dx_plan) || !weight_grad_serves(dy, x) || !pr::loadable(x)
+      || (dy.size(0) < 1600 && dy.size(1) * x.size(1) > (1L << 23))) return {};
+  const pr::Plan dw_plan = pr::plan(dy.size(1), x.size(1), dy.size(0), false);
+  if (dw_plan.tm != 128 || dw_plan.us > 25.0) return {};
+  const c10::hip::HIPGuard guard(dy.device().index());
+  const pr::Call dx = pr::call<false, true>(dy, w, dx_plan, c10::nullopt, false), dw = pr::call<true, true>(dy, x, dw_plan, c10::nullopt, false);
+  const auto stream = at::hip::getCurrentHIPStream();
+  constexpr int LDS = (128 + 128) * pr::KT * 2 * 4;
+  pr::product_pair_kernel<<<dx.blocks() + dw.blocks(), 256, LDS, stream>>>(dx.a, dw.a, dx.blocks());
+  if (dx.rest) pr::product_sum_kernel<128, 128><<<dx.rest * 16, 256, 0, stream>>>(dx.a);
+  if (dw.rest) pr::product_sum_kernel<128, 128><<<dw.rest * 16, 256, 0, stream>>>(dw.a);
+  HIP_CHECK_LAST();
+  return {dx.out, dw.out};
 }
 
 }  // namespace cai

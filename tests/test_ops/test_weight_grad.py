@@ -128,6 +128,25 @@ def test_products_against_64_bits(M, N, K):
     assert got[M // 2].isnan().all() and got.isnan().sum() == N
 
 
+# both of a small layer's gradients by one launch: either whole, cut in parts, with remainders; the last two are too large for it
+@pytest.mark.gpu
+@pytest.mark.parametrize("K,M,N,one", [(1, 32, 8, True), (127, 96, 136, True), (512, 2048, 512, True), (512, 1536, 512, True), (2000, 256, 520, True),
+                                       (33, 4096, 264, True), (4096, 64, 128, True), (500, 4096, 4096, False), (512, 24, 64, False)])
+def test_both_gradients_of_a_small_layer(K, M, N, one):
+    torch.manual_seed(M + N + K)
+    x, w, dy = (torch.randn(*s, device="cuda").to(BF16) for s in ((K, N), (M, N), (K, M)))
+    x.requires_grad_(), w.requires_grad_()
+    out = kernels().linear(x, w)
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CUDA]) as seen:
+        dx, dw = torch.autograd.grad(out, (x, w), dy)
+        torch.cuda.synchronize()
+    assert any("product_pair" in e.key for e in seen.key_averages()) == one
+    _close(dw, dy, x.detach())
+    _close(dx, dy.t(), w.detach())
+    only = torch.autograd.grad(kernels().linear(x, w), x, dy)[0]
+    _close(only, dy.t(), w.detach())
+
+
 def _step(call, x, w, g):
     x, w = x.detach().requires_grad_(), w.detach().requires_grad_()
     y = call(x, w)
