@@ -380,12 +380,13 @@ struct Plan {
 // 768 x 2048 x 8192: 161 / 46, 43, 83 / 50; 768 x 768 x 8192: 161 / 35, 28, 78 / 26; 32000 x 768 x 8184: 377 / 342, 410 (whole), 498; 3072 x 1024 x
 // 2048: 60 / 37, 32, 28 / 33; 6144 x 2048 x 4096: 106 / 127, 130 (whole), 121 / 133; and the same product over and over: 22016 x 4096 x 16384:
 // 2174 / 2056, 2746, 3237; 4096 x 11008 x 16384: 1050 / 1105, 1217 (whole), 1969 / 1708.
-Plan plan(long M, long N, long K, bool small_only) {
+// Small products (`small`) have 128 x 128 tiles, operands from near, 0.25 us a step and 5 around, and sums that a launch behind them waits for, 5 TB/s.
+Plan plan(long M, long N, long K, bool small) {
   struct { int tm, tn; double step, around; long slots; bool one_round; } forms[] = {
-      {256, 256, 0.705, 16.0, 256, false}, {256, 128, 0.40, 11.0, 256, true}, {128, 128, 0.27, 6.0, 512, false}};
+      {256, 256, 0.705, 16.0, 256, false}, {256, 128, 0.40, 11.0, 256, true}, {128, 128, small ? 0.25 : 0.27, small ? 5.0 : 6.0, 512, false}};
   Plan best{0, 0, 0, 1, 0.0};
   for (const auto& form : forms) {
-    if (small_only && form.tm != 128) continue;
+    if (small && form.tm != 128) continue;
     const long tiles = ((M + form.tm - 1) / form.tm) * ((N + form.tn - 1) / form.tn), steps = (K + KT - 1) / KT;
     if (form.one_round && tiles > 256) continue;
     auto take = [&](long full, long parts, double us) {
@@ -395,7 +396,7 @@ Plan plan(long M, long N, long K, bool small_only) {
     take(tiles, 1, round(tiles, steps));
     const long full = tiles / form.slots * form.slots, rest = tiles - full;
     for (long p = 2; rest && p * rest <= (form.one_round ? 256 : 512) && p * 8 <= steps; ++p)
-      take(full, p, round(full, steps) + round(rest * p, (steps + p - 1) / p) + 3.0 + rest * p * form.tm * form.tn * 8 / 10e6);
+      take(full, p, round(full, steps) + round(rest * p, (steps + p - 1) / p) + 3.0 + rest * p * form.tm * form.tn * 8 / (small ? 5e6 : 10e6));
   }
   return best;
 }
@@ -500,9 +501,11 @@ at::Tensor weight_grad(const at::Tensor& dy, const at::Tensor& x, const c10::opt
                              pr::loadable(x) ? x : x.clone(at::MemoryFormat::Contiguous), plan, add, keep);
 }
 
-// x [M, K] times w [N, K]^T, or with `slow` times w [K, N]. Products that should take at most 15 us by the plan are formed here, because the host
+// x [M, K] times w [N, K]^T, or with `slow` times w [K, N]. Products that should take at most 14 us by the plan are formed here, because the host
 // takes 19 to 20 us for the library's call and 9 for this one, and a chain of such products waits for it. On the device they
-// are no faster, 6 to 13 us where the library's kernels take 4 to 11. Steps of two layers, us, library and here: width 512, 512 tokens 1320
+// are no faster, 6 to 13 us where the library's kernels take 4 to 11. Where the line lies, us in a chain and from a graph, here and there: 512, 3072, 1152
+// (whole; here) 12.9 and 13.7, 18.7 and 11.2; 512, 1024, 2048 (cut; there) 14.8 and 15.0, 18.9 and 9.6; 256, 3072, 1536 (there) 15.7 and 16.0, 19.0 and 9.4.
+// Steps of two layers, us, library and here: width 512, 512 tokens 1320
 // and 1050 (kernels 490 and 525); 1024, 512 tokens 1130 and 900; where the device is the bound nothing shows: 512, 4096 tokens 1316 and
 // 1301, 1024, 2048 tokens 1343 and 1347.
 static bool small_product(const at::Tensor& x, const at::Tensor& w, bool slow, pr::Plan& plan) {
@@ -511,7 +514,7 @@ static bool small_product(const at::Tensor& x, const at::Tensor& w, bool slow, p
     const long M = x.size(0), N = w.size(slow ? 1 : 0), K = x.size(1);
     if (((M + 127) / 128) * ((N + 127) / 128) <= 256) {
       plan = pr::plan(M, N, K, true);
-      return plan.us <= 15.0;
+      return plan.us <= 14.0;
     }
   }
   return false;
