@@ -380,6 +380,8 @@ struct Plan {
 // 768 x 2048 x 8192: 161 / 46, 43, 83 / 50; 768 x 768 x 8192: 161 / 35, 28, 78 / 26; 32000 x 768 x 8184: 377 / 342, 410 (whole), 498; 3072 x 1024 x
 // 2048: 60 / 37, 32, 28 / 33; 6144 x 2048 x 4096: 106 / 127, 130 (whole), 121 / 133; and the same product over and over: 22016 x 4096 x 16384:
 // 2174 / 2056, 2746, 3237; 4096 x 11008 x 16384: 1050 / 1105, 1217 (whole), 1969 / 1708.
+// Many parts of few tiles are summed by few blocks, one part after the other: 0.15 us for each part of 128 x 128 tiles. us by parts, operands from memory: 168 x 352 x 9685:
+// 34 22.6, 22 19.9; 1328 x 72 x 5463: 19 19.8, 9 17.7; 208 x 480 x 14360: 30 26.6, 18 24.6; 368 x 1304 x 2893: 7 20.4, 4 19.5; 952 x 408 x 970: 3 13.1, whole 17.4.
 // Small products (`small`) have 128 x 128 tiles, operands from near, 0.25 us a step and 5 around, and sums that a launch behind them waits for, 5 TB/s.
 Plan plan(long M, long N, long K, bool small) {
   struct { int tm, tn; double step, around; long slots; bool one_round; } forms[] = {
@@ -396,7 +398,8 @@ Plan plan(long M, long N, long K, bool small) {
     take(tiles, 1, round(tiles, steps));
     const long full = tiles / form.slots * form.slots, rest = tiles - full;
     for (long p = 2; rest && p * rest <= (form.one_round ? 256 : 512) && p * 8 <= steps; ++p)
-      take(full, p, round(full, steps) + round(rest * p, (steps + p - 1) / p) + 3.0 + rest * p * form.tm * form.tn * 8 / (small ? 5e6 : 10e6));
+      take(full, p, round(full, steps) + round(rest * p, (steps + p - 1) / p) + 3.0 + rest * p * form.tm * form.tn * 8 / (small ? 5e6 : 10e6)
+                    + (form.tm == 128 && !small ? 0.15 * p : 0.0));
   }
   return best;
 }

@@ -1,5 +1,7 @@
 """Weight gradients and small products of linear layers (csrc/products.hip) and the layer that uses them (csrc/linear.cpp)."""
 
+import json
+
 import pytest
 import torch
 import torch.nn as nn
@@ -159,6 +161,22 @@ def test_which_products_are_small(M, N, K, own, slow):
         torch.cuda.synchronize()
     assert any("product_kernel" in e.key for e in seen.key_averages()) == own
     _close(y, x.t(), w if slow else w.t())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("K,M,N,most", [(9685, 168, 352, 22), (5463, 1328, 72, 9), (14360, 208, 480, 18), (11817, 552, 128, 25), (970, 952, 408, 3)])
+def test_parts_of_few_tiles(K, M, N, most, tmp_path):
+    """Each part costs the sum, which few tiles give to few blocks: up to half as many parts as their bytes alone would allow."""
+    dy, x = (torch.randn(K, n, device="cuda").to(BF16) for n in (M, N))
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CUDA]) as seen:
+        dw = kernels().weight_grad(dy, x)
+        torch.cuda.synchronize()
+    seen.export_chrome_trace(str(tmp_path / "trace.json"))
+    with open(tmp_path / "trace.json") as f:
+        (grid,) = [e["args"]["grid"][0] for e in json.load(f)["traceEvents"] if e.get("cat") == "kernel" and "::product_kernel" in e["name"]]
+    tiles = -(-M // 128) * -(-N // 128)
+    assert 1 < grid // tiles <= most
+    _close(dw, dy, x)
 
 
 def _step(call, x, w, g):
