@@ -163,10 +163,15 @@ __global__ __launch_bounds__(256) void sum_kernel(const unsigned short* __restri
   }
 }
 
-// what the kernels take; everything else is the library's
+// What the kernels take; everything else is the library's. One row's tokens are summed by one block for each 512 channels, the library's segments by many: over
+// many tokens, of which the frequent rows have their share (a row's number is log-uniform below), narrow tables and tables of few rows wait for the most frequent.
+// us, here and there, 16384, 32768 and 131072 tokens: 8192 rows of 128 97 and 101, 191 and 148, 767 and 391; 2048 of 512 116 and 112, 229 and 182, 877 and 504; 32000 of
+// 768 103 and 132, 185 and 206, 705 and 583; 8192 of 1024 105 and 133, 205 and 205, 834 and 667, 32000 of 1024 104 and 144, 185 and 226, 773 and 781; 512 of 2048
+// 139 and 156, 267 and 259, 1147 and 1207; 32000 of 2048 107 and 214, 195 and 406, 828 and 1119. All tokens alike: 131072 in 32000 rows of 1024 3600 and 3960, in 256 of
+// 4096 3400 and 6000. Every listing block goes through all tokens: up to 2^26 of them in all that is no more than the library's sort takes (1048576 tokens, 8192 rows).
 bool serves(const at::Tensor& dy, const at::Tensor& tokens, int64_t V) {
   const long T = tokens.numel(), W = dy.size(-1);
-  // every listing block goes through all tokens: 2^26 of them in all take about 0.1 ms
+  if (T > 16384 && W < 2048 && (W < 1024 || V < 32000)) return false;
   return plain(dy) && plain(tokens) && dy.is_cuda() && tokens.device() == dy.device() && dy.scalar_type() == at::kBFloat16 && tokens.scalar_type() == at::kLong
       && W > 0 && W % 8 == 0 && T > 0 && V > 0 && (V + 255) / 256 * 64 * ((W + 511) / 512) < (1L << 23) && (V + ROWS - 1) / ROWS * T <= (1L << 26);
 }

@@ -67,6 +67,31 @@ def test_repeats_and_second_derivatives():
     assert torch.allclose(ddy.float(), 2 * dw.float()[tokens], rtol=1e-2, atol=1e-2)
 
 
+def _is_native(V, W, T):
+    weight = torch.zeros(V, W, device="cuda", dtype=torch.bfloat16, requires_grad=True)
+    from colossalai_amd import _C
+
+    out = _C.embedding(torch.randint(0, V, (T,), device="cuda"), weight)
+    dy = torch.ones_like(out)
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CUDA]) as seen:
+        torch.autograd.grad(out, weight, dy)
+        torch.cuda.synchronize()
+    return any("list_kernel" in e.key for e in seen.key_averages())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("V,W,T,native", [
+    (2048, 512, 16384, True), (2048, 512, 16385, False), (50304, 1016, 16385, False),   # narrow
+    (31999, 1024, 16385, False), (32000, 1024, 16385, True), (1024, 2040, 16385, False), (512, 2048, 16385, True),   # few rows
+])
+def test_many_tokens(V, W, T, native):
+    """Over many tokens one row's are too many for the few blocks that a narrow or a small table has for it: the library's."""
+    assert _is_native(V, W, T) == native
+    if V < 32000:
+        layer = nn.Embedding(V, W, device="cuda", dtype=torch.bfloat16)
+        _check(layer, (torch.rand(T, device="cuda") * 7).exp().long().clamp(max=V - 1))   # by frequency
+
+
 @pytest.mark.gpu
 def test_what_a_layer_takes():
     tokens = torch.randint(0, 2048, (3, 50), device="cuda")
