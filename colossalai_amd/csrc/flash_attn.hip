@@ -96,7 +96,10 @@ DEV_INLINE bool deal(int f, int n_x, int n_y, int W, bool pairs, int& x, int& y)
   const int parts = row_parts(n_y), rows = n_y * parts / 8, tiles = (n_x + parts - 1) / parts, all = rows * tiles;
   int i = f >> 3;
   if (i >= all) return false;
-  if (pairs && all <= 64 && i >= 32) i = all - 1 - (i - 32);
+  if (pairs && all <= 64) {   // all of its rows, whatever its L2 holds: in fours a long tile of the last rows met another one (B2 S4500 H5 D128 92 us for 80)
+    W = rows;
+    if (i >= 32) i = all - 1 - (i - 32);
+  }
   const int first = i / (W * tiles) * W, wide = min(W, rows - first);
   i -= first * tiles;
   const int row = (f & 7) * rows + first + i % wide;
@@ -174,7 +177,8 @@ DEV_INLINE void row_of_batch(int y, int B, int H, int group, bool padded, int& b
 // Which (q tile, sequence, head) a block of the forward works on, false if on none. Blocks of one (sequence, head) share an
 // XCD's L2. Packed batches run head by head, each head over all sequences: the other way round
 // the longest sequence is one XCD's work (10 sequences of 256..4096 tokens: 1488 against 463 us). Under a causal
-// mask the late tiles see the most keys: they start first. `dealt`: tiles of a row that deal() takes, of the packed batch or of a causal sequence.
+// mask the late tiles see the most keys: they start first. Up to 512 blocks run at once, two on a CU: every second head of a dense batch goes the other way, so that the
+// two are a long one and a short one. `dealt`: tiles of a row that deal() takes, of the packed batch or of a causal sequence.
 template <bool VARLEN>
 DEV_INLINE bool q_block(const int* __restrict__ CU, int rows, int B, int Hq, int group, int causal, int W, int dealt, int most, int& tile, int& b, int& h) {
   int y;
@@ -195,7 +199,7 @@ DEV_INLINE bool q_block(const int* __restrict__ CU, int rows, int B, int Hq, int
     const int i = b * (int)gridDim.x + tile;
     tile = (int)gridDim.x - 1 - i / B;
     b = i % B;
-  } else if (causal) {
+  } else if (causal && (VARLEN || !(y & 1) || (int)(gridDim.x * gridDim.y) > 512)) {
     tile = (int)gridDim.x - 1 - tile;
   }
   return true;
@@ -1308,6 +1312,19 @@ int fwd_waves(long blocks) { return blocks <= 128 ? 2 : 4; }
 // and 276, 74 and 269, 74 and 272; B1 S8192 H12 D64 (two of three rows an XCD) 175 and 386, 123 and 338; B1 S8192 H32/8 D128 554 and 1645, 527 and 1579.
 int rows_together(int group, long kv_bytes) { return (int)std::max(4L, group * std::min(16L, (8L << 20) / std::max(1L, kv_bytes))); }
 
+// Whether rows that row_parts XCDs share are dealt tile by tile. Those of few tiles are not: the parts differ by a tile, or its place stays empty. us, in order and dealt,
+// forward of 64 channels unless said: three tiles, 140 rows (2 XCDs a row) 11.4, 14.6, 99 rows (8) 10.8, 14.3; five of 128 channels, 66 rows (4) 20.9, 24.5; six, 63 rows (8)
+// 14.8, 17.6; eight, 40 rows (1) 29, 22, 36 (2) 20.7, 15.8, 76 (2) 28.6, 28.3; 16 of 128, 30 (4) 55, 48; 32, 20 (2) 90, 61; 64, 9 (8) 152, 105. Backward: three of 128,
+// 366 (4) 84, 113.
+bool worth_dealing(long tiles, int n_y) { return tiles >= 4 * fa::row_parts(n_y); }
+
+// The causal dense forward's rows, of more than 256 blocks: three tiles too where all blocks run at once. us, in order and dealt: B8 S384 H16/4 D128 17.5, 15.2, but
+// B64 S384 H16/4 80, 87; B64 S36 H12 D64 6.5, 7.5; B24 S256 H12 14.2, 14.8.
+bool deals(int S, int n_y, long blocks) {
+  const long tiles = (S + 127) / 128;
+  return blocks > 256 && (worth_dealing(tiles, n_y) || (tiles == 3 && n_y % 8 == 0 && blocks <= 512));
+}
+
 // Tiles of a packed batch that its blocks look up (packed_tile), an upper bound; 0: sequence by sequence or tile by tile. Sequences of one tile need no
 // order, and small grids run at once in any. us, forward and backward, before and by lookup: 16384 tokens of up to 4096 in 12 sequences, 32/8 heads of
 // 128 363 and 1110, 346 and 1072; 12 of 64 96 and 257, 80 and 235; 64 sequences of up to 900, 8/2 of 128 54 and 187, 37 and 138; 46 of 1024, 32/8 of 128 169
@@ -1374,29 +1391,30 @@ std::vector<at::Tensor> flash_attn_fwd(at::Tensor q, at::Tensor k, at::Tensor v,
   auto stream = at::hip::getCurrentHIPStream();
   const long qbs = q.stride(0), qts = q.stride(1), kbs = k.stride(0), kts = k.stride(1);
 
-#define LAUNCH_FWD_AS(DD, NW, DEAL)                                                                            \
+#define LAUNCH_FWD(DD, NW, DEAL)                                                                            \
   do {                                                                                            \
-    const int tiles = (S + NW * QW - 1) / (NW * QW), dealt = causal && (long)tiles * B * Hq > 256 ? tiles : 0;  \
+    const int tiles = (S + NW * QW - 1) / (NW * QW);                                                \
     const size_t lds = 4 * tile_bytes<KVB, DD>();                                                  \
     set_lds_limit((const void*)fa_fwd_kernel<DD, NW, false, DEAL>, lds);                                \
-    hipLaunchKernelGGL((fa_fwd_kernel<DD, NW, false, DEAL>), dealt ? wide_grid(dealt_blocks(tiles, B * Hq)) : dim3((unsigned)tiles, B * Hq), \
+    hipLaunchKernelGGL((fa_fwd_kernel<DD, NW, false, DEAL>), DEAL ? wide_grid(dealt_blocks(tiles, B * Hq)) : dim3((unsigned)tiles, B * Hq), \
                        dim3(NW * 64), lds, stream.stream(),                                       \
                        (const unsigned short*)q.data_ptr(), (const unsigned short*)k.data_ptr(),  \
                        (const unsigned short*)v.data_ptr(), (unsigned short*)o.data_ptr(),        \
                        lse.data_ptr<float>(), cu, cuk, qbs, qts, kbs, kts,                        \
-                       B, S, Sk, Hq, Hkv, (float)scale, causal ? 1 : 0, rows_together(Hq / Hkv, Sk * DD * 4L), dealt, 0);  \
+                       B, S, Sk, Hq, Hkv, (float)scale, causal ? 1 : 0, rows_together(Hq / Hkv, Sk * DD * 4L), DEAL ? tiles : 0, 0);  \
   } while (0)
-#define LAUNCH_FWD(DD, NW)                                                                              \
-  do {                                                                                            \
-    if (causal && (S + NW * QW - 1L) / (NW * QW) * B * Hq > 256) LAUNCH_FWD_AS(DD, NW, true);      \
-    else LAUNCH_FWD_AS(DD, NW, false);                                                             \
+#define LAUNCH_FWD_D(NW, DEAL)            \
+  do {                                     \
+    if (D == 128) LAUNCH_FWD(128, NW, DEAL); \
+    else LAUNCH_FWD(64, NW, DEAL);           \
   } while (0)
 
-  const int nw = fwd_waves((S + 4 * QW - 1L) / (4 * QW) * B * Hq);
-  if (D == 128) { if (nw == 4) LAUNCH_FWD(128, 4); else LAUNCH_FWD(128, 2); }
-  else { if (nw == 4) LAUNCH_FWD(64, 4); else LAUNCH_FWD(64, 2); }
+  const long blocks = (S + 4 * QW - 1L) / (4 * QW) * B * Hq;   // of four waves
+  if (fwd_waves(blocks) == 2) LAUNCH_FWD_D(2, false);
+  else if (causal && deals(S, B * Hq, blocks)) LAUNCH_FWD_D(4, true);
+  else LAUNCH_FWD_D(4, false);
 #undef LAUNCH_FWD
-#undef LAUNCH_FWD_AS
+#undef LAUNCH_FWD_D
   HIP_CHECK_LAST();
   return {o, lse};
 }
@@ -1497,8 +1515,9 @@ void launch_bwd(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, c
   const long n_part = (VARLEN ? (long)Sk : (long)seqs * Sk) * Hkv * D;
   at::Tensor part;
   if (gs > 1) part = at::empty({gs * 2 * n_part}, q.options().dtype(at::kFloat));
-  const long dealt = VARLEN ? packed_tiles(S, seqs, q_tiles, rows, Hq) : causal && S_max == Sk_max ? q_tiles : 0;
   const int each = VARLEN ? 1 : seqs;
+  auto even = [&](int n_y) { return fa::row_parts(n_y) == 1 ? q_tiles > 1 : worth_dealing(q_tiles, n_y); };
+  const long dealt = VARLEN ? packed_tiles(S, seqs, q_tiles, rows, Hq) : causal && S_max == Sk_max && even(each * Hkv * gs) && even(each * Hq) ? q_tiles : 0;
   const long n_kv = dealt ? (dealt_blocks(dealt, each * Hkv * gs) + 7) / 8 * 8 : ((long)kv_tiles * seqs * Hkv * gs + 7) / 8 * 8;
   const long n_q = dealt ? dealt_blocks(dealt, each * Hq) : (long)q_tiles * seqs * Hq, blocks = n_kv + n_q;
   TORCH_CHECK(blocks < (1L << 31) - (1L << 23), "flash_attn_bwd: too many tiles");

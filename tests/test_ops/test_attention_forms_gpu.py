@@ -7,6 +7,8 @@ their gradients, the output in delta): three such errors add up to 2^-8 in the 2
 is left for their not being independent.
 """
 
+import json
+
 import pytest
 import torch
 
@@ -227,6 +229,47 @@ def test_rows_dealt_to_the_chips_parts(B, S, H, G):
 
     o = flash_attention(*a, causal=True)
     for name, x, y in zip(("out", "dq", "dk", "dv"), [o] + list(torch.autograd.grad(o, a, dout)), _reference(q, k, v, dout, True, 0.125)):
+        _near(x, y, name)
+
+
+def _launches(call, tmp_path):
+    """Template arguments and grids of the attention kernels that a call runs, and what it returns."""
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CUDA]) as seen:
+        out = call()
+        torch.cuda.synchronize()
+    seen.export_chrome_trace(str(tmp_path / "trace.json"))
+    with open(tmp_path / "trace.json") as f:
+        kernels = [e for e in json.load(f)["traceEvents"] if e.get("cat") == "kernel"]
+    found = {k: [e for e in kernels if k in e["name"]] for k in ("fa_fwd_kernel", "fa_bwd_kernel")}
+    return {k: (e[0]["name"].split("<")[1].split(">")[0].replace(" ", ""), e[0]["args"]["grid"]) for k, e in found.items() if e}, out
+
+
+@pytest.mark.parametrize("B,S,H,D,forward,backward", [
+    (64, 100, 6, 64, False, False), (60, 200, 4, 64, False, True), (8, 384, 16, 128, True, True), (26, 300, 8, 64, False, True),   # one tile, two, three
+    (8, 400, 16, 64, True, True),                                                                                                   # four
+    (11, 300, 9, 64, False, False), (7, 600, 10, 128, False, False), (3, 1000, 14, 64, False, False), (9, 500, 12, 64, False, False),   # an XCD has a part of a row
+    (2, 1000, 18, 64, True, True),
+])
+def test_rows_of_few_tiles_stay_in_order(B, S, H, D, forward, backward, tmp_path):
+    """Rows that several XCDs would share are dealt if each gets four tiles of them or more, whole ones of four tiles or more (the backward's: of two),
+    of three if all blocks run at once."""
+    from colossalai_amd.ops import flash_attention
+
+    q, k, v, dout = _inputs(B, S, H, H, D, S)
+    a = [t.clone().requires_grad_() for t in (q, k, v)]
+
+    def step():
+        o = flash_attention(*a, causal=True)
+        return [o] + list(torch.autograd.grad(o, a, dout))
+
+    seen, got = _launches(step, tmp_path)
+    tiles, rows = (S + 127) // 128, B * H
+    parts = next(n for n in (1, 2, 4, 8) if rows * n % 8 == 0)
+    assert tiles * rows > 256
+    assert seen["fa_fwd_kernel"][0] == f"{D},4,false,{str(forward).lower()}"
+    in_order = (tiles * rows + 7) // 8 * 8 + tiles * rows
+    assert seen["fa_bwd_kernel"][1][0] == (2 * -(-tiles // parts) * parts * rows if backward else in_order)
+    for name, x, y in zip(("out", "dq", "dk", "dv"), got, _reference(q, k, v, dout, True, D ** -0.5)):
         _near(x, y, name)
 
 
