@@ -160,11 +160,12 @@ DEV_INLINE bool packed_tile(const int* __restrict__ CU, int B, int rows, int mos
   return true;
 }
 
-// Sequence and head of row y of a dense batch: sequence by sequence, or with lengths (`padded`) key head by key head over all sequences, so that no XCD has
-// only long ones. us, forward and backward, lengths between a quarter and all: B16 S512 H12 D64 20.6 and 55.4 -> 18.8 and 52.9; B8 S2048 H12 D64 103 and 292 ->
+// Sequence and head of row y of a dense batch: sequence by sequence, or with lengths and more than a tile (the forward: two) `by_head`, key head by key head over all
+// sequences, so that no XCD has only long ones. Tiles of one row take about as long whatever their length, and neighbours in memory are read together (forward, us, by
+// sequence and by head: B32 S128 H12 D64 9.3, 9.8; B16 S256 H12 10.1, 10.9, but B24 S256 H16/4 D128 24.6, 22.6). With lengths that differ little both take the same. us, forward and backward, lengths between a quarter and all: B16 S512 H12 D64 20.6 and 55.4 -> 18.8 and 52.9; B8 S2048 H12 D64 103 and 292 ->
 // 90 and 231; B4 S4096 H8 D64 147 and 425 -> 100 and 261; causal, D128: B8 S2048 H32/8 244 and 760 -> 212 and 595, B2 S4096 H16/4 136 and 451 -> 118 and 366.
-DEV_INLINE void row_of_batch(int y, int B, int H, int group, bool padded, int& b, int& h) {
-  if (padded) {
+DEV_INLINE void row_of_batch(int y, int B, int H, int group, bool by_head, int& b, int& h) {
+  if (by_head) {
     const int k = y / group;
     b = k % B;
     h = k / B * group + y % group;
@@ -180,12 +181,12 @@ DEV_INLINE void row_of_batch(int y, int B, int H, int group, bool padded, int& b
 // mask the late tiles see the most keys: they start first. Up to 512 blocks run at once, two on a CU: every second head of a dense batch goes the other way, so that the
 // two are a long one and a short one. `dealt`: tiles of a row that deal() takes, of the packed batch or of a causal sequence.
 template <bool VARLEN>
-DEV_INLINE bool q_block(const int* __restrict__ CU, int rows, int B, int Hq, int group, int causal, int W, int dealt, int most, int& tile, int& b, int& h) {
+DEV_INLINE bool q_block(const int* __restrict__ CU, int rows, int B, int Hq, int group, int causal, int W, int dealt, int most, bool by_head, int& tile, int& b, int& h) {
   int y;
   if (dealt) {
     if (!deal((int)(blockIdx.y * gridDim.x + blockIdx.x), dealt, (VARLEN ? 1 : B) * Hq, W, true, tile, y)) return false;
     h = y;
-    if (!VARLEN) row_of_batch(y, B, Hq, group, CU != nullptr, b, h);
+    if (!VARLEN) row_of_batch(y, B, Hq, group, by_head, b, h);
     int tiles = dealt;
     if (VARLEN && !packed_tile(CU, B, rows, most, tile, b, tile, tiles)) return false;
     if (causal) tile = tiles - 1 - tile;
@@ -194,7 +195,7 @@ DEV_INLINE bool q_block(const int* __restrict__ CU, int rows, int B, int Hq, int
   xcd_swizzle_xy(tile, y);
   b = y % B;
   h = y / B;
-  if (!VARLEN) row_of_batch(y, B, Hq, group, CU != nullptr, b, h);
+  if (!VARLEN) row_of_batch(y, B, Hq, group, by_head, b, h);
   if (VARLEN && causal && by_tile((int)gridDim.x, (long)gridDim.x * gridDim.y, group)) {
     const int i = b * (int)gridDim.x + tile;
     tile = (int)gridDim.x - 1 - i / B;
@@ -316,7 +317,7 @@ __global__ __launch_bounds__(NW * 64, 2) void fa_fwd_kernel(
   const int ln = lane & 31;
 
   int tile, b, h;
-  if (!q_block<VARLEN>(CU, NW * QW, B, Hq, Hq / Hkv, causal, W, DEAL ? dealt : 0, most, tile, b, h)) return;
+  if (!q_block<VARLEN>(CU, NW * QW, B, Hq, Hq / Hkv, causal, W, DEAL ? dealt : 0, most, CU != nullptr && S > 2 * NWB * QW, tile, b, h)) return;
   const int hk = h / (Hq / Hkv);
   const int q0 = tile * (NW * QW);
   const int qw = q0 + w * QW;  // this wave's first q row
@@ -721,12 +722,13 @@ DEV_INLINE void bwd_dkdv(
   // key/value tile fastest, then the part of the group's heads, then (sequence, kv head): their
   // Q/dO streams meet in one XCD's L2. Under a causal mask the first tiles see the most queries.
   int tile, part, b, hk;
+  const bool by_head = CU != nullptr && S > NWB * QW;
   if (dealt) {
     int y, all;
     if (!deal(f, dealt, (VARLEN ? 1 : B) * Hkv * GS, W, false, tile, y)) return;
     part = y % GS;
     hk = y / GS;
-    if (!VARLEN) row_of_batch(y / GS, B, Hkv, 1, CU != nullptr, b, hk);
+    if (!VARLEN) row_of_batch(y / GS, B, Hkv, 1, by_head, b, hk);
     if (VARLEN && !packed_tile(CU, B, NWB * QW, tiles, tile, b, tile, all)) return;
   } else {
     f = xcd_chunk(f, nblocks);
@@ -736,7 +738,7 @@ DEV_INLINE void bwd_dkdv(
     if (y >= B * Hkv) return;
     b = y % B;
     hk = y / B;
-    if (!VARLEN) row_of_batch(y, B, Hkv, 1, CU != nullptr, b, hk);
+    if (!VARLEN) row_of_batch(y, B, Hkv, 1, by_head, b, hk);
   }
   const int kv0 = tile * (NWB * QW);
   const int group = Hq / Hkv, h_first = part * group / GS;
@@ -1020,11 +1022,12 @@ DEV_INLINE void bwd_dq(
   const int ln = lane & 31;
 
   int y, tile, b, h;
+  const bool by_head = CU != nullptr && S > NWB * QW;
   if (dealt) {
     int all = dealt;
     if (!deal(f, dealt, (VARLEN ? 1 : B) * Hq, W, false, tile, y)) return;
     h = y;
-    if (!VARLEN) row_of_batch(y, B, Hq, Hq / Hkv, CU != nullptr, b, h);
+    if (!VARLEN) row_of_batch(y, B, Hq, Hq / Hkv, by_head, b, h);
     if (VARLEN && !packed_tile(CU, B, NWB * QW, tiles, tile, b, tile, all)) return;
     if (causal) tile = all - 1 - tile;  // late tiles see the most keys
   } else {
@@ -1034,7 +1037,7 @@ DEV_INLINE void bwd_dq(
     if (y >= B * Hq) return;
     b = y % B;
     h = y / B;
-    if (!VARLEN) row_of_batch(y, B, Hq, Hq / Hkv, CU != nullptr, b, h);
+    if (!VARLEN) row_of_batch(y, B, Hq, Hq / Hkv, by_head, b, h);
     if (VARLEN && causal && by_tile(tiles, nblocks, Hq / Hkv)) {
       const int i = b * tiles + tile;
       tile = tiles - 1 - i / B;

@@ -273,6 +273,25 @@ def test_rows_of_few_tiles_stay_in_order(B, S, H, D, forward, backward, tmp_path
         _near(x, y, name)
 
 
+@pytest.mark.parametrize("S", [100, 200, 300])
+@pytest.mark.parametrize("H,G,causal", [(6, 6, False), (8, 2, True)])
+def test_padded_batches_of_few_tiles(S, H, G, causal):
+    """One tile: sequence by sequence. Two: so in the forward. Three: key head by key head."""
+    from colossalai_amd.ops import flash_attention
+
+    B = 50
+    q, k, v, dout = _inputs(B, S, H, G, 64, S)
+    lens = [0 if b == 7 else max(20, S - 37 * b % (3 * S // 4)) for b in range(B)]
+    a = [t.clone().requires_grad_() for t in (q, k, v)]
+    o = flash_attention(*a, causal=causal, seqlens=torch.tensor(lens, dtype=torch.int32, device="cuda"))
+    got = [o] + list(torch.autograd.grad(o, a, dout))
+    for b, n in enumerate(lens):
+        assert not any(x[b, n:].any() for x in got)
+        if n:
+            for name, x, y in zip(("out", "dq", "dk", "dv"), got, _reference(*(t[b: b + 1, :n] for t in (q, k, v, dout)), causal, 0.125)):
+                _near(x[b: b + 1, :n], y, f"{name} {b}")
+
+
 @pytest.mark.parametrize("causal", [True, False])
 @pytest.mark.parametrize("lens,H,G", [
     ([900, 1, 0, 900, 129, 1500, 128, 640], 12, 12),               # equal lengths, an empty one, tiles that are just full
