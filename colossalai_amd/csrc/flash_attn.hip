@@ -80,7 +80,7 @@ DEV_INLINE constexpr int crow(int j, int half) { return (j & 3) + 8 * (j >> 2) +
 // met in L2 by the tiles that run together. By sequence / by tile, us, forward and backward: 186 sequences of up to 256 tokens, 16/4
 // heads of 64: 48 / 39, 151 / 141; 54 of 900, 8/2 of 128: 58 / 49, 210 / 200; 46 of 1024, 32/8: 193 / 179, 534 / 531 (41: 188 / 185,
 // 541 / 554); but 14 of 4096: 406 / 437, 1108 / 1147; 81 of 600, 12 heads of 64: 39 / 45, 110 / 116; 20 of 300, 8 heads: 9.3 / 10.4.
-DEV_INLINE bool by_tile(int tiles, long blocks, int group) { return tiles <= 8 && blocks > 512 && group > 1; }
+__host__ __device__ __forceinline__ bool by_tile(int tiles, long blocks, int group) { return tiles <= 8 && blocks > 512 && group > 1; }
 
 // XCDs that share a row of tiles, so that all of them get as much: 1, 2, 4 or 8
 __host__ __device__ __forceinline__ int row_parts(int n_y) { return n_y % 8 == 0 ? 1 : n_y % 4 == 0 ? 2 : n_y % 2 == 0 ? 4 : 8; }
@@ -1337,6 +1337,14 @@ long packed_tiles(long T, int n_seq, long tiles, int rows, int H) {
   return n_seq <= fa::MOST_PACKED && tiles > 1 && all * H > 512 ? all : 0;
 }
 
+// The forward's. Where tile by tile is the other order (by_tile) a look-up, longer than the one it takes the place of, pays with 128 channels, three tiles or more and 1024
+// blocks. us, by tile and looked up: 16384 tokens of up to 160, 16/4 heads of 64 34, 39, 64/8 133, 156, 16/8 of 128 60, 66; of up to 400, 32/4 of 128 142, 129, 32/8
+// 141, 134, 16/4 of 64 35.5, 37.3; 12000 of up to 700, 8/2 of 128 30.3, 32.4; 16384 of up to 1000, 32/4 of 128 183, 159, 32/8 199, 169, 16/4 of 64 45.3, 48.5, 64/8 192, 189.
+long packed_tiles_fwd(long T, int n_seq, long tiles, int rows, int H, int group, int D, bool causal) {
+  const long all = packed_tiles(T, n_seq, tiles, rows, H);
+  return causal && fa::by_tile((int)tiles, tiles * n_seq * H, group) && (D == 64 || tiles <= 2 || all * H <= 1024) ? 0 : all;
+}
+
 // a grid dimension of 2^32 threads or more is cut short without an error
 dim3 wide_grid(long blocks) {
   const long width = std::max(1L, std::min(blocks, 1L << 23));
@@ -1447,7 +1455,7 @@ std::vector<at::Tensor> flash_attn_varlen_fwd(at::Tensor q, at::Tensor k, at::Te
 #define LAUNCH_VFWD(DD, NW)                                                                           \
   do {                                                                                            \
     const size_t lds = 4 * tile_bytes<KVB, DD>();                                                  \
-    const long tiles = (max_seqlen + NW * QW - 1) / (NW * QW), packed = packed_tiles(T, n_seq, tiles, NW * QW, Hq);  \
+    const long tiles = (max_seqlen + NW * QW - 1) / (NW * QW), packed = packed_tiles_fwd(T, n_seq, tiles, NW * QW, Hq, Hq / Hkv, D, causal);  \
     set_lds_limit((const void*)fa_fwd_kernel<DD, NW, true, true>, lds);                                 \
     hipLaunchKernelGGL((fa_fwd_kernel<DD, NW, true, true>),                                             \
                        packed ? wide_grid(dealt_blocks(packed, Hq)) : dim3((unsigned)tiles, n_seq * Hq), dim3(NW * 64), lds, stream.stream(), \

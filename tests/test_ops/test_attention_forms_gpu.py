@@ -292,6 +292,29 @@ def test_padded_batches_of_few_tiles(S, H, G, causal):
                 _near(x[b: b + 1, :n], y, f"{name} {b}")
 
 
+@pytest.mark.parametrize("lens,H,G,D,looked_up", [
+    ([150, 60] * 30, 16, 4, 64, False), ([150, 60] * 30, 32, 4, 128, False),                                                # two tiles
+    ([400, 250, 130] * 10, 32, 8, 64, False), ([400, 250, 130] * 5, 16, 8, 128, False), ([400, 250, 130] * 10, 32, 4, 128, True),
+    ([150, 60] * 30, 12, 12, 64, True), ([1100, 250] * 5, 16, 4, 64, True),                                                  # ungrouped heads; long sequences
+])
+def test_packed_forward_tile_by_tile(lens, H, G, D, looked_up, tmp_path):
+    """Grouped heads over short sequences: the forward looks tiles up with 128 channels, more than two tiles and 1024 blocks."""
+    from colossalai_amd.ops import flash_attention_varlen
+
+    T = sum(lens)
+    q, k, v, dout = (t[0] for t in _inputs(1, T, H, G, D, T))
+    a = [t.clone().requires_grad_() for t in (q, k, v)]
+    cu = torch.tensor([0] + lens).cumsum(0).int().cuda()
+    seen, o = _launches(lambda: flash_attention_varlen(*a, cu, max(lens), causal=True), tmp_path)
+    assert (seen["fa_fwd_kernel"][1][1] == 1) == looked_up   # a line of blocks, or one of tiles for each sequence and head
+    got = [o] + list(torch.autograd.grad(o, a, dout))
+    at = 0
+    for n in lens:
+        for name, x, y in zip(("out", "dq", "dk", "dv"), got, _reference(*(t[None, at: at + n] for t in (q, k, v, dout)), True, D ** -0.5)):
+            _near(x[at: at + n], y[0], f"{name} {n}")
+        at += n
+
+
 @pytest.mark.parametrize("causal", [True, False])
 @pytest.mark.parametrize("lens,H,G", [
     ([900, 1, 0, 900, 129, 1500, 128, 640], 12, 12),               # equal lengths, an empty one, tiles that are just full
