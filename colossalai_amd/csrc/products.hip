@@ -144,7 +144,7 @@ DEV_INLINE void put(const Args& a, long at, float4v v) {
 
 // c += x y. The compiler copies sums that are loop-carried in accumulation registers to other ones and back around each product of this size (128 moves and 50
 // waits in a loop of 32 products), so it is told the register. What the compiler would otherwise look after: settled() stands between these products and
-// any other use of the sums, ahead of them and behind them.
+// any other use of the sums, ahead of them and behind them. check_products.py looks for these distances in what each build has made of it.
 template <bool ACC>
 DEV_INLINE void mac(float4v& c, bf16x8_v x, bf16x8_v y) {
   if constexpr (ACC) asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(x), "v"(y));

@@ -6,6 +6,7 @@ fatbins, no CUDA paths.
 """
 
 import os
+import sys
 
 from setuptools import find_packages, setup
 
@@ -71,6 +72,19 @@ cpu_ext = CppExtension(
     extra_link_args=["-fopenmp"],
 )
 
+
+class Build(BuildExtension):
+    """Looks the training kernels' machine code over once they are built."""
+
+    def run(self):
+        super().run()
+        if ext in self.extensions:
+            sys.path.insert(0, CSRC)
+            import check_products
+
+            check_products.check(self.get_ext_fullpath(ext.name))
+
+
 setup(
     name="colossalai_amd",
     version="0.1.0",
@@ -78,5 +92,5 @@ setup(
     # COLOSSALAI_AMD_EXTENSIONS=serving / serving_state builds just that one serving extension
     ext_modules={"serving": [serving_ext], "serving_state": [state_ext]}.get(
         os.environ.get("COLOSSALAI_AMD_EXTENSIONS"), [ext, cpu_ext, serving_ext, state_ext]),
-    cmdclass={"build_ext": BuildExtension.with_options(use_ninja=True)},
+    cmdclass={"build_ext": Build.with_options(use_ninja=True)},
 )
