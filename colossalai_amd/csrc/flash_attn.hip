@@ -232,8 +232,7 @@ struct TileLoad {
     off = (unsigned)(r * stride) * 2u + unit * 16;
   }
   // what the loads of the tile from row0 on share
-  DEV_INLINE __amdgpu_buffer_rsrc_t tile(int row0) const { return tile(base, row0); }
-  DEV_INLINE __amdgpu_buffer_rsrc_t tile(const unsigned short* base, int row0) const {   // of another matrix of these rows
+  DEV_INLINE __amdgpu_buffer_rsrc_t tile(int row0) const {
     const int left = min(rows - row0, ROWS);
     const unsigned bytes = left > 0 ? (unsigned)((left - 1) * stride + D) * 2u : 0u;
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<unsigned short*>(base + (left > 0 ? row0 * stride : 0)), 0, (int)bytes, 0x00027000);
@@ -691,9 +690,10 @@ constexpr bool CAN_OWN = D == 64 && !VARLEN;
 
 // A block of 4 waves owns 128 key/value rows, 32 a wave, and streams the query tiles of its group's heads
 // (32 rows, double-buffered). dK and dV stay in registers. What a query row adds (its -lse log2e and
-// -delta) enters as the accumulator the product starts from and as the exponent's addend; a row
-// that counts nothing (padding, or no visible key) has an addend of -inf.
-// GS blocks share a key/value tile's heads, as evenly as they go, when there would be too few blocks otherwise; they leave
+// -delta) enters as the accumulator the product starts from and as the exponent's addend; a row of the sequence that sees
+// no key has an addend of -inf. Rows past the sequence's end add nothing because those of Q and dO are zeros: their descriptors
+// have to end with its last row. Their statistics are zeros by another such one, and so weights of 1, or (formed here) addends of -inf.
+// GS blocks share a key/value tile's heads, as evenly as they go, where a model of the launch (launch_bwd) says that it pays; they leave
 // float32 partial sums in PART [GS][2][B * Sk * Hkv * D] for fa_bwd_sum_kernel.
 template <int D, bool VARLEN>
 DEV_INLINE void bwd_dkdv(
@@ -832,7 +832,6 @@ DEV_INLINE void bwd_dkdv(
     if (own) {
       constexpr int TPR = D / 8, AT_ONCE = NTB / TPR;   // threads of a row, rows
       const int c = threadIdx.x % TPR, sub = threadIdx.x / TPR;
-#pragma unroll 4
       for (int at = 0; at < min(steps, OWN_TILES) * QB; at += AT_ONCE) {
         const int step = at / QB, head = step / nq, in = at % QB + sub, row = first + (step - head * nq) * QB + in;
         float dot = 0.0f, lse = -INFINITY;
@@ -859,7 +858,7 @@ DEV_INLINE void bwd_dkdv(
 
   int stats_at = 0;
   // A query tile, while the next one arrives in the other buffers.
-  auto step = [&](int qt0, int buf, const char* __restrict__ Qlds, const char* __restrict__ dOlds, char* __restrict__ Qn,
+  auto step = [&](int qt0, const char* __restrict__ Qlds, const char* __restrict__ dOlds, char* __restrict__ Qn,
                   char* __restrict__ dOn) __attribute__((always_inline)) {
     const float* stats = reinterpret_cast<const float*>(stats_lds + stats_at) + 4 * half;
     // ---- S[q][kv] = Q · K^T and dP[q][kv] - delta[q] = dO · V^T - delta: column = kv (ln), row = q
@@ -967,7 +966,7 @@ DEV_INLINE void bwd_dkdv(
     }
     for (; qt0 < last; qt0 += QB) {
       begin(qt0);
-      step(qt0, buf, Qbuf + buf * TB, dObuf + buf * TB, Qn, dOn);
+      step(qt0, Qbuf + buf * TB, dObuf + buf * TB, Qn, dOn);
       finish();
     }
   }
@@ -1412,7 +1411,7 @@ std::vector<at::Tensor> flash_attn_fwd(at::Tensor q, at::Tensor k, at::Tensor v,
                        (const unsigned short*)q.data_ptr(), (const unsigned short*)k.data_ptr(),  \
                        (const unsigned short*)v.data_ptr(), (unsigned short*)o.data_ptr(),        \
                        lse.data_ptr<float>(), cu, cuk, qbs, qts, kbs, kts,                        \
-                       B, S, Sk, Hq, Hkv, (float)scale, causal ? 1 : 0, rows_together(Hq / Hkv, Sk * DD * 4L), DEAL ? tiles : 0, 0);  \
+                       B, S, Sk, Hq, Hkv, (float)scale, causal ? 1 : 0, rows_together(Hq / Hkv, 4L * Sk * DD), DEAL ? tiles : 0, 0);  \
   } while (0)
 #define LAUNCH_FWD_D(NW, DEAL)            \
   do {                                     \
@@ -1555,7 +1554,7 @@ void launch_bwd(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, c
                      own ? nullptr : (const float2v*)stats.data_ptr(), (const unsigned short*)out.data_ptr(), lse.data_ptr<float>(), (unsigned short*)dq.data_ptr(), (unsigned short*)dk.data_ptr(),
                      (unsigned short*)dv.data_ptr(), gs > 1 ? part.data_ptr<float>() : nullptr, gs, cu, cuk, qbs, qts, kbs,
                      kts, dqbs, dqts, dkbs, dkts, (int)n_kv, (int)n_q, kv_tiles, q_tiles, seqs, S, Sk, Hq, Hkv, scale, causal ? 1 : 0,
-                     rows_together(G, Sk_max * D * 4L), (int)dealt);
+                     rows_together(G, 4L * Sk_max * D), (int)dealt);
   HIP_CHECK_LAST();
   if (gs > 1) {
     hipLaunchKernelGGL(fa_bwd_sum_kernel, dim3((unsigned)((n_part / 4 + 255) / 256)), dim3(256), 0, stream,

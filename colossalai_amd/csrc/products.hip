@@ -478,6 +478,12 @@ bool weight_grad_serves(const at::Tensor& dy, const at::Tensor& x) {
       && x.size(1) % 8 == 0 && ((dy.size(1) + 127) / 128) * ((x.size(1) + 127) / 128) < (1L << 20);
 }
 
+// Over few tokens storing a large result is most of the work, which the library does faster. Its time and the kernel's, us: 22016 x 4096 over
+// 64, 256, 512, 1024 and 2048 tokens 63, 103, 126, 213, 404 and 112, 143, 176, 241, 373; 4096 x 4096 12, 18, 26, 40, 71 and 23, 27,
+// 33, 45, 70. Over results of 9 to 131 million elements the kernel takes 1.5 times the library's at 100 tokens, 1.2 at 500, 1.06 from 1000 to
+// 1500 (1.2 at 1536) and 1 at 1700 to 2000; below 2^23 elements it is ahead or, up to 10 us, bound by the host (see multiply).
+static bool mostly_stores(const at::Tensor& dy, const at::Tensor& x) { return dy.size(0) < 1600 && dy.size(1) * x.size(1) > (1L << 23); }
+
 // dy [K, M], x [K, N] -> dy^T x (+ add, float32 [M, N]) in bfloat16, or in float32 with `keep`: then in `add` if that is given.
 at::Tensor weight_grad(const at::Tensor& dy, const at::Tensor& x, const c10::optional<at::Tensor>& add, bool keep) {
   if (add)
@@ -490,12 +496,8 @@ at::Tensor weight_grad(const at::Tensor& dy, const at::Tensor& x, const c10::opt
   }
   const bool serves = weight_grad_serves(dy, x);
   const pr::Plan plan = serves ? pr::plan(dy.size(1), x.size(1), dy.size(0), false) : pr::Plan{};
-  // Over few tokens storing a large result is most of the work, which the library does faster. Its time and the kernel's, us: 22016 x 4096 over
-  // 64, 256, 512, 1024 and 2048 tokens 63, 103, 126, 213, 404 and 112, 143, 176, 241, 373; 4096 x 4096 12, 18, 26, 40, 71 and 23, 27,
-  // 33, 45, 70. Over results of 9 to 131 million elements the kernel takes 1.5 times the library's at 100 tokens, 1.2 at 500, 1.06 from 1000 to
-  // 1500 (1.2 at 1536) and 1 at 1700 to 2000; below 2^23 elements it is ahead or, up to 10 us, bound by the host (see multiply). A
-  // float32 result the library does not have.
-  if (!serves || (!add && !keep && dy.size(0) < 1600 && dy.size(1) * x.size(1) > (1L << 23))) {
+  // a float32 result the library does not have
+  if (!serves || (!add && !keep && mostly_stores(dy, x))) {
     at::Tensor r = at::mm(dy.t(), x);
     if (add) r = keep ? add->add_(r) : at::add(*add, r);
     return r.to(keep ? at::kFloat : dy.scalar_type());
@@ -530,14 +532,14 @@ at::Tensor multiply(const at::Tensor& x, const at::Tensor& w, bool slow) {
 }
 
 // Both gradients of a small linear layer, dy [K, M] times w [M, N] and dy^T x with x [K, N], by one launch; empty where one of them is not small. Neither
-// fills the chip, and the host takes some 4 us for a launch, of which a step of two layers has eight less. Such steps' kernels, us: width 512, 512 tokens
-// 504 -> 441; 256, 2000 tokens 608 -> 553; 512, 2800 tokens 748 -> 720; 1024, 600 tokens 682 -> 654.
+// fills the chip, and the host takes some 4 us for a launch, of which a step of two layers has eight less. A weight gradient of 128 x 128 tiles beside a small
+// product takes at most 27 us by the plan, over all sizes. Kernels of both, us, one after the other and together, tokens, M, N: 512, 512, 512 18.5, 9.9;
+// 3000, 512, 512 24.3, 17.4; 512, 1024, 2048 22.6, 13.9; 1500, 1024, 2048 30.9, 24.4; 2000, 1024, 2048 33.6, 28.4; 12000, 256, 256 32.9, 26.1; 16000, 128, 256 33.1, 29.1.
 std::vector<at::Tensor> linear_grads(const at::Tensor& dy, const at::Tensor& w, const at::Tensor& x) {
   pr::Plan dx_plan;
-  if (!small_product(dy, w, true, dx_plan) || !weight_grad_serves(dy, x) || !pr::loadable(x)
-      || (dy.size(0) < 1600 && dy.size(1) * x.size(1) > (1L << 23))) return {};
+  if (!small_product(dy, w, true, dx_plan) || !weight_grad_serves(dy, x) || !pr::loadable(x) || mostly_stores(dy, x)) return {};
   const pr::Plan dw_plan = pr::plan(dy.size(1), x.size(1), dy.size(0), false);
-  if (dw_plan.tm != 128 || dw_plan.us > 25.0) return {};
+  if (dw_plan.tm != 128) return {};
   const c10::hip::HIPGuard guard(dy.device().index());
   const pr::Call dx = pr::call<false, true>(dy, w, dx_plan, c10::nullopt, false), dw = pr::call<true, true>(dy, x, dw_plan, c10::nullopt, false);
   const auto stream = at::hip::getCurrentHIPStream();

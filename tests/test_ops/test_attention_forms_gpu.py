@@ -244,6 +244,27 @@ def _launches(call, tmp_path):
     return {k: (e[0]["name"].split("<")[1].split(">")[0].replace(" ", ""), e[0]["args"]["grid"]) for k, e in found.items() if e}, out
 
 
+# more than 256 blocks of four waves, and from 513 on not all at once; rows a multiple of 8, of 4 and of 2, and odd ones: an XCD has whole ones, every
+# second, fourth or eighth tile. In the last but one an XCD's rows are more than it would take together.
+@pytest.mark.parametrize("B,S,H,G,D", [(2, 1100, 16, 4, 64), (1, 2900, 12, 12, 64), (1, 3600, 10, 5, 128), (1, 4100, 9, 3, 64),
+                                       (4, 620, 32, 8, 128), (1, 3000, 28, 4, 64), (1, 4700, 14, 2, 64), (2, 4500, 5, 5, 128), (1, 4200, 17, 17, 64)])
+@pytest.mark.parametrize("padded", [False, True])
+def test_forward_rows_dealt_to_the_chips_parts(B, S, H, G, D, padded, tmp_path):
+    """Causal batches beyond 256 blocks whose rows have tiles enough: the forward deals them too; padded ones go key head by key head."""
+    from colossalai_amd.ops import flash_attention
+
+    q, k, v, dout = _inputs(B, S, H, G, D, S)
+    lens = [S - (S // 3 + 5) * ((b + 1) % 3) for b in range(B)] if padded else [S] * B
+    a = [t.clone().requires_grad_() for t in (q, k, v)]
+    seen, o = _launches(lambda: flash_attention(*a, causal=True, seqlens=torch.tensor(lens, dtype=torch.int32, device="cuda") if padded else None), tmp_path)
+    assert seen["fa_fwd_kernel"][0] == f"{D},4,false,true"
+    got = [o] + list(torch.autograd.grad(o, a, dout))
+    for b, n in enumerate(lens):
+        for name, x, y in zip(("out", "dq", "dk", "dv"), got, _reference(*(t[b: b + 1, :n] for t in (q, k, v, dout)), True, D ** -0.5)):
+            _near(x[b: b + 1, :n], y, f"{name} {b}")
+            assert not x[b, n:].any()
+
+
 @pytest.mark.parametrize("B,S,H,D,forward,backward", [
     (64, 100, 6, 64, False, False), (60, 200, 4, 64, False, True), (8, 384, 16, 128, True, True), (26, 300, 8, 64, False, True),   # one tile, two, three
     (8, 400, 16, 64, True, True),                                                                                                   # four
@@ -312,6 +333,28 @@ def test_packed_forward_tile_by_tile(lens, H, G, D, looked_up, tmp_path):
     for n in lens:
         for name, x, y in zip(("out", "dq", "dk", "dv"), got, _reference(*(t[None, at: at + n] for t in (q, k, v, dout)), True, D ** -0.5)):
             _near(x[at: at + n], y[0], f"{name} {n}")
+        at += n
+
+
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("H,G,D", [(16, 16, 64), (18, 2, 64), (16, 4, 128), (20, 20, 128)])
+def test_packed_tiles_by_lookup_at_their_edges(H, G, D, causal):
+    """Equal lengths, an empty sequence ahead, between and behind, tiles that are just full and one row more."""
+    from colossalai_amd.ops import flash_attention_varlen
+
+    lens = [0, 900, 21, 0, 900, 129, 1500, 128, 640, 0]
+    T = sum(lens)
+    assert min(T // 128 + len(lens), 12 * len(lens)) * H > 512   # tiles by their bound and heads: beyond 512 blocks they are looked up
+    q, k, v, dout = (t[0] for t in _inputs(1, T, H, G, D, T))
+    a = [t.clone().requires_grad_() for t in (q, k, v)]
+    o = flash_attention_varlen(*a, torch.tensor([0] + lens).cumsum(0).int().cuda(), max(lens), causal=causal)
+    got = [o] + list(torch.autograd.grad(o, a, dout))
+    at = 0
+    for n in lens:
+        if n:
+            want = _reference(*(t[None, at: at + n] for t in (q, k, v, dout)), causal, D ** -0.5)
+            for name, x, y in zip(("out", "dq", "dk", "dv"), got, want):
+                _near(x[at: at + n], y[0], f"{name} {n}")
         at += n
 
 
