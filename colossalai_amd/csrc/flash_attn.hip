@@ -452,7 +452,11 @@ __global__ __launch_bounds__(NW * 64, 2) void fa_fwd_kernel(
   // the 32 ahead of them add, weights `pp` times the values from row vr at `V_`; none of these waits for another, and a
   // wave's instructions alternate between them. A product takes the matrix unit 32 cycles and the SIMD's issue 11; whatever else the SIMD's
   // waves issue (4 to 5 cycles, an exponential 8) fits beside it only if it stands between the products.
-  // Fragments are read a group ahead of the products that take them, with one wait a group (a wait for each was 16 of a turn's 190 instructions).
+  // Fragments are read a group ahead of the products that take them, with one wait a group (a wait for each was 16 of a turn's 190 instructions) or, in unmasked and
+  // small calls of four waves, as the compiler places them: few steps of two blocks a CU lose by the first group's wait more than they gain, longer ones nothing. us, one
+  // and several: B24 S117 H16 D64 9.0, 8.5; B20 S100 H16 D128 12.5, 11.9; B8 S1024 H12 D64 35.9, 35.6; B4 S4096 H16/4 D128 493, 492; but causal (dealt) B4 S1024 H32/8
+  // D128 46.5, 48.4, two waves B1 S1024 H16/4 D128 19.1, 19.6.
+  constexpr bool ONE_WAIT = DEAL || NW == 2;
   constexpr int NB = D / 32, GROUPS = D / 32;   // a group: two fragments of keys, two of values
   auto turn = [&](auto with_scores, auto with_weights, auto with_values, const char* __restrict__ K_, int kr, const char* __restrict__ V_, int vr,
                   f32x16& sn, const f32x16& s, Weights& p, const Weights& pp, auto load) __attribute__((always_inline)) {
@@ -486,7 +490,7 @@ __global__ __launch_bounds__(NW * 64, 2) void fa_fwd_kernel(
     for (int g = 0; g < GROUPS; ++g) {
       read(g + 1);
       __builtin_amdgcn_sched_barrier(0);
-      reads_left<READS>(g + 1 < GROUPS);
+      if (ONE_WAIT) reads_left<READS>(g + 1 < GROUPS);
 #pragma unroll
       for (int i = 2 * g; i < 2 * g + 2; ++i) {
         if (with_scores) {
